@@ -18,9 +18,13 @@
 // waves then take their operands from there.  (The first kernel converted in every wave that used an
 // element, twice per workgroup, and the conversions, not the matrix instructions, set its pace.)
 //
-// Range: activation scales are renormalised per row and weight scales per column by powers of two
-// (largest scale of a row / column moved into [2^10, 2^11)), so the fp16 products never overflow and
-// only contributions 2^-25 below the largest of their row / column can underflow.  The shifts are
+// Range: an activation code times its scale is a multiple of 2^-10 (half the E2M1 step times the smallest E4M3
+// scale) of at most six significant bits and at most 6 x 448 = 2688: every such value is an fp16 number as it
+// is, and the kernel needs no pass over a tile's scales ahead of its main loop.  (An earlier form shifted the scales of
+// every row so that the largest lay in [2^10, 2^11), which took that pass, one memory latency per eight k-groups and
+// tile: at M = 4608 a layer of K = 3072, N = 21504 took 514 us with it and 485 without, one of K = 15360, N = 3072 401
+// and 376.)  Weight scales are renormalised per column by powers of two when they are repacked (largest scale of a
+// column in [2^10, 2^11)); only contributions 2^-25 below the largest of their column can underflow.  That shift is
 // undone exactly in the epilogue.
 //
 // Tiling: workgroup = 4 waves (2 x 2), block tile 256 x 256, wave tile 128 x 128 = 4 x 4 MFMA tiles,
@@ -49,11 +53,6 @@ __device__ inline half8_t dequant_word_fp4(uint32_t w, half2_t s) {
     const half2_t t2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 2) * s;
     const half2_t t3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 3) * s;
     return half8_t{t0[0], t0[1], t1[0], t1[1], t2[0], t2[1], t3[0], t3[1]};
-}
-
-__device__ inline float e4m3_to_f32(uint32_t b) {
-    const uint32_t ex = (b >> 3) & 0xF, m = b & 7;
-    return ex == 0 ? ldexpf((float)m, -9) : ldexpf((float)(8 + m), (int)ex - 10);
 }
 
 __device__ inline float gelu_tanh(float x) {
@@ -159,7 +158,6 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
         lo = (int)(((t0 + 1) * nwg + units - 1) / units) - 1;  // first v with units (v + 1) / nwg > t0
         hi = (int)((t1 * nwg - 1) / units);                    // last v with units v / nwg < t1
     };
-    int *rowshift = (int *)(lds + SHIFT_OFF);  // [MAX_BATCH][256] power-of-two renormalisation of the rows
     constexpr uint32_t AS_ELT = 4, BS_ELT = 8;  // bytes of scales per (64-group, row / column)
     const uint32_t as_stride = (uint32_t)p.M_pad * AS_ELT, bs_stride = (uint32_t)p.N * BS_ELT;
 
@@ -168,12 +166,12 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
     // and k-group; scales: one word of four e4m3 per row, four fp16 per column and k-group).
     struct TileCtx {
         int tile, gb, ge;  // k-groups [gb, ge) of the tile
-        int m0, n0, shift;
+        int m0, n0;
         int col_ok;
         const uint8_t *a_ptr, *b_ptr, *as_ptr, *bs_ptr;
     };
     // follow: the segment after the one given by prev_* (the next tile, from its first k-group), without divisions
-    auto make_ctx = [&](int sidx, int slot, int tid, bool follow, int prev_tile, int prev_m0, int prev_n0) {
+    auto make_ctx = [&](int sidx, int tid, bool follow, int prev_tile, int prev_m0, int prev_n0) {
         TileCtx c;
         if (follow && !p.whole_band) {
             c.tile = prev_tile + 1;
@@ -190,7 +188,6 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
             segment(sidx, c.tile, c.gb, c.ge);
             tile_coords(c.tile, c.m0, c.n0);
         }
-        c.shift = rowshift[slot * 256 + tid];  // thread tid stages row tid
         // (N is a multiple of 128: the columns of a 32-column tile are inside or outside together; a thread beyond N
         // fetches the last tile's codes instead and converts them with scale zero)
         c.col_ok = c.n0 + tid < p.N;
@@ -226,10 +223,9 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
     // instruction (step w / 2, half w % 2); a wave's 64 threads write 64 consecutive 16-byte slots per word.
     // `which`: 0, 1 the two words of the row, 2, 3 those of the column.
     auto group_scales = [&](const TileCtx &c, const Raw &r, int ks, half2_t &sa2, half2_t &sb2) {
-        // e4m3 -> fp16 with the row's shift, without branches (a branch would end the scheduling region in which the
-        // conversions are interleaved with the matrix instructions)
-        const uint32_t e8 = (r.as >> (8 * ks)) & 0x7Fu, ex = e8 >> 3;
-        const _Float16 sa = (_Float16)ldexpf((float)((e8 & 7u) | (ex ? 8u : 0u)), (int)(ex ? ex : 1u) - 10 + c.shift);
+        // (the hardware conversion of a pair of e4m3 scales to fp16, exact)
+        const half2_t pair = ks >= 2 ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(r.as, 1.0f, true) : __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(r.as, 1.0f, false);
+        const _Float16 sa = pair[ks & 1];
         const uint32_t hb = c.col_ok ? (r.bs[ks >> 1] >> (16 * (ks & 1))) & 0xFFFFu : 0u;
         sa2 = half2_t{sa, sa};
         sb2 = as_half2(hb | (hb << 16));
@@ -343,45 +339,10 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
         }
     };
 
-  for (int batch0 = 0; batch0 < nseg; batch0 += MAX_BATCH) {
-    const int nbatch = nseg - batch0 < MAX_BATCH ? nseg - batch0 : MAX_BATCH;
-    {
-    int tid_p = threadIdx.x;  // opaque copy: nothing derived from it is kept in registers beyond this block
-    asm volatile("" : "+v"(tid_p));
-    const int tid = tid_p;
-    // ---- largest activation scale of every row of the batch's tiles -> power-of-two shift that
-    //      moves it into [2^10, 2^11)
-    __syncthreads();  // the previous batch is done with the table
-    {
-        // four e4m3 scales per (row, 64-group) packed in one word; e4m3 patterns of
-        // non-negative values order like unsigned bytes
-        for (int t = 0; t < nbatch; t++) {
-            int m0, n0;
-            int tile_t, gb_t, ge_t;
-            segment(batch0 + t, tile_t, gb_t, ge_t);
-            tile_coords(tile_t, m0, n0);
-            const uint32_t *sp = (const uint32_t *)p.ascales + m0 + tid;
-            uint32_t mx = 0;
-            for (int g0 = 0; g0 < kgroups; g0 += 8) {  // eight requests in flight (a maximum does not mind seeing the last group again)
-                uint32_t v[8];
-#pragma unroll
-                for (int u = 0; u < 8; u++) v[u] = sp[(size_t)(g0 + u < kgroups ? g0 + u : kgroups - 1) * p.M_pad];
-#pragma unroll
-                for (int u = 0; u < 8; u++)
-                    mx = max(max(mx, v[u] & 0x7Fu), max((v[u] >> 8) & 0x7Fu, max((v[u] >> 16) & 0x7Fu, (v[u] >> 24) & 0x7Fu)));
-            }
-            int ex = 0;
-            if (mx) frexpf(e4m3_to_f32(mx), &ex);  // value in [2^(ex-1), 2^ex)
-            rowshift[t * 256 + tid] = mx == 0 ? 0 : NORM_TARGET_EXP - (ex - 1);
-        }
-    }
-    }
-    __syncthreads();
-
-    TileCtx cur = make_ctx(batch0, 0, threadIdx.x, false, 0, 0, 0);
-
-   for (int ti = 0; ti < nbatch; ti++) {
-    const bool have_next = ti + 1 < nbatch;
+  if (nseg == 0) return;
+  TileCtx cur = make_ctx(0, threadIdx.x, false, 0, 0, 0);
+  for (int ti = 0; ti < nseg; ti++) {
+    const bool have_next = ti + 1 < nseg;
     refresh_thread_coordinates();
 #pragma unroll
     for (int i = 0; i < 4; i++)
@@ -427,7 +388,6 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
     const int tid = tid_e, lane = tid_e & 63, wave = __builtin_amdgcn_readfirstlane(tid_e >> 6);
     const int wm = wave >> 1, wn = wave & 1, r32 = lane & 31, h = lane >> 5;
     const int m0 = cur.m0, n0 = cur.n0, tile_e = cur.tile;
-    const int *tile_shift = rowshift + ti * 256;
 
     // ---- a tile shared with other workgroups ---------------------------------------------------
     // Every party holds the sum over its part of K.  Whoever finishes last adds all parties' sums in ascending order
@@ -501,10 +461,9 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
     }
     // Low-rank up projection (lora.cuh:110-241): out += bf16(lora_act * scale) @ up^T on the matrix cores.
     // The projection is added to the accumulators BEFORE they are scaled.  The accumulators are in
-    // normalised units (out = acc * rn[row] * cf[col] + bias), so the operands are divided by rn and cf
-    // first; the matrix cores then update the accumulators in place and the operands are dead before the
-    // output pass starts.  rn is a power of two (the division only changes exponents); cf
-    // (column normalisation x alpha x wcscales) is an arbitrary number, so up / cf is passed as the sum of
+    // normalised units (out = acc * cf[col] + bias), so the second operand is divided by cf first; the
+    // matrix cores then update the accumulators in place and the operands are dead before the output pass
+    // starts.  cf (column normalisation x alpha x wcscales) is an arbitrary number, so up / cf is passed as the sum of
     // two bf16 numbers (the rounded quotient and the rounded remainder: relative error 2^-17, below the
     // rounding noise of the main loop) in two matrix-core steps; wcscales must not be zero.
     const int nsteps = p.R_up / 16;
@@ -517,7 +476,7 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
                 const int s1 = two ? s0 + 1 : s0;
                 float4_t ra[4][2][2];
                 u32x4_t rb[4][2];
-                float rcf[4], lsr[4];
+                float rcf[4];
 #pragma unroll
                 for (int t = 0; t < 4; t++) {
                     const float4_t *ap = (const float4_t *)(p.lora_act + (size_t)(wrow0 + t * 32 + r32) * p.R_up + 8 * h);
@@ -531,7 +490,6 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
                     float cf = ok ? p.colnorm[n] * p.alpha : 1.f;
                     if (ok && p.wcscales) cf *= bf16_bits_to_f32(p.wcscales[n]);
                     rcf[t] = ok ? __fdiv_rn(1.0f, cf) : 0.f;
-                    lsr[t] = ldexpf(1.0f, tile_shift[wm * 128 + t * 32 + r32]);
                 }
 #pragma unroll
                 for (int k = 0; k < 2; k++) {
@@ -540,13 +498,12 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
                     bf16x8_t la[4], lb[4], lb_rem[4];
 #pragma unroll
                     for (int t = 0; t < 4; t++) {
-                        const float f = ls * lsr[t];
                         const float4_t v0 = ra[t][k][0], v1 = ra[t][k][1];
                         u32x4_t w;
-                        w[0] = pack_bf16x2(v0[0] * f, v0[1] * f);
-                        w[1] = pack_bf16x2(v0[2] * f, v0[3] * f);
-                        w[2] = pack_bf16x2(v1[0] * f, v1[1] * f);
-                        w[3] = pack_bf16x2(v1[2] * f, v1[3] * f);
+                        w[0] = pack_bf16x2(v0[0] * ls, v0[1] * ls);
+                        w[1] = pack_bf16x2(v0[2] * ls, v0[3] * ls);
+                        w[2] = pack_bf16x2(v1[0] * ls, v1[1] * ls);
+                        w[3] = pack_bf16x2(v1[2] * ls, v1[3] * ls);
                         la[t] = __builtin_bit_cast(bf16x8_t, w);
                         u32x4_t bw = rb[t][k], br = u32x4_t{0, 0, 0, 0};
 #pragma unroll
@@ -592,8 +549,6 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
     auto slab_epilogue = [&](auto MT, auto COMBINE_T) {
         constexpr int mt = decltype(MT)::value;
         constexpr bool COMBINE = decltype(COMBINE_T)::value;  // a tile shared with a neighbour: add its partial sums
-        // undo the power-of-two normalisation of the lane's row
-        const float rn = ldexpf(1.0f, -tile_shift[wm * 128 + mt * 32 + r32]);
         // (the accumulators are only read from here on: updating them in place makes the register
         // allocator copy and spill whole tuples)
         float4_t other[16];  // COMBINE: the parties' sums of this slab, added in ascending order of the workgroups
@@ -637,10 +592,10 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
                 if (COMBINE) {
                     const float4_t o = other[nt * 4 + q];
 #pragma unroll
-                    for (int i = 0; i < 4; i++) v[nt][4 * q + i] = __builtin_fmaf(o[i] * rn, cf[i], bs[i]);
+                    for (int i = 0; i < 4; i++) v[nt][4 * q + i] = __builtin_fmaf(o[i], cf[i], bs[i]);
                 } else {
 #pragma unroll
-                    for (int i = 0; i < 4; i++) v[nt][4 * q + i] = __builtin_fmaf(acc[mt][nt][4 * q + i] * rn, cf[i], bs[i]);
+                    for (int i = 0; i < 4; i++) v[nt][4 * q + i] = __builtin_fmaf(acc[mt][nt][4 * q + i], cf[i], bs[i]);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -835,10 +790,9 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
     }
     // (the next tile's context is worked out here, behind the epilogue: its four addresses would otherwise sit in
     // scratch memory while the epilogue needs the registers)
-    if (have_next) cur = make_ctx(batch0 + ti + 1, ti + 1, threadIdx.x, true, tile_e, m0, n0);
+    if (have_next) cur = make_ctx(ti + 1, threadIdx.x, true, tile_e, m0, n0);
     __syncthreads();
-   }  // tiles of the batch
-  }    // batches
+  }
 }
 
 

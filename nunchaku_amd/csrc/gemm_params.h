@@ -17,16 +17,13 @@ constexpr int BM = 256, BN = 256;
 constexpr int OP_BYTES = 8 * 4 * 2 * 32 * 16;    // one operand of one k-group
 constexpr int OPBUF_BYTES = 2 * OP_BYTES;          // activations + weights
 constexpr int OUT_LD = 136;                // bf16 elements per row of the store-staging slab (128 + pad)
-constexpr int MAX_BATCH = 8;                       // tiles whose row shifts are tabulated at once
 constexpr int SLAB_OFF = 0;                        // 4 waves x (32 rows x OUT_LD bf16): epilogue staging, in the operand buffers' place
 static_assert(4 * 32 * OUT_LD * 2 <= 2 * OPBUF_BYTES, "the epilogue's slabs reuse the operand buffers");
-constexpr int SHIFT_OFF = 2 * OPBUF_BYTES;                 // int [MAX_BATCH][256] row renormalisation shifts
-constexpr int TAB_OFF = SHIFT_OFF + MAX_BATCH * 256 * 4;   // 4 waves x float [2][128]: column factors and biases
+constexpr int TAB_OFF = 2 * OPBUF_BYTES;                   // 4 waves x float [2][128]: column factors and biases
 constexpr int FLAG_OFF = TAB_OFF + 4 * 1024;               // one word: a thread's reading of an arrival counter, for all
 constexpr int NORMW_OFF = FLAG_OFF + 16;                   // 4 waves x float [128]: RMS-norm weights of the wave's head
 constexpr int LDS_BYTES = NORMW_OFF + 4 * 512;
 static_assert(LDS_BYTES <= 160 * 1024, "one workgroup per compute unit");
-constexpr int NORM_TARGET_EXP = 10;
 
 
 // Separate q / k / v outputs of a fused QKV projection (EpiloguePackQKV, epilogues.cuh:427-550): fp16

@@ -44,6 +44,30 @@ def test_nvfp4_gemm_handmade_operands(dev, M, K, N, R):
     check_output(out, want)
 
 
+@pytest.mark.parametrize("M,K,N", [(256, 128, 256), (130, 256, 384)])
+def test_every_activation_scale_pattern_by_rows(dev, M, K, N):
+    """Row m carries the E4M3 pattern m % 127 in all its groups (zero, the subnormals, up to 448): code x scale must be exact
+    in the kernel's fp16 operands at both ends of that range.  Compared row by row: one bf16 rounding of the result, at
+    most 2^-8 of a value, and fp32 sums of K terms (2^-24 K of the row's norm at most)."""
+    from nunchaku_amd import packing
+    from nunchaku_amd.ops import svdq_gemm_w4a4
+
+    announce(f"nvfp4 gemm, a scale pattern per row, M={M} K={K} N={N}")
+    g = torch.Generator().manual_seed(K + N)
+    layer = synth.make_layer(N, K, 0, seed=K + N, fp4=True, bias=False)
+    M_pad = (M + 255) // 256 * 256
+    codes = torch.randint(0, 16, (M_pad, K), generator=g).to(torch.uint8)
+    scales = (torch.arange(M_pad) % 127).to(torch.uint8).expand(K // 16, M_pad).contiguous().view(torch.float8_e4m3fn)
+    t = make_module(layer, dev).native_tensors()
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev)
+    svdq_gemm_w4a4(act=packing.logical_to_act(codes, fp4=True).to(dev), wgt=t["qweight"], out=out,
+                   ascales=packing.logical_to_scales(scales, fp4=True).to(dev), wscales=t["wscales"], fp4=True, alpha=1.0, wcscales=t["wcscales"])
+    torch.cuda.synchronize()
+    want = olin.gemm_w4a4(quant.dequant_nvfp4(codes, scales), quant.dequant_nvfp4(layer.wq, layer.ws), alpha=1.0)[:M]
+    err = (out.float().cpu() - want).norm(dim=1)
+    assert (err <= (2.0**-8 + K * 2.0**-24) * want.norm(dim=1)).all(), (err / want.norm(dim=1)).max().item()
+
+
 def test_nvfp4_layer_end_to_end(dev):
     from nunchaku_amd import packing
 
