@@ -123,7 +123,8 @@ int svdq_quantize_w4a4_act_fuse_lora(const svdq_quantize_args *args, void *strea
  * The GELU is applied exactly when `qout` is given (launch_impl.cuh:282-309).
  *
  * INT4 runs on the fp6 matrix instruction (one workgroup per 128 x 256 output tile); NVFP4 runs on the
- * fp16 matrix instruction with dequantized operands (persistent workgroups, 256 x 256 tiles).
+ * fp16 matrix instruction with dequantized operands (persistent workgroups, 256 x 256 tiles).  Launches with few
+ * rows take a kernel with tiles of 32 or 64 rows x 128 columns of either precision (unless k_split is given).
  *
  * Workspace.  Most INT4 calls need none and touch no global state.  Four kinds of call keep a
  * workspace per (device, stream) pair, allocated with hipMalloc the first time the pair needs it:
@@ -168,7 +169,9 @@ typedef struct svdq_gemm_args {
     const void *next_lora_down;   /* native proj_down of the next layer ([N, R_down]) or NULL       */
     float *next_lora_act_out;     /* fp32 [M_pad, R_down]; fully written by the call                */
     int64_t M_pad, N, K;
-    int64_t M_out, N_out;   /* shape of `out` (M_out <= M_pad, N_out <= N)                          */
+    int64_t M_out, N_out;   /* shape of `out` (M_out <= M_pad, N_out <= N).  Without `out`: the rows of
+                               qout / oscales / next_lora_act_out the caller will read (rounded up to
+                               whole tiles; what the others hold is unspecified), 0 for all M_pad     */
     int64_t R_up, R_down;
     float alpha;            /* per-tensor scale (NVFP4 wtscale; the reference asserts 1 for INT4,
                                launch_impl.cuh:107, this library applies whatever is given)          */

@@ -7,6 +7,12 @@ using namespace svdq;
 namespace svdq {
 int launch_gemm_fp4_v4(const GemmParams &p, int nwg, hipStream_t stream);
 int launch_gemm_fp4_v5(const GemmParams &p, int nwg, hipStream_t stream);
+namespace direct {
+int launch_int4_plain(const GemmParams &p, int shape, hipStream_t stream);
+int launch_int4_next(const GemmParams &p, int shape, hipStream_t stream);
+int launch_fp4_plain(const GemmParams &p, int shape, hipStream_t stream);
+int launch_fp4_next(const GemmParams &p, int shape, hipStream_t stream);
+}  // namespace direct
 namespace g6 {
 int launch_plain(const Params &p, int nwg, hipStream_t stream);
 int launch_next(const Params &p, int nwg, hipStream_t stream);
@@ -219,6 +225,26 @@ bool acquire_workspace(bool noalloc, int dev, hipStream_t st, size_t zero_bytes,
     return true;
 }
 
+// The small kernels behind a GEMM that left shares in the workspace: the shares of the next layer's low-rank projection
+// (one per column block) and the linear-attention sums (one per vk_block rows), each added in ascending order.
+template <typename P>
+int add_shares(const P &p, int nshares, int vk_block, hipStream_t st) {
+    if (p.next_down) {
+        const int quads = p.M_pad * p.R_down / 4;
+        SVDQ_LAUNCH(reduce_shares_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, (const float4_t *)p.next_lora_part,
+                    p.next_lora_out, nshares, p.M_pad, p.R_down);
+        const int rc = check_launch("gemm_w4a4 (low-rank shares)");
+        if (rc != SVDQ_OK) return rc;
+    }
+    if (p.vk) {
+        const int heads = p.N / 96, n = (p.M_pad / p.vk_rows) * heads * VK_HEAD_FLOATS;
+        SVDQ_LAUNCH(reduce_vk_kernel, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, st, (const float *)p.vk_part, p.vk, p.M_pad / p.vk_rows,
+                    p.vk_rows / vk_block, heads);
+        return check_launch("gemm_w4a4 (linear-attention sums)");
+    }
+    return SVDQ_OK;
+}
+
 // Into how many parts along K the tiles of an INT4 launch are split when the caller leaves that to the library.
 // Launches with more tiles than compute units are not split: every part parks 128 KB of sums and the last one fetches
 // them all, which only pays while compute units would otherwise stand idle.  Below that, a model of the time in us,
@@ -228,8 +254,13 @@ bool acquire_workspace(bool noalloc, int dev, hipStream_t st, size_t zero_bytes,
 // again when compute units are shared.  Measured, whole / best split: 24 tiles at K = 3072 31.2 / 22.5 (4 parts; 3
 // parts 24.2), 72 tiles 31.3 / 27.3 (3), 96 tiles 31.8 / 31.0 (2; not split), 144 tiles 32.1 / 38.1 (not split);
 // K = 12288: 24 tiles 105.9 / 39.6 (6), 72 tiles 105.6 / 51.7 (3), 144 tiles 106.2 / 78.4 (3).
-int choose_kparts(int ntiles, int kgroups, int ncu) {
-    if (ntiles > ncu) return 1;
+// `time`: the model's time in us for the choice; beyond one tile per compute unit (288 tiles at K = 3072 45 us, 384 tiles
+// 52-56, 512 tiles 50, 1728 tiles 165) 0.83 us per k-group until two share every compute unit, then in proportion.
+int choose_kparts(int ntiles, int kgroups, int ncu, double *time) {
+    if (ntiles > ncu) {
+        *time = (0.83 * kgroups + 5.0) * (ntiles > 2 * ncu ? ntiles / (2.0 * ncu) : 1.0);
+        return 1;
+    }
     int best = 1;
     double best_t = 0.55 * kgroups + 4.4;
     for (int k : {2, 3, 4, 6, 8}) {
@@ -242,7 +273,56 @@ int choose_kparts(int ntiles, int kgroups, int ncu) {
             best_t = t;
         }
     }
+    *time = best_t;
     return best;
+}
+
+// (the kernels with the next-layer epilogue also carry the norm + rotary, SiLU and linear-attention epilogues)
+bool needs_next_epilogue(const svdq_gemm_args *a) {
+    return a->qout != nullptr || a->next_lora_down != nullptr || a->rotary_emb != nullptr || a->fuse_silu || a->out_vk != nullptr;
+}
+
+// The argument block of the NVFP4 kernel and of the few-rows kernels.
+void fill_params(const svdq_gemm_args *a, GemmParams &p) {
+    p.act = (const uint8_t *)a->act;
+    p.ascales = (const uint16_t *)a->ascales;
+    p.wgt = (const uint8_t *)a->wgt;
+    p.wscales = (const _Float16 *)a->wscales;
+    p.colnorm = a->colnorm;
+    p.bias = (const uint16_t *)a->bias;
+    p.wcscales = (const uint16_t *)a->wcscales;
+    p.lora_act = a->lora_act_in;
+    p.lora_up = (const uint16_t *)a->lora_up;
+    p.out = (uint16_t *)a->out;
+    p.qout = (uint8_t *)a->qout;
+    p.oscales = a->oscales;
+    p.next_smooth_rcp = a->next_smooth_rcp;
+    p.next_down = (const bf16x8_t *)a->next_lora_down;
+    p.next_lora_out = a->next_lora_act_out;
+    p.R_down = (int)a->R_down;
+    p.M_pad = (int)a->M_pad; p.N = (int)a->N; p.K = (int)a->K;
+    p.M_out = (int)a->M_out; p.N_out = (int)a->N_out; p.R_up = (int)a->R_up;
+    p.alpha = a->alpha;
+    for (int i = 0; i < MAX_RANK / 16; i++) p.lora_scales[i] = (a->lora_scales && i < (a->R_up + 15) / 16) ? a->lora_scales[i] : 1.0f;
+    p.norm_q = (const uint16_t *)a->norm_q;
+    p.norm_k = (const uint16_t *)a->norm_k;
+    p.rotary = a->rotary_emb;
+    p.rot_rows = (int)a->rot_rows;
+    p.rope_cols = (int)(a->N / 3 * 2);
+    p.norm_eps = a->norm_eps;
+    p.qkv.q = (uint16_t *)a->out_q; p.qkv.k = (uint16_t *)a->out_k; p.qkv.v = (uint16_t *)a->out_v;
+    p.qkv.stride_q = a->qkv_head_stride[0]; p.qkv.stride_k = a->qkv_head_stride[1]; p.qkv.stride_v = a->qkv_head_stride[2];
+    p.qkv.attn_tokens = (int)a->attn_tokens; p.qkv.rows = (int)a->qkv_rows;
+    p.silu = a->fuse_silu != 0;
+    p.gelu = a->qout != nullptr;
+    p.vk = a->out_vk;
+    p.vk_rows = (int)a->vk_rows;
+    p.vk_part = nullptr;
+    p.next_lora_part = nullptr;
+    p.partials = nullptr;
+    p.counters = nullptr;
+    p.whole_band = 0;
+    p.row_blocks = 0;
 }
 
 // ---- INT4: fp6 matrix instruction on the bare codes (gemm6_kernel.h) --------------------------------
@@ -286,11 +366,12 @@ int gemm_int4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool no
     // One workgroup per 128 x 256 output tile (or per part of one split along K), two resident per compute unit.
     const int mblocks = p.M_pad / g6::BM, nblocks = (p.N + g6::BN - 1) / g6::BN;
     const int ntiles = mblocks * nblocks, kgroups = p.K / 64;
-    const int kparts = a->k_split > 0 ? (int)(a->k_split < kgroups ? a->k_split : kgroups) : choose_kparts(ntiles, kgroups, ncu);
+    double model_time;
+    const int kparts = a->k_split > 0 ? (int)(a->k_split < kgroups ? a->k_split : kgroups) : choose_kparts(ntiles, kgroups, ncu, &model_time);
     p.kparts = kparts;
     // bands of about ten row blocks, all of the same height where the count allows it
     p.band = (mblocks + (mblocks + 9) / 10 - 1) / ((mblocks + 9) / 10);
-    const bool next = a->qout != nullptr || a->next_lora_down != nullptr || a->rotary_emb != nullptr || a->fuse_silu || a->out_vk != nullptr;
+    const bool next = needs_next_epilogue(a);
     const size_t cnt_bytes = (size_t)ntiles * 4;
     const size_t part_bytes = kparts > 1 ? (size_t)ntiles * kparts * g6::BM * g6::BN * 4 : 0;
     const size_t share_bytes = p.next_down ? (size_t)nblocks * p.M_pad * p.R_down * 4 : 0;  // every column block's share of the next projection
@@ -307,20 +388,7 @@ int gemm_int4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool no
     p.next_lora_part = (float *)(w.scratch + part_bytes);
     p.vk_part = (float *)(w.scratch + part_bytes + share_bytes);
     int rc = next ? g6::launch_next(p, ntiles * kparts, st) : g6::launch_plain(p, ntiles * kparts, st);
-    if (rc == SVDQ_OK && p.next_down) {
-        // the column blocks' shares of the next layer's low-rank projection, added in ascending order
-        const int quads = p.M_pad * p.R_down / 4;
-        SVDQ_LAUNCH(reduce_shares_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, (const float4_t *)p.next_lora_part,
-                           p.next_lora_out, nblocks, p.M_pad, p.R_down);
-        rc = check_launch("gemm_w4a4 (low-rank shares)");
-    }
-    if (rc == SVDQ_OK && p.vk) {
-        // the row blocks' linear-attention sums, added per batch entry in ascending order of the rows
-        const int heads = p.N / 96, n = (p.M_pad / p.vk_rows) * heads * VK_HEAD_FLOATS;
-        SVDQ_LAUNCH(reduce_vk_kernel, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, st, (const float *)p.vk_part, p.vk, p.M_pad / p.vk_rows,
-                           p.vk_rows / g6::BM, heads);
-        rc = check_launch("gemm_w4a4 (linear-attention sums)");
-    }
+    if (rc == SVDQ_OK) rc = add_shares(p, nblocks, g6::BM, st);
     if (rc != SVDQ_OK && w.owner) w.owner->dirty = true;
     return rc;
 }
@@ -328,37 +396,7 @@ int gemm_int4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool no
 // ---- NVFP4: fp16 matrix instruction on dequantized operands (gemm_kernel.h) -------------------------
 int gemm_fp4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool noalloc) {
     GemmParams p;
-    p.act = (const uint8_t *)a->act;
-    p.ascales = (const uint16_t *)a->ascales;
-    p.wgt = (const uint8_t *)a->wgt;
-    p.wscales = (const _Float16 *)a->wscales;
-    p.colnorm = a->colnorm;
-    p.bias = (const uint16_t *)a->bias;
-    p.wcscales = (const uint16_t *)a->wcscales;
-    p.lora_act = a->lora_act_in;
-    p.lora_up = (const uint16_t *)a->lora_up;
-    p.out = (uint16_t *)a->out;
-    p.qout = (uint8_t *)a->qout;
-    p.oscales = a->oscales;
-    p.next_smooth_rcp = a->next_smooth_rcp;
-    p.next_down = (const bf16x8_t *)a->next_lora_down;
-    p.next_lora_out = a->next_lora_act_out;
-    p.R_down = (int)a->R_down;
-    p.M_pad = (int)a->M_pad; p.N = (int)a->N; p.K = (int)a->K;
-    p.M_out = (int)a->M_out; p.N_out = (int)a->N_out; p.R_up = (int)a->R_up;
-    p.alpha = a->alpha;
-    for (int i = 0; i < MAX_RANK / 16; i++) p.lora_scales[i] = (a->lora_scales && i < (a->R_up + 15) / 16) ? a->lora_scales[i] : 1.0f;
-    p.norm_q = (const uint16_t *)a->norm_q;
-    p.norm_k = (const uint16_t *)a->norm_k;
-    p.rotary = a->rotary_emb;
-    p.rot_rows = (int)a->rot_rows;
-    p.rope_cols = (int)(a->N / 3 * 2);
-    p.norm_eps = a->norm_eps;
-    p.qkv.q = (uint16_t *)a->out_q; p.qkv.k = (uint16_t *)a->out_k; p.qkv.v = (uint16_t *)a->out_v;
-    p.qkv.stride_q = a->qkv_head_stride[0]; p.qkv.stride_k = a->qkv_head_stride[1]; p.qkv.stride_v = a->qkv_head_stride[2];
-    p.qkv.attn_tokens = (int)a->attn_tokens; p.qkv.rows = (int)a->qkv_rows;
-    p.silu = a->fuse_silu != 0;
-    p.gelu = a->qout != nullptr;
+    fill_params(a, p);
 
     // persistent workgroups: one per compute unit, each walking over its share of the output tiles
     const int ntiles = (int)(a->M_pad / BM) * (int)((a->N + BN - 1) / BN);
@@ -400,14 +438,7 @@ int gemm_fp4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool noa
     }
     // the work is split evenly in units of two k-groups; unless the tile count is a multiple of the
     // workgroup count, some tiles are then shared by two or more workgroups and need the workspace
-    p.partials = nullptr;
-    p.counters = nullptr;
-    // (the kernels with the next-layer epilogue also carry the norm + rotary epilogue)
-    p.vk = a->out_vk;
-    p.vk_rows = (int)a->vk_rows;
-    p.vk_part = nullptr;
-    p.next_lora_part = nullptr;
-    const bool next = a->qout != nullptr || a->next_lora_down != nullptr || a->rotary_emb != nullptr || a->fuse_silu || a->out_vk != nullptr;
+    const bool next = needs_next_epilogue(a);
     const bool shared_tiles = !(nwg <= ntiles && ntiles % nwg == 0);
     p.whole_band = 0;
     if (!shared_tiles) {
@@ -436,19 +467,77 @@ int gemm_fp4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool noa
     p.next_lora_part = (float *)(w.scratch + part_bytes);
     p.vk_part = (float *)(w.scratch + part_bytes + share_bytes);
     int rc = next ? launch_gemm_fp4_v5(p, nwg, st) : launch_gemm_fp4_v4(p, nwg, st);
-    if (rc == SVDQ_OK && p.next_down) {
-        const int quads = p.M_pad * p.R_down / 4;
-        SVDQ_LAUNCH(reduce_shares_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, (const float4_t *)p.next_lora_part,
-                           p.next_lora_out, p.N / 128, p.M_pad, p.R_down);
-        rc = check_launch("gemm_w4a4 (low-rank shares)");
-    }
-    if (rc == SVDQ_OK && p.vk) {
-        const int heads = p.N / 96, n = (p.M_pad / p.vk_rows) * heads * VK_HEAD_FLOATS;
-        SVDQ_LAUNCH(reduce_vk_kernel, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, st, (const float *)p.vk_part, p.vk, p.M_pad / p.vk_rows,
-                           p.vk_rows / 32, heads);
-        rc = check_launch("gemm_w4a4 (linear-attention sums)");
-    }
+    if (rc == SVDQ_OK) rc = add_shares(p, p.N / 128, 32, st);
     if (rc != SVDQ_OK && w.owner) w.owner->dirty = true;
+    return rc;
+}
+
+// ---- few rows, either precision: small tiles, operands straight to registers (gemm_direct_kernel.h) ------
+// Rows the call has to work out: those of `out` where nothing else is written, those the caller names where `out` is not
+// given, all of them otherwise.
+int rows_needed(const svdq_gemm_args *a) {
+    if (a->out_q || a->out_vk || (a->out && (a->qout || a->next_lora_down)) || a->M_out == 0) return (int)a->M_pad;
+    return (int)a->M_out;
+}
+
+// Which of the two shapes of the few-rows kernel (0: neither) a launch takes.  Shape 1: tiles of 32 rows, four waves split
+// K.  Shape 2: tiles of 64 rows, two waves split K and two the columns: 23 % fewer operand bytes per product, from about
+// 400 tiles of 32 rows on.  Both are models of the time in us fitted to launches at K = 1024, 3072 and 12288 on 256 compute
+// units, linear in the number of tiles that the busiest compute unit works through and in the k-groups; they meet the
+// measurements within about 10 %.  Measured at K = 3072, large tiles (split along K where that pays) / shape 1 / shape 2:
+//   INT4   M = 256, N = 3072   22.8 /  9.6 / 12.3     NVFP4  59.9 / 11.2 / 15.4
+//          M = 505, N = 9216   33.6 / 33.7 / 30.4            64.0 / 39.2 / 38.1
+//          M = 1157, N = 3072  29.7 / 27.6 / 21.8            63.5 / 31.5 / 26.9
+//          M = 1024, N = 9216  45.0 / 57.4 / 48.4            70.3 / 69.8 / 61.7
+//          M = 1024, N = 12288                               74.4 / 90.3 / 76.2
+//   K = 12288, N = 3072: M = 256  42.1 / 24.8 / -           113.6 / 29.5 / -
+//          M = 505             44.7 / 44.6 / 34.9           115.6 / 51.2 / 46.2
+//          M = 1157            66.6 / 86.6 / 65.6           126.3 / 102.3 / 90.6
+int choose_direct(const svdq_gemm_args *a, int ncu) {
+    if (a->k_split > 0) return 0;  // (the caller asks for the tiles that k_split is about)
+    if (((uintptr_t)a->bias | (uintptr_t)a->wcscales | (uintptr_t)a->oscales) % 8 || (uintptr_t)a->colnorm % 16) return 0;  // (read four columns at a time)
+    const int rows = rows_needed(a), kg = (int)(a->K / 64);
+    const long long ncols = a->N / 128;
+    const double c1 = (double)((((rows + 31) / 32) * ncols + ncu - 1) / ncu), c2 = (double)((((rows + 63) / 64) * ncols + ncu - 1) / ncu);
+    double t_large, t1, t2;
+    if (a->fp4) {
+        // (one 256 x 256 tile per compute unit: 62 us at K = 3072 with 48 tiles, 78 with 216; 32 at K = 1024)
+        const double tiles = (double)(a->M_pad / BM) * ((a->N + BN - 1) / BN) / ncu;
+        t_large = ((1.0 + 0.3 * (tiles < 1.0 ? tiles : 1.0)) * kg + 14.0) * (tiles > 1.0 ? tiles : 1.0);
+        t1 = 4.3 + c1 * (1.1 + 0.127 * kg);
+        t2 = 3.0 + c2 * (2.1 + 0.214 * kg);
+    } else {
+        choose_kparts((int)(a->M_pad / g6::BM) * (int)((a->N + g6::BN - 1) / g6::BN), kg, ncu, &t_large);
+        t_large = 0.96 * t_large + 2.8;  // (144 tiles, one per compute unit: 15.6 us at K = 1024, 33 at K = 3072, 105 at K = 12288)
+        t1 = 3.5 + c1 * (1.1 + 0.106 * kg);
+        t2 = 3.3 + c2 * (1.6 + 0.158 * kg);
+    }
+    if (t1 < t2) return t1 < t_large ? 1 : 0;
+    return t2 < t_large ? 2 : 0;
+}
+
+int gemm_direct(const svdq_gemm_args *a, int shape, hipStream_t st, int dev, bool noalloc) {
+    GemmParams p;
+    fill_params(a, p);
+    const int rows = rows_needed(a);
+    p.row_blocks = (rows + 32 * shape - 1) / (32 * shape);  // (shape s: tiles of 32 s rows)
+    const bool next = needs_next_epilogue(a);
+    auto launch = [&]() {
+        if (a->fp4) return next ? direct::launch_fp4_next(p, shape, st) : direct::launch_fp4_plain(p, shape, st);
+        return next ? direct::launch_int4_next(p, shape, st) : direct::launch_int4_plain(p, shape, st);
+    };
+    // every 128-column chunk's share of the next layer's low-rank projection, every 32-row block's linear-attention sums
+    const size_t share_bytes = p.next_down ? (size_t)(p.N / 128) * p.M_pad * p.R_down * 4 : 0;
+    const size_t vk_bytes = p.vk ? (size_t)(p.M_pad / 32) * (p.N / 96) * VK_HEAD_FLOATS * 4 : 0;
+    if (!share_bytes && !vk_bytes) return launch();
+    std::unique_lock<std::mutex> lock(g_ws_mutex, std::defer_lock);
+    if (!noalloc) lock.lock();
+    WorkspaceView w;
+    if (!acquire_workspace(noalloc, dev, st, 0, share_bytes + vk_bytes, &w)) return noalloc && share_bytes + vk_bytes > NOALLOC_SCRATCH_BYTES ? SVDQ_EUNSUPPORTED : SVDQ_ELAUNCH;
+    p.next_lora_part = (float *)w.scratch;
+    p.vk_part = (float *)(w.scratch + share_bytes);
+    int rc = launch();
+    if (rc == SVDQ_OK) rc = add_shares(p, p.N / 128, 32, st);
     return rc;
 }
 }  // namespace
@@ -466,6 +555,7 @@ int gemm_entry(const svdq_gemm_args *a, void *stream, bool noalloc) {
     SVDQ_REQUIRE(a->R_up >= 0 && a->R_up % 16 == 0 && a->R_up <= MAX_RANK, "gemm: R_up (%lld) must be a multiple of 16, at most %d", (long long)a->R_up, MAX_RANK);
     SVDQ_REQUIRE((a->R_up > 0) == (a->lora_up != nullptr), "gemm: R_up and lora_up disagree");
     SVDQ_REQUIRE(a->k_split >= 0, "gemm: k_split must not be negative");
+    SVDQ_REQUIRE(a->M_out >= 0 && a->M_out <= a->M_pad, "gemm: M_out (%lld) does not fit M_pad (%lld)", (long long)a->M_out, (long long)a->M_pad);
     if (a->out) {
         SVDQ_REQUIRE(a->M_out > 0 && a->M_out <= a->M_pad && a->M_pad - a->M_out < 256, "gemm: M_out (%lld) does not fit M_pad (%lld)",
                      (long long)a->M_out, (long long)a->M_pad);
@@ -532,6 +622,8 @@ int gemm_entry(const svdq_gemm_args *a, void *stream, bool noalloc) {
     if (hipGetDevice(&dev) != hipSuccess) return fail(SVDQ_ELAUNCH, "gemm: cannot identify the current device");
     const int ncu = compute_units(dev);
     if (ncu <= 0) return fail(SVDQ_ELAUNCH, "gemm: cannot query the number of compute units");
+    const int shape = choose_direct(a, ncu);
+    if (shape) return gemm_direct(a, shape, (hipStream_t)stream, dev, noalloc);
     return a->fp4 ? gemm_fp4(a, (hipStream_t)stream, dev, ncu, noalloc) : gemm_int4(a, (hipStream_t)stream, dev, ncu, noalloc);
 }
 }  // namespace

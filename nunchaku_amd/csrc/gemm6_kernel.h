@@ -37,52 +37,12 @@
 
 #include <type_traits>
 
+#include "gemm_math.h"
 #include "gemm_params.h"
 #include "svdq_quant.h"
 
 namespace svdq {
 namespace g6 {
-
-typedef int v8i_t __attribute__((ext_vector_type(8)));
-typedef int v4i_t __attribute__((ext_vector_type(4)));
-typedef int v2i_t __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
-
-struct Frag {
-    u32x4_t lo;  // bits [0, 128) of the lane's 192-bit code string
-    u32x2_t hi;  // bits [128, 192)
-};
-
-// inner sums of one 32 x 32 tile over one k-group (elements 6 and 7 of the operand vectors are not
-// read by the fp6 form of the instruction)
-__device__ inline float16_t mfma_codes(const Frag &w, const Frag &x) {
-    const v8i_t a = __builtin_shufflevector(__builtin_shufflevector(__builtin_bit_cast(v4i_t, w.lo), __builtin_bit_cast(v4i_t, w.lo), 0, 1, 2, 3, -1, -1, -1, -1),
-                                            __builtin_shufflevector(__builtin_bit_cast(v2i_t, w.hi), __builtin_bit_cast(v2i_t, w.hi), 0, 1, -1, -1, -1, -1, -1, -1),
-                                            0, 1, 2, 3, 8, 9, -1, -1);
-    const v8i_t b = __builtin_shufflevector(__builtin_shufflevector(__builtin_bit_cast(v4i_t, x.lo), __builtin_bit_cast(v4i_t, x.lo), 0, 1, 2, 3, -1, -1, -1, -1),
-                                            __builtin_shufflevector(__builtin_bit_cast(v2i_t, x.hi), __builtin_bit_cast(v2i_t, x.hi), 0, 1, -1, -1, -1, -1, -1, -1),
-                                            0, 1, 2, 3, 8, 9, -1, -1);
-    const float16_t z = {};
-    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, z, 2, 2, 0, 0, 0, 0);  // E2M3 x E2M3, no block scales
-}
-
-// factor tile 64 ws[n] * as[m]: the weight operand is {64 s, 0, 0, 0} in both half-waves (k slots 0-3 and
-// 4-7), the activation operand carries its scale in k slot 0 and zero in k slot 4, anything finite
-// elsewhere
-__device__ inline float16_t mfma_factor(u32x2_t ws, uint32_t as) {
-    const float16_t z = {};
-    return __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(__builtin_bit_cast(bf16x4_t, ws), __builtin_bit_cast(bf16x4_t, u32x2_t{as, 0u}), z, 0, 0, 0);
-}
-
-__device__ inline float gelu_tanh(float x) {
-    // x * (0.5 + 0.5 * tanh(u)), u = 0.79788456 * (x + 0.044715 x^3)   (epilogues.cuh:22-44)
-    // With tanh(u) = 1 - 2 / (exp(2u) + 1) this is x - x / (exp(2u) + 1): one hardware exp2 and one hardware
-    // reciprocal (1 ulp each), safe at both ends (exp2 -> inf gives x, exp2 -> 0 gives 0).
-    constexpr float C1 = 2.0f * 0.79788456f * 1.4426950408889634f, C2 = C1 * 0.044715f;  // 2u * log2(e) = x (C1 + C2 x^2)
-    const float w = x * __builtin_fmaf(C2, x * x, C1);
-    const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(w) + 1.0f);
-    return __builtin_fmaf(-x, r, x);
-}
 
 // Partial sums of a tile split along K travel through memory with system-scope accesses (sc0 sc1): they
 // bypass the caches that are not coherent between the XCDs, so no cache write-back or invalidation is

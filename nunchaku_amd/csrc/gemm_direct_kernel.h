@@ -1,0 +1,466 @@
+// Operator 2 for few rows, INT4 and NVFP4: the same product and epilogues as gemm6_kernel.h and gemm_kernel.h, with
+// small output tiles whose operands go from memory straight to the registers of the wave that multiplies them.
+//
+// The kernels with 128 x 256 and 256 x 256 tiles need thousands of rows to occupy the chip: with a few hundred, a
+// layer of N = 3072 is 24 or 12 such tiles, each walking K alone on its compute unit.  Here a workgroup of four waves owns
+// a tile of 32 MT rows x 128 columns; its waves split the columns WN ways and take the k-groups g = part, part + KP, ...
+// of their part of K in turn, and the parts' sums meet in LDS at the end.  An operand fragment is contiguous in memory in
+// the lanes' order (svdq_common.h), so a wave fetches it with one or two wide loads, DEPTH of its k-groups ahead, and
+// neither LDS nor barriers appear in the main loop.
+// Bound by the bytes the L2s hand out: 2.15 KB per 32 x 32 tile and k-group with one row block and four column tiles per
+// wave, 1.65 KB with two of each; at 192 workgroups (M = 256, N = 3072) they arrive at 82 GB/s per compute unit, 15.7 TB/s
+// in all.  M = 256, K = N = 3072: 22.8 -> 9.6 us (INT4; 4.7 us of it do not depend on K), 59.9 -> 11.2 us (NVFP4).
+//
+// INT4: one fp6 matrix instruction on the codes, one factor instruction and 16 multiply-adds per 32 x 32 tile and
+// k-group (gemm6_kernel.h).  NVFP4: both operands are dequantized to fp16 in registers by the wave that uses them
+// (gemm_kernel.h dequantizes once per workgroup; here every wave has its own k-groups, so that is the same).
+//
+// The epilogue is shared out by columns: wave w of four adds up the parts' sums of the 32 columns 32 w ... of the tile
+// in ascending order, projects the low-rank branch onto them and applies bias, norm, rotation and activation; the
+// bf16 tile meets in LDS again and all waves store it, project and quantize it for the next layer.
+#pragma once
+
+#include <type_traits>
+#include <utility>
+
+#include "gemm_math.h"
+#include "gemm_params.h"
+#include "svdq_quant.h"
+
+namespace svdq {
+namespace direct {
+
+template <bool FP4, int MT, int NT>
+struct Stage;  // one k-group of a wave's operands on their way from memory
+template <int MT, int NT>
+struct Stage<false, MT, NT> {
+    v6i_t w[NT], x[MT];
+    uint32_t ws[NT], as[MT];
+};
+template <int MT, int NT>
+struct Stage<true, MT, NT> {
+    u32x4_t w[NT], x[MT];
+    uint32_t ws[NT], as[MT];
+};
+
+template <int... I, typename F>
+__device__ inline void each(std::integer_sequence<int, I...>, F &&f) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+
+constexpr int SLAB_BYTES = 32 * OUT_LD * 2;
+// LDS: the waves' sums of 32 rows x 128 columns, [KP][4 column tiles][4 quads][64 lanes] x float4; behind them the sums of
+// squares of the RMS norm, [MT][4][32] floats.  The bf16 slabs take the place of the sums.
+template <int MT, int KP>
+constexpr int lds_bytes() {
+    return KP * 16384 + MT * 512;
+}
+
+template <bool FP4, int MT, int WN, int KP, int DEPTH, bool NEXT>
+__global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams p) {
+    constexpr int NT = 4 / WN;  // 32-column tiles of a wave
+    constexpr int WAVES = WN * KP;
+    static_assert(WAVES == 4, "the epilogue gives each wave one column tile");
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r32 = lane & 31, h = lane >> 5;
+    const int kgroups = p.K / 64;
+    const int kpart = wave / WN, cw = wave % WN;
+
+    // Workgroups go to the XCDs round robin (blockIdx % 8): each XCD gets one contiguous run of numbers, down the rows
+    // first, so that the row blocks of a weight column meet in one L2 and every XCD streams its own share of the weights.
+    const int total = (int)gridDim.x, xcd = (int)blockIdx.x % 8, extra = total % 8;
+    const int v = xcd * (total / 8) + (xcd < extra ? xcd : extra) + (int)blockIdx.x / 8;
+    const int nb = v / p.row_blocks, mb = v - nb * p.row_blocks;
+    const int n0 = nb * 128, f0 = mb * MT;  // first column; first 32-row block
+
+    // ---- operands ----------------------------------------------------------------------------------
+    // (DEPTH + 1 register sets, indexed by compile-time constants.  The lambdas below reach them through their captures: taken
+    // by reference as an argument, a set is known to be readable as a whole, the compiler reads vectors of six words
+    // eight wide from it, and then cannot keep it in registers)
+    Stage<FP4, MT, NT> sets[DEPTH + 1];
+    // The k-group requested next and the wave-uniform addresses of its operands, which advance by constants; behind the
+    // last group they stay where they are (such a request is never used).
+    int g_load = kpart < kgroups ? kpart : kgroups - 1;
+    const uint8_t *wp, *sp, *xp[MT];
+    const uint16_t *ap;
+    const uint32_t w_step = KP * (FP4 ? TILE_BYTES : 8 * FRAG_BYTES), x_step = KP * (FP4 ? TILE_BYTES : 4 * FRAG_BYTES);
+    const uint32_t s_step = FP4 ? (uint32_t)p.N * (8 * KP) : 2048 * KP, a_step = (uint32_t)p.M_pad * (FP4 ? 2 * KP : KP);
+    if constexpr (!FP4) {
+        wp = p.wgt + ((size_t)(nb >> 1) * kgroups + g_load) * (8 * FRAG_BYTES) + ((nb & 1) * 4 + cw * NT) * FRAG_BYTES;
+        sp = (const uint8_t *)p.wscales + ((size_t)(nb >> 1) * kgroups + g_load) * 2048 + (nb & 1) * 1024 + cw * (NT * 256);
+        each(std::make_integer_sequence<int, MT>{}, [&](auto I) {
+            constexpr int mt = decltype(I)::value;
+            xp[mt] = p.act + ((size_t)((f0 + mt) >> 2) * kgroups + g_load) * (4 * FRAG_BYTES) + ((f0 + mt) & 3) * FRAG_BYTES;
+        });
+        ap = p.ascales + (size_t)g_load * p.M_pad + f0 * 32;
+    } else {
+        wp = p.wgt + ((size_t)(nb * 4 + cw * NT) * kgroups + g_load) * TILE_BYTES;
+        sp = (const uint8_t *)p.wscales + ((size_t)g_load * p.N + n0 + cw * (NT * 32)) * 8;
+        each(std::make_integer_sequence<int, MT>{}, [&](auto I) {
+            constexpr int mt = decltype(I)::value;
+            xp[mt] = p.act + ((size_t)(f0 + mt) * kgroups + g_load) * TILE_BYTES;
+        });
+        ap = p.ascales + ((size_t)g_load * p.M_pad + f0 * 32) * 2;
+    }
+    const uint32_t off16 = (uint32_t)lane * 16u, off8 = 1024u + (uint32_t)lane * 8u, off_ws = (uint32_t)r32 * 8u + (FP4 ? (uint32_t)h * 4u : 0u);
+    const uint32_t off_as = FP4 ? (uint32_t)r32 * 4u + (uint32_t)h * 2u : (uint32_t)r32 * 2u, off_fp4 = (uint32_t)r32 * 32u + (uint32_t)h * 16u;
+    const uint32_t tile_stride = (uint32_t)kgroups * TILE_BYTES;  // NVFP4: from one 32-column tile to the next
+    auto load = [&](auto S) {
+        auto &st = sets[decltype(S)::value];
+        each(std::make_integer_sequence<int, MT>{}, [&](auto I) {
+            constexpr int mt = decltype(I)::value;
+            if constexpr (!FP4) st.x[mt] = codes6(*(const u32x4_t *)(xp[mt] + off16), *(const u32x2_t *)(xp[mt] + off8));
+            else st.x[mt] = *(const u32x4_t *)(xp[mt] + off_fp4);
+            st.as[mt] = *(const uint16_t *)((const uint8_t *)ap + mt * (FP4 ? 128 : 64) + off_as);
+        });
+        each(std::make_integer_sequence<int, NT>{}, [&](auto I) {
+            constexpr int nt = decltype(I)::value;
+            if constexpr (!FP4) st.w[nt] = codes6(*(const u32x4_t *)(wp + nt * FRAG_BYTES + off16), *(const u32x2_t *)(wp + nt * FRAG_BYTES + off8));
+            else st.w[nt] = *(const u32x4_t *)(wp + nt * tile_stride + off_fp4);
+            st.ws[nt] = *(const uint32_t *)(sp + nt * 256 + off_ws);
+        });
+        const bool more = g_load + KP < kgroups;
+        g_load += more ? KP : 0;
+        wp += more ? w_step : 0u;
+        sp += more ? s_step : 0u;
+        ap += more ? a_step : 0u;
+        each(std::make_integer_sequence<int, MT>{}, [&](auto I) { xp[decltype(I)::value] += more ? x_step : 0u; });
+    };
+
+    // ---- main loop -----------------------------------------------------------------------------------
+    float16_t acc[NT * MT];  // tile t = nt MT + mt
+#pragma unroll
+    for (int t = 0; t < NT * MT; t++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[t][e] = 0.f;
+    // INT4: products and factors of two tiles, one being multiplied while the other is accumulated
+    float16_t P[FP4 ? 1 : 2], F[FP4 ? 1 : 2];
+#pragma unroll
+    for (int b = 0; b < (FP4 ? 1 : 2); b++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) P[b][e] = F[b][e] = 0.f;
+
+    auto compute = [&](auto S) {
+        auto &st = sets[decltype(S)::value];
+        if constexpr (!FP4) {
+            // step t issues the two matrix instructions of tile t and accumulates the tile before it (in the first step the
+            // last tile of the k-group before)
+            auto tile = [&](auto T) {
+                constexpr int t = decltype(T)::value, nt = t / MT, mt = t % MT, b = t & 1, prev = (t + NT * MT - 1) % (NT * MT);
+                P[b] = mfma_codes6(st.w[nt], st.x[mt]);
+                F[b] = mfma_factor(u32x2_t{st.ws[nt], 0u}, h ? 0u : st.as[mt]);
+#pragma unroll
+                for (int e = 0; e < 16; e++) acc[prev][e] = __builtin_fmaf(P[b ^ 1][e], F[b ^ 1][e], acc[prev][e]);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 9, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            each(std::make_integer_sequence<int, NT * MT>{}, tile);
+        } else {
+            half2_t sx[MT][2], sw[NT][2];  // a lane's two 16-groups
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                const half2_t s = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(st.as[mt], 1.0f, false);
+                sx[mt][0] = half2_t{s[0], s[0]};
+                sx[mt][1] = half2_t{s[1], s[1]};
+            }
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                const half2_t s = as_half2(st.ws[nt]);
+                sw[nt][0] = half2_t{s[0], s[0]};
+                sw[nt][1] = half2_t{s[1], s[1]};
+            }
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) {
+                half8_t x[MT];
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) x[mt] = dequant_word_fp4(st.x[mt][ks], sx[mt][ks >> 1]);
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++) {
+                    const half8_t w = dequant_word_fp4(st.w[nt][ks], sw[nt][ks >> 1]);
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++) acc[nt * MT + mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w, x[mt], acc[nt * MT + mt], 0, 0, 0);
+                }
+            }
+        }
+    };
+
+    each(std::make_integer_sequence<int, DEPTH>{}, [&](auto D) { load(D); });
+    int g = kpart;
+    auto step = [&](auto S) {
+        load(std::integral_constant<int, (decltype(S)::value + DEPTH) % (DEPTH + 1)>{});
+        __builtin_amdgcn_sched_barrier(0);
+        compute(S);
+        g += KP;
+    };
+    // (whole turns of the ring in the loop, what is left behind it: leaving the loop in the middle of a turn makes the
+    // compiler carry two copies of the accumulators)
+    while (g + DEPTH * KP < kgroups) each(std::make_integer_sequence<int, DEPTH + 1>{}, step);
+    if (g < kgroups) step(std::integral_constant<int, 0>{});
+    if constexpr (DEPTH > 1) {
+        if (g < kgroups) step(std::integral_constant<int, 1>{});
+    }
+    if constexpr (!FP4) {
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[NT * MT - 1][e] = __builtin_fmaf(P[1][e], F[1][e], acc[NT * MT - 1][e]);
+    }
+
+    // ---- the epilogue's own operands, requested before the waves meet ------------------------------------
+    // Wave w gets the 32 columns 32 w ... of all MT row blocks.
+    const int nt = wave, c0 = n0 + nt * 32, row0 = f0 * 32;
+    const int nsteps = p.R_up / 16;
+    constexpr int LSTEPS = 2;  // 16-rank steps of the low-rank up projection requested at once
+    float4_t la_raw[MT][LSTEPS][2];
+    u32x4_t up_raw[LSTEPS];
+    auto load_lora = [&](int s0) {
+#pragma unroll
+        for (int s = 0; s < LSTEPS; s++) {
+            const int step = s0 + s < nsteps ? s0 + s : nsteps - 1;
+#pragma unroll
+            for (int o = 0; o < MT; o++) {
+                const float4_t *ap = (const float4_t *)(p.lora_act + (size_t)(row0 + o * 32 + r32) * p.R_up + 16 * step + 8 * h);
+                la_raw[o][s][0] = ap[0];
+                la_raw[o][s][1] = ap[1];
+            }
+            up_raw[s] = *(const u32x4_t *)(p.lora_up + (size_t)(c0 + r32) * p.R_up + 16 * step + 8 * h);
+        }
+    };
+    float cf[4][4], bs[4][4];  // factor and bias of the lane's columns c0 + 8 q + 4 h + i
+    if (nsteps > 0) load_lora(0);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int c = c0 + 8 * q + 4 * h;
+        const float4_t cn = FP4 ? *(const float4_t *)(p.colnorm + c) : float4_t{1.f, 1.f, 1.f, 1.f};
+        const u32x2_t wc = p.wcscales ? *(const u32x2_t *)(p.wcscales + c) : u32x2_t{0x3F803F80u, 0x3F803F80u};
+        const u32x2_t bi = p.bias ? *(const u32x2_t *)(p.bias + c) : u32x2_t{0u, 0u};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            cf[q][i] = cn[i] * p.alpha * bits_f32(i & 1 ? wc[i >> 1] & 0xFFFF0000u : wc[i >> 1] << 16);
+            bs[q][i] = bits_f32(i & 1 ? bi[i >> 1] & 0xFFFF0000u : bi[i >> 1] << 16);
+        }
+    }
+
+    // ---- the waves' sums meet, 32 rows at a time, added in ascending order of the waves ---------------------
+    float16_t val[MT];
+    float4_t *park = (float4_t *)lds;
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+        if (mt > 0) __syncthreads();
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                park[((kpart * 4 + cw * NT + t) * 4 + q) * 64 + lane] =
+                    float4_t{acc[t * MT + mt][4 * q], acc[t * MT + mt][4 * q + 1], acc[t * MT + mt][4 * q + 2], acc[t * MT + mt][4 * q + 3]};
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            float4_t s = park[(nt * 4 + q) * 64 + lane];
+#pragma unroll
+            for (int j = 1; j < KP; j++) s += park[((j * 4 + nt) * 4 + q) * 64 + lane];
+#pragma unroll
+            for (int i = 0; i < 4; i++) val[mt][4 * q + i] = s[i];
+        }
+    }
+    __syncthreads();  // the sums have been read: the slabs take their place
+
+    float *ssq = (float *)(lds + KP * 16384);  // [MT][4 column tiles][32 rows]
+    const bool rope = NEXT && p.rotary && n0 < p.rope_cols;  // the tile is one head of q or k
+#pragma unroll
+    for (int o = 0; o < MT; o++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) val[o][e] *= cf[e >> 2][e & 3];
+    // low-rank up projection (lora.cuh:110-241): out += bf16(lora_act * scale) @ up^T
+    for (int s0 = 0; s0 < nsteps; s0 += LSTEPS) {
+        if (s0 > 0) load_lora(s0);
+#pragma unroll
+        for (int s = 0; s < LSTEPS; s++) {
+            if (s0 + s >= nsteps) break;
+            const float ls = p.lora_scales[s0 + s];
+#pragma unroll
+            for (int o = 0; o < MT; o++) {
+                const float4_t v0 = la_raw[o][s][0], v1 = la_raw[o][s][1];
+                u32x4_t w;
+                w[0] = pack_bf16x2(v0[0] * ls, v0[1] * ls);
+                w[1] = pack_bf16x2(v0[2] * ls, v0[3] * ls);
+                w[2] = pack_bf16x2(v1[0] * ls, v1[1] * ls);
+                w[3] = pack_bf16x2(v1[2] * ls, v1[3] * ls);
+                val[o] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, up_raw[s]), __builtin_bit_cast(bf16x8_t, w), val[o], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int o = 0; o < MT; o++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) val[o][e] += bs[e >> 2][e & 3];
+    if (rope) {
+#pragma unroll
+        for (int o = 0; o < MT; o++) {
+            float ss = 0.f;
+#pragma unroll
+            for (int e = 0; e < 16; e++) ss += val[o][e] * val[o][e];
+            ss += __shfl_xor(ss, 32);
+            if (h == 0) ssq[(o * 4 + nt) * 32 + r32] = ss;
+        }
+        // EpilogueRMSNormRope (epilogues.cuh:269-425); the (sin, cos) table is stored in this loop's order, see
+        // gemm6_kernel.h
+        __syncthreads();
+        const uint16_t *nw = (n0 < p.rope_cols / 2 ? p.norm_q : p.norm_k) + nt * 32 + 4 * h;
+#pragma unroll
+        for (int o = 0; o < MT; o++) {
+            int blk = f0 + o;
+            blk = blk < (p.rot_rows >> 5) ? blk : (p.rot_rows >> 5) - 1;  // (rows beyond the output are never stored)
+            const float4_t *rp = (const float4_t *)p.rotary + ((size_t)blk * 16 + nt * 4) * 64 + lane;
+            const float *sp = ssq + o * 128 + r32;
+            const float coef = __builtin_amdgcn_rsqf((((sp[0] + sp[32]) + sp[64]) + sp[96]) * (1.0f / 128.0f) + p.norm_eps);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const float4_t s4 = rp[q * 64];  // sin, cos of two pairs
+                const u32x2_t w2 = *(const u32x2_t *)(nw + 8 * q);
+#pragma unroll
+                for (int pr = 0; pr < 2; pr++) {
+                    const float x = val[o][4 * q + 2 * pr] * (coef * bits_f32(w2[pr] << 16));
+                    const float y = val[o][4 * q + 2 * pr + 1] * (coef * bits_f32(w2[pr] & 0xFFFF0000u));
+                    const float sn = s4[2 * pr], cs = s4[2 * pr + 1];
+                    val[o][4 * q + 2 * pr] = x * cs - y * sn;
+                    val[o][4 * q + 2 * pr + 1] = x * sn + y * cs;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int o = 0; o < MT; o++) {
+        if (NEXT && p.silu) {
+#pragma unroll
+            for (int e = 0; e < 16; e++) val[o][e] *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * val[o][e]));
+        }
+        if (NEXT && p.gelu) {
+#pragma unroll
+            for (int e = 0; e < 16; e++) val[o][e] = gelu_tanh(val[o][e]);
+        }
+        if (NEXT && p.vk && n0 < p.N / 3) {
+            // the q third of a linear-attention projection is stored after a ReLU (epilogues.cuh:662-674)
+#pragma unroll
+            for (int e = 0; e < 16; e++) val[o][e] = __builtin_fmaxf(val[o][e], 0.f);
+        }
+        uint16_t *slab = (uint16_t *)(lds + o * SLAB_BYTES);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            u32x2_t w;
+            w[0] = pack_bf16x2(val[o][4 * q], val[o][4 * q + 1]);
+            w[1] = pack_bf16x2(val[o][4 * q + 2], val[o][4 * q + 3]);
+            *(u32x2_t *)(slab + r32 * OUT_LD + nt * 32 + 8 * q + 4 * h) = w;
+        }
+    }
+    // the reciprocal smoothing factors of the next layer for the 32 columns a lane quantizes
+    float nrs[32];
+    const bool quantizes = NEXT && p.qout && wave < 2 * MT;
+    if (quantizes) {
+        const float4_t *sp = (const float4_t *)(p.next_smooth_rcp + n0 + (lane & 3) * 32);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const float4_t v4 = sp[i];
+            nrs[4 * i] = v4[0]; nrs[4 * i + 1] = v4[1]; nrs[4 * i + 2] = v4[2]; nrs[4 * i + 3] = v4[3];
+        }
+    }
+    __syncthreads();
+
+    // ---- the bf16 tile, MT slabs of 32 rows, is in LDS ------------------------------------------------------
+    if (p.out) {
+#pragma unroll
+        for (int it = 0; it < MT * 8 / WAVES; it++) {
+            const int item = it * WAVES + wave, mt = item >> 3, rr = (item & 7) * 4 + (lane >> 4), cc = (lane & 15) * 8;
+            const int m = (f0 + mt) * 32 + rr, n = n0 + cc;
+            const u32x4_t d = *(const u32x4_t *)((const uint16_t *)(lds + mt * SLAB_BYTES) + rr * OUT_LD + cc);
+            if (m < p.M_out && n < p.N_out) __builtin_nontemporal_store(d, (u32x4_t *)(p.out + (size_t)m * p.N_out + n));
+        }
+    }
+    if (NEXT && p.qkv.q && wave < MT) store_qkv_slab(p.qkv, (const uint16_t *)(lds + wave * SLAB_BYTES), OUT_LD, lane, (f0 + wave) * 32, n0, p.N / 3);
+    if (NEXT && p.vk && n0 >= p.N / 3 && wave < MT) {
+        VkSums vks;
+        litela_clear(vks);
+        litela_add_slab(vks, (const uint16_t *)(lds + wave * SLAB_BYTES), OUT_LD, lane);
+        const int third = p.N / 3;
+        litela_park<true>(vks, p.vk_part + ((size_t)(f0 + wave) * (2 * third / 64) + (n0 - third) / 64) * VK_HEAD_FLOATS, lane);
+    }
+    if (NEXT && p.next_down) {
+        // low-rank down projection of the next layer on the bf16 tile (EpilogueLoraDown, lora.cuh:243-353): the tile's 128
+        // columns are one chunk of the next layer's K, whose share goes to the workspace (reduce_shares_kernel in gemm.hip)
+        const int RT = p.R_down / 16, r16 = lane & 15, q = lane >> 4;
+        for (int item = wave; item < MT * RT * 2; item += WAVES) {
+            const int m2 = item & 1, rt = (item >> 1) % RT, mt = (item >> 1) / RT;
+            const uint16_t *slab = (const uint16_t *)(lds + mt * SLAB_BYTES);
+            float4_t d = {0.f, 0.f, 0.f, 0.f};
+            bf16x8_t b[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) b[i] = p.next_down[((size_t)(nb * 4 + i) * RT + rt) * 64 + lane];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const bf16x8_t a = *(const bf16x8_t *)(slab + (16 * m2 + r16) * OUT_LD + 32 * q + 8 * i);
+                d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[i], d, 0, 0, 0);
+            }
+            __builtin_nontemporal_store(d, (float4_t *)(p.next_lora_part + (size_t)nb * p.M_pad * p.R_down) + (((size_t)(f0 + mt) * RT + rt) * 2 + m2) * 64 + lane);
+        }
+    }
+    if (quantizes) {
+        // EpilogueQuantize (gemm_w4a4.cuh:930-1043): INT4 with the shift and unsigned codes, NVFP4 without
+        const int item = (wave & 1) * 64 + lane, rr = item >> 2, qc = item & 3;
+        const u32x4_t *sp = (const u32x4_t *)((const uint16_t *)(lds + (wave >> 1) * SLAB_BYTES) + rr * OUT_LD + qc * 32);
+        float y[32];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const u32x4_t v4 = sp[i];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                float lo = bits_f32(v4[j] << 16), hi = bits_f32(v4[j] & 0xFFFF0000u);
+                if (!FP4) {
+                    lo = bf16_bits_to_f32(f32_to_bf16_bits(__fadd_rn(lo, 0.171875f)));
+                    hi = bf16_bits_to_f32(f32_to_bf16_bits(__fadd_rn(hi, 0.171875f)));
+                }
+                y[8 * i + 2 * j] = smooth_quotient(lo, nrs[8 * i + 2 * j]);
+                y[8 * i + 2 * j + 1] = smooth_quotient(hi, nrs[8 * i + 2 * j + 1]);
+            }
+        }
+        const int m = (f0 + (wave >> 1)) * 32 + rr, gidx = (n0 + qc * 32) / 64, ngroups_out = p.N / 64;
+        if constexpr (!FP4) {
+            u32x4_t lo4;
+            u32x2_t hi2;
+            float sc;
+            quantize_int4_half_group_e2m3<true>(y, 1, lo4, hi2, sc);
+            if ((qc & 1) == 0) ((uint16_t *)p.oscales)[(size_t)gidx * p.M_pad + m] = (uint16_t)f32_to_bf16_bits(sc);
+            uint8_t *frag = p.qout + (((size_t)(m / ACT_BLOCK_ROWS) * ngroups_out + gidx) * 4 + (m % ACT_BLOCK_ROWS) / 32) * FRAG_BYTES;
+            const int slot = (m % 32) + 32 * (qc & 1);
+            *(u32x4_t *)(frag + slot * 16) = lo4;
+            *(u32x2_t *)(frag + 1024 + slot * 8) = hi2;
+        } else {
+            u32x4_t words;
+            uint32_t sc[2];
+            quantize_nvfp4_two_groups(y, words, sc);
+            ((uint16_t *)p.oscales)[((size_t)gidx * p.M_pad + m) * 2 + (qc & 1)] = (uint16_t)(sc[0] | (sc[1] << 8));  // [N/64][M_pad][4]
+            *(u32x4_t *)(p.qout + ((size_t)(m / 32) * ngroups_out + gidx) * TILE_BYTES + (m % 32) * 32 + 16 * (qc & 1)) = words;
+        }
+    }
+}
+
+template <bool FP4, int MT, int WN, int KP, int DEPTH, bool NEXT>
+int launch_direct(const GemmParams &p, hipStream_t stream) {
+    auto kern = gemm_direct_kernel<FP4, MT, WN, KP, DEPTH, NEXT>;
+    constexpr int smem = lds_bytes<MT, KP>();
+    static bool lds_reserved[64] = {false};  // set once per device (racing first calls both set it, which is harmless)
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(SVDQ_ELAUNCH, "gemm: cannot identify the current device");
+    if (!lds_reserved[dev]) {
+        hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+        if (e != hipSuccess) return fail(SVDQ_ELAUNCH, "gemm: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
+        lds_reserved[dev] = true;
+    }
+    SVDQ_LAUNCH(kern, dim3((unsigned)(p.row_blocks * (p.N / 128))), dim3(64 * WN * KP), smem, stream, p);
+    return check_launch("gemm_w4a4 (few rows)");
+}
+
+}  // namespace direct
+}  // namespace svdq

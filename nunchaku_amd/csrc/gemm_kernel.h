@@ -36,34 +36,12 @@
 
 #include <type_traits>
 
+#include "gemm_math.h"
 #include "gemm_params.h"
 #include "svdq_quant.h"
 
 namespace svdq {
 
-
-__device__ inline half2_t as_half2(uint32_t u) { return __builtin_bit_cast(half2_t, u); }
-__device__ inline uint32_t as_u32(half2_t h) { return __builtin_bit_cast(uint32_t, h); }
-
-// 8 E2M1 patterns of one word -> 8 fp16 values pattern_value * scale, slot order [0..7].  The
-// hardware conversion yields the exact E2M1 value (its scale operand only contributes an exponent).
-__device__ inline half8_t dequant_word_fp4(uint32_t w, half2_t s) {
-    const half2_t t0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 0) * s;
-    const half2_t t1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 1) * s;
-    const half2_t t2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 2) * s;
-    const half2_t t3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 3) * s;
-    return half8_t{t0[0], t0[1], t1[0], t1[1], t2[0], t2[1], t3[0], t3[1]};
-}
-
-__device__ inline float gelu_tanh(float x) {
-    // x * (0.5 + 0.5 * tanh(u)), u = 0.79788456 * (x + 0.044715 x^3)   (epilogues.cuh:22-44)
-    // With tanh(u) = 1 - 2 / (exp(2u) + 1) this is x - x / (exp(2u) + 1): one hardware exp2 and one hardware
-    // reciprocal (1 ulp each), safe at both ends (exp2 -> inf gives x, exp2 -> 0 gives 0).
-    constexpr float C1 = 2.0f * 0.79788456f * 1.4426950408889634f, C2 = C1 * 0.044715f;  // 2u * log2(e) = x (C1 + C2 x^2)
-    const float w = x * __builtin_fmaf(C2, x * x, C1);
-    const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(w) + 1.0f);
-    return __builtin_fmaf(-x, r, x);
-}
 
 // Partial sums of a tile shared by two workgroups travel through memory with system-scope accesses
 // (sc0 sc1): they bypass the caches that are not coherent between the XCDs, so no cache write-back or

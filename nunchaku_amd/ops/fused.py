@@ -33,6 +33,7 @@ def fused_gelu_mlp(x: torch.Tensor, fc1, fc2, pad_size: int = 256) -> torch.Tens
         c1, quantized_x, ascales, lora_act, M_pad,
         qout=qout_act.data_ptr(), oscales=qout_ascales.data_ptr(), next_smooth_rcp=c2.q.smooth_rcp,
         next_lora_down=c2.q.lora_down, next_lora_act_out=qout_lora_act.data_ptr() if fc2.rank else None, R_down=fc2.rank,
+        M_out=M,  # (fc2 reads nothing of the padding rows that reaches its output)
     )
     output = torch.empty(M, fc2.out_features, dtype=x.dtype, device=dev)
     fc2._gemm_prepared(c2, qout_act, qout_ascales, qout_lora_act, M_pad, out=output.data_ptr(), M_out=M)
