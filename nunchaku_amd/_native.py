@@ -84,6 +84,24 @@ GEMM_VARIANT_UNITS = [("gemm6_variant.hip", 0), ("gemm6_variant.hip", 1), ("gemm
                       ("gemm_direct_variant.hip", 0), ("gemm_direct_variant.hip", 1), ("gemm_direct_variant.hip", 2), ("gemm_direct_variant.hip", 3)]
 
 
+HOST_PATH = _PKG_DIR / "_host.so"
+
+
+def _host_commands(obj: Path, lib_path: Path, out: Path):
+    """Compile and link commands of the host extension (``csrc/host_ext.cpp``: no device code, torch's headers)."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+
+    torch_lib = Path(torch.__file__).resolve().parent / "lib"
+    includes = [*cpp_extension.include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    compile_ = ["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+                *[a for d in includes for a in ("-isystem", d)], "-c", str(_CSRC / "host_ext.cpp"), "-o", str(obj)]
+    link = ["g++", "-shared", str(obj), "-o", str(out), f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python",
+            f"-L{lib_path.parent}", f"-l:{lib_path.name}", "-Wl,-rpath,$ORIGIN"]
+    return compile_, link
+
+
 def build(verbose: bool = False, extra_flags: tuple[str, ...] = (), lib_path: Path | None = None) -> Path:
     """Compile the HIP sources for gfx950 into ``libsvdq_amd.so`` next to this file (hipcc
     cross-compiles; no GPU is needed).  Translation units are compiled in parallel, then linked."""
@@ -101,7 +119,9 @@ def build(verbose: bool = False, extra_flags: tuple[str, ...] = (), lib_path: Pa
             args, obj = job
             return subprocess.run([hipcc, *flags, "-c", *args, "-o", str(obj)], capture_output=True, text=True)
 
+        host_compile, host_link = _host_commands(Path(tmp) / "host_ext.o", out, HOST_PATH)
         with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1)) as pool:
+            host = pool.submit(subprocess.run, host_compile, capture_output=True, text=True) if lib_path is None else None
             results = list(pool.map(compile_one, jobs))
         for (args, _), res in zip(jobs, results):
             if res.returncode != 0:
@@ -110,6 +130,10 @@ def build(verbose: bool = False, extra_flags: tuple[str, ...] = (), lib_path: Pa
                               capture_output=True, text=True)
         if link.returncode != 0:
             raise RuntimeError("hipcc link failed:\n" + link.stderr[-4000:])
+        if host is not None:  # (the extension belongs to the library next to it: not for a library built elsewhere)
+            for res in (host.result(), subprocess.run(host_link, capture_output=True, text=True)):
+                if res.returncode != 0:
+                    raise RuntimeError("building the host extension failed:\n" + res.stderr[-4000:])
     if verbose:
         print(f"built {out}")
     return out
@@ -154,6 +178,22 @@ def lib() -> ctypes.CDLL:
             raise RuntimeError("libsvdq_amd.so was built from a different header version; rebuild it")
         _lib = L
     return _lib
+
+
+_host_module = None
+
+
+def host():
+    """The host extension module (``csrc/host_ext.cpp``), which calls the same library.  Raises if it has not been built."""
+    global _host_module
+    if _host_module is None:
+        lib()
+        if not HOST_PATH.exists():
+            raise RuntimeError(f"{HOST_PATH} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`")
+        from . import _host
+
+        _host_module = _host
+    return _host_module
 
 
 def check(rc: int) -> None:

@@ -9,7 +9,6 @@ tensors are what the kernels read.
 from __future__ import annotations
 
 import ctypes
-import threading
 
 import torch
 from torch import nn
@@ -22,10 +21,11 @@ from ..ops.quantize import svdq_quantize_w4a4_act_fuse_lora
 
 
 class _LayerCall:
-    """The argument blocks of a layer's two C-ABI calls with everything filled in that does not change from one
-    forward to the next (the layer's own tensors and sizes); ``SVDQW4A4Linear.forward`` only sets the pointers and
-    row counts of the call.  The layer's tensors were checked when they were converted; the per-call tensors are
-    allocated by ``forward`` itself, so the checks of the operator wrappers have nothing left to find."""
+    """A layer prepared for the host extension (``csrc/host_ext.cpp``): the argument blocks of its two C-ABI calls with
+    everything filled in that does not change from one forward to the next (the layer's own tensors and sizes).  A forward
+    only sets the pointers and row counts of the call.  The layer's tensors were checked when they were converted; the
+    per-call tensors are allocated by the extension itself, so the checks of the operator wrappers have nothing left to
+    find."""
 
     def __init__(self, mod: "SVDQW4A4Linear", t: dict):
         fp4 = mod.precision == "nvfp4"
@@ -42,26 +42,26 @@ class _LayerCall:
             if p is None or tuple(p.shape) != shape or p.dtype != dtype:
                 raise ValueError(f"{name} must be {dtype} {shape} for in_features={K}, out_features={N}, rank={R}, got "
                                  f"{None if p is None else (p.dtype, tuple(p.shape))}")
-        self.fp4 = fp4
-        self.act_bytes = packing.act_nbytes_per_row(K, fp4)
-        self.groups = K // mod.group_size
-        self.scale_dtype = torch.float8_e4m3fn if fp4 else torch.bfloat16
-        self.tensors = t  # keeps the converted tensors alive as long as their addresses are in the blocks
-        self.q = nv.QuantizeArgs(
+        self.tensors = t
+        self.device = t["qweight"].device
+        q = nv.QuantizeArgs(
             lora_down=nv.ptr(t["proj_down"]) if R else None, smooth_rcp=nv.ptr(t["smooth_factor"]),
             K=K, R=R, fp4=int(fp4), fuse_glu=0,
         )
-        self.device = t["qweight"].device
-        self.sc = (ctypes.c_float * max(1, (R + 15) // 16))()
-        self.scales_src = ()  # what self.sc was last written from (never a list or None: the first call writes)
-        self.g = nv.GemmArgs(
+        g = nv.GemmArgs(
             wgt=nv.ptr(t["qweight"]), wscales=nv.ptr(t["wscales"]), colnorm=nv.ptr(t["wscales"].colnorm), bias=nv.ptr(t["bias"]),
-            wcscales=nv.ptr(t["wcscales"]), lora_up=nv.ptr(t["proj_up"]) if R else None, lora_scales=self.sc,
+            wcscales=nv.ptr(t["wcscales"]), lora_up=nv.ptr(t["proj_up"]) if R else None,
             N=N, K=K, N_out=N, R_up=R, R_down=0, alpha=float(mod.alpha), act_unsigned=int(mod.act_unsigned), fuse_silu=0, fp4=int(fp4),
             norm_eps=_gemm_op.NORM_EPS,
         )
-        self.q_ref, self.g_ref = ctypes.byref(self.q), ctypes.byref(self.g)
-        self.lock = threading.Lock()  # the blocks are shared by the threads that call the layer
+        keep = [v for v in t.values() if v is not None]
+        if t["wscales"].colnorm is not None:
+            keep.append(t["wscales"].colnorm)
+        # (the tensors the blocks point into live as long as the handle, whatever becomes of the layer)
+        self.handle = nv.host().make_layer(
+            mod._NATIVE_SOURCES, mod._native_stamp, tuple(keep), ctypes.addressof(q), ctypes.addressof(g),
+            (self.device.index, packing.act_nbytes_per_row(K, fp4), K // mod.group_size * (1 if fp4 else 2)),
+        )
 
 
 class SVDQW4A4Linear(nn.Module):
@@ -209,7 +209,6 @@ class SVDQW4A4Linear(nn.Module):
             raise ValueError("skip_ranks must be a multiple of 16")
         groups = (self.rank + 15) // 16
         self.lora_scales = [1.0 if i < skip_ranks // 16 else float(scale) for i in range(groups)]
-        self._call = None
 
     @property
     def alpha(self) -> float:
@@ -222,28 +221,30 @@ class SVDQW4A4Linear(nn.Module):
 
     # ---- forward path (nunchaku/models/linear.py:89-132) ----------------------------------------
     def forward(self, x: torch.Tensor, output: torch.Tensor | None = None) -> torch.Tensor:
-        """``quantize`` then ``forward_quant`` (nunchaku/models/linear.py:89-110), through argument blocks prepared
-        once per layer: a forward costs the host four allocations and two calls into the library."""
+        """``quantize`` then ``forward_quant`` (nunchaku/models/linear.py:89-110), both launches from one call into the
+        host extension once the layer is converted."""
+        c = self._call
+        if c is not None:
+            y = nv.host().linear(c.handle, self, x, output, _gemm_op.K_SPLIT or 0, _gemm_op.NO_ALLOC)
+            if y is not None:
+                return y
+        # the first call, one on changed parameters, or one the extension has no fast way for: convert and check
         batch_size, seq_len, channels = x.shape
-        M = batch_size * seq_len
-        x = x.view(M, channels)
-        if M == 0:
-            return self._forward_by_operators(x, output).view(batch_size, seq_len, -1)
-        c = self._prepared(x)
-        dev = c.device
-        if output is None:
-            output = torch.empty(M, self.out_features, dtype=x.dtype, device=dev)
-        elif not (output.is_cuda and output.device == dev and output.dtype == torch.bfloat16 and output.is_contiguous()
-                  and output.numel() == M * self.out_features and output.shape[-1] == self.out_features):
-            raise ValueError(f"output must be a contiguous bf16 tensor of {M} x {self.out_features} elements on {dev}")
-        M_pad = (M + 255) // 256 * 256
-        qx, ascales, lora_act = self._quantize_prepared(c, x, M_pad)
-        self._gemm_prepared(c, qx, ascales, lora_act, M_pad, out=output.data_ptr(), M_out=M)
-        return output.view(batch_size, seq_len, -1)
+        x2 = x.view(batch_size * seq_len, channels)
+        if x2.shape[0]:
+            c = self._prepared(x2)
+            if output is not None and not (output.is_cuda and output.device == c.device and output.dtype == torch.bfloat16 and output.is_contiguous()
+                                           and output.numel() == x2.shape[0] * self.out_features and output.shape[-1] == self.out_features):
+                raise ValueError(f"output must be a contiguous bf16 tensor of {x2.shape[0]} x {self.out_features} elements on {c.device}")
+            y = nv.host().linear(c.handle, self, x, output, _gemm_op.K_SPLIT or 0, _gemm_op.NO_ALLOC)
+            if y is not None:
+                return y
+            if output is None:
+                output = torch.empty(x2.shape[0], self.out_features, dtype=x.dtype, device=c.device)
+        return self._forward_by_operators(x2, output).view(batch_size, seq_len, -1)
 
-    # The three steps of ``forward``, also used by ``ops.fused``: no argument is checked twice, none is looked up twice.
     def _prepared(self, x: torch.Tensor) -> _LayerCall:
-        """Checks the activations ``x`` [M, K] against the layer and returns the layer's argument blocks."""
+        """Checks the activations ``x`` [M, K] against the layer and returns the layer prepared for the extension."""
         if not x.is_cuda:
             raise RuntimeError(f"x must live on a GPU (got {x.device}); this path has no CPU implementation")
         if not x.is_contiguous():
@@ -262,44 +263,6 @@ class SVDQW4A4Linear(nn.Module):
         if c.device != dev:
             raise ValueError(f"the activations are on {dev}, the layer on {c.device}")
         return c
-
-    def _quantize_prepared(self, c: _LayerCall, x: torch.Tensor, M_pad: int):
-        dev = c.device
-        qx = torch.empty(M_pad, c.act_bytes, dtype=torch.uint8, device=dev)
-        ascales = torch.empty(c.groups, M_pad, dtype=c.scale_dtype, device=dev)
-        lora_act = torch.empty(M_pad, self.rank, dtype=torch.float32, device=dev)
-        with c.lock:
-            q = c.q
-            q.input, q.output, q.oscales = x.data_ptr(), qx.data_ptr(), ascales.data_ptr()
-            q.lora_act_out = lora_act.data_ptr() if self.rank else None
-            q.M, q.M_pad = x.shape[0], M_pad
-            nv.launch(nv.lib().svdq_quantize_w4a4_act_fuse_lora, c.q_ref, dev)
-        return qx, ascales, lora_act
-
-    def _gemm_prepared(self, c: _LayerCall, qx: torch.Tensor, ascales: torch.Tensor, lora_act: torch.Tensor, M_pad: int,
-                       out: int | None = None, M_out: int = 0, **epilogue) -> None:
-        """The layer's GEMM on quantized activations made for it (``_quantize_prepared``, or another layer's
-        next-layer epilogue).  ``out``: address of a bf16 [M_out, N] buffer.  ``epilogue``: further fields of the
-        argument block (addresses and sizes), in force for this call only."""
-        lib = nv.lib()
-        with c.lock:
-            g = c.g
-            ls = self.lora_scales
-            if ls is not None or c.scales_src is not None:  # one factor per 16 ranks; missing entries count as zero, None as all ones
-                for i in range(len(c.sc)):
-                    c.sc[i] = 1.0 if ls is None else (float(ls[i]) if i < len(ls) else 0.0)
-                c.scales_src = ls
-            g.act, g.ascales, g.out = qx.data_ptr(), ascales.data_ptr(), out
-            g.lora_act_in = lora_act.data_ptr() if self.rank else None
-            g.M_pad, g.M_out = M_pad, M_out
-            g.k_split = int(_gemm_op.K_SPLIT or 0)
-            for name, value in epilogue.items():
-                setattr(g, name, value)
-            try:
-                nv.launch(lib.svdq_gemm_w4a4_noalloc if _gemm_op.NO_ALLOC else lib.svdq_gemm_w4a4, c.g_ref, c.device)
-            finally:
-                for name in epilogue:
-                    setattr(g, name, 0 if name in ("R_down",) else None)
 
     def _forward_by_operators(self, x: torch.Tensor, output: torch.Tensor | None) -> torch.Tensor:
         """The same through the two operator wrappers (every argument checked on every call)."""
@@ -353,6 +316,9 @@ class AWQW4A16Linear(nn.Module):
         self.wzeros = nn.Parameter(torch.empty(in_features // group_size, out_features, dtype=torch_dtype, device=device), requires_grad=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        y = nv.host().awq_linear(self, x)
+        if y is not None:
+            return y
         from ..ops.gemv import awq_gemv_w4a16
 
         x = x.contiguous()

@@ -2,41 +2,56 @@
 
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
-from ..utils import ceil_divide
+from .. import _native as nv
+from .. import packing
+from . import gemm as _gemm_op
 from .gemm import svdq_gemm_w4a4
+from .quantize import svdq_quantize_w4a4_act_fuse_lora
 
 
 def fused_gelu_mlp(x: torch.Tensor, fc1, fc2, pad_size: int = 256) -> torch.Tensor:
     """fc1 -> GELU -> fc2 with the GELU, fc2's activation quantization (unsigned INT4 after a
     +0.171875 shift) and fc2's low-rank down projection fused into fc1's GEMM epilogue
-    (nunchaku/ops/fused.py:10-47).  Three calls into the library through the layers' prepared argument blocks."""
+    (nunchaku/ops/fused.py:10-47).  All launches come from one call into the host extension once the layers are converted."""
+    c1, c2 = fc1._call, fc2._call
+    if c1 is not None and c2 is not None:
+        y = nv.host().gelu_mlp(c1.handle, fc1, c2.handle, fc2, x, pad_size, _gemm_op.K_SPLIT or 0, _gemm_op.NO_ALLOC)
+        if y is not None:
+            return y
+    # the first call, one on changed parameters, or one the extension has no fast way for: convert and check
     batch_size, seq_len, channels = x.shape
     M = batch_size * seq_len
-    x = x.view(M, channels)
+    x2 = x.view(M, channels)
     if pad_size % 256 != 0:
         raise ValueError("pad_size must be a multiple of 256")
     if fc1.out_features != fc2.in_features or fc1.precision != fc2.precision:
         raise ValueError(f"fc2 ({fc2}) does not take what fc1 ({fc1}) gives")
     if M == 0:
         return x.new_empty(batch_size, seq_len, fc2.out_features)
-    c1 = fc1._prepared(x)
+    c1 = fc1._prepared(x2)
     dev = c1.device
     c2 = fc2._blocks(dev)
-    M_pad = ceil_divide(M, pad_size) * pad_size
-    quantized_x, ascales, lora_act = fc1._quantize_prepared(c1, x, M_pad)
-    qout_act = torch.empty(M_pad, c2.act_bytes, dtype=torch.uint8, device=dev)
-    qout_ascales = torch.empty(c2.groups, M_pad, dtype=c2.scale_dtype, device=dev)
-    qout_lora_act = torch.empty(M_pad, fc2.rank, dtype=torch.float32, device=dev)
-    fc1._gemm_prepared(
-        c1, quantized_x, ascales, lora_act, M_pad,
-        qout=qout_act.data_ptr(), oscales=qout_ascales.data_ptr(), next_smooth_rcp=c2.q.smooth_rcp,
-        next_lora_down=c2.q.lora_down, next_lora_act_out=qout_lora_act.data_ptr() if fc2.rank else None, R_down=fc2.rank,
-        M_out=M,  # (fc2 reads nothing of the padding rows that reaches its output)
+    y = nv.host().gelu_mlp(c1.handle, fc1, c2.handle, fc2, x, pad_size, _gemm_op.K_SPLIT or 0, _gemm_op.NO_ALLOC)
+    if y is not None:
+        return y
+    t1, t2 = c1.tensors, c2.tensors
+    fp4 = fc1.precision == "nvfp4"
+    act, ascales, lora_act = svdq_quantize_w4a4_act_fuse_lora(x2, lora_down=t1["proj_down"], smooth=t1["smooth_factor"], fp4=fp4, pad_size=pad_size)
+    M_pad = act.shape[0]
+    qout = torch.empty(M_pad, packing.act_nbytes_per_row(fc2.in_features, fp4), dtype=torch.uint8, device=dev)
+    oscales = torch.empty(fc2.in_features // fc2.group_size, M_pad, dtype=ascales.dtype, device=dev)
+    lora_out = torch.empty(M_pad, fc2.rank, dtype=torch.float32, device=dev)
+    svdq_gemm_w4a4(
+        act=act, wgt=t1["qweight"], qout=qout, ascales=ascales, wscales=t1["wscales"], oscales=oscales, lora_act_in=lora_act, lora_up=t1["proj_up"],
+        lora_down=t2["proj_down"], lora_act_out=lora_out, bias=t1["bias"], smooth_factor=t2["smooth_factor"], fp4=fp4, alpha=fc1.alpha,
+        wcscales=t1["wcscales"], act_unsigned=fc1.act_unsigned, lora_scales=fc1.lora_scales,
     )
     output = torch.empty(M, fc2.out_features, dtype=x.dtype, device=dev)
-    fc2._gemm_prepared(c2, qout_act, qout_ascales, qout_lora_act, M_pad, out=output.data_ptr(), M_out=M)
+    fc2.forward_quant(qout, oscales, lora_out, output)
     return output.view(batch_size, seq_len, -1)
 
 
@@ -49,13 +64,22 @@ def fused_qkv_norm_rottary(x: torch.Tensor, proj, norm_q, norm_k, rotary_emb: to
     fp16 [1, heads, tokens_pad, 128] tensors: the three apart, per head, rows from ``attn_tokens`` on
     masked (see ``svdq_gemm_w4a4``)."""
     batch_size, seq_len, channels = x.shape
-    x = x.view(batch_size * seq_len, channels)
-    c = proj._prepared(x)
-    quantized_x, ascales, lora_act = proj._quantize_prepared(c, x, ceil_divide(x.shape[0], 256) * 256)
+    x2 = x.view(batch_size * seq_len, channels)
+    c = proj._call
+    if c is None:
+        c = proj._prepared(x2)
+    if output is None or isinstance(output, tuple):
+        rot = packing.native(rotary_emb, "rotemb")
+        y = nv.host().qkv_norm_rope(c.handle, proj, x, norm_q.weight, norm_k.weight, rot, output, attn_tokens, _gemm_op.NORM_EPS, _gemm_op.K_SPLIT or 0,
+                                    _gemm_op.NO_ALLOC)
+        if y is not None:
+            return y
+    c = proj._prepared(x2)
+    quantized_x, ascales, lora_act = proj.quantize(x2)
     t = c.tensors
     common = dict(
         act=quantized_x, wgt=t["qweight"], ascales=ascales, wscales=t["wscales"], lora_act_in=lora_act, lora_up=t["proj_up"],
-        bias=t["bias"], fp4=c.fp4, alpha=c.g.alpha, wcscales=t["wcscales"], norm_q=norm_q.weight,
+        bias=t["bias"], fp4=proj.precision == "nvfp4", alpha=proj.alpha, wcscales=t["wcscales"], norm_q=norm_q.weight,
         norm_k=norm_k.weight, rotary_emb=rotary_emb, lora_scales=proj.lora_scales,
     )
     if isinstance(output, tuple):
@@ -75,10 +99,6 @@ def linearattn_vk_mul_q(q: torch.Tensor, vk: torch.Tensor, num_tokens: int | Non
     in place (kernels::linearattn_vk_mul_q, gemm_w4a4_launch_impl.cuh:427-448).  q bf16 [B, tokens_pad, heads * 32]
     (``out_linearattn`` of ``svdq_gemm_w4a4``), vk fp32 [B, heads, 33, 32] (its ``out_vk``); only the first
     ``num_tokens`` rows of every batch entry are touched (all by default, as in the reference)."""
-    import ctypes
-
-    from .. import _native as nv
-
     nv.require_gpu(q, "q")
     nv.require_gpu(vk, "vk")
     if q.dim() != 3 or vk.dim() != 4 or q.dtype != torch.bfloat16 or vk.dtype != torch.float32:

@@ -27,6 +27,10 @@ def awq_gemv_w4a16(
     (not in the reference signature: AWQW4A16Linear adds it afterwards, linear.py:183-185) is added to the
     rounded result inside the kernel when given.
     """
+    y = nv.host().awq_gemv(in_feats, kernel, scaling_factors, zeros, m, n, k, group_size, bias)
+    if y is not None:
+        return y
+    # not the plain case: say what is wrong, or take the call on another device than the current one
     for name, t in (("in_feats", in_feats), ("kernel", kernel), ("scaling_factors", scaling_factors), ("zeros", zeros)):
         nv.require_gpu(t, name)
         if not t.is_contiguous():
