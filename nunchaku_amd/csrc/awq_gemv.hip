@@ -24,13 +24,128 @@ struct AwqParams {
 };
 
 
-// The products go to the matrix cores (with v_dot2_f32_bf16 per row of x and pair instead, one row took 11.9 us
-// against 11.3 at K = 3072, N = 18432, four rows 17.4 against 12.0, eight 28.0 against 14.7).
-// A workgroup owns 16 output channels; its four waves take the 128-channel steps of K in turn and meet in LDS at the
-// end.  Lane l holds output channel l % 16 and the 32 input channels 128 it + 32 (l / 16) + [0, 32) of a step: the four
-// packed pairs of nibble position p (channels 8 p ... 8 p + 7 of the 32) are the second operand of the p-th
-// v_mfma_f32_16x16x32_bf16 of the step as they come, the first is x[m = l % 16][the same 8 channels] (zero for rows
-// beyond M).  The result tile has channel l % 16 and rows 4 (l / 16) + [0, 4) in lane l.
+// 32 codes of one channel, the 16 bytes a lane holds of a 32-channel half, to the second operands of four
+// v_mfma_f32_16x16x32_bf16: operand q holds bf16(code * scale + zero) of input channels 8 q ... 8 q + 7.  A code as a byte is
+// the E4M3 pattern of code * 2^-9 (subnormals and the first binade are evenly spaced), so the hardware conversion makes two
+// floats per instruction; s512 = 512 * scale undoes the 2^-9 exactly and the sum is rounded once, by the fused multiply-add,
+// before the rounding to bf16.  (One v_cvt_f32_ubyte per code: 11.1 us against 10.0 at K = 3072, N = 18432, one row, the
+// kernel being bound by its vector instructions.)
+__device__ inline void dequantize32(u32x4_t w, float s512, float zero, u32x4_t (&wb)[4]) {
+    typedef float f32x2_t __attribute__((ext_vector_type(2)));
+    float f[4][8];  // word i2, nibble p + 4 b = channel 8 p + 2 i2 + b
+#pragma unroll
+    for (int i2 = 0; i2 < 4; i2++) {
+        const uint32_t even = w[i2] & 0x0F0F0F0Fu, odd = (w[i2] >> 4) & 0x0F0F0F0Fu;
+        const f32x2_t e0 = __builtin_amdgcn_cvt_pk_f32_fp8(even, false), e1 = __builtin_amdgcn_cvt_pk_f32_fp8(even, true);
+        const f32x2_t o0 = __builtin_amdgcn_cvt_pk_f32_fp8(odd, false), o1 = __builtin_amdgcn_cvt_pk_f32_fp8(odd, true);
+        f[i2][0] = e0[0]; f[i2][2] = e0[1]; f[i2][4] = e1[0]; f[i2][6] = e1[1];
+        f[i2][1] = o0[0]; f[i2][3] = o0[1]; f[i2][5] = o1[0]; f[i2][7] = o1[1];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+        for (int i2 = 0; i2 < 4; i2++) wb[q][i2] = pack_bf16x2(__builtin_fmaf(f[i2][q], s512, zero), __builtin_fmaf(f[i2][q + 4], s512, zero));
+}
+
+// the reference stores bf16 and adds the bias to that (linear.py:183-185): two roundings
+__device__ inline void store_result(const AwqParams &p, int m, int row, float sum) {
+    float o = bf16_bits_to_f32(f32_to_bf16_bits(sum));
+    if (p.bias) o = bf16_bits_to_f32(f32_to_bf16_bits(o + bf16_bits_to_f32(p.bias[row])));
+    p.out[(size_t)m * p.N + row] = (uint16_t)f32_to_bf16_bits(o);
+}
+
+// K up to 4096: one workgroup of eight waves per compute unit, each wave with SPW steps of 128 input channels
+// (wave, wave + 8, ...) whose activations stay in its registers for all the tiles of 16 output channels the workgroup
+// walks through; the codes, scales and zeros of the next AHEAD tiles are requested while one is multiplied.  Lane l holds
+// output channel l % 16 of the tile and input channels 32 (l / 16) + [0, 32) of a step: the second operand of four matrix
+// instructions as dequantized (above), the first being x[m = l % 16] of the same channels, zero for rows beyond M and
+// channels beyond K.  The result tile has channel l % 16 and rows 4 (l / 16) + [0, 4) in lane l; the waves' tiles meet in
+// LDS once per BATCH tiles and are added in ascending order.
+// Per step and wave this leaves 84 vector instructions for 32 codes per lane, where a workgroup per tile, with its
+// activations in LDS, needed 140.  Measured with weights from HBM (12 layers in turn), before / now: K = 3072,
+// N = 18432 one row 11.9 / 10.7 us, four 13.0 / 10.8, eight 15.7 / 11.4; K = 4096, N = 20480, eight rows 24.1 / 15.3;
+// K = 3072, N = 9216, one row 8.5 / 8.0.  About 3 us of that are launch and latency, the rest 4.2 TB/s.  Further ahead is slower
+// (three tiles 11.7, four 12.4), two workgroups of half the tiles per compute unit too (13.0).
+constexpr int WAVES = 8, BATCH = 6, AHEAD = 2;
+static_assert(BATCH % (AHEAD + 1) == 0, "the ring of register sets is indexed by the position in a batch");
+template <int SPW>
+__global__ void __launch_bounds__(64 * WAVES, 2) awq_gemv_rows_kernel(AwqParams p) {
+    __shared__ float4_t red[BATCH][WAVES][64];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = lane & 15, kb = lane >> 4;
+    const int kblocks = p.K / 64;
+    int wg = blockIdx.x;
+    if (gridDim.x % 8 == 0) wg = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;  // neighbours in N on one XCD: they share lines of scales
+    const int ntiles = (p.N + 15) / 16;
+    const int t_begin = (int)((long long)ntiles * wg / gridDim.x), t_end = (int)((long long)ntiles * (wg + 1) / gridDim.x);
+
+    u32x4_t x[SPW][4];
+    uint32_t w_off[SPW], s_off[SPW];
+#pragma unroll
+    for (int j = 0; j < SPW; j++) {
+        const int cb = (wave + WAVES * j) * 2 + (kb >> 1), block = cb < kblocks ? cb : kblocks - 1;  // the lane's 64-channel block
+        const uint16_t *xp = p.x + (size_t)(n < p.M ? n : 0) * p.K + block * 64 + 32 * (kb & 1);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const u32x4_t v = *(const u32x4_t *)(xp + 8 * q);
+            x[j][q] = cb < kblocks && n < p.M ? v : u32x4_t{0, 0, 0, 0};
+        }
+        w_off[j] = (uint32_t)(n >> 2) * (uint32_t)(kblocks * 128) + (uint32_t)(n & 3) * 32u + (uint32_t)(kb & 1) * 16u + (uint32_t)block * 128u;
+        s_off[j] = (uint32_t)block * (uint32_t)p.N * 2u + (uint32_t)n * 2u;
+    }
+    struct Tile {
+        u32x4_t w[SPW];
+        uint16_t s[SPW], z[SPW];
+    };
+    // first channel of a tile: the last one of a ragged N begins early and works some channels out twice
+    auto first_channel = [&](int t) { return 16 * t < p.N - 16 ? 16 * t : p.N - 16; };
+    auto load = [&](int t, Tile &d) {
+        const int c0 = first_channel(t);
+        const uint8_t *wp = p.qweight + (size_t)(c0 >> 2) * kblocks * 128;
+        const uint8_t *sp = (const uint8_t *)(p.scales + c0), *zp = (const uint8_t *)(p.zeros + c0);
+#pragma unroll
+        for (int j = 0; j < SPW; j++) {
+            d.w[j] = __builtin_nontemporal_load((const u32x4_t *)(wp + w_off[j]));
+            d.s[j] = *(const uint16_t *)(sp + s_off[j]);
+            d.z[j] = *(const uint16_t *)(zp + s_off[j]);
+        }
+    };
+    Tile ring[AHEAD + 1];
+#pragma unroll
+    for (int a = 0; a < AHEAD; a++) load(t_begin + a, ring[a]);
+    for (int t0 = t_begin; t0 < t_end; t0 += BATCH) {
+        const int count = t_end - t0 < BATCH ? t_end - t0 : BATCH;
+        if (t0 > t_begin) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < BATCH; i++) {
+            if (i >= count) continue;
+            load(t0 + i + AHEAD, ring[(i + AHEAD) % (AHEAD + 1)]);
+            __builtin_amdgcn_sched_barrier(0);
+            const Tile &d = ring[i % (AHEAD + 1)];
+            float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < SPW; j++) {
+                u32x4_t wb[4];
+                dequantize32(d.w[j], bf16_bits_to_f32(d.s[j]) * 512.0f, bf16_bits_to_f32(d.z[j]), wb);
+#pragma unroll
+                for (int q = 0; q < 4; q++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[j][q]), __builtin_bit_cast(bf16x8_t, wb[q]), acc, 0, 0, 0);
+            }
+            red[i][wave][lane] = acc;
+        }
+        __syncthreads();
+        for (int idx = threadIdx.x; idx < count * 16 * p.M; idx += 64 * WAVES) {
+            const int c = idx & 15, m = (idx >> 4) % p.M, i = (idx >> 4) / p.M;
+            float sum = 0.f;
+#pragma unroll
+            for (int w = 0; w < WAVES; w++) sum += ((const float *)&red[i][w][(m >> 2) * 16 + c])[m & 3];
+            store_result(p, m, first_channel(t0 + i) + c, sum);
+        }
+    }
+}
+
+// Longer rows: a workgroup of four waves owns 16 output channels; the waves take the 128-channel steps of K in turn, with
+// the activations in LDS where they fit.
 template <bool XLDS>
 __global__ void __launch_bounds__(256) awq_gemv_mfma_kernel(AwqParams p) {
     extern __shared__ u32x4_t xlds[];  // XLDS (x fits: up to 64 KB): [M][K] bf16; then, always, 4 waves x 64 lanes x float4
@@ -80,21 +195,10 @@ __global__ void __launch_bounds__(256) awq_gemv_mfma_kernel(AwqParams p) {
                 xa[j] = XLDS ? xlds[xoff / 8] : *(const u32x4_t *)(p.x + xoff);
             }
         }
-        const uint32_t lo[4] = {w[0] & 0x0F0F0F0Fu, w[1] & 0x0F0F0F0Fu, w[2] & 0x0F0F0F0Fu, w[3] & 0x0F0F0F0Fu};
-        const uint32_t hi[4] = {(w[0] >> 4) & 0x0F0F0F0Fu, (w[1] >> 4) & 0x0F0F0F0Fu, (w[2] >> 4) & 0x0F0F0F0Fu, (w[3] >> 4) & 0x0F0F0F0Fu};
+        u32x4_t wb[4];
+        dequantize32(w, s * 512.0f, z, wb);
 #pragma unroll
-        for (int pq = 0; pq < 4; pq++) {
-            // nibbles pq and pq + 4 of word i2 are channels 8 pq + 2 i2 and 8 pq + 2 i2 + 1
-            u32x4_t wb;
-#pragma unroll
-            for (int i2 = 0; i2 < 4; i2++) {
-                const uint32_t src = (pq & 1) ? hi[i2] : lo[i2];
-                const int byte = pq >> 1;
-                const float q0 = (float)((src >> (8 * byte)) & 0xFFu), q1 = (float)((src >> (8 * byte + 16)) & 0xFFu);
-                wb[i2] = pack_bf16x2(__builtin_fmaf(q0, s, z), __builtin_fmaf(q1, s, z));  // bf16(code * scale + zero), see above
-            }
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, xa[pq]), __builtin_bit_cast(bf16x8_t, wb), acc, 0, 0, 0);
-        }
+        for (int q = 0; q < 4; q++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, xa[q]), __builtin_bit_cast(bf16x8_t, wb[q]), acc, 0, 0, 0);
     };
     // wave w takes the steps w, w + 4, ...; the ring of DEPTH + 1 register sets is indexed statically
 #pragma unroll
@@ -115,14 +219,18 @@ done:
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int m = 4 * kb + i;
-            if (m < p.M && row_raw < p.N) {
-                // the reference stores bf16 and adds the bias to that (linear.py:183-185): two roundings
-                float o = bf16_bits_to_f32(f32_to_bf16_bits(((acc[i] + a1[i]) + a2[i]) + a3[i]));
-                if (p.bias) o = bf16_bits_to_f32(f32_to_bf16_bits(o + bf16_bits_to_f32(p.bias[row])));
-                p.out[(size_t)m * p.N + row] = (uint16_t)f32_to_bf16_bits(o);
-            }
+            if (m < p.M && row_raw < p.N) store_result(p, m, row, ((acc[i] + a1[i]) + a2[i]) + a3[i]);
         }
     }
+}
+
+template <int SPW>
+int launch_rows(const AwqParams &p, hipStream_t stream) {
+    int dev = 0;
+    const int ncu = hipGetDevice(&dev) == hipSuccess && compute_units(dev) > 0 ? compute_units(dev) : 256;
+    const int ntiles = (p.N + 15) / 16;
+    SVDQ_LAUNCH((awq_gemv_rows_kernel<SPW>), dim3(ntiles < ncu ? ntiles : ncu), dim3(64 * WAVES), 0, stream, p);
+    return check_launch("awq_gemv_w4a16");
 }
 
 int launch_mfma(const AwqParams &p, hipStream_t stream) {
@@ -155,5 +263,13 @@ extern "C" int svdq_awq_gemv_w4a16(const svdq_awq_gemv_args *a, void *stream) {
     AwqParams p{(const uint16_t *)a->x, (const uint8_t *)a->qweight, (const uint16_t *)a->scales, (const uint16_t *)a->zeros,
                 (const uint16_t *)a->bias, (uint16_t *)a->out, (int)a->M, (int)a->N, (int)a->K};
     hipStream_t st = (hipStream_t)stream;
+    // (byte offsets of a lane's scales are 32 bits wide)
+    const int64_t steps = (a->K + 127) / 128;
+    if (a->N >= 16 && steps <= 4 * WAVES && a->K / 64 * a->N < (1ll << 30)) {
+        if (steps <= WAVES) return launch_rows<1>(p, st);
+        if (steps <= 2 * WAVES) return launch_rows<2>(p, st);
+        if (steps <= 3 * WAVES) return launch_rows<3>(p, st);
+        return launch_rows<4>(p, st);
+    }
     return launch_mfma(p, st);
 }

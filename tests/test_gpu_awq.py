@@ -48,6 +48,19 @@ def test_against_oracle(dev, rows, oc, ic):
     _check(y, awq.gemv(x, codes, scales, zeros), bias)
 
 
+@pytest.mark.parametrize("rows", [1, 5, 8])
+@pytest.mark.parametrize("oc,ic", [(16, 64), (20, 128), (12, 192), (100, 2112), (52, 4096), (28676, 128)])
+def test_edges_of_the_tile_walk(dev, rows, oc, ic):
+    """A last tile that begins early (oc not a multiple of 16), fewer channels than a tile, one to four steps of K per wave
+    with and without a remainder, and more tiles per workgroup than meet at once."""
+    announce(f"awq gemv rows={rows} oc={oc} ic={ic}")
+    m, (codes, scales, zeros, bias) = _module(dev, oc, ic, seed=oc + ic)
+    x = torch.randn(rows, ic, generator=torch.Generator().manual_seed(rows)).to(torch.bfloat16)
+    y = m(x.to(dev))
+    torch.cuda.synchronize()
+    _check(y, awq.gemv(x, codes, scales, zeros), bias)
+
+
 def test_long_k_takes_the_path_without_lds_staging(dev):
     """8 rows of K=4160 do not fit the 64 KB the kernel stages x in: the activations then come from global memory."""
     oc, ic, rows = 64, 4160, 8
