@@ -20,9 +20,6 @@
 // bf16 tile meets in LDS again and all waves store it, project and quantize it for the next layer.
 #pragma once
 
-#include <type_traits>
-#include <utility>
-
 #include "gemm_math.h"
 #include "gemm_params.h"
 #include "svdq_quant.h"
@@ -42,11 +39,6 @@ struct Stage<true, MT, NT> {
     u32x4_t w[NT], x[MT];
     uint32_t ws[NT], as[MT];
 };
-
-template <int... I, typename F>
-__device__ inline void each(std::integer_sequence<int, I...>, F &&f) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
 
 constexpr int SLAB_BYTES = 32 * OUT_LD * 2;
 // LDS: the waves' sums of 32 rows x 128 columns, [KP][4 column tiles][4 quads][64 lanes] x float4; behind them the sums of

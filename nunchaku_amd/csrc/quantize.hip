@@ -36,6 +36,7 @@ struct QuantParams {
     float *lora_out;         // [M_pad, R]
     const float *smooth_rcp; // [K] or null
     int M, M_pad, K, R;
+    int splits;              // few-rows kernel: workgroups that share the chunks of 16 rows
     int rt_base;             // first 16-rank tile of the projection this launch computes (ranks above 128 take several launches)
 };
 
@@ -59,8 +60,10 @@ constexpr uint32_t RSRC_WORD3 = 0x00020000;  // raw buffer, 32-bit data format
 // Ranks above 16 RT_MAX: a launch projects onto the rank tiles [rt_base, rt_base + RT_MAX) only (its accumulators
 // live in registers), so the operator launches the kernel once per window of 128 ranks; the launches after the
 // first (QUANT false) read x again, which the caches still hold, and neither quantize nor store codes.
-template <int NW, int MT, int RT_MAX, int DEPTH, bool FP4, int SMOOTH, bool GLU, bool ROWS, bool QUANT = true>
-__global__ void __launch_bounds__(64 * NW) quantize_fuse_lora_kernel(QuantParams p) {
+//
+// QUANT, PROJECT: what this workgroup does with its chunks; cfirst, cstep: the chunks of this wave.
+template <int NW, int MT, int RT_MAX, int DEPTH, bool FP4, int SMOOTH, bool GLU, bool ROWS, bool QUANT, bool PROJECT>
+__device__ __forceinline__ void quantize_rows(const QuantParams &p, int cfirst, int cstep, uint8_t *tr) {
     // smoothing factors [K] during the walk; then, chunks split: [NW waves][MT][RT][64][4] partial projections;
     // rows split: behind the factors two buffers of [4 steps][RT][64 lanes] x 16 bytes of proj_down
     extern __shared__ __attribute__((aligned(16))) float lds[];  // (the alignment lets the factors be read 16 bytes at a time)
@@ -100,8 +103,6 @@ __global__ void __launch_bounds__(64 * NW) quantize_fuse_lora_kernel(QuantParams
     // on the whole kernel.)  The pieces are brought into that layout through a per-wave LDS area, see below.
     constexpr int PPR = 16 * XW, RPI = 64 / PPR;  // pieces per row, rows per instruction
     const uint32_t x_voff = (uint32_t)((lane / PPR) * ld * 2 + (lane % PPR) * 16);
-    __shared__ __attribute__((aligned(16))) uint8_t transpose_area[NW][16 * PPR * 16];
-    uint8_t *tr = transpose_area[wave];
 
     // x of one chunk: MT tiles x 4 steps x 8 bf16 per lane (twice that with GLU)
     // Requests are unconditional (a request behind a branch makes the compiler's wait counting assume the
@@ -124,10 +125,8 @@ __global__ void __launch_bounds__(64 * NW) quantize_fuse_lora_kernel(QuantParams
 
     // DEPTH chunks are requested ahead of the one being worked on
     u32x4_t xv[DEPTH + 1][MT][XL];
-    constexpr int CSTEP = ROWS ? 1 : NW;  // distance between the chunks a wave works on
-    const int cfirst = ROWS ? 0 : wave;
 #pragma unroll
-    for (int s = 0; s < DEPTH; s++) load_x(cfirst + s * CSTEP, xv[s]);
+    for (int s = 0; s < DEPTH; s++) load_x(cfirst + s * cstep, xv[s]);
 
     if (QUANT && SMOOTH == 1) {
         for (int k = threadIdx.x * 4; k < p.K; k += 64 * NW * 4) *(float4_t *)&lds[k] = *(const float4_t *)(p.smooth_rcp + k);
@@ -187,7 +186,7 @@ __global__ void __launch_bounds__(64 * NW) quantize_fuse_lora_kernel(QuantParams
         // ---- requests first: the low-rank operands of this chunk (all four steps when they fit the
         // registers), then the activations DEPTH chunks ahead.  In this order a wait for the operands
         // does not wait for the activations.
-        constexpr bool DOWN_UPFRONT = !ROWS && RT_MAX <= 2;
+        constexpr bool DOWN_UPFRONT = PROJECT && !ROWS && RT_MAX <= 2;
         bf16x8_t dn[DOWN_UPFRONT ? 4 : 1][RT_MAX];
         if (ROWS) fetch_down(c + 1);
         if (DOWN_UPFRONT) {
@@ -196,7 +195,7 @@ __global__ void __launch_bounds__(64 * NW) quantize_fuse_lora_kernel(QuantParams
 #pragma unroll
                 for (int rt = 0; rt < RT_MAX; rt++) dn[i][rt] = load_down(c, i, rt);
         }
-        load_x(c + DEPTH * CSTEP, x_ahead);
+        load_x(c + DEPTH * cstep, x_ahead);
         __builtin_amdgcn_sched_barrier(0);
 
         // ---- the gated unit: 16 (value, gate) pairs of two loads become the 8 bf16 of one step
@@ -290,7 +289,7 @@ __global__ void __launch_bounds__(64 * NW) quantize_fuse_lora_kernel(QuantParams
         // ---- low-rank down projection on the raw activations (rank tiles beyond R repeat tile 0 into
         // accumulators that are never stored: cheaper than a branch per tile)
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int i = 0; i < (PROJECT ? 4 : 0); i++)
 #pragma unroll
             for (int rt = 0; rt < RT_MAX; rt++) {
                 bf16x8_t b;
@@ -309,10 +308,10 @@ __global__ void __launch_bounds__(64 * NW) quantize_fuse_lora_kernel(QuantParams
     };
 
     // wave w walks the chunks w, w + NW, ...; the ring of DEPTH + 1 register buffers is indexed statically
-    for (int c0 = cfirst;; c0 += (DEPTH + 1) * CSTEP) {
+    for (int c0 = cfirst;; c0 += (DEPTH + 1) * cstep) {
 #pragma unroll
         for (int s = 0; s <= DEPTH; s++) {
-            const int c = c0 + s * CSTEP;
+            const int c = c0 + s * cstep;
             if (c >= nchunks) goto walked;
             process(c, xv[s], xv[(s + DEPTH) % (DEPTH + 1)]);
         }
@@ -332,7 +331,7 @@ walked:
         return;
     }
     // ---- reduce the waves' partial projections and write lora_act[row][rank]
-    if (RT > 0) {
+    if (PROJECT && RT > 0) {
         if (QUANT && SMOOTH == 1) __syncthreads();  // the factors in LDS are not needed any more
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
@@ -352,6 +351,98 @@ walked:
             p.lora_out[(size_t)(row0 + row) * p.R + 16 * p.rt_base + rank] = sum;
         }
     }
+}
+
+template <int NW, bool GLU>
+struct TransposeArea {  // per wave: 16 rows of a chunk on their way from the load layout to the operand layout
+    uint8_t bytes[NW][16 * (GLU ? 32 : 16) * 16];
+};
+
+template <int NW, int MT, int RT_MAX, int DEPTH, bool FP4, int SMOOTH, bool GLU, bool ROWS, bool QUANT = true>
+__global__ void __launch_bounds__(64 * NW) quantize_fuse_lora_kernel(QuantParams p) {
+    __shared__ __attribute__((aligned(16))) TransposeArea<NW, GLU> area;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    quantize_rows<NW, MT, RT_MAX, DEPTH, FP4, SMOOTH, GLU, ROWS, QUANT, true>(p, ROWS ? 0 : wave, ROWS ? 1 : NW, area.bytes[wave]);
+}
+
+// The projection alone, onto the RTW rank tiles from rt0 on (the second one may lie beyond the rank: not stored), of the 16
+// rows 16 blockIdx.x ...: wave w takes the chunks w, w + NW, ..., DEPTH of them requested ahead, proj_down included (in
+// quantize_rows the quantizer covers the latency of its operands).  x goes from whole-line requests to the operand layout
+// through the wave's transposition area `tr` as there (fetched in the operand layout, 16 rows x 64 bytes per instruction:
+// 7.1 us against 5.4 at M = 256, K = 3072); the waves' sums meet in `red` and are added in ascending order.
+template <int NW, int DEPTH, int RTW>
+__device__ __forceinline__ void project_rows(const QuantParams &p, int rt0, uint8_t *tr, float *red) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    const int row0 = blockIdx.x * 16, nchunks = p.K / 128, RT_all = p.R / 16;
+    const int rt1 = rt0 + 1 < RT_all ? rt0 + 1 : rt0;
+    int rows_valid = (p.M < row0 + 16 ? p.M : row0 + 16) - row0;
+    rows_valid = rows_valid < 0 ? 0 : rows_valid;
+    const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(p.x + (size_t)row0 * p.K), 0, rows_valid * p.K * 2, RSRC_WORD3);
+    const __amdgpu_buffer_rsrc_t drsrc = __builtin_amdgcn_make_buffer_rsrc((void *)p.down, 0, p.K * p.R * 2, RSRC_WORD3);
+    const uint32_t x_voff = (uint32_t)((lane / 16) * p.K * 2 + (lane % 16) * 16);
+    auto rot = [](int row) { return row & 11; };
+
+    u32x4_t x[DEPTH + 1][4], d[DEPTH + 1][RTW][4];
+    auto load = [&](int c, auto S) {
+        constexpr int s = decltype(S)::value;
+        const uint32_t beyond = c < nchunks ? 0u : 0x80000000u;  // (reads zeros and touches no memory, see quantize_rows)
+        each(std::make_integer_sequence<int, 4>{}, [&](auto I) {
+            constexpr int i = decltype(I)::value;
+            x[s][i] = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, (x_voff | beyond) + (uint32_t)(4 * i * p.K * 2), c * 256, 0);
+            d[s][0][i] = __builtin_amdgcn_raw_buffer_load_b128(drsrc, (uint32_t)(lane * 16) | beyond, ((c * 4 + i) * RT_all + rt0) * 1024, 0);
+            if constexpr (RTW > 1) d[s][1][i] = __builtin_amdgcn_raw_buffer_load_b128(drsrc, (uint32_t)(lane * 16) | beyond, ((c * 4 + i) * RT_all + rt1) * 1024, 0);
+        });
+    };
+    float4_t acc[2] = {float4_t{0.f, 0.f, 0.f, 0.f}, float4_t{0.f, 0.f, 0.f, 0.f}};
+    each(std::make_integer_sequence<int, DEPTH>{}, [&](auto D) { load(wave + decltype(D)::value * NW, D); });
+    // (chunks past the end multiply zeros: whole turns of the ring)
+    for (int c = wave; c < nchunks; c += (DEPTH + 1) * NW) {
+        each(std::make_integer_sequence<int, DEPTH + 1>{}, [&](auto S) {
+            constexpr int s = decltype(S)::value;
+            load(c + (s + DEPTH) * NW, std::integral_constant<int, (s + DEPTH) % (DEPTH + 1)>{});
+            __builtin_amdgcn_sched_barrier(0);
+            each(std::make_integer_sequence<int, 4>{}, [&](auto I) {
+                constexpr int i = decltype(I)::value;
+                const int row = 4 * i + lane / 16;
+                *(u32x4_t *)(tr + row * 256 + ((lane + rot(row)) % 16) * 16) = x[s][i];
+            });
+            each(std::make_integer_sequence<int, 4>{}, [&](auto I) {
+                constexpr int i = decltype(I)::value;
+                x[s][i] = *(const u32x4_t *)(tr + r * 256 + ((4 * q + i + rot(r)) % 16) * 16);
+                acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[s][i]), __builtin_bit_cast(bf16x8_t, d[s][0][i]), acc[0], 0, 0, 0);
+                if constexpr (RTW > 1) acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[s][i]), __builtin_bit_cast(bf16x8_t, d[s][1][i]), acc[1], 0, 0, 0);
+            });
+        });
+    }
+    __syncthreads();  // (`red` lies where the waves' transposition areas do)
+    *(float4_t *)&red[(wave * 2 * 64 + lane) * 4] = acc[0];
+    *(float4_t *)&red[((wave * 2 + 1) * 64 + lane) * 4] = acc[1];
+    __syncthreads();
+    // 512 sums: rank tile, row and rank of it by the result layout of the 16 x 16 matrix instruction
+    for (int idx = threadIdx.x; idx < 256 * RTW; idx += 64 * NW) {
+        const int rank = idx & 15, row = (idx >> 4) & 15, rt = idx >> 8;
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; w++) sum += red[((w * 2 + rt) * 64 + 16 * (row / 4) + rank) * 4 + row % 4];
+        if (rt0 + rt < RT_all) p.lora_out[(size_t)(row0 + row) * p.R + 16 * (rt0 + rt) + rank] = sum;
+    }
+}
+
+// Few rows (dispatch: up to 8 per compute unit).  One workgroup per 16 rows leaves most of the chip idle while eight waves
+// walk K, about 1 us per chunk of 128 columns, most of it the quantizer's arithmetic.  Nothing ties the codes of one
+// chunk to those of another, or to the projection: blockIdx.y < p.splits quantize a share of the chunks each, the
+// workgroups behind them project the same rows onto RTW rank tiles each, so that all ranks take one launch.  What is left is
+// launch, two or three memory latencies and, for long rows, the projection's walk over K.  Before / now: K = 3072, rank 32:
+// M = 256 6.9 / 4.4 us, M = 1024 8.1 / 5.4, M = 2048 8.8 / 7.2; K = 12288: M = 256 18.1 / 8.8, M = 1024 23.3 / 12.5;
+// rank 128: M = 256, K = 3072 18.7 / 4.6, M = 1024, K = 12288 107 / 21; rank 256: M = 256 36 / 5.7.
+template <int NW, int RTW, bool FP4, bool SMOOTH>
+__global__ void __launch_bounds__(64 * NW) quantize_few_rows_kernel(QuantParams p) {
+    __shared__ __attribute__((aligned(16))) TransposeArea<NW, false> area;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if ((int)blockIdx.y < p.splits) quantize_rows<NW, 1, 1, 1, FP4, SMOOTH ? 2 : 0, false, false, true, false>(p, blockIdx.y * NW + wave, p.splits * NW, area.bytes[wave]);
+    else project_rows<NW, RTW == 1 ? 2 : 1, RTW>(p, ((int)blockIdx.y - p.splits) * RTW, area.bytes[wave], (float *)area.bytes);
 }
 
 constexpr size_t SMOOTH_LDS_MAX = 64 * 1024;  // two workgroups of a compute unit must fit side by side
@@ -390,6 +481,14 @@ int project_further(const QuantParams &p0, hipStream_t stream) {
     return SVDQ_OK;
 }
 
+template <int RTW, bool FP4>
+int launch_few_rows(const QuantParams &p, hipStream_t stream) {
+    const dim3 grid(p.M_pad / 16, p.splits + (p.R / 16 + RTW - 1) / RTW);
+    if (p.smooth_rcp) SVDQ_LAUNCH((quantize_few_rows_kernel<8, RTW, FP4, true>), grid, dim3(512), 0, stream, p);
+    else SVDQ_LAUNCH((quantize_few_rows_kernel<8, RTW, FP4, false>), grid, dim3(512), 0, stream, p);
+    return check_launch("quantize_w4a4_act_fuse_lora (few rows)");
+}
+
 template <bool FP4, bool GLU>
 int dispatch(const QuantParams &p, hipStream_t stream) {
     // Rows and waves per workgroup by shape and rank, from measurements (below).
@@ -404,6 +503,20 @@ int dispatch(const QuantParams &p, hipStream_t stream) {
     } else {
         int dev = 0;
         const int ncu = hipGetDevice(&dev) == hipSuccess && compute_units(dev) > 0 ? compute_units(dev) : 256;
+        // Up to 8 rows per compute unit: quantizing and projecting workgroups apart, about one workgroup per compute unit (M = 1024,
+        // rank 32: 256 workgroups 5.4 us, 320 6.4).  One rank tile per projecting workgroup where they all fit beside the
+        // quantizing ones (M = 256: 4.4 us, with two 5.5), otherwise two; at ranks above 32 at least three shares of the
+        // quantizing (M = 1024, rank 128: 7.9 us, with one 10.4).  From 16 rows per compute unit on the forms below are
+        // faster (M = 4096: 11.5 us against 13.0).
+        if (p.M_pad <= 8 * ncu) {
+            QuantParams q = p;
+            const int row_blocks = p.M_pad / 16, most = (p.K / 128 + 7) / 8;
+            const bool one = row_blocks * (RT + 1) <= ncu;
+            q.splits = ncu / row_blocks - (one ? RT : (RT + 1) / 2);
+            if (q.splits < (RT > 2 ? 3 : 1)) q.splits = RT > 2 ? 3 : 1;
+            if (q.splits > most) q.splits = most;
+            return one ? launch_few_rows<1, FP4>(q, stream) : launch_few_rows<2, FP4>(q, stream);
+        }
         // High ranks with many rows: the waves split the rows (eight waves, 128 rows per workgroup) and share each chunk
         // of proj_down through LDS.  Ranks 80 ... 128, K = 3072: M = 18432 52.4 us (four waves on 32 rows each: 61.8; the
         // chunk-split forms 87 and more), M = 12288 51.3 against 58.3; below 32 rows per compute unit the chunk-split
@@ -411,9 +524,7 @@ int dispatch(const QuantParams &p, hipStream_t stream) {
         if (RT > 4 && RT <= 8 && (FP4 ? p.M_pad >= 128 * 128 : p.M_pad > 32 * ncu)) return launch<8, 1, 8, 1, FP4, false, true>(p, stream);
         if (RT > 2 && RT <= 4 && p.M_pad >= 256 * 64) return launch<8, 1, 4, 1, FP4, false, true>(p, stream);
         // Up to one 16-row workgroup per compute unit (256 of them) the walk over K is what takes the time: eight waves
-        // split it (M = 256 ... 4096 at K = 3072: 7.9 ... 10.1 us against 9.0 ... 11.3 with four; K = 12288, M = 256:
-        // 19.6 against 25.5).
-        // (two chunks requested ahead: the same at K = 3072, M = 256 and K = 12288: 16.5 us against 20.1)
+        // split it (M = 4096 at K = 3072: 10.1 us against 11.3 with four).
         if (RT <= 2 && p.M_pad <= 16 * ncu) return launch<8, 1, 2, 2, FP4, false>(p, stream);
         // Beyond that, at ranks up to 32 (measured at K = 3072 unless noted, on 256 compute units):
         //   up to two 16-row blocks per compute unit, and long rows at any M: eight waves on 32 rows, fewer workgroups
@@ -428,19 +539,12 @@ int dispatch(const QuantParams &p, hipStream_t stream) {
         if (RT <= 2 && (p.K > 6144 || p.M_pad >= 128 * ncu || (!FP4 && p.M_pad <= 32 * ncu))) return launch<8, 2, 2, 1, FP4, false>(p, stream);
         if (RT <= 2) return launch<4, 1, 2, 2, FP4, false>(p, stream);
         // Ranks 48 ... 128 below the row counts of the rows-split form: eight waves on 32 rows (M = 4608, K = 3072: rank
-        // 128 28.8 us, rank 64 16.0; four waves on the same rows 44.8 and 22.5; K = 12288, rank 128: 97 against 167);
-        // with few rows (up to 8 per compute unit) many small workgroups with two chunks ahead (M = 2048, rank 128: 18.9
-        // against 25.6; M = 256: 18.2 against 18.6).
-        const bool few_rows = p.M_pad <= 8 * ncu;
-        if (RT <= 4) return few_rows ? launch<4, 1, 4, 2, FP4, false>(p, stream) : launch<8, 2, 4, 1, FP4, false>(p, stream);
+        // 128 28.8 us, rank 64 16.0; four waves on the same rows 44.8 and 22.5; K = 12288, rank 128: 97 against 167).
+        if (RT <= 4) return launch<8, 2, 4, 1, FP4, false>(p, stream);
         // (NVFP4 at ranks 80 ... 128: the small workgroups at any row count, M = 4608: 29.7 us against 36.0, M = 12288: 57.7
         // against 71.1, K = 6144: 55.2 against 63.3; at rank 64 the large ones as for INT4, 16.5 against 25.1)
-        if (RT <= 8) return few_rows || FP4 ? launch<4, 1, 8, 2, FP4, false>(p, stream) : launch<8, 2, 8, 1, FP4, false>(p, stream);
+        if (RT <= 8) return FP4 ? launch<4, 1, 8, 2, FP4, false>(p, stream) : launch<8, 2, 8, 1, FP4, false>(p, stream);
         // ranks above 128: the first 128 with the codes, the rest in further launches over the same rows
-        if (few_rows) {
-            const int rc = launch<4, 1, 8, 2, FP4, false>(p, stream);
-            return rc != SVDQ_OK ? rc : project_further<4, 1, 2, false>(p, stream);
-        }
         const int rc = launch<8, 2, 8, 1, FP4, false>(p, stream);
         return rc != SVDQ_OK ? rc : project_further<8, 2, 1, false>(p, stream);
     }
@@ -469,6 +573,7 @@ extern "C" int svdq_quantize_w4a4_act_fuse_lora(const svdq_quantize_args *a, voi
     p.smooth_rcp = a->smooth_rcp;
     p.M = (int)a->M; p.M_pad = (int)a->M_pad; p.K = (int)a->K; p.R = (int)a->R;
     p.rt_base = 0;
+    p.splits = 0;
     hipStream_t s = (hipStream_t)stream;
     if (a->fuse_glu) return a->fp4 ? dispatch<true, true>(p, s) : dispatch<false, true>(p, s);
     return a->fp4 ? dispatch<true, false>(p, s) : dispatch<false, false>(p, s);

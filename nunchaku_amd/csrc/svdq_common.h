@@ -6,6 +6,9 @@
 #include <stdio.h>
 #include <stdarg.h>
 
+#include <type_traits>
+#include <utility>
+
 #include "../../include/svdq_amd.h"
 
 namespace svdq {
@@ -63,6 +66,12 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef float float16_t __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+
+// f(0), f(1), ... with compile-time arguments: arrays that such code indexes stay in registers
+template <int... I, typename F>
+__device__ inline void each(std::integer_sequence<int, I...>, F &&f) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
 
 // ---- bf16 <-> fp32 bit helpers ------------------------------------------------------------------
 __host__ __device__ inline float bf16_bits_to_f32(uint32_t b) {

@@ -246,3 +246,21 @@ def _check_row_sample(dev, M, K, R, fp4, smooth):
     assert (la[rows] - want_la[:n]).abs().max().item() <= 2e-5 * want_la.abs().max().item() + 1e-6
     assert (codes[M:] == 0).all() and (osc.float()[:, M:] == 0).all() and (la[M:] == 0).all()
     assert not torch.isnan(la).any()
+
+
+@pytest.mark.parametrize("M,K,R,fp4,smooth", [(1, 128, 16, False, True), (250, 1152, 48, False, True), (33, 3200, 0, False, False), (600, 2176, 80, True, True),
+                                              (257, 9216, 32, True, False), (700, 512, 272, False, True), (2048, 1152, 32, False, True), (2000, 384, 144, True, True)])
+def test_few_rows_split_into_quantizing_and_projecting_workgroups(dev, M, K, R, fp4, smooth):
+    """Up to 8 rows per compute unit: one chunk, fewer chunks than waves, counts of chunks that neither the shares nor the
+    projection's ring divide; one rank tile per projecting workgroup and two, with a rank tile left over (ranks 48, 80, 144,
+    272); no low-rank branch; no smoothing; both precisions."""
+    announce(f"quantize few rows M={M} K={K} R={R} fp4={fp4} smooth={smooth}")
+    if M >= 1000:
+        return _check_row_sample(dev, M, K, R, fp4, smooth)
+    layer = synth.make_layer(128, K, R, seed=R + K, fp4=fp4)
+    x = synth.make_activations(M, K, seed=M + K)
+    codes, osc, la = _run(dev, x, layer, fp4=fp4, smooth=smooth)
+    _check(x, layer, codes, osc, la, fp4=fp4, smooth=smooth) if R else None
+    if not R:
+        want_codes, want_scales, _ = olin.quantize_act_fuse_lora(x, layer.proj_down, None, fp4=fp4)
+        assert torch.equal(codes, want_codes) and torch.equal(osc.view(torch.int16), want_scales.view(torch.int16))
