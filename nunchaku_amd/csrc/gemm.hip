@@ -54,26 +54,43 @@ __global__ void zero_f32_kernel(float *p, int64_t n) {
     else for (int64_t j = i; j < n; j++) p[j] = 0.f;
 }
 
-// Sums the shares that the column blocks (INT4 kernel: 256 columns each) or chunks (NVFP4 kernel: 128 columns) of a
-// GEMM launch left for the next layer's low-rank projection, in ascending order, and writes lora_act [M_pad][R]
-// row-major.  A share is [M_pad / 32 slabs][R / 16 rank tiles][2 halves of 16 rows][64 lanes] x float4, lane l holding
-// rows 4 (l / 16) + [0, 4), rank l % 16 of a 16 x 16 tile (the result registers of the matrix instruction).
-__global__ void __launch_bounds__(256) reduce_shares_kernel(const float4_t *part, float *out, int nshares, int M_pad, int R) {
-    const int RT = R / 16, quads = M_pad * R / 4;
-    const int item = blockIdx.x * 256 + threadIdx.x;
-    if (item >= quads) return;
+// The sum of float4 number `item` over n shares that lie `stride` float4 apart, worked out by the eight threads of a
+// workgroup that have the same threadIdx.x % 32: each adds an eighth of the shares in ascending order, eight requests in
+// flight, and the first of them adds the eighths in ascending order.  `item` of the threads without work is any valid one.
+// Valid in the workgroup's first 32 threads.
+__device__ inline float4_t sum_of_shares(const float4_t *part, size_t item, size_t stride, int n) {
+    __shared__ float4_t eighth[8][32];
+    const int e = threadIdx.x >> 5, lane = threadIdx.x & 31;
+    const int first = n * e / 8, last = n * (e + 1) / 8;
     float4_t sum = float4_t{0.f, 0.f, 0.f, 0.f};
-    for (int b0 = 0; b0 < nshares; b0 += 8) {  // eight requests in flight
+    for (int b0 = first; b0 < last; b0 += 8) {
         float4_t v[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) v[u] = part[(size_t)(b0 + u < nshares ? b0 + u : nshares - 1) * quads + item];
+        for (int u = 0; u < 8; u++) v[u] = part[(size_t)(b0 + u < last ? b0 + u : last - 1) * stride + item];
 #pragma unroll
         for (int u = 0; u < 8; u++)
-            if (b0 + u < nshares) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) sum[e] += v[u][e];
-            }
+            if (b0 + u < last) sum += v[u];
     }
+    eighth[e][lane] = sum;
+    __syncthreads();
+    if (e == 0) {
+#pragma unroll
+        for (int u = 1; u < 8; u++) sum += eighth[u][lane];
+    }
+    return sum;
+}
+
+// Sums the shares that the column blocks (INT4 kernel: 256 columns each) or chunks (NVFP4 and few-rows kernels: 128 columns)
+// of a GEMM launch left for the next layer's low-rank projection, and writes lora_act [M_pad][R] row-major.  A share is
+// [M_pad / 32 slabs][R / 16 rank tiles][2 halves of 16 rows][64 lanes] x float4, lane l holding rows 4 (l / 16) + [0, 4),
+// rank l % 16 of a 16 x 16 tile (the result registers of the matrix instruction).
+// Bound by latency at few rows, where one thread per sum had 6 to 12 rounds of requests to wait for: 96 shares of 1280 rows, rank
+// 32, 11.5 us before and 5.5 now; 48 shares of 4608 rows (28 MB) 6.2 and 6.2.
+__global__ void __launch_bounds__(256) reduce_shares_kernel(const float4_t *part, float *out, int nshares, int M_pad, int R) {
+    const int RT = R / 16, quads = M_pad * R / 4;  // (M_pad is a multiple of 256 and R of 16: whole workgroups)
+    const int item = blockIdx.x * 32 + (threadIdx.x & 31);
+    const float4_t sum = sum_of_shares(part, item, quads, nshares);
+    if (threadIdx.x >= 32) return;
     const int ln = item & 63, m2 = (item >> 6) & 1, rest = item >> 7;  // rest = slab * RT + rank tile
     const int rt = rest % RT, slab32 = rest / RT;
     const int row = slab32 * 32 + 16 * m2 + 4 * (ln >> 4), rank = 16 * rt + (ln & 15);
@@ -84,38 +101,23 @@ __global__ void __launch_bounds__(256) reduce_shares_kernel(const float4_t *part
 // Sums the linear-attention shares of the row blocks of a GEMM launch (gemm_params.h; per row block and head 1056 floats:
 // the 32 x 32 part [i][j] in the order of the matrix instruction's result registers, element e of lane l at
 // ((e / 4) * 64 + l) * 4 + e % 4 with i = 8 (e / 4) + 4 (l / 32) + e % 4, j = l % 32; then the 32 column sums) into
-// out_vk [batch][head][33][32].
-__global__ void __launch_bounds__(256) reduce_vk_kernel(const float *part, float *out, int batch, int blocks_per_batch, int heads) {
-    // 64 outputs per workgroup; the row blocks of an output are split over four threads (more requests in flight),
-    // whose sums are added in ascending order
-    __shared__ float quarter[4][64];
-    const int idx = blockIdx.x * 64 + (threadIdx.x & 63), qt = threadIdx.x >> 6;
-    const bool live = idx < batch * heads * VK_HEAD_FLOATS;
-    float sum = 0.f;
-    if (live) {
-        const int pos = idx % VK_HEAD_FLOATS, head = (idx / VK_HEAD_FLOATS) % heads, b = idx / (VK_HEAD_FLOATS * heads);
-        int src = pos;  // row 32: stored as it is
-        if (pos < 1024) {
-            const int i = pos >> 5, j = pos & 31;
-            const int g = i >> 3, kb = (i >> 2) & 1, e3 = i & 3;
-            src = (g * 64 + kb * 32 + j) * 4 + e3;
-        }
-        const float *p0 = part + ((size_t)b * blocks_per_batch * heads + head) * VK_HEAD_FLOATS + src;
-        const size_t stride = (size_t)heads * VK_HEAD_FLOATS;
-        const int per = (blocks_per_batch + 3) / 4, first = qt * per, last = first + per < blocks_per_batch ? first + per : blocks_per_batch;
-        for (int s0 = first; s0 < last; s0 += 8) {  // eight requests in flight
-            float v[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) v[u] = p0[(size_t)(s0 + u < last ? s0 + u : last - 1) * stride];
-#pragma unroll
-            for (int u = 0; u < 8; u++)
-                if (s0 + u < last) sum += v[u];
-        }
+// out_vk [batch][head][33][32].  A workgroup's 32 float4 are 4 rows i of all 32 columns j, or the 8 of the column sums.
+__global__ void __launch_bounds__(256) reduce_vk_kernel(const float4_t *part, float *out, int blocks_per_batch, int heads) {
+    constexpr int QUADS = VK_HEAD_FLOATS / 4, PIECES = (QUADS + 31) / 32;
+    const int piece = blockIdx.x % PIECES, head = (blockIdx.x / PIECES) % heads, b = blockIdx.x / (PIECES * heads);
+    const int lane = threadIdx.x & 31, quad = piece * 32 + lane;
+    const size_t item = ((size_t)b * blocks_per_batch * heads + head) * QUADS + (quad < QUADS ? quad : QUADS - 1);
+    const float4_t sum = sum_of_shares(part, item, (size_t)heads * QUADS, blocks_per_batch);
+    if (threadIdx.x >= 32 || quad >= QUADS) return;
+    float *o = out + ((size_t)b * heads + head) * VK_HEAD_FLOATS;
+    if (piece == PIECES - 1) {
+        *(float4_t *)(o + 1024 + 4 * lane) = sum;
+        return;
     }
-    quarter[qt][threadIdx.x & 63] = sum;
-    __syncthreads();
-    if (live && qt == 0) out[idx] = ((quarter[0][threadIdx.x] + quarter[1][threadIdx.x]) + quarter[2][threadIdx.x]) + quarter[3][threadIdx.x];
+#pragma unroll
+    for (int e = 0; e < 4; e++) o[(4 * piece + e) * 32 + lane] = sum[e];  // (pieces 2 g and 2 g + 1 are lanes 0-31 and 32-63 of group g)
 }
+static_assert(VK_HEAD_FLOATS == 33 * 32, "eight whole pieces of the 32 x 32 part, then the column sums");
 
 void clear_zero_region(Workspace *w) {
     const int64_t n = (int64_t)(w->zero_bytes / 4);
@@ -231,15 +233,14 @@ template <typename P>
 int add_shares(const P &p, int nshares, int vk_block, hipStream_t st) {
     if (p.next_down) {
         const int quads = p.M_pad * p.R_down / 4;
-        SVDQ_LAUNCH(reduce_shares_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, (const float4_t *)p.next_lora_part,
+        SVDQ_LAUNCH(reduce_shares_kernel, dim3((unsigned)(quads / 32)), dim3(256), 0, st, (const float4_t *)p.next_lora_part,
                     p.next_lora_out, nshares, p.M_pad, p.R_down);
         const int rc = check_launch("gemm_w4a4 (low-rank shares)");
         if (rc != SVDQ_OK) return rc;
     }
     if (p.vk) {
-        const int heads = p.N / 96, n = (p.M_pad / p.vk_rows) * heads * VK_HEAD_FLOATS;
-        SVDQ_LAUNCH(reduce_vk_kernel, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, st, (const float *)p.vk_part, p.vk, p.M_pad / p.vk_rows,
-                    p.vk_rows / vk_block, heads);
+        const int heads = p.N / 96, batch = p.M_pad / p.vk_rows;
+        SVDQ_LAUNCH(reduce_vk_kernel, dim3((unsigned)(batch * heads * 9)), dim3(256), 0, st, (const float4_t *)p.vk_part, p.vk, p.vk_rows / vk_block, heads);
         return check_launch("gemm_w4a4 (linear-attention sums)");
     }
     return SVDQ_OK;
