@@ -102,12 +102,16 @@ __global__ void __launch_bounds__(256) reduce_shares_kernel(const float4_t *part
 // the 32 x 32 part [i][j] in the order of the matrix instruction's result registers, element e of lane l at
 // ((e / 4) * 64 + l) * 4 + e % 4 with i = 8 (e / 4) + 4 (l / 32) + e % 4, j = l % 32; then the 32 column sums) into
 // out_vk [batch][head][33][32].  A workgroup's 32 float4 are 4 rows i of all 32 columns j, or the 8 of the column sums.
-__global__ void __launch_bounds__(256) reduce_vk_kernel(const float4_t *part, float *out, int blocks_per_batch, int heads) {
+// The shares are those of row blocks of vk_block rows up to row `full_rows` and of 64 rows from there on; a batch entry is
+// vk_rows of them.
+__global__ void __launch_bounds__(256) reduce_vk_kernel(const float4_t *part, float *out, int vk_rows, int vk_block, int full_rows, int heads) {
     constexpr int QUADS = VK_HEAD_FLOATS / 4, PIECES = (QUADS + 31) / 32;
     const int piece = blockIdx.x % PIECES, head = (blockIdx.x / PIECES) % heads, b = blockIdx.x / (PIECES * heads);
     const int lane = threadIdx.x & 31, quad = piece * 32 + lane;
-    const size_t item = ((size_t)b * blocks_per_batch * heads + head) * QUADS + (quad < QUADS ? quad : QUADS - 1);
-    const float4_t sum = sum_of_shares(part, item, (size_t)heads * QUADS, blocks_per_batch);
+    auto slots_before = [&](int row) { return row <= full_rows ? row / vk_block : full_rows / vk_block + (row - full_rows) / 64; };
+    const int slot = slots_before(b * vk_rows);
+    const size_t item = ((size_t)slot * heads + head) * QUADS + (quad < QUADS ? quad : QUADS - 1);
+    const float4_t sum = sum_of_shares(part, item, (size_t)heads * QUADS, slots_before((b + 1) * vk_rows) - slot);
     if (threadIdx.x >= 32 || quad >= QUADS) return;
     float *o = out + ((size_t)b * heads + head) * VK_HEAD_FLOATS;
     if (piece == PIECES - 1) {
@@ -228,9 +232,10 @@ bool acquire_workspace(bool noalloc, int dev, hipStream_t st, size_t zero_bytes,
 }
 
 // The small kernels behind a GEMM that left shares in the workspace: the shares of the next layer's low-rank projection
-// (one per column block) and the linear-attention sums (one per vk_block rows), each added in ascending order.
+// (one per column block) and the linear-attention sums (one per vk_block rows, from row `full_rows` on one per 64), each
+// added in ascending order.
 template <typename P>
-int add_shares(const P &p, int nshares, int vk_block, hipStream_t st) {
+int add_shares(const P &p, int nshares, int vk_block, int full_rows, hipStream_t st) {
     if (p.next_down) {
         const int quads = p.M_pad * p.R_down / 4;
         SVDQ_LAUNCH(reduce_shares_kernel, dim3((unsigned)(quads / 32)), dim3(256), 0, st, (const float4_t *)p.next_lora_part,
@@ -240,7 +245,7 @@ int add_shares(const P &p, int nshares, int vk_block, hipStream_t st) {
     }
     if (p.vk) {
         const int heads = p.N / 96, batch = p.M_pad / p.vk_rows;
-        SVDQ_LAUNCH(reduce_vk_kernel, dim3((unsigned)(batch * heads * 9)), dim3(256), 0, st, (const float4_t *)p.vk_part, p.vk, p.vk_rows / vk_block, heads);
+        SVDQ_LAUNCH(reduce_vk_kernel, dim3((unsigned)(batch * heads * 9)), dim3(256), 0, st, (const float4_t *)p.vk_part, p.vk, p.vk_rows, vk_block, full_rows, heads);
         return check_launch("gemm_w4a4 (linear-attention sums)");
     }
     return SVDQ_OK;
@@ -255,13 +260,10 @@ int add_shares(const P &p, int nshares, int vk_block, hipStream_t st) {
 // again when compute units are shared.  Measured, whole / best split: 24 tiles at K = 3072 31.2 / 22.5 (4 parts; 3
 // parts 24.2), 72 tiles 31.3 / 27.3 (3), 96 tiles 31.8 / 31.0 (2; not split), 144 tiles 32.1 / 38.1 (not split);
 // K = 12288: 24 tiles 105.9 / 39.6 (6), 72 tiles 105.6 / 51.7 (3), 144 tiles 106.2 / 78.4 (3).
-// `time`: the model's time in us for the choice; beyond one tile per compute unit (288 tiles at K = 3072 45 us, 384 tiles
-// 52-56, 512 tiles 50, 1728 tiles 165) 0.83 us per k-group until two share every compute unit, then in proportion.
+// `time`: the model's time in us for the choice where there is one.
 int choose_kparts(int ntiles, int kgroups, int ncu, double *time) {
-    if (ntiles > ncu) {
-        *time = (0.83 * kgroups + 5.0) * (ntiles > 2 * ncu ? ntiles / (2.0 * ncu) : 1.0);
-        return 1;
-    }
+    *time = 0.0;
+    if (ntiles > ncu) return 1;
     int best = 1;
     double best_t = 0.55 * kgroups + 4.4;
     for (int k : {2, 3, 4, 6, 8}) {
@@ -282,6 +284,91 @@ int choose_kparts(int ntiles, int kgroups, int ncu, double *time) {
 bool needs_next_epilogue(const svdq_gemm_args *a) {
     return a->qout != nullptr || a->next_lora_down != nullptr || a->rotary_emb != nullptr || a->fuse_silu || a->out_vk != nullptr;
 }
+
+// Rows the call has to work out: those of `out` where nothing else is written, those the caller names where `out` is not
+// given, all of them otherwise.
+int rows_needed(const svdq_gemm_args *a) {
+    if (a->out_q || a->out_vk || (a->out && (a->qout || a->next_lora_down)) || a->M_out == 0) return (int)a->M_pad;
+    return (int)a->M_out;
+}
+
+// How the rows of an INT4 launch are divided into blocks of 128 rows, and blocks of 64 rows behind them, when the caller
+// leaves the split along K to the library.  The last tiles of a launch leave compute units idle for the time of a whole
+// tile (the hardware hands tiles to the emptiest compute unit; with 1296 tiles 16 of 256 work 22 us longer than the
+// others); in tiles of half the height the last rows fill them up.
+// A model of the busiest compute unit's time, in units of a whole tile alone on one, fitted to 600 launches of 70 shapes (M = 300
+// ... 9216, K = 1024 ... 12800, N = 1024 ... 21504): a pair of whole tiles side by side takes 1.55, of half tiles 0.9, a half tile alone
+// 0.7; a half tile next to a last odd whole one 1.1 together with it, two of them 2.0 (the second starts when the first is done).
+// Every compute unit gets `tiles / ncu` whole tiles or one more, the half tiles go where they end first.  Considered are whole
+// tiles only, whole tiles up to the last and the last but one multiple of the compute units, and (few tiles) half tiles only; a
+// division with half tiles has to be 4 % faster by the model.  Measured, whole tiles / the choice: M = 4608, K = 3072, N = 9216
+// 140 / 131 us; M = 4096, K = 2304, N = 6912 72.3 / 66.3; M = 1024, K = 3072, N = 9216 44.5 / 34.3; M = 505 of the same layer 32.9 / 28.7;
+// over the 70 shapes 1.16 times as fast, 1.4 % off the best division measured.
+double half_tiles_time(int n) { return 0.9 * (n / 2) + 0.7 * (n % 2); }
+double unit_time(int whole, int half) {
+    const double pairs = 1.55 * (whole / 2);
+    if (whole % 2 == 0) return pairs + half_tiles_time(half);
+    return pairs + (half == 0 ? 1.0 : half == 1 ? 1.1 : 2.0 + 0.25 * (half - 2));
+}
+double launch_time(long long whole, long long half, int ncu) {  // (in tiles)
+    const int q = (int)(whole / ncu);
+    const long long more = whole % ncu, fewer = ncu - more;  // compute units with q + 1 whole tiles, with q
+    double t = more ? unit_time(q + 1, 0) : unit_time(q, 0);
+    for (int h0 = 0, h1 = 0;;) {  // half tiles on each unit of either kind that end by t
+        while (unit_time(q, h0 + 1) <= t) h0++;
+        while (unit_time(q + 1, h1 + 1) <= t) h1++;
+        if (h0 * fewer + h1 * more >= half) return t;
+        const double t0 = unit_time(q, h0 + 1), t1 = unit_time(q + 1, h1 + 1);
+        t = more && t1 < t0 ? t1 : t0;
+    }
+}
+// Returns the time in us: 8 + 0.51 per k-group and tile (one tile or less per compute unit: 18 us at K = 1280, 26.5 at K = 2304, 107 at
+// K = 12288).
+double choose_row_blocks(int rows, int nblocks, int kgroups, int ncu, int *full_blocks, int *half_blocks) {
+    const int units = (rows + 63) / 64, all = (units + 1) / 2;
+    const long long tiles = (long long)all * nblocks;
+    const int q = (int)((tiles - 1) / ncu);
+    double best = launch_time(tiles, 0, ncu);
+    *full_blocks = all;
+    *half_blocks = 0;
+    double to_beat = 0.96 * best;
+    auto consider = [&](int full) {
+        if (full > units / 2) full = units / 2;
+        const int half = units - 2 * full;
+        if (half == 0) return;
+        const double t = launch_time((long long)full * nblocks, (long long)half * nblocks, ncu);
+        if (t > to_beat) return;
+        to_beat = t;
+        best = t;
+        *full_blocks = full;
+        *half_blocks = half;
+    };
+    consider((int)((long long)q * ncu / nblocks));
+    if (q >= 1) consider((int)((long long)(q - 1) * ncu / nblocks));
+    if (tiles <= 2 * ncu) consider(0);
+    return 8.0 + 0.51 * kgroups * best;
+}
+
+// How the tiles of an INT4 launch are laid out: split along K (kparts > 1) or in row blocks of two heights; returns the time by
+// the models.
+double choose_tiles_int4(const svdq_gemm_args *a, int ncu, int *full_blocks, int *half_blocks, int *kparts) {
+    const int nblocks = (int)((a->N + g6::BN - 1) / g6::BN), kgroups = (int)(a->K / 64);
+    double t_split;
+    *kparts = choose_kparts((int)(a->M_pad / g6::BM) * nblocks, kgroups, ncu, &t_split);
+    t_split = 0.96 * t_split + 2.8;  // (144 tiles, one per compute unit: 15.6 us at K = 1024, 33 at K = 3072, 105 at K = 12288)
+    const double t_rows = choose_row_blocks(rows_needed(a), nblocks, kgroups, ncu, full_blocks, half_blocks);
+    if (*kparts > 1 && t_split < t_rows) {
+        *full_blocks = (int)(a->M_pad / g6::BM);
+        *half_blocks = 0;
+        return t_split;
+    }
+    *kparts = 1;
+    return t_rows;
+}
+
+// Workspace: every row block's linear-attention sums; every column block's share of the next layer's low-rank projection.
+size_t vk_share_bytes(const svdq_gemm_args *a, long long row_blocks) { return (size_t)row_blocks * (a->N / 96) * VK_HEAD_FLOATS * 4; }
+size_t lora_share_bytes(const svdq_gemm_args *a, long long column_blocks) { return (size_t)column_blocks * a->M_pad * a->R_down * 4; }
 
 // The argument block of the NVFP4 kernel and of the few-rows kernels.
 void fill_params(const svdq_gemm_args *a, GemmParams &p) {
@@ -365,18 +452,33 @@ int gemm_int4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool no
     p.gelu = a->qout != nullptr;  // the GELU is composed exactly when the next layer's input is produced (launch_impl.cuh:282-309)
 
     // One workgroup per 128 x 256 output tile (or per part of one split along K), two resident per compute unit.
-    const int mblocks = p.M_pad / g6::BM, nblocks = (p.N + g6::BN - 1) / g6::BN;
-    const int ntiles = mblocks * nblocks, kgroups = p.K / 64;
-    double model_time;
-    const int kparts = a->k_split > 0 ? (int)(a->k_split < kgroups ? a->k_split : kgroups) : choose_kparts(ntiles, kgroups, ncu, &model_time);
-    p.kparts = kparts;
-    // bands of about ten row blocks, all of the same height where the count allows it
-    p.band = (mblocks + (mblocks + 9) / 10 - 1) / ((mblocks + 9) / 10);
+    const int nblocks = (p.N + g6::BN - 1) / g6::BN, kgroups = p.K / 64;
+    p.full_blocks = p.M_pad / g6::BM;
+    p.half_blocks = 0;
+    p.kparts = 1;
+    if (a->k_split > 0) {
+        p.kparts = (int)(a->k_split < kgroups ? a->k_split : kgroups);
+    } else {
+        choose_tiles_int4(a, ncu, &p.full_blocks, &p.half_blocks, &p.kparts);
+        if (noalloc && a->out_vk && vk_share_bytes(a, p.full_blocks + p.half_blocks) > NOALLOC_SCRATCH_BYTES) {
+            // (more row blocks, more shares: not where only 128-row blocks' fit the fixed scratch)
+            p.full_blocks = (int)(a->M_pad / g6::BM);
+            p.half_blocks = 0;
+        }
+    }
+    const int kparts = p.kparts, ntiles = (p.full_blocks + p.half_blocks) * nblocks;
+    // bands of about ten 128-row blocks, all of the same height where the count allows it
+    auto band_height = [](int blocks, int most) {
+        const int bands = (blocks + most - 1) / most;
+        return bands > 0 ? (blocks + bands - 1) / bands : 1;
+    };
+    p.band = band_height(p.full_blocks, 10);
+    p.half_band = band_height(p.half_blocks, 20);
     const bool next = needs_next_epilogue(a);
     const size_t cnt_bytes = (size_t)ntiles * 4;
     const size_t part_bytes = kparts > 1 ? (size_t)ntiles * kparts * g6::BM * g6::BN * 4 : 0;
-    const size_t share_bytes = p.next_down ? (size_t)nblocks * p.M_pad * p.R_down * 4 : 0;  // every column block's share of the next projection
-    const size_t vk_bytes = p.vk ? (size_t)(p.M_pad / g6::BM) * (p.N / 96) * VK_HEAD_FLOATS * 4 : 0;  // every row block's linear-attention sums
+    const size_t share_bytes = p.next_down ? lora_share_bytes(a, nblocks) : 0;  // every column block's share of the next projection
+    const size_t vk_bytes = p.vk ? vk_share_bytes(a, p.full_blocks + p.half_blocks) : 0;  // every row block's linear-attention sums
     if (kparts == 1 && !p.next_down && !p.vk) return next ? g6::launch_next(p, ntiles, st) : g6::launch_plain(p, ntiles, st);
     std::unique_lock<std::mutex> lock(g_ws_mutex, std::defer_lock);
     if (!noalloc) lock.lock();
@@ -389,7 +491,7 @@ int gemm_int4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool no
     p.next_lora_part = (float *)(w.scratch + part_bytes);
     p.vk_part = (float *)(w.scratch + part_bytes + share_bytes);
     int rc = next ? g6::launch_next(p, ntiles * kparts, st) : g6::launch_plain(p, ntiles * kparts, st);
-    if (rc == SVDQ_OK) rc = add_shares(p, nblocks, g6::BM, st);
+    if (rc == SVDQ_OK) rc = add_shares(p, nblocks, g6::BM, p.full_blocks * g6::BM, st);
     if (rc != SVDQ_OK && w.owner) w.owner->dirty = true;
     return rc;
 }
@@ -452,8 +554,8 @@ int gemm_fp4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool noa
         p.whole_band = (mblocks + nbands - 1) / nbands;
     }
     // every 128-column chunk's share of the next layer's low-rank projection, every row block's linear-attention sums
-    const size_t share_bytes = p.next_down ? (size_t)(p.N / 128) * p.M_pad * p.R_down * 4 : 0;
-    const size_t vk_bytes = p.vk ? (size_t)(p.M_pad / 32) * (p.N / 96) * VK_HEAD_FLOATS * 4 : 0;  // (this kernel: per 32-row slab)
+    const size_t share_bytes = p.next_down ? lora_share_bytes(a, a->N / 128) : 0;
+    const size_t vk_bytes = p.vk ? vk_share_bytes(a, a->M_pad / 32) : 0;  // (this kernel: per 32-row slab)
     if (!shared_tiles && !share_bytes && !vk_bytes) return next ? launch_gemm_fp4_v5(p, nwg, st) : launch_gemm_fp4_v4(p, nwg, st);
     std::unique_lock<std::mutex> lock(g_ws_mutex, std::defer_lock);
     if (!noalloc) lock.lock();
@@ -468,19 +570,12 @@ int gemm_fp4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool noa
     p.next_lora_part = (float *)(w.scratch + part_bytes);
     p.vk_part = (float *)(w.scratch + part_bytes + share_bytes);
     int rc = next ? launch_gemm_fp4_v5(p, nwg, st) : launch_gemm_fp4_v4(p, nwg, st);
-    if (rc == SVDQ_OK) rc = add_shares(p, p.N / 128, 32, st);
+    if (rc == SVDQ_OK) rc = add_shares(p, p.N / 128, 32, p.M_pad, st);
     if (rc != SVDQ_OK && w.owner) w.owner->dirty = true;
     return rc;
 }
 
 // ---- few rows, either precision: small tiles, operands straight to registers (gemm_direct_kernel.h) ------
-// Rows the call has to work out: those of `out` where nothing else is written, those the caller names where `out` is not
-// given, all of them otherwise.
-int rows_needed(const svdq_gemm_args *a) {
-    if (a->out_q || a->out_vk || (a->out && (a->qout || a->next_lora_down)) || a->M_out == 0) return (int)a->M_pad;
-    return (int)a->M_out;
-}
-
 // Which of the two shapes of the few-rows kernel (0: neither) a launch takes.  Shape 1: tiles of 32 rows, four waves split
 // K.  Shape 2: tiles of 64 rows, two waves split K and two the columns: 23 % fewer operand bytes per product, from about
 // 400 tiles of 32 rows on.  Both are models of the time in us fitted to launches at K = 1024, 3072 and 12288 on 256 compute
@@ -508,8 +603,8 @@ int choose_direct(const svdq_gemm_args *a, int ncu) {
         t1 = 4.3 + c1 * (1.1 + 0.127 * kg);
         t2 = 3.0 + c2 * (2.1 + 0.214 * kg);
     } else {
-        choose_kparts((int)(a->M_pad / g6::BM) * (int)((a->N + g6::BN - 1) / g6::BN), kg, ncu, &t_large);
-        t_large = 0.96 * t_large + 2.8;  // (144 tiles, one per compute unit: 15.6 us at K = 1024, 33 at K = 3072, 105 at K = 12288)
+        int full, half, kparts;
+        t_large = choose_tiles_int4(a, ncu, &full, &half, &kparts);
         t1 = 3.5 + c1 * (1.1 + 0.106 * kg);
         t2 = 3.3 + c2 * (1.6 + 0.158 * kg);
     }
@@ -528,8 +623,8 @@ int gemm_direct(const svdq_gemm_args *a, int shape, hipStream_t st, int dev, boo
         return next ? direct::launch_int4_next(p, shape, st) : direct::launch_int4_plain(p, shape, st);
     };
     // every 128-column chunk's share of the next layer's low-rank projection, every 32-row block's linear-attention sums
-    const size_t share_bytes = p.next_down ? (size_t)(p.N / 128) * p.M_pad * p.R_down * 4 : 0;
-    const size_t vk_bytes = p.vk ? (size_t)(p.M_pad / 32) * (p.N / 96) * VK_HEAD_FLOATS * 4 : 0;
+    const size_t share_bytes = p.next_down ? lora_share_bytes(a, a->N / 128) : 0;
+    const size_t vk_bytes = p.vk ? vk_share_bytes(a, a->M_pad / 32) : 0;
     if (!share_bytes && !vk_bytes) return launch();
     std::unique_lock<std::mutex> lock(g_ws_mutex, std::defer_lock);
     if (!noalloc) lock.lock();
@@ -538,7 +633,7 @@ int gemm_direct(const svdq_gemm_args *a, int shape, hipStream_t st, int dev, boo
     p.next_lora_part = (float *)w.scratch;
     p.vk_part = (float *)(w.scratch + share_bytes);
     int rc = launch();
-    if (rc == SVDQ_OK) rc = add_shares(p, p.N / 128, 32, st);
+    if (rc == SVDQ_OK) rc = add_shares(p, p.N / 128, 32, p.M_pad, st);
     return rc;
 }
 }  // namespace
@@ -623,7 +718,9 @@ int gemm_entry(const svdq_gemm_args *a, void *stream, bool noalloc) {
     if (hipGetDevice(&dev) != hipSuccess) return fail(SVDQ_ELAUNCH, "gemm: cannot identify the current device");
     const int ncu = compute_units(dev);
     if (ncu <= 0) return fail(SVDQ_ELAUNCH, "gemm: cannot query the number of compute units");
-    const int shape = choose_direct(a, ncu);
+    int shape = choose_direct(a, ncu);
+    // (its shares are those of 128 columns and 32 rows each: where they do not fit the fixed scratch, the kernels with larger tiles)
+    if (noalloc && (a->next_lora_down ? lora_share_bytes(a, a->N / 128) : 0) + (a->out_vk ? vk_share_bytes(a, a->M_pad / 32) : 0) > NOALLOC_SCRATCH_BYTES) shape = 0;
     if (shape) return gemm_direct(a, shape, (hipStream_t)stream, dev, noalloc);
     return a->fp4 ? gemm_fp4(a, (hipStream_t)stream, dev, ncu, noalloc) : gemm_int4(a, (hipStream_t)stream, dev, ncu, noalloc);
 }

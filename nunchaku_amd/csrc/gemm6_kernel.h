@@ -54,53 +54,51 @@ __device__ inline __amdgpu_buffer_rsrc_t partial_rsrc(const float *slot) {
     return __builtin_amdgcn_make_buffer_rsrc((void *)slot, 0, PARTIAL_SLOT_FLOATS * 4, 0x00020000);
 }
 
-template <bool NEXT>
-__global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
+// The output tile of 64 MT rows x 256 columns from (m0, 256 nb) on.  MT = 2 is the ordinary tile; MT = 1 (wave tile
+// 32 x 128) serves the last rows of a launch, see gemm6_kernel below.  `tile`, `part`: the tile's number and this workgroup's share
+// of its k-groups where tiles are split along K (MT = 2 only); `vk_slot`: the slot of its linear-attention sums.
+template <bool NEXT, int MT>
+__device__ __forceinline__ void output_tile(const Params &p, const int m0, const int nb, const int tile, const int part, const int vk_slot) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     const int r32 = lane & 31, h = lane >> 5;
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
-
-    // ---- which tile, which part of its k-groups ------------------------------------------------
-    // Workgroups go to the XCDs round robin (blockIdx % 8); the remap gives each XCD one contiguous run
-    // of tile numbers, and the tiles are numbered in bands of p.band row blocks (about ten), down the band
-    // first: the 64 workgroups resident on an XCD at one time then cover about 10 row blocks x 6 column
-    // blocks, whose operands (6 KB per row block and k-group, 14 KB per column block) they share in that
-    // XCD's L2.  Measured at 36 x 48 tiles, bytes fetched from beyond the L2 per launch: bands of 6 / 9 / 12 /
-    // 16 / 18 / 36 row blocks 317 / 296 / 308 / 355 / 396 / 604 MB (the time does not change: 169-171 us).
-    const int mblocks = p.M_pad / BM, nblocks = (p.N + BN - 1) / BN;
+    constexpr int TILE_M = 64 * MT;
     const int kgroups = p.K / 64;
-    const int total = (int)gridDim.x;
-    int v = (int)blockIdx.x;
-    if (total % 8 == 0) v = (v % 8) * (total / 8) + v / 8;
-    const int tile = v / p.kparts, part = v - tile * p.kparts;
-    const int BAND = p.band;
-    const int band = tile / (BAND * nblocks), in_band = tile - band * (BAND * nblocks);
-    const int band_rows = mblocks - band * BAND < BAND ? mblocks - band * BAND : BAND;
-    const int mb = band * BAND + in_band % band_rows, nb = in_band / band_rows;
-    const int gb = (int)((long long)kgroups * part / p.kparts);
-    const int ng = (int)((long long)kgroups * (part + 1) / p.kparts) - gb;
-    const int m0 = mb * BM, n0 = nb * BN;
+    const int kparts = MT == 2 ? p.kparts : 1;
+    const int gb = (int)((long long)kgroups * part / kparts);
+    const int ng = (int)((long long)kgroups * (part + 1) / kparts) - gb;
+    const int n0 = nb * BN;
+    const int mb = m0 / ACT_BLOCK_ROWS, slab0 = (m0 % ACT_BLOCK_ROWS) / 32;  // 128-row block of the fragment layout, first 32-row slab in it
 
     // ---- staging ---------------------------------------------------------------------------------
-    // Every wave issues COPIES_PER_WAVE copies per k-group: three consecutive 1 KB chunks of the weight
-    // fragments (one base, the instruction's offset field advances both the memory and the LDS address),
-    // one chunk of the activation fragments, one more of those (waves 0, 1) or of the weight scales
-    // (waves 2, 3), and the 256 bytes of activation scales (all four waves write the same bytes: the
-    // counts stay equal, which keeps the wait below a constant).  The four source pointers are
-    // wave-uniform and advance by a constant per k-group.
+    // Every wave issues the same number of copies per k-group, three of them consecutive 1 KB chunks of the weight
+    // fragments (one base, the instruction's offset field advances both the memory and the LDS address).  128 rows: one
+    // chunk of the activation fragments, one more of those (waves 0, 1) or of the weight scales (waves 2, 3), and the
+    // 256 bytes of activation scales (all four waves write the same bytes: the counts stay equal, which keeps the wait
+    // below a constant).  64 rows: one chunk of the activation fragments (waves 0-2) or of the weight scales (wave 3), then
+    // the 128 bytes of activation scales, eight times over in a whole chunk (waves 0-2: the same bytes), or the other chunk of
+    // weight scales (wave 3).  The source pointers are wave-uniform and advance by a constant per k-group.
+    constexpr int COPIES = MT == 2 ? COPIES_PER_WAVE : 5;
+    constexpr int ST_A = StageOf<MT>::A, ST_W = StageOf<MT>::W, ST_WS = StageOf<MT>::WS, ST_AS = StageOf<MT>::AS, ST_Z = StageOf<MT>::Z;
     const uint32_t copy_voff = lane * 16;
     const bool low = wave < 2;
+    const uint8_t *act0 = p.act + ((size_t)mb * kgroups + gb) * (4 * FRAG_BYTES) + slab0 * FRAG_BYTES;
+    const uint8_t *ws0 = p.wscales + ((size_t)nb * kgroups + gb) * 2048, *as0 = (const uint8_t *)(p.ascales + (size_t)gb * p.M_pad + m0);
+    const uint32_t stride_q = (uint32_t)p.M_pad * 2;
     const uint8_t *src_w = p.wgt + ((size_t)nb * kgroups + gb) * (8 * FRAG_BYTES) + wave * 3072;
-    const uint8_t *src_a = p.act + ((size_t)mb * kgroups + gb) * (4 * FRAG_BYTES) + wave * 1024;
-    const uint8_t *src_x = low ? p.act + ((size_t)mb * kgroups + gb) * (4 * FRAG_BYTES) + (4 + wave) * 1024
-                               : p.wscales + ((size_t)nb * kgroups + gb) * 2048 + (wave - 2) * 1024;
-    const uint8_t *src_q = (const uint8_t *)(p.ascales + (size_t)gb * p.M_pad + m0);
-    const uint32_t stride_x = low ? 4 * FRAG_BYTES : 2048, stride_q = (uint32_t)p.M_pad * 2;
-    const uint32_t dst_w = lds_base + ST_W + wave * 3072, dst_a = lds_base + ST_A + wave * 1024;
-    const uint32_t dst_x = lds_base + (low ? ST_A + (4 + wave) * 1024 : ST_WS + (wave - 2) * 1024), dst_q = lds_base + ST_AS;
+    const uint8_t *src_a = MT == 2 || wave < 3 ? act0 + wave * 1024 : ws0;
+    const uint8_t *src_x = MT == 2 ? (low ? act0 + (4 + wave) * 1024 : ws0 + (wave - 2) * 1024) : (wave < 3 ? as0 : ws0 + 1024);
+    const uint8_t *src_q = as0;  // (128 rows only)
+    const uint32_t stride_a = MT == 2 || wave < 3 ? 4 * FRAG_BYTES : 2048;
+    const uint32_t stride_x = MT == 2 ? (low ? 4 * FRAG_BYTES : 2048) : (wave < 3 ? stride_q : 2048);
+    const uint32_t dst_w = lds_base + ST_W + wave * 3072;
+    const uint32_t dst_a = lds_base + (MT == 2 || wave < 3 ? ST_A + wave * 1024 : ST_WS);
+    const uint32_t dst_x = lds_base + (MT == 2 ? (low ? ST_A + (4 + wave) * 1024 : ST_WS + (wave - 2) * 1024) : (wave < 3 ? ST_AS : ST_WS + 1024));
+    const uint32_t dst_q = lds_base + ST_AS;
+    const uint32_t x_voff = MT == 2 || wave == 3 ? lane * 16 : (lane & 7) * 16;
     // The requests of a k-group are issued one at a time, spread over the steps of the main loop: a wave
     // that issues its six requests back to back stands still until the memory pipeline has taken them,
     // about 30 cycles each.  First the three weight chunks (W), later the other three (R).
@@ -112,16 +110,18 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
             src_w += 8 * FRAG_BYTES;
         }
     };
-    auto copy_r = [&](uint32_t stage_off, int i) {  // the rest: activation chunk, activation / weight-scale chunk, activation scales
+    auto copy_r = [&](uint32_t stage_off, int i) {  // the other COPIES - 3
         if (i == 0) asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3" :: "s"(dst_a), "s"(stage_off), "v"(copy_voff), "s"(src_a) : "memory", "m0", "scc");
-        if (i == 1) asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3" :: "s"(dst_x), "s"(stage_off), "v"(copy_voff), "s"(src_x) : "memory", "m0", "scc");
-        if (i == 2) {
+        if (i == 1) asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3" :: "s"(dst_x), "s"(stage_off), "v"(x_voff), "s"(src_x) : "memory", "m0", "scc");
+        if (MT == 2 && i == 2) {
             uint32_t voff4;
             asm volatile("v_lshrrev_b32 %0, 2, %1" : "=v"(voff4) : "v"(copy_voff));
             asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, %3" :: "s"(dst_q), "s"(stage_off), "v"(voff4), "s"(src_q) : "memory", "m0", "scc");
-            src_a += 4 * FRAG_BYTES;
-            src_x += stride_x;
             src_q += stride_q;
+        }
+        if (i == COPIES - 4) {
+            src_a += stride_a;
+            src_x += stride_x;
         }
     };
 
@@ -130,10 +130,10 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
 
     // groups 0 and 1 entirely, the weights of group 2
     for (int i = 0; i < 3; i++) copy_w(0, i);
-    for (int i = 0; i < 3; i++) copy_r(0, i);
+    for (int i = 0; i < COPIES - 3; i++) copy_r(0, i);
     if (ng > 1) {
         for (int i = 0; i < 3; i++) copy_w(STAGE_BYTES, i);
-        for (int i = 0; i < 3; i++) copy_r(STAGE_BYTES, i);
+        for (int i = 0; i < COPIES - 3; i++) copy_r(STAGE_BYTES, i);
     }
     if (ng > 2)
         for (int i = 0; i < 3; i++) copy_w(2 * STAGE_BYTES, i);
@@ -141,9 +141,9 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
     // per-lane read offsets inside a stage
     const uint32_t off16 = lane * 16, off8 = 1024 + lane * 8;
     const uint32_t off_ws = ST_WS + (128 * wn + r32) * 8;
-    const uint32_t off_as = h ? ST_Z : ST_AS + (64 * wm + r32) * 2;
+    const uint32_t off_as = h ? ST_Z : ST_AS + (32 * MT * wm + r32) * 2;
     auto read_x = [&](uint32_t sb, int mt, Frag &f, uint32_t &as) {
-        const uint8_t *base = lds + sb + ST_A + (2 * wm + mt) * FRAG_BYTES;
+        const uint8_t *base = lds + sb + ST_A + (MT * wm + mt) * FRAG_BYTES;
         f.lo = *(const u32x4_t *)(base + off16);
         f.hi = *(const u32x2_t *)(base + off8);
         as = *(const uint16_t *)(lds + sb + off_as + mt * 64);
@@ -155,25 +155,29 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
         ws = *(const u32x2_t *)(lds + sb + off_ws + nt * 256);
     };
 
-    float16_t acc[8];  // tile t = 2 nt + mt
+    float16_t acc[4 * MT];  // tile t = MT nt + mt
 #pragma unroll
-    for (int t = 0; t < 8; t++)
+    for (int t = 0; t < 4 * MT; t++)
 #pragma unroll
         for (int e = 0; e < 16; e++) acc[t][e] = 0.f;
 
     // group 0 has landed
-    if (ng > 2) asm volatile("s_waitcnt vmcnt(9)" ::: "memory");
-    else if (ng > 1) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+    if (ng > 2) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(COPIES + 3) : "memory");
+    else if (ng > 1) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(COPIES) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
 
-    Frag X[2], W[2];
-    u32x2_t wsop[2];
-    uint32_t asop[2];
+    Frag X[MT], W[MT == 2 ? 2 : 4];
+    u32x2_t wsop[MT == 2 ? 2 : 4];
+    uint32_t asop[MT];
     float16_t P[2], F[2];
     read_x(0, 0, X[0], asop[0]);
-    read_x(0, 1, X[1], asop[1]);
+    if constexpr (MT == 2) read_x(0, 1, X[1], asop[1]);
     read_w(0, 0, W[0], wsop[0]);
+    if constexpr (MT == 1) {
+        read_w(0, 1, W[1], wsop[1]);
+        read_w(0, 2, W[2], wsop[2]);
+    }
     P[0] = mfma_codes(W[0], X[0]);
     F[0] = mfma_factor(wsop[0], asop[0]);
 
@@ -208,33 +212,57 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
         constexpr int MODE = decltype(MODE_T)::value;
         const uint32_t sb_next = sb == (STAGES - 1) * STAGE_BYTES ? 0 : sb + STAGE_BYTES;
         const uint32_t sb_prev = sb == 0 ? (STAGES - 1) * STAGE_BYTES : sb - STAGE_BYTES;
-        // step t issues the matrix instructions of tile t + 1 (tile = 2 nt + mt) and accumulates tile t
-        if (MODE >= 1) copy_r(sb_prev, 0);
-        SVDQ_STEP(0, 0, 1, W[0], X[1], wsop[0], asop[1], 3, read_w(sb, 1, W[1], wsop[1]))
-        if (MODE >= 1) copy_r(sb_prev, 1);
-        SVDQ_STEP(1, 1, 0, W[1], X[0], wsop[1], asop[0], 0, )
-        if (MODE >= 1) copy_r(sb_prev, 2);
-        SVDQ_STEP(2, 0, 1, W[1], X[1], wsop[1], asop[1], 3, read_w(sb, 2, W[0], wsop[0]))
-        SVDQ_STEP(3, 1, 0, W[0], X[0], wsop[0], asop[0], 0, )
-        SVDQ_STEP(4, 0, 1, W[0], X[1], wsop[0], asop[1], 3, read_w(sb, 3, W[1], wsop[1]))
-        P[0] = mfma_codes(W[1], X[0]);
-        F[0] = mfma_factor(wsop[1], asop[0]);
-        __builtin_amdgcn_sched_barrier(0);
-        // Every LDS read of this group has been issued, and the last one has arrived (the instruction
-        // above needed it).  Behind the barrier the stage may be overwritten, and the next group's
-        // stage, whose copies every wave has waited for, may be read.
-        if (MODE >= 1) asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (MODE == 2) copy_w(sb, 0);
-        read_x(sb_next, 0, X[0], asop[0]);
-        read_w(sb_next, 0, W[0], wsop[0]);
-        SVDQ_FMA(5, 1)
-        __builtin_amdgcn_sched_barrier(0);
-        if (MODE == 2) copy_w(sb, 1);
-        SVDQ_STEP(6, 0, 1, W[1], X[1], wsop[1], asop[1], 3, read_x(sb_next, 1, X[1], asop[1]))
-        if (MODE == 2) copy_w(sb, 2);
-        // (tile 0 of the next group; of nothing after the last group)
-        SVDQ_STEP(7, 1, 0, W[0], X[0], wsop[0], asop[0], 0, )
+        if constexpr (MT == 2) {
+            // step t issues the matrix instructions of tile t + 1 (tile = 2 nt + mt) and accumulates tile t
+            if (MODE >= 1) copy_r(sb_prev, 0);
+            SVDQ_STEP(0, 0, 1, W[0], X[1], wsop[0], asop[1], 3, read_w(sb, 1, W[1], wsop[1]))
+            if (MODE >= 1) copy_r(sb_prev, 1);
+            SVDQ_STEP(1, 1, 0, W[1], X[0], wsop[1], asop[0], 0, )
+            if (MODE >= 1) copy_r(sb_prev, 2);
+            SVDQ_STEP(2, 0, 1, W[1], X[1], wsop[1], asop[1], 3, read_w(sb, 2, W[0], wsop[0]))
+            SVDQ_STEP(3, 1, 0, W[0], X[0], wsop[0], asop[0], 0, )
+            SVDQ_STEP(4, 0, 1, W[0], X[1], wsop[0], asop[1], 3, read_w(sb, 3, W[1], wsop[1]))
+            P[0] = mfma_codes(W[1], X[0]);
+            F[0] = mfma_factor(wsop[1], asop[0]);
+            __builtin_amdgcn_sched_barrier(0);
+            // Every LDS read of this group has been issued, and the last one has arrived (the instruction
+            // above needed it).  Behind the barrier the stage may be overwritten, and the next group's
+            // stage, whose copies every wave has waited for, may be read.
+            if (MODE >= 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(COPIES) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (MODE == 2) copy_w(sb, 0);
+            read_x(sb_next, 0, X[0], asop[0]);
+            read_w(sb_next, 0, W[0], wsop[0]);
+            SVDQ_FMA(5, 1)
+            __builtin_amdgcn_sched_barrier(0);
+            if (MODE == 2) copy_w(sb, 1);
+            SVDQ_STEP(6, 0, 1, W[1], X[1], wsop[1], asop[1], 3, read_x(sb_next, 1, X[1], asop[1]))
+            if (MODE == 2) copy_w(sb, 2);
+            // (tile 0 of the next group; of nothing after the last group)
+            SVDQ_STEP(7, 1, 0, W[0], X[0], wsop[0], asop[0], 0, )
+        } else {
+            // The same with four tiles (tile = nt): the weights two tiles ahead, the barrier once the last tile's
+            // instructions have been issued.
+            if (MODE >= 1) copy_r(sb_prev, 0);
+            SVDQ_STEP(0, 0, 1, W[1], X[0], wsop[1], asop[0], 3, read_w(sb, 3, W[3], wsop[3]))
+            if (MODE >= 1) copy_r(sb_prev, 1);
+            SVDQ_STEP(1, 1, 0, W[2], X[0], wsop[2], asop[0], 0, )
+            P[1] = mfma_codes(W[3], X[0]);
+            F[1] = mfma_factor(wsop[3], asop[0]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (MODE >= 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(COPIES) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (MODE == 2) copy_w(sb, 0);
+            read_x(sb_next, 0, X[0], asop[0]);
+            read_w(sb_next, 0, W[0], wsop[0]);
+            SVDQ_FMA(2, 0)
+            __builtin_amdgcn_sched_barrier(0);
+            if (MODE == 2) copy_w(sb, 1);
+            read_w(sb_next, 1, W[1], wsop[1]);
+            if (MODE == 2) copy_w(sb, 2);
+            // (tile 0 of the next group; of nothing after the last group)
+            SVDQ_STEP(3, 1, 0, W[0], X[0], wsop[0], asop[0], 3, read_w(sb_next, 2, W[2], wsop[2]))
+        }
         sb = sb_next;
     };
     int l = 0;
@@ -252,7 +280,7 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
     // Every part parks its sums in its slot of the workspace; whoever arrives last adds all parts in
     // ascending order, so the result does not depend on who that is, and runs the epilogue.  Nobody waits for
     // anybody.
-    if (p.kparts > 1) {
+    if (MT == 2 && kparts > 1) {
         float *slot = p.partials + ((size_t)tile * p.kparts + part) * PARTIAL_SLOT_FLOATS;
         const __amdgpu_buffer_rsrc_t mine = partial_rsrc(slot);
 #pragma unroll
@@ -348,7 +376,7 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
     }
 
     // ---- epilogue --------------------------------------------------------------------------------
-    const int wrow0 = m0 + wm * 64, wcol0 = n0 + wn * 128;
+    const int wrow0 = m0 + wm * (32 * MT), wcol0 = n0 + wn * 128;
     // per-column factor (alpha and wcscales; EpilogueBias, gemm_base.cuh:710-781) and bias of the
     // workgroup's 256 columns
     float *coltab = (float *)(lds + EP_TAB);
@@ -385,9 +413,9 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
             for (int q = 0; q < 4; q++) {
                 const float4_t cf = *(const float4_t *)(cfw + nt * 32 + 8 * q + 4 * h);
 #pragma unroll
-                for (int mt = 0; mt < 2; mt++)
+                for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++) acc[2 * nt + mt][4 * q + i] *= cf[i];
+                    for (int i = 0; i < 4; i++) acc[MT * nt + mt][4 * q + i] *= cf[i];
             }
     }
     // Low-rank up projection (lora.cuh:110-241): out += bf16(lora_act * scale) @ up^T on the matrix
@@ -397,10 +425,10 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
     for (int s0 = 0; s0 < nsteps; s0 += 2) {
         const bool two = s0 + 1 < nsteps;
         const int s1 = two ? s0 + 1 : s0;
-        float4_t ra[2][2][2];
+        float4_t ra[MT][2][2];
         u32x4_t rb[4][2];
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
+        for (int t = 0; t < MT; t++) {
             const float4_t *ap = (const float4_t *)(p.lora_act + (size_t)(wrow0 + t * 32 + r32) * p.R_up + 8 * h);
             ra[t][0][0] = ap[4 * s0]; ra[t][0][1] = ap[4 * s0 + 1];
             ra[t][1][0] = ap[4 * s1]; ra[t][1][1] = ap[4 * s1 + 1];
@@ -417,9 +445,9 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
         for (int k = 0; k < 2; k++) {
             if (k == 1 && !two) break;
             const float ls = p.lora_scales[s0 + k];
-            bf16x8_t la[2];
+            bf16x8_t la[MT];
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
+            for (int t = 0; t < MT; t++) {
                 const float4_t v0 = ra[t][k][0], v1 = ra[t][k][1];
                 u32x4_t w;
                 w[0] = pack_bf16x2(v0[0] * ls, v0[1] * ls);
@@ -431,8 +459,8 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
 #pragma unroll
             for (int nt = 0; nt < 4; nt++)
 #pragma unroll
-                for (int mt = 0; mt < 2; mt++)
-                    acc[2 * nt + mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, rb[nt][k]), la[mt], acc[2 * nt + mt], 0, 0, 0);
+                for (int mt = 0; mt < MT; mt++)
+                    acc[MT * nt + mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, rb[nt][k]), la[mt], acc[MT * nt + mt], 0, 0, 0);
         }
     }
 
@@ -448,18 +476,18 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
         }
     }
     const bool down_in_lds = NEXT && p.next_down && p.R_down <= 32;
-    const bool interior = m0 + BM <= p.M_out && n0 + BN <= p.N_out;  // the whole tile lies inside the output
+    const bool interior = m0 + TILE_M <= p.M_out && n0 + BN <= p.N_out;  // the whole tile lies inside the output
     uint16_t *slab = (uint16_t *)(lds + wave * SLAB_BYTES);
     const int ngroups_out = p.N / 64;
     VkSums vks;  // linear attention: the sums of the wave's two slabs
     if (NEXT && p.vk) litela_clear(vks);
     // next layer's low-rank projection at ranks up to 32: [slab][rank tile][16-row half] sums of the wave's 128 columns,
     // kept until both slabs are done so that the column halves meet once per tile
-    float4_t down_sums[2][2][2];
+    float4_t down_sums[MT][2][2];
     const bool down_once = NEXT && p.next_down && p.R_down <= 32;
     // one 32-row slab of the wave tile, instantiated twice with a compile-time slab index
-    auto slab_epilogue = [&](auto MT) {
-        constexpr int mt = decltype(MT)::value;
+    auto slab_epilogue = [&](auto SLAB) {
+        constexpr int mt = decltype(SLAB)::value;
         float16_t v[4];
 #pragma unroll
         for (int nt = 0; nt < 4; nt++)
@@ -467,7 +495,7 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
             for (int q = 0; q < 4; q++) {
                 const float4_t bs = *(const float4_t *)(bsw + nt * 32 + 8 * q + 4 * h);
 #pragma unroll
-                for (int i = 0; i < 4; i++) v[nt][4 * q + i] = acc[2 * nt + mt][4 * q + i] + bs[i];
+                for (int i = 0; i < 4; i++) v[nt][4 * q + i] = acc[MT * nt + mt][4 * q + i] + bs[i];
             }
         if (NEXT && p.rotary && wcol0 < p.rope_cols) {
             // EpilogueRMSNormRope (epilogues.cuh:269-425): the wave's 128 columns are one head of q or k.
@@ -629,9 +657,9 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
                             if (rt0 + g >= RT) continue;
                             const float4_t o = *(const float4_t *)(red + (((g * 2 + wm) * 2 + m2) * 64 + lane) * 4);
                             const float4_t sum = float4_t{d[g][m2][0] + o[0], d[g][m2][1] + o[1], d[g][m2][2] + o[2], d[g][m2][3] + o[3]};
-                            // share layout [32-row slab][rank tile][m2][64 lanes] x float4; this workgroup's slabs are 4 mb + 2 wm + mt
+                            // share layout [32-row slab][rank tile][m2][64 lanes] x float4; this workgroup's slabs are slab0 + MT wm + mt of row block mb
                             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, sum), slot,
-                                                                   (((((wm * 2 + mt) * RT + rt0 + g) * 2 + m2) * 64) + lane) * 16, 0, 0);
+                                                                   (((((slab0 + wm * MT + mt) * RT + rt0 + g) * 2 + m2) * 64) + lane) * 16, 0, 0);
                         }
                 }
                 __syncthreads();
@@ -677,16 +705,16 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
     };
     __builtin_amdgcn_sched_barrier(0);
     slab_epilogue(std::integral_constant<int, 0>{});
-    slab_epilogue(std::integral_constant<int, 1>{});
+    if constexpr (MT == 2) slab_epilogue(std::integral_constant<int, 1>{});
     if (down_once) {
         // the right column half hands its sums over through its own slab area, which it no longer needs; the left
-        // one adds and stores the workgroup's share: [32-row slab 2 wm + mt][rank tile][16-row half][64 lanes] x float4
+        // one adds and stores the workgroup's share: [32-row slab of the row block][rank tile][16-row half][64 lanes] x float4
         static_assert(SLAB_BYTES >= 2 * 2 * 2 * 64 * 16, "a wave's sums pass through its slab area");
         const int RT = p.R_down / 16;
         float4_t *xchg = (float4_t *)(lds + (2 * wm + 1) * SLAB_BYTES);
         if (wn == 1) {
 #pragma unroll
-            for (int mt = 0; mt < 2; mt++)
+            for (int mt = 0; mt < MT; mt++)
 #pragma unroll
                 for (int g = 0; g < 2; g++)
 #pragma unroll
@@ -697,7 +725,7 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
             const __amdgpu_buffer_rsrc_t slot = __builtin_amdgcn_make_buffer_rsrc(
                 (void *)(p.next_lora_part + ((size_t)nb * (p.M_pad / BM) + mb) * (size_t)(BM * p.R_down)), 0, BM * p.R_down * 4, 0x00020000);
 #pragma unroll
-            for (int mt = 0; mt < 2; mt++)
+            for (int mt = 0; mt < MT; mt++)
 #pragma unroll
                 for (int g = 0; g < 2; g++) {
                     if (g >= RT) continue;
@@ -706,7 +734,7 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
                         const float4_t o = xchg[((mt * 2 + g) * 2 + m2) * 64 + lane], d = down_sums[mt][g][m2];
                         const float4_t sum = float4_t{d[0] + o[0], d[1] + o[1], d[2] + o[2], d[3] + o[3]};
                         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, sum), slot,
-                                                               (((((wm * 2 + mt) * RT + g) * 2 + m2) * 64) + lane) * 16, 0, 0);
+                                                               (((((slab0 + wm * MT + mt) * RT + g) * 2 + m2) * 64) + lane) * 16, 0, 0);
                     }
                 }
         }
@@ -715,8 +743,33 @@ __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
         static_assert(SLAB_BYTES >= 2 * VK_HEAD_FLOATS * 4, "a wave's two heads pass through its slab area");
         const int third = p.N / 3;
         litela_finish(vks, wcol0 >= third && wcol0 < p.N, wm, wn, lds, SLAB_BYTES,
-                      p.vk_part + ((size_t)mb * (2 * third / 64) + (wcol0 - third) / 64) * VK_HEAD_FLOATS, lane);
+                      p.vk_part + ((size_t)vk_slot * (2 * third / 64) + (wcol0 - third) / 64) * VK_HEAD_FLOATS, lane);
     }
+}
+
+// Which tile: row blocks [0, full_blocks) are 128 rows high, the half_blocks behind them 64 (or, with full_blocks = all, tiles
+// split along K).  Workgroups go to the XCDs round robin (blockIdx % 8): each XCD takes one contiguous run of the
+// numbers of the 128-row tiles (or their parts), then one of the 64-row tiles'.  The tiles are numbered in bands of about ten
+// 128-row blocks, down the band first: the 64 workgroups resident on an XCD at one time then cover about 10 row blocks
+// x 6 column blocks, whose operands (6 KB per row block and k-group, 14 KB per column block) they share in that
+// XCD's L2.  Measured at 36 x 48 tiles, bytes fetched from beyond the L2 per launch: bands of 6 / 9 / 12 /
+// 16 / 18 / 36 row blocks 317 / 296 / 308 / 355 / 396 / 604 MB (the time does not change: 169-171 us).
+template <bool NEXT>
+__global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
+    const int nblocks = (p.N + BN - 1) / BN, total = (int)gridDim.x, full = p.full_blocks * nblocks * p.kparts;
+    const int xcd = (int)blockIdx.x % 8, j = (int)blockIdx.x / 8;
+    const int first = xcd * (full / 8) + (xcd < full % 8 ? xcd : full % 8);  // of this XCD's 128-row tiles
+    const int count = full / 8 + (xcd < full % 8 ? 1 : 0);
+    const bool whole = j < count;
+    // (the 64-row tiles of the XCDs before this one: their workgroups less their 128-row tiles)
+    const int v = whole ? first + j : xcd * (total / 8) + (xcd < total % 8 ? xcd : total % 8) - first + (j - count);
+    const int tile = whole ? v / p.kparts : v, part = whole ? v - tile * p.kparts : 0;
+    const int blocks = whole ? p.full_blocks : p.half_blocks, BAND = whole ? p.band : p.half_band;
+    const int band = tile / (BAND * nblocks), in_band = tile - band * (BAND * nblocks);
+    const int band_rows = blocks - band * BAND < BAND ? blocks - band * BAND : BAND;
+    const int mb = band * BAND + in_band % band_rows, nb = in_band / band_rows;
+    if (whole) output_tile<NEXT, 2>(p, mb * BM, nb, tile, part, mb);
+    else output_tile<NEXT, 1>(p, p.full_blocks * BM + mb * (BM / 2), nb, 0, 0, p.full_blocks + mb);
 }
 
 template <bool NEXT>

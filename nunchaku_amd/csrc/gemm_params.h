@@ -199,10 +199,15 @@ constexpr int BM = 128, BN = 256;  // workgroup tile; 4 waves as 2 x 2, wave til
 // One stage of the LDS ring holds one k-group of the workgroup's operands:
 //   4 activation fragments | 8 weight fragments | weight scales 256 x {64 s, 0, 0, 0} bf16 |
 //   activation scales 128 x bf16 | zeros (what the upper half-wave reads as its activation scale)
-constexpr int ST_A = 0, ST_W = 4 * FRAG_BYTES, ST_WS = ST_W + 8 * FRAG_BYTES, ST_AS = ST_WS + 256 * 8, ST_Z = ST_AS + 256;
-constexpr int STAGE_BYTES = ST_Z + 128;
+// (tiles of 64 rows: 2 activation fragments, and 1 KB for the activation scales)
+template <int MT>
+struct StageOf {
+    static constexpr int A = 0, W = 2 * MT * FRAG_BYTES, WS = W + 8 * FRAG_BYTES, AS = WS + 256 * 8, Z = AS + (MT == 2 ? 256 : 1024), BYTES = Z + 128;
+};
+constexpr int STAGE_BYTES = StageOf<2>::BYTES;
+static_assert(StageOf<1>::BYTES <= STAGE_BYTES, "both tile heights use the same ring");
 constexpr int STAGES = 3;
-constexpr int COPIES_PER_WAVE = 6;  // asynchronous copies every wave issues per k-group
+constexpr int COPIES_PER_WAVE = 6;  // asynchronous copies every wave issues per k-group (128-row tiles)
 // epilogue (reuses the ring): per wave one 32-row slab of bf16, then the column tables
 constexpr int OUT_LD = 136;
 constexpr int SLAB_BYTES = 32 * OUT_LD * 2;
@@ -236,8 +241,9 @@ struct Params {
     // tiles split along K: parked partial sums and one arrival counter per tile (zero between launches)
     float *partials;
     int *counters;
-    int band;          // row blocks per band of the tile numbering
-    int kparts;
+    // Row blocks of 128 rows, then of 64 rows; and of either kind the row blocks per band of the tile numbering
+    int full_blocks, half_blocks, band, half_band;
+    int kparts;        // (1 where half_blocks > 0)
     int M_pad, N, K, M_out, N_out, R_up, R_down;
     float alpha;
     float lora_scales[MAX_RANK / 16];
@@ -251,7 +257,7 @@ struct Params {
     // stored through `out` after a ReLU; the rest is [head][k 32 | v 32]; vk[batch][head][i][j] += sum over the
     // tile's rows of v[i] relu(k[j]) (i < 32) and of relu(k[j]) (i = 32)
     float *vk;           // fp32 [batch][2 N / 3 / 64][33][32]; null: no such epilogue
-    float *vk_part;      // workspace: [M_pad / 128 row blocks][heads] x 1056 floats, every row block's sums
+    float *vk_part;      // workspace: [full_blocks + half_blocks][heads] x 1056 floats, every row block's sums
     int vk_rows;         // rows per batch entry, a multiple of 256
 };
 }  // namespace g6
