@@ -497,6 +497,14 @@ int gemm_int4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool no
 }
 
 // ---- NVFP4: fp16 matrix instruction on dequantized operands (gemm_kernel.h) -------------------------
+// The number of workgroups that share the tiles of an NVFP4 launch out whole, where it is at least 84 % of the compute units; 0
+// otherwise.
+int whole_tiles_fp4(long long ntiles, int ncu) {
+    long long divisor = ntiles < ncu ? ntiles : ncu;
+    while (ntiles % divisor != 0) divisor--;
+    return ntiles >= ncu && divisor * 100 >= ncu * 84 ? (int)divisor : 0;
+}
+
 int gemm_fp4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool noalloc) {
     GemmParams p;
     fill_params(a, p);
@@ -506,7 +514,7 @@ int gemm_fp4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool noa
     int nwg = ntiles < ncu ? ntiles : ncu;
     int divisor = nwg;  // the largest workgroup count that divides the tile count
     while (ntiles % divisor != 0) divisor--;
-    if (a->k_split == 1 || (a->k_split == 0 && ntiles >= ncu && divisor * 100 >= ncu * 84)) {
+    if (a->k_split == 1 || (a->k_split == 0 && whole_tiles_fp4(ntiles, ncu) > 0)) {
         // Whole tiles only: asked for, or at least 84 % of the compute units get a whole number of tiles (M = 4608,
         // N = 9216: 216 workgroups x 3 tiles 257 us, 256 even shares 256).  Then the
         // workgroups that share a block of weight columns walk K in step and find it in their L2, and no sums
@@ -577,18 +585,19 @@ int gemm_fp4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool noa
 
 // ---- few rows, either precision: small tiles, operands straight to registers (gemm_direct_kernel.h) ------
 // Which of the two shapes of the few-rows kernel (0: neither) a launch takes.  Shape 1: tiles of 32 rows, four waves split
-// K.  Shape 2: tiles of 64 rows, two waves split K and two the columns: 23 % fewer operand bytes per product, from about
-// 400 tiles of 32 rows on.  Both are models of the time in us fitted to launches at K = 1024, 3072 and 12288 on 256 compute
-// units, linear in the number of tiles that the busiest compute unit works through and in the k-groups; they meet the
-// measurements within about 10 %.  Measured at K = 3072, large tiles (split along K where that pays) / shape 1 / shape 2:
-//   INT4   M = 256, N = 3072   22.8 /  9.6 / 12.3     NVFP4  59.9 / 11.2 / 15.4
-//          M = 505, N = 9216   33.6 / 33.7 / 30.4            64.0 / 39.2 / 38.1
-//          M = 1157, N = 3072  29.7 / 27.6 / 21.8            63.5 / 31.5 / 26.9
-//          M = 1024, N = 9216  45.0 / 57.4 / 48.4            70.3 / 69.8 / 61.7
-//          M = 1024, N = 12288                               74.4 / 90.3 / 76.2
-//   K = 12288, N = 3072: M = 256  42.1 / 24.8 / -           113.6 / 29.5 / -
-//          M = 505             44.7 / 44.6 / 34.9           115.6 / 51.2 / 46.2
-//          M = 1157            66.6 / 86.6 / 65.6           126.3 / 102.3 / 90.6
+// K.  Shape 2: tiles of 64 rows, a quarter fewer operand bytes per product, from about 400 tiles of 32 rows on; INT4: two waves
+// split K and two the columns, NVFP4: four waves split K.  Models of the time in us fitted to launches at K = 1024 ... 12288
+// on 256 compute units, linear in the number of tiles that the busiest compute unit works through and in the k-groups; they meet
+// the measurements within about 10 %.  Measured at K = 3072, large tiles (split along K where that pays) / shape 1 / shape 2:
+//   INT4   M = 256, N = 3072   22.8 /  9.6 / 12.3     NVFP4  60.7 / 11.8 / 13.8
+//          M = 505, N = 9216   28.7 / 33.1 / 30.6            62.9 / 38.4 / 34.1
+//          M = 1157, N = 3072  29.7 / 27.6 / 21.8            62.1 / 31.7 / 25.7
+//          M = 1024, N = 9216  36.1 / 57.7 / 48.5            68.4 / 69.7 / 57.9
+//          M = 1157, N = 12288                               80.1 / 103.8 / 88.6, with the quantizing epilogue 106.7 / 126.2 / 105.4
+//          M = 4608, N = 12288                               298 / 407 / 317, with the quantizing epilogue 387 / 457 / 358
+//   K = 12288, N = 3072: M = 256  42.1 / 24.8 / 34.4           113.6 / 30.8 / 35.0
+//          M = 505             45.4 / 44.1 / 34.6           115.2 / 50.8 / 37.9
+//          M = 1157            66.6 / 86.6 / 65.6           127.5 / 99.5 / 81.2
 int choose_direct(const svdq_gemm_args *a, int ncu) {
     if (a->k_split > 0) return 0;  // (the caller asks for the tiles that k_split is about)
     if (((uintptr_t)a->bias | (uintptr_t)a->wcscales | (uintptr_t)a->oscales) % 8 || (uintptr_t)a->colnorm % 16) return 0;  // (read four columns at a time)
@@ -597,11 +606,24 @@ int choose_direct(const svdq_gemm_args *a, int ncu) {
     const double c1 = (double)((((rows + 31) / 32) * ncols + ncu - 1) / ncu), c2 = (double)((((rows + 63) / 64) * ncols + ncu - 1) / ncu);
     double t_large, t1, t2;
     if (a->fp4) {
-        // (one 256 x 256 tile per compute unit: 62 us at K = 3072 with 48 tiles, 78 with 216; 32 at K = 1024)
-        const double tiles = (double)(a->M_pad / BM) * ((a->N + BN - 1) / BN) / ncu;
-        t_large = ((1.0 + 0.3 * (tiles < 1.0 ? tiles : 1.0)) * kg + 14.0) * (tiles > 1.0 ? tiles : 1.0);
+        // Large tiles: one per compute unit 62 us at K = 3072 with 48 tiles, 78 with 216; 32 at K = 1024.  Whole tiles of several
+        // rounds cost that many times as much, even shares of them 26 to 40 us for the sums that meet in the workspace.
+        const long long ntiles = (a->M_pad / BM) * ((a->N + BN - 1) / BN);
+        const double tiles = (double)ntiles / ncu, one = (1.0 + 0.3 * (tiles < 1.0 ? tiles : 1.0)) * kg + 14.0;
+        const int nwg = whole_tiles_fp4(ntiles, ncu);
+        const double rounds = tiles <= 1.0 ? 1.0 : nwg ? (double)(ntiles / nwg) : tiles;
+        t_large = one * rounds + (tiles > 1.0 && !nwg ? 33.0 : 0.0);
         t1 = 4.3 + c1 * (1.1 + 0.127 * kg);
-        t2 = 3.0 + c2 * (2.1 + 0.214 * kg);
+        t2 = 5.0 + c2 * (1.6 + 0.205 * kg) - (c2 < 3.0 ? 0.04 * kg : 0.0);
+        if (a->qout) {  // (the quantizing epilogue: M = 4608, K = 3072, N = 12288 298 -> 387 us in large tiles, 317 -> 358 in shape 2)
+            t_large += 20.0 * rounds;
+            t1 += 1.1 * c1;
+            t2 += 1.4 * c2;
+        } else if (a->rotary_emb) {  // (M = 4608, K = 3072, N = 9216 223 -> 253 and 241 -> 261)
+            t_large += 10.0 * rounds;
+            t1 += 0.9 * c1;
+            t2 += 1.0 * c2;
+        }
     } else {
         int full, half, kparts;
         t_large = choose_tiles_int4(a, ncu, &full, &half, &kparts);

@@ -13,7 +13,13 @@
 //
 // INT4: one fp6 matrix instruction on the codes, one factor instruction and 16 multiply-adds per 32 x 32 tile and
 // k-group (gemm6_kernel.h).  NVFP4: both operands are dequantized to fp16 in registers by the wave that uses them
-// (gemm_kernel.h dequantizes once per workgroup; here every wave has its own k-groups, so that is the same).
+// (gemm_kernel.h dequantizes once per workgroup; here every wave has its own k-groups, so that is the same).  A wave alone on
+// its SIMD issues a vector instruction every 8 cycles at most and stands still behind a matrix instruction while the next one
+// waits for the matrix core (32 cycles), so the conversions are counted: 64 rows x 128 columns per wave take 6 of them per matrix
+// instruction (64 x 64: 8), converted one step ahead and spread evenly between the matrix instructions (left to itself the
+// compiler issues these in pairs, with the conversions behind).  K = 12288, N = 3072, 64 x 64 per wave / 64 x 128 / with the
+// conversions a step ahead: M = 256 45.5 / 39.6 / 35.0 us, M = 1157 91.7 / 84.3 / 81.2; from two tiles per compute unit on 1.2
+// PFLOP/s, where the large kernel's 1.25 is the power limit.
 //
 // The epilogue is shared out by columns: wave w of four adds up the parts' sums of the 32 columns 32 w ... of the tile
 // in ascending order, projects the low-rank branch onto them and applies bias, norm, rotation and activation; the
@@ -134,6 +140,19 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
 #pragma unroll
         for (int e = 0; e < 16; e++) P[b][e] = F[b][e] = 0.f;
 
+    // NVFP4: converted operands of two steps, and the rows' scales of the k-group that is being converted
+    half8_t wop[FP4 ? 2 : 1], xop[FP4 ? 2 : 1][MT];
+    half2_t xs[MT];
+    auto column_scale = [](uint32_t ws, bool second) {
+        const half2_t s = as_half2(ws);
+        return second ? half2_t{s[1], s[1]} : half2_t{s[0], s[0]};
+    };
+    auto row_scale = [&](int mt, bool second) { return second ? half2_t{xs[mt][1], xs[mt][1]} : half2_t{xs[mt][0], xs[mt][0]}; };
+    auto read_row_scales = [&](const uint32_t (&as)[MT]) {
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) xs[mt] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(as[mt], 1.0f, false);
+    };
+
     auto compute = [&](auto S) {
         auto &st = sets[decltype(S)::value];
         if constexpr (!FP4) {
@@ -153,35 +172,43 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
             };
             each(std::make_integer_sequence<int, NT * MT>{}, tile);
         } else {
-            half2_t sx[MT][2], sw[NT][2];  // a lane's two 16-groups
+            // step t = (ks, nt) multiplies the operands that the step before has converted, and between its matrix instructions
+            // converts the column operand of the next step and a share of the rows' operands of the next 16 k (in the last
+            // steps those of the next k-group, which arrived while this one was multiplied)
+            auto &next = sets[(decltype(S)::value + 1) % (DEPTH + 1)];
+            each(std::make_integer_sequence<int, 4 * NT>{}, [&](auto T) {
+                constexpr int t = decltype(T)::value, ks = t / NT, nt = t % NT, t1 = (t + 1) % (4 * NT), ks1 = (ks + 1) % 4;
+                constexpr bool w_wraps = t1 < t, x_wraps = ks1 < ks;
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-                const half2_t s = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(st.as[mt], 1.0f, false);
-                sx[mt][0] = half2_t{s[0], s[0]};
-                sx[mt][1] = half2_t{s[1], s[1]};
-            }
+                for (int mt = 0; mt < MT; mt++) acc[nt * MT + mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wop[t & 1], xop[ks & 1][mt], acc[nt * MT + mt], 0, 0, 0);
+                wop[(t + 1) & 1] = dequant_word_fp4((w_wraps ? next : st).w[t1 % NT][t1 / NT], column_scale((w_wraps ? next : st).ws[t1 % NT], t1 / NT >= 2));
+                constexpr int share = 4 * MT / NT;  // pairs of the rows' operands per step
+                each(std::make_integer_sequence<int, share>{}, [&](auto I) {
+                    constexpr int pair = nt * share + decltype(I)::value, mt = pair / 4, b = pair % 4;
+                    if constexpr (x_wraps && pair == 0) read_row_scales(next.as);
+                    const half2_t v = dequant_pair_fp4<b>((x_wraps ? next : st).x[mt][ks1], row_scale(mt, ks1 >= 2));
+                    xop[(ks + 1) & 1][mt][2 * b] = v[0];
+                    xop[(ks + 1) & 1][mt][2 * b + 1] = v[1];
+                });
+                constexpr int valu = (8 + 2 * share + MT - 1) / MT;
 #pragma unroll
-            for (int nt = 0; nt < NT; nt++) {
-                const half2_t s = as_half2(st.ws[nt]);
-                sw[nt][0] = half2_t{s[0], s[0]};
-                sw[nt][1] = half2_t{s[1], s[1]};
-            }
-#pragma unroll
-            for (int ks = 0; ks < 4; ks++) {
-                half8_t x[MT];
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++) x[mt] = dequant_word_fp4(st.x[mt][ks], sx[mt][ks >> 1]);
-#pragma unroll
-                for (int nt = 0; nt < NT; nt++) {
-                    const half8_t w = dequant_word_fp4(st.w[nt][ks], sw[nt][ks >> 1]);
-#pragma unroll
-                    for (int mt = 0; mt < MT; mt++) acc[nt * MT + mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w, x[mt], acc[nt * MT + mt], 0, 0, 0);
+                for (int mt = 0; mt < MT; mt++) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, valu, 0);
                 }
-            }
+                __builtin_amdgcn_sched_barrier(0);
+            });
         }
     };
 
     each(std::make_integer_sequence<int, DEPTH>{}, [&](auto D) { load(D); });
+    if constexpr (FP4) {
+        auto &st = sets[0];
+        read_row_scales(st.as);
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) xop[0][mt] = dequant_word_fp4(st.x[mt][0], row_scale(mt, false));
+        wop[0] = dequant_word_fp4(st.w[0][0], column_scale(st.ws[0], false));
+    }
     int g = kpart;
     auto step = [&](auto S) {
         load(std::integral_constant<int, (decltype(S)::value + DEPTH) % (DEPTH + 1)>{});

@@ -40,11 +40,12 @@ __device__ inline uint32_t as_u32(half2_t h) { return __builtin_bit_cast(uint32_
 
 // 8 E2M1 patterns of one word -> 8 fp16 values pattern_value * scale, slot order [0..7].  The
 // hardware conversion yields the exact E2M1 value (its scale operand only contributes an exponent).
+template <int PAIR>
+__device__ inline half2_t dequant_pair_fp4(uint32_t w, half2_t s) {
+    return __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, PAIR) * s;
+}
 __device__ inline half8_t dequant_word_fp4(uint32_t w, half2_t s) {
-    const half2_t t0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 0) * s;
-    const half2_t t1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 1) * s;
-    const half2_t t2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 2) * s;
-    const half2_t t3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 3) * s;
+    const half2_t t0 = dequant_pair_fp4<0>(w, s), t1 = dequant_pair_fp4<1>(w, s), t2 = dequant_pair_fp4<2>(w, s), t3 = dequant_pair_fp4<3>(w, s);
     return half8_t{t0[0], t0[1], t1[0], t1[1], t2[0], t2[1], t3[0], t3[1]};
 }
 

@@ -17,6 +17,7 @@ CASES = [
     ("silu", 96, 384, 256, 16), ("next", 33, 128, 128, 16), ("next", 97, 640, 384, 48), ("rope", 40, 384, 384, 32), ("split", 256, 256, 768, 16),
     ("litela", 256, 256, 384, 16),
     ("plain", 1200, 384, 3072, 32), ("next", 1185, 256, 3072, 32), ("rope", 1217, 256, 3072, 16), ("split", 1280, 128, 3072, 32), ("litela", 1024, 256, 3456, 32),
+    ("plain", 1217, 640, 3072, 32), ("next", 1200, 1152, 3072, 48), ("rope", 1153, 512, 3072, 0),  # (5 and 4, 3 and 2, 2 k-groups per wave)
 ]
 
 
