@@ -91,6 +91,7 @@ bool unchanged(const Layer &l, PyObject *module) {
 
 // The module's lora_scales (one factor per 16 ranks; None: all ones; missing entries count as zero) into `sc`.
 bool read_lora_scales(PyObject *module, int groups, float *sc) {
+    if (groups > MAX_GROUPS) return false;
     PyObject *d = dict_of(module);
     PyObject *ls = d ? PyDict_GetItem(d, s_lora_scales) : nullptr;
     if (!ls) return false;
@@ -148,20 +149,28 @@ svdq_quantize_args quantize_args(const Layer &l, const void *x, int64_t M, int64
     q.M_pad = M_pad;
     return q;
 }
-svdq_gemm_args gemm_args(const Layer &l, int64_t M_pad, const Activations &a, const float *sc, int k_split) {
+svdq_gemm_args gemm_args(const Layer &l, int64_t M_pad, const Activations &a, const float *sc, int64_t k_split) {
     svdq_gemm_args g = l.g;
     g.act = a.codes;
     g.ascales = a.scales;
     g.lora_act_in = a.lora;
     g.lora_scales = sc;
     g.M_pad = M_pad;
-    g.k_split = k_split;
+    g.k_split = (int)k_split;
     return g;
 }
 int gemm(const svdq_gemm_args &g, bool no_alloc, hipStream_t st) { return no_alloc ? svdq_gemm_w4a4_noalloc(&g, st) : svdq_gemm_w4a4(&g, st); }
 
 at::Tensor new_bf16(at::IntArrayRef sizes, int device) {
     return at::empty(sizes, at::TensorOptions().dtype(at::kBFloat16).device(at::Device(at::kCUDA, (c10::DeviceIndex)device)));
+}
+
+// a whole number among the arguments; false (and no exception left) where it is something else
+bool as_int(PyObject *o, int64_t *v) {
+    *v = PyLong_AsLongLong(o);
+    if (*v != -1 || !PyErr_Occurred()) return true;
+    PyErr_Clear();
+    return false;
 }
 
 Layer *layer_of(PyObject *capsule) { return (Layer *)PyCapsule_GetPointer(capsule, LAYER); }
@@ -233,7 +242,8 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         if (!as_tensor(args[3], &given) || !given->is_cuda() || given->device() != x->device() || given->scalar_type() != at::kBFloat16 ||
             !given->is_contiguous() || given->numel() != M * l->N || given->size(-1) != l->N) Py_RETURN_NONE;
     }
-    const int k_split = (int)PyLong_AsLong(args[4]);
+    int64_t k_split;
+    if (!as_int(args[4], &k_split)) Py_RETURN_NONE;
     const bool no_alloc = args[5] == Py_True;
     at::Tensor out = given ? given->view({B, S, l->N}) : new_bf16({B, S, l->N}, l->device);
     hipStream_t st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)l->device).stream();
@@ -261,12 +271,11 @@ PyObject *gelu_mlp(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     if (!l1 || !l2) return nullptr;
     const at::Tensor *x;
     float sc1[MAX_GROUPS], sc2[MAX_GROUPS];
-    const int64_t pad = PyLong_AsLongLong(args[5]);
-    if (!as_tensor(args[4], &x) || !plain_activations(*l1, *x) || l2->device != l1->device || l1->N != l2->K || l1->g.fp4 != l2->g.fp4 || pad <= 0 || pad % 256 ||
+    int64_t pad, k_split;
+    if (!as_int(args[5], &pad) || !as_int(args[6], &k_split) || !as_tensor(args[4], &x) || !plain_activations(*l1, *x) || l2->device != l1->device || l1->N != l2->K || l1->g.fp4 != l2->g.fp4 || pad <= 0 || pad % 256 ||
         !unchanged(*l1, args[1]) || !unchanged(*l2, args[3]) || !read_lora_scales(args[1], (int)(l1->rank + 15) / 16, sc1) ||
         !read_lora_scales(args[3], (int)(l2->rank + 15) / 16, sc2)) Py_RETURN_NONE;
     const int64_t B = x->size(0), S = x->size(1), M = B * S, M_pad = (M + pad - 1) / pad * pad;
-    const int k_split = (int)PyLong_AsLong(args[6]);
     const bool no_alloc = args[7] == Py_True;
     at::Tensor out = new_bf16({B, S, l2->N}, l1->device);
     hipStream_t st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)l1->device).stream();
@@ -312,7 +321,12 @@ PyObject *qkv_norm_rope(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     const int64_t B = x->size(0), S = x->size(1), M = B * S, M_pad = (M + 255) / 256 * 256;
     at::Tensor out;
     const at::Tensor *qkv[3] = {nullptr, nullptr, nullptr};
-    const int64_t attn_tokens = PyLong_AsLongLong(args[7]);
+    int64_t attn_tokens, k_split;
+    const double norm_eps = PyFloat_AsDouble(args[8]);
+    if ((norm_eps == -1.0 && PyErr_Occurred()) || !as_int(args[7], &attn_tokens) || !as_int(args[9], &k_split)) {
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
     const bool split = args[6] != Py_None;
     if (split) {
         if (!PyTuple_Check(args[6]) || PyTuple_GET_SIZE(args[6]) != 3 || attn_tokens < 0 || attn_tokens > M_pad) Py_RETURN_NONE;
@@ -325,7 +339,6 @@ PyObject *qkv_norm_rope(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     } else {
         out = new_bf16({M_pad, l->N}, l->device);
     }
-    const int k_split = (int)PyLong_AsLong(args[9]);
     const bool no_alloc = args[10] == Py_True;
     hipStream_t st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)l->device).stream();
     Scratch mem(Activations(*l, M_pad, nullptr).bytes, st);
@@ -336,7 +349,7 @@ PyObject *qkv_norm_rope(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     g.norm_k = nk->data_ptr();
     g.rotary_emb = (const float *)rot->data_ptr();
     g.rot_rows = rot->size(0);
-    g.norm_eps = (float)PyFloat_AsDouble(args[8]);
+    g.norm_eps = (float)norm_eps;
     if (split) {
         g.out_q = qkv[0]->data_ptr();
         g.out_k = qkv[1]->data_ptr();
@@ -406,8 +419,7 @@ PyObject *awq_gemv(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     if (args[8] != Py_None && !as_tensor(args[8], &bias)) Py_RETURN_NONE;
     int64_t v[4];
     for (int i = 0; i < 4; i++) {
-        if (!PyLong_Check(args[4 + i])) Py_RETURN_NONE;
-        v[i] = PyLong_AsLongLong(args[4 + i]);
+        if (!PyLong_Check(args[4 + i]) || !as_int(args[4 + i], &v[i])) Py_RETURN_NONE;
     }
     return awq_call(*t[0], *t[1], *t[2], *t[3], bias, v[0], v[1], v[2], (int)v[3]);
     END_HANDLE_TH_ERRORS
@@ -424,8 +436,9 @@ PyObject *awq_linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     PyObject *b = PyDict_GetItem(params, s_bias);
     if (b && b != Py_None && !as_tensor(b, &bias)) Py_RETURN_NONE;
     PyObject *in = PyDict_GetItem(d, s_in_features), *out = PyDict_GetItem(d, s_out_features), *gs = PyDict_GetItem(d, s_group_size);
-    if (!in || !out || !gs || !PyLong_Check(in) || !PyLong_Check(out) || !PyLong_Check(gs) || x->dim() < 1 || x->size(-1) <= 0) Py_RETURN_NONE;
-    return awq_call(*x, *w, *s, *z, bias, x->numel() / x->size(-1), PyLong_AsLongLong(out), PyLong_AsLongLong(in), (int)PyLong_AsLong(gs));
+    int64_t n, k, group_size;
+    if (!in || !out || !gs || !as_int(in, &k) || !as_int(out, &n) || !as_int(gs, &group_size) || x->dim() < 1 || x->size(-1) <= 0) Py_RETURN_NONE;
+    return awq_call(*x, *w, *s, *z, bias, x->numel() / x->size(-1), n, k, (int)group_size);
     END_HANDLE_TH_ERRORS
 }
 

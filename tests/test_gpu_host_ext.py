@@ -78,3 +78,26 @@ def test_mlp_and_awq_fast_and_checked_path(dev, M, pad, monkeypatch):
 
     monkeypatch.setattr(nv, "_host_module", Declines())
     assert torch.equal(fused_gelu_mlp(x, m1, m2, pad_size=pad), y) and torch.equal(awq(v), z)
+
+
+def test_arguments_outside_the_plain_case(dev):
+    """A rank above the largest one (its factors would not fit the extension's array) and numbers that are not whole are
+    refused as the checked path refuses them."""
+    from nunchaku_amd.models.linear import SVDQW4A4Linear
+    from nunchaku_amd.ops import fused_gelu_mlp
+
+    announce("host extension: rank 1040, pad_size 256.0")
+    m = SVDQW4A4Linear(256, 384, rank=1040, device=dev)
+    with torch.no_grad():
+        for p in m.parameters():
+            p.copy_(torch.ones(p.shape, dtype=p.dtype, device=dev))
+    x = synth.make_activations(16, 256, seed=1).to(dev).view(1, 16, 256)
+    m.lora_scales = [1.0] * 65
+    for _ in range(2):  # the call that converts the layer and the one behind it
+        with pytest.raises(ValueError, match="rank"):
+            m(x)
+    m1 = make_module(synth.make_layer(512, 256, 32, seed=1), dev)
+    m2 = make_module(synth.make_layer(256, 512, 32, seed=2), dev, act_unsigned=True)
+    fused_gelu_mlp(x, m1, m2)
+    with pytest.raises(TypeError):
+        fused_gelu_mlp(x, m1, m2, pad_size=256.0)
