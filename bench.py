@@ -45,12 +45,12 @@ INT8_PEAK_TOPS = 5000.0  # MI355X dense INT8 MFMA, the peak the metric is quoted
 FETCH_SCALE, WRITE_SCALE = 2.0, 1.0
 PROFILED_GEMM_FETCH_WRITE_KIB = {
     "flux_mlp_fc1": (143432.6, 110593.0),
-    "flux_qkv": (103458.7, 82944.7),
+    "flux_qkv": (124439.7, 82945.3),
     "flux_mlp_fc2": (154337.3, 27648.0),
     "qwen_batched_r128": (696300.5, 442369.8),
-    "c1_small": (12905.7, 13827.8),
-    "flux_single_nvfp4": (146101.8, 197586.7),
-    "flux_single_out_nvfp4": (121730.6, 28944.1),
+    "c1_small": (6719.3, 1536.0),
+    "flux_single_nvfp4": (141551.3, 197082.0),
+    "flux_single_out_nvfp4": (114618.8, 28512.4),
 }
 PROFILED_GEMM_TRAFFIC_BYTES = {w: (FETCH_SCALE * f + WRITE_SCALE * wr) * 1024 for w, (f, wr) in PROFILED_GEMM_FETCH_WRITE_KIB.items()}
 HBM_PEAK_GBS = 8000.0
