@@ -433,8 +433,10 @@ PyObject *awq_linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     const at::Tensor *x, *w, *s, *z, *bias = nullptr;
     if (!d || !params || !as_tensor(args[1], &x) || !as_tensor(PyDict_GetItem(params, s_qweight), &w) || !as_tensor(PyDict_GetItem(params, s_wscales), &s) ||
         !as_tensor(PyDict_GetItem(params, s_wzeros), &z)) Py_RETURN_NONE;
-    PyObject *b = PyDict_GetItem(params, s_bias);
-    if (b && b != Py_None && !as_tensor(b, &bias)) Py_RETURN_NONE;
+    // `module.bias` is what the instance's dictionary holds (None in a layer built without one), else the parameter; a bias
+    // anywhere else (a buffer, a property, an attribute of the class) is not the plain case
+    PyObject *own = PyDict_GetItem(d, s_bias), *b = own ? own : PyDict_GetItem(params, s_bias);
+    if (!b || (b != Py_None && !as_tensor(b, &bias))) Py_RETURN_NONE;
     PyObject *in = PyDict_GetItem(d, s_in_features), *out = PyDict_GetItem(d, s_out_features), *gs = PyDict_GetItem(d, s_group_size);
     int64_t n, k, group_size;
     if (!in || !out || !gs || !as_int(in, &k) || !as_int(out, &n) || !as_int(gs, &group_size) || x->dim() < 1 || x->size(-1) <= 0) Py_RETURN_NONE;

@@ -99,3 +99,47 @@ def test_rejects_bad_arguments(dev):
         awq_gemv_w4a16_cuda(x[:1], m.qweight, m.wscales, m.wzeros, 1, 64, 128, group_size=128)
     with pytest.raises(RuntimeError, match="GPU"):
         awq_gemv_w4a16_cuda(x[:1].cpu(), m.qweight, m.wscales, m.wzeros, 1, 64, 128)
+
+
+def test_bias_wherever_the_module_keeps_it(dev):
+    """The bias is what ``module.bias`` gives: a parameter, a tensor assigned to a layer built without one, a buffer, a
+    parametrization, a class attribute."""
+    from torch import nn
+    from torch.nn.utils import parametrize
+
+    from nunchaku_amd.models import AWQW4A16Linear
+    from nunchaku_amd.ops import awq_gemv_w4a16_cuda
+
+    oc, ic = 64, 128
+    announce("awq layer with its bias in other places than its parameters")
+    g = torch.Generator().manual_seed(1)
+    x = torch.randn(2, ic, generator=g).to(torch.bfloat16).to(dev)
+    bias = torch.randn(oc, generator=g).to(torch.bfloat16).to(dev)
+
+    def want(m, b):
+        return awq_gemv_w4a16_cuda(x, m.qweight, m.wscales, m.wzeros, 2, oc, ic, 64, b)
+
+    m, _ = _module(dev, oc, ic, seed=1, bias=False)
+    assert torch.equal(m(x), want(m, None)) and not torch.equal(want(m, bias), want(m, None))
+    m.bias = bias
+    assert torch.equal(m(x), want(m, bias))
+    del m.bias
+    m.register_buffer("bias", bias)
+    assert torch.equal(m(x), want(m, bias))
+
+    class Twice(nn.Module):
+        def forward(self, b):
+            return b * 2
+
+    m, _ = _module(dev, oc, ic, seed=1)
+    parametrize.register_parametrization(m, "bias", Twice())
+    assert torch.equal(m(x), want(m, m.bias.detach())) and not torch.equal(m(x), want(m, m.parametrizations.bias.original.detach()))
+
+    class WithClassBias(AWQW4A16Linear):
+        pass
+
+    m, _ = _module(dev, oc, ic, seed=1, bias=False)
+    del m.bias
+    m.__class__ = WithClassBias
+    WithClassBias.bias = bias
+    assert torch.equal(m(x), want(m, bias))
