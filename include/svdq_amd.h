@@ -169,9 +169,7 @@ typedef struct svdq_gemm_args {
     const void *next_lora_down;   /* native proj_down of the next layer ([N, R_down]) or NULL       */
     float *next_lora_act_out;     /* fp32 [M_pad, R_down]; fully written by the call                */
     int64_t M_pad, N, K;
-    int64_t M_out, N_out;   /* shape of `out` (M_out <= M_pad, N_out <= N).  Without `out`: the rows of
-                               qout / oscales / next_lora_act_out the caller will read (rounded up to
-                               whole tiles; what the others hold is unspecified), 0 for all M_pad     */
+    int64_t M_out, N_out;   /* shape of `out` (M_out <= M_pad, N_out <= N); ignored without `out`          */
     int64_t R_up, R_down;
     float alpha;            /* per-tensor scale (NVFP4 wtscale; the reference asserts 1 for INT4,
                                launch_impl.cuh:107, this library applies whatever is given)          */

@@ -1,6 +1,7 @@
 // Host entry point of operator 2 (argument validation, kernel variant selection).  The device code
 // lives in gemm_kernel.h and is instantiated per variant in gemm_variant.hip.
 #include "gemm_params.h"
+#include "internal_api.h"
 
 using namespace svdq;
 
@@ -285,8 +286,8 @@ bool needs_next_epilogue(const svdq_gemm_args *a) {
     return a->qout != nullptr || a->next_lora_down != nullptr || a->rotary_emb != nullptr || a->fuse_silu || a->out_vk != nullptr;
 }
 
-// Rows the call has to work out: those of `out` where nothing else is written, those the caller names where `out` is not
-// given, all of them otherwise.
+// Rows the call has to work out: those of `out` where nothing else is written, those that svdq_gemm_w4a4_rows names where
+// `out` is not given, all of them otherwise.
 int rows_needed(const svdq_gemm_args *a) {
     if (a->out_q || a->out_vk || (a->out && (a->qout || a->next_lora_down)) || a->M_out == 0) return (int)a->M_pad;
     return (int)a->M_out;
@@ -748,9 +749,26 @@ int gemm_entry(const svdq_gemm_args *a, void *stream, bool noalloc) {
 }
 }  // namespace
 
-extern "C" int svdq_gemm_w4a4(const svdq_gemm_args *a, void *stream) { return gemm_entry(a, stream, false); }
+namespace {
+// `M_out` without `out` is the number of rows to work out (rows_needed): not a caller's to set, it is the shape of `out`
+int public_entry(const svdq_gemm_args *a, void *stream, bool noalloc) {
+    if (!a || a->out || a->M_out == 0) return gemm_entry(a, stream, noalloc);
+    svdq_gemm_args all = *a;
+    all.M_out = 0;
+    return gemm_entry(&all, stream, noalloc);
+}
+}  // namespace
 
-extern "C" int svdq_gemm_w4a4_noalloc(const svdq_gemm_args *a, void *stream) { return gemm_entry(a, stream, true); }
+extern "C" int svdq_gemm_w4a4(const svdq_gemm_args *a, void *stream) { return public_entry(a, stream, false); }
+
+extern "C" int svdq_gemm_w4a4_noalloc(const svdq_gemm_args *a, void *stream) { return public_entry(a, stream, true); }
+
+extern "C" int svdq_gemm_w4a4_rows(const svdq_gemm_args *a, int64_t rows, int noalloc, void *stream) {
+    SVDQ_REQUIRE(a && !a->out && rows > 0, "gemm: rows go with a call without `out`");
+    svdq_gemm_args some = *a;
+    some.M_out = rows;
+    return gemm_entry(&some, stream, noalloc != 0);
+}
 
 extern "C" int svdq_release_workspaces(void) {
     std::lock_guard<std::mutex> lock(g_ws_mutex);

@@ -22,7 +22,7 @@
 
 #include <vector>
 
-#include "../../include/svdq_amd.h"
+#include "internal_api.h"
 
 namespace {
 
@@ -290,13 +290,12 @@ PyObject *gelu_mlp(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     g1.next_lora_down = l2->q.lora_down;
     g1.next_lora_act_out = a2.lora;
     g1.R_down = l2->rank;
-    g1.M_out = M;  // (layer 2 reads nothing of the padding rows that reaches its output)
     g2.out = out.data_ptr();
     g2.M_out = M;
     int rc;
     Py_BEGIN_ALLOW_THREADS
     rc = svdq_quantize_w4a4_act_fuse_lora(&q, st);
-    if (rc == SVDQ_OK) rc = gemm(g1, no_alloc, st);
+    if (rc == SVDQ_OK) rc = svdq_gemm_w4a4_rows(&g1, M, no_alloc, st);  // (layer 2 reads nothing of the padding rows that reaches its output)
     if (rc == SVDQ_OK) rc = gemm(g2, no_alloc, st);
     Py_END_ALLOW_THREADS
     if (rc != SVDQ_OK) return raise(rc);

@@ -126,6 +126,12 @@ def test_gemm_rejects_bad_arguments(lib):
     bad = nv.GemmArgs.from_buffer_copy(a)
     bad.R_down = 32  # without next_lora_down / next_lora_act_out
     assert lib.svdq_gemm_w4a4(ctypes.byref(bad), None) == -1
+    # without `out`, M_out means nothing: the call gets as far as the next mistake
+    bad.out = None
+    bad.qout = bad.oscales = bad.next_smooth_rcp = 16
+    bad.M_out = 300
+    assert lib.svdq_gemm_w4a4(ctypes.byref(bad), None) == -1
+    assert b"next_lora_down" in lib.svdq_last_error()
     # the norm + rotary epilogue: needs both norm weights, three equal parts of whole heads, enough table rows
     bad = nv.GemmArgs.from_buffer_copy(a)
     bad.norm_q = 16

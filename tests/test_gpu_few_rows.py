@@ -92,3 +92,38 @@ def test_against_large_tiles(dev, kind, M, K, N, R, fp4, monkeypatch):
         logical = packing.act_to_logical(got["qout"].cpu(), N, fp4=fp4, unsigned=not fp4)
         assert torch.equal(logical.to(codes.dtype), codes)
         assert torch.equal(packing.scales_to_logical(got["oscales"].cpu(), fp4).view(torch.uint8), scales.view(torch.uint8))
+
+
+@pytest.mark.parametrize("fp4", [False, True])
+def test_all_rows_of_qout_whatever_M_out(dev, fp4):
+    """``M_out`` and ``N_out`` are the shape of ``out``: a call of the C ABI that writes ``qout`` alone works out all M_pad rows,
+    whatever they hold."""
+    import ctypes
+
+    from nunchaku_amd import _native as nv
+    from nunchaku_amd import packing
+
+    M, K, N, R, R2 = 512, 256, 384, 16, 32
+    announce(f"qout without out, M_out set, fp4={fp4}")
+    m, nxt = make_module(synth.make_layer(N, K, R, seed=3, fp4=fp4), dev), make_module(synth.make_layer(128, N, R2, seed=9, fp4=fp4), dev)
+    t, n = m.native_tensors(), nxt.native_tensors()
+    act, asc, la = m.quantize(synth.make_activations(M, K, seed=M).to(dev))
+
+    def run(M_out):
+        qout = torch.full((M, packing.act_nbytes_per_row(N, fp4)), 0xA5, dtype=torch.uint8, device=dev)
+        osc = torch.full((N // (16 if fp4 else 64), M * (1 if fp4 else 2)), 0xA5, dtype=torch.uint8, device=dev)
+        down = torch.full((M, R2), float("nan"), dtype=torch.float32, device=dev)
+        a = nv.GemmArgs(act=act.data_ptr(), ascales=asc.data_ptr(), wgt=t["qweight"].data_ptr(), wscales=t["wscales"].data_ptr(),
+                        colnorm=nv.ptr(t["wscales"].colnorm), bias=t["bias"].data_ptr(), wcscales=nv.ptr(t["wcscales"]), lora_act_in=la.data_ptr(),
+                        lora_up=t["proj_up"].data_ptr(), qout=qout.data_ptr(), oscales=osc.data_ptr(), next_smooth_rcp=n["smooth_factor"].data_ptr(),
+                        next_lora_down=n["proj_down"].data_ptr(), next_lora_act_out=down.data_ptr(), M_pad=M, N=N, K=K, M_out=M_out, R_up=R, R_down=R2,
+                        alpha=m.alpha, fp4=int(fp4))
+        nv.launch(nv.lib().svdq_gemm_w4a4, ctypes.byref(a), dev)
+        torch.cuda.synchronize()
+        return qout, osc, down
+
+    want = run(0)
+    assert not torch.isnan(want[2]).any()
+    for M_out in (40, M, M + 1):
+        for a, b in zip(run(M_out), want):
+            assert torch.equal(a, b), M_out
