@@ -143,8 +143,8 @@ int svdq_quantize_w4a4_act_fuse_lora(const svdq_quantize_args *args, void *strea
  * synchronises.  svdq_release_workspaces frees them all.  A call that would have to allocate while its stream is
  * being captured returns SVDQ_EUNSUPPORTED: make the call once before the capture (the block is then there), or
  * use svdq_gemm_w4a4_noalloc, the variant for callers that cannot allocate.
- * Calls on one stream run in order and share the workspace safely; the same stream must not be used
- * from two threads at once.
+ * Calls on one stream run in order and share the workspace safely, also when several threads make them: the
+ * launches of a call that uses the workspace are enqueued under one lock.
  *
  * Ranks: R_up and R_down are multiples of 16 up to 1024 (the reference's MAX_RANK, lora.cuh:22).
  * ------------------------------------------------------------------------------------------ */
@@ -231,9 +231,10 @@ int svdq_gemm_w4a4(const svdq_gemm_args *args, void *stream);
  * of allocating one: no hipMalloc, hipFree or other allocating call is made.  A call whose need exceeds
  * the array returns SVDQ_EUNSUPPORTED with a message that says how much it wanted (examples that fit:
  * INT4 M_pad = 256, K = N = 3072 split six ways (k_split = 6), 18.9 MB of partial sums; next_lora_down at
- * M_pad = 4608, N = 12288, R_down = 32, 28.3 MB of shares).  All calls on one GPU share the array, whatever their stream: calls that overlap
- * in time on one GPU race with each other.  What a launch needs to be zero at its start is cleared by a
- * fill kernel on `stream` first. */
+ * M_pad = 4608, N = 12288, R_down = 32, 28.3 MB of shares).  All calls on one GPU share the array, whatever their stream: the launches
+ * of a call are enqueued under one lock, so several threads may call it on one stream, but calls on different
+ * streams of a GPU that overlap in time race with each other.  What a launch needs to be zero at its start is
+ * cleared by a fill kernel on `stream` first. */
 int svdq_gemm_w4a4_noalloc(const svdq_gemm_args *args, void *stream);
 
 /* Frees every workspace block svdq_gemm_w4a4 has allocated, on all devices, after waiting for the work

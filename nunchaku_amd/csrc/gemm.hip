@@ -179,15 +179,17 @@ Workspace *get_workspace(int dev, hipStream_t stream, size_t zero_bytes, size_t 
 constexpr size_t NOALLOC_ZERO_BYTES = 1u << 20, NOALLOC_SCRATCH_BYTES = 80u << 20;
 static __device__ __align__(256) unsigned char scratch[NOALLOC_ZERO_BYTES + NOALLOC_SCRATCH_BYTES];
 uint8_t *g_scratch_ptr[64] = {nullptr};  // the array's device address on each GPU, asked once per GPU
+// Held from before the fill kernel until the last kernel of a call that uses the array has been enqueued: between the GEMM and
+// the sums of its shares no other thread's GEMM on the stream may write shares of its own to the same place.
 std::mutex g_scratch_mutex;
 
-// the array's address on device `dev` (which is the current device), or nullptr with the error text set
+// (the caller holds g_scratch_mutex) the array's address on device `dev` (which is the current device), or nullptr with the error
+// text set
 uint8_t *scratch_address(int dev) {
     if (dev < 0 || dev >= 64) {
         fail(SVDQ_ELAUNCH, "gemm: device index %d out of range", dev);
         return nullptr;
     }
-    std::lock_guard<std::mutex> lock(g_scratch_mutex);
     if (!g_scratch_ptr[dev]) {
         void *ptr = nullptr;
         hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
@@ -208,7 +210,10 @@ struct WorkspaceView {
     Workspace *owner;  // the allocation behind it (nullptr for the fixed array)
 };
 
-// (the caller holds g_ws_mutex when `noalloc` is false) false, with the error text set, on failure
+// Every call that uses a workspace holds this lock from here until all its launches have been enqueued.
+std::mutex &workspace_mutex(bool noalloc) { return noalloc ? g_scratch_mutex : g_ws_mutex; }
+
+// (the caller holds workspace_mutex(noalloc)) false, with the error text set, on failure
 bool acquire_workspace(bool noalloc, int dev, hipStream_t st, size_t zero_bytes, size_t scratch_bytes, WorkspaceView *v) {
     if (!noalloc) {
         Workspace *w = get_workspace(dev, st, zero_bytes, scratch_bytes);
@@ -481,8 +486,7 @@ int gemm_int4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool no
     const size_t share_bytes = p.next_down ? lora_share_bytes(a, nblocks) : 0;  // every column block's share of the next projection
     const size_t vk_bytes = p.vk ? vk_share_bytes(a, p.full_blocks + p.half_blocks) : 0;  // every row block's linear-attention sums
     if (kparts == 1 && !p.next_down && !p.vk) return next ? g6::launch_next(p, ntiles, st) : g6::launch_plain(p, ntiles, st);
-    std::unique_lock<std::mutex> lock(g_ws_mutex, std::defer_lock);
-    if (!noalloc) lock.lock();
+    std::lock_guard<std::mutex> lock(workspace_mutex(noalloc));
     const size_t cnt_pad = kparts > 1 ? (cnt_bytes + 255) & ~(size_t)255 : 0;
     WorkspaceView w;
     const size_t scratch_bytes = part_bytes + share_bytes + vk_bytes;
@@ -566,8 +570,7 @@ int gemm_fp4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool noa
     const size_t share_bytes = p.next_down ? lora_share_bytes(a, a->N / 128) : 0;
     const size_t vk_bytes = p.vk ? vk_share_bytes(a, a->M_pad / 32) : 0;  // (this kernel: per 32-row slab)
     if (!shared_tiles && !share_bytes && !vk_bytes) return next ? launch_gemm_fp4_v5(p, nwg, st) : launch_gemm_fp4_v4(p, nwg, st);
-    std::unique_lock<std::mutex> lock(g_ws_mutex, std::defer_lock);
-    if (!noalloc) lock.lock();
+    std::lock_guard<std::mutex> lock(workspace_mutex(noalloc));
     const size_t zero_bytes = shared_tiles ? (size_t)ntiles * 4 : 0, part_bytes = shared_tiles ? (size_t)2 * nwg * 256 * 64 * 16 : 0;
     const size_t scratch_bytes = part_bytes + share_bytes + vk_bytes;
     WorkspaceView w;
@@ -649,8 +652,7 @@ int gemm_direct(const svdq_gemm_args *a, int shape, hipStream_t st, int dev, boo
     const size_t share_bytes = p.next_down ? lora_share_bytes(a, a->N / 128) : 0;
     const size_t vk_bytes = p.vk ? vk_share_bytes(a, a->M_pad / 32) : 0;
     if (!share_bytes && !vk_bytes) return launch();
-    std::unique_lock<std::mutex> lock(g_ws_mutex, std::defer_lock);
-    if (!noalloc) lock.lock();
+    std::lock_guard<std::mutex> lock(workspace_mutex(noalloc));
     WorkspaceView w;
     if (!acquire_workspace(noalloc, dev, st, 0, share_bytes + vk_bytes, &w)) return noalloc && share_bytes + vk_bytes > NOALLOC_SCRATCH_BYTES ? SVDQ_EUNSUPPORTED : SVDQ_ELAUNCH;
     p.next_lora_part = (float *)w.scratch;

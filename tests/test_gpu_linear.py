@@ -213,3 +213,42 @@ def test_one_layer_from_two_threads(dev):
     for t in threads:
         t.join()
     assert not errors, errors
+
+
+@pytest.mark.parametrize("no_alloc", [True, False])
+@pytest.mark.parametrize("fp4,k_split", [(False, None), (False, 1), (True, None)])
+def test_one_layer_pair_from_two_threads(dev, fp4, k_split, no_alloc, monkeypatch):
+    """The first GEMM of the fused MLP leaves shares of the second layer's low-rank input in the workspace, which the kernel
+    behind it adds up: both launches are enqueued under the workspace's lock, so that a thread on the same stream never
+    puts its own shares between them, in the fixed scratch as in an allocated block."""
+    import threading
+
+    from nunchaku_amd.ops import fused_gelu_mlp
+    from nunchaku_amd.ops import gemm as gemm_mod
+
+    announce(f"a fused MLP called from two threads, fp4={fp4} k_split={k_split} no_alloc={no_alloc}")
+    monkeypatch.setattr(gemm_mod, "NO_ALLOC", no_alloc)
+    monkeypatch.setattr(gemm_mod, "K_SPLIT", k_split)
+    m1, m2 = make_module(synth.make_layer(1024, 256, 32, seed=1, fp4=fp4), dev), make_module(synth.make_layer(256, 1024, 64, seed=2, fp4=fp4), dev, act_unsigned=not fp4)
+    xs = [synth.make_activations(rows, 256, seed=rows).to(dev).view(1, rows, 256) for rows in (200, 250)]
+    want = [fused_gelu_mlp(x, m1, m2).clone() for x in xs]
+    torch.cuda.synchronize()
+    errors = []
+
+    def work(x, y):
+        try:
+            for _ in range(20):
+                got = [fused_gelu_mlp(x, m1, m2) for _ in range(10)]  # (enqueued without a wait: the threads' calls alternate)
+                torch.cuda.synchronize()
+                if not all(torch.equal(g, y) for g in got):
+                    errors.append(f"rows={x.shape[1]}: a call differs")
+                    return
+        except Exception as e:  # (an exception in a thread would otherwise pass unnoticed)
+            errors.append(repr(e))
+
+    threads = [threading.Thread(target=work, args=a) for a in zip(xs, want)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
