@@ -173,6 +173,15 @@ bool as_int(PyObject *o, int64_t *v) {
     return false;
 }
 
+// what `if o:` decides; false (and no exception left) where that raises
+bool as_bool(PyObject *o, bool *v) {
+    const int r = PyObject_IsTrue(o);
+    *v = r > 0;
+    if (r >= 0) return true;
+    PyErr_Clear();
+    return false;
+}
+
 Layer *layer_of(PyObject *capsule) { return (Layer *)PyCapsule_GetPointer(capsule, LAYER); }
 
 #define SVDQ_NARGS(n)                                                              \
@@ -243,8 +252,8 @@ PyObject *linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
             !given->is_contiguous() || given->numel() != M * l->N || given->size(-1) != l->N) Py_RETURN_NONE;
     }
     int64_t k_split;
-    if (!as_int(args[4], &k_split)) Py_RETURN_NONE;
-    const bool no_alloc = args[5] == Py_True;
+    bool no_alloc;
+    if (!as_int(args[4], &k_split) || !as_bool(args[5], &no_alloc)) Py_RETURN_NONE;
     at::Tensor out = given ? given->view({B, S, l->N}) : new_bf16({B, S, l->N}, l->device);
     hipStream_t st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)l->device).stream();
     Scratch mem(Activations(*l, M_pad, nullptr).bytes, st);
@@ -272,11 +281,11 @@ PyObject *gelu_mlp(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     const at::Tensor *x;
     float sc1[MAX_GROUPS], sc2[MAX_GROUPS];
     int64_t pad, k_split;
-    if (!as_int(args[5], &pad) || !as_int(args[6], &k_split) || !as_tensor(args[4], &x) || !plain_activations(*l1, *x) || l2->device != l1->device || l1->N != l2->K || l1->g.fp4 != l2->g.fp4 || pad <= 0 || pad % 256 ||
+    bool no_alloc;
+    if (!as_int(args[5], &pad) || !as_int(args[6], &k_split) || !as_bool(args[7], &no_alloc) || !as_tensor(args[4], &x) || !plain_activations(*l1, *x) || l2->device != l1->device || l1->N != l2->K || l1->g.fp4 != l2->g.fp4 || pad <= 0 || pad % 256 ||
         !unchanged(*l1, args[1]) || !unchanged(*l2, args[3]) || !read_lora_scales(args[1], (int)(l1->rank + 15) / 16, sc1) ||
         !read_lora_scales(args[3], (int)(l2->rank + 15) / 16, sc2)) Py_RETURN_NONE;
     const int64_t B = x->size(0), S = x->size(1), M = B * S, M_pad = (M + pad - 1) / pad * pad;
-    const bool no_alloc = args[7] == Py_True;
     at::Tensor out = new_bf16({B, S, l2->N}, l1->device);
     hipStream_t st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)l1->device).stream();
     const size_t first = Activations(*l1, M_pad, nullptr).bytes;
@@ -321,8 +330,9 @@ PyObject *qkv_norm_rope(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     at::Tensor out;
     const at::Tensor *qkv[3] = {nullptr, nullptr, nullptr};
     int64_t attn_tokens, k_split;
+    bool no_alloc;
     const double norm_eps = PyFloat_AsDouble(args[8]);
-    if ((norm_eps == -1.0 && PyErr_Occurred()) || !as_int(args[7], &attn_tokens) || !as_int(args[9], &k_split)) {
+    if ((norm_eps == -1.0 && PyErr_Occurred()) || !as_int(args[7], &attn_tokens) || !as_int(args[9], &k_split) || !as_bool(args[10], &no_alloc)) {
         PyErr_Clear();
         Py_RETURN_NONE;
     }
@@ -338,7 +348,6 @@ PyObject *qkv_norm_rope(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     } else {
         out = new_bf16({M_pad, l->N}, l->device);
     }
-    const bool no_alloc = args[10] == Py_True;
     hipStream_t st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)l->device).stream();
     Scratch mem(Activations(*l, M_pad, nullptr).bytes, st);
     const Activations a(*l, M_pad, (uint8_t *)mem.ptr);

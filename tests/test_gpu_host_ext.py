@@ -101,3 +101,29 @@ def test_arguments_outside_the_plain_case(dev):
     fused_gelu_mlp(x, m1, m2)
     with pytest.raises(TypeError):
         fused_gelu_mlp(x, m1, m2, pad_size=256.0)
+
+
+def test_a_true_NO_ALLOC_of_any_type(dev, monkeypatch):
+    """``NO_ALLOC = 1`` selects the fixed scratch as ``True`` does, through every call of the extension: a split that does not
+    fit it is refused."""
+    from nunchaku_amd import packing
+    from nunchaku_amd.ops import fused_gelu_mlp, fused_qkv_norm_rottary
+    from nunchaku_amd.ops import gemm as gemm_mod
+
+    announce("host extension: NO_ALLOC = 1")
+    m1 = make_module(synth.make_layer(2048, 1024, 16, seed=1), dev)
+    m2 = make_module(synth.make_layer(1024, 2048, 16, seed=2), dev, act_unsigned=True)
+    x = synth.make_activations(2048, 1024, seed=1).to(dev).view(1, 2048, 1024)
+    m3 = make_module(synth.make_layer(2304, 1024, 16, seed=3), dev)
+    norm = torch.nn.RMSNorm(128, device=dev, dtype=torch.bfloat16)
+    rot = packing.repack_rotemb(torch.zeros(2048, 128, device=dev))
+    m1(x), fused_gelu_mlp(x, m1, m2), fused_qkv_norm_rottary(x, m3, norm, norm, rot)
+    monkeypatch.setattr(gemm_mod, "K_SPLIT", 16)  # 128 tiles and more x 16 parts x 128 KB
+    for value in (True, 1):
+        monkeypatch.setattr(gemm_mod, "NO_ALLOC", value)
+        with pytest.raises(NotImplementedError, match="fixed scratch"):
+            m1(x)
+        with pytest.raises(NotImplementedError, match="fixed scratch"):
+            fused_gelu_mlp(x, m1, m2)
+        with pytest.raises(NotImplementedError, match="fixed scratch"):
+            fused_qkv_norm_rottary(x, m3, norm, norm, rot)
