@@ -27,24 +27,25 @@ struct AwqParams {
 // 32 codes of one channel, the 16 bytes a lane holds of a 32-channel half, to the second operands of four
 // v_mfma_f32_16x16x32_bf16: operand q holds bf16(code * scale + zero) of input channels 8 q ... 8 q + 7.  A code as a byte is
 // the E4M3 pattern of code * 2^-9 (subnormals and the first binade are evenly spaced), so the hardware conversion makes two
-// floats per instruction; s512 = 512 * scale undoes the 2^-9 exactly and the sum is rounded once, by the fused multiply-add,
-// before the rounding to bf16.  (One v_cvt_f32_ubyte per code: 11.1 us against 10.0 at K = 3072, N = 18432, one row, the
-// kernel being bound by its vector instructions.)
-__device__ inline void dequantize32(u32x4_t w, float s512, float zero, u32x4_t (&wb)[4]) {
+// floats per instruction, and its scale operand, 2^9, makes them the codes themselves: the scale is used as it is stored (512
+// times it is infinite from 2^119 on) and the sum is rounded once, by the fused multiply-add, before the rounding to bf16.
+// (One v_cvt_f32_ubyte per code: 11.1 us against 10.0 at K = 3072, N = 18432, one row, the kernel being bound by its vector
+// instructions.)
+__device__ inline void dequantize32(u32x4_t w, float scale, float zero, u32x4_t (&wb)[4]) {
     typedef float f32x2_t __attribute__((ext_vector_type(2)));
     float f[4][8];  // word i2, nibble p + 4 b = channel 8 p + 2 i2 + b
 #pragma unroll
     for (int i2 = 0; i2 < 4; i2++) {
         const uint32_t even = w[i2] & 0x0F0F0F0Fu, odd = (w[i2] >> 4) & 0x0F0F0F0Fu;
-        const f32x2_t e0 = __builtin_amdgcn_cvt_pk_f32_fp8(even, false), e1 = __builtin_amdgcn_cvt_pk_f32_fp8(even, true);
-        const f32x2_t o0 = __builtin_amdgcn_cvt_pk_f32_fp8(odd, false), o1 = __builtin_amdgcn_cvt_pk_f32_fp8(odd, true);
+        const f32x2_t e0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(even, 512.0f, false), e1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(even, 512.0f, true);
+        const f32x2_t o0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(odd, 512.0f, false), o1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(odd, 512.0f, true);
         f[i2][0] = e0[0]; f[i2][2] = e0[1]; f[i2][4] = e1[0]; f[i2][6] = e1[1];
         f[i2][1] = o0[0]; f[i2][3] = o0[1]; f[i2][5] = o1[0]; f[i2][7] = o1[1];
     }
 #pragma unroll
     for (int q = 0; q < 4; q++)
 #pragma unroll
-        for (int i2 = 0; i2 < 4; i2++) wb[q][i2] = pack_bf16x2(__builtin_fmaf(f[i2][q], s512, zero), __builtin_fmaf(f[i2][q + 4], s512, zero));
+        for (int i2 = 0; i2 < 4; i2++) wb[q][i2] = pack_bf16x2(__builtin_fmaf(f[i2][q], scale, zero), __builtin_fmaf(f[i2][q + 4], scale, zero));
 }
 
 // the reference stores bf16 and adds the bias to that (linear.py:183-185): two roundings
@@ -61,7 +62,7 @@ __device__ inline void store_result(const AwqParams &p, int m, int row, float su
 // instructions as dequantized (above), the first being x[m = l % 16] of the same channels, zero for rows beyond M and
 // channels beyond K.  The result tile has channel l % 16 and rows 4 (l / 16) + [0, 4) in lane l; the waves' tiles meet in
 // LDS once per BATCH tiles and are added in ascending order.
-// Per step and wave this leaves 84 vector instructions for 32 codes per lane, where a workgroup per tile, with its
+// Per step and wave this leaves about 85 vector instructions for 32 codes per lane, where a workgroup per tile, with its
 // activations in LDS, needed 140.  Measured with weights from HBM (12 layers in turn), before / now: K = 3072,
 // N = 18432 one row 11.9 / 10.7 us, four 13.0 / 10.8, eight 15.7 / 11.4; K = 4096, N = 20480, eight rows 24.1 / 15.3;
 // K = 3072, N = 9216, one row 8.5 / 8.0.  About 3 us of that are launch and latency, the rest 4.2 TB/s.  Further ahead is slower
@@ -82,14 +83,16 @@ __global__ void __launch_bounds__(64 * WAVES, 2) awq_gemv_rows_kernel(AwqParams 
 
     u32x4_t x[SPW][4];
     uint32_t w_off[SPW], s_off[SPW];
+    bool live[SPW];  // the lane's channels of the step exist
 #pragma unroll
     for (int j = 0; j < SPW; j++) {
         const int cb = (wave + WAVES * j) * 2 + (kb >> 1), block = cb < kblocks ? cb : kblocks - 1;  // the lane's 64-channel block
+        live[j] = cb < kblocks;
         const uint16_t *xp = p.x + (size_t)(n < p.M ? n : 0) * p.K + block * 64 + 32 * (kb & 1);
 #pragma unroll
         for (int q = 0; q < 4; q++) {
             const u32x4_t v = *(const u32x4_t *)(xp + 8 * q);
-            x[j][q] = cb < kblocks && n < p.M ? v : u32x4_t{0, 0, 0, 0};
+            x[j][q] = live[j] && n < p.M ? v : u32x4_t{0, 0, 0, 0};
         }
         w_off[j] = (uint32_t)(n >> 2) * (uint32_t)(kblocks * 128) + (uint32_t)(n & 3) * 32u + (uint32_t)(kb & 1) * 16u + (uint32_t)block * 128u;
         s_off[j] = (uint32_t)block * (uint32_t)p.N * 2u + (uint32_t)n * 2u;
@@ -127,7 +130,8 @@ __global__ void __launch_bounds__(64 * WAVES, 2) awq_gemv_rows_kernel(AwqParams 
 #pragma unroll
             for (int j = 0; j < SPW; j++) {
                 u32x4_t wb[4];
-                dequantize32(d.w[j], bf16_bits_to_f32(d.s[j]) * 512.0f, bf16_bits_to_f32(d.z[j]), wb);
+                // (channels beyond K have weights of zero: the repeated block's may be infinite, and zero times that is no zero)
+                dequantize32(d.w[j], live[j] ? bf16_bits_to_f32(d.s[j]) : 0.f, live[j] ? bf16_bits_to_f32(d.z[j]) : 0.f, wb);
 #pragma unroll
                 for (int q = 0; q < 4; q++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[j][q]), __builtin_bit_cast(bf16x8_t, wb[q]), acc, 0, 0, 0);
             }
@@ -196,7 +200,7 @@ __global__ void __launch_bounds__(256) awq_gemv_mfma_kernel(AwqParams p) {
             }
         }
         u32x4_t wb[4];
-        dequantize32(w, s * 512.0f, z, wb);
+        dequantize32(w, s, z, wb);
 #pragma unroll
         for (int q = 0; q < 4; q++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, xa[q]), __builtin_bit_cast(bf16x8_t, wb[q]), acc, 0, 0, 0);
     };

@@ -143,3 +143,31 @@ def test_bias_wherever_the_module_keeps_it(dev):
     m.__class__ = WithClassBias
     WithClassBias.bias = bias
     assert torch.equal(m(x), want(m, bias))
+
+
+@pytest.mark.parametrize("K", [64, 192, 1088, 4160])
+def test_scales_and_zeros_up_to_infinity(dev, K):
+    """A scale near the top of bf16's range and an infinite zero in the last group of channels, at lengths of K that end inside a
+    step of 128 channels and leave waves without a step: each only reaches the outputs of its own channel, and there gives
+    what the weights bf16(code * scale + zero) give."""
+    from nunchaku_amd.ops import awq_gemv_w4a16_cuda
+
+    N, M = 64, 3
+    announce(f"awq gemv with extreme scales and zeros K={K}")
+    g = torch.Generator().manual_seed(K)
+    codes = torch.randint(0, 16, (N, K), generator=g)
+    scales = (0.5 + torch.rand(K // 64, N, generator=g)).to(torch.bfloat16)
+    zeros = (torch.randint(-16, 17, (K // 64, N), generator=g) / 8).to(torch.bfloat16)  # (sums with code * scale are exact in fp32)
+    scales[-1, 5], zeros[-1, 5] = 2.0**120, 0.0
+    scales[0, 21] = 2.0**123
+    zeros[-1, 9], zeros[-1, 40] = float("inf"), float("-inf")
+    x = (2.0**-20 * (0.5 + torch.rand(M, K, generator=g))).to(torch.bfloat16)  # (positive: an infinite weight gives infinity)
+    qweight = torch.from_numpy(awq.pack_w4(codes.numpy()).view(np.int32).copy())
+    out = awq_gemv_w4a16_cuda(x.to(dev), qweight.to(dev), scales.to(dev), zeros.to(dev), M, N, K).cpu()
+    w = awq.dequant(codes, scales, zeros)
+    want = x.double() @ w.double().T
+    finite = torch.isfinite(want)
+    assert (~finite).sum() == 2 * M and torch.equal(out[~finite].double(), want[~finite])
+    # one rounding to bf16 and fp32 sums of K positive and negative terms
+    bound = 2.0**-8 * want.abs() + K * 2.0**-24 * (x.double() @ w.double().abs().T)
+    assert ((out.double() - want).abs() <= bound)[finite].all()
