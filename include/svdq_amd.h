@@ -189,7 +189,8 @@ typedef struct svdq_gemm_args {
                                slot s = 4 nt + q, lane l = r + 32 h hold floats 32 nt + 8 q + 4 h + [0, 4)
                                of row 32 b + r, where float 2i of a row is sin and 2i + 1 cos of pair i
                                (svdq_repack_rotemb writes it from the reference's pack_rotemb order)  */
-    int64_t rot_rows;       /* rows of rotary_emb: M_out <= rot_rows <= M_pad, a multiple of 32      */
+    int64_t rot_rows;       /* rows of rotary_emb: M_out (with out_q: attn_tokens, and at least 32) <= rot_rows
+                               <= M_pad, a multiple of 32                                           */
     float norm_eps;         /* the reference uses 1e-6 (launch_impl.cuh:374)                        */
     int32_t k_split;        /* 0: the library decides.  n > 0: split every output tile along K into n parts
                                whose partial sums meet in the workspace (1: never split); a tuning and

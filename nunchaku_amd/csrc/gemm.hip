@@ -730,7 +730,8 @@ int gemm_entry(const svdq_gemm_args *a, void *stream, bool noalloc) {
         } else {
             SVDQ_REQUIRE(a->out && a->N_out == a->N, "gemm: rotary_emb goes with a full-width `out` (or with out_q, out_k, out_v)");
         }
-        SVDQ_REQUIRE(a->rot_rows >= covered && a->rot_rows <= a->M_pad && a->rot_rows % 32 == 0,
+        // (the kernels read the last block of the table for rows beyond it: an empty table has none)
+        SVDQ_REQUIRE(a->rot_rows > 0 && a->rot_rows >= covered && a->rot_rows <= a->M_pad && a->rot_rows % 32 == 0,
                      "gemm: rotary_emb has %lld rows for %lld output rows (must cover them, in whole blocks of 32)", (long long)a->rot_rows, covered);
         SVDQ_REQUIRE(((uintptr_t)a->rotary_emb % 16 == 0) && ((uintptr_t)a->norm_q % 8 == 0) && ((uintptr_t)a->norm_k % 8 == 0),
                      "gemm: rotary_emb / norm pointers are not aligned");

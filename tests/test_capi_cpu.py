@@ -145,6 +145,15 @@ def test_gemm_rejects_bad_arguments(lib):
     bad.rot_rows = 128
     assert lib.svdq_gemm_w4a4(ctypes.byref(bad), None) == -1
     assert b"rows" in lib.svdq_last_error()
+    # q, k and v apart with no token to attend to: still a table of one block at least (the kernels read its last block for the
+    # rows beyond it)
+    bad.out = None
+    bad.M_out = bad.N_out = 0
+    bad.out_q = bad.out_k = bad.out_v = 16
+    bad.qkv_rows, bad.attn_tokens, bad.rot_rows = 256, 0, 0
+    bad.qkv_head_stride = (ctypes.c_int64 * 3)(256 * 128, 256 * 128, 256 * 128)
+    assert lib.svdq_gemm_w4a4(ctypes.byref(bad), None) == -1
+    assert b"rotary_emb has 0 rows" in lib.svdq_last_error()
 
 
 def test_awq_gemv_rejects_bad_arguments(lib):
