@@ -466,8 +466,9 @@ int gemm_int4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool no
         p.kparts = (int)(a->k_split < kgroups ? a->k_split : kgroups);
     } else {
         choose_tiles_int4(a, ncu, &p.full_blocks, &p.half_blocks, &p.kparts);
-        if (noalloc && a->out_vk && vk_share_bytes(a, p.full_blocks + p.half_blocks) > NOALLOC_SCRATCH_BYTES) {
-            // (more row blocks, more shares: not where only 128-row blocks' fit the fixed scratch)
+        if (a->out_vk && vk_share_bytes(a, p.full_blocks + p.half_blocks) > NOALLOC_SCRATCH_BYTES && vk_share_bytes(a, a->M_pad / g6::BM) <= NOALLOC_SCRATCH_BYTES) {
+            // (more row blocks, more shares: not where only 128-row blocks' fit the fixed scratch, and not in the other entry
+            // point either, which gives the same bits)
             p.full_blocks = (int)(a->M_pad / g6::BM);
             p.half_blocks = 0;
         }
@@ -745,8 +746,14 @@ int gemm_entry(const svdq_gemm_args *a, void *stream, bool noalloc) {
     const int ncu = compute_units(dev);
     if (ncu <= 0) return fail(SVDQ_ELAUNCH, "gemm: cannot query the number of compute units");
     int shape = choose_direct(a, ncu);
-    // (its shares are those of 128 columns and 32 rows each: where they do not fit the fixed scratch, the kernels with larger tiles)
-    if (noalloc && (a->next_lora_down ? lora_share_bytes(a, a->N / 128) : 0) + (a->out_vk ? vk_share_bytes(a, a->M_pad / 32) : 0) > NOALLOC_SCRATCH_BYTES) shape = 0;
+    // Its shares are those of 128 columns and 32 rows each.  Where only the shares of the INT4 kernel's larger tiles fit the fixed
+    // scratch, both entry points take that one: they give the same bits.  (NVFP4: the shares of both kernels are as many.)
+    if (shape && !a->fp4) {
+        auto shares = [&](int64_t column_blocks, int64_t row_blocks) {
+            return (a->next_lora_down ? lora_share_bytes(a, column_blocks) : 0) + (a->out_vk ? vk_share_bytes(a, row_blocks) : 0);
+        };
+        if (shares(a->N / 128, a->M_pad / 32) > NOALLOC_SCRATCH_BYTES && shares((a->N + g6::BN - 1) / g6::BN, a->M_pad / g6::BM) <= NOALLOC_SCRATCH_BYTES) shape = 0;
+    }
     if (shape) return gemm_direct(a, shape, (hipStream_t)stream, dev, noalloc);
     return a->fp4 ? gemm_fp4(a, (hipStream_t)stream, dev, ncu, noalloc) : gemm_int4(a, (hipStream_t)stream, dev, ncu, noalloc);
 }

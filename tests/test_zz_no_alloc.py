@@ -75,6 +75,32 @@ def test_noalloc_next_layer_sums_two_calls_in_a_row(dev, monkeypatch):
         assert torch.equal(results[(name, True)], results[(name, False)])
 
 
+def test_noalloc_same_bits_where_only_the_larger_tiles_fit(dev, monkeypatch):
+    """96 shares of 128 columns (100 MB, the few-rows kernel) do not fit the fixed array, 48 of 256 columns (50 MB) do: both entry
+    points take the kernel with the larger tiles, whose shares are added in another order."""
+    from nunchaku_amd import packing
+    from nunchaku_amd.ops import gemm as gemm_mod
+
+    M, K, N, R, R2 = 256, 128, 12288, 16, 1024
+    announce(f"noalloc, shares of rank {R2}")
+    m, nxt = make_module(synth.make_layer(N, K, R, seed=21), dev), make_module(synth.make_layer(128, N, R2, seed=22), dev)
+    t, n = m.native_tensors(), nxt.native_tensors()
+    act, asc, la = m.quantize(synth.make_activations(M, K, seed=23).to(dev))
+    got = []
+    for no_alloc in (False, True):
+        monkeypatch.setattr(gemm_mod, "NO_ALLOC", no_alloc)
+        qout = torch.empty(M, packing.act_nbytes_per_row(N, False), dtype=torch.uint8, device=dev)
+        osc = torch.empty(N // 64, M, dtype=torch.bfloat16, device=dev)
+        down = torch.full((M, R2), float("nan"), dtype=torch.float32, device=dev)
+        gemm_mod.svdq_gemm_w4a4(act=act, wgt=t["qweight"], qout=qout, oscales=osc, ascales=asc, wscales=t["wscales"], lora_act_in=la, lora_up=t["proj_up"],
+                                lora_down=n["proj_down"], lora_act_out=down, smooth_factor=n["smooth_factor"], bias=t["bias"])
+        torch.cuda.synchronize()
+        got.append((qout, osc, down))
+    assert not torch.isnan(got[0][2]).any()
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
 def test_noalloc_refuses_what_does_not_fit(dev, monkeypatch):
     from nunchaku_amd.ops import gemm as gemm_mod
 
