@@ -357,18 +357,18 @@ double choose_row_blocks(int rows, int nblocks, int kgroups, int ncu, int *full_
 
 // How the tiles of an INT4 launch are laid out: split along K (kparts > 1) or in row blocks of two heights; returns the time by
 // the models.
-double choose_tiles_int4(const svdq_gemm_args *a, int ncu, int *full_blocks, int *half_blocks, int *kparts) {
+double choose_tiles_int4(const svdq_gemm_args *a, int ncu, svdq_gemm_plan *plan) {
     const int nblocks = (int)((a->N + g6::BN - 1) / g6::BN), kgroups = (int)(a->K / 64);
     double t_split;
-    *kparts = choose_kparts((int)(a->M_pad / g6::BM) * nblocks, kgroups, ncu, &t_split);
+    plan->kparts = choose_kparts((int)(a->M_pad / g6::BM) * nblocks, kgroups, ncu, &t_split);
     t_split = 0.96 * t_split + 2.8;  // (144 tiles, one per compute unit: 15.6 us at K = 1024, 33 at K = 3072, 105 at K = 12288)
-    const double t_rows = choose_row_blocks(rows_needed(a), nblocks, kgroups, ncu, full_blocks, half_blocks);
-    if (*kparts > 1 && t_split < t_rows) {
-        *full_blocks = (int)(a->M_pad / g6::BM);
-        *half_blocks = 0;
+    const double t_rows = choose_row_blocks(rows_needed(a), nblocks, kgroups, ncu, &plan->full_blocks, &plan->half_blocks);
+    if (plan->kparts > 1 && t_split < t_rows) {
+        plan->full_blocks = (int)(a->M_pad / g6::BM);
+        plan->half_blocks = 0;
         return t_split;
     }
-    *kparts = 1;
+    plan->kparts = 1;
     return t_rows;
 }
 
@@ -420,7 +420,27 @@ void fill_params(const svdq_gemm_args *a, GemmParams &p) {
 }
 
 // ---- INT4: fp6 matrix instruction on the bare codes (gemm6_kernel.h) --------------------------------
-int gemm_int4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool noalloc) {
+void plan_int4(const svdq_gemm_args *a, int ncu, svdq_gemm_plan *plan) {
+    const int kgroups = (int)(a->K / 64), all = (int)(a->M_pad / g6::BM);
+    plan->full_blocks = all;
+    plan->half_blocks = 0;
+    plan->kparts = 1;
+    if (a->k_split > 0) {
+        plan->kparts = (int)(a->k_split < kgroups ? a->k_split : kgroups);
+        return;
+    }
+    choose_tiles_int4(a, ncu, plan);
+    if (a->out_vk && vk_share_bytes(a, plan->full_blocks + plan->half_blocks) > NOALLOC_SCRATCH_BYTES && vk_share_bytes(a, all) <= NOALLOC_SCRATCH_BYTES) {
+        // (more row blocks, more shares: not where only 128-row blocks' fit the fixed scratch, and not in the other entry
+        // point either, which gives the same bits)
+        plan->full_blocks = all;
+        plan->half_blocks = 0;
+    }
+}
+
+constexpr int FULL_BAND = 10, HALF_BAND = 20;  // row blocks per band at most, see g6::tile_of
+
+int gemm_int4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t st, int dev, bool noalloc) {
     g6::Params p;
     p.act = (const uint8_t *)a->act;
     p.ascales = (const uint16_t *)a->ascales;
@@ -457,30 +477,14 @@ int gemm_int4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool no
     p.silu = a->fuse_silu != 0;
     p.gelu = a->qout != nullptr;  // the GELU is composed exactly when the next layer's input is produced (launch_impl.cuh:282-309)
 
-    // One workgroup per 128 x 256 output tile (or per part of one split along K), two resident per compute unit.
-    const int nblocks = (p.N + g6::BN - 1) / g6::BN, kgroups = p.K / 64;
-    p.full_blocks = p.M_pad / g6::BM;
-    p.half_blocks = 0;
-    p.kparts = 1;
-    if (a->k_split > 0) {
-        p.kparts = (int)(a->k_split < kgroups ? a->k_split : kgroups);
-    } else {
-        choose_tiles_int4(a, ncu, &p.full_blocks, &p.half_blocks, &p.kparts);
-        if (a->out_vk && vk_share_bytes(a, p.full_blocks + p.half_blocks) > NOALLOC_SCRATCH_BYTES && vk_share_bytes(a, a->M_pad / g6::BM) <= NOALLOC_SCRATCH_BYTES) {
-            // (more row blocks, more shares: not where only 128-row blocks' fit the fixed scratch, and not in the other entry
-            // point either, which gives the same bits)
-            p.full_blocks = (int)(a->M_pad / g6::BM);
-            p.half_blocks = 0;
-        }
-    }
+    // One workgroup per output tile (or per part of one split along K), two resident per compute unit.
+    const int nblocks = (p.N + g6::BN - 1) / g6::BN;
+    p.full_blocks = plan.full_blocks;
+    p.half_blocks = plan.half_blocks;
+    p.kparts = plan.kparts;
     const int kparts = p.kparts, ntiles = (p.full_blocks + p.half_blocks) * nblocks;
-    // bands of about ten 128-row blocks, all of the same height where the count allows it
-    auto band_height = [](int blocks, int most) {
-        const int bands = (blocks + most - 1) / most;
-        return bands > 0 ? (blocks + bands - 1) / bands : 1;
-    };
-    p.band = band_height(p.full_blocks, 10);
-    p.half_band = band_height(p.half_blocks, 20);
+    p.band = g6::band_height(p.full_blocks, FULL_BAND);
+    p.half_band = g6::band_height(p.half_blocks, HALF_BAND);
     const bool next = needs_next_epilogue(a);
     const size_t cnt_bytes = (size_t)ntiles * 4;
     const size_t part_bytes = kparts > 1 ? (size_t)ntiles * kparts * g6::BM * g6::BN * 4 : 0;
@@ -511,11 +515,8 @@ int whole_tiles_fp4(long long ntiles, int ncu) {
     return ntiles >= ncu && divisor * 100 >= ncu * 84 ? (int)divisor : 0;
 }
 
-int gemm_fp4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool noalloc) {
-    GemmParams p;
-    fill_params(a, p);
-
-    // persistent workgroups: one per compute unit, each walking over its share of the output tiles
+// Persistent workgroups: one per compute unit, each walking over its share of the output tiles.
+void plan_fp4(const svdq_gemm_args *a, int ncu, svdq_gemm_plan *plan) {
     const int ntiles = (int)(a->M_pad / BM) * (int)((a->N + BN - 1) / BN);
     int nwg = ntiles < ncu ? ntiles : ncu;
     int divisor = nwg;  // the largest workgroup count that divides the tile count
@@ -553,10 +554,18 @@ int gemm_fp4(const svdq_gemm_args *a, hipStream_t st, int dev, int ncu, bool noa
         if (w > ncu) w = ncu;
         if (w > nwg) nwg = (int)w;
     }
+    plan->workgroups = nwg;
+    plan->shared_tiles = !(nwg <= ntiles && ntiles % nwg == 0);
+}
+
+int gemm_fp4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t st, int dev, bool noalloc) {
+    GemmParams p;
+    fill_params(a, p);
+    const int ntiles = (int)(a->M_pad / BM) * (int)((a->N + BN - 1) / BN), nwg = plan.workgroups;
     // the work is split evenly in units of two k-groups; unless the tile count is a multiple of the
     // workgroup count, some tiles are then shared by two or more workgroups and need the workspace
     const bool next = needs_next_epilogue(a);
-    const bool shared_tiles = !(nwg <= ntiles && ntiles % nwg == 0);
+    const bool shared_tiles = plan.shared_tiles;
     p.whole_band = 0;
     if (!shared_tiles) {
         // bands about as high as the window of an XCD's workgroups (an eighth of them) is wide, all of the same height
@@ -630,8 +639,8 @@ int choose_direct(const svdq_gemm_args *a, int ncu) {
             t2 += 1.0 * c2;
         }
     } else {
-        int full, half, kparts;
-        t_large = choose_tiles_int4(a, ncu, &full, &half, &kparts);
+        svdq_gemm_plan tiles;
+        t_large = choose_tiles_int4(a, ncu, &tiles);
         t1 = 3.5 + c1 * (1.1 + 0.106 * kg);
         t2 = 3.3 + c2 * (1.6 + 0.158 * kg);
     }
@@ -639,11 +648,30 @@ int choose_direct(const svdq_gemm_args *a, int ncu) {
     return t2 < t_large ? 2 : 0;
 }
 
-int gemm_direct(const svdq_gemm_args *a, int shape, hipStream_t st, int dev, bool noalloc) {
+// Which kernel a call takes and how it divides the work.  A function of the arguments and the number of compute units alone:
+// the entry points with and without an allocation give the same bits.
+void make_plan(const svdq_gemm_args *a, int ncu, svdq_gemm_plan *plan) {
+    *plan = svdq_gemm_plan{};
+    int shape = choose_direct(a, ncu);
+    // Its shares are those of 128 columns and 32 rows each.  Where only the shares of the INT4 kernel's larger tiles fit the fixed
+    // scratch, that one is taken.  (NVFP4: the shares of both kernels are as many.)
+    if (shape && !a->fp4) {
+        auto shares = [&](int64_t column_blocks, int64_t row_blocks) {
+            return (a->next_lora_down ? lora_share_bytes(a, column_blocks) : 0) + (a->out_vk ? vk_share_bytes(a, row_blocks) : 0);
+        };
+        if (shares(a->N / 128, a->M_pad / 32) > NOALLOC_SCRATCH_BYTES && shares((a->N + g6::BN - 1) / g6::BN, a->M_pad / g6::BM) <= NOALLOC_SCRATCH_BYTES) shape = 0;
+    }
+    plan->few_rows = shape;
+    if (shape) plan->row_blocks = (rows_needed(a) + 32 * shape - 1) / (32 * shape);  // (shape s: tiles of 32 s rows)
+    else if (a->fp4) plan_fp4(a, ncu, plan);
+    else plan_int4(a, ncu, plan);
+}
+
+int gemm_direct(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t st, int dev, bool noalloc) {
     GemmParams p;
     fill_params(a, p);
-    const int rows = rows_needed(a);
-    p.row_blocks = (rows + 32 * shape - 1) / (32 * shape);  // (shape s: tiles of 32 s rows)
+    const int shape = plan.few_rows;
+    p.row_blocks = plan.row_blocks;
     const bool next = needs_next_epilogue(a);
     auto launch = [&]() {
         if (a->fp4) return next ? direct::launch_fp4_next(p, shape, st) : direct::launch_fp4_plain(p, shape, st);
@@ -665,7 +693,7 @@ int gemm_direct(const svdq_gemm_args *a, int shape, hipStream_t st, int dev, boo
 }  // namespace
 
 namespace {
-int gemm_entry(const svdq_gemm_args *a, void *stream, bool noalloc) {
+int check_arguments(const svdq_gemm_args *a) {
     SVDQ_REQUIRE(a, "gemm: null args");
     SVDQ_REQUIRE(a->act && a->ascales && a->wgt && a->wscales, "gemm: act/ascales/wgt/wscales must not be null");
     SVDQ_REQUIRE(!a->fp4 || a->colnorm, "gemm: NVFP4 needs colnorm");
@@ -741,21 +769,20 @@ int gemm_entry(const svdq_gemm_args *a, void *stream, bool noalloc) {
         SVDQ_REQUIRE(!a->out_q && !a->out_k && !a->out_v, "gemm: out_q / out_k / out_v need rotary_emb (the reference composes them only there)");
     }
 
+    return SVDQ_OK;
+}
+
+int gemm_entry(const svdq_gemm_args *a, void *stream, bool noalloc) {
+    const int rc = check_arguments(a);
+    if (rc != SVDQ_OK) return rc;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return fail(SVDQ_ELAUNCH, "gemm: cannot identify the current device");
     const int ncu = compute_units(dev);
     if (ncu <= 0) return fail(SVDQ_ELAUNCH, "gemm: cannot query the number of compute units");
-    int shape = choose_direct(a, ncu);
-    // Its shares are those of 128 columns and 32 rows each.  Where only the shares of the INT4 kernel's larger tiles fit the fixed
-    // scratch, both entry points take that one: they give the same bits.  (NVFP4: the shares of both kernels are as many.)
-    if (shape && !a->fp4) {
-        auto shares = [&](int64_t column_blocks, int64_t row_blocks) {
-            return (a->next_lora_down ? lora_share_bytes(a, column_blocks) : 0) + (a->out_vk ? vk_share_bytes(a, row_blocks) : 0);
-        };
-        if (shares(a->N / 128, a->M_pad / 32) > NOALLOC_SCRATCH_BYTES && shares((a->N + g6::BN - 1) / g6::BN, a->M_pad / g6::BM) <= NOALLOC_SCRATCH_BYTES) shape = 0;
-    }
-    if (shape) return gemm_direct(a, shape, (hipStream_t)stream, dev, noalloc);
-    return a->fp4 ? gemm_fp4(a, (hipStream_t)stream, dev, ncu, noalloc) : gemm_int4(a, (hipStream_t)stream, dev, ncu, noalloc);
+    svdq_gemm_plan plan;
+    make_plan(a, ncu, &plan);
+    if (plan.few_rows) return gemm_direct(a, plan, (hipStream_t)stream, dev, noalloc);
+    return a->fp4 ? gemm_fp4(a, plan, (hipStream_t)stream, dev, noalloc) : gemm_int4(a, plan, (hipStream_t)stream, dev, noalloc);
 }
 }  // namespace
 
@@ -778,6 +805,23 @@ extern "C" int svdq_gemm_w4a4_rows(const svdq_gemm_args *a, int64_t rows, int no
     svdq_gemm_args some = *a;
     some.M_out = rows;
     return gemm_entry(&some, stream, noalloc != 0);
+}
+
+extern "C" int svdq_gemm_plan_of(const svdq_gemm_args *a, int64_t rows, int compute_units, svdq_gemm_plan *plan) {
+    SVDQ_REQUIRE(a && plan && compute_units > 0 && rows >= 0 && !(a->out && rows), "gemm: rows go with a call without `out`");
+    svdq_gemm_args some = *a;
+    if (!a->out) some.M_out = rows;
+    const int rc = check_arguments(&some);
+    if (rc == SVDQ_OK) make_plan(&some, compute_units, plan);
+    return rc;
+}
+
+extern "C" void svdq_gemm_int4_tile(const svdq_gemm_plan *plan, int64_t N, int block, svdq_gemm_tile *tile) {
+    const int nblocks = (int)((N + g6::BN - 1) / g6::BN);
+    const g6::TileOf t = g6::tile_of(block, (plan->full_blocks * plan->kparts + plan->half_blocks) * nblocks, nblocks, plan->full_blocks, plan->half_blocks,
+                                     g6::band_height(plan->full_blocks, FULL_BAND), g6::band_height(plan->half_blocks, HALF_BAND), plan->kparts);
+    const int rows = t.whole ? g6::BM : g6::BM / 2, before = t.whole ? 0 : plan->full_blocks;
+    *tile = svdq_gemm_tile{before * g6::BM + t.row_block * rows, rows, t.column_block, t.part, before + t.row_block, t.tile};
 }
 
 extern "C" int svdq_release_workspaces(void) {

@@ -747,29 +747,11 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
     }
 }
 
-// Which tile: row blocks [0, full_blocks) are 128 rows high, the half_blocks behind them 64 (or, with full_blocks = all, tiles
-// split along K).  Workgroups go to the XCDs round robin (blockIdx % 8): each XCD takes one contiguous run of the
-// numbers of the 128-row tiles (or their parts), then one of the 64-row tiles'.  The tiles are numbered in bands of about ten
-// 128-row blocks, down the band first: the 64 workgroups resident on an XCD at one time then cover about 10 row blocks
-// x 6 column blocks, whose operands (6 KB per row block and k-group, 14 KB per column block) they share in that
-// XCD's L2.  Measured at 36 x 48 tiles, bytes fetched from beyond the L2 per launch: bands of 6 / 9 / 12 /
-// 16 / 18 / 36 row blocks 317 / 296 / 308 / 355 / 396 / 604 MB (the time does not change: 169-171 us).
 template <bool NEXT>
 __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
-    const int nblocks = (p.N + BN - 1) / BN, total = (int)gridDim.x, full = p.full_blocks * nblocks * p.kparts;
-    const int xcd = (int)blockIdx.x % 8, j = (int)blockIdx.x / 8;
-    const int first = xcd * (full / 8) + (xcd < full % 8 ? xcd : full % 8);  // of this XCD's 128-row tiles
-    const int count = full / 8 + (xcd < full % 8 ? 1 : 0);
-    const bool whole = j < count;
-    // (the 64-row tiles of the XCDs before this one: their workgroups less their 128-row tiles)
-    const int v = whole ? first + j : xcd * (total / 8) + (xcd < total % 8 ? xcd : total % 8) - first + (j - count);
-    const int tile = whole ? v / p.kparts : v, part = whole ? v - tile * p.kparts : 0;
-    const int blocks = whole ? p.full_blocks : p.half_blocks, BAND = whole ? p.band : p.half_band;
-    const int band = tile / (BAND * nblocks), in_band = tile - band * (BAND * nblocks);
-    const int band_rows = blocks - band * BAND < BAND ? blocks - band * BAND : BAND;
-    const int mb = band * BAND + in_band % band_rows, nb = in_band / band_rows;
-    if (whole) output_tile<NEXT, 2>(p, mb * BM, nb, tile, part, mb);
-    else output_tile<NEXT, 1>(p, p.full_blocks * BM + mb * (BM / 2), nb, 0, 0, p.full_blocks + mb);
+    const TileOf t = tile_of((int)blockIdx.x, (int)gridDim.x, (p.N + BN - 1) / BN, p.full_blocks, p.half_blocks, p.band, p.half_band, p.kparts);
+    if (t.whole) output_tile<NEXT, 2>(p, t.row_block * BM, t.column_block, t.tile, t.part, t.row_block);
+    else output_tile<NEXT, 1>(p, p.full_blocks * BM + t.row_block * (BM / 2), t.column_block, 0, 0, p.full_blocks + t.row_block);
 }
 
 template <bool NEXT>

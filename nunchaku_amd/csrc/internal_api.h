@@ -12,6 +12,31 @@ extern "C" {
 // first GEMM: M = 1157 of 1280 padded rows.
 int svdq_gemm_w4a4_rows(const svdq_gemm_args *args, int64_t rows, int noalloc, void *stream);
 
+// Which kernel a GEMM call takes and how it divides the work (zero where a field does not apply).
+typedef struct svdq_gemm_plan {
+    int32_t few_rows;      // 0: a kernel with large tiles; 1, 2: the few-rows kernel in tiles of 32, 64 rows x 128 columns
+    int32_t row_blocks;    // few rows: tiles along M
+    int32_t full_blocks;   // INT4, large tiles: row blocks of 128 rows,
+    int32_t half_blocks;   // of 64 rows behind them,
+    int32_t kparts;        // and parts along K of every tile
+    int32_t workgroups;    // NVFP4, large tiles: persistent workgroups;
+    int32_t shared_tiles;  // some tiles are shared by two or more of them
+} svdq_gemm_plan;
+
+// What svdq_gemm_w4a4 (`rows` > 0: svdq_gemm_w4a4_rows) would do with these arguments on a GPU of so many compute units.  Checks the
+// arguments as the call does, launches nothing and needs no GPU.
+int svdq_gemm_plan_of(const svdq_gemm_args *args, int64_t rows, int compute_units, svdq_gemm_plan *plan);
+
+// The work of workgroup `block` of an INT4 launch with large tiles.
+typedef struct svdq_gemm_tile {
+    int32_t row, rows;     // first row, height
+    int32_t column_block;  // of 256 columns
+    int32_t part;          // along K
+    int32_t row_block;     // its number among the blocks of both heights
+    int32_t tile;          // the number that the parts of a tile meet under
+} svdq_gemm_tile;
+void svdq_gemm_int4_tile(const svdq_gemm_plan *plan, int64_t N, int block, svdq_gemm_tile *tile);
+
 #ifdef __cplusplus
 }
 #endif

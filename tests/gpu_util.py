@@ -46,6 +46,33 @@ def make_oracle(layer: synth.LogicalLayer, act_unsigned=False):
     )
 
 
+def off_alignment(vector: torch.Tensor) -> torch.Tensor:
+    """The same native vector (``packing.repack_vector``) two bytes off an 8-byte address.  The few-rows GEMM reads a bias four values
+    at a time and does not take such a call: it goes to the kernels with large tiles, divided as the library divides it."""
+    from nunchaku_amd import packing
+
+    raw = torch.empty(vector.numel() + 1, dtype=vector.dtype, device=vector.device)
+    raw[1:].copy_(vector)
+    assert raw[1:].data_ptr() % 8 == 2
+    return packing._tag(raw[1:], "vector")
+
+
+def record_plans(monkeypatch, dev) -> list:
+    """The plans (``plan_util.Plan``) of the GEMM operator's calls from here on, in order."""
+    from nunchaku_amd import _native as nv
+    from plan_util import plan_of
+
+    plans, real, ncu = [], nv.launch, torch.cuda.get_device_properties(dev).multi_processor_count
+
+    def launch(entry, args_ref, device):
+        if isinstance(args_ref._obj, nv.GemmArgs):
+            plans.append(plan_of(args_ref._obj, compute_units=ncu))
+        return real(entry, args_ref, device)
+
+    monkeypatch.setattr(nv, "launch", launch)
+    return plans
+
+
 class Guarded:
     """A tensor placed inside a larger buffer filled with a byte pattern: ``check()`` asserts that the bands before and
     behind it still hold the pattern, i.e. that no kernel wrote outside the tensor."""

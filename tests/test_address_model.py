@@ -1,9 +1,10 @@
-"""Host-side model of every global address the INT4 GEMM kernel and the quantize kernel form, checked against the sizes of
-the buffers the operators are given (CPU only; nothing here touches a GPU).
+"""Host-side model of every global address the INT4 GEMM kernel, the few-rows GEMM kernel and the quantize kernel form, checked
+against the sizes of the buffers the operators are given (CPU only; nothing here touches a GPU).
 
-The model restates the index arithmetic of ``csrc/gemm6_kernel.h`` (tile numbering, k-parts, the schedule of the
-asynchronous copies with its look-ahead, parked partial sums, output stores) and of ``csrc/quantize.hip`` (the row buffer
-whose size ends at the last valid row, code / scale / projection stores) for whole grids, over the shape distribution of
+Which tile a workgroup takes is asked of the library (``plan_util``).  The model restates the index arithmetic of
+``csrc/gemm6_kernel.h`` (k-parts, the schedule of the asynchronous copies with its look-ahead, parked partial sums, output
+stores), of ``csrc/gemm_direct_kernel.h`` (operands of both precisions) and of ``csrc/quantize.hip`` (the row buffer whose size
+ends at the last valid row, code / scale / projection stores) for whole grids, over the shape distribution of
 ``tests/test_gpu_shape_sweep.py`` and of the randomized loop that once ended in a GPU fault (M = 100, K = 3072, N = 768,
 rank 0, three k-parts among them).  It guards the arithmetic; the fault itself came from the compiler keeping a carry flag
 alive across an inline-asm statement that overwrote it (``tests/test_build_guard.py`` checks the generated code for that).
@@ -13,38 +14,19 @@ import random
 
 import pytest
 
+from plan_util import call, plan_of, tile_of
+
 FRAG = 1536
 BM, BN = 128, 256
 SLOT_BYTES = 32 * 256 * 4 * 4
 
 
-def choose_kparts(ntiles, kgroups, ncu=256):
-    """csrc/gemm.hip::choose_kparts"""
-    if ntiles > ncu:
-        return 1
-    best, best_t = 1, 0.55 * kgroups + 4.4
-    for k in (2, 3, 4, 6, 8):
-        units, g = ntiles * k, (kgroups + k - 1) // k
-        if g < 12 or units > 2 * ncu:
-            break
-        shared = units > ncu
-        t = g * (0.95 if shared else 0.55) + 4.4 + (11.5 if k == 4 else 5.3 + 2.6 * (k - 1)) * (1.5 if shared else 1.0)
-        if t < (0.90 if best == 1 else 0.95) * best_t:
-            best, best_t = k, t
-    return best
-
-
-def gemm6_grid(M_pad, N, K, k_split=0):
-    mblocks, nblocks, kgroups = M_pad // BM, (N + BN - 1) // BN, K // 64
-    ntiles = mblocks * nblocks
-    kparts = min(k_split, kgroups) if k_split > 0 else choose_kparts(ntiles, kgroups)
-    nbands = (mblocks + 9) // 10
-    band = (mblocks + nbands - 1) // nbands
-    return mblocks, nblocks, kgroups, ntiles, kparts, band
-
-
 def check_gemm6(M_pad, N, K, M_out, N_out, k_split=0):
-    mblocks, nblocks, kgroups, ntiles, kparts, BAND = gemm6_grid(M_pad, N, K, k_split)
+    """The launch in large tiles (by the library's own division for k_split 0, an operand being off its alignment)."""
+    plan = plan_of(call("plain", M_out, K, N, 0, False, k_split=k_split, aligned=False))
+    assert not plan.few_rows
+    nblocks, kgroups, kparts = (N + BN - 1) // BN, K // 64, plan.kparts
+    ntiles = (plan.full_blocks + plan.half_blocks) * nblocks
     act_bytes = M_pad * K * 3 // 4
     wgt_bytes = nblocks * BN * K * 3 // 4
     wsc_bytes = nblocks * kgroups * 2048
@@ -53,20 +35,15 @@ def check_gemm6(M_pad, N, K, M_out, N_out, k_split=0):
     total = ntiles * kparts
     seen = {}
     for bid in range(total):
-        v = (bid % 8) * (total // 8) + bid // 8 if total % 8 == 0 else bid
-        assert 0 <= v < total
-        tile, part = divmod(v, kparts)
-        band = tile // (BAND * nblocks)
-        in_band = tile - band * BAND * nblocks
-        band_rows = min(mblocks - band * BAND, BAND)
-        assert band_rows > 0
-        mb, nb = band * BAND + in_band % band_rows, in_band // band_rows
-        assert 0 <= mb < mblocks and 0 <= nb < nblocks, (tile, mb, nb)
+        t = tile_of(plan, N, bid)
+        m0, nb, part, MT = t.row, t.column_block, t.part, t.rows // 64
+        assert 0 <= m0 and m0 + t.rows <= M_pad and 0 <= nb < nblocks and 0 <= part < kparts, (bid, m0, nb)
+        mb, slab0 = m0 // 128, m0 % 128 // 32
         gb = kgroups * part // kparts
         ng = kgroups * (part + 1) // kparts - gb
         assert ng >= 1
-        assert (mb, nb, part) not in seen
-        seen[(mb, nb, part)] = True
+        assert (m0, nb, part) not in seen
+        seen[(m0, nb, part)] = True
         # the copy schedule: which k-groups get their weights (W) and the rest (R) requested
         w_req, r_req = [0], [0]
         if ng > 1:
@@ -84,35 +61,81 @@ def check_gemm6(M_pad, N, K, M_out, N_out, k_split=0):
             l += 1
         assert w_req == list(range(ng)) and r_req == list(range(ng)), (ng, w_req, r_req)
         for wave in range(4):
-            for g in range(ng):
+            for g in (0, ng // 2, ng - 1):  # (addresses grow with g)
                 # three 1 KB weight chunks, 16 bytes per lane
                 src_w = (nb * kgroups + gb + g) * 8 * FRAG + wave * 3072
                 assert src_w + 2048 + 63 * 16 + 16 <= wgt_bytes
-                src_a = (mb * kgroups + gb + g) * 4 * FRAG + wave * 1024
-                assert src_a + 63 * 16 + 16 <= act_bytes
-                if wave < 2:
-                    src_x = (mb * kgroups + gb + g) * 4 * FRAG + (4 + wave) * 1024
-                    assert src_x + 63 * 16 + 16 <= act_bytes
+                act0 = (mb * kgroups + gb + g) * 4 * FRAG + slab0 * FRAG
+                ws0 = (nb * kgroups + gb + g) * 2048
+                as0 = ((gb + g) * M_pad + m0) * 2
+                if MT == 2:
+                    assert act0 + wave * 1024 + 1024 <= act_bytes
+                    if wave < 2:
+                        assert act0 + (4 + wave) * 1024 + 1024 <= act_bytes
+                    else:
+                        assert ws0 + (wave - 2) * 1024 + 1024 <= wsc_bytes
+                    assert as0 + 63 * 4 + 4 <= asc_bytes
+                elif wave < 3:  # two fragments are three chunks; the scales of 64 rows, eight times over
+                    assert act0 + wave * 1024 + 1024 <= act0 + 2 * FRAG and act0 + 2 * FRAG <= act_bytes
+                    assert as0 + 7 * 16 + 16 == as0 + 64 * 2 <= asc_bytes
                 else:
-                    src_x = (nb * kgroups + gb + g) * 2048 + (wave - 2) * 1024
-                    assert src_x + 63 * 16 + 16 <= wsc_bytes
-                src_q = ((gb + g) * M_pad + mb * BM) * 2
-                assert src_q + 63 * 4 + 4 <= asc_bytes
+                    assert ws0 + 1024 + 1024 <= wsc_bytes
         if kparts > 1:
-            slot = (tile * kparts + part) * SLOT_BYTES
+            slot = (t.tile * kparts + part) * SLOT_BYTES
             assert slot + ((7 * 4 + 3) * 256 + 255) * 16 + 16 <= part_bytes
-            assert tile * 4 + 4 <= ntiles * 4  # arrival counter
+            assert t.tile * 4 + 4 <= ntiles * 4  # arrival counter
         # output stores: rows below M_out, 16-byte pieces below N_out
         for wm in range(2):
             for wn in range(2):
-                for mt in range(2):
+                for mt in range(MT):
                     for rr in (0, 31):
                         for cc in (0, 120):
-                            m, n = mb * BM + wm * 64 + mt * 32 + rr, nb * BN + wn * 128 + cc
+                            m, n = m0 + wm * 32 * MT + mt * 32 + rr, nb * BN + wn * 128 + cc
                             if m < M_out and n < N_out:
                                 assert (m * N_out + n) * 2 + 16 <= M_out * N_out * 2
     assert len(seen) == total
     return kparts
+
+
+def check_direct(M, K, N, fp4, shape, rows):
+    """The operands of the few-rows kernel (csrc/gemm_direct_kernel.h) in tiles of 32 `shape` rows."""
+    M_pad, kgroups = (M + 255) // 256 * 256, K // 64
+    MT, WN, KP = (1, 1, 4) if shape == 1 else (2, 1, 4) if fp4 else (2, 2, 2)
+    NT, TILE = 4 // WN, 1024
+    row_blocks = (rows + 32 * MT - 1) // (32 * MT)
+    act_bytes, asc_bytes = (M_pad * K // 2, kgroups * M_pad * 4) if fp4 else (M_pad * K * 3 // 4, kgroups * M_pad * 2)
+    padded = (N + 255) // 256 * 256  # (INT4 weights are stored in whole blocks of 256 columns)
+    wgt_bytes, wsc_bytes = (N * K // 2, kgroups * N * 8) if fp4 else (padded * K * 3 // 4, padded // 256 * kgroups * 2048)
+    total = row_blocks * (N // 128)
+    seen = set()
+    for bid in range(total):
+        xcd, extra = bid % 8, total % 8
+        v = xcd * (total // 8) + min(xcd, extra) + bid // 8
+        nb, mb = divmod(v, row_blocks)
+        seen.add((nb, mb))
+        assert nb < N // 128 and (mb + 1) * 32 * MT <= M_pad
+        f0 = mb * MT
+        for kpart in range(KP):
+            g_load = min(kpart, kgroups - 1)
+            last = kpart + (kgroups - 1 - kpart) // KP * KP if kpart < kgroups else g_load  # the group the requests stop at
+            assert last < kgroups and last + KP >= kgroups
+            for g in {g_load, last}:
+                for mt in range(MT):
+                    if fp4:
+                        assert ((f0 + mt) * kgroups + g) * TILE + 31 * 32 + 16 + 16 <= act_bytes
+                        assert (g * M_pad + f0 * 32) * 4 + mt * 128 + 31 * 4 + 2 + 2 <= asc_bytes
+                    else:
+                        assert ((f0 + mt) // 4 * kgroups + g) * 4 * FRAG + (f0 + mt) % 4 * FRAG + 1024 + 63 * 8 + 8 <= act_bytes
+                        assert (g * M_pad + f0 * 32) * 2 + mt * 64 + 31 * 2 + 2 <= asc_bytes
+                for cw in range(WN):
+                    for nt in range(NT):
+                        if fp4:
+                            assert ((nb * 4 + cw * NT) * kgroups + g) * TILE + nt * kgroups * TILE + 31 * 32 + 16 + 16 <= wgt_bytes
+                            assert (g * N + nb * 128 + cw * NT * 32) * 8 + nt * 256 + 31 * 8 + 4 + 4 <= wsc_bytes
+                        else:
+                            assert (nb // 2 * kgroups + g) * 8 * FRAG + (nb % 2 * 4 + cw * NT + nt) * FRAG + 1024 + 63 * 8 + 8 <= wgt_bytes
+                            assert (nb // 2 * kgroups + g) * 2048 + nb % 2 * 1024 + cw * NT * 256 + nt * 256 + 31 * 8 + 4 <= wsc_bytes
+    assert len(seen) == total and rows <= row_blocks * 32 * MT
 
 
 def sweep_shapes():
@@ -139,7 +162,7 @@ def test_gemm6_addresses_stay_inside_their_buffers():
     for M, K, N, ks in shapes:
         M_pad = (M + 255) // 256 * 256
         check_gemm6(M_pad, N, K, M, N, ks)
-    # the case that faulted: six tiles, by the library's own choice split in three parts then and in four now
+    # the case that faulted: six tiles, by the library's own choice split in three parts then and, in large tiles, in four now
     assert check_gemm6(256, 768, 3072, 100, 768, 0) == 4
     assert check_gemm6(256, 768, 3072, 100, 768, 3) == 3
 
@@ -147,6 +170,28 @@ def test_gemm6_addresses_stay_inside_their_buffers():
 def test_gemm6_addresses_large_shapes():
     for M_pad, N, K in ((4608, 12288, 3072), (4608, 3072, 12288), (4608, 9216, 3072), (256, 3072, 3072)):
         check_gemm6(M_pad, N, K, M_pad, N, 0)
+
+
+@pytest.mark.parametrize("fp4", [False, True])
+def test_few_rows_addresses_stay_inside_their_buffers(fp4):
+    for M, K, N, _ in sweep_shapes()[::3] + [(1, 128, 128, 0), (4608, 3072, 3072, 0), (1157, 12288, 3072, 0)]:
+        M_pad = (M + 255) // 256 * 256
+        for shape in (1, 2):
+            for rows in {M, M_pad}:
+                check_direct(M, K, N, fp4, shape, rows)
+
+
+def test_projecting_workgroups_read_inside_proj_down():
+    """csrc/quantize.hip, project_rows: rank tile rt of step i of chunk c is the KB behind ((4 c + i) R / 16 + rt) KB; a second rank
+    tile beyond the rank repeats the first.  (Its rows are read as the quantize kernel's with 16 rows are.)"""
+    for K in (128, 1152, 12288):
+        for R in (16, 48, 80, 1024):
+            RT = R // 16
+            for RTW in (1, 2):
+                for rt0 in range(0, RT, RTW):
+                    rt1 = rt0 + 1 if rt0 + 1 < RT else rt0
+                    for rt in (rt0, rt1):
+                        assert ((K // 128 - 1) * 4 + 3) * RT * 1024 + rt * 1024 + 63 * 16 + 16 <= K * R * 2
 
 
 @pytest.mark.parametrize("glu", [False, True])

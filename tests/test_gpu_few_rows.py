@@ -6,12 +6,13 @@ import pytest
 import torch
 
 from conftest import announce
-from gpu_util import bf16_ulp, make_module
+from gpu_util import bf16_ulp, make_module, record_plans
 from oracle import synth
 
 pytestmark = pytest.mark.gpu
 
-# (epilogue, M, K, N, R); the launcher takes 32-row tiles for all but the last rows, which are large enough for 64-row tiles
+# (epilogue, M, K, N, R); the launcher takes 32-row tiles for the first two rows of this list, and 64-row tiles, on 256 compute
+# units, for the others
 CASES = [
     ("plain", 1, 128, 128, 16), ("plain", 31, 128, 256, 0), ("plain", 33, 640, 384, 48), ("plain", 64, 1152, 128, 80), ("plain", 65, 256, 640, 32),
     ("silu", 96, 384, 256, 16), ("next", 33, 128, 128, 16), ("next", 97, 640, 384, 48), ("rope", 40, 384, 384, 32), ("split", 256, 256, 768, 16),
@@ -39,6 +40,7 @@ def test_against_large_tiles(dev, kind, M, K, N, R, fp4, monkeypatch):
     if R:
         kw.update(lora_act_in=la, lora_up=t["proj_up"], lora_scales=[0.5 + 0.25 * i for i in range((R + 15) // 16)])
     new = lambda *shape, dtype=torch.bfloat16: torch.full(shape, float("nan"), dtype=dtype, device=dev)  # noqa: E731
+    plans = record_plans(monkeypatch, dev)
 
     def run(split):
         monkeypatch.setattr(gemm_mod, "K_SPLIT", split)
@@ -66,6 +68,9 @@ def test_against_large_tiles(dev, kind, M, K, N, R, fp4, monkeypatch):
         rot = packing.repack_rotemb(torch.stack((ang.sin(), ang.cos()), dim=-1).reshape(M_pad, 128).to(dev))
         nq = (1.0 + 0.2 * torch.randn(128, generator=g)).to(torch.bfloat16).to(dev)
     want, got, again = run(1), run(None), run(None)
+    assert plans[0].few_rows == 0
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+        assert plans[1].few_rows == plans[2].few_rows == (1 if M <= 256 else 2), plans
     for name in got:
         a, b = got[name].cpu(), want[name].cpu()
         assert torch.equal(a.view(torch.uint8), again[name].cpu().view(torch.uint8)), f"{name} changed between two launches"

@@ -6,9 +6,8 @@ import pytest
 import torch
 
 from conftest import announce
-from gpu_util import make_module
+from gpu_util import make_module, record_plans
 from oracle import synth
-from test_gemm6_tiles_cpu import choose_row_blocks
 
 pytestmark = pytest.mark.gpu
 
@@ -27,9 +26,7 @@ def test_same_bits_as_whole_tiles(dev, kind, M, K, N, R, monkeypatch):
 
     announce(f"row blocks {kind} M={M} K={K} N={N} R={R}")
     M_pad = (M + 255) // 256 * 256
-    needed = M if kind in ("plain", "silu", "rope") else M_pad
-    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
-        assert choose_row_blocks(needed, (N + 255) // 256)[1] > 0, "the case has no 64-row tiles"
+    plans = record_plans(monkeypatch, dev)
     g = torch.Generator().manual_seed(M + K + N)
     layer = synth.make_layer(N, K, R, seed=K + N)
     m = make_module(layer, dev)
@@ -66,6 +63,9 @@ def test_same_bits_as_whole_tiles(dev, kind, M, K, N, R, monkeypatch):
         rot = packing.repack_rotemb(torch.stack((ang.sin(), ang.cos()), dim=-1).reshape(M_pad, 128).to(dev))
         nq = (1.0 + 0.2 * torch.randn(128, generator=g)).to(torch.bfloat16).to(dev)
     want, got = run(1), run(None)
+    assert plans[0].half_blocks == 0 and plans[0].kparts == 1
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+        assert plans[1].few_rows == 0 and plans[1].half_blocks > 0, "the case has no 64-row tiles"
     for name in got:
         a, b = got[name], want[name]
         if name == "out_vk":  # 256 or 2048 products per sum, added in other pieces: 2^-24 of the largest per addition
