@@ -125,14 +125,17 @@ def test_mlp_flux_shape(dev):
     check_output(y[rows], want_y)
 
 
-def test_side_streams_give_the_same_bits(dev):
+@pytest.mark.parametrize("k_split", [None, 4])
+def test_side_streams_give_the_same_bits(dev, k_split, monkeypatch):
     """The library launches on the caller's current stream and keeps one workspace per (device, stream): the fused
-    MLP whose first GEMM is split along K (parked sums, arrival counters) and leaves low-rank shares, run in turn on
-    two side streams, gives what the default stream gave."""
+    MLP whose first GEMM leaves low-rank shares, and with k_split = 4 is split along K (parked sums, arrival counters),
+    run in turn on two side streams, gives what the default stream gave."""
     from nunchaku_amd.ops import fused_gelu_mlp
+    from nunchaku_amd.ops import gemm as gemm_mod
 
     M, K1, N1, N2, R = 256, 3072, 512, 256, 32
-    announce(f"fused_gelu_mlp on side streams M={M} K1={K1} N1={N1} N2={N2}")
+    announce(f"fused_gelu_mlp on side streams M={M} K1={K1} N1={N1} N2={N2} k_split={k_split}")
+    monkeypatch.setattr(gemm_mod, "K_SPLIT", k_split)
     fc1, fc2, x, m1, m2 = _mlp(dev, M, K1, N1, N2, R, seed=77)
     xd = x.to(dev).view(1, M, K1)
     want = fused_gelu_mlp(xd, m1, m2)

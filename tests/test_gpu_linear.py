@@ -183,13 +183,18 @@ def test_forward_refuses_a_parameter_of_the_wrong_shape(dev):
         m(x)
 
 
-def test_one_layer_from_two_threads(dev):
-    """A layer's prepared argument blocks are shared by the threads that call it: each call fills them and launches
-    under the layer's lock, so concurrent forwards with different row counts give what they give alone."""
+@pytest.mark.parametrize("k_split", [None, 4])
+def test_one_layer_from_two_threads(dev, k_split, monkeypatch):
+    """What a layer keeps between calls is shared by the threads that call it and only read; a call's argument blocks and
+    scratch are its own.  Concurrent forwards with different row counts give what they give alone, also where the tiles are
+    split along K and the calls share a workspace (k_split = 4)."""
     import threading
 
-    announce("one layer called from two threads")
-    layer = synth.make_layer(384, 3072, 32, seed=35)  # (K = 3072 with few tiles: the GEMM takes the split path and its workspace)
+    from nunchaku_amd.ops import gemm as gemm_mod
+
+    announce(f"one layer called from two threads k_split={k_split}")
+    monkeypatch.setattr(gemm_mod, "K_SPLIT", k_split)
+    layer = synth.make_layer(384, 3072, 32, seed=35)
     m = make_module(layer, dev)
     xs = {rows: synth.make_activations(rows, 3072, seed=rows).to(dev).view(1, rows, 3072) for rows in (100, 300)}
     want = {rows: m(x).clone() for rows, x in xs.items()}

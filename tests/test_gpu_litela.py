@@ -5,24 +5,31 @@ import pytest
 import torch
 
 from conftest import announce
-from gpu_util import check_output, make_module, make_oracle
+from gpu_util import check_output, make_module, make_oracle, off_alignment, record_plans
 from oracle import linear as olin
 from oracle import synth
 
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("tiles", ["few rows", "large", "large whole"])
 @pytest.mark.parametrize("B,T,K,heads,R,fp4", [(1, 256, 256, 4, 16, False), (2, 256, 384, 8, 32, False), (1, 1024, 256, 12, 32, False),
                                                (3, 512, 128, 20, 0, False), (2, 512, 256, 12, 32, True), (1, 2304, 128, 80, 16, True)])
-def test_litela_epilogue(dev, B, T, K, heads, R, fp4):
+def test_litela_epilogue(dev, B, T, K, heads, R, fp4, tiles, monkeypatch):
     """heads = 4: N = 384, one 256-column block of q + k/v and a ragged half block; 12 and 20 heads: the q third ends
     inside a 256-column block, so one workgroup holds a q half and a k/v half.  Several row blocks per batch entry add
     up in a fixed order; several batch entries must not mix.  NVFP4: the other GEMM kernel (256 x 256 tiles; 2304 rows x
-    7680 columns are 270 tiles, which its workgroups share).  heads = 80: the q third ends inside a tile."""
+    7680 columns are 270 tiles, which its workgroups share).  heads = 80: the q third ends inside a tile.
+    All of this is about the large tiles, which these shapes take with a bias that the few-rows kernel (32 or 64 x 128) does
+    not take (INT4 in row blocks of 64, as the library divides them), or with k_split = 1 (INT4 in row blocks of 128); that
+    kernel has them otherwise."""
+    from nunchaku_amd.ops import gemm as gemm_mod
     from nunchaku_amd.ops import svdq_gemm_w4a4
 
     N = heads * 96
-    announce(f"litela B={B} T={T} K={K} heads={heads} R={R} fp4={fp4}")
+    announce(f"litela B={B} T={T} K={K} heads={heads} R={R} fp4={fp4} tiles={tiles}")
+    monkeypatch.setattr(gemm_mod, "K_SPLIT", 1 if tiles == "large whole" else None)
+    plans = record_plans(monkeypatch, dev)
     layer = synth.make_layer(N, K, R, seed=heads + K, fp4=fp4)
     m = make_module(layer, dev)
     ref = make_oracle(layer)
@@ -33,13 +40,17 @@ def test_litela_epilogue(dev, B, T, K, heads, R, fp4):
     t = m.native_tensors()
     q = torch.full((B, T, N // 3), float("nan"), dtype=torch.bfloat16, device=dev)
     vk = torch.full((B, heads, 33, 32), float("nan"), dtype=torch.float32, device=dev)  # the operator clears it
-    kw = dict(act=qx, wgt=t["qweight"], ascales=asc, wscales=t["wscales"], bias=t["bias"])
+    kw = dict(act=qx, wgt=t["qweight"], ascales=asc, wscales=t["wscales"], bias=off_alignment(t["bias"]) if tiles == "large" else t["bias"])
     if fp4:
         kw.update(fp4=True, alpha=m.alpha, wcscales=t["wcscales"])
     if R:
         kw.update(lora_act_in=la, lora_up=t["proj_up"])
     svdq_gemm_w4a4(**kw, out_vk=vk, out_linearattn=q)
     torch.cuda.synchronize()
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+        plan = plans[-1]
+        assert (plan.few_rows > 0) == (tiles == "few rows") and plan.shared_tiles == (heads == 80 and tiles == "large"), plan
+        assert fp4 or tiles == "few rows" or (plan.half_blocks > 0) == (tiles == "large"), plan
     # what the plain layer gives, on the GPU: q must be its ReLU bit for bit, and vk follows from its bf16 values exactly
     plain = torch.empty(B * T, N, dtype=torch.bfloat16, device=dev)
     svdq_gemm_w4a4(**kw, out=plain)

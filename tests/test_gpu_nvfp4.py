@@ -5,17 +5,22 @@ import pytest
 import torch
 
 from conftest import announce
-from gpu_util import check_output, make_module, make_oracle
+from gpu_util import check_output, make_module, make_oracle, off_alignment, record_plans
 from oracle import linear as olin
 from oracle import quant, synth
 
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("k_split", [None, 1])  # (the few-rows kernel; large tiles)
 @pytest.mark.parametrize("M,K,N,R", [(256, 128, 256, 16), (256, 512, 384, 32), (130, 1024, 256, 32)])
-def test_nvfp4_gemm_handmade_operands(dev, M, K, N, R):
+def test_nvfp4_gemm_handmade_operands(dev, M, K, N, R, k_split, monkeypatch):
     from nunchaku_amd import packing
+    from nunchaku_amd.ops import gemm as gemm_mod
     from nunchaku_amd.ops import svdq_gemm_w4a4
+
+    monkeypatch.setattr(gemm_mod, "K_SPLIT", k_split)
+    plans = record_plans(monkeypatch, dev)
 
     announce(f"nvfp4 gemm M={M} K={K} N={N} R={R}")
     g = torch.Generator().manual_seed(M + K + N)
@@ -36,6 +41,7 @@ def test_nvfp4_gemm_handmade_operands(dev, M, K, N, R):
         lora_up=t["proj_up"], bias=t["bias"], fp4=True, alpha=m.alpha, wcscales=t["wcscales"],
     )
     torch.cuda.synchronize()
+    assert (plans[-1].few_rows > 0) == (k_split is None)
     want = olin.gemm_w4a4(
         quant.dequant_nvfp4(codes, scales), quant.dequant_nvfp4(layer.wq, layer.ws), bias=layer.bias, lora_act_in=lora_act,
         lora_up=layer.proj_up, alpha=float(torch.tensor(layer.wtscale).to(torch.bfloat16)), wcscales=layer.wcscales,
@@ -44,15 +50,19 @@ def test_nvfp4_gemm_handmade_operands(dev, M, K, N, R):
     check_output(out, want)
 
 
+@pytest.mark.parametrize("k_split", [None, 1])  # (the few-rows kernel; large tiles)
 @pytest.mark.parametrize("M,K,N", [(256, 128, 256), (130, 256, 384)])
-def test_every_activation_scale_pattern_by_rows(dev, M, K, N):
+def test_every_activation_scale_pattern_by_rows(dev, M, K, N, k_split, monkeypatch):
     """Row m carries the E4M3 pattern m % 127 in all its groups (zero, the subnormals, up to 448): code x scale must be exact
     in the kernel's fp16 operands at both ends of that range.  Compared row by row: one bf16 rounding of the result, at
     most 2^-8 of a value, and fp32 sums of K terms (2^-24 K of the row's norm at most)."""
     from nunchaku_amd import packing
+    from nunchaku_amd.ops import gemm as gemm_mod
     from nunchaku_amd.ops import svdq_gemm_w4a4
 
-    announce(f"nvfp4 gemm, a scale pattern per row, M={M} K={K} N={N}")
+    announce(f"nvfp4 gemm, a scale pattern per row, M={M} K={K} N={N} k_split={k_split}")
+    monkeypatch.setattr(gemm_mod, "K_SPLIT", k_split)
+    plans = record_plans(monkeypatch, dev)
     g = torch.Generator().manual_seed(K + N)
     layer = synth.make_layer(N, K, 0, seed=K + N, fp4=True, bias=False)
     M_pad = (M + 255) // 256 * 256
@@ -63,6 +73,7 @@ def test_every_activation_scale_pattern_by_rows(dev, M, K, N):
     svdq_gemm_w4a4(act=packing.logical_to_act(codes, fp4=True).to(dev), wgt=t["qweight"], out=out,
                    ascales=packing.logical_to_scales(scales, fp4=True).to(dev), wscales=t["wscales"], fp4=True, alpha=1.0, wcscales=t["wcscales"])
     torch.cuda.synchronize()
+    assert (plans[-1].few_rows > 0) == (k_split is None)
     want = olin.gemm_w4a4(quant.dequant_nvfp4(codes, scales), quant.dequant_nvfp4(layer.wq, layer.ws), alpha=1.0)[:M]
     err = (out.float().cpu() - want).norm(dim=1)
     assert (err <= (2.0**-8 + K * 2.0**-24) * want.norm(dim=1)).all(), (err / want.norm(dim=1)).max().item()
@@ -100,16 +111,18 @@ def test_nvfp4_zero_per_channel_scale_is_refused(dev):
         m(synth.make_activations(M, K, seed=32).to(dev).view(1, M, K))
 
 
-@pytest.mark.parametrize("M,K1,N1,R", [(256, 256, 512, 16), (2304, 256, 7680, 32), (3072, 256, 10752, 32)])
-def test_nvfp4_fused_mlp_epilogue(dev, M, K1, N1, R):
-    """NVFP4 GEMM producing the next layer's NVFP4 input (no shift, signed patterns).  The second shape has 270 tiles,
-    which the persistent workgroups share, and 60 column chunks whose shares of the low-rank projection are added in
-    order afterwards: the projection must be fully written (it starts as NaN) and the same from launch to launch.  The
-    third has 504 tiles: 252 workgroups of two whole tiles each, taken in the windowed order."""
+@pytest.mark.parametrize("M,K1,N1,R,aligned", [(256, 256, 512, 16, True), (2304, 256, 7680, 32, True), (2304, 256, 7680, 32, False), (3072, 256, 10752, 32, False)])
+def test_nvfp4_fused_mlp_epilogue(dev, M, K1, N1, R, aligned, monkeypatch):
+    """NVFP4 GEMM producing the next layer's NVFP4 input (no shift, signed patterns), in the few-rows kernel and, with a bias it
+    does not take, in large tiles.  The second shape then has 270 tiles, which the persistent workgroups share, and in either kernel
+    60 column chunks whose shares of the low-rank projection are added in order afterwards: the projection must be fully
+    written (it starts as NaN) and the same from launch to launch.  The third has 504 tiles: 252 workgroups of two whole
+    tiles each, taken in the windowed order."""
     from nunchaku_amd import packing
     from nunchaku_amd.ops import svdq_gemm_w4a4
 
-    announce(f"nvfp4 next-layer epilogue M={M} K1={K1} N1={N1} R={R}")
+    announce(f"nvfp4 next-layer epilogue M={M} K1={K1} N1={N1} R={R} aligned={aligned}")
+    plans = record_plans(monkeypatch, dev)
     fc1 = synth.make_layer(N1, K1, R, seed=41, fp4=True)
     fc2 = synth.make_layer(256, N1, R, seed=42, fp4=True)
     x = synth.make_activations(M, K1, seed=41)
@@ -120,12 +133,16 @@ def test_nvfp4_fused_mlp_epilogue(dev, M, K1, N1, R):
     qout = torch.empty(M, N1 // 2, dtype=torch.uint8, device=dev)
     osc = torch.empty(N1 // 16, M, dtype=torch.float8_e4m3fn, device=dev)
     la2 = torch.full((M, R), float("nan"), dtype=torch.float32, device=dev)
+    bias = t1["bias"] if aligned else off_alignment(t1["bias"])
 
     def run():
         svdq_gemm_w4a4(act=qx, wgt=t1["qweight"], out=out, qout=qout, ascales=asc, wscales=t1["wscales"], oscales=osc,
-                       lora_act_in=la, lora_up=t1["proj_up"], lora_down=t2["proj_down"], lora_act_out=la2, bias=t1["bias"],
+                       lora_act_in=la, lora_up=t1["proj_up"], lora_down=t2["proj_down"], lora_act_out=la2, bias=bias,
                        smooth_factor=t2["smooth_factor"], fp4=True, alpha=m1.alpha, wcscales=t1["wcscales"])
         torch.cuda.synchronize()
+        if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+            plan = plans[-1]
+            assert (plan.few_rows > 0) == aligned and (aligned or (plan.workgroups, plan.shared_tiles) == ((256, 1) if M == 2304 else (252, 0))), plan
 
     run()
     first, first_out, first_codes = la2.clone(), out.clone(), qout.clone()

@@ -1,5 +1,5 @@
 """fused_qkv_norm_rottary on the GPU (RMS norm per 128-wide head of q and k, then the rotary embedding,
-fused into the GEMM epilogue) against the oracle: a small case with ragged tokens and shared tiles,
+fused into the GEMM epilogue) against the oracle: small cases with ragged tokens,
 the NVFP4 variant, the FLUX QKV shape, and properties that hold at any size."""
 
 import pytest

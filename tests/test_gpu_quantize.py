@@ -215,15 +215,16 @@ def test_high_rank_many_rows(dev, M, K, R, fp4, smooth):
     _check_row_sample(dev, M, K, R, fp4, smooth)
 
 
-@pytest.mark.parametrize("M,K,R,fp4", [(4608, 256, 32, False), (9000, 384, 32, False), (4500, 6272, 16, False), (2300, 256, 128, False),
-                                       (2300, 384, 64, False), (9000, 256, 128, False), (2300, 256, 256, False), (1000, 256, 144, False),
+@pytest.mark.parametrize("M,K,R,fp4", [(2300, 384, 32, False), (4000, 128, 16, True), (4608, 256, 32, False), (9000, 384, 32, False), (4500, 6272, 16, False),
+                                       (2300, 256, 128, False), (2300, 384, 64, False), (9000, 256, 128, False), (2300, 256, 256, False), (1000, 256, 144, False),
                                        (4608, 256, 32, True), (2300, 256, 128, True), (2300, 384, 64, True), (9000, 256, 32, True)])
 def test_workgroup_shapes_by_rows_and_rank(dev, M, K, R, fp4):
     """The launcher picks the workgroup's shape (waves, rows, requests ahead, rows or chunks split among the waves) by
     precision, rank, row count and row length; one case per branch of that choice beyond those the other tests take:
-    32 rows on eight waves (M = 4608; long rows; ranks 64 and 128 from 8 rows per compute unit on; the windows of rank
-    256), 16 rows on four waves with two chunks ahead (many short rows; NVFP4 at 4608 rows and at rank 128; few rows at
-    ranks above 128), the rows-split form from 32 rows per compute unit on at rank 128."""
+    16 rows on eight waves with two chunks ahead (from 8 to 16 rows per compute unit at ranks up to 32), 32 rows on eight
+    waves (M = 4608; long rows; ranks 64 and 128 from 8 rows per compute unit on; the windows of rank 256), 16 rows on four
+    waves with two chunks ahead (many short rows; NVFP4 at 4608 rows and at rank 128), the rows-split form from 32 rows
+    per compute unit on at rank 128; 1000 rows of rank 144 in quantizing and projecting workgroups."""
     announce(f"quantize workgroup shapes M={M} K={K} R={R} fp4={fp4}")
     _check_row_sample(dev, M, K, R, fp4, True)
 

@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from conftest import announce
-from gpu_util import Guarded, check_output, make_module, make_oracle
+from gpu_util import Guarded, check_output, make_module, make_oracle, off_alignment, record_plans
 from oracle import layouts as L
 from oracle import synth
 
@@ -30,8 +30,8 @@ def _cases():
         opts = dict(bias=rng.random() < 0.7, scales=rng.random() < 0.4, alpha=rng.choice([1.0, 1.0, 0.5, 1.7]) if not fp4 else None,
                     lora_scales=rng.random() < 0.4, k_split=rng.choice([None, None, 1, 2, 3]) if not fp4 else rng.choice([None, 1]))
         cases.append((i, M, K, N, R, fp4, opts))
-    # long K with few tiles: the shapes where the library splits tiles along K by its own choice (INT4: in 2 to 8 parts;
-    # NVFP4: parties of equal size)
+    # long K with few tiles: the few-rows kernel's, and with a bias it does not take the shapes where the library splits tiles
+    # along K by its own choice (INT4: in 2 to 8 parts; NVFP4: parties of equal size)
     rng = random.Random(77)
     for i in range(100, 112):
         fp4 = i % 4 == 3
@@ -42,6 +42,7 @@ def _cases():
         opts = dict(bias=rng.random() < 0.7, scales=rng.random() < 0.4, alpha=rng.choice([1.0, 0.5]) if not fp4 else None,
                     lora_scales=rng.random() < 0.4, k_split=None)
         cases.append((i, M, K, N, R, fp4, opts))
+        cases.append((i + 20, M, K, N, R, fp4, dict(opts, bias=True, large_tiles=True)))
     # ranks above 128 (a stock rank-32 branch with a rank-128 user LoRA appended is 160): the quantize operator
     # projects in windows of 128 ranks, the GEMM's up projection walks all of them
     rng = random.Random(99)
@@ -99,12 +100,16 @@ def test_layer_sweep(dev, i, M, K, N, R, fp4, opts, monkeypatch):
         # an INT4 module has no such parameter: the operator takes the reference's packed vector
         packed = L.pack_vector(layer.wcscales.view(torch.int16).numpy().view(np.uint16))
         wcs = torch.from_numpy(packed.view(np.int16).copy()).view(torch.bfloat16).to(dev)
-    kw = dict(act=qx, wgt=t["qweight"], out=out, ascales=asc, wscales=t["wscales"], bias=t["bias"], fp4=fp4, alpha=alpha,
-              wcscales=wcs, lora_scales=lora_scales)
+    large_tiles = opts.get("large_tiles", False)
+    kw = dict(act=qx, wgt=t["qweight"], out=out, ascales=asc, wscales=t["wscales"], bias=off_alignment(t["bias"]) if large_tiles else t["bias"], fp4=fp4,
+              alpha=alpha, wcscales=wcs, lora_scales=lora_scales)
     if R:
         kw.update(lora_act_in=la, lora_up=t["proj_up"])
+    plans = record_plans(monkeypatch, dev)
     svdq_gemm_w4a4(**kw)
     torch.cuda.synchronize()
+    if large_tiles:
+        assert plans[-1].few_rows == 0
     for name, gd in (("quantized activations", g_qx), ("activation scales", g_asc), ("lora_act", g_la), ("out", g_out)):
         gd.check(name)
     assert not torch.isnan(out.float()).any()

@@ -13,7 +13,7 @@ import pytest
 import torch
 
 from conftest import announce
-from gpu_util import check_output, make_module
+from gpu_util import check_output, make_module, off_alignment, record_plans
 from oracle import linear as olin
 from oracle import quant, synth
 
@@ -29,12 +29,14 @@ def _inputs(M_pad, K, R, seed):
 
 
 @pytest.mark.parametrize(
-    "M,K,N,R,k_split",
-    [(256, 3072, 3072, 32, None), (512, 12288, 512, 32, None), (256, 1024, 512, 16, 4), (512, 12288, 256, 32, 24), (300, 640, 768, 32, 10), (256, 256, 384, 16, 3), (2304, 256, 1280, 32, 2)],
+    "M,K,N,R,k_split,parts",
+    [(1536, 6144, 1536, 32, None, 3), (256, 3072, 3072, 32, None, 4), (512, 12288, 512, 32, None, 4), (256, 1024, 512, 16, 4, 4), (512, 12288, 256, 32, 24, 24),
+     (300, 640, 768, 32, 10, 10), (256, 256, 384, 16, 3, 3), (2304, 256, 1280, 32, 2, 2)],
 )
-def test_split_tiles_match_whole_tiles(dev, M, K, N, R, k_split, monkeypatch):
-    """k_split None: the library's own choice for a shape with few tiles (M = 256, K = N = 3072: 24 tiles,
-    4 parts each; M = 512, K = 12288, N = 512: 8 tiles, 8 parts each); 10 parts of K = 640: one k-group each; N = 384 and 1280: a ragged last column block."""
+def test_split_tiles_match_whole_tiles(dev, M, K, N, R, k_split, parts, monkeypatch):
+    """k_split None: the library's own choice (M = 1536, K = 6144, N = 1536: 72 tiles, 3 parts each), and for shapes with so few
+    tiles that the few-rows kernel has them unless an operand's alignment keeps it away (M = 256, K = N = 3072: 24 tiles,
+    4 parts each; M = 512, K = 12288, N = 512: 8 tiles, 4 parts each); 10 parts of K = 640: one k-group each; N = 384 and 1280: a ragged last column block."""
     from nunchaku_amd import packing
     from nunchaku_amd.ops import gemm as gemm_mod
 
@@ -45,14 +47,18 @@ def test_split_tiles_match_whole_tiles(dev, M, K, N, R, k_split, monkeypatch):
     t = m.native_tensors()
     ins = [_inputs(M_pad, K, R, seed) for seed in (1, 2)]
     dev_ins = [(packing.logical_to_act(c).to(dev), s.to(dev), la.to(dev)) for c, s, la in ins]
+    plans = record_plans(monkeypatch, dev)
+    bias = off_alignment(t["bias"]) if k_split is None and M < 1536 else t["bias"]
 
     def run(i, split):
         monkeypatch.setattr(gemm_mod, "K_SPLIT", split)
         out = torch.full((M_out, N), float("nan"), dtype=torch.bfloat16, device=dev)
         act, sc, la = dev_ins[i]
         gemm_mod.svdq_gemm_w4a4(act=act, wgt=t["qweight"], out=out, ascales=sc, wscales=t["wscales"], lora_act_in=la,
-                                lora_up=t["proj_up"], bias=t["bias"])
+                                lora_up=t["proj_up"], bias=bias)
         torch.cuda.synchronize()
+        if k_split is not None or torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+            assert plans[-1].few_rows == 0 and plans[-1].kparts == (1 if split == 1 else parts), plans[-1]
         return out
 
     whole = [run(0, 1), run(1, 1)]
@@ -80,20 +86,22 @@ def test_split_tiles_match_whole_tiles(dev, M, K, N, R, k_split, monkeypatch):
     check_output(run(1, k_split)[rows.to(dev)], want)
 
 
-def test_nvfp4_shared_tiles_match_whole_tiles(dev, monkeypatch):
+@pytest.mark.parametrize("M,K,N,aligned", [(4608, 3072, 4608, True), (2304, 256, 7680, False), (1024, 3072, 768, False)])
+def test_nvfp4_shared_tiles_match_whole_tiles(dev, M, K, N, aligned, monkeypatch):
     """The NVFP4 GEMM keeps its even work split over persistent workgroups: tiles shared by two workgroups
-    (more tiles than compute units, not a multiple) against whole-tile mode (k_split = 1)."""
-    from nunchaku_amd import packing
+    (more tiles than compute units, not a multiple) against whole-tile mode (k_split = 1).  Small K, and few tiles (12, in
+    two parties each): shapes that the few-rows kernel has unless an operand's alignment keeps it away."""
     from nunchaku_amd.ops import gemm as gemm_mod
 
-    M, K, N, R = 2304, 256, 7680, 32
+    R = 32
     ncu = torch.cuda.get_device_properties(dev).multi_processor_count
     ntiles = (M // 256) * (N // 256)
-    assert ntiles > ncu and ntiles % ncu != 0, "the shape must make the even split cut tiles"
     announce(f"nvfp4 shared tiles M={M} K={K} N={N}: {ntiles} tiles on {ncu} compute units")
     layer = synth.make_layer(N, K, R, seed=K + N, fp4=True)
     m = make_module(layer, dev)
     t = m.native_tensors()
+    bias = t["bias"] if aligned else off_alignment(t["bias"])
+    plans = record_plans(monkeypatch, dev)
     acts = []
     for seed in (1, 2):
         x = synth.make_activations(M, K, seed=seed)
@@ -104,8 +112,10 @@ def test_nvfp4_shared_tiles_match_whole_tiles(dev, monkeypatch):
         out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev)
         qx, asc, la = acts[i]
         gemm_mod.svdq_gemm_w4a4(act=qx, wgt=t["qweight"], out=out, ascales=asc, wscales=t["wscales"], lora_act_in=la,
-                                lora_up=t["proj_up"], bias=t["bias"], fp4=True, alpha=m.alpha, wcscales=t["wcscales"])
+                                lora_up=t["proj_up"], bias=bias, fp4=True, alpha=m.alpha, wcscales=t["wcscales"])
         torch.cuda.synchronize()
+        if ncu == 256:
+            assert plans[-1].few_rows == 0 and plans[-1].shared_tiles == (split != 1), plans[-1]
         return out
 
     whole = [run(0, 1), run(1, 1)]

@@ -110,15 +110,16 @@ def test_noalloc_refuses_what_does_not_fit(dev, monkeypatch):
         _run(dev, gemm_mod, m, **c, seed=3, no_alloc=True, k_split=16, monkeypatch=monkeypatch)
 
 
-def test_noalloc_forward_in_a_graph(dev, monkeypatch):
-    """What the entry point is for: the layer's forward (quantize, then a GEMM split along K whose parked sums and
-    arrival counters live in the fixed array) captured into a graph and replayed, with eager work of the same layer
+@pytest.mark.parametrize("k_split", [None, 4])
+def test_noalloc_forward_in_a_graph(dev, k_split, monkeypatch):
+    """What the entry point is for: the layer's forward (quantize, then a GEMM without a workspace, or with k_split = 4 one whose
+    parked sums and arrival counters live in the fixed array) captured into a graph and replayed, with eager work of the same layer
     between the replays; every replay gives the eager result."""
     from nunchaku_amd.ops import gemm as gemm_mod
 
-    announce("forward through svdq_gemm_w4a4_noalloc captured into a graph")
+    announce(f"forward through svdq_gemm_w4a4_noalloc captured into a graph k_split={k_split}")
     monkeypatch.setattr(gemm_mod, "NO_ALLOC", True)
-    monkeypatch.setattr(gemm_mod, "K_SPLIT", None)
+    monkeypatch.setattr(gemm_mod, "K_SPLIT", k_split)
     M, K, N, R = 256, 3072, 512, 32
     m = make_module(synth.make_layer(N, K, R, seed=9), dev)
     xs = [synth.make_activations(M, K, seed=100 + i).to(dev).view(1, M, K) for i in range(3)]
