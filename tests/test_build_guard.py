@@ -3,7 +3,9 @@ cross-compiles gfx950 without a GPU).
 
 * Registers.  ``g6::gemm6_kernel`` holds 128 accumulators per lane and runs two workgroups per compute unit: it must
   fit 256 vector registers without scratch.  A compiler that spills there costs time silently (spills of 236 and 518
-  registers were seen while the kernel was written).  The NVFP4 kernel's figures are recorded with a ceiling.
+  registers were seen while the kernel was written).  So must the few-rows kernels, whose operands go straight to
+  registers (with packed fp32 instructions allowed the INT4 forms spill 328 to 380 bytes per lane).  The NVFP4 kernel's figures
+  are recorded with a ceiling.
 * Flags across inline assembly.  The asynchronous global -> LDS copies are inline assembly that writes ``m0`` and, where
   it adds, the scalar condition code (SCC).  A build whose asm statements did not declare that had the compiler keep the
   carry of a 64-bit pointer addition (``s_add_u32`` ... ``s_addc_u32``) and the result of ``ng < 2`` in SCC across such
@@ -102,7 +104,7 @@ def test_fp6_conversion_never_overwrites_its_own_inputs():
     assert not fp6_conversions_with_overlap(["\tv_cvt_scalef32_2xpk16_fp6_f32 v[34:39], v[2:17], v[18:33], s52"])[1]
     flags = [f for f in nv.HIPCC_FLAGS if f not in ("-shared", "-fPIC")]
     with tempfile.TemporaryDirectory(prefix="svdq_guard_") as tmp:
-        for src, extra in (("quantize.hip", []), ("gemm6_variant.hip", ["-DSVDQ_VARIANT=1"])):
+        for src, extra in (("quantize.hip", []), ("gemm6_variant.hip", ["-DSVDQ_VARIANT=1"]), ("gemm_direct_variant.hip", ["-DSVDQ_VARIANT=1"])):
             out = Path(tmp) / (src + ".s")
             res = subprocess.run(["/opt/rocm/bin/hipcc", *flags, *extra, "-S", "--cuda-device-only", str(CSRC / src), "-o", str(out)],
                                  capture_output=True, text=True)
@@ -159,7 +161,7 @@ def test_the_build_before_the_clobbers_were_declared_kept_flags_across_the_copie
 
 @pytest.fixture(scope="module")
 def compiled():
-    units = [("gemm6_variant.hip", 0), ("gemm6_variant.hip", 1), ("gemm_variant.hip", 4), ("gemm_variant.hip", 5)]
+    units = nv.GEMM_VARIANT_UNITS
     with tempfile.TemporaryDirectory(prefix="svdq_guard_") as tmp:
         with ThreadPoolExecutor(max_workers=4) as pool:
             results = list(pool.map(lambda u: compile_variant(u[0], u[1], tmp), units))
@@ -182,6 +184,16 @@ def test_int4_gemm_fits_its_registers(compiled, variant):
     assert u["Occupancy"] >= 2, u
 
 
+@pytest.mark.parametrize("variant", [0, 1, 2, 3])
+def test_few_rows_gemm_fits_its_registers(compiled, variant):
+    usage, _ = compiled[("gemm_direct_variant.hip", variant)]
+    kernels = {k: u for k, u in usage.items() if "gemm_direct_kernel" in k}
+    assert len(kernels) == 2, list(usage)  # tiles of 32 and of 64 rows
+    for name, u in kernels.items():
+        print(name, u)
+        assert u["VGPRs"] <= 256 and u["AGPRs"] == 0 and u["ScratchSize"] == 0 and u["Occupancy"] >= 2, (name, u)
+
+
 @pytest.mark.parametrize("variant,max_scratch", [(4, 48), (5, 256)])
 def test_nvfp4_gemm_register_figures(compiled, variant, max_scratch):
     usage, _ = compiled[("gemm_variant.hip", variant)]
@@ -192,8 +204,9 @@ def test_nvfp4_gemm_register_figures(compiled, variant, max_scratch):
     assert u["ScratchSize"] <= max_scratch, u
 
 
-@pytest.mark.parametrize("unit", [("gemm6_variant.hip", 0), ("gemm6_variant.hip", 1), ("gemm_variant.hip", 4), ("gemm_variant.hip", 5)])
+@pytest.mark.parametrize("unit", nv.GEMM_VARIANT_UNITS)
 def test_no_condition_code_kept_across_inline_asm(compiled, unit):
     _, lines = compiled[unit]
-    assert sum("#ASMSTART" in l for l in lines) > 0
+    # (of the few-rows kernels only the INT4 one with the quantizing epilogue has inline assembly, the fp6 conversion)
+    assert sum("#ASMSTART" in l for l in lines) > 0 or (unit[0] == "gemm_direct_variant.hip" and unit[1] != 1)
     assert scc_live_across_asm(lines) == []
