@@ -438,7 +438,13 @@ void plan_int4(const svdq_gemm_args *a, int ncu, svdq_gemm_plan *plan) {
     }
 }
 
-constexpr int FULL_BAND = 10, HALF_BAND = 20;  // row blocks per band at most, see g6::tile_of
+void lay_out_tiles(const svdq_gemm_plan &plan, g6::Params &p) {
+    p.full_blocks = plan.full_blocks;
+    p.half_blocks = plan.half_blocks;
+    p.kparts = plan.kparts;
+    p.band = g6::band_height(p.full_blocks, 10);  // (see g6::tile_of)
+    p.half_band = g6::band_height(p.half_blocks, 20);
+}
 
 int gemm_int4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t st, int dev, bool noalloc) {
     g6::Params p;
@@ -479,12 +485,8 @@ int gemm_int4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t s
 
     // One workgroup per output tile (or per part of one split along K), two resident per compute unit.
     const int nblocks = (p.N + g6::BN - 1) / g6::BN;
-    p.full_blocks = plan.full_blocks;
-    p.half_blocks = plan.half_blocks;
-    p.kparts = plan.kparts;
+    lay_out_tiles(plan, p);
     const int kparts = p.kparts, ntiles = (p.full_blocks + p.half_blocks) * nblocks;
-    p.band = g6::band_height(p.full_blocks, FULL_BAND);
-    p.half_band = g6::band_height(p.half_blocks, HALF_BAND);
     const bool next = needs_next_epilogue(a);
     const size_t cnt_bytes = (size_t)ntiles * 4;
     const size_t part_bytes = kparts > 1 ? (size_t)ntiles * kparts * g6::BM * g6::BN * 4 : 0;
@@ -818,8 +820,9 @@ extern "C" int svdq_gemm_plan_of(const svdq_gemm_args *a, int64_t rows, int comp
 
 extern "C" void svdq_gemm_int4_tile(const svdq_gemm_plan *plan, int64_t N, int block, svdq_gemm_tile *tile) {
     const int nblocks = (int)((N + g6::BN - 1) / g6::BN);
-    const g6::TileOf t = g6::tile_of(block, (plan->full_blocks * plan->kparts + plan->half_blocks) * nblocks, nblocks, plan->full_blocks, plan->half_blocks,
-                                     g6::band_height(plan->full_blocks, FULL_BAND), g6::band_height(plan->half_blocks, HALF_BAND), plan->kparts);
+    g6::Params p;
+    lay_out_tiles(*plan, p);
+    const g6::TileOf t = g6::tile_of(p, block, (p.full_blocks * p.kparts + p.half_blocks) * nblocks, nblocks);
     const int rows = t.whole ? g6::BM : g6::BM / 2, before = t.whole ? 0 : plan->full_blocks;
     *tile = svdq_gemm_tile{before * g6::BM + t.row_block * rows, rows, t.column_block, t.part, before + t.row_block, t.tile};
 }

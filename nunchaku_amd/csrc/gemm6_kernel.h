@@ -749,7 +749,7 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
 
 template <bool NEXT>
 __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
-    const TileOf t = tile_of((int)blockIdx.x, (int)gridDim.x, (p.N + BN - 1) / BN, p.full_blocks, p.half_blocks, p.band, p.half_band, p.kparts);
+    const TileOf t = tile_of(p, (int)blockIdx.x, (int)gridDim.x, (p.N + BN - 1) / BN);
     if (t.whole) output_tile<NEXT, 2>(p, t.row_block * BM, t.column_block, t.tile, t.part, t.row_block);
     else output_tile<NEXT, 1>(p, p.full_blocks * BM + t.row_block * (BM / 2), t.column_block, 0, 0, p.full_blocks + t.row_block);
 }

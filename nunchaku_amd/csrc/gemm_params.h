@@ -233,16 +233,17 @@ struct TileOf {
     int row_block;  // among the blocks of its height
     int column_block, tile, part;
 };
-__host__ __device__ inline TileOf tile_of(int block, int total, int nblocks, int full_blocks, int half_blocks, int full_band, int half_band, int kparts) {
-    const int full = full_blocks * nblocks * kparts;
+template <typename P>
+__host__ __device__ __forceinline__ TileOf tile_of(const P &p, int block, int total, int nblocks) {
+    const int full = p.full_blocks * nblocks * p.kparts;
     const int xcd = block % 8, j = block / 8;
     const int first = xcd * (full / 8) + (xcd < full % 8 ? xcd : full % 8);  // of this XCD's 128-row tiles
     const int count = full / 8 + (xcd < full % 8 ? 1 : 0);
     const bool whole = j < count;
     // (the 64-row tiles of the XCDs before this one: their workgroups less their 128-row tiles)
     const int v = whole ? first + j : xcd * (total / 8) + (xcd < total % 8 ? xcd : total % 8) - first + (j - count);
-    const int tile = whole ? v / kparts : v, part = whole ? v - tile * kparts : 0;
-    const int blocks = whole ? full_blocks : half_blocks, band_blocks = whole ? full_band : half_band;
+    const int tile = whole ? v / p.kparts : v, part = whole ? v - tile * p.kparts : 0;
+    const int blocks = whole ? p.full_blocks : p.half_blocks, band_blocks = whole ? p.band : p.half_band;
     const int band = tile / (band_blocks * nblocks), in_band = tile - band * (band_blocks * nblocks);
     const int rows = blocks - band * band_blocks < band_blocks ? blocks - band * band_blocks : band_blocks;
     const int mb = band * band_blocks + in_band % rows, nb = in_band / rows;
