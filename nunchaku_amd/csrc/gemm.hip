@@ -302,19 +302,22 @@ int rows_needed(const svdq_gemm_args *a) {
 // leaves the split along K to the library.  The last tiles of a launch leave compute units idle for the time of a whole
 // tile (the hardware hands tiles to the emptiest compute unit; with 1296 tiles 16 of 256 work 22 us longer than the
 // others); in tiles of half the height the last rows fill them up.
-// A model of the busiest compute unit's time, in units of a whole tile alone on one, fitted to 600 launches of 70 shapes (M = 300
-// ... 9216, K = 1024 ... 12800, N = 1024 ... 21504): a pair of whole tiles side by side takes 1.55, of half tiles 0.9, a half tile alone
-// 0.7; a half tile next to a last odd whole one 1.1 together with it, two of them 2.0 (the second starts when the first is done).
+// A model of the busiest compute unit's time, in units of a whole tile alone on one, fitted to every division considered of 700
+// shapes (M = 256 ... 18432, K = 1024 ... 12288, N = 1024 ... 21504) and checked on 700 others: a pair of whole tiles side by side
+// takes 1.55, of half tiles 0.9, a half tile alone 0.7; a half tile next to a last odd whole one 1.2 together with it, two of them 2.0
+// (the second starts when the first is done), each one more 0.45.
 // Every compute unit gets `tiles / ncu` whole tiles or one more, the half tiles go where they end first.  Considered are whole
 // tiles only, whole tiles up to the last and the last but one multiple of the compute units, and (few tiles) half tiles only; a
 // division with half tiles has to be 4 % faster by the model.  Measured, whole tiles / the choice: M = 4608, K = 3072, N = 9216
-// 140 / 131 us; M = 4096, K = 2304, N = 6912 72.3 / 66.3; M = 1024, K = 3072, N = 9216 44.5 / 34.3; M = 505 of the same layer 32.9 / 28.7;
-// over the 70 shapes 1.16 times as fast, 1.4 % off the best division measured.
+// 140 / 131 us; M = 4096, K = 2304, N = 6912 72.3 / 66.3; M = 1024, K = 3072, N = 9216 44.5 / 34.3; M = 505 of the same layer 32.9 / 28.7.
+// Over the 700 other shapes 1.10 times as fast as whole tiles, 0.2 % off the best division measured, more than 3 % slower than whole
+// tiles in one.  (With 1.1 and 0.25, where three half tiles fit behind an odd whole one: slower in six, M = 4096, K = 3072, N = 9216, which
+// is whole tiles only now, 129 against 124.)
 double half_tiles_time(int n) { return 0.9 * (n / 2) + 0.7 * (n % 2); }
 double unit_time(int whole, int half) {
     const double pairs = 1.55 * (whole / 2);
     if (whole % 2 == 0) return pairs + half_tiles_time(half);
-    return pairs + (half == 0 ? 1.0 : half == 1 ? 1.1 : 2.0 + 0.25 * (half - 2));
+    return pairs + (half == 0 ? 1.0 : half == 1 ? 1.2 : 2.0 + 0.45 * (half - 2));
 }
 double launch_time(long long whole, long long half, int ncu) {  // (in tiles)
     const int q = (int)(whole / ncu);

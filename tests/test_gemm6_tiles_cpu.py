@@ -59,6 +59,8 @@ def test_rows_of_a_call_without_out():
     ("plain", 256, 3072, 3072, False, dict(few_rows=1)), ("plain", 1157, 3072, 3072, False, dict(few_rows=2)), ("plain", 505, 3072, 9216, False, dict(half_blocks=8)),
     ("plain", 256, 12288, 3072, False, dict(few_rows=1)), ("plain", 505, 12288, 3072, False, dict(few_rows=2)), ("plain", 1536, 6144, 1536, False, dict(kparts=3)),
     ("plain", 4608, 3072, 9216, False, dict(full_blocks=35, half_blocks=2)), ("plain", 4608, 3072, 12288, False, dict(full_blocks=36)),
+    # (slower in blocks of two heights than in whole tiles: they would fit exactly by an even finish that the hardware does not reach)
+    ("plain", 4096, 3072, 9216, False, dict(full_blocks=32)), ("rope", 4096, 6144, 9216, False, dict(full_blocks=32)), ("plain", 2048, 3072, 18432, False, dict(full_blocks=16)),
     ("plain", 300, 3072, 3072, True, dict(few_rows=1)), ("plain", 1157, 12288, 3072, True, dict(few_rows=2)), ("plain", 4608, 3072, 21504, True, dict(workgroups=252)),
     ("plain", 4608, 15360, 3072, True, dict(workgroups=216)), ("plain", 4608, 3072, 4608, True, dict(workgroups=256, shared_tiles=1)),
     ("next", 2304, 256, 7680, True, dict(few_rows=2)), ("next", 4608, 4096, 4608, True, dict(workgroups=256, shared_tiles=1)),
