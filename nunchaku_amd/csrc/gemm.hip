@@ -634,6 +634,10 @@ int choose_direct(const svdq_gemm_args *a, int ncu) {
         t_large = one * rounds + (tiles > 1.0 && !nwg ? 33.0 : 0.0);
         t1 = 4.3 + c1 * (1.1 + 0.127 * kg);
         t2 = 5.0 + c2 * (1.6 + 0.205 * kg) - (c2 < 3.0 ? 0.04 * kg : 0.0);
+        // Short rows and many rounds: the outputs set the pace of both kernels, and the large tiles write them faster (M = 4608, K = 384,
+        // N = 9088 69 us in shape 2 against 63; M = 6400, K = 640, N = 16384 210 against 181; M = 11008, K = 1024, N = 8576 242 against 229; of
+        // 1572 random shapes 22 were slower by more than 3 % in the kernel chosen, with this term two).
+        if (kg <= 16 && c2 > 12.0) t2 += 0.9 * (c2 - 12.0);
         if (a->qout) {  // (the quantizing epilogue: M = 4608, K = 3072, N = 12288 298 -> 387 us in large tiles, 317 -> 358 in shape 2)
             t_large += 20.0 * rounds;
             t1 += 1.1 * c1;
