@@ -42,6 +42,79 @@ struct QuantParams {
 
 constexpr uint32_t RSRC_WORD3 = 0x00020000;  // raw buffer, 32-bit data format
 
+// A wave-uniform number made scalar explicitly, where the compiler would work it out in a vector register.
+__device__ inline int scalar(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+template <int NW, bool GLU>
+struct TransposeArea {  // per wave: 16 rows of a chunk on their way from the load layout to the operand layout
+    uint8_t bytes[NW][16 * (GLU ? 32 : 16) * 16];
+};
+
+// The projection alone, onto the RTW rank tiles from rt0 on (the second one may lie beyond the rank: not stored), of the 16
+// rows 16 blockIdx.x ...: wave w takes the chunks w, w + NW, ..., DEPTH of them requested ahead, proj_down included (in
+// the kernel below the quantizer covers the latency of its operands).  x goes from whole-line requests to the operand layout
+// through the wave's transposition area `tr` as there (fetched in the operand layout, 16 rows x 64 bytes per instruction:
+// 7.1 us against 5.4 at M = 256, K = 3072); the waves' sums meet in `red` and are added in ascending order.
+template <int NW, int DEPTH, int RTW>
+__device__ __forceinline__ void project_rows(const QuantParams &p, int rt0, uint8_t *tr, float *red) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    const int row0 = blockIdx.x * 16, nchunks = p.K / 128, RT_all = p.R / 16;
+    const int rt1 = rt0 + 1 < RT_all ? rt0 + 1 : rt0;
+    int rows_valid = (p.M < row0 + 16 ? p.M : row0 + 16) - row0;
+    rows_valid = rows_valid < 0 ? 0 : rows_valid;
+    const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(p.x + (size_t)row0 * p.K), 0, rows_valid * p.K * 2, RSRC_WORD3);
+    const __amdgpu_buffer_rsrc_t drsrc = __builtin_amdgcn_make_buffer_rsrc((void *)p.down, 0, p.K * p.R * 2, RSRC_WORD3);
+    const uint32_t x_voff = (uint32_t)((lane / 16) * p.K * 2 + (lane % 16) * 16);
+    auto rot = [](int row) { return row & 11; };
+
+    u32x4_t x[DEPTH + 1][4], d[DEPTH + 1][RTW][4];
+    auto load = [&](int c, auto S) {
+        constexpr int s = decltype(S)::value;
+        const uint32_t beyond = c < nchunks ? 0u : 0x80000000u;  // (reads zeros and touches no memory, see the kernel below)
+        each(std::make_integer_sequence<int, 4>{}, [&](auto I) {
+            constexpr int i = decltype(I)::value;
+            x[s][i] = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, (x_voff | beyond) + (uint32_t)(4 * i * p.K * 2), c * 256, 0);
+            d[s][0][i] = __builtin_amdgcn_raw_buffer_load_b128(drsrc, (uint32_t)(lane * 16) | beyond, ((c * 4 + i) * RT_all + rt0) * 1024, 0);
+            if constexpr (RTW > 1) d[s][1][i] = __builtin_amdgcn_raw_buffer_load_b128(drsrc, (uint32_t)(lane * 16) | beyond, ((c * 4 + i) * RT_all + rt1) * 1024, 0);
+        });
+    };
+    float4_t acc[2] = {float4_t{0.f, 0.f, 0.f, 0.f}, float4_t{0.f, 0.f, 0.f, 0.f}};
+    each(std::make_integer_sequence<int, DEPTH>{}, [&](auto D) { load(wave + decltype(D)::value * NW, D); });
+    // (chunks past the end multiply zeros: whole turns of the ring)
+    for (int c = wave; c < nchunks; c += (DEPTH + 1) * NW) {
+        each(std::make_integer_sequence<int, DEPTH + 1>{}, [&](auto S) {
+            constexpr int s = decltype(S)::value;
+            load(c + (s + DEPTH) * NW, std::integral_constant<int, (s + DEPTH) % (DEPTH + 1)>{});
+            __builtin_amdgcn_sched_barrier(0);
+            each(std::make_integer_sequence<int, 4>{}, [&](auto I) {
+                constexpr int i = decltype(I)::value;
+                const int row = 4 * i + lane / 16;
+                *(u32x4_t *)(tr + row * 256 + ((lane + rot(row)) % 16) * 16) = x[s][i];
+            });
+            each(std::make_integer_sequence<int, 4>{}, [&](auto I) {
+                constexpr int i = decltype(I)::value;
+                x[s][i] = *(const u32x4_t *)(tr + r * 256 + ((4 * q + i + rot(r)) % 16) * 16);
+                acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[s][i]), __builtin_bit_cast(bf16x8_t, d[s][0][i]), acc[0], 0, 0, 0);
+                if constexpr (RTW > 1) acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[s][i]), __builtin_bit_cast(bf16x8_t, d[s][1][i]), acc[1], 0, 0, 0);
+            });
+        });
+    }
+    __syncthreads();  // (`red` lies where the waves' transposition areas do)
+    *(float4_t *)&red[(wave * 2 * 64 + lane) * 4] = acc[0];
+    *(float4_t *)&red[((wave * 2 + 1) * 64 + lane) * 4] = acc[1];
+    __syncthreads();
+    // 512 sums: rank tile, row and rank of it by the result layout of the 16 x 16 matrix instruction
+    for (int idx = threadIdx.x; idx < 256 * RTW; idx += 64 * NW) {
+        const int rank = idx & 15, row = (idx >> 4) & 15, rt = idx >> 8;
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; w++) sum += red[((w * 2 + rt) * 64 + 16 * (row / 4) + rank) * 4 + row % 4];
+        if (rt0 + rt < RT_all) p.lora_out[(size_t)(row0 + row) * p.R + 16 * (rt0 + rt) + rank] = sum;
+    }
+}
+
 // SMOOTH: 0 = no smoothing factors, 1 = the K reciprocal factors are copied to LDS once per workgroup,
 // 2 = read from global memory per chunk (K too large for LDS).
 //
@@ -61,14 +134,29 @@ constexpr uint32_t RSRC_WORD3 = 0x00020000;  // raw buffer, 32-bit data format
 // live in registers), so the operator launches the kernel once per window of 128 ranks; the launches after the
 // first (QUANT false) read x again, which the caches still hold, and neither quantize nor store codes.
 //
-// QUANT, PROJECT: what this workgroup does with its chunks; cfirst, cstep: the chunks of this wave.
-template <int NW, int MT, int RT_MAX, int DEPTH, bool FP4, int SMOOTH, bool GLU, bool ROWS, bool QUANT, bool PROJECT>
-__device__ __forceinline__ void quantize_rows(const QuantParams &p, int cfirst, int cstep, uint8_t *tr) {
+// FEW: few rows (dispatch: up to 8 per compute unit).  One workgroup per 16 rows leaves most of the chip idle while eight waves
+// walk K, about 1 us per chunk of 128 columns, most of it the quantizer's arithmetic.  Nothing ties the codes of one
+// chunk to those of another, or to the projection: blockIdx.y < p.splits quantize a share of the chunks each, the
+// workgroups behind them project the same rows onto FEW rank tiles each, so that all ranks take one launch.  What is left is
+// launch, two or three memory latencies and, for long rows, the projection's walk over K.  Before / now: K = 3072, rank 32:
+// M = 256 6.9 / 4.4 us, M = 1024 8.1 / 5.4, M = 2048 8.8 / 7.2; K = 12288: M = 256 18.1 / 8.8, M = 1024 23.3 / 12.5;
+// rank 128: M = 256, K = 3072 18.7 / 4.6, M = 1024, K = 12288 107 / 21; rank 256: M = 256 36 / 5.7.
+// (One kernel for all forms: with the body in a function that two kernels called, the compiler carried the chunk's offset in a vector
+// register in 27 instances that had it in a scalar one, and looped over it lane by lane for every request.  Rank 128: M = 8448, K = 6144
+// 96.6 us as it is, 100.3 from a function; M = 5120, K = 16512 106 and 402.)
+template <int NW, int MT, int RT_MAX, int DEPTH, bool FP4, int SMOOTH, bool GLU, bool ROWS, bool QUANT = true, int FEW = 0>
+__global__ void __launch_bounds__(64 * NW) quantize_fuse_lora_kernel(QuantParams p) {
     // smoothing factors [K] during the walk; then, chunks split: [NW waves][MT][RT][64][4] partial projections;
     // rows split: behind the factors two buffers of [4 steps][RT][64 lanes] x 16 bytes of proj_down
     extern __shared__ __attribute__((aligned(16))) float lds[];  // (the alignment lets the factors be read 16 bytes at a time)
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    __shared__ __attribute__((aligned(16))) TransposeArea<NW, GLU> area;
+    uint8_t *tr = area.bytes[wave];
+    constexpr bool PROJECT = FEW == 0;
+    if constexpr (FEW > 0) {
+        if ((int)blockIdx.y >= p.splits) return project_rows<NW, FEW == 1 ? 2 : 1, FEW>(p, ((int)blockIdx.y - p.splits) * FEW, tr, (float *)area.bytes);
+    }
     const int r = lane & 15, q = lane >> 4;
     const int row0 = ROWS ? (blockIdx.x * NW + wave) * (16 * MT) : blockIdx.x * (16 * MT);
     const int row_end = row0 + 16 * MT;  // the rows this workgroup (ROWS: wave) writes are [row0, row_end)
@@ -109,7 +197,12 @@ __device__ __forceinline__ void quantize_rows(const QuantParams &p, int cfirst, 
     // worst on every path and wait for the chunks requested ahead): a chunk index past the end gets a lane
     // offset beyond the buffer size instead, which reads zeros and touches no memory.  (The hardware checks
     // the lane offset against the size, not the scalar offset that carries the chunk.)
-    auto load_x = [&](int c, u32x4_t (&xv)[MT][XL]) {
+    // (Eight waves on 32 rows at ranks above 64, where the loads of proj_down have their offsets worked out lane by lane otherwise:
+    // M = 4608, K = 6144, rank 128 52.9 -> 41.8 us, rank 256 107 -> 77.  Not in the other forms: no change or a loss, four waves at rank 128 in
+    // NVFP4 51 -> 77.)
+    constexpr bool SCALAR_CHUNK = MT == 2 && RT_MAX == 8;
+    auto load_x = [&](int chunk, u32x4_t (&xv)[MT][XL]) {
+        const int c = SCALAR_CHUNK ? scalar(chunk) : chunk;
         const uint32_t beyond = c < nchunks ? 0u : 0x80000000u;
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
@@ -125,6 +218,8 @@ __device__ __forceinline__ void quantize_rows(const QuantParams &p, int cfirst, 
 
     // DEPTH chunks are requested ahead of the one being worked on
     u32x4_t xv[DEPTH + 1][MT][XL];
+    const int cstep = FEW ? p.splits * NW : ROWS ? 1 : NW;  // distance between the chunks a wave works on
+    const int cfirst = FEW ? blockIdx.y * NW + wave : ROWS ? 0 : wave;
 #pragma unroll
     for (int s = 0; s < DEPTH; s++) load_x(cfirst + s * cstep, xv[s]);
 
@@ -160,7 +255,8 @@ __device__ __forceinline__ void quantize_rows(const QuantParams &p, int cfirst, 
         __syncthreads();
     }
 
-    auto process = [&](int c, u32x4_t (&xin)[MT][XL], u32x4_t (&x_ahead)[MT][XL]) {
+    auto process = [&](int chunk, u32x4_t (&xin)[MT][XL], u32x4_t (&x_ahead)[MT][XL]) {
+        const int c = SCALAR_CHUNK ? scalar(chunk) : chunk;
         const int kbase = 128 * c + 32 * q;
         // ---- from the load layout to the operand layout: lane (r, q) gets the XL pieces XL * q + i of row r.
         // Row-major in LDS with the pieces of row r rotated by rot(r).  A 16-byte write is served eight consecutive
@@ -353,98 +449,6 @@ walked:
     }
 }
 
-template <int NW, bool GLU>
-struct TransposeArea {  // per wave: 16 rows of a chunk on their way from the load layout to the operand layout
-    uint8_t bytes[NW][16 * (GLU ? 32 : 16) * 16];
-};
-
-template <int NW, int MT, int RT_MAX, int DEPTH, bool FP4, int SMOOTH, bool GLU, bool ROWS, bool QUANT = true>
-__global__ void __launch_bounds__(64 * NW) quantize_fuse_lora_kernel(QuantParams p) {
-    __shared__ __attribute__((aligned(16))) TransposeArea<NW, GLU> area;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    quantize_rows<NW, MT, RT_MAX, DEPTH, FP4, SMOOTH, GLU, ROWS, QUANT, true>(p, ROWS ? 0 : wave, ROWS ? 1 : NW, area.bytes[wave]);
-}
-
-// The projection alone, onto the RTW rank tiles from rt0 on (the second one may lie beyond the rank: not stored), of the 16
-// rows 16 blockIdx.x ...: wave w takes the chunks w, w + NW, ..., DEPTH of them requested ahead, proj_down included (in
-// quantize_rows the quantizer covers the latency of its operands).  x goes from whole-line requests to the operand layout
-// through the wave's transposition area `tr` as there (fetched in the operand layout, 16 rows x 64 bytes per instruction:
-// 7.1 us against 5.4 at M = 256, K = 3072); the waves' sums meet in `red` and are added in ascending order.
-template <int NW, int DEPTH, int RTW>
-__device__ __forceinline__ void project_rows(const QuantParams &p, int rt0, uint8_t *tr, float *red) {
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int r = lane & 15, q = lane >> 4;
-    const int row0 = blockIdx.x * 16, nchunks = p.K / 128, RT_all = p.R / 16;
-    const int rt1 = rt0 + 1 < RT_all ? rt0 + 1 : rt0;
-    int rows_valid = (p.M < row0 + 16 ? p.M : row0 + 16) - row0;
-    rows_valid = rows_valid < 0 ? 0 : rows_valid;
-    const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(p.x + (size_t)row0 * p.K), 0, rows_valid * p.K * 2, RSRC_WORD3);
-    const __amdgpu_buffer_rsrc_t drsrc = __builtin_amdgcn_make_buffer_rsrc((void *)p.down, 0, p.K * p.R * 2, RSRC_WORD3);
-    const uint32_t x_voff = (uint32_t)((lane / 16) * p.K * 2 + (lane % 16) * 16);
-    auto rot = [](int row) { return row & 11; };
-
-    u32x4_t x[DEPTH + 1][4], d[DEPTH + 1][RTW][4];
-    auto load = [&](int c, auto S) {
-        constexpr int s = decltype(S)::value;
-        const uint32_t beyond = c < nchunks ? 0u : 0x80000000u;  // (reads zeros and touches no memory, see quantize_rows)
-        each(std::make_integer_sequence<int, 4>{}, [&](auto I) {
-            constexpr int i = decltype(I)::value;
-            x[s][i] = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, (x_voff | beyond) + (uint32_t)(4 * i * p.K * 2), c * 256, 0);
-            d[s][0][i] = __builtin_amdgcn_raw_buffer_load_b128(drsrc, (uint32_t)(lane * 16) | beyond, ((c * 4 + i) * RT_all + rt0) * 1024, 0);
-            if constexpr (RTW > 1) d[s][1][i] = __builtin_amdgcn_raw_buffer_load_b128(drsrc, (uint32_t)(lane * 16) | beyond, ((c * 4 + i) * RT_all + rt1) * 1024, 0);
-        });
-    };
-    float4_t acc[2] = {float4_t{0.f, 0.f, 0.f, 0.f}, float4_t{0.f, 0.f, 0.f, 0.f}};
-    each(std::make_integer_sequence<int, DEPTH>{}, [&](auto D) { load(wave + decltype(D)::value * NW, D); });
-    // (chunks past the end multiply zeros: whole turns of the ring)
-    for (int c = wave; c < nchunks; c += (DEPTH + 1) * NW) {
-        each(std::make_integer_sequence<int, DEPTH + 1>{}, [&](auto S) {
-            constexpr int s = decltype(S)::value;
-            load(c + (s + DEPTH) * NW, std::integral_constant<int, (s + DEPTH) % (DEPTH + 1)>{});
-            __builtin_amdgcn_sched_barrier(0);
-            each(std::make_integer_sequence<int, 4>{}, [&](auto I) {
-                constexpr int i = decltype(I)::value;
-                const int row = 4 * i + lane / 16;
-                *(u32x4_t *)(tr + row * 256 + ((lane + rot(row)) % 16) * 16) = x[s][i];
-            });
-            each(std::make_integer_sequence<int, 4>{}, [&](auto I) {
-                constexpr int i = decltype(I)::value;
-                x[s][i] = *(const u32x4_t *)(tr + r * 256 + ((4 * q + i + rot(r)) % 16) * 16);
-                acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[s][i]), __builtin_bit_cast(bf16x8_t, d[s][0][i]), acc[0], 0, 0, 0);
-                if constexpr (RTW > 1) acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[s][i]), __builtin_bit_cast(bf16x8_t, d[s][1][i]), acc[1], 0, 0, 0);
-            });
-        });
-    }
-    __syncthreads();  // (`red` lies where the waves' transposition areas do)
-    *(float4_t *)&red[(wave * 2 * 64 + lane) * 4] = acc[0];
-    *(float4_t *)&red[((wave * 2 + 1) * 64 + lane) * 4] = acc[1];
-    __syncthreads();
-    // 512 sums: rank tile, row and rank of it by the result layout of the 16 x 16 matrix instruction
-    for (int idx = threadIdx.x; idx < 256 * RTW; idx += 64 * NW) {
-        const int rank = idx & 15, row = (idx >> 4) & 15, rt = idx >> 8;
-        float sum = 0.f;
-#pragma unroll
-        for (int w = 0; w < NW; w++) sum += red[((w * 2 + rt) * 64 + 16 * (row / 4) + rank) * 4 + row % 4];
-        if (rt0 + rt < RT_all) p.lora_out[(size_t)(row0 + row) * p.R + 16 * (rt0 + rt) + rank] = sum;
-    }
-}
-
-// Few rows (dispatch: up to 8 per compute unit).  One workgroup per 16 rows leaves most of the chip idle while eight waves
-// walk K, about 1 us per chunk of 128 columns, most of it the quantizer's arithmetic.  Nothing ties the codes of one
-// chunk to those of another, or to the projection: blockIdx.y < p.splits quantize a share of the chunks each, the
-// workgroups behind them project the same rows onto RTW rank tiles each, so that all ranks take one launch.  What is left is
-// launch, two or three memory latencies and, for long rows, the projection's walk over K.  Before / now: K = 3072, rank 32:
-// M = 256 6.9 / 4.4 us, M = 1024 8.1 / 5.4, M = 2048 8.8 / 7.2; K = 12288: M = 256 18.1 / 8.8, M = 1024 23.3 / 12.5;
-// rank 128: M = 256, K = 3072 18.7 / 4.6, M = 1024, K = 12288 107 / 21; rank 256: M = 256 36 / 5.7.
-template <int NW, int RTW, bool FP4, bool SMOOTH>
-__global__ void __launch_bounds__(64 * NW) quantize_few_rows_kernel(QuantParams p) {
-    __shared__ __attribute__((aligned(16))) TransposeArea<NW, false> area;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if ((int)blockIdx.y < p.splits) quantize_rows<NW, 1, 1, 1, FP4, SMOOTH ? 2 : 0, false, false, true, false>(p, blockIdx.y * NW + wave, p.splits * NW, area.bytes[wave]);
-    else project_rows<NW, RTW == 1 ? 2 : 1, RTW>(p, ((int)blockIdx.y - p.splits) * RTW, area.bytes[wave], (float *)area.bytes);
-}
-
 constexpr size_t SMOOTH_LDS_MAX = 64 * 1024;  // two workgroups of a compute unit must fit side by side
 
 template <int NW, int MT, int RT_MAX, int DEPTH, bool FP4, int SMOOTH, bool GLU, bool ROWS = false, bool QUANT = true>
@@ -484,8 +488,8 @@ int project_further(const QuantParams &p0, hipStream_t stream) {
 template <int RTW, bool FP4>
 int launch_few_rows(const QuantParams &p, hipStream_t stream) {
     const dim3 grid(p.M_pad / 16, p.splits + (p.R / 16 + RTW - 1) / RTW);
-    if (p.smooth_rcp) SVDQ_LAUNCH((quantize_few_rows_kernel<8, RTW, FP4, true>), grid, dim3(512), 0, stream, p);
-    else SVDQ_LAUNCH((quantize_few_rows_kernel<8, RTW, FP4, false>), grid, dim3(512), 0, stream, p);
+    if (p.smooth_rcp) SVDQ_LAUNCH((quantize_fuse_lora_kernel<8, 1, 1, 1, FP4, 2, false, false, true, RTW>), grid, dim3(512), 0, stream, p);
+    else SVDQ_LAUNCH((quantize_fuse_lora_kernel<8, 1, 1, 1, FP4, 0, false, false, true, RTW>), grid, dim3(512), 0, stream, p);
     return check_launch("quantize_w4a4_act_fuse_lora (few rows)");
 }
 
@@ -506,14 +510,16 @@ int dispatch(const QuantParams &p, hipStream_t stream) {
         // Up to 8 rows per compute unit: quantizing and projecting workgroups apart, about one workgroup per compute unit (M = 1024,
         // rank 32: 256 workgroups 5.4 us, 320 6.4).  One rank tile per projecting workgroup where they all fit beside the
         // quantizing ones (M = 256: 4.4 us, with two 5.5), otherwise two; at ranks above 32 at least three shares of the
-        // quantizing (M = 1024, rank 128: 7.9 us, with one 10.4).  From 16 rows per compute unit on the forms below are
+        // quantizing (M = 1024, rank 128: 7.9 us, with one 10.4), or two where no more workgroups are resident at once (two per compute
+        // unit: M = 2048, rank 64, K = 12288: 22.2 us, with three 26.9).  From 16 rows per compute unit on the forms below are
         // faster (M = 4096: 11.5 us against 13.0).
         if (p.M_pad <= 8 * ncu) {
             QuantParams q = p;
             const int row_blocks = p.M_pad / 16, most = (p.K / 128 + 7) / 8;
             const bool one = row_blocks * (RT + 1) <= ncu;
             q.splits = ncu / row_blocks - (one ? RT : (RT + 1) / 2);
-            if (q.splits < (RT > 2 ? 3 : 1)) q.splits = RT > 2 ? 3 : 1;
+            const int least = RT <= 2 ? 1 : 2 * ncu / row_blocks - (RT + 1) / 2 == 2 ? 2 : 3;
+            if (q.splits < least) q.splits = least;
             if (q.splits > most) q.splits = most;
             return one ? launch_few_rows<1, FP4>(q, stream) : launch_few_rows<2, FP4>(q, stream);
         }
@@ -539,7 +545,7 @@ int dispatch(const QuantParams &p, hipStream_t stream) {
         if (RT <= 2 && (p.K > 6144 || p.M_pad >= 128 * ncu || (!FP4 && p.M_pad <= 32 * ncu))) return launch<8, 2, 2, 1, FP4, false>(p, stream);
         if (RT <= 2) return launch<4, 1, 2, 2, FP4, false>(p, stream);
         // Ranks 48 ... 128 below the row counts of the rows-split form: eight waves on 32 rows (M = 4608, K = 3072: rank
-        // 128 28.8 us, rank 64 16.0; four waves on the same rows 44.8 and 22.5; K = 12288, rank 128: 97 against 167).
+        // 128 24.8 us, rank 64 16.0; four waves on the same rows 44.8 and 22.5; K = 12288, rank 128: 76 against 167).
         if (RT <= 4) return launch<8, 2, 4, 1, FP4, false>(p, stream);
         // (NVFP4 at ranks 80 ... 128: the small workgroups at any row count, M = 4608: 29.7 us against 36.0, M = 12288: 57.7
         // against 71.1, K = 6144: 55.2 against 63.3; at rank 64 the large ones as for INT4, 16.5 against 25.1)

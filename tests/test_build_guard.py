@@ -18,6 +18,8 @@ cross-compiles gfx950 without a GPU).
   out wrong on the GPU (one instantiation of the quantize kernel, found by comparing configurations).  The compiler
   does not know; the source issues the instruction through inline assembly with an early-clobber destination, and the
   generated code of every kernel that converts is scanned for overlapping registers.
+* Buffer requests.  A descriptor or scalar offset that the compiler keeps in vector registers costs a loop over the lanes'
+  values around every request (``v_readfirstlane`` ... ``s_cbranch_execnz``), though all of them are the same.
 """
 
 import re
@@ -97,6 +99,44 @@ def fp6_conversions_with_overlap(lines):
             if not (d1 < a0 or d0 > a1) or not (d1 < b0 or d0 > b1):
                 bad.append((n + 1, l.strip()))
     return total, bad
+
+
+def lane_by_lane_requests(lines):
+    """Buffer requests inside a loop over the lanes' values, per kernel: {mangled name: count}."""
+    found, kernel, recent = {}, "", []
+    for text in lines:
+        m = re.match(r"^(_Z\w+):", text)
+        kernel = m.group(1) if m else kernel
+        if re.match(r"^\t[a-z]", text):
+            recent = [*recent[-3:], text.strip()]
+            if recent[-1].startswith("s_cbranch_execnz") and any(t.startswith("buffer_") for t in recent):
+                found[kernel] = found.get(kernel, 0) + 1
+    return found
+
+
+def test_quantize_requests_are_not_made_lane_by_lane():
+    """Not in the forms with the smoothing factors in LDS or without any.  (Those for longer rows than fit, K > 16384, and the few-rows
+    form have such loops.)"""
+    loop = """
+	v_readfirstlane_b32 s0, v0
+	s_nop 1
+	v_cmp_eq_u32_e32 vcc, s0, v0
+	s_and_saveexec_b64 vcc, vcc
+	s_nop 0
+	buffer_load_dwordx4 v[56:59], v1, s[20:23], s0 offen
+	s_xor_b64 exec, exec, vcc
+	s_cbranch_execnz .LBB53_16
+""".splitlines()
+    assert lane_by_lane_requests(loop) == {"": 1} and not lane_by_lane_requests(loop[:-1])
+    flags = [f for f in nv.HIPCC_FLAGS if f not in ("-shared", "-fPIC")]
+    with tempfile.TemporaryDirectory(prefix="svdq_guard_") as tmp:
+        out = Path(tmp) / "quantize.s"
+        res = subprocess.run(["/opt/rocm/bin/hipcc", *flags, "-S", "--cuda-device-only", str(CSRC / "quantize.hip"), "-o", str(out)], capture_output=True, text=True)
+        assert res.returncode == 0, res.stderr[-3000:]
+        bad = lane_by_lane_requests(out.read_text().splitlines())
+    # <NW, MT, RT_MAX, DEPTH, FP4, SMOOTH, GLU, ROWS, QUANT, FEW>
+    args = {name: [int(v) for v in re.findall(r"L[ib](\d+)E", name)] for name in bad}
+    assert not [name for name, a in args.items() if "quantize_fuse_lora_kernel" in name and a[5] != 2 and (a + [0])[9] == 0], bad
 
 
 def test_fp6_conversion_never_overwrites_its_own_inputs():

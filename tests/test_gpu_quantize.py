@@ -57,7 +57,8 @@ def test_int4_no_smooth_and_padding_rows(dev):
 
 @pytest.mark.parametrize("fp4", [False, True])
 def test_long_k_reads_smoothing_factors_from_global_memory(dev, fp4):
-    """K = 16512 (129 chunks, an odd count, 66 KB of reciprocal factors): beyond what the kernel keeps in LDS."""
+    """K = 16512 (129 chunks, an odd count, 66 KB of reciprocal factors): beyond what the kernel keeps in LDS.  (Few rows: that form
+    reads them from global memory at any K; the others below.)"""
     M, K, R = 40, 16512, 32
     announce(f"quantize long K M={M} K={K} fp4={fp4}")
     layer = synth.make_layer(128, K, R, seed=5, fp4=fp4)
@@ -229,6 +230,14 @@ def test_workgroup_shapes_by_rows_and_rank(dev, M, K, R, fp4):
     _check_row_sample(dev, M, K, R, fp4, True)
 
 
+@pytest.mark.parametrize("M,K,R,fp4", [(2049, 16512, 16, False), (2100, 16512, 64, True), (2304, 16512, 128, False), (8300, 16512, 80, False)])
+def test_long_k_beyond_the_few_rows(dev, M, K, R, fp4):
+    """The forms that read the smoothing factors from global memory for more rows than the few-rows form takes: 16 rows on eight
+    waves, 32 rows on eight waves at ranks 64 and 128, the rows-split form."""
+    announce(f"quantize long K M={M} K={K} R={R} fp4={fp4}")
+    _check_row_sample(dev, M, K, R, fp4, True)
+
+
 def _check_row_sample(dev, M, K, R, fp4, smooth):
     layer = synth.make_layer(128, K, R, seed=R + K, fp4=fp4)
     x = synth.make_activations(M, K, seed=M % 1000 + K)
@@ -250,7 +259,8 @@ def _check_row_sample(dev, M, K, R, fp4, smooth):
 
 
 @pytest.mark.parametrize("M,K,R,fp4,smooth", [(1, 128, 16, False, True), (250, 1152, 48, False, True), (33, 3200, 0, False, False), (600, 2176, 80, True, True),
-                                              (257, 9216, 32, True, False), (700, 512, 272, False, True), (2048, 1152, 32, False, True), (2000, 384, 144, True, True)])
+                                              (257, 9216, 32, True, False), (700, 512, 272, False, True), (2048, 1152, 32, False, True), (2000, 384, 144, True, True),
+                                              (1800, 3200, 64, False, True)])
 def test_few_rows_split_into_quantizing_and_projecting_workgroups(dev, M, K, R, fp4, smooth):
     """Up to 8 rows per compute unit: one chunk, fewer chunks than waves, counts of chunks that neither the shares nor the
     projection's ring divide; one rank tile per projecting workgroup and two, with a rank tile left over (ranks 48, 80, 144,
