@@ -511,14 +511,15 @@ int dispatch(const QuantParams &p, hipStream_t stream) {
         // rank 32: 256 workgroups 5.4 us, 320 6.4).  One rank tile per projecting workgroup where they all fit beside the
         // quantizing ones (M = 256: 4.4 us, with two 5.5), otherwise two; at ranks above 32 at least three shares of the
         // quantizing (M = 1024, rank 128: 7.9 us, with one 10.4), or two where no more workgroups are resident at once (two per compute
-        // unit: M = 2048, rank 64, K = 12288: 22.2 us, with three 26.9).  From 16 rows per compute unit on the forms below are
+        // unit: M = 2048, rank 64, K = 12288: 22.2 us, with three 26.9), and at rank 16 two where the rows are long (M = 2048, K = 12288: INT4
+        // 18.7 us, with one 19.6; NVFP4 17.6 and 21.7).  From 16 rows per compute unit on the forms below are
         // faster (M = 4096: 11.5 us against 13.0).
         if (p.M_pad <= 8 * ncu) {
             QuantParams q = p;
             const int row_blocks = p.M_pad / 16, most = (p.K / 128 + 7) / 8;
             const bool one = row_blocks * (RT + 1) <= ncu;
             q.splits = ncu / row_blocks - (one ? RT : (RT + 1) / 2);
-            const int least = RT <= 2 ? 1 : 2 * ncu / row_blocks - (RT + 1) / 2 == 2 ? 2 : 3;
+            const int least = RT <= 2 ? (RT == 1 && p.K > 9216 ? 2 : 1) : 2 * ncu / row_blocks - (RT + 1) / 2 == 2 ? 2 : 3;
             if (q.splits < least) q.splits = least;
             if (q.splits > most) q.splits = most;
             return one ? launch_few_rows<1, FP4>(q, stream) : launch_few_rows<2, FP4>(q, stream);

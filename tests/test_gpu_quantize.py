@@ -260,7 +260,7 @@ def _check_row_sample(dev, M, K, R, fp4, smooth):
 
 @pytest.mark.parametrize("M,K,R,fp4,smooth", [(1, 128, 16, False, True), (250, 1152, 48, False, True), (33, 3200, 0, False, False), (600, 2176, 80, True, True),
                                               (257, 9216, 32, True, False), (700, 512, 272, False, True), (2048, 1152, 32, False, True), (2000, 384, 144, True, True),
-                                              (1800, 3200, 64, False, True)])
+                                              (1800, 3200, 64, False, True), (1537, 9344, 16, True, True)])
 def test_few_rows_split_into_quantizing_and_projecting_workgroups(dev, M, K, R, fp4, smooth):
     """Up to 8 rows per compute unit: one chunk, fewer chunks than waves, counts of chunks that neither the shares nor the
     projection's ring divide; one rank tile per projecting workgroup and two, with a rank tile left over (ranks 48, 80, 144,
