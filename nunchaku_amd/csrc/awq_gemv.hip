@@ -267,9 +267,13 @@ extern "C" int svdq_awq_gemv_w4a16(const svdq_awq_gemv_args *a, void *stream) {
     AwqParams p{(const uint16_t *)a->x, (const uint8_t *)a->qweight, (const uint16_t *)a->scales, (const uint16_t *)a->zeros,
                 (const uint16_t *)a->bias, (uint16_t *)a->out, (int)a->M, (int)a->N, (int)a->K};
     hipStream_t st = (hipStream_t)stream;
+    // Short rows (up to 4 steps of K) and more than 16384 channels: half of the eight waves have nothing to multiply, and many
+    // workgroups of four waves are faster than few with several tiles one after the other (N = 21504, eight rows: K = 256 5.3 us against
+    // 6.0, K = 384 5.6 against 6.0; K = 640 6.9 against 6.2, and the same on either side at N = 12288).
     // (byte offsets of a lane's scales are 32 bits wide)
     const int64_t steps = (a->K + 127) / 128;
-    if (a->N >= 16 && steps <= 4 * WAVES && a->K / 64 * a->N < (1ll << 30)) {
+    const bool rows = a->N >= 16 && steps <= 4 * WAVES && (steps > 4 || a->N <= 16384);
+    if (rows && a->K / 64 * a->N < (1ll << 30)) {
         if (steps <= WAVES) return launch_rows<1>(p, st);
         if (steps <= 2 * WAVES) return launch_rows<2>(p, st);
         if (steps <= 3 * WAVES) return launch_rows<3>(p, st);

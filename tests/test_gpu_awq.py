@@ -52,13 +52,27 @@ def test_against_oracle(dev, rows, oc, ic):
 @pytest.mark.parametrize("oc,ic", [(16, 64), (20, 128), (12, 192), (100, 2112), (52, 4096), (28676, 128)])
 def test_edges_of_the_tile_walk(dev, rows, oc, ic):
     """A last tile that begins early (oc not a multiple of 16), fewer channels than a tile, one to four steps of K per wave
-    with and without a remainder, and more tiles per workgroup than meet at once."""
+    with and without a remainder, and many channels with short rows (a workgroup per tile)."""
     announce(f"awq gemv rows={rows} oc={oc} ic={ic}")
     m, (codes, scales, zeros, bias) = _module(dev, oc, ic, seed=oc + ic)
     x = torch.randn(rows, ic, generator=torch.Generator().manual_seed(rows)).to(torch.bfloat16)
     y = m(x.to(dev))
     torch.cuda.synchronize()
     _check(y, awq.gemv(x, codes, scales, zeros), bias)
+
+
+@pytest.mark.parametrize("rows", [1, 5, 8])
+@pytest.mark.parametrize("oc,ic", [(28676, 640), (16384, 512), (16388, 512)])
+def test_many_channels(dev, rows, oc, ic):
+    """More tiles per workgroup than meet at once, and either side of the line behind which short rows have a workgroup per tile.
+    Bound: one rounding to bf16, and fp32 sums of ic terms."""
+    announce(f"awq gemv rows={rows} oc={oc} ic={ic} (many channels)")
+    m, (codes, scales, zeros, _) = _module(dev, oc, ic, seed=oc + ic, bias=False)
+    x = torch.randn(rows, ic, generator=torch.Generator().manual_seed(rows)).to(torch.bfloat16)
+    y = m(x.to(dev)).double().cpu()
+    w = awq.dequant(codes, scales, zeros).double()
+    want = x.double() @ w.T
+    assert ((y - want).abs() <= 2.0**-8 * want.abs() + ic * 2.0**-24 * (x.double().abs() @ w.abs().T)).all()
 
 
 def test_long_k_takes_the_path_without_lds_staging(dev):
