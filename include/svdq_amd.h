@@ -122,7 +122,8 @@ int svdq_quantize_w4a4_act_fuse_lora(const svdq_quantize_args *args, void *strea
  *   layer] -> store bf16 `out` and/or shift + smooth + quantize for the next layer (`qout`).
  * The GELU is applied exactly when `qout` is given (launch_impl.cuh:282-309).
  *
- * INT4 runs on the fp6 matrix instruction (one workgroup per 128 x 256 output tile); NVFP4 runs on the
+ * INT4 runs on the fp6 matrix instruction (one workgroup per 128 x 256 output tile, the last rows of many
+ * launches in tiles of 64 x 256); NVFP4 runs on the
  * fp16 matrix instruction with dequantized operands (persistent workgroups, 256 x 256 tiles).  Launches with few
  * rows take a kernel with tiles of 32 or 64 rows x 128 columns of either precision (unless k_split is given).
  *
@@ -131,10 +132,11 @@ int svdq_quantize_w4a4_act_fuse_lora(const svdq_quantize_args *args, void *strea
  *   - INT4 with so few output tiles that they are split along K (no more tiles than compute units and a long
  *     enough K, or k_split > 1): 128 KB of fp32 partial sums per tile and part, at most 64 MB by the library's
  *     own choice;
- *   - next_lora_down: 4 bytes per element of next_lora_act_out and 256-column block of N (128 for NVFP4) (every
- *     block leaves its share there and a small kernel launched behind the GEMM adds the shares in ascending
+ *   - next_lora_down: 4 bytes per element of next_lora_act_out and 256-column block of N, or 128-column block
+ *     (NVFP4, and the kernel for few rows in either precision) (every block leaves its share there and a small kernel launched behind the GEMM adds the shares in ascending
  *     order, so the result does not depend on the order in which the blocks finish);
- *   - out_vk: 4224 bytes per head and 128 rows (NVFP4: 32 rows);
+ *   - out_vk: 4224 bytes per head and row block: 32 rows (NVFP4, and the kernel for few rows), otherwise 128, or 64
+ *     for the last rows;
  *   - NVFP4 whenever the number of 256 x 256 tiles is not a multiple of the number of compute units:
  *     512 KB per compute unit.
  * A block that a launch has used is never freed or moved by a later call: a HIP graph that captured a call keeps

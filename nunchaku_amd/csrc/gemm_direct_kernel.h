@@ -7,9 +7,13 @@
 // of their part of K in turn, and the parts' sums meet in LDS at the end.  An operand fragment is contiguous in memory in
 // the lanes' order (svdq_common.h), so a wave fetches it with one or two wide loads, DEPTH of its k-groups ahead, and
 // neither LDS nor barriers appear in the main loop.
-// Bound by the bytes the L2s hand out: 2.15 KB per 32 x 32 tile and k-group with one row block and four column tiles per
-// wave, 1.65 KB with two of each; at 192 workgroups (M = 256, N = 3072) they arrive at 82 GB/s per compute unit, 15.7 TB/s
-// in all.  M = 256, K = N = 3072: 22.8 -> 9.6 us (INT4; 4.7 us of it do not depend on K), 59.9 -> 11.2 us (NVFP4).
+// What bounds it: with one workgroup per compute unit, no single resource.  M = 256, K = N = 3072 (192 workgroups): a wave takes 0.41 us
+// per k-group, about one memory latency, with one k-group on its way (INT4, 32 rows; two in NVFP4); of the waves' cycles 27 % are
+// waits for operands, 29 % waits to issue behind the matrix core, 28 % vector instructions (NVFP4, M = 300: 33, 13 and 41 %).  84 % of
+// the operand requests hit in the L2s, which hand out 2.15 KB per 32 x 32 tile and k-group with one row block and four column tiles
+// per wave, 1.65 KB with two of each (82 GB/s per compute unit, 64 bytes per clock being about 150).  With several tiles per compute
+// unit the matrix core and the conversions are (M = 1157, K = 12288, NVFP4: 10 % waits for operands, 49 and 34 % the others).
+// M = 256, K = N = 3072: 22.8 -> 9.6 us (INT4; 4.7 us of it do not depend on K), 59.9 -> 11.2 us (NVFP4).
 //
 // INT4: one fp6 matrix instruction on the codes, one factor instruction and 16 multiply-adds per 32 x 32 tile and
 // k-group (gemm6_kernel.h).  NVFP4: both operands are dequantized to fp16 in registers by the wave that uses them
