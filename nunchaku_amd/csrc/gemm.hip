@@ -608,8 +608,8 @@ int gemm_fp4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t st
 // K.  Shape 2: tiles of 64 rows, a quarter fewer operand bytes per product, from about 400 tiles of 32 rows on; INT4: two waves
 // split K and two the columns, NVFP4: four waves split K.  Models of the time in us fitted to launches at K = 1024 ... 12288
 // on 256 compute units, linear in the number of tiles that the busiest compute unit works through and in the k-groups; they meet
-// the measurements within about 10 %.  Over 2200 random shapes the choice takes 0.5 % (NVFP4) and 0.3 % (INT4) longer than the fastest
-// of the three, and is more than 3 % slower than the large tiles in three.  Measured at K = 3072, large tiles (split along K where that pays) / shape 1 / shape 2:
+// the measurements within about 10 %.  Over 2200 random shapes the choice takes 0.6 % (NVFP4) and 0.3 % (INT4) longer than the fastest
+// of the three, and is more than 3 % slower than the large tiles in 17, 14 of them short rows whose large tiles would be shared (below).  Measured at K = 3072, large tiles (split along K where that pays) / shape 1 / shape 2:
 //   INT4   M = 256, N = 3072   22.8 /  9.6 / 12.3     NVFP4  60.7 / 11.8 / 13.8
 //          M = 505, N = 9216   28.7 / 33.1 / 30.6            62.9 / 38.4 / 34.1
 //          M = 1157, N = 3072  29.7 / 27.6 / 21.8            62.1 / 31.7 / 25.7
@@ -636,10 +636,12 @@ int choose_direct(const svdq_gemm_args *a, int ncu) {
         t_large = one * rounds + (tiles > 1.0 && !nwg ? 33.0 : 0.0);
         t1 = 4.3 + c1 * (1.1 + 0.127 * kg);
         t2 = 5.0 + c2 * (1.6 + 0.205 * kg) - (c2 < 3.0 ? 0.04 * kg : 0.0);
-        // Short rows and many rounds: the outputs set the pace of both kernels, and the large tiles write them faster (M = 4608, K = 384,
-        // N = 9088 69 us in shape 2 against 63; M = 6400, K = 640, N = 16384 210 against 181; M = 11008, K = 1024, N = 8576 242 against 229; of
-        // 1572 random shapes 22 were slower by more than 3 % in the kernel chosen, with this term two).
-        if (kg <= 16 && c2 > 12.0) t2 += 0.9 * (c2 - 12.0);
+        // Short rows and many rounds without the quantizing epilogue: the outputs set the pace, and whole large tiles write them faster (M =
+        // 4608, K = 384, N = 9088 69 us in shape 2 against 63; N = 19200 138 against 121; M = 4096, K = 384, N = 14592 with norm and rotary 117
+        // against 110; of 500 random shapes of 257 large tiles and more 14 take them by this term, 1.12 times as fast, none slower).  Not
+        // where the large tiles would be shared, up to 17 % faster still at such sizes (M = 6400, K = 640, N = 16384 210 against 181): those
+        // need 128 MB of workspace, more than the fixed scratch has, and a call gives the same bits with either.
+        if (nwg > 0 && kg <= 12 && c2 > 12.0 && !a->qout) t2 += 0.9 * (c2 - 12.0);
         if (a->qout) {  // (the quantizing epilogue: M = 4608, K = 3072, N = 12288 298 -> 387 us in large tiles, 317 -> 358 in shape 2)
             t_large += 20.0 * rounds;
             t1 += 1.1 * c1;
