@@ -63,8 +63,8 @@ def test_rows_of_a_call_without_out():
     ("plain", 4096, 3072, 9216, False, dict(full_blocks=32)), ("rope", 4096, 6144, 9216, False, dict(full_blocks=32)), ("plain", 2048, 3072, 18432, False, dict(full_blocks=16)),
     ("plain", 300, 3072, 3072, True, dict(few_rows=1)), ("plain", 1157, 12288, 3072, True, dict(few_rows=2)), ("plain", 4608, 3072, 21504, True, dict(workgroups=252)),
     ("plain", 4608, 15360, 3072, True, dict(workgroups=216)), ("plain", 4608, 3072, 4608, True, dict(workgroups=256, shared_tiles=1)),
-    ("plain", 4608, 384, 9088, True, dict(workgroups=216)), # (short rows: whole large tiles, but not shared ones, whose workspace the fixed scratch has not)
-    ("plain", 6400, 640, 16384, True, dict(few_rows=2)),
+    # (short rows: whole large tiles, but not shared ones, whose workspace the fixed scratch has not)
+    ("plain", 4608, 384, 9088, True, dict(workgroups=216)), ("plain", 6400, 640, 16384, True, dict(few_rows=2)),
     ("plain", 11008, 1024, 8576, True, dict(few_rows=2)), ("rope", 4096, 384, 14592, True, dict(workgroups=228)), ("next", 4096, 3072, 6144, True, dict(few_rows=2)),
     ("next", 2304, 256, 7680, True, dict(few_rows=2)), ("next", 4608, 4096, 4608, True, dict(workgroups=256, shared_tiles=1)),
 ])
