@@ -380,6 +380,36 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
     // per-column factor (alpha and wcscales; EpilogueBias, gemm_base.cuh:710-781) and bias of the
     // workgroup's 256 columns
     float *coltab = (float *)(lds + EP_TAB);
+    const bool down_in_lds = NEXT && p.next_down && p.R_down <= 32;
+    // Operands of the low-rank up projection: 32 ranks at a time of the tile's rows (fp32, 128 bytes of a row of lora_act)
+    // and columns (bf16, 64 bytes of a row of lora_up) go to LDS by asynchronous copies, once for the whole workgroup, the
+    // next chunk's while one is multiplied.  A copy takes whole 64- or 128-byte pieces of rows; which 16 bytes of its row
+    // a lane fetches is permuted so that the operands' reads (32 rows, the same 16 bytes of each) hit all banks.
+    // What this bounds: read by every wave for itself, 32 bytes of each of 32 rows at a time, the operands cost the vector
+    // memory unit of a compute unit 10 k cycles per tile at rank 128, now 2 k.  M = 18432, K = 3072, N = 12288, rank 128: 740 -> 681 us
+    // (without a low-rank branch 621), M = 4608: rank 64 172 -> 167, rank 32 164 -> 161, rank 16 159 -> 160; with the next layer's
+    // epilogue, M = 1157, N = 9216, rank 128: 68.6 -> 60.5.  Same products, same order: same bits.
+    const int nsteps = p.R_up / 16, nchunks = (nsteps + 1) / 2;
+    constexpr int LR_COPIES = 4 + 2 * MT;  // requests of a wave per chunk
+    auto request_chunk = [&](int c) {
+        const uint32_t buf = lds_base + (c & 1 ? LR_BUF1 : LR_BUF0);
+        const bool half = nsteps - 2 * c < 2;  // 16 ranks only: the other half of the places is filled with anything
+        const uint8_t *up = (const uint8_t *)p.lora_up + (size_t)n0 * p.R_up * 2 + c * 64, *la = (const uint8_t *)p.lora_act + (size_t)m0 * p.R_up * 4 + c * 128;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int row = (wave * 4 + i) * 16 + (lane >> 2), piece = (lane & 3) ^ lr_up_swizzle(row);
+            const int valid = n0 + row < p.N ? row : p.N - 1 - n0;  // (columns beyond N are computed and never used)
+            const uint32_t voff = (uint32_t)valid * (uint32_t)(p.R_up * 2) + (half ? piece & 1 : piece) * 16;
+            asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3" :: "s"(buf), "s"((wave * 4 + i) * 1024), "v"(voff), "s"(up) : "memory", "m0", "scc");
+        }
+#pragma unroll
+        for (int i = 0; i < 2 * MT; i++) {
+            const int row = (wave * 2 * MT + i) * 8 + (lane >> 3), piece = (lane & 7) ^ lr_act_swizzle(row);
+            const uint32_t voff = (uint32_t)row * (uint32_t)(p.R_up * 4) + (half ? piece & 3 : piece) * 16;
+            asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3" :: "s"(buf), "s"(LR_ACT + (wave * 2 * MT + i) * 1024), "v"(voff), "s"(la) : "memory", "m0", "scc");
+        }
+    };
+    if (nchunks > 0) request_chunk(0);
     const bool has_cf = p.alpha != 1.0f || p.wcscales != nullptr;
     {
         const int n = n0 + tid;
@@ -388,21 +418,17 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
         if (ok && p.wcscales) cf *= bf16_bits_to_f32(p.wcscales[n]);
         coltab[tid] = cf;
         coltab[256 + tid] = (ok && p.bias) ? bf16_bits_to_f32(p.bias[n]) : 0.f;
-        if (NEXT && p.next_down && p.R_down <= 32) {
-            // the next layer's proj_down for the tile's 256 columns (two 128-chunks, 4 KB per rank tile each,
-            // contiguous in memory) goes to LDS once: both row halves and both slabs read it from there
-            const int npieces = 8 * (p.R_down / 16);
-            for (int pc = wave; pc < npieces; pc += 4) {
-                if (n0 + (pc / (npieces / 2)) * 128 < p.N)
-                    *(u32x4_t *)(lds + EP_DOWN + pc * 1024 + lane * 16) =
-                        *(const u32x4_t *)((const uint8_t *)p.next_down + ((size_t)(n0 / 128) * (npieces / 2) + pc) * 1024 + lane * 16);
-            }
-        }
         if (NEXT && p.rotary && tid < 128) {
             // RMS-norm weights of the heads the two column halves are (q below N/3, k below 2N/3)
             ((float *)(lds + EP_NORMW))[tid] = bf16_bits_to_f32((n0 < p.rope_cols / 2 ? p.norm_q : p.norm_k)[tid]);
             ((float *)(lds + EP_NORMW))[128 + tid] = bf16_bits_to_f32((n0 + 128 < p.rope_cols / 2 ? p.norm_q : p.norm_k)[tid]);
         }
+    }
+    if (nchunks > 1) {
+        request_chunk(1);
+        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(LR_COPIES) : "memory");
+    } else {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     __syncthreads();
     const float *cfw = coltab + wn * 128, *bsw = coltab + 256 + wn * 128;
@@ -418,37 +444,27 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
                     for (int i = 0; i < 4; i++) acc[MT * nt + mt][4 * q + i] *= cf[i];
             }
     }
-    // Low-rank up projection (lora.cuh:110-241): out += bf16(lora_act * scale) @ up^T on the matrix
-    // cores, straight into the accumulators.  Two 16-rank steps per round; every request of a round is
-    // issued before any of its data is touched, so a round costs one memory latency.
-    const int nsteps = p.R_up / 16;
-    for (int s0 = 0; s0 < nsteps; s0 += 2) {
-        const bool two = s0 + 1 < nsteps;
-        const int s1 = two ? s0 + 1 : s0;
-        float4_t ra[MT][2][2];
-        u32x4_t rb[4][2];
-#pragma unroll
-        for (int t = 0; t < MT; t++) {
-            const float4_t *ap = (const float4_t *)(p.lora_act + (size_t)(wrow0 + t * 32 + r32) * p.R_up + 8 * h);
-            ra[t][0][0] = ap[4 * s0]; ra[t][0][1] = ap[4 * s0 + 1];
-            ra[t][1][0] = ap[4 * s1]; ra[t][1][1] = ap[4 * s1 + 1];
+    // Low-rank up projection (lora.cuh:110-241): out += bf16(lora_act * scale) @ up^T on the matrix cores, straight into
+    // the accumulators, chunk by chunk of 32 ranks.
+    for (int c = 0; c < nchunks; c++) {
+        if (c > 0) {
+            if (c + 1 < nchunks) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(LR_COPIES) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
         }
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const int n = wcol0 + t * 32 + r32;
-            const u32x4_t *bp = (const u32x4_t *)(p.lora_up + (size_t)(n < p.N ? n : 0) * p.R_up + 8 * h);
-            rb[t][0] = bp[2 * s0];
-            rb[t][1] = bp[2 * s1];
-            if (n >= p.N) rb[t][0] = rb[t][1] = u32x4_t{0, 0, 0, 0};
-        }
+        const uint8_t *buf = lds + (c & 1 ? LR_BUF1 : LR_BUF0);
+        const bool two = nsteps - 2 * c > 1;
 #pragma unroll
         for (int k = 0; k < 2; k++) {
             if (k == 1 && !two) break;
-            const float ls = p.lora_scales[s0 + k];
+            const float ls = p.lora_scales[2 * c + k];
             bf16x8_t la[MT];
 #pragma unroll
             for (int t = 0; t < MT; t++) {
-                const float4_t v0 = ra[t][k][0], v1 = ra[t][k][1];
+                const int row = (wm * MT + t) * 32 + r32;
+                const uint8_t *ap = buf + LR_ACT + row * 128;
+                const float4_t v0 = *(const float4_t *)(ap + (((4 * k + 2 * h) ^ lr_act_swizzle(row)) << 4));
+                const float4_t v1 = *(const float4_t *)(ap + (((4 * k + 2 * h + 1) ^ lr_act_swizzle(row)) << 4));
                 u32x4_t w;
                 w[0] = pack_bf16x2(v0[0] * ls, v0[1] * ls);
                 w[1] = pack_bf16x2(v0[2] * ls, v0[3] * ls);
@@ -457,11 +473,29 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
                 la[t] = __builtin_bit_cast(bf16x8_t, w);
             }
 #pragma unroll
-            for (int nt = 0; nt < 4; nt++)
+            for (int nt = 0; nt < 4; nt++) {
+                const int col = wn * 128 + nt * 32 + r32;
+                const bf16x8_t up = *(const bf16x8_t *)(buf + col * 64 + (((2 * k + h) ^ lr_up_swizzle(col)) << 4));
 #pragma unroll
-                for (int mt = 0; mt < MT; mt++)
-                    acc[MT * nt + mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, rb[nt][k]), la[mt], acc[MT * nt + mt], 0, 0, 0);
+                for (int mt = 0; mt < MT; mt++) acc[MT * nt + mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(up, la[mt], acc[MT * nt + mt], 0, 0, 0);
+            }
         }
+        if (c + 2 < nchunks) {
+            __syncthreads();  // everybody has read the buffer
+            request_chunk(c + 2);
+        }
+    }
+    if (nchunks > 0) __syncthreads();  // the slabs and the next layer's operands take the buffers' place
+    if (NEXT && down_in_lds) {
+        // the next layer's proj_down for the tile's 256 columns (two 128-chunks, 4 KB per rank tile each,
+        // contiguous in memory) goes to LDS once: both row halves and both slabs read it from there
+        const int npieces = 8 * (p.R_down / 16);
+        for (int pc = wave; pc < npieces; pc += 4) {
+            if (n0 + (pc / (npieces / 2)) * 128 < p.N)
+                *(u32x4_t *)(lds + EP_DOWN + pc * 1024 + lane * 16) =
+                    *(const u32x4_t *)((const uint8_t *)p.next_down + ((size_t)(n0 / 128) * (npieces / 2) + pc) * 1024 + lane * 16);
+        }
+        __syncthreads();
     }
 
     // reciprocal smoothing factors of the next layer for the 32 columns this lane quantizes
@@ -475,7 +509,6 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
             nrs[4 * i] = v4[0]; nrs[4 * i + 1] = v4[1]; nrs[4 * i + 2] = v4[2]; nrs[4 * i + 3] = v4[3];
         }
     }
-    const bool down_in_lds = NEXT && p.next_down && p.R_down <= 32;
     const bool interior = m0 + TILE_M <= p.M_out && n0 + BN <= p.N_out;  // the whole tile lies inside the output
     uint16_t *slab = (uint16_t *)(lds + wave * SLAB_BYTES);
     const int ngroups_out = p.N / 64;

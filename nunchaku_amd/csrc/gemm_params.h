@@ -218,7 +218,17 @@ constexpr int EP_RED = EP_FLAG + 16;       // [2 rank tiles][2 row halves][2][64
 constexpr int EP_RED_BYTES = 2 * 2 * 2 * 64 * 16;  // two rank tiles at a time
 constexpr int EP_DOWN = EP_RED + EP_RED_BYTES;  // the next layer's proj_down for the tile's 256 columns, up to 2 rank tiles
 constexpr int EP_END = EP_DOWN + 16384;
-constexpr int LDS_BYTES = STAGES * STAGE_BYTES > EP_END ? STAGES * STAGE_BYTES : EP_END;
+// Before the slabs and the low-rank sums: two chunks of 32 ranks of the low-rank up projection's operands, each
+// [256 columns][4 pieces of 16 bytes of lora_up], then [128 rows][8 pieces of 16 bytes of lora_act].  Piece q of a row stands at
+// place q ^ swizzle(row): a 16-byte read is served 16 lanes at a time in the order lanes 0-3, 12-15, 20-27, then 4-11, 16-19,
+// 28-31, and these 16 rows of 64 (128) bytes then fall on 16 different places of 16 bytes.
+constexpr int LR_ACT = 256 * 64, LR_BYTES = LR_ACT + 128 * 128;
+constexpr int LR_BUF0 = 0, LR_BUF1 = EP_RED;
+static_assert(LR_BUF0 + LR_BYTES <= EP_TAB, "the first chunk lies in the slabs' place");
+__host__ __device__ constexpr int lr_up_swizzle(int row) { return (row >> 2) & 3; }
+__host__ __device__ constexpr int lr_act_swizzle(int row) { return (row >> 1) & 7; }
+constexpr int EP_BYTES = LR_BUF1 + LR_BYTES > EP_END ? LR_BUF1 + LR_BYTES : EP_END;
+constexpr int LDS_BYTES = STAGES * STAGE_BYTES > EP_BYTES ? STAGES * STAGE_BYTES : EP_BYTES;
 static_assert(2 * LDS_BYTES <= 160 * 1024, "two workgroups share a compute unit's LDS");
 
 // Which tile a workgroup takes: row blocks [0, full_blocks) are 128 rows high, the half_blocks behind them 64 (or, with
