@@ -253,11 +253,7 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
         }
     };
     float cf[4][4], bs[4][4];  // factor and bias of the lane's columns c0 + 8 q + 4 h + i
-    float rcf = 1.f;           // NVFP4: reciprocal factor of column c0 + r32, see below
-    if (nsteps > 0) {
-        load_lora(0);
-        if (FP4) rcf = __fdiv_rn(1.0f, p.colnorm[c0 + r32] * p.alpha * (p.wcscales ? bf16_bits_to_f32(p.wcscales[c0 + r32]) : 1.f));
-    }
+    if (nsteps > 0) load_lora(0);
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         const int c = c0 + 8 * q + 4 * h;
@@ -297,30 +293,17 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
 
     float *ssq = (float *)(lds + KP * 16384);  // [MT][4 column tiles][32 rows]
     const bool rope = NEXT && p.rotary && n0 < p.rope_cols;  // the tile is one head of q or k
-    if (!FP4) {
 #pragma unroll
-        for (int o = 0; o < MT; o++)
+    for (int o = 0; o < MT; o++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) val[o][e] *= cf[e >> 2][e & 3];
-    }
-    // Low-rank up projection (lora.cuh:110-241): out += bf16(lora_act * scale) @ up^T.  NVFP4: in units of the column factor
-    // and with the quotient up / factor as the sum of two bf16 numbers, as in gemm_kernel.h, so that a row gives the same
-    // values whichever kernel its batch takes (they differ in the order of the fp32 sums only).
+        for (int e = 0; e < 16; e++) val[o][e] *= cf[e >> 2][e & 3];
+    // Low-rank up projection (lora.cuh:110-241): out += bf16(lora_act * scale) @ up^T
     for (int s0 = 0; s0 < nsteps; s0 += LSTEPS) {
         if (s0 > 0) load_lora(s0);
 #pragma unroll
         for (int s = 0; s < LSTEPS; s++) {
             if (s0 + s >= nsteps) break;
             const float ls = p.lora_scales[s0 + s];
-            u32x4_t up = up_raw[s], up_rem = u32x4_t{0, 0, 0, 0};
-            if (FP4) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float q0 = bits_f32(up[i] << 16) * rcf, q1 = bits_f32(up[i] & 0xFFFF0000u) * rcf;
-                    up[i] = pack_bf16x2(q0, q1);
-                    up_rem[i] = pack_bf16x2(q0 - bits_f32(up[i] << 16), q1 - bits_f32(up[i] & 0xFFFF0000u));
-                }
-            }
 #pragma unroll
             for (int o = 0; o < MT; o++) {
                 const float4_t v0 = la_raw[o][s][0], v1 = la_raw[o][s][1];
@@ -329,15 +312,14 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
                 w[1] = pack_bf16x2(v0[2] * ls, v0[3] * ls);
                 w[2] = pack_bf16x2(v1[0] * ls, v1[1] * ls);
                 w[3] = pack_bf16x2(v1[2] * ls, v1[3] * ls);
-                val[o] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, up), __builtin_bit_cast(bf16x8_t, w), val[o], 0, 0, 0);
-                if (FP4) val[o] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, up_rem), __builtin_bit_cast(bf16x8_t, w), val[o], 0, 0, 0);
+                val[o] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, up_raw[s]), __builtin_bit_cast(bf16x8_t, w), val[o], 0, 0, 0);
             }
         }
     }
 #pragma unroll
     for (int o = 0; o < MT; o++)
 #pragma unroll
-        for (int e = 0; e < 16; e++) val[o][e] = FP4 ? __builtin_fmaf(val[o][e], cf[e >> 2][e & 3], bs[e >> 2][e & 3]) : val[o][e] + bs[e >> 2][e & 3];
+        for (int e = 0; e < 16; e++) val[o][e] += bs[e >> 2][e & 3];
     if (rope) {
 #pragma unroll
         for (int o = 0; o < MT; o++) {

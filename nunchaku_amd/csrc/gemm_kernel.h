@@ -437,73 +437,88 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
                 ((float *)(lds + NORMW_OFF + wave * 512))[2 * lane + j] = bf16_bits_to_f32((wcol0 < p.rope_cols / 2 ? p.norm_q : p.norm_k)[2 * lane + j]);
         }
     }
-    // Low-rank up projection (lora.cuh:110-241): out += bf16(lora_act * scale) @ up^T on the matrix cores.
-    // The projection is added to the accumulators BEFORE they are scaled.  The accumulators are in
-    // normalised units (out = acc * cf[col] + bias), so the second operand is divided by cf first; the
-    // matrix cores then update the accumulators in place and the operands are dead before the output pass
-    // starts.  cf (column normalisation x alpha x wcscales) is an arbitrary number, so up / cf is passed as the sum of
-    // two bf16 numbers (the rounded quotient and the rounded remainder: relative error 2^-17, below the
-    // rounding noise of the main loop) in two matrix-core steps; wcscales must not be zero.
+    // Low-rank up projection (lora.cuh:110-241): out += bf16(lora_act * scale) @ up^T on the matrix cores.  The operands of up to
+    // 128 ranks go to LDS once for the workgroup, read in whole pieces of rows and written in the matrix instruction's order
+    // (gemm_params.h), and every slab adds the product to its 64 outputs per lane once these are scaled.
+    // Ranks from 128 on, whose operands do not fit beside those, are added to the accumulators before the slabs.  The
+    // accumulators are in normalised units (out = acc * cf[col] + bias), so there the second operand is divided by cf.  cf
+    // (column normalisation x alpha x wcscales) is an arbitrary number: up / cf is passed as the sum of two bf16 numbers
+    // (the rounded quotient and the rounded remainder: relative error 2^-17, below the rounding noise of the main loop) in two
+    // matrix-core steps; wcscales must not be zero.
+    // Before, all ranks went that way, with operands that every wave read for itself, 32 bytes of each of 32 rows at a time.  K = 3072,
+    // before / now / without a low-rank branch: M = 4608, N = 21504, rank 32 490 / 480 / 461 us; M = 4608, N = 12288, rank 16 291 / 290,
+    // rank 64 319 / 300, rank 256 453 / 361; M = 18432, N = 12288, rank 128 1432 / 1231.  What is left is one latency of the requests per tile, the
+    // writes to LDS and the matrix instructions, half as many as before.
     const int nsteps = p.R_up / 16;
     if (run_epilogue && nsteps > 0) {
-        {
-            // two 16-rank steps per round; every request of a round is issued before any of its data is
-            // touched, so a round costs one memory latency
-            for (int s0 = 0; s0 < nsteps; s0 += 2) {
-                const bool two = s0 + 1 < nsteps;
-                const int s1 = two ? s0 + 1 : s0;
-                float4_t ra[4][2][2];
-                u32x4_t rb[4][2];
-                float rcf[4];
+        for (int w = (nsteps - 1) / LR_STEPS; w >= 0; w--) {
+            const int first = w * LR_STEPS, steps = nsteps - first < LR_STEPS ? nsteps - first : LR_STEPS;
+            // 32 ranks at a time: a thread's share of the 256 rows of lora_act (eight lanes per row) and columns of lora_up (four)
+            float4_t la[8];
+            u32x4_t up[4];
+            auto request = [&](int c) {
+                const int step = first + 2 * c + ((lane & 4) && 2 * c + 1 < steps ? 1 : 0), up_step = first + 2 * c + ((lane & 2) && 2 * c + 1 < steps ? 1 : 0);
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+                    la[i] = *(const float4_t *)(p.lora_act + (size_t)(m0 + i * 32 + wave * 8 + (lane >> 3)) * p.R_up + 16 * step + (lane & 3) * 4);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int n = n0 + i * 64 + wave * 16 + (lane >> 2);
+                    up[i] = *(const u32x4_t *)(p.lora_up + (size_t)(n < p.N ? n : p.N - 1) * p.R_up + 16 * up_step + (lane & 1) * 8);  // (columns beyond N are computed and never used)
+                }
+            };
+            request(0);
+            if (w < (nsteps - 1) / LR_STEPS) __syncthreads();  // the window before has been multiplied
+            for (int c = 0; 2 * c < steps; c++) {
+                const int step = 2 * c + ((lane & 4) >> 2), up_step = 2 * c + ((lane & 2) >> 1);
+                const float ls = p.lora_scales[first + (step < steps ? step : 2 * c)];
+                if (step < steps) {
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        const int row = wave * 8 + (lane >> 3);  // of 32-row block i
+                        u32x2_t b;
+                        b[0] = pack_bf16x2(la[i][0] * ls, la[i][1] * ls);
+                        b[1] = pack_bf16x2(la[i][2] * ls, la[i][3] * ls);
+                        *(u32x2_t *)(lds + lr_act_block(i >> 2, i & 3) + step * 1024 + (((lane & 2) << 4) + row) * 16 + (lane & 1) * 8) = b;
+                    }
+                }
+                if (up_step < steps) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const int col = i * 64 + wave * 16 + (lane >> 2);
+                        *(u32x4_t *)(lds + LR_UP + (col >> 5) * LR_BLOCK + up_step * 1024 + (((lane & 1) << 5) + (col & 31)) * 16) = up[i];
+                    }
+                }
+                if (2 * c + 2 < steps) request(c + 1);
+            }
+            __syncthreads();
+            if (w == 0) break;
+            float rcf[4];
+#pragma unroll
+            for (int nt = 0; nt < 4; nt++) rcf[nt] = wcol0 + nt * 32 < p.N ? __fdiv_rn(1.0f, coltab[nt * 32 + r32]) : 0.f;
+            for (int st = 0; st < steps; st++) {
+                bf16x8_t x[4], q[4], rem[4];
 #pragma unroll
                 for (int t = 0; t < 4; t++) {
-                    const float4_t *ap = (const float4_t *)(p.lora_act + (size_t)(wrow0 + t * 32 + r32) * p.R_up + 8 * h);
-                    ra[t][0][0] = ap[4 * s0]; ra[t][0][1] = ap[4 * s0 + 1];
-                    ra[t][1][0] = ap[4 * s1]; ra[t][1][1] = ap[4 * s1 + 1];
-                    const int n = wcol0 + t * 32 + r32;
-                    const bool ok = n < p.N;
-                    const u32x4_t *bp = (const u32x4_t *)(p.lora_up + (size_t)(ok ? n : 0) * p.R_up + 8 * h);
-                    rb[t][0] = bp[2 * s0];
-                    rb[t][1] = bp[2 * s1];
-                    float cf = ok ? p.colnorm[n] * p.alpha : 1.f;
-                    if (ok && p.wcscales) cf *= bf16_bits_to_f32(p.wcscales[n]);
-                    rcf[t] = ok ? __fdiv_rn(1.0f, cf) : 0.f;
-                }
+                    x[t] = *(const bf16x8_t *)(lds + lr_act_block(wm, t) + st * 1024 + lane * 16);
+                    u32x4_t bw = *(const u32x4_t *)(lds + LR_UP + (wn * 4 + t) * LR_BLOCK + st * 1024 + lane * 16), br;
 #pragma unroll
-                for (int k = 0; k < 2; k++) {
-                    if (k == 1 && !two) break;
-                    const float ls = p.lora_scales[s0 + k];
-                    bf16x8_t la[4], lb[4], lb_rem[4];
-#pragma unroll
-                    for (int t = 0; t < 4; t++) {
-                        const float4_t v0 = ra[t][k][0], v1 = ra[t][k][1];
-                        u32x4_t w;
-                        w[0] = pack_bf16x2(v0[0] * ls, v0[1] * ls);
-                        w[1] = pack_bf16x2(v0[2] * ls, v0[3] * ls);
-                        w[2] = pack_bf16x2(v1[0] * ls, v1[1] * ls);
-                        w[3] = pack_bf16x2(v1[2] * ls, v1[3] * ls);
-                        la[t] = __builtin_bit_cast(bf16x8_t, w);
-                        u32x4_t bw = rb[t][k], br = u32x4_t{0, 0, 0, 0};
-#pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            const float q0 = bits_f32(bw[i] << 16) * rcf[t], q1 = bits_f32(bw[i] & 0xFFFF0000u) * rcf[t];
-                            bw[i] = pack_bf16x2(q0, q1);
-                            br[i] = pack_bf16x2(q0 - bits_f32(bw[i] << 16), q1 - bits_f32(bw[i] & 0xFFFF0000u));
-                        }
-                        lb[t] = __builtin_bit_cast(bf16x8_t, bw);
-                        lb_rem[t] = __builtin_bit_cast(bf16x8_t, br);
+                    for (int i = 0; i < 4; i++) {
+                        const float q0 = bits_f32(bw[i] << 16) * rcf[t], q1 = bits_f32(bw[i] & 0xFFFF0000u) * rcf[t];
+                        bw[i] = pack_bf16x2(q0, q1);
+                        br[i] = pack_bf16x2(q0 - bits_f32(bw[i] << 16), q1 - bits_f32(bw[i] & 0xFFFF0000u));
                     }
-#pragma unroll
-                    for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-                        for (int nt = 0; nt < 4; nt++)
-                            acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lb[nt], la[mt], acc[mt][nt], 0, 0, 0);
-#pragma unroll
-                    for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-                        for (int nt = 0; nt < 4; nt++)
-                            acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lb_rem[nt], la[mt], acc[mt][nt], 0, 0, 0);
+                    q[t] = __builtin_bit_cast(bf16x8_t, bw);
+                    rem[t] = __builtin_bit_cast(bf16x8_t, br);
                 }
+#pragma unroll
+                for (int mt = 0; mt < 4; mt++)
+#pragma unroll
+                    for (int nt = 0; nt < 4; nt++) acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(q[nt], x[mt], acc[mt][nt], 0, 0, 0);
+#pragma unroll
+                for (int mt = 0; mt < 4; mt++)
+#pragma unroll
+                    for (int nt = 0; nt < 4; nt++) acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(rem[nt], x[mt], acc[mt][nt], 0, 0, 0);
             }
         }
     }
@@ -559,7 +574,20 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
                 bs[q] = *(const float4_t *)(coltab + 128 + nt * 32 + 8 * q + 4 * h);
             }
         };
+        // (and so are the low-rank operands of two steps of 16 ranks)
+        const int lr_steps = nsteps < LR_STEPS ? nsteps : LR_STEPS;
+        bf16x8_t lr_x[2], lr_up[2][4];
+        auto read_low_rank = [&](int st) {
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const int at = (st + k < lr_steps ? st + k : st) * 1024 + lane * 16;
+                lr_x[k] = *(const bf16x8_t *)(lds + lr_act_block(wm, mt) + at);
+#pragma unroll
+                for (int nt = 0; nt < 4; nt++) lr_up[k][nt] = *(const bf16x8_t *)(lds + LR_UP + (wn * 4 + nt) * LR_BLOCK + at);
+            }
+        };
         load_cols(0, cfv[0], bsv[0]);
+        if (nsteps > 0) read_low_rank(0);
 #pragma unroll
         for (int nt = 0; nt < 4; nt++) {
             if (nt < 3) load_cols(nt + 1, cfv[(nt + 1) & 1], bsv[(nt + 1) & 1]);
@@ -577,6 +605,18 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
+        }
+        if (nsteps > 0) {
+            for (int st = 0; st < lr_steps; st += 2) {
+                if (st > 0) read_low_rank(st);
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    if (st + k >= lr_steps) break;
+#pragma unroll
+                    for (int nt = 0; nt < 4; nt++) v[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lr_up[k][nt], lr_x[k], v[nt], 0, 0, 0);
+                }
+            }
+            if (mt == 0) __syncthreads();  // the slabs take the place of the operands of the first one
         }
         if (NEXT && p.rotary && wcol0 < p.rope_cols) {
             // EpilogueRMSNormRope (epilogues.cuh:269-425): the wave's 128 columns are one head of q or k.

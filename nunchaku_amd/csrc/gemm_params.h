@@ -19,10 +19,17 @@ constexpr int OPBUF_BYTES = 2 * OP_BYTES;          // activations + weights
 constexpr int OUT_LD = 136;                // bf16 elements per row of the store-staging slab (128 + pad)
 constexpr int SLAB_OFF = 0;                        // 4 waves x (32 rows x OUT_LD bf16): epilogue staging, in the operand buffers' place
 static_assert(4 * 32 * OUT_LD * 2 <= 2 * OPBUF_BYTES, "the epilogue's slabs reuse the operand buffers");
-constexpr int TAB_OFF = 2 * OPBUF_BYTES;                   // 4 waves x float [2][128]: column factors and biases
+// Operands of the low-rank up projection in the epilogue, up to LR_STEPS x 16 ranks: per block of 32 columns (or rows) and 16 ranks 1 KB
+// in the order of v_mfma_f32_32x32x16_bf16.  Those of the rows of the waves' first slabs stand where the slabs will.
+constexpr int LR_STEPS = 8, LR_BLOCK = LR_STEPS * 1024;
+constexpr int LR_UP = 4 * 32 * OUT_LD * 2, LR_ACT = LR_UP + 8 * LR_BLOCK;
+static_assert(2 * LR_BLOCK <= LR_UP, "");
+__host__ __device__ constexpr int lr_act_block(int wm, int slab) { return slab == 0 ? wm * LR_BLOCK : LR_ACT + ((slab - 1) * 2 + wm) * LR_BLOCK; }
+constexpr int TAB_OFF = LR_ACT + 6 * LR_BLOCK;             // 4 waves x float [2][128]: column factors and biases
 constexpr int FLAG_OFF = TAB_OFF + 4 * 1024;               // one word: a thread's reading of an arrival counter, for all
 constexpr int NORMW_OFF = FLAG_OFF + 16;                   // 4 waves x float [128]: RMS-norm weights of the wave's head
 constexpr int LDS_BYTES = NORMW_OFF + 4 * 512;
+static_assert(TAB_OFF >= 2 * OPBUF_BYTES, "the tables lie behind the operand buffers");
 static_assert(LDS_BYTES <= 160 * 1024, "one workgroup per compute unit");
 
 

@@ -166,9 +166,9 @@ def native(t: torch.Tensor | None, kind: str, fp4: bool = False) -> torch.Tensor
 
 
 def require_nonzero(t: torch.Tensor | None, what: str) -> None:
-    """Raise if a native per-channel vector holds a zero.  The NVFP4 GEMM adds the low-rank term in units of
-    the column factor (column normalisation x alpha x wcscales), i.e. divides by it: a zero there would silently
-    drop the term.  Checked once per tensor object (the check reads the tensor back: one synchronisation)."""
+    """Raise if a native per-channel vector holds a zero.  The NVFP4 GEMM with large tiles adds the low-rank term of ranks
+    from 128 on in units of the column factor (column normalisation x alpha x wcscales), i.e. divides by it: a zero there
+    would silently drop the term.  Checked once per tensor object (the check reads the tensor back: one synchronisation)."""
     if t is None or getattr(t, "_svdq_nonzero", False):
         return
     if bool((t == 0).any()):
