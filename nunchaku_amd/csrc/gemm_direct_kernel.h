@@ -441,8 +441,8 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
             for (int j = 0; j < 4; j++) {
                 float lo = bits_f32(v4[j] << 16), hi = bits_f32(v4[j] & 0xFFFF0000u);
                 if (!FP4) {
-                    lo = bf16_bits_to_f32(f32_to_bf16_bits(__fadd_rn(lo, 0.171875f)));
-                    hi = bf16_bits_to_f32(f32_to_bf16_bits(__fadd_rn(hi, 0.171875f)));
+                    lo = round_to_bf16(__fadd_rn(lo, 0.171875f));
+                    hi = round_to_bf16(__fadd_rn(hi, 0.171875f));
                 }
                 y[8 * i + 2 * j] = smooth_quotient(lo, nrs[8 * i + 2 * j]);
                 y[8 * i + 2 * j + 1] = smooth_quotient(hi, nrs[8 * i + 2 * j + 1]);

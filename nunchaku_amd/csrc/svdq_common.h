@@ -101,6 +101,14 @@ __host__ __device__ inline uint32_t f32_to_bf16_bits(float f) {
 #endif
 }
 
+// fp32 rounded to bf16, as fp32: as the upper of a converted pair whose lower half is zero the result is in place, one
+// instruction (converted into a lower half it takes a shift to get there: the quantizing epilogue 361 vector instructions per 32
+// outputs, now 296; INT4, M = 4608, K = 3072, N = 12288 with that epilogue 200.2 -> 198.4 us, M = 500 37.7 -> 37.2)
+__device__ inline float round_to_bf16(float f) {
+    typedef float float2_t __attribute__((ext_vector_type(2)));
+    return bits_f32(__builtin_bit_cast(uint32_t, __builtin_convertvector(float2_t{0.0f, f}, bf16x2_t)));
+}
+
 // two fp32 -> packed bf16 pair (lo in bits [15:0]), round-to-nearest-even: one v_cvt_pk_bf16_f32
 __device__ inline uint32_t pack_bf16x2(float lo, float hi) {
     typedef float float2_t __attribute__((ext_vector_type(2)));

@@ -19,7 +19,7 @@ constexpr float RNE_MAGIC = 12582912.0f;  // 1.5 * 2^23: adding it rounds to an 
 
 __device__ inline float smooth_quotient(float x, float rcp) {
     // bf16(x / smooth) as fp32, see the header comment
-    return bf16_bits_to_f32(f32_to_bf16_bits(__fmul_rn(x, rcp)));
+    return round_to_bf16(__fmul_rn(x, rcp));
 }
 
 // fp32 (finite, >= 0, <= 448) -> e4m3 bit pattern, round to nearest even
