@@ -17,6 +17,8 @@ int launch_fp4_next(const GemmParams &p, int shape, hipStream_t stream);
 namespace g6 {
 int launch_plain(const Params &p, int nwg, hipStream_t stream);
 int launch_next(const Params &p, int nwg, hipStream_t stream);
+int launch_plain_rolled(const Params &p, int nwg, hipStream_t stream);
+int launch_next_rolled(const Params &p, int nwg, hipStream_t stream);
 }  // namespace g6
 }  // namespace svdq
 
@@ -489,13 +491,18 @@ int gemm_int4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t s
     // One workgroup per output tile (or per part of one split along K), two resident per compute unit.
     const int nblocks = (p.N + g6::BN - 1) / g6::BN;
     lay_out_tiles(plan, p);
+    // (see gemm6_kernel's TURNS)
+    const bool rolled = p.half_blocks > 0 && p.full_blocks > 0 && p.full_blocks * nblocks <= compute_units(dev);
+    auto launch = [&](int nwg) {
+        if (needs_next_epilogue(a)) return rolled ? g6::launch_next_rolled(p, nwg, st) : g6::launch_next(p, nwg, st);
+        return rolled ? g6::launch_plain_rolled(p, nwg, st) : g6::launch_plain(p, nwg, st);
+    };
     const int kparts = p.kparts, ntiles = (p.full_blocks + p.half_blocks) * nblocks;
-    const bool next = needs_next_epilogue(a);
     const size_t cnt_bytes = (size_t)ntiles * 4;
     const size_t part_bytes = kparts > 1 ? (size_t)ntiles * kparts * g6::BM * g6::BN * 4 : 0;
     const size_t share_bytes = p.next_down ? lora_share_bytes(a, nblocks) : 0;  // every column block's share of the next projection
     const size_t vk_bytes = p.vk ? vk_share_bytes(a, p.full_blocks + p.half_blocks) : 0;  // every row block's linear-attention sums
-    if (kparts == 1 && !p.next_down && !p.vk) return next ? g6::launch_next(p, ntiles, st) : g6::launch_plain(p, ntiles, st);
+    if (kparts == 1 && !p.next_down && !p.vk) return launch(ntiles);
     std::lock_guard<std::mutex> lock(workspace_mutex(noalloc));
     const size_t cnt_pad = kparts > 1 ? (cnt_bytes + 255) & ~(size_t)255 : 0;
     WorkspaceView w;
@@ -505,7 +512,7 @@ int gemm_int4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t s
     p.partials = (float *)w.scratch;
     p.next_lora_part = (float *)(w.scratch + part_bytes);
     p.vk_part = (float *)(w.scratch + part_bytes + share_bytes);
-    int rc = next ? g6::launch_next(p, ntiles * kparts, st) : g6::launch_plain(p, ntiles * kparts, st);
+    int rc = launch(ntiles * kparts);
     if (rc == SVDQ_OK) rc = add_shares(p, nblocks, g6::BM, p.full_blocks * g6::BM, st);
     if (rc != SVDQ_OK && w.owner) w.owner->dirty = true;
     return rc;

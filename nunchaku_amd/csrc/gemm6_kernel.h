@@ -57,13 +57,13 @@ __device__ inline __amdgpu_buffer_rsrc_t partial_rsrc(const float *slot) {
 // The output tile of 64 MT rows x 256 columns from (m0, 256 nb) on.  MT = 2 is the ordinary tile; MT = 1 (wave tile
 // 32 x 128) serves the last rows of a launch, see gemm6_kernel below.  `tile`, `part`: the tile's number and this workgroup's share
 // of its k-groups where tiles are split along K (MT = 2 only); `vk_slot`: the slot of its linear-attention sums.
-template <bool NEXT, int MT>
+template <bool NEXT, int MT, bool TURNS>
 __device__ __forceinline__ void output_tile(const Params &p, const int m0, const int nb, const int tile, const int part, const int vk_slot) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    const int tid = threadIdx.x, lane = tid & 63;
+    int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
-    const int r32 = lane & 31, h = lane >> 5;
+    int r32 = lane & 31, h = lane >> 5;
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
     constexpr int TILE_M = 64 * MT;
     const int kgroups = p.K / 64;
@@ -83,22 +83,27 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
     // weight scales (wave 3).  The source pointers are wave-uniform and advance by a constant per k-group.
     constexpr int COPIES = MT == 2 ? COPIES_PER_WAVE : 5;
     constexpr int ST_A = StageOf<MT>::A, ST_W = StageOf<MT>::W, ST_WS = StageOf<MT>::WS, ST_AS = StageOf<MT>::AS, ST_Z = StageOf<MT>::Z;
-    const uint32_t copy_voff = lane * 16;
+    // (the lanes' offset of a copy is the one that the first activation fragment is read with, which saves a register: the sources
+    // stand `lead` bytes further ahead)
+    const uint32_t lead = ST_A + MT * wm * FRAG_BYTES;
+    uint32_t x16 = lead + lane * 16;
+    asm volatile("" : "+v"(x16));
+    const uint32_t &copy_voff = x16;
     const bool low = wave < 2;
     const uint8_t *act0 = p.act + ((size_t)mb * kgroups + gb) * (4 * FRAG_BYTES) + slab0 * FRAG_BYTES;
     const uint8_t *ws0 = p.wscales + ((size_t)nb * kgroups + gb) * 2048, *as0 = (const uint8_t *)(p.ascales + (size_t)gb * p.M_pad + m0);
     const uint32_t stride_q = (uint32_t)p.M_pad * 2;
-    const uint8_t *src_w = p.wgt + ((size_t)nb * kgroups + gb) * (8 * FRAG_BYTES) + wave * 3072;
-    const uint8_t *src_a = MT == 2 || wave < 3 ? act0 + wave * 1024 : ws0;
-    const uint8_t *src_x = MT == 2 ? (low ? act0 + (4 + wave) * 1024 : ws0 + (wave - 2) * 1024) : (wave < 3 ? as0 : ws0 + 1024);
-    const uint8_t *src_q = as0;  // (128 rows only)
+    const uint8_t *src_w = p.wgt + ((size_t)nb * kgroups + gb) * (8 * FRAG_BYTES) + wave * 3072 - lead;
+    const uint8_t *src_a = (MT == 2 || wave < 3 ? act0 + wave * 1024 : ws0) - lead;
+    const uint8_t *src_x = MT == 2 ? (low ? act0 + (4 + wave) * 1024 : ws0 + (wave - 2) * 1024) - lead : (wave < 3 ? as0 : ws0 + 1024);
+    const uint8_t *src_q = as0 - lead / 4;  // (128 rows only)
     const uint32_t stride_a = MT == 2 || wave < 3 ? 4 * FRAG_BYTES : 2048;
     const uint32_t stride_x = MT == 2 ? (low ? 4 * FRAG_BYTES : 2048) : (wave < 3 ? stride_q : 2048);
     const uint32_t dst_w = lds_base + ST_W + wave * 3072;
     const uint32_t dst_a = lds_base + (MT == 2 || wave < 3 ? ST_A + wave * 1024 : ST_WS);
     const uint32_t dst_x = lds_base + (MT == 2 ? (low ? ST_A + (4 + wave) * 1024 : ST_WS + (wave - 2) * 1024) : (wave < 3 ? ST_AS : ST_WS + 1024));
     const uint32_t dst_q = lds_base + ST_AS;
-    const uint32_t x_voff = MT == 2 || wave == 3 ? lane * 16 : (lane & 7) * 16;
+    const uint32_t x_voff = MT == 2 ? x16 : wave == 3 ? lane * 16 : (lane & 7) * 16;
     // The requests of a k-group are issued one at a time, spread over the steps of the main loop: a wave
     // that issues its six requests back to back stands still until the memory pipeline has taken them,
     // about 30 cycles each.  First the three weight chunks (W), later the other three (R).
@@ -138,21 +143,21 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
     if (ng > 2)
         for (int i = 0; i < 3; i++) copy_w(2 * STAGE_BYTES, i);
 
-    // per-lane read offsets inside a stage
-    const uint32_t off16 = lane * 16, off8 = 1024 + lane * 8;
-    const uint32_t off_ws = ST_WS + (128 * wn + r32) * 8;
-    const uint32_t off_as = h ? ST_Z : ST_AS + (32 * MT * wm + r32) * 2;
+    // Per-lane read offsets inside a stage.  Opaque, so that the unrolled loop and the last groups, whose stage is not a
+    // constant, share these registers.
+    uint32_t x8 = ST_A + MT * wm * FRAG_BYTES + 1024 + lane * 8;
+    uint32_t w16 = ST_W + 4 * wn * FRAG_BYTES + lane * 16, w8 = ST_W + 4 * wn * FRAG_BYTES + 1024 + lane * 8;
+    uint32_t off_ws = ST_WS + (128 * wn + r32) * 8, off_as = h ? ST_Z : ST_AS + (32 * MT * wm + r32) * 2;
+    asm volatile("" : "+v"(x8), "+v"(w16), "+v"(w8), "+v"(off_ws), "+v"(off_as));
     auto read_x = [&](uint32_t sb, int mt, Frag &f, uint32_t &as) {
-        const uint8_t *base = lds + sb + ST_A + (MT * wm + mt) * FRAG_BYTES;
-        f.lo = *(const u32x4_t *)(base + off16);
-        f.hi = *(const u32x2_t *)(base + off8);
-        as = *(const uint16_t *)(lds + sb + off_as + mt * 64);
+        f.lo = *(const u32x4_t *)(lds + x16 + (sb + mt * FRAG_BYTES));
+        f.hi = *(const u32x2_t *)(lds + x8 + (sb + mt * FRAG_BYTES));
+        as = *(const uint16_t *)(lds + off_as + (sb + mt * 64));
     };
     auto read_w = [&](uint32_t sb, int nt, Frag &f, u32x2_t &ws) {
-        const uint8_t *base = lds + sb + ST_W + (4 * wn + nt) * FRAG_BYTES;
-        f.lo = *(const u32x4_t *)(base + off16);
-        f.hi = *(const u32x2_t *)(base + off8);
-        ws = *(const u32x2_t *)(lds + sb + off_ws + nt * 256);
+        f.lo = *(const u32x4_t *)(lds + w16 + (sb + nt * FRAG_BYTES));
+        f.hi = *(const u32x2_t *)(lds + w8 + (sb + nt * FRAG_BYTES));
+        ws = *(const u32x2_t *)(lds + off_ws + (sb + nt * 256));
     };
 
     float16_t acc[4 * MT];  // tile t = MT nt + mt
@@ -208,8 +213,9 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
     // of group l.  At the barrier group l + 1 must have landed; the six requests of group l + 2 are the
     // only ones issued after it.  MODE 2: both (l + 3 < ng), 1: only the rest of group l + 2 (l = ng - 3),
     // 0: nothing left to request.
-    auto group_body = [&](auto MODE_T) {
-        constexpr int MODE = decltype(MODE_T)::value;
+    auto group_body = [&](auto MODE_T, auto STAGE_T) {
+        constexpr int MODE = decltype(MODE_T)::value, STAGE = decltype(STAGE_T)::value;
+        if (STAGE >= 0) sb = STAGE * STAGE_BYTES;
         const uint32_t sb_next = sb == (STAGES - 1) * STAGE_BYTES ? 0 : sb + STAGE_BYTES;
         const uint32_t sb_prev = sb == 0 ? (STAGES - 1) * STAGE_BYTES : sb - STAGE_BYTES;
         if constexpr (MT == 2) {
@@ -266,15 +272,27 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
         sb = sb_next;
     };
     int l = 0;
-    for (; l + 3 < ng; l++) group_body(std::integral_constant<int, 2>{});
+    // Whole turns of the ring with the stages as constants: every LDS address is a lane's offset and an instruction's, 211
+    // instructions per k-group (64 rows: 122) against 233 (144).
+    for (; (TURNS || MT == 1) && l + 5 < ng; l += STAGES) {
+        group_body(std::integral_constant<int, 2>{}, std::integral_constant<int, 0>{});
+        group_body(std::integral_constant<int, 2>{}, std::integral_constant<int, 1>{});
+        group_body(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});
+    }
+    for (; l + 3 < ng; l++) group_body(std::integral_constant<int, 2>{}, std::integral_constant<int, -1>{});
     if (l + 2 < ng) {
-        group_body(std::integral_constant<int, 1>{});
+        group_body(std::integral_constant<int, 1>{}, std::integral_constant<int, -1>{});
         l++;
     }
-    for (; l < ng; l++) group_body(std::integral_constant<int, 0>{});
+    for (; l < ng; l++) group_body(std::integral_constant<int, 0>{}, std::integral_constant<int, -1>{});
 #undef SVDQ_STEP
 #undef SVDQ_FMA
     __syncthreads();  // the ring is free: the epilogue reuses it
+    // (the thread's coordinates once more, from its lane's number: none of them occupies a register in the main loop)
+    lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    tid = wave * 64 + lane;
+    r32 = lane & 31;
+    h = lane >> 5;
 
     // ---- a tile split along K --------------------------------------------------------------------
     // Every part parks its sums in its slot of the workspace; whoever arrives last adds all parts in
@@ -780,16 +798,20 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
     }
 }
 
-template <bool NEXT>
+// TURNS: the main loop of the 128-row tiles runs in whole turns of the LDS ring (output_tile).  K = 3072, without / with: M = 4608, N =
+// 12288 162 / 159 us, with the quantizing epilogue 194 / 188, N = 9216 126.7 / 123.1; M = 18432, N = 12288, rank 128 679 / 661; K = 12288, M =
+// 4608, N = 3072 162.8 / 157.7.  Not where compute units have one 128-row tile each and 64-row tiles next to some: the longest then take
+// longer (M = 1024, N = 9216 32.9 / 33.4; K = 4096, M = 1157 45.0 / 45.9).  (64-row tiles always do: M = 505, N = 9216 27.7 / 25.4.)
+template <bool NEXT, bool TURNS>
 __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
     const TileOf t = tile_of(p, (int)blockIdx.x, (int)gridDim.x, (p.N + BN - 1) / BN);
-    if (t.whole) output_tile<NEXT, 2>(p, t.row_block * BM, t.column_block, t.tile, t.part, t.row_block);
-    else output_tile<NEXT, 1>(p, p.full_blocks * BM + t.row_block * (BM / 2), t.column_block, 0, 0, p.full_blocks + t.row_block);
+    if (t.whole) output_tile<NEXT, 2, TURNS>(p, t.row_block * BM, t.column_block, t.tile, t.part, t.row_block);
+    else output_tile<NEXT, 1, TURNS>(p, p.full_blocks * BM + t.row_block * (BM / 2), t.column_block, 0, 0, p.full_blocks + t.row_block);
 }
 
-template <bool NEXT>
+template <bool NEXT, bool TURNS>
 int launch_gemm6(const Params &p, int nwg, hipStream_t stream) {
-    auto kern = gemm6_kernel<NEXT>;
+    auto kern = gemm6_kernel<NEXT, TURNS>;
     // the attribute is set once per device (racing first calls both set it, which is harmless)
     static bool lds_reserved[64] = {false};
     int dev = 0;
