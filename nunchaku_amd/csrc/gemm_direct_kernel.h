@@ -165,7 +165,7 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
             auto tile = [&](auto T) {
                 constexpr int t = decltype(T)::value, nt = t / MT, mt = t % MT, b = t & 1, prev = (t + NT * MT - 1) % (NT * MT);
                 P[b] = mfma_codes6(st.w[nt], st.x[mt]);
-                F[b] = mfma_factor(u32x2_t{st.ws[nt], 0u}, h ? 0u : st.as[mt]);
+                F[b] = mfma_factor(u32x2_t{st.ws[nt], 0u}, u32x2_t{h ? 0u : st.as[mt], 0u});
 #pragma unroll
                 for (int e = 0; e < 16; e++) acc[prev][e] = __builtin_fmaf(P[b ^ 1][e], F[b ^ 1][e], acc[prev][e]);
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);

@@ -28,10 +28,11 @@ __device__ inline float16_t mfma_codes(const Frag &w, const Frag &x) { return mf
 
 // factor tile 64 ws[n] * as[m]: the weight operand is {64 s, 0, 0, 0} in both half-waves (k slots 0-3 and
 // 4-7), the activation operand carries its scale in k slot 0 and zero in k slot 4, anything finite
-// elsewhere
-__device__ inline float16_t mfma_factor(u32x2_t ws, uint32_t as) {
+// elsewhere.  (A pair of registers whose second one stays zero: put together from a scale and a zero, the operand costs the
+// caller up to two instructions each time.)
+__device__ inline float16_t mfma_factor(u32x2_t ws, u32x2_t as) {
     const float16_t z = {};
-    return __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(__builtin_bit_cast(bf16x4_t, ws), __builtin_bit_cast(bf16x4_t, u32x2_t{as, 0u}), z, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(__builtin_bit_cast(bf16x4_t, ws), __builtin_bit_cast(bf16x4_t, as), z, 0, 0, 0);
 }
 
 // ---- NVFP4 ------------------------------------------------------------------------------------------
