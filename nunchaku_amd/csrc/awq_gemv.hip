@@ -67,6 +67,9 @@ __device__ inline void store_result(const AwqParams &p, int m, int row, float su
 // N = 18432 one row 11.9 / 10.7 us, four 13.0 / 10.8, eight 15.7 / 11.4; K = 4096, N = 20480, eight rows 24.1 / 15.3;
 // K = 3072, N = 9216, one row 8.5 / 8.0.  About 3 us of that are launch and latency, the rest 4.2 TB/s.  Further ahead is slower
 // (three tiles 11.7, four 12.4), two workgroups of half the tiles per compute unit too (13.0).
+// Equal shares of the channels (N = 18432 is 4.5 tiles per workgroup, which were 4 or 5), no requests behind a share's end (the tiles
+// requested ahead made 40 % more of them) and one division in place of two of 64 bits, in a graph of eight layers in turn, before / now:
+// K = 3072, N = 18432 one row 10.4 / 10.0 us, eight 11.5 / 11.1; N = 9216 7.5 / 7.0; N = 3072, four rows 5.2 / 4.7; K = 1024, N = 2048 2.77 / 2.70.
 constexpr int WAVES = 8, BATCH = 6, AHEAD = 2;
 static_assert(BATCH % (AHEAD + 1) == 0, "the ring of register sets is indexed by the position in a batch");
 template <int SPW>
@@ -78,8 +81,10 @@ __global__ void __launch_bounds__(64 * WAVES, 2) awq_gemv_rows_kernel(AwqParams 
     const int kblocks = p.K / 64;
     int wg = blockIdx.x;
     if (gridDim.x % 8 == 0) wg = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;  // neighbours in N on one XCD: they share lines of scales
-    const int ntiles = (p.N + 15) / 16;
-    const int t_begin = (int)((long long)ntiles * wg / gridDim.x), t_end = (int)((long long)ntiles * (wg + 1) / gridDim.x);
+    // The workgroup's channels, in units of the storage's four; tile t holds 16 of them from c_begin + 16 t on, the last one what is left.
+    const int share = (int)((unsigned)(p.N / 4) / gridDim.x), more = p.N / 4 - share * (int)gridDim.x;
+    const int c_begin = 4 * (wg * share + (wg < more ? wg : more)), c_end = c_begin + 4 * (share + (wg < more ? 1 : 0));
+    const int t_end = (c_end - c_begin + 15) / 16;
 
     u32x4_t x[SPW][4];
     uint32_t w_off[SPW], s_off[SPW];
@@ -101,25 +106,27 @@ __global__ void __launch_bounds__(64 * WAVES, 2) awq_gemv_rows_kernel(AwqParams 
         u32x4_t w[SPW];
         uint16_t s[SPW], z[SPW];
     };
-    // first channel of a tile: the last one of a ragged N begins early and works some channels out twice
-    auto first_channel = [&](int t) { return 16 * t < p.N - 16 ? 16 * t : p.N - 16; };
+    // Requests are branch-free: a lane whose channel lies behind the workgroup's last one (the end of its last tile, and the tiles
+    // requested ahead at the end) gets an offset beyond its buffer, which reads zeros and touches no memory.
+    const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(p.qweight + (size_t)(c_begin >> 2) * kblocks * 128), 0, ((c_end - c_begin) >> 2) * kblocks * 128, 0x00020000);
+    const __amdgpu_buffer_rsrc_t srsrc = __builtin_amdgcn_make_buffer_rsrc((void *)p.scales, 0, kblocks * p.N * 2, 0x00020000);
+    const __amdgpu_buffer_rsrc_t zrsrc = __builtin_amdgcn_make_buffer_rsrc((void *)p.zeros, 0, kblocks * p.N * 2, 0x00020000);
     auto load = [&](int t, Tile &d) {
-        const int c0 = first_channel(t);
-        const uint8_t *wp = p.qweight + (size_t)(c0 >> 2) * kblocks * 128;
-        const uint8_t *sp = (const uint8_t *)(p.scales + c0), *zp = (const uint8_t *)(p.zeros + c0);
+        const uint32_t beyond = c_begin + 16 * t + n < c_end ? 0u : 0x80000000u;
+        const int wt = t * kblocks * 512, st = (c_begin + 16 * t) * 2;
 #pragma unroll
         for (int j = 0; j < SPW; j++) {
-            d.w[j] = __builtin_nontemporal_load((const u32x4_t *)(wp + w_off[j]));
-            d.s[j] = *(const uint16_t *)(sp + s_off[j]);
-            d.z[j] = *(const uint16_t *)(zp + s_off[j]);
+            d.w[j] = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_off[j] | beyond, wt, 2);  // (2: a streaming load)
+            d.s[j] = __builtin_amdgcn_raw_buffer_load_b16(srsrc, s_off[j] | beyond, st, 0);
+            d.z[j] = __builtin_amdgcn_raw_buffer_load_b16(zrsrc, s_off[j] | beyond, st, 0);
         }
     };
     Tile ring[AHEAD + 1];
 #pragma unroll
-    for (int a = 0; a < AHEAD; a++) load(t_begin + a, ring[a]);
-    for (int t0 = t_begin; t0 < t_end; t0 += BATCH) {
+    for (int a = 0; a < AHEAD; a++) load(a, ring[a]);
+    for (int t0 = 0; t0 < t_end; t0 += BATCH) {
         const int count = t_end - t0 < BATCH ? t_end - t0 : BATCH;
-        if (t0 > t_begin) __syncthreads();
+        if (t0 > 0) __syncthreads();
 #pragma unroll
         for (int i = 0; i < BATCH; i++) {
             if (i >= count) continue;
@@ -143,7 +150,8 @@ __global__ void __launch_bounds__(64 * WAVES, 2) awq_gemv_rows_kernel(AwqParams 
             float sum = 0.f;
 #pragma unroll
             for (int w = 0; w < WAVES; w++) sum += ((const float *)&red[i][w][(m >> 2) * 16 + c])[m & 3];
-            store_result(p, m, first_channel(t0 + i) + c, sum);
+            const int channel = c_begin + 16 * (t0 + i) + c;
+            if (channel < c_end) store_result(p, m, channel, sum);
         }
     }
 }
