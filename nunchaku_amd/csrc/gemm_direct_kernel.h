@@ -13,7 +13,7 @@
 // the operand requests hit in the L2s, which hand out 2.15 KB per 32 x 32 tile and k-group with one row block and four column tiles
 // per wave, 1.65 KB with two of each (82 GB/s per compute unit, 64 bytes per clock being about 150).  With several tiles per compute
 // unit the matrix core and the conversions are (M = 1157, K = 12288, NVFP4: 10 % waits for operands, 49 and 34 % the others).
-// M = 256, K = N = 3072: 22.8 -> 9.6 us (INT4; 4.7 us of it do not depend on K), 59.9 -> 11.2 us (NVFP4).
+// M = 256, K = N = 3072: 22.8 -> 8.8 us (INT4; 4.2 us of it do not depend on K), 59.9 -> 10.6 us (NVFP4).
 //
 // INT4: one fp6 matrix instruction on the codes, one factor instruction and 16 multiply-adds per 32 x 32 tile and
 // k-group (gemm6_kernel.h).  NVFP4: both operands are dequantized to fp16 in registers by the wave that uses them
@@ -82,13 +82,15 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
     // by reference as an argument, a set is known to be readable as a whole, the compiler reads vectors of six words
     // eight wide from it, and then cannot keep it in registers)
     Stage<FP4, MT, NT> sets[DEPTH + 1];
-    // The k-group requested next and the wave-uniform addresses of its operands, which advance by constants; behind the
-    // last group they stay where they are (such a request is never used).
+    // The k-group requested next; behind the last one it stays where it is (such a request is never used).
+    // INT4: wave-uniform addresses of the operands, which advance by constants.  NVFP4: buffers; a request is a lane's offset that never
+    // changes, a scalar one that carries the k-group, and a constant, so that no vector instruction is spent on addresses (21 of 684
+    // instructions per three k-groups before): M = 1157, K = 12288, N = 3072 87.4 -> 76.4 us, M = 300, K = N = 3072 10.8 -> 10.6, M = 512, K = 2048,
+    // N = 6144 with norm and rotary 22.1 -> 20.0; same bits.  (INT4 with buffers: 8.77 -> 8.99 at M = 256, K = N = 3072, though its loop has a
+    // fifth fewer instructions then.)
     int g_load = kpart < kgroups ? kpart : kgroups - 1;
     const uint8_t *wp, *sp, *xp[MT];
     const uint16_t *ap;
-    const uint32_t w_step = KP * (FP4 ? TILE_BYTES : 8 * FRAG_BYTES), x_step = KP * (FP4 ? TILE_BYTES : 4 * FRAG_BYTES);
-    const uint32_t s_step = FP4 ? (uint32_t)p.N * (8 * KP) : 2048 * KP, a_step = (uint32_t)p.M_pad * (FP4 ? 2 * KP : KP);
     if constexpr (!FP4) {
         wp = p.wgt + ((size_t)(nb >> 1) * kgroups + g_load) * (8 * FRAG_BYTES) + ((nb & 1) * 4 + cw * NT) * FRAG_BYTES;
         sp = (const uint8_t *)p.wscales + ((size_t)(nb >> 1) * kgroups + g_load) * 2048 + (nb & 1) * 1024 + cw * (NT * 256);
@@ -97,38 +99,48 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
             xp[mt] = p.act + ((size_t)((f0 + mt) >> 2) * kgroups + g_load) * (4 * FRAG_BYTES) + ((f0 + mt) & 3) * FRAG_BYTES;
         });
         ap = p.ascales + (size_t)g_load * p.M_pad + f0 * 32;
-    } else {
-        wp = p.wgt + ((size_t)(nb * 4 + cw * NT) * kgroups + g_load) * TILE_BYTES;
-        sp = (const uint8_t *)p.wscales + ((size_t)g_load * p.N + n0 + cw * (NT * 32)) * 8;
-        each(std::make_integer_sequence<int, MT>{}, [&](auto I) {
-            constexpr int mt = decltype(I)::value;
-            xp[mt] = p.act + ((size_t)(f0 + mt) * kgroups + g_load) * TILE_BYTES;
-        });
-        ap = p.ascales + ((size_t)g_load * p.M_pad + f0 * 32) * 2;
     }
     const uint32_t off16 = (uint32_t)lane * 16u, off8 = 1024u + (uint32_t)lane * 8u, off_ws = (uint32_t)r32 * 8u + (FP4 ? (uint32_t)h * 4u : 0u);
     const uint32_t off_as = FP4 ? (uint32_t)r32 * 4u + (uint32_t)h * 2u : (uint32_t)r32 * 2u, off_fp4 = (uint32_t)r32 * 32u + (uint32_t)h * 16u;
-    const uint32_t tile_stride = (uint32_t)kgroups * TILE_BYTES;  // NVFP4: from one 32-column tile to the next
+    const uint32_t tile_stride = (uint32_t)kgroups * TILE_BYTES;  // NVFP4: from one 32-column (or 32-row) tile to the next
+    auto buffer = [](const void *base, uint32_t bytes) { return __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (int)bytes, 0x00020000); };
+    const uint32_t s_group = (uint32_t)p.N * 8, a_group = (uint32_t)p.M_pad * 4, s_lead = (n0 + cw * (NT * 32)) * 8, a_lead = f0 * 32 * 4;
+    const __amdgpu_buffer_rsrc_t wrsrc = buffer(p.wgt + (size_t)(nb * 4 + cw * NT) * kgroups * TILE_BYTES, NT * tile_stride);
+    const __amdgpu_buffer_rsrc_t xrsrc = buffer(p.act + (size_t)f0 * kgroups * TILE_BYTES, MT * tile_stride);
+    const __amdgpu_buffer_rsrc_t srsrc = buffer((const uint8_t *)p.wscales + s_lead, kgroups * s_group - s_lead);
+    const __amdgpu_buffer_rsrc_t arsrc = buffer((const uint8_t *)p.ascales + a_lead, kgroups * a_group - a_lead);
     auto load = [&](auto S) {
         auto &st = sets[decltype(S)::value];
-        each(std::make_integer_sequence<int, MT>{}, [&](auto I) {
-            constexpr int mt = decltype(I)::value;
-            if constexpr (!FP4) st.x[mt] = codes6(*(const u32x4_t *)(xp[mt] + off16), *(const u32x2_t *)(xp[mt] + off8));
-            else st.x[mt] = *(const u32x4_t *)(xp[mt] + off_fp4);
-            st.as[mt] = *(const uint16_t *)((const uint8_t *)ap + mt * (FP4 ? 128 : 64) + off_as);
-        });
-        each(std::make_integer_sequence<int, NT>{}, [&](auto I) {
-            constexpr int nt = decltype(I)::value;
-            if constexpr (!FP4) st.w[nt] = codes6(*(const u32x4_t *)(wp + nt * FRAG_BYTES + off16), *(const u32x2_t *)(wp + nt * FRAG_BYTES + off8));
-            else st.w[nt] = *(const u32x4_t *)(wp + nt * tile_stride + off_fp4);
-            st.ws[nt] = *(const uint32_t *)(sp + nt * 256 + off_ws);
-        });
         const bool more = g_load + KP < kgroups;
+        if constexpr (FP4) {
+            const int o = g_load * TILE_BYTES, so = g_load * (int)s_group, ao = g_load * (int)a_group;
+            each(std::make_integer_sequence<int, MT>{}, [&](auto I) {
+                constexpr int mt = decltype(I)::value;
+                st.x[mt] = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, off_fp4, o + mt * (int)tile_stride, 0);
+                st.as[mt] = __builtin_amdgcn_raw_buffer_load_b16(arsrc, off_as + mt * 128, ao, 0);
+            });
+            each(std::make_integer_sequence<int, NT>{}, [&](auto I) {
+                constexpr int nt = decltype(I)::value;
+                st.w[nt] = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, off_fp4, o + nt * (int)tile_stride, 0);
+                st.ws[nt] = __builtin_amdgcn_raw_buffer_load_b32(srsrc, off_ws + nt * 256, so, 0);
+            });
+        } else {
+            each(std::make_integer_sequence<int, MT>{}, [&](auto I) {
+                constexpr int mt = decltype(I)::value;
+                st.x[mt] = codes6(*(const u32x4_t *)(xp[mt] + off16), *(const u32x2_t *)(xp[mt] + off8));
+                st.as[mt] = *(const uint16_t *)((const uint8_t *)ap + mt * 64 + off_as);
+            });
+            each(std::make_integer_sequence<int, NT>{}, [&](auto I) {
+                constexpr int nt = decltype(I)::value;
+                st.w[nt] = codes6(*(const u32x4_t *)(wp + nt * FRAG_BYTES + off16), *(const u32x2_t *)(wp + nt * FRAG_BYTES + off8));
+                st.ws[nt] = *(const uint32_t *)(sp + nt * 256 + off_ws);
+            });
+            wp += more ? KP * 8 * FRAG_BYTES : 0u;
+            sp += more ? 2048u * KP : 0u;
+            ap += more ? (uint32_t)p.M_pad * KP : 0u;
+            each(std::make_integer_sequence<int, MT>{}, [&](auto I) { xp[decltype(I)::value] += more ? KP * 4 * FRAG_BYTES : 0u; });
+        }
         g_load += more ? KP : 0;
-        wp += more ? w_step : 0u;
-        sp += more ? s_step : 0u;
-        ap += more ? a_step : 0u;
-        each(std::make_integer_sequence<int, MT>{}, [&](auto I) { xp[decltype(I)::value] += more ? x_step : 0u; });
     };
 
     // ---- main loop -----------------------------------------------------------------------------------

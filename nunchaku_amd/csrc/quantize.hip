@@ -195,8 +195,8 @@ __global__ void __launch_bounds__(64 * NW) quantize_fuse_lora_kernel(QuantParams
     // x of one chunk: MT tiles x 4 steps x 8 bf16 per lane (twice that with GLU)
     // Requests are unconditional (a request behind a branch makes the compiler's wait counting assume the
     // worst on every path and wait for the chunks requested ahead): a chunk index past the end gets a lane
-    // offset beyond the buffer size instead, which reads zeros and touches no memory.  (The hardware checks
-    // the lane offset against the size, not the scalar offset that carries the chunk.)
+    // offset beyond the buffer size instead, which reads zeros and touches no memory.  (Whether the hardware counts the scalar
+    // offset, which carries the chunk, in its check makes no difference: it stays inside the lane's row.)
     // (Eight waves on 32 rows at ranks above 64, where the loads of proj_down have their offsets worked out lane by lane otherwise:
     // M = 4608, K = 6144, rank 128 52.9 -> 41.8 us, rank 256 107 -> 77.  Not in the other forms: no change or a loss, four waves at rank 128 in
     // NVFP4 51 -> 77.)
