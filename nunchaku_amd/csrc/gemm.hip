@@ -311,7 +311,8 @@ int rows_needed(const svdq_gemm_args *a) {
 // Every compute unit gets `tiles / ncu` whole tiles or one more, the half tiles go where they end first.  Considered are whole
 // tiles only, whole tiles up to the last and the last but one multiple of the compute units, and (few tiles) half tiles only; a
 // division with half tiles has to be 4 % faster by the model.  Measured, whole tiles / the choice: M = 4608, K = 3072, N = 9216
-// 140 / 131 us; M = 4096, K = 2304, N = 6912 72.3 / 66.3; M = 1024, K = 3072, N = 9216 44.5 / 34.3; M = 505 of the same layer 32.9 / 28.7.
+// 140 / 131 us; M = 4096, K = 2304, N = 6912 72.3 / 66.3; M = 1024, K = 3072, N = 9216 44.5 / 34.3; M = 505 of the same layer 32.9 / 28.7
+// (with the main loop in whole turns of its ring 122, and 25.3 at M = 505).
 // Over the 700 other shapes 1.10 times as fast as whole tiles, 0.2 % off the best division measured, more than 3 % slower than whole
 // tiles in one.  (With 1.1 and 0.25, where three half tiles fit behind an odd whole one: slower in six, M = 4096, K = 3072, N = 9216, which
 // is whole tiles only now, 129 against 124.)
@@ -626,6 +627,8 @@ int gemm_fp4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t st
 //   K = 12288, N = 3072: M = 256  42.1 / 24.8 / 34.4           113.6 / 30.8 / 35.0
 //          M = 505             45.4 / 44.1 / 34.6           115.2 / 50.8 / 37.9
 //          M = 1157            66.6 / 86.6 / 65.6           127.5 / 99.5 / 81.2
+// (Measured when the models were fitted.  Since then the INT4 large tiles have become 3 to 9 % faster, M = 505, N = 9216 25.3, and NVFP4 in the
+// few-rows kernel as much, M = 1157, K = 12288 76.4: the INT4 choice still takes 0.8 % longer than the fastest over 323 shapes, the NVFP4 one 1.6 %.)
 int choose_direct(const svdq_gemm_args *a, int ncu) {
     if (a->k_split > 0) return 0;  // (the caller asks for the tiles that k_split is about)
     if (((uintptr_t)a->bias | (uintptr_t)a->wcscales | (uintptr_t)a->oscales) % 8 || (uintptr_t)a->colnorm % 16) return 0;  // (read four columns at a time)

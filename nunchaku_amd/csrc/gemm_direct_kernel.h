@@ -22,7 +22,7 @@
 // waits for the matrix core (32 cycles), so the conversions are counted: 64 rows x 128 columns per wave take 6 of them per matrix
 // instruction (64 x 64: 8), converted one step ahead and spread evenly between the matrix instructions (left to itself the
 // compiler issues these in pairs, with the conversions behind).  K = 12288, N = 3072, 64 x 64 per wave / 64 x 128 / with the
-// conversions a step ahead: M = 256 45.5 / 39.6 / 35.0 us, M = 1157 91.7 / 84.3 / 81.2; from two tiles per compute unit on 1.2
+// conversions a step ahead: M = 256 45.5 / 39.6 / 35.0 us, M = 1157 91.7 / 84.3 / 81.2 (76.4 with buffers, below); from two tiles per compute unit on 1.2
 // PFLOP/s, where the large kernel's 1.25 is the power limit.
 //
 // The epilogue is shared out by columns: wave w of four adds up the parts' sums of the 32 columns 32 w ... of the tile
