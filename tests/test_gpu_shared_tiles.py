@@ -128,3 +128,46 @@ def test_nvfp4_shared_tiles_match_whole_tiles(dev, M, K, N, aligned, monkeypatch
         tol = torch.maximum(ulp, 1e-5 * whole[i].float().abs().max())
         assert (diff <= tol).all(), f"launch with input {i}: max difference {diff.max().item()} beyond one bf16 ulp"
         assert (diff > 0).float().mean().item() < 1e-3
+
+
+@pytest.mark.parametrize("M,K,N,R,split,next_layer", [(2304, 256, 7680, 144, None, False), (2304, 256, 7680, 256, None, True), (512, 768, 512, 176, 4, False), (1024, 512, 768, 128, 3, False)])
+def test_nvfp4_shared_tiles_and_high_ranks_repeat(dev, M, K, N, R, split, next_layer, monkeypatch):
+    """Low-rank terms above rank 128 go through the accumulators of whoever finishes a shared tile last: launches with the same input
+    agree bit for bit whoever that is, and with whole tiles within the order of the fp32 sums.  Two, and (few tiles) three and four
+    parties per tile; rank 128 is the last whose term does not go that way."""
+    from nunchaku_amd import packing
+    from nunchaku_amd.ops import gemm as gemm_mod
+
+    announce(f"nvfp4 shared tiles, rank {R}: M={M} K={K} N={N} split={split} next_layer={next_layer}")
+    layer = synth.make_layer(N, K, R, seed=K + N + R, fp4=True)
+    m = make_module(layer, dev)
+    t = m.native_tensors()
+    n = make_module(synth.make_layer(128, N, 32, seed=9, fp4=True), dev).native_tensors() if next_layer else None
+    plans = record_plans(monkeypatch, dev)
+    act, asc, _ = m.quantize(synth.make_activations(M, K, seed=R).to(dev))
+    lora_act = torch.randn(M, R, generator=torch.Generator().manual_seed(R)).to(dev)
+
+    def run(k_split):
+        monkeypatch.setattr(gemm_mod, "K_SPLIT", k_split)
+        outs = dict(out=torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev))
+        extra = {}
+        if next_layer:
+            outs.update(qout=torch.zeros(M, packing.act_nbytes_per_row(N, True), dtype=torch.uint8, device=dev),
+                        oscales=torch.zeros(N // 16, M, dtype=torch.float8_e4m3fn, device=dev), lora_act_out=torch.zeros(M, 32, device=dev))
+            extra = dict(lora_down=n["proj_down"], smooth_factor=n["smooth_factor"])
+        gemm_mod.svdq_gemm_w4a4(act=act, wgt=t["qweight"], ascales=asc, wscales=t["wscales"], lora_act_in=lora_act, lora_up=t["proj_up"],
+                                bias=off_alignment(t["bias"]), fp4=True, alpha=m.alpha, wcscales=t["wcscales"], **outs, **extra)
+        torch.cuda.synchronize()
+        if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+            assert plans[-1].few_rows == 0 and plans[-1].shared_tiles == (k_split != 1), plans[-1]
+        return outs
+
+    first, whole = run(split), run(1)["out"].float()
+    for launch in range(12):
+        again = run(split)
+        for name, value in first.items():
+            assert torch.equal(again[name].view(torch.uint8), value.view(torch.uint8)), f"launch {launch}: {name} changed: the sum depends on the order of arrival"
+    got = first["out"].float()
+    big = torch.maximum(torch.maximum(whole.abs(), got.abs()), torch.tensor(2.0**-126, device=dev))
+    tol = torch.maximum(big.log2().floor().exp2() * 2.0**-7, 1e-5 * whole.abs().max())
+    assert ((got - whole).abs() <= tol).all() and (got != whole).float().mean().item() < 1e-3
