@@ -375,8 +375,8 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
     // a slot [64 quads][256 threads] x float4, a wave's access covers 1 KB) and go on.  (Starting the accumulators
     // from a neighbour's parked sums where they happen to be there already saves the parking, but changes the order
     // of the additions with the timing: outputs then differed in their last bit from launch to launch.)
-    // Where low-rank windows are added to the accumulators (ranks above 128, below), whoever finishes last parks its own sums too and
-    // starts the windows from zero: they join the sum of all the parties, whoever that is.
+    // Where low-rank windows are added to the accumulators (ranks above 128, below) they join the first party's sums, whoever finishes
+    // last: another party, which has parked its own sums by then, fetches the first one's in their place before the windows.
     const bool lr_windows = p.R_up > LR_STEPS * 16;
     bool run_epilogue = true, combine = false;
     int party_lo = 0, party_hi = -1;  // (worked out here, not ahead of the main loop, where they would occupy registers)
@@ -390,7 +390,7 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
         // (a look at the counter first saves the parking when everybody else is already done; not worth a
         // round trip where that is unlikely: a share begins with its shared tile and ends with the other)
         bool last = false;
-        if (!is_head && !lr_windows) {
+        if (!is_head) {
             if (tid == 0) *flag = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __syncthreads();
             last = *flag == others;
@@ -454,13 +454,21 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
     // writes to LDS and the matrix instructions, half as many as before.
     const int nsteps = p.R_up / 16;
     if (run_epilogue && nsteps > 0) {
-        if (combine && lr_windows) {
+        if (combine && lr_windows && vwg != party_lo) {
+            const bool begins_inside = units * party_lo / nwg > (long long)tile_e * kunits;
+            const __amdgpu_buffer_rsrc_t r = partial_rsrc((const float4_t *)p.partials + (size_t)(2 * party_lo + (begins_inside ? 0 : 1)) * (64 * 256));
 #pragma unroll
             for (int i = 0; i < 4; i++)
 #pragma unroll
-                for (int j = 0; j < 4; j++)
+                for (int j = 0; j < 4; j++) {
 #pragma unroll
-                    for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
+                    for (int q = 0; q < 4; q++) {
+                        const float4_t s0 = load_partial(r, tid, (i * 4 + j) * 4 + q);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) acc[i][j][4 * q + e] = s0[e];
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
         }
         for (int w = (nsteps - 1) / LR_STEPS; w >= 0; w--) {
             const int first = w * LR_STEPS, steps = nsteps - first < LR_STEPS ? nsteps - first : LR_STEPS;
@@ -559,9 +567,8 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
         if (COMBINE) {
 #pragma unroll
             for (int k = 0; k < 16; k++) other[k] = float4_t{0.f, 0.f, 0.f, 0.f};
-            const int own_place = __builtin_amdgcn_readfirstlane(lr_windows ? party_hi + 1 : vwg);  // (behind all others with low-rank windows)
-            for (int v = party_lo; v <= party_hi || v == own_place; v++) {
-                if (v == own_place) {
+            for (int v = party_lo; v <= party_hi; v++) {
+                if (v - party_lo == (lr_windows ? 0 : vwg - party_lo)) {  // (whose sums the accumulators hold)
 #pragma unroll
                     for (int k = 0; k < 16; k++)
 #pragma unroll
