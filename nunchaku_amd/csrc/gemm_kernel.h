@@ -426,18 +426,21 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
     // wave's 128 columns, tabulated in LDS (EpilogueBias, gemm_base.cuh:710-781)
     // (kept across tiles: consecutive tiles of a workgroup mostly lie in the same 256 columns)
     float *coltab = (float *)(lds + TAB_OFF + wave * 1024);  // [128] factors, then [128] biases
+    float *next_tab = (float *)(lds + NEXT_TAB_OFF + wave * NEXT_TAB_BYTES);
     if (run_epilogue && n0 != coltab_n0) {
         coltab_n0 = n0;
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            const int n = wcol0 + 2 * lane + j;
+            const int c = 2 * lane + j, n = wcol0 + c;
             const bool ok = n < p.N;
             float cf = ok ? p.colnorm[n] * p.alpha : 0.f;
             if (ok && p.wcscales) cf *= bf16_bits_to_f32(p.wcscales[n]);
-            coltab[2 * lane + j] = cf;
-            coltab[128 + 2 * lane + j] = (ok && p.bias) ? bf16_bits_to_f32(p.bias[n]) : 0.f;
+            coltab[c] = cf;
+            coltab[128 + c] = (ok && p.bias) ? bf16_bits_to_f32(p.bias[n]) : 0.f;
+            if (NEXT && p.qout)  // reciprocal smoothing factors of the next layer, every 32 of them NEXT_TAB_LD apart
+                next_tab[c / 32 * NEXT_TAB_LD + c % 32] = ok ? p.next_smooth_rcp[n] : 1.f;
             if (NEXT && p.rotary)  // RMS-norm weights of the head these 128 columns are (q below N/3, k below 2N/3)
-                ((float *)(lds + NORMW_OFF + wave * 512))[2 * lane + j] = bf16_bits_to_f32((wcol0 < p.rope_cols / 2 ? p.norm_q : p.norm_k)[2 * lane + j]);
+                next_tab[c] = bf16_bits_to_f32((wcol0 < p.rope_cols / 2 ? p.norm_q : p.norm_k)[c]);
         }
     }
     // Low-rank up projection (lora.cuh:110-241): out += bf16(lora_act * scale) @ up^T on the matrix cores.  The operands of up to
@@ -541,17 +544,6 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
             }
         }
     }
-    // reciprocal smoothing factors of the next layer for the 32 columns this lane quantizes
-    // (work item of the quantizing pass: row = item / 4, 32-column quarter = item % 4 = lane % 4)
-    float nrs[32];
-    if (NEXT && p.qout && run_epilogue) {
-        const float4_t *sp = (const float4_t *)(p.next_smooth_rcp + (wcol0 < p.N ? wcol0 : 0) + (lane & 3) * 32);
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float4_t v = sp[i];
-            nrs[4 * i] = v[0]; nrs[4 * i + 1] = v[1]; nrs[4 * i + 2] = v[2]; nrs[4 * i + 3] = v[3];
-        }
-    }
     const bool interior = m0 + BM <= p.M_out && n0 + BN <= p.N_out;  // the whole tile lies inside the output
     uint16_t *slab = (uint16_t *)(lds + SLAB_OFF + wave * (32 * OUT_LD * 2));
     const int ngroups_out = p.N / 64;
@@ -593,7 +585,10 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
                 bs[q] = *(const float4_t *)(coltab + 128 + nt * 32 + 8 * q + 4 * h);
             }
         };
-        // (and so are the low-rank operands of two steps of 16 ranks)
+        // (and so are the low-rank operands of two steps of 16 ranks, but not with the next layer's epilogue, which has no registers for them:
+        // with them read ahead, and the 32 smoothing factors of a lane in registers from slab to slab instead of in LDS, 66 registers went
+        // through scratch memory, now 10.  K = 3072, before / now: M = 4608, N = 9216 with norm and rotary 261 / 250 us, rank 128 276 / 264; with the
+        // quantizing epilogue M = 1157, N = 12288 104.5 / 100.7, K = 4096, M = N = 4608 206 / 196)
         const int lr_steps = nsteps < LR_STEPS ? nsteps : LR_STEPS;
         bf16x8_t lr_x[2], lr_up[2][4];
         auto read_low_rank = [&](int st) {
@@ -606,7 +601,7 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
             }
         };
         load_cols(0, cfv[0], bsv[0]);
-        if (nsteps > 0) read_low_rank(0);
+        if (!NEXT && nsteps > 0) read_low_rank(0);
 #pragma unroll
         for (int nt = 0; nt < 4; nt++) {
             if (nt < 3) load_cols(nt + 1, cfv[(nt + 1) & 1], bsv[(nt + 1) & 1]);
@@ -627,7 +622,7 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
         }
         if (nsteps > 0) {
             for (int st = 0; st < lr_steps; st += 2) {
-                if (st > 0) read_low_rank(st);
+                if (NEXT || st > 0) read_low_rank(st);
 #pragma unroll
                 for (int k = 0; k < 2; k++) {
                     if (st + k >= lr_steps) break;
@@ -645,7 +640,6 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
             int blk = (wrow0 + mt * 32) >> 5;
             blk = blk < (p.rot_rows >> 5) ? blk : (p.rot_rows >> 5) - 1;  // (rows beyond the output are never stored)
             const float4_t *rp = (const float4_t *)p.rotary + (size_t)blk * (16 * 64) + lane;
-            const float *normw = (const float *)(lds + NORMW_OFF + wave * 512);
             float4_t sc[2][4];
 #pragma unroll
             for (int nt = 0; nt < 2; nt++)
@@ -662,7 +656,7 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
             for (int nt = 0; nt < 4; nt++) {
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
-                    const float4_t w4 = *(const float4_t *)(normw + nt * 32 + 8 * q + 4 * h);
+                    const float4_t w4 = *(const float4_t *)(next_tab + nt * 32 + 8 * q + 4 * h);
                     const float4_t s4 = sc[nt & 1][q];  // sin, cos of the two pairs
 #pragma unroll
                     for (int pr = 0; pr < 2; pr++) {
@@ -780,6 +774,13 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
         }
         if (NEXT && p.qout && wcol0 < p.N) {
             // EpilogueQuantize (gemm_w4a4.cuh:930-1043): shift, smooth, quantize for the next layer
+            // (work item: row = item / 4, 32-column quarter = item % 4 = lane % 4)
+            float nrs[32];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const float4_t v = *(const float4_t *)(next_tab + (lane & 3) * NEXT_TAB_LD + 4 * i);
+                nrs[4 * i] = v[0]; nrs[4 * i + 1] = v[1]; nrs[4 * i + 2] = v[2]; nrs[4 * i + 3] = v[3];
+            }
 #pragma unroll
             for (int pass = 0; pass < 2; pass++) {
                 const int item = pass * 64 + lane;

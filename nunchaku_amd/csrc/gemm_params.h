@@ -27,8 +27,10 @@ static_assert(2 * LR_BLOCK <= LR_UP, "");
 __host__ __device__ constexpr int lr_act_block(int wm, int slab) { return slab == 0 ? wm * LR_BLOCK : LR_ACT + ((slab - 1) * 2 + wm) * LR_BLOCK; }
 constexpr int TAB_OFF = LR_ACT + 6 * LR_BLOCK;             // 4 waves x float [2][128]: column factors and biases
 constexpr int FLAG_OFF = TAB_OFF + 4 * 1024;               // one word: a thread's reading of an arrival counter, for all
-constexpr int NORMW_OFF = FLAG_OFF + 16;                   // 4 waves x float [128]: RMS-norm weights of the wave's head
-constexpr int LDS_BYTES = NORMW_OFF + 4 * 512;
+// 4 waves: RMS-norm weights of the wave's head, float [128], or the next layer's reciprocal smoothing factors for the wave's columns, float
+// [4][NEXT_TAB_LD], 32 of each row used (the lanes of the quantizing pass read the four rows at a time)
+constexpr int NEXT_TAB_LD = 36, NEXT_TAB_BYTES = 4 * NEXT_TAB_LD * 4, NEXT_TAB_OFF = FLAG_OFF + 16;
+constexpr int LDS_BYTES = NEXT_TAB_OFF + 4 * NEXT_TAB_BYTES;
 static_assert(TAB_OFF >= 2 * OPBUF_BYTES, "the tables lie behind the operand buffers");
 static_assert(LDS_BYTES <= 160 * 1024, "one workgroup per compute unit");
 

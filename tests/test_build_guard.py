@@ -234,7 +234,7 @@ def test_few_rows_gemm_fits_its_registers(compiled, variant):
         assert u["VGPRs"] <= 256 and u["AGPRs"] == 0 and u["ScratchSize"] == 0 and u["Occupancy"] >= 2, (name, u)
 
 
-@pytest.mark.parametrize("variant,max_scratch", [(4, 48), (5, 256)])
+@pytest.mark.parametrize("variant,max_scratch", [(4, 48), (5, 144)])
 def test_nvfp4_gemm_register_figures(compiled, variant, max_scratch):
     usage, _ = compiled[("gemm_variant.hip", variant)]
     u = kernel_usage(usage, "gemm_w4a4_kernel")
