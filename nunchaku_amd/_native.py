@@ -78,9 +78,9 @@ class AwqGemvArgs(ctypes.Structure):
     ]
 
 
-# kernel variants, one translation unit each (-DSVDQ_VARIANT=n): the INT4 GEMM (gemm6_variant.hip: plain /
-# next-layer epilogue, both without the unrolled main loop), the NVFP4 GEMM (gemm_variant.hip: the same two) and the few-rows GEMM of either precision
-GEMM_VARIANT_UNITS = [("gemm6_variant.hip", 0), ("gemm6_variant.hip", 1), ("gemm6_variant.hip", 2), ("gemm6_variant.hip", 3), ("gemm_variant.hip", 4), ("gemm_variant.hip", 5),
+# kernel variants, one translation unit each (-DSVDQ_VARIANT=n): the INT4 GEMM (gemm6_variant.hip: plain, next-layer epilogue), the NVFP4
+# GEMM (gemm_variant.hip: the same two) and the few-rows GEMM (gemm_direct_variant.hip: the same two of INT4, then of NVFP4)
+GEMM_VARIANT_UNITS = [("gemm6_variant.hip", 0), ("gemm6_variant.hip", 1), ("gemm_variant.hip", 4), ("gemm_variant.hip", 5),
                       ("gemm_direct_variant.hip", 0), ("gemm_direct_variant.hip", 1), ("gemm_direct_variant.hip", 2), ("gemm_direct_variant.hip", 3)]
 
 

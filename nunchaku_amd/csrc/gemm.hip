@@ -17,8 +17,6 @@ int launch_fp4_next(const GemmParams &p, int shape, hipStream_t stream);
 namespace g6 {
 int launch_plain(const Params &p, int nwg, hipStream_t stream);
 int launch_next(const Params &p, int nwg, hipStream_t stream);
-int launch_plain_rolled(const Params &p, int nwg, hipStream_t stream);
-int launch_next_rolled(const Params &p, int nwg, hipStream_t stream);
 }  // namespace g6
 }  // namespace svdq
 
@@ -492,12 +490,7 @@ int gemm_int4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t s
     // One workgroup per output tile (or per part of one split along K), two resident per compute unit.
     const int nblocks = (p.N + g6::BN - 1) / g6::BN;
     lay_out_tiles(plan, p);
-    // (see gemm6_kernel's TURNS)
-    const bool rolled = p.half_blocks > 0 && p.full_blocks > 0 && p.full_blocks * nblocks <= compute_units(dev);
-    auto launch = [&](int nwg) {
-        if (needs_next_epilogue(a)) return rolled ? g6::launch_next_rolled(p, nwg, st) : g6::launch_next(p, nwg, st);
-        return rolled ? g6::launch_plain_rolled(p, nwg, st) : g6::launch_plain(p, nwg, st);
-    };
+    auto launch = [&](int nwg) { return needs_next_epilogue(a) ? g6::launch_next(p, nwg, st) : g6::launch_plain(p, nwg, st); };
     const int kparts = p.kparts, ntiles = (p.full_blocks + p.half_blocks) * nblocks;
     const size_t cnt_bytes = (size_t)ntiles * 4;
     const size_t part_bytes = kparts > 1 ? (size_t)ntiles * kparts * g6::BM * g6::BN * 4 : 0;

@@ -57,7 +57,7 @@ __device__ inline __amdgpu_buffer_rsrc_t partial_rsrc(const float *slot) {
 // The output tile of 64 MT rows x 256 columns from (m0, 256 nb) on.  MT = 2 is the ordinary tile; MT = 1 (wave tile
 // 32 x 128) serves the last rows of a launch, see gemm6_kernel below.  `tile`, `part`: the tile's number and this workgroup's share
 // of its k-groups where tiles are split along K (MT = 2 only); `vk_slot`: the slot of its linear-attention sums.
-template <bool NEXT, int MT, bool TURNS>
+template <bool NEXT, int MT>
 __device__ __forceinline__ void output_tile(const Params &p, const int m0, const int nb, const int tile, const int part, const int vk_slot) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     int tid = threadIdx.x, lane = tid & 63;
@@ -279,9 +279,12 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
         sb = sb_next;
     };
     int l = 0;
-    // Whole turns of the ring with the stages as constants: every LDS address is a lane's offset and an instruction's, 211
-    // instructions per k-group (64 rows: 122) against 233 (144).
-    for (; (TURNS || MT == 1) && l + 5 < ng; l += STAGES) {
+    // Whole turns of the ring with the stages as constants: every LDS address is a lane's offset and an instruction's, 203
+    // instructions per k-group (64 rows: 119).  K = 3072, one group after the other / in turns: M = 4608, N = 12288 162 / 159 us, with the
+    // quantizing epilogue 194 / 188, N = 9216 126.7 / 123.1; M = 18432, N = 12288, rank 128 679 / 661; K = 12288, M = 4608, N = 3072 162.8 / 157.7; 64-row
+    // tiles, M = 505, N = 9216 27.7 / 25.4.  Launches with one 128-row tile per compute unit and 64-row ones next to some, M = 275 ... 4379, K = 1152 ...
+    // 13056: the same in the plain epilogue (14 shapes, -3 to +1.3 %), up to 5 % faster with the next layer's (28).
+    for (; l + 5 < ng; l += STAGES) {
         group_body(std::integral_constant<int, 2>{}, std::integral_constant<int, 0>{});
         group_body(std::integral_constant<int, 2>{}, std::integral_constant<int, 1>{});
         group_body(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});
@@ -805,20 +808,16 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
     }
 }
 
-// TURNS: the main loop of the 128-row tiles runs in whole turns of the LDS ring (output_tile).  K = 3072, without / with: M = 4608, N =
-// 12288 162 / 159 us, with the quantizing epilogue 194 / 188, N = 9216 126.7 / 123.1; M = 18432, N = 12288, rank 128 679 / 661; K = 12288, M =
-// 4608, N = 3072 162.8 / 157.7.  Not where compute units have one 128-row tile each and 64-row tiles next to some: the longest then take
-// longer (M = 1024, N = 9216 32.9 / 33.4; K = 4096, M = 1157 45.0 / 45.9).  (64-row tiles always do: M = 505, N = 9216 27.7 / 25.4.)
-template <bool NEXT, bool TURNS>
+template <bool NEXT>
 __global__ void __launch_bounds__(256, 2) gemm6_kernel(Params p) {
     const TileOf t = tile_of(p, (int)blockIdx.x, (int)gridDim.x, (p.N + BN - 1) / BN);
-    if (t.whole) output_tile<NEXT, 2, TURNS>(p, t.row_block * BM, t.column_block, t.tile, t.part, t.row_block);
-    else output_tile<NEXT, 1, TURNS>(p, p.full_blocks * BM + t.row_block * (BM / 2), t.column_block, 0, 0, p.full_blocks + t.row_block);
+    if (t.whole) output_tile<NEXT, 2>(p, t.row_block * BM, t.column_block, t.tile, t.part, t.row_block);
+    else output_tile<NEXT, 1>(p, p.full_blocks * BM + t.row_block * (BM / 2), t.column_block, 0, 0, p.full_blocks + t.row_block);
 }
 
-template <bool NEXT, bool TURNS>
+template <bool NEXT>
 int launch_gemm6(const Params &p, int nwg, hipStream_t stream) {
-    auto kern = gemm6_kernel<NEXT, TURNS>;
+    auto kern = gemm6_kernel<NEXT>;
     // the attribute is set once per device (racing first calls both set it, which is harmless)
     static bool lds_reserved[64] = {false};
     int dev = 0;

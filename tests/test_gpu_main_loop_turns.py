@@ -1,6 +1,6 @@
 """The INT4 GEMM's main loop in whole turns of its LDS ring (three k-groups a turn, the rest behind them one by one) at every
-remainder, whole and split along K (odd counts of k-groups), against the oracle; and the kernels without the turns, which launches
-with one 128-row tile per compute unit and 64-row tiles next to them take, against those with: the same bits."""
+remainder, whole and split along K (odd counts of k-groups), against the oracle; and launches with at most one 128-row tile per
+compute unit and 64-row tiles next to them against whole tiles only: the same bits."""
 
 import pytest
 import torch
@@ -35,7 +35,7 @@ def test_one_whole_tile_per_unit_and_half_ones(dev, kind, M, K, N, monkeypatch):
     from nunchaku_amd import packing
     from nunchaku_amd.ops import gemm as gemm_mod
 
-    announce(f"without turns {kind} M={M} K={K} N={N}")
+    announce(f"both heights {kind} M={M} K={K} N={N}")
     m, nxt = make_module(synth.make_layer(N, K, 32, seed=K), dev), make_module(synth.make_layer(128, N, 32, seed=9), dev)
     t, n = m.native_tensors(), nxt.native_tensors()
     act, asc, la = m.quantize(synth.make_activations(M, K, seed=M).to(dev))
