@@ -309,8 +309,9 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
     // ascending order, so the result does not depend on who that is, and runs the epilogue.  Nobody waits for
     // anybody.
     if (MT == 2 && kparts > 1) {
-        float *slot = p.partials + ((size_t)tile * p.kparts + part) * PARTIAL_SLOT_FLOATS;
-        const __amdgpu_buffer_rsrc_t mine = partial_rsrc(slot);
+        // (scalar: the tile's number comes out of divisions in vector registers, and every request would be a loop over the lanes' descriptors)
+        auto slot_of = [&](int pt) { return partial_rsrc(p.partials + (size_t)__builtin_amdgcn_readfirstlane(tile * kparts + pt) * PARTIAL_SLOT_FLOATS); };
+        const __amdgpu_buffer_rsrc_t mine = slot_of(part);
 #pragma unroll
         for (int t = 0; t < 8; t++)
 #pragma unroll
@@ -337,7 +338,7 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
             constexpr int NOTH = 3;  // the other parts, j-th of them in ascending order: part j + (j >= own)
             __amdgpu_buffer_rsrc_t r[NOTH];
 #pragma unroll
-            for (int j = 0; j < NOTH; j++) r[j] = partial_rsrc(p.partials + ((size_t)tile * 4 + j + (j >= part ? 1 : 0)) * PARTIAL_SLOT_FLOATS);
+            for (int j = 0; j < NOTH; j++) r[j] = slot_of(j + (j >= part ? 1 : 0));
             // (items of half a 32 x 32 block: 8 accumulators per lane and part; a ring of three, two in flight)
             float4_t o[3][NOTH][2];
             auto request = [&](int i) {
@@ -377,8 +378,8 @@ __device__ __forceinline__ void output_tile(const Params &p, const int m0, const
                 for (int e = 0; e < 16; e++) acc[t][e] = 0.f;
             for (int pt0 = 0; pt0 < p.kparts; pt0 += 2) {
                 const bool two = pt0 + 1 < p.kparts;
-                const __amdgpu_buffer_rsrc_t r0 = partial_rsrc(p.partials + ((size_t)tile * p.kparts + pt0) * PARTIAL_SLOT_FLOATS);
-                const __amdgpu_buffer_rsrc_t r1 = partial_rsrc(p.partials + ((size_t)tile * p.kparts + (two ? pt0 + 1 : pt0)) * PARTIAL_SLOT_FLOATS);
+                const __amdgpu_buffer_rsrc_t r0 = slot_of(pt0);
+                const __amdgpu_buffer_rsrc_t r1 = slot_of(two ? pt0 + 1 : pt0);
                 float4_t o[2][2][4];
                 auto request = [&](int t, int b) {
 #pragma unroll

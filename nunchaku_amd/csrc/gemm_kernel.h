@@ -459,7 +459,8 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
     if (run_epilogue && nsteps > 0) {
         if (combine && lr_windows && vwg != party_lo) {
             const bool begins_inside = units * party_lo / nwg > (long long)tile_e * kunits;
-            const __amdgpu_buffer_rsrc_t r = partial_rsrc((const float4_t *)p.partials + (size_t)(2 * party_lo + (begins_inside ? 0 : 1)) * (64 * 256));
+            const int slot = __builtin_amdgcn_readfirstlane(2 * party_lo + (begins_inside ? 0 : 1));  // (or every request is a loop over the lanes' descriptors)
+            const __amdgpu_buffer_rsrc_t r = partial_rsrc((const float4_t *)p.partials + (size_t)slot * (64 * 256));
 #pragma unroll
             for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -587,7 +588,7 @@ __global__ void __launch_bounds__(256, 1) gemm_w4a4_kernel(GemmParams p) {
         };
         // (and so are the low-rank operands of two steps of 16 ranks, but not with the next layer's epilogue, which has no registers for them:
         // with them read ahead, and the 32 smoothing factors of a lane in registers from slab to slab instead of in LDS, 66 registers went
-        // through scratch memory, now 10.  K = 3072, before / now: M = 4608, N = 9216 with norm and rotary 261 / 250 us, rank 128 276 / 264; with the
+        // through scratch memory, now 8.  K = 3072, before / now: M = 4608, N = 9216 with norm and rotary 261 / 250 us, rank 128 276 / 264; with the
         // quantizing epilogue M = 1157, N = 12288 104.5 / 100.7, K = 4096, M = N = 4608 206 / 196)
         const int lr_steps = nsteps < LR_STEPS ? nsteps : LR_STEPS;
         bf16x8_t lr_x[2], lr_up[2][4];

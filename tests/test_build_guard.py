@@ -245,6 +245,13 @@ def test_nvfp4_gemm_register_figures(compiled, variant, max_scratch):
 
 
 @pytest.mark.parametrize("unit", nv.GEMM_VARIANT_UNITS)
+def test_gemm_requests_are_not_made_lane_by_lane(compiled, unit):
+    _, lines = compiled[unit]
+    assert sum("buffer_" in l for l in lines) > 0 or unit[0] == "gemm_direct_variant.hip"  # (parked sums of the large tiles)
+    assert lane_by_lane_requests(lines) == {}
+
+
+@pytest.mark.parametrize("unit", nv.GEMM_VARIANT_UNITS)
 def test_no_condition_code_kept_across_inline_asm(compiled, unit):
     _, lines = compiled[unit]
     # (of the few-rows kernels only the INT4 one with the quantizing epilogue has inline assembly, the fp6 conversion)
