@@ -1,13 +1,18 @@
-"""Host-side model of every global address the INT4 GEMM kernel, the few-rows GEMM kernel and the quantize kernel form, checked
-against the sizes of the buffers the operators are given (CPU only; nothing here touches a GPU).
+"""Host-side model of the global addresses that the INT4 GEMM kernel, the low-rank term of the NVFP4 GEMM kernel, the few-rows GEMM
+kernel, the quantize kernel and the AWQ GEMV kernel form, checked against the sizes of the buffers the operators are given (CPU only;
+nothing here touches a GPU).
 
 Which tile a workgroup takes is asked of the library (``plan_util``).  The model restates the index arithmetic of
-``csrc/gemm6_kernel.h`` (k-parts, the schedule of the asynchronous copies with its look-ahead, parked partial sums, output
-stores), of ``csrc/gemm_direct_kernel.h`` (operands of both precisions) and of ``csrc/quantize.hip`` (the row buffer whose size
-ends at the last valid row, code / scale / projection stores) for whole grids, over the shape distribution of
+``csrc/gemm6_kernel.h`` (k-parts, the schedule of the asynchronous copies with its look-ahead, the copies of the low-rank operands,
+parked partial sums, output stores), of ``csrc/gemm_kernel.h`` (low-rank operands), of ``csrc/gemm_direct_kernel.h`` (operands of both
+precisions, NVFP4 ones as buffers), of ``csrc/quantize.hip`` (the row buffer whose size ends at the last valid row, code / scale /
+projection stores) and of ``csrc/awq_gemv.hip`` (the shares' buffers) for whole grids, over the shape distribution of
 ``tests/test_gpu_shape_sweep.py`` and of the randomized loop that once ended in a GPU fault (M = 100, K = 3072, N = 768,
 rank 0, three k-parts among them).  It guards the arithmetic; the fault itself came from the compiler keeping a carry flag
 alive across an inline-asm statement that overwrote it (``tests/test_build_guard.py`` checks the generated code for that).
+
+Buffer requests (a descriptor, a lane's offset and a scalar offset) are modelled with a range check that counts the scalar offset and
+with one that does not: what a lane reads must not depend on it, and no sum may pass 4 GB.
 """
 
 import random
@@ -97,6 +102,17 @@ def check_gemm6(M_pad, N, K, M_out, N_out, k_split=0):
     return kparts
 
 
+def buffer_read(size, voff, soff, nbytes, memory):
+    """A request that is meant to read: inside the descriptor's size by either check, and inside the memory behind its base."""
+    assert 0 <= size < 1 << 31 and 0 <= voff and 0 <= soff < 1 << 31
+    assert voff + soff + nbytes <= size <= memory
+
+
+def buffer_skip(size, voff, soff):
+    """A request that is meant to touch no memory: outside by either check, without a sum beyond 32 bits."""
+    assert voff >= size and voff + soff < 1 << 32
+
+
 def check_direct(M, K, N, fp4, shape, rows):
     """The operands of the few-rows kernel (csrc/gemm_direct_kernel.h) in tiles of 32 `shape` rows."""
     M_pad, kgroups = (M + 255) // 256 * 256, K // 64
@@ -130,6 +146,13 @@ def check_direct(M, K, N, fp4, shape, rows):
                 for cw in range(WN):
                     for nt in range(NT):
                         if fp4:
+                            # as buffers: size, lane's offset, scalar offset
+                            s_lead, a_lead = (nb * 128 + cw * NT * 32) * 8, f0 * 32 * 4
+                            buffer_read(NT * kgroups * TILE, 31 * 32 + 16, g * TILE + nt * kgroups * TILE, 16, wgt_bytes - (nb * 4 + cw * NT) * kgroups * TILE)
+                            buffer_read(kgroups * N * 8 - s_lead, 31 * 8 + 4 + nt * 256, g * N * 8, 4, wsc_bytes - s_lead)
+                            for mt in range(MT):
+                                buffer_read(MT * kgroups * TILE, 31 * 32 + 16, g * TILE + mt * kgroups * TILE, 16, act_bytes - f0 * kgroups * TILE)
+                                buffer_read(kgroups * M_pad * 4 - a_lead, 31 * 4 + 2 + mt * 128, g * M_pad * 4, 2, asc_bytes - a_lead)
                             assert ((nb * 4 + cw * NT) * kgroups + g) * TILE + nt * kgroups * TILE + 31 * 32 + 16 + 16 <= wgt_bytes
                             assert (g * N + nb * 128 + cw * NT * 32) * 8 + nt * 256 + 31 * 8 + 4 + 4 <= wsc_bytes
                         else:
@@ -197,9 +220,9 @@ def test_projecting_workgroups_read_inside_proj_down():
 @pytest.mark.parametrize("glu", [False, True])
 def test_quantize_row_buffer_cuts_exactly_at_the_last_row(glu):
     """The kernel reads x through a raw buffer whose size (num_records) ends with the workgroup's last valid row, and
-    carries the 128-column chunk in the scalar offset.  The hardware's range check for a raw buffer compares the lane
-    offset plus the access size with num_records and ignores the scalar offset, so a lane reads memory if and only
-    if its row is valid (and the chunk exists: past the last chunk the kernel sets bit 31 of the lane offset)."""
+    carries the 128-column chunk in the scalar offset.  Whether the hardware's range check counts the scalar offset or not, a
+    lane reads memory if and only if its row is valid (and the chunk exists: past the last chunk the kernel sets bit 31
+    of the lane offset)."""
     XW = 2 if glu else 1
     PPR, RPI = 16 * XW, 64 // (16 * XW)
     for K in (128, 256, 1152, 3072, 12288):
@@ -220,6 +243,7 @@ def test_quantize_row_buffer_cuts_exactly_at_the_last_row(glu):
                                 voff += (16 * mt + RPI * i) * ld * 2
                                 in_range = voff + 16 <= num_records
                                 assert in_range == (row < rv and c < nchunks), (K, MT, rows_valid, c, mt, i, lane)
+                                assert in_range == (voff + soffset + 16 <= num_records) and voff + soffset < 1 << 32
                                 if in_range:  # the bytes a lane in range touches belong to its row and chunk
                                     first = voff + soffset
                                     assert row * ld * 2 + c * 256 * XW <= first and first + 16 <= row * ld * 2 + (c + 1) * 256 * XW
@@ -243,3 +267,103 @@ def test_quantize_store_addresses():
                     rts = min(R // 16 - rt_base, 8)
                     for rank in (0, 16 * rts - 1):
                         assert row * R + 16 * rt_base + rank < lora_elems
+
+
+@pytest.mark.parametrize("R", [16, 32, 48, 128, 144, 256, 1024])
+def test_low_rank_operands_stay_inside_their_buffers(R):
+    """The operands of the up projection, lora_act [M_pad][R] fp32 and lora_up [N][R] bf16.  INT4 (csrc/gemm6_kernel.h, request_chunk):
+    chunks of 32 ranks by asynchronous copies, 64 bytes of each of 256 columns and 128 bytes of each of 64 MT rows; columns beyond N
+    repeat the last, half a chunk repeats its 16 ranks.  NVFP4 (csrc/gemm_kernel.h, request): windows of 128 ranks, 32 at a time."""
+    steps = R // 16
+    for N in (128, 256, 384, 640):
+        for n0 in range(0, N, 256):
+            for c in range((steps + 1) // 2):
+                half = steps - 2 * c < 2
+                pieces, places = set(), {}
+                for wave in range(4):
+                    for i in range(4):
+                        for lane in range(64):
+                            row = (wave * 4 + i) * 16 + (lane >> 2)
+                            piece = (lane & 3) ^ ((row >> 2) & 3)
+                            column = n0 + (row if n0 + row < N else N - 1 - n0)
+                            first = column * R * 2 + c * 64 + (piece & 1 if half else piece) * 16
+                            assert column * R * 2 <= first and first + 16 <= (column + 1) * R * 2 <= N * R * 2
+                            place = (wave * 4 + i) * 1024 + lane * 16
+                            assert place not in places and place == row * 64 + (piece ^ ((row >> 2) & 3)) * 16
+                            places[place] = (row, piece)
+                            pieces.add((row, piece))
+                assert len(pieces) == 256 * 4
+    for MT in (1, 2):
+        for M_pad in (256, 512):
+            for m0 in range(0, M_pad, 64 * MT):
+                for c in range((steps + 1) // 2):
+                    half = steps - 2 * c < 2
+                    pieces = set()
+                    for wave in range(4):
+                        for i in range(2 * MT):
+                            for lane in range(64):
+                                row = (wave * 2 * MT + i) * 8 + (lane >> 3)
+                                piece = (lane & 7) ^ ((row >> 1) & 7)
+                                first = (m0 + row) * R * 4 + c * 128 + (piece & 3 if half else piece) * 16
+                                assert first + 16 <= (m0 + row + 1) * R * 4 <= M_pad * R * 4
+                                assert (wave * 2 * MT + i) * 1024 + lane * 16 == row * 128 + (piece ^ ((row >> 1) & 7)) * 16
+                                pieces.add((row, piece))
+                    assert len(pieces) == 64 * MT * 8
+    for first in range(0, steps, 8):
+        window, seen = min(steps - first, 8), set()
+        for c in range((window + 1) // 2):
+            for lane in range(64):
+                step = first + 2 * c + (1 if lane & 4 and 2 * c + 1 < window else 0)
+                up_step = first + 2 * c + (1 if lane & 2 and 2 * c + 1 < window else 0)
+                assert 16 * step + (lane & 3) * 4 + 4 <= R and 16 * up_step + (lane & 1) * 8 + 8 <= R
+                for place, limit in ((2 * c + ((lane & 4) >> 2), "act"), (2 * c + ((lane & 2) >> 1), "up")):
+                    if place < window:  # (what is written to LDS is what was requested)
+                        assert first + place == (step if limit == "act" else up_step)
+                        seen.add((limit, place))
+        assert seen == {(name, place) for name in ("act", "up") for place in range(window)}
+
+
+@pytest.mark.parametrize("N,K,ncu", [(16, 640, 256), (20, 1088, 256), (4092, 640, 256), (9220, 640, 256), (18432, 3072, 256), (24572, 640, 256), (20480, 4096, 304),
+                                     ((1 << 24) - 4, 4096, 256)])
+def test_awq_shares_read_inside_their_buffers(N, K, ncu):
+    """The AWQ GEMV with one workgroup per compute unit: the shares cover the channels once; a lane whose channel is the share's reads its
+    codes, scale and zero, any other (the share's last tile, the tiles requested ahead) nothing."""
+    kblocks, BATCH, AHEAD = K // 64, 6, 2
+    assert kblocks * N < 1 << 30  # (the launcher's condition)
+    spw = ((K + 127) // 128 + 7) // 8
+    grid = min((N + 15) // 16, ncu)
+    share, more, covered = N // 4 // grid, N // 4 % grid, 0
+    for wg in range(grid):
+        begin = 4 * (wg * share + min(wg, more))
+        end = begin + 4 * (share + (1 if wg < more else 0))
+        assert begin == covered
+        covered = end
+        if wg not in (0, 1, more - 1, more, grid - 2, grid - 1):
+            continue
+        tiles = (end - begin + 15) // 16
+        requested = list(range(AHEAD))
+        for t0 in range(0, tiles, BATCH):
+            requested += [t0 + i + AHEAD for i in range(min(tiles - t0, BATCH))]
+        assert set(range(tiles)) <= set(requested)
+        w_size, s_size = (end - begin) // 4 * kblocks * 128, kblocks * N * 2
+        assert w_size < 1 << 31 and s_size < 1 << 31
+        for t in {0, 1, tiles - 1, tiles, tiles + 1} & set(requested):
+            for n in range(16):
+                for j in (0, spw - 1):
+                    for wave in (0, 7):
+                        for kb in range(4):
+                            cb = (wave + 8 * j) * 2 + (kb >> 1)
+                            block = min(cb, kblocks - 1)
+                            w_off = (n >> 2) * kblocks * 128 + (n & 3) * 32 + (kb & 1) * 16 + block * 128
+                            s_off = block * N * 2 + n * 2
+                            wt, st = t * kblocks * 512, (begin + 16 * t) * 2
+                            channel = begin + 16 * t + n
+                            if channel < end:
+                                buffer_read(w_size, w_off, wt, 16, N // 4 * kblocks * 128 - begin // 4 * kblocks * 128)
+                                buffer_read(s_size, s_off, st, 2, s_size)
+                                assert begin // 4 * kblocks * 128 + w_off + wt == ((channel // 4 * kblocks + block) * 4 + channel % 4) * 32 + (kb & 1) * 16
+                                assert (s_off + st) // 2 == block * N + channel
+                            else:
+                                buffer_skip(w_size, w_off | 0x80000000, wt)
+                                buffer_skip(s_size, s_off | 0x80000000, st)
+    assert covered == N
