@@ -68,8 +68,10 @@ __device__ inline void store_result(const AwqParams &p, int m, int row, float su
 // K = 3072, N = 9216, one row 8.5 / 8.0.  About 3 us of that are launch and latency, the rest 4.2 TB/s.  Further ahead is slower
 // (three tiles 11.7, four 12.4), two workgroups of half the tiles per compute unit too (13.0).
 // Equal shares of the channels (N = 18432 is 4.5 tiles per workgroup, which were 4 or 5), no requests behind a share's end (the tiles
-// requested ahead made 40 % more of them) and one division in place of two of 64 bits, in a graph of eight layers in turn, before / now:
-// K = 3072, N = 18432 one row 10.4 / 10.0 us, eight 11.5 / 11.1; N = 9216 7.5 / 7.0; N = 3072, four rows 5.2 / 4.7; K = 1024, N = 2048 2.77 / 2.70.
+// requested ahead made 40 % more of them) and one division in place of two of 64 bits, in a graph of layers in turn that hold 520 MB together,
+// twice the memory-side cache, before / now: K = 3072, N = 18432 one row 10.5 / 10.1 us (3.1 TB/s), four 10.7 / 10.7, eight 11.5 / 11.2; N = 9216
+// 7.9 / 7.4; N = 3072, four rows 5.5 / 5.0; K = 4096, N = 20480 13.5 / 13.2, eight rows 15.0 / 14.4; K = 1024, N = 2048 3.3 / 3.1.  One layer again and again
+// (its weights in that cache): K = 3072, N = 18432 8.4 / 8.2, 9.6 / 9.4 and 10.1 / 9.9.
 constexpr int WAVES = 8, BATCH = 6, AHEAD = 2;
 static_assert(BATCH % (AHEAD + 1) == 0, "the ring of register sets is indexed by the position in a batch");
 template <int SPW>

@@ -265,7 +265,8 @@ int add_shares(const P &p, int nshares, int vk_block, int full_rows, hipStream_t
 // 5.3 + 2.6 per part beyond the first (four parts, whose last one keeps its own sums in registers: 11.5), half as much
 // again when compute units are shared.  Measured, whole / best split: 24 tiles at K = 3072 31.2 / 22.5 (4 parts; 3
 // parts 24.2), 72 tiles 31.3 / 27.3 (3), 96 tiles 31.8 / 31.0 (2; not split), 144 tiles 32.1 / 38.1 (not split);
-// K = 12288: 24 tiles 105.9 / 39.6 (6), 72 tiles 105.6 / 51.7 (3), 144 tiles 106.2 / 78.4 (3).
+// K = 12288: 24 tiles 105.9 / 39.6 (6), 72 tiles 105.6 / 51.7 (3), 144 tiles 106.2 / 78.4 (3).  (The price of a split is that of requests made lane by lane;
+// since they have scalar descriptors it is up to 1.4 us less, M = 856, K = 4992, N = 2432 in three parts 30.7 -> 29.5.)
 // `time`: the model's time in us for the choice where there is one.
 int choose_kparts(int ntiles, int kgroups, int ncu, double *time) {
     *time = 0.0;
@@ -609,8 +610,10 @@ int gemm_fp4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t st
 // K.  Shape 2: tiles of 64 rows, a quarter fewer operand bytes per product, from about 400 tiles of 32 rows on; INT4: two waves
 // split K and two the columns, NVFP4: four waves split K.  Models of the time in us fitted to launches at K = 1024 ... 12288
 // on 256 compute units, linear in the number of tiles that the busiest compute unit works through and in the k-groups; they meet
-// the measurements within about 10 %.  Over 2200 random shapes the choice takes 0.6 % (NVFP4) and 0.3 % (INT4) longer than the fastest
-// of the three, and is more than 3 % slower than the large tiles in 17, 14 of them short rows whose large tiles would be shared (below).  Measured at K = 3072, large tiles (split along K where that pays) / shape 1 / shape 2:
+// the measurements within about 10 %.  When they were fitted the choice took 0.6 % (NVFP4) and 0.3 % (INT4) longer than the fastest of the
+// three over 2200 random shapes, and was more than 3 % slower than the large tiles in 17, 14 of them short rows whose large tiles would be shared
+// (below); with the kernels as they are now it is 1.6 % (NVFP4, 316 shapes) and 0.8 % (INT4, 323).  A refit of the NVFP4 side gives 0.1 %, and
+// moves choices at 4608 rows.  Measured at K = 3072 at the time of the fit, large tiles (split along K where that pays) / shape 1 / shape 2:
 //   INT4   M = 256, N = 3072   22.8 /  9.6 / 12.3     NVFP4  60.7 / 11.8 / 13.8
 //          M = 505, N = 9216   28.7 / 33.1 / 30.6            62.9 / 38.4 / 34.1
 //          M = 1157, N = 3072  29.7 / 27.6 / 21.8            62.1 / 31.7 / 25.7
@@ -620,8 +623,8 @@ int gemm_fp4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t st
 //   K = 12288, N = 3072: M = 256  42.1 / 24.8 / 34.4           113.6 / 30.8 / 35.0
 //          M = 505             45.4 / 44.1 / 34.6           115.2 / 50.8 / 37.9
 //          M = 1157            66.6 / 86.6 / 65.6           127.5 / 99.5 / 81.2
-// (Measured when the models were fitted.  Since then the INT4 large tiles have become 3 to 9 % faster, M = 505, N = 9216 25.3, and NVFP4 in the
-// few-rows kernel as much, M = 1157, K = 12288 76.4: the INT4 choice still takes 0.8 % longer than the fastest over 323 shapes, the NVFP4 one 1.6 %.)
+// (Since then: INT4 large tiles 3 to 10 % faster, M = 505, N = 9216 24.9, M = 1024, N = 9216 32.3; NVFP4 large tiles with the quantizing epilogue M = 1157,
+// N = 12288 100; NVFP4 in the few-rows kernel M = 1157, K = 12288 76.4.)
 int choose_direct(const svdq_gemm_args *a, int ncu) {
     if (a->k_split > 0) return 0;  // (the caller asks for the tiles that k_split is about)
     if (((uintptr_t)a->bias | (uintptr_t)a->wcscales | (uintptr_t)a->oscales) % 8 || (uintptr_t)a->colnorm % 16) return 0;  // (read four columns at a time)

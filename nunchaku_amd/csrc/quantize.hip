@@ -321,8 +321,9 @@ __global__ void __launch_bounds__(64 * NW) quantize_fuse_lora_kernel(QuantParams
 
         // ---- smooth, quantize, store
         // (rounded one by one, an instruction each, instead of in pairs that have to be taken apart again: K = 12288, M = 1157 17.7 -> 16.9
-        // us; K = 15360, NVFP4, M = 4608 45.7 -> 44.8; rank 64, K = 3072, M = 4608 16.2 -> 16.0.  Not in the one form that came out
-        // slower, INT4, M = 4608, K = 3072, rank 32 11.6 -> 11.9.)
+        // us; K = 15360, NVFP4, M = 4608 45.7 -> 44.8; rank 64, K = 3072, M = 4608 16.2 -> 16.0.  The INT4 form with 32 rows and two rank tiles
+        // stays in pairs: there it depends on the row length, and over 18 sizes the two are equal (M = 4608, in pairs / one by one: K = 2048 8.7 / 8.9,
+        // 3072 11.7 / 12.0, 4096 17.1 / 16.8, 6144 18.9 / 19.0, 8192 26.8 / 26.4, 12288 33.5 / 33.4; M = 8192, K = 3072 15.2 / 15.3, 2304 13.0 / 12.8).)
         constexpr bool PACKED_ROUNDING = !FP4 && MT == 2 && RT_MAX == 2;
 #pragma unroll
         for (int mt = 0; mt < (QUANT ? MT : 0); mt++) {
