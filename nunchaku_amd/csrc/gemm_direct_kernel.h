@@ -3,17 +3,18 @@
 //
 // The kernels with 128 x 256 and 256 x 256 tiles need thousands of rows to occupy the chip: with a few hundred, a
 // layer of N = 3072 is 24 or 12 such tiles, each walking K alone on its compute unit.  Here a workgroup of four waves owns
-// a tile of 32 MT rows x 128 columns; its waves split the columns WN ways and take the k-groups g = part, part + KP, ...
+// a tile of 32 MT rows x 32 NT WN columns; its waves split the columns WN ways and take the k-groups g = part, part + KP, ...
 // of their part of K in turn, and the parts' sums meet in LDS at the end.  An operand fragment is contiguous in memory in
 // the lanes' order (svdq_common.h), so a wave fetches it with one or two wide loads, DEPTH of its k-groups ahead, and
 // neither LDS nor barriers appear in the main loop.
-// What bounds it: with one workgroup per compute unit, no single resource.  M = 256, K = N = 3072 (192 workgroups): a wave takes 0.41 us
-// per k-group, about one memory latency, with one k-group on its way (INT4, 32 rows; two in NVFP4); of the waves' cycles 27 % are
-// waits for operands, 29 % waits to issue behind the matrix core, 28 % vector instructions (NVFP4, M = 300: 33, 13 and 41 %).  84 % of
-// the operand requests hit in the L2s, which hand out 2.15 KB per 32 x 32 tile and k-group with one row block and four column tiles
-// per wave, 1.65 KB with two of each (82 GB/s per compute unit, 64 bytes per clock being about 150).  With several tiles per compute
-// unit the matrix core and the conversions are (M = 1157, K = 12288, NVFP4: 10 % waits for operands, 49 and 34 % the others).
-// M = 256, K = N = 3072: 22.8 -> 8.8 us (INT4; 4.2 us of it do not depend on K), 59.9 -> 10.6 us (NVFP4).
+// What bounds it where compute units have one tile or two: the vector memory path of a compute unit.  It hands out 120 GB/s to requests of
+// 16 bytes a lane and 80 to those of 8 (operands in the L2, 48 or 192 compute units at work, 4, 8 or 16 waves each: the same), so that a
+// k-group of an INT4 tile of 32 x 128 takes 90 ns, its five fragments 75 of them, and neither more waves nor more k-groups on their way change
+// that (eight waves 9.9, three k-groups 9.5 to 10.9 against 8.6 us, M = 256, K = N = 3072).  Plain epilogues therefore choose among six tiles, see
+// plain_tile in gemm.hip: square ones fetch least per product, small ones use more compute units.  The others have 128 columns, which a
+// head of the norm and a chunk of the next layer's projection have.  With several tiles per compute
+// unit the matrix core and the conversions bound it (M = 1157, K = 12288, NVFP4: 10 % waits for operands, 49 and 34 % the others).
+// M = 256, K = N = 3072: 22.8 -> 8.8 -> 7.9 us (INT4; 4 us of it do not depend on K), 59.9 -> 10.6 -> 9.4 us (NVFP4); M = 64: 8.6 -> 5.6 and 9.7 -> 5.5.
 //
 // INT4: one fp6 matrix instruction on the codes, one factor instruction and 16 multiply-adds per 32 x 32 tile and
 // k-group (gemm6_kernel.h).  NVFP4: both operands are dequantized to fp16 in registers by the wave that uses them
@@ -25,7 +26,7 @@
 // conversions a step ahead: M = 256 45.5 / 39.6 / 35.0 us, M = 1157 91.7 / 84.3 / 81.2 (76.4 with buffers, below); from two tiles per compute unit on 1.2
 // PFLOP/s, where the large kernel's 1.25 is the power limit.
 //
-// The epilogue is shared out by columns: wave w of four adds up the parts' sums of the 32 columns 32 w ... of the tile
+// The epilogue is shared out by columns (tiles narrower than 128: by blocks of 32 x 32): wave w of four adds up the parts' sums of the 32 columns 32 w ... of the tile
 // in ascending order, projects the low-rank branch onto them and applies bias, norm, rotation and activation; the
 // bf16 tile meets in LDS again and all waves store it, project and quantize it for the next layer.
 #pragma once
@@ -53,16 +54,20 @@ struct Stage<true, MT, NT> {
 constexpr int SLAB_BYTES = 32 * OUT_LD * 2;
 // LDS: the waves' sums of 32 rows x 128 columns, [KP][4 column tiles][4 quads][64 lanes] x float4; behind them the sums of
 // squares of the RMS norm, [MT][4][32] floats.  The bf16 slabs take the place of the sums.
-template <int MT, int KP>
+// Tiles narrower than 128 columns: the sums of all row blocks at once, and a slab of its own for every wave behind them.
+constexpr int NARROW_LD = 40, NARROW_SLAB_BYTES = 32 * NARROW_LD * 2;
+template <int MT, int NC, int KP>
 constexpr int lds_bytes() {
-    return KP * 16384 + MT * 512;
+    return NC == 4 ? KP * 16384 + MT * 512 : KP * MT * NC * 4096 + MT * NC * NARROW_SLAB_BYTES;
 }
 
-template <bool FP4, int MT, int WN, int KP, int DEPTH, bool NEXT>
+template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT>
 __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams p) {
-    constexpr int NT = 4 / WN;  // 32-column tiles of a wave
+    constexpr int NC = NT * WN;  // 32-column tiles of the workgroup; a wave has NT of them
     constexpr int WAVES = WN * KP;
-    static_assert(WAVES == 4, "the epilogue gives each wave one column tile");
+    constexpr bool NARROW = NC < 4;
+    static_assert(WAVES == 4 && MT * NC <= (NARROW ? 4 : 8), "the epilogue gives each wave one column tile, of one row block where the tile is narrow");
+    static_assert(!NARROW || !NEXT, "the norm, the rotation and the next layer's operands need whole 128-column blocks");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -75,7 +80,7 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
     const int total = (int)gridDim.x, xcd = (int)blockIdx.x % 8, extra = total % 8;
     const int v = xcd * (total / 8) + (xcd < extra ? xcd : extra) + (int)blockIdx.x / 8;
     const int nb = v / p.row_blocks, mb = v - nb * p.row_blocks;
-    const int n0 = nb * 128, f0 = mb * MT;  // first column; first 32-row block
+    const int n0 = nb * (32 * NC), f0 = mb * MT;  // first column; first 32-row block
 
     // ---- operands ----------------------------------------------------------------------------------
     // (DEPTH + 1 register sets, indexed by compile-time constants.  The lambdas below reach them through their captures: taken
@@ -92,8 +97,10 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
     const uint8_t *wp, *sp, *xp[MT];
     const uint16_t *ap;
     if constexpr (!FP4) {
-        wp = p.wgt + ((size_t)(nb >> 1) * kgroups + g_load) * (8 * FRAG_BYTES) + ((nb & 1) * 4 + cw * NT) * FRAG_BYTES;
-        sp = (const uint8_t *)p.wscales + ((size_t)(nb >> 1) * kgroups + g_load) * 2048 + (nb & 1) * 1024 + cw * (NT * 256);
+        constexpr int PER256 = 8 / NC;  // tiles of this width in the 256 columns that the operands are laid out by
+        const int blk = nb / PER256, tile0 = nb % PER256 * NC + cw * NT;
+        wp = p.wgt + ((size_t)blk * kgroups + g_load) * (8 * FRAG_BYTES) + tile0 * FRAG_BYTES;
+        sp = (const uint8_t *)p.wscales + ((size_t)blk * kgroups + g_load) * 2048 + tile0 * 256;
         each(std::make_integer_sequence<int, MT>{}, [&](auto I) {
             constexpr int mt = decltype(I)::value;
             xp[mt] = p.act + ((size_t)((f0 + mt) >> 2) * kgroups + g_load) * (4 * FRAG_BYTES) + ((f0 + mt) & 3) * FRAG_BYTES;
@@ -105,7 +112,7 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
     const uint32_t tile_stride = (uint32_t)kgroups * TILE_BYTES;  // NVFP4: from one 32-column (or 32-row) tile to the next
     auto buffer = [](const void *base, uint32_t bytes) { return __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (int)bytes, 0x00020000); };
     const uint32_t s_group = (uint32_t)p.N * 8, a_group = (uint32_t)p.M_pad * 4, s_lead = (n0 + cw * (NT * 32)) * 8, a_lead = f0 * 32 * 4;
-    const __amdgpu_buffer_rsrc_t wrsrc = buffer(p.wgt + (size_t)(nb * 4 + cw * NT) * kgroups * TILE_BYTES, NT * tile_stride);
+    const __amdgpu_buffer_rsrc_t wrsrc = buffer(p.wgt + (size_t)(nb * NC + cw * NT) * kgroups * TILE_BYTES, NT * tile_stride);
     const __amdgpu_buffer_rsrc_t xrsrc = buffer(p.act + (size_t)f0 * kgroups * TILE_BYTES, MT * tile_stride);
     const __amdgpu_buffer_rsrc_t srsrc = buffer((const uint8_t *)p.wscales + s_lead, kgroups * s_group - s_lead);
     const __amdgpu_buffer_rsrc_t arsrc = buffer((const uint8_t *)p.ascales + a_lead, kgroups * a_group - a_lead);
@@ -150,6 +157,7 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
 #pragma unroll
         for (int e = 0; e < 16; e++) acc[t][e] = 0.f;
     // INT4: products and factors of two tiles, one being multiplied while the other is accumulated
+    constexpr bool LAG = MT * NT > 1;  // (a single tile per k-group is accumulated at once)
     float16_t P[FP4 ? 1 : 2], F[FP4 ? 1 : 2];
 #pragma unroll
     for (int b = 0; b < (FP4 ? 1 : 2); b++)
@@ -179,7 +187,7 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
                 P[b] = mfma_codes6(st.w[nt], st.x[mt]);
                 F[b] = mfma_factor(u32x2_t{st.ws[nt], 0u}, u32x2_t{h ? 0u : st.as[mt], 0u});
 #pragma unroll
-                for (int e = 0; e < 16; e++) acc[prev][e] = __builtin_fmaf(P[b ^ 1][e], F[b ^ 1][e], acc[prev][e]);
+                for (int e = 0; e < 16; e++) acc[prev][e] = __builtin_fmaf(P[LAG ? b ^ 1 : b][e], F[LAG ? b ^ 1 : b][e], acc[prev][e]);
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -239,24 +247,29 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
     if constexpr (DEPTH > 1) {
         if (g < kgroups) step(std::integral_constant<int, 1>{});
     }
-    if constexpr (!FP4) {
+    if constexpr (DEPTH > 2) {
+        if (g < kgroups) step(std::integral_constant<int, 2>{});
+    }
+    if constexpr (!FP4 && LAG) {
 #pragma unroll
         for (int e = 0; e < 16; e++) acc[NT * MT - 1][e] = __builtin_fmaf(P[1][e], F[1][e], acc[NT * MT - 1][e]);
     }
 
     // ---- the epilogue's own operands, requested before the waves meet ------------------------------------
-    // Wave w gets the 32 columns 32 w ... of all MT row blocks.
-    const int nt = wave, c0 = n0 + nt * 32, row0 = f0 * 32;
+    // Wave w gets the 32 columns 32 w ... of all MT row blocks; of a narrow tile one of the MT NC blocks of 32 x 32, where there is one.
+    constexpr int OWN = NARROW ? 1 : MT;
+    const bool owner = !NARROW || wave < MT * NC;
+    const int nt = NARROW ? wave % NC : wave, c0 = n0 + nt * 32, row0 = f0 * 32 + (NARROW ? wave / NC * 32 : 0);
     const int nsteps = p.R_up / 16;
     constexpr int LSTEPS = 2;  // 16-rank steps of the low-rank up projection requested at once
-    float4_t la_raw[MT][LSTEPS][2];
+    float4_t la_raw[OWN][LSTEPS][2];
     u32x4_t up_raw[LSTEPS];
     auto load_lora = [&](int s0) {
 #pragma unroll
         for (int s = 0; s < LSTEPS; s++) {
             const int step = s0 + s < nsteps ? s0 + s : nsteps - 1;
 #pragma unroll
-            for (int o = 0; o < MT; o++) {
+            for (int o = 0; o < OWN; o++) {
                 const float4_t *ap = (const float4_t *)(p.lora_act + (size_t)(row0 + o * 32 + r32) * p.R_up + 16 * step + 8 * h);
                 la_raw[o][s][0] = ap[0];
                 la_raw[o][s][1] = ap[1];
@@ -265,9 +278,10 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
         }
     };
     float cf[4][4], bs[4][4];  // factor and bias of the lane's columns c0 + 8 q + 4 h + i
-    if (nsteps > 0) load_lora(0);
+    if (owner && nsteps > 0) load_lora(0);
 #pragma unroll
     for (int q = 0; q < 4; q++) {
+        if (!owner) break;
         const int c = c0 + 8 * q + 4 * h;
         const float4_t cn = FP4 ? *(const float4_t *)(p.colnorm + c) : float4_t{1.f, 1.f, 1.f, 1.f};
         const u32x2_t wc = p.wcscales ? *(const u32x2_t *)(p.wcscales + c) : u32x2_t{0x3F803F80u, 0x3F803F80u};
@@ -280,33 +294,53 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
     }
 
     // ---- the waves' sums meet, 32 rows at a time, added in ascending order of the waves ---------------------
-    float16_t val[MT];
+    float16_t val[OWN];
     float4_t *park = (float4_t *)lds;
+    if constexpr (NARROW) {
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-        if (mt > 0) __syncthreads();
-#pragma unroll
-        for (int t = 0; t < NT; t++)
+        for (int t = 0; t < NT * MT; t++) {
+            const int tile = t % MT * NC + cw * NT + t / MT;
 #pragma unroll
             for (int q = 0; q < 4; q++)
-                park[((kpart * 4 + cw * NT + t) * 4 + q) * 64 + lane] =
-                    float4_t{acc[t * MT + mt][4 * q], acc[t * MT + mt][4 * q + 1], acc[t * MT + mt][4 * q + 2], acc[t * MT + mt][4 * q + 3]};
+                park[((kpart * (MT * NC) + tile) * 4 + q) * 64 + lane] = float4_t{acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]};
+        }
         __syncthreads();
+        if (!owner) return;
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            float4_t s = park[(nt * 4 + q) * 64 + lane];
+            float4_t s = park[(wave * 4 + q) * 64 + lane];
 #pragma unroll
-            for (int j = 1; j < KP; j++) s += park[((j * 4 + nt) * 4 + q) * 64 + lane];
+            for (int j = 1; j < KP; j++) s += park[((j * (MT * NC) + wave) * 4 + q) * 64 + lane];
 #pragma unroll
-            for (int i = 0; i < 4; i++) val[mt][4 * q + i] = s[i];
+            for (int i = 0; i < 4; i++) val[0][4 * q + i] = s[i];
         }
+    } else {
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            if (mt > 0) __syncthreads();
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    park[((kpart * 4 + cw * NT + t) * 4 + q) * 64 + lane] =
+                        float4_t{acc[t * MT + mt][4 * q], acc[t * MT + mt][4 * q + 1], acc[t * MT + mt][4 * q + 2], acc[t * MT + mt][4 * q + 3]};
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                float4_t s = park[(nt * 4 + q) * 64 + lane];
+#pragma unroll
+                for (int j = 1; j < KP; j++) s += park[((j * 4 + nt) * 4 + q) * 64 + lane];
+#pragma unroll
+                for (int i = 0; i < 4; i++) val[mt][4 * q + i] = s[i];
+            }
+        }
+        __syncthreads();  // the sums have been read: the slabs take their place
     }
-    __syncthreads();  // the sums have been read: the slabs take their place
 
     float *ssq = (float *)(lds + KP * 16384);  // [MT][4 column tiles][32 rows]
     const bool rope = NEXT && p.rotary && n0 < p.rope_cols;  // the tile is one head of q or k
 #pragma unroll
-    for (int o = 0; o < MT; o++)
+    for (int o = 0; o < OWN; o++)
 #pragma unroll
         for (int e = 0; e < 16; e++) val[o][e] *= cf[e >> 2][e & 3];
     // Low-rank up projection (lora.cuh:110-241): out += bf16(lora_act * scale) @ up^T
@@ -317,7 +351,7 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
             if (s0 + s >= nsteps) break;
             const float ls = p.lora_scales[s0 + s];
 #pragma unroll
-            for (int o = 0; o < MT; o++) {
+            for (int o = 0; o < OWN; o++) {
                 const float4_t v0 = la_raw[o][s][0], v1 = la_raw[o][s][1];
                 u32x4_t w;
                 w[0] = pack_bf16x2(v0[0] * ls, v0[1] * ls);
@@ -329,9 +363,29 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
         }
     }
 #pragma unroll
-    for (int o = 0; o < MT; o++)
+    for (int o = 0; o < OWN; o++)
 #pragma unroll
         for (int e = 0; e < 16; e++) val[o][e] += bs[e >> 2][e & 3];
+    if constexpr (NARROW) {
+        // the wave's 32 x 32 block through its own slab, in rows of 64 contiguous bytes
+        uint16_t *slab = (uint16_t *)(lds + KP * MT * NC * 4096 + wave * NARROW_SLAB_BYTES);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            u32x2_t w;
+            w[0] = pack_bf16x2(val[0][4 * q], val[0][4 * q + 1]);
+            w[1] = pack_bf16x2(val[0][4 * q + 2], val[0][4 * q + 3]);
+            *(u32x2_t *)(slab + r32 * NARROW_LD + 8 * q + 4 * h) = w;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the slab is the wave's own, whose LDS operations complete in order)
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int it = 0; it < 2; it++) {
+            const int rr = it * 16 + (lane >> 2), cc = (lane & 3) * 8, m = row0 + rr, n = c0 + cc;
+            const u32x4_t d = *(const u32x4_t *)(slab + rr * NARROW_LD + cc);
+            if (p.out && m < p.M_out && n < p.N_out) __builtin_nontemporal_store(d, (u32x4_t *)(p.out + (size_t)m * p.N_out + n));
+        }
+        return;
+    } else {
     if (rope) {
 #pragma unroll
         for (int o = 0; o < MT; o++) {
@@ -479,12 +533,13 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
             *(u32x4_t *)(p.qout + ((size_t)(m / 32) * ngroups_out + gidx) * TILE_BYTES + (m % 32) * 32 + 16 * (qc & 1)) = words;
         }
     }
+    }
 }
 
-template <bool FP4, int MT, int WN, int KP, int DEPTH, bool NEXT>
+template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT>
 int launch_direct(const GemmParams &p, hipStream_t stream) {
-    auto kern = gemm_direct_kernel<FP4, MT, WN, KP, DEPTH, NEXT>;
-    constexpr int smem = lds_bytes<MT, KP>();
+    auto kern = gemm_direct_kernel<FP4, MT, NT, WN, KP, DEPTH, NEXT>;
+    constexpr int smem = lds_bytes<MT, NT * WN, KP>();
     static bool lds_reserved[64] = {false};  // set once per device (racing first calls both set it, which is harmless)
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(SVDQ_ELAUNCH, "gemm: cannot identify the current device");
@@ -493,7 +548,7 @@ int launch_direct(const GemmParams &p, hipStream_t stream) {
         if (e != hipSuccess) return fail(SVDQ_ELAUNCH, "gemm: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
         lds_reserved[dev] = true;
     }
-    SVDQ_LAUNCH(kern, dim3((unsigned)(p.row_blocks * (p.N / 128))), dim3(64 * WN * KP), smem, stream, p);
+    SVDQ_LAUNCH(kern, dim3((unsigned)(p.row_blocks * (p.N / (32 * NT * WN)))), dim3(64 * WN * KP), smem, stream, p);
     return check_launch("gemm_w4a4 (few rows)");
 }
 

@@ -1,0 +1,81 @@
+"""The few-rows GEMM's tiles with the plain epilogue (csrc/gemm.hip, ``plain_tile``; csrc/gemm_narrow_variant.hip) on the CPU: which one
+a launch takes, that no operand is read outside its buffer, and that the kernels keep out of scratch memory."""
+
+import ctypes
+
+import pytest
+
+from nunchaku_amd import _native as nv
+from plan_util import call
+from test_address_model import FRAG, buffer_read
+from test_build_guard import compiled  # noqa: F401  (the fixture)
+
+TILES = [(32, 32), (32, 64), (64, 32), (64, 64), (32, 128), (64, 128)]
+
+
+def plain_tile(M, K, N, fp4, compute_units=256):
+    rows, columns = ctypes.c_int32(), ctypes.c_int32()
+    nv.check(nv.lib().svdq_gemm_plain_tile_of(ctypes.byref(call("plain", M, K, N, 32, fp4)), compute_units, ctypes.byref(rows), ctypes.byref(columns)))
+    return rows.value, columns.value
+
+
+# (shape, the tile on 256 compute units; the same for both precisions)
+@pytest.mark.parametrize("M,K,N,want", [
+    (16, 1024, 1024, (32, 32)), (64, 3072, 3072, (32, 32)), (64, 12288, 3072, (32, 32)), (32, 3072, 12288, (32, 64)), (128, 3072, 3072, (64, 32)),
+    (256, 3072, 3072, (64, 64)), (300, 3072, 3072, (64, 64)), (256, 12288, 3072, (64, 64)), (89, 2432, 20480, (32, 128)), (1157, 12288, 3072, (64, 128)),
+])
+@pytest.mark.parametrize("fp4", [False, True])
+def test_the_tile_of_a_launch(M, K, N, want, fp4):
+    assert plain_tile(M, K, N, fp4) == want
+
+
+def check_addresses(M, K, N, fp4, MT, NC):
+    """The requests of the first and the last k-group of every wave (four of them split K) for every tile of a launch."""
+    M_pad, kgroups, TILE = (M + 255) // 256 * 256, K // 64, 1024
+    row_blocks, column_blocks = (M + 32 * MT - 1) // (32 * MT), N // (32 * NC)
+    act_bytes, asc_bytes = (M_pad * K // 2, kgroups * M_pad * 4) if fp4 else (M_pad * K * 3 // 4, kgroups * M_pad * 2)
+    padded = (N + 255) // 256 * 256  # (INT4 weights are stored in whole blocks of 256 columns)
+    wgt_bytes, wsc_bytes = (N * K // 2, kgroups * N * 8) if fp4 else (padded * K * 3 // 4, padded // 256 * kgroups * 2048)
+    total, seen = row_blocks * column_blocks, set()
+    for bid in range(total):
+        xcd, extra = bid % 8, total % 8
+        nb, mb = divmod(xcd * (total // 8) + min(xcd, extra) + bid // 8, row_blocks)
+        seen.add((nb, mb))
+        f0 = mb * MT
+        assert nb < column_blocks and (f0 + MT) * 32 <= M_pad
+        for g in {min(k, kgroups - 1) for k in range(4)} | {kgroups - 1, max(kgroups - 4, 0)}:
+            for mt in range(MT):
+                if fp4:
+                    a_lead = f0 * 32 * 4
+                    buffer_read(MT * kgroups * TILE, 31 * 32 + 16, g * TILE + mt * kgroups * TILE, 16, act_bytes - f0 * kgroups * TILE)
+                    buffer_read(kgroups * M_pad * 4 - a_lead, 31 * 4 + 2 + mt * 128, g * M_pad * 4, 2, asc_bytes - a_lead)
+                else:
+                    assert ((f0 + mt) // 4 * kgroups + g) * 4 * FRAG + (f0 + mt) % 4 * FRAG + 1024 + 63 * 8 + 8 <= act_bytes
+                    assert (g * M_pad + f0 * 32) * 2 + mt * 64 + 31 * 2 + 2 <= asc_bytes
+            for nt in range(NC):
+                if fp4:
+                    s_lead = nb * 32 * NC * 8
+                    buffer_read(NC * kgroups * TILE, 31 * 32 + 16, g * TILE + nt * kgroups * TILE, 16, wgt_bytes - nb * NC * kgroups * TILE)
+                    buffer_read(kgroups * N * 8 - s_lead, 31 * 8 + 4 + nt * 256, g * N * 8, 4, wsc_bytes - s_lead)
+                else:
+                    block, tile = divmod(nb * NC + nt, 8)
+                    assert divmod(nb, 8 // NC) == (block, (tile - nt) // NC)  # as the kernel has it
+                    assert (block * kgroups + g) * 8 * FRAG + tile * FRAG + 1024 + 63 * 8 + 8 <= wgt_bytes
+                    assert (block * kgroups + g) * 2048 + tile * 256 + 31 * 8 + 4 <= wsc_bytes
+    assert len(seen) == total
+
+
+@pytest.mark.parametrize("fp4", [False, True])
+def test_addresses_stay_inside_their_buffers(fp4):
+    for M, K, N in ((1, 128, 128), (33, 640, 384), (100, 3072, 768), (256, 3072, 3072), (300, 256, 1152), (769, 192 * 2, 640)):
+        for MT, NC in ((1, 1), (1, 2), (2, 1), (2, 2)):
+            check_addresses(M, K, N, fp4, MT, NC)
+
+
+@pytest.mark.parametrize("variant", [0, 1])
+def test_narrow_tiles_fit_their_registers(compiled, variant):  # noqa: F811
+    usage, _ = compiled[("gemm_narrow_variant.hip", variant)]
+    kernels = {k: u for k, u in usage.items() if "gemm_direct_kernel" in k}
+    assert len(kernels) == 4, list(usage)
+    for name, u in kernels.items():
+        assert u["VGPRs"] <= 256 and u["AGPRs"] == 0 and u["ScratchSize"] == 0 and u["Occupancy"] >= 2, (name, u)
