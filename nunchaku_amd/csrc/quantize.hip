@@ -55,6 +55,10 @@ struct TransposeArea {  // per wave: 16 rows of a chunk on their way from the lo
 // the kernel below the quantizer covers the latency of its operands).  x goes from whole-line requests to the operand layout
 // through the wave's transposition area `tr` as there (fetched in the operand layout, 16 rows x 64 bytes per instruction:
 // 7.1 us against 5.4 at M = 256, K = 3072); the waves' sums meet in `red` and are added in ascending order.
+// A chain of latencies: chunks beyond the end are neither requested nor walked through (whole turns of the ring, with zeros, took 4.1 us at
+// K = 1024 where it is 3.1 now, the same as quantizing alone), and three chunks are on their way where one rank tile leaves the registers
+// for it, all that a wave has at K = 3072 (4.2 -> 3.8 us; two rank tiles: one chunk, M = 1157, rank 128 9.0 -> 7.5).  Long rows are bound by the
+// 120 GB/s that a compute unit gets of x and proj_down (K = 12288: 786 KB, 8.6 us).
 template <int NW, int DEPTH, int RTW>
 __device__ __forceinline__ void project_rows(const QuantParams &p, int rt0, uint8_t *tr, float *red) {
     const int lane = threadIdx.x & 63;
@@ -81,26 +85,35 @@ __device__ __forceinline__ void project_rows(const QuantParams &p, int rt0, uint
         });
     };
     float4_t acc[2] = {float4_t{0.f, 0.f, 0.f, 0.f}, float4_t{0.f, 0.f, 0.f, 0.f}};
-    each(std::make_integer_sequence<int, DEPTH>{}, [&](auto D) { load(wave + decltype(D)::value * NW, D); });
-    // (chunks past the end multiply zeros: whole turns of the ring)
-    for (int c = wave; c < nchunks; c += (DEPTH + 1) * NW) {
+    each(std::make_integer_sequence<int, DEPTH>{}, [&](auto D) {
+        if (wave + decltype(D)::value * NW < nchunks) load(wave + decltype(D)::value * NW, D);
+    });
+    auto step = [&](auto S) {
+        constexpr int s = decltype(S)::value;
+        each(std::make_integer_sequence<int, 4>{}, [&](auto I) {
+            constexpr int i = decltype(I)::value;
+            const int row = 4 * i + lane / 16;
+            *(u32x4_t *)(tr + row * 256 + ((lane + rot(row)) % 16) * 16) = x[s][i];
+        });
+        each(std::make_integer_sequence<int, 4>{}, [&](auto I) {
+            constexpr int i = decltype(I)::value;
+            x[s][i] = *(const u32x4_t *)(tr + r * 256 + ((4 * q + i + rot(r)) % 16) * 16);
+            acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[s][i]), __builtin_bit_cast(bf16x8_t, d[s][0][i]), acc[0], 0, 0, 0);
+            if constexpr (RTW > 1) acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[s][i]), __builtin_bit_cast(bf16x8_t, d[s][1][i]), acc[1], 0, 0, 0);
+        });
+    };
+    int c = wave;
+    for (; c + DEPTH * NW < nchunks; c += (DEPTH + 1) * NW) {
         each(std::make_integer_sequence<int, DEPTH + 1>{}, [&](auto S) {
             constexpr int s = decltype(S)::value;
             load(c + (s + DEPTH) * NW, std::integral_constant<int, (s + DEPTH) % (DEPTH + 1)>{});
             __builtin_amdgcn_sched_barrier(0);
-            each(std::make_integer_sequence<int, 4>{}, [&](auto I) {
-                constexpr int i = decltype(I)::value;
-                const int row = 4 * i + lane / 16;
-                *(u32x4_t *)(tr + row * 256 + ((lane + rot(row)) % 16) * 16) = x[s][i];
-            });
-            each(std::make_integer_sequence<int, 4>{}, [&](auto I) {
-                constexpr int i = decltype(I)::value;
-                x[s][i] = *(const u32x4_t *)(tr + r * 256 + ((4 * q + i + rot(r)) % 16) * 16);
-                acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[s][i]), __builtin_bit_cast(bf16x8_t, d[s][0][i]), acc[0], 0, 0, 0);
-                if constexpr (RTW > 1) acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[s][i]), __builtin_bit_cast(bf16x8_t, d[s][1][i]), acc[1], 0, 0, 0);
-            });
+            step(S);
         });
     }
+    each(std::make_integer_sequence<int, DEPTH>{}, [&](auto S) {
+        if (c + decltype(S)::value * NW < nchunks) step(S);
+    });
     __syncthreads();  // (`red` lies where the waves' transposition areas do)
     *(float4_t *)&red[(wave * 2 * 64 + lane) * 4] = acc[0];
     *(float4_t *)&red[((wave * 2 + 1) * 64 + lane) * 4] = acc[1];
@@ -139,8 +152,8 @@ __device__ __forceinline__ void project_rows(const QuantParams &p, int rt0, uint
 // chunk to those of another, or to the projection: blockIdx.y < p.splits quantize a share of the chunks each, the
 // workgroups behind them project the same rows onto FEW rank tiles each, so that all ranks take one launch.  What is left is
 // launch, two or three memory latencies and, for long rows, the projection's walk over K.  Before / now: K = 3072, rank 32:
-// M = 256 6.9 / 4.4 us, M = 1024 8.1 / 5.4, M = 2048 8.8 / 7.2; K = 12288: M = 256 18.1 / 8.8, M = 1024 23.3 / 12.5;
-// rank 128: M = 256, K = 3072 18.7 / 4.6, M = 1024, K = 12288 107 / 21; rank 256: M = 256 36 / 5.7.
+// M = 256 6.9 / 3.8 us, M = 1024 8.1 / 4.4, M = 2048 8.8 / 6.0; K = 12288: M = 256 18.1 / 8.7, M = 1024 23.3 / 11.2;
+// rank 128: M = 256, K = 3072 18.7 / 3.9, M = 1024, K = 12288 107 / 18.8; rank 256: M = 256 36 / 5.7 (with the ring in whole turns).
 // (One kernel for all forms: with the body in a function that two kernels called, the compiler carried the chunk's offset in a vector
 // register in 27 instances that had it in a scalar one, and looped over it lane by lane for every request.  Rank 128: M = 8448, K = 6144
 // 96.6 us as it is, 100.3 from a function; M = 5120, K = 16512 106 and 402.)
@@ -155,7 +168,7 @@ __global__ void __launch_bounds__(64 * NW) quantize_fuse_lora_kernel(QuantParams
     uint8_t *tr = area.bytes[wave];
     constexpr bool PROJECT = FEW == 0;
     if constexpr (FEW > 0) {
-        if ((int)blockIdx.y >= p.splits) return project_rows<NW, FEW == 1 ? 2 : 1, FEW>(p, ((int)blockIdx.y - p.splits) * FEW, tr, (float *)area.bytes);
+        if ((int)blockIdx.y >= p.splits) return project_rows<NW, FEW == 1 ? 3 : 1, FEW>(p, ((int)blockIdx.y - p.splits) * FEW, tr, (float *)area.bytes);
     }
     const int r = lane & 15, q = lane >> 4;
     const int row0 = ROWS ? (blockIdx.x * NW + wave) * (16 * MT) : blockIdx.x * (16 * MT);
@@ -517,19 +530,25 @@ int dispatch(const QuantParams &p, hipStream_t stream) {
         int dev = 0;
         const int ncu = hipGetDevice(&dev) == hipSuccess && compute_units(dev) > 0 ? compute_units(dev) : 256;
         // Up to 8 rows per compute unit: quantizing and projecting workgroups apart, about one workgroup per compute unit (M = 1024,
-        // rank 32: 256 workgroups 5.4 us, 320 6.4).  One rank tile per projecting workgroup where they all fit beside the
-        // quantizing ones (M = 256: 4.4 us, with two 5.5), otherwise two; at ranks above 32 at least three shares of the
-        // quantizing (M = 1024, rank 128: 7.9 us, with one 10.4), or two where no more workgroups are resident at once (two per compute
-        // unit: M = 2048, rank 64, K = 12288: 22.2 us, with three 26.9), and at rank 16 two where the rows are long (M = 2048, K = 12288: INT4
-        // 18.7 us, with one 19.6; NVFP4 17.6 and 21.7).  From 16 rows per compute unit on the forms below are
-        // faster (M = 4096: 11.5 us against 13.0).
+        // rank 32: 256 workgroups 4.5 us, 320 5.4).  One rank tile per projecting workgroup where two shares of the quantizing
+        // fit beside them (M = 256: 3.8 us, with two tiles 4.3), otherwise two tiles: a share of the quantizing is an eighth of the chunks
+        // one after the other, so a second share is worth more than projecting by single tiles (M = 1280, rank 32: 4.7 us, single tiles 5.7, K = 12288 14.9
+        // and 17.5; M = 1024, rank 64: 4.7 and 6.0).  Ranks above 32 for which not even that fits take the workgroups that are
+        // resident at once, two per compute unit, or two shares beyond those (K = 12288, rank 128: M = 1536 27.7 us with one share, three 33.8;
+        // M = 2048 37.8 with two, one 42.5, three 43.4; M = 1024 18.8 with four).  Over 224 shapes (K = 1280 ... 12288, M = 256 ... 2048, ranks 16 ...
+        // 128, both precisions) 1.3 % off the fastest division measured, 2.5 % at most behind the rule before, which was 5.4 % off.  From 16 rows per compute unit on the
+        // forms below are faster (M = 4096: 11.5 us against 13.0).
         if (p.M_pad <= 8 * ncu) {
             QuantParams q = p;
             const int row_blocks = p.M_pad / 16, most = (p.K / 128 + 7) / 8;
-            const bool one = row_blocks * (RT + 1) <= ncu;
-            q.splits = ncu / row_blocks - (one ? RT : (RT + 1) / 2);
-            const int least = RT <= 2 ? (RT == 1 && p.K > 9216 ? 2 : 1) : 2 * ncu / row_blocks - (RT + 1) / 2 == 2 ? 2 : 3;
-            if (q.splits < least) q.splits = least;
+            const bool one = RT == 1 || row_blocks * (RT + 2) <= ncu;
+            const int projecting = one ? RT : (RT + 1) / 2;
+            q.splits = ncu / row_blocks - projecting;
+            if (q.splits < 2 && RT > 2) {
+                q.splits = 2 * ncu / row_blocks - projecting;
+                if (q.splits < 1) q.splits = 2;
+            }
+            if (q.splits < 1) q.splits = 1;
             if (q.splits > most) q.splits = most;
             return one ? launch_few_rows<1, FP4>(q, stream) : launch_few_rows<2, FP4>(q, stream);
         }
