@@ -85,9 +85,6 @@ __device__ __forceinline__ void project_rows(const QuantParams &p, int rt0, uint
         });
     };
     float4_t acc[2] = {float4_t{0.f, 0.f, 0.f, 0.f}, float4_t{0.f, 0.f, 0.f, 0.f}};
-    each(std::make_integer_sequence<int, DEPTH>{}, [&](auto D) {
-        if (wave + decltype(D)::value * NW < nchunks) load(wave + decltype(D)::value * NW, D);
-    });
     auto step = [&](auto S) {
         constexpr int s = decltype(S)::value;
         each(std::make_integer_sequence<int, 4>{}, [&](auto I) {
@@ -102,13 +99,21 @@ __device__ __forceinline__ void project_rows(const QuantParams &p, int rt0, uint
             if constexpr (RTW > 1) acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[s][i]), __builtin_bit_cast(bf16x8_t, d[s][1][i]), acc[1], 0, 0, 0);
         });
     };
+    // (Two paths: where a request of the first turn stood behind a condition, the loop would wait for all of them at its start.)
     int c = wave;
-    for (; c + DEPTH * NW < nchunks; c += (DEPTH + 1) * NW) {
-        each(std::make_integer_sequence<int, DEPTH + 1>{}, [&](auto S) {
-            constexpr int s = decltype(S)::value;
-            load(c + (s + DEPTH) * NW, std::integral_constant<int, (s + DEPTH) % (DEPTH + 1)>{});
-            __builtin_amdgcn_sched_barrier(0);
-            step(S);
+    if (c + DEPTH * NW < nchunks) {
+        each(std::make_integer_sequence<int, DEPTH>{}, [&](auto D) { load(c + decltype(D)::value * NW, D); });
+        for (; c + DEPTH * NW < nchunks; c += (DEPTH + 1) * NW) {
+            each(std::make_integer_sequence<int, DEPTH + 1>{}, [&](auto S) {
+                constexpr int s = decltype(S)::value;
+                load(c + (s + DEPTH) * NW, std::integral_constant<int, (s + DEPTH) % (DEPTH + 1)>{});
+                __builtin_amdgcn_sched_barrier(0);
+                step(S);
+            });
+        }
+    } else {
+        each(std::make_integer_sequence<int, DEPTH>{}, [&](auto D) {
+            if (c + decltype(D)::value * NW < nchunks) load(c + decltype(D)::value * NW, D);
         });
     }
     each(std::make_integer_sequence<int, DEPTH>{}, [&](auto S) {
@@ -147,10 +152,11 @@ __device__ __forceinline__ void project_rows(const QuantParams &p, int rt0, uint
 // live in registers), so the operator launches the kernel once per window of 128 ranks; the launches after the
 // first (QUANT false) read x again, which the caches still hold, and neither quantize nor store codes.
 //
-// FEW: few rows (dispatch: up to 8 per compute unit).  One workgroup per 16 rows leaves most of the chip idle while eight waves
+// FEW: few rows (dispatch: up to 8 per compute unit, more at ranks above 32 and in NVFP4).  One workgroup per 16 rows leaves most of the chip idle while eight waves
 // walk K, about 1 us per chunk of 128 columns, most of it the quantizer's arithmetic.  Nothing ties the codes of one
 // chunk to those of another, or to the projection: blockIdx.y < p.splits quantize a share of the chunks each, the
-// workgroups behind them project the same rows onto FEW rank tiles each, so that all ranks take one launch.  What is left is
+// workgroups behind them project the same rows onto one rank tile each (FEW = 1; FEW = 3: with fewer chunks on their way, two workgroups per
+// compute unit) or two (FEW = 2), so that all ranks take one launch.  What is left is
 // launch, two or three memory latencies and, for long rows, the projection's walk over K.  Before / now: K = 3072, rank 32:
 // M = 256 6.9 / 3.8 us, M = 1024 8.1 / 4.4, M = 2048 8.8 / 6.0; K = 12288: M = 256 18.1 / 8.7, M = 1024 23.3 / 11.2;
 // rank 128: M = 256, K = 3072 18.7 / 3.9, M = 1024, K = 12288 107 / 18.8; rank 256: M = 256 36 / 5.7 (with the ring in whole turns).
@@ -158,7 +164,7 @@ __device__ __forceinline__ void project_rows(const QuantParams &p, int rt0, uint
 // register in 27 instances that had it in a scalar one, and looped over it lane by lane for every request.  Rank 128: M = 8448, K = 6144
 // 96.6 us as it is, 100.3 from a function; M = 5120, K = 16512 106 and 402.)
 template <int NW, int MT, int RT_MAX, int DEPTH, bool FP4, int SMOOTH, bool GLU, bool ROWS, bool QUANT = true, int FEW = 0>
-__global__ void __launch_bounds__(64 * NW) quantize_fuse_lora_kernel(QuantParams p) {
+__global__ void __launch_bounds__(64 * NW, FEW > 1 ? 4 : 1) quantize_fuse_lora_kernel(QuantParams p) {
     // smoothing factors [K] during the walk; then, chunks split: [NW waves][MT][RT][64][4] partial projections;
     // rows split: behind the factors two buffers of [4 steps][RT][64 lanes] x 16 bytes of proj_down
     extern __shared__ __attribute__((aligned(16))) float lds[];  // (the alignment lets the factors be read 16 bytes at a time)
@@ -168,7 +174,8 @@ __global__ void __launch_bounds__(64 * NW) quantize_fuse_lora_kernel(QuantParams
     uint8_t *tr = area.bytes[wave];
     constexpr bool PROJECT = FEW == 0;
     if constexpr (FEW > 0) {
-        if ((int)blockIdx.y >= p.splits) return project_rows<NW, FEW == 1 ? 3 : 1, FEW>(p, ((int)blockIdx.y - p.splits) * FEW, tr, (float *)area.bytes);
+        constexpr int RTW = FEW == 2 ? 2 : 1;
+        if ((int)blockIdx.y >= p.splits) return project_rows<NW, FEW == 1 ? 3 : FEW == 2 ? 1 : 2, RTW>(p, ((int)blockIdx.y - p.splits) * RTW, tr, (float *)area.bytes);
     }
     const int r = lane & 15, q = lane >> 4;
     const int row0 = ROWS ? (blockIdx.x * NW + wave) * (16 * MT) : blockIdx.x * (16 * MT);
@@ -507,12 +514,32 @@ int project_further(const QuantParams &p0, hipStream_t stream) {
     return SVDQ_OK;
 }
 
-template <int RTW, bool FP4>
+template <int FEW, bool FP4>
 int launch_few_rows(const QuantParams &p, hipStream_t stream) {
+    constexpr int RTW = FEW == 2 ? 2 : 1;
     const dim3 grid(p.M_pad / 16, p.splits + (p.R / 16 + RTW - 1) / RTW);
-    if (p.smooth_rcp) SVDQ_LAUNCH((quantize_fuse_lora_kernel<8, 1, 1, 1, FP4, 2, false, false, true, RTW>), grid, dim3(512), 0, stream, p);
-    else SVDQ_LAUNCH((quantize_fuse_lora_kernel<8, 1, 1, 1, FP4, 0, false, false, true, RTW>), grid, dim3(512), 0, stream, p);
+    if (p.smooth_rcp) SVDQ_LAUNCH((quantize_fuse_lora_kernel<8, 1, 1, 1, FP4, 2, false, false, true, FEW>), grid, dim3(512), 0, stream, p);
+    else SVDQ_LAUNCH((quantize_fuse_lora_kernel<8, 1, 1, 1, FP4, 0, false, false, true, FEW>), grid, dim3(512), 0, stream, p);
     return check_launch("quantize_w4a4_act_fuse_lora (few rows)");
+}
+
+// The most rows per compute unit for which quantizing and projecting go apart.  Both walk x then, which costs long rows and many of them, but
+// the quantizer is not held up by the projection's operands, which ranks above 32 and NVFP4 gain most by.  Quantizing with the other
+// forms / apart, K = 3072 unless noted, us:
+//   INT4   rank 64   M = 2304 13.9 / 8.2, M = 3072 14.5 / 10.7, M = 4096 15.3 / 14.5, M = 4608 15.8 / 16.9; K = 12288: M = 3072 46.3 / 43.3, M = 4096 47.7 / 52.3
+//          rank 128  M = 2304 19.1 / 11.4, M = 3072 21.8 / 15.3, M = 4096 23.5 / 21.7, M = 4608 24.9 / 24.7; K = 12288: M = 3072 73.6 / 61.0, M = 4096 74.5 / 84.4
+//          rank 32   M = 2304 7.4 / 7.2, M = 3072 7.9 / 8.0
+//   NVFP4  rank 64   M = 2304 15.3 / 7.4, M = 4608 16.7 / 14.2, M = 6144 18.4 / 19.7; K = 12288: M = 3072 47.6 / 41.5, M = 4096 48.6 / 49.2
+//          rank 128  M = 4608 29.4 / 20.5, M = 6144 30.5 / 28.0, M = 7168 30.8 / 33.5; K = 12288: M = 4608 98.5 / 88.5, M = 6144 99.6 / 118
+//          rank 32   M = 2304 7.8 / 6.5, M = 4096 9.1 / 8.0, M = 4608 13.1 / 12.3 (the layer is no faster); K = 2304: M = 4608 10.7 / 9.8; K = 6144: M = 4096 17.1 / 16.0, M = 4608 24.2 / 25.9
+//          rank 16   M = 2304 7.6 / 6.5, M = 4096 8.8 / 9.2
+int few_rows_most(int RT, int K, bool fp4) {
+    if (RT > 8) return 8;
+    if (!fp4) return RT <= 2 ? 8 : K <= 4096 ? 16 : 12;
+    if (RT == 1) return K <= 6144 ? 9 : 8;
+    if (RT == 2) return K <= 2304 ? 18 : K <= 6144 ? 16 : 8;
+    if (RT <= 4) return K <= 4096 ? 18 : K <= 6144 ? 16 : 12;
+    return K <= 3072 ? 24 : 18;
 }
 
 template <bool FP4, bool GLU>
@@ -536,9 +563,11 @@ int dispatch(const QuantParams &p, hipStream_t stream) {
         // and 17.5; M = 1024, rank 64: 4.7 and 6.0).  Ranks above 32 for which not even that fits take the workgroups that are
         // resident at once, two per compute unit, or two shares beyond those (K = 12288, rank 128: M = 1536 27.7 us with one share, three 33.8;
         // M = 2048 37.8 with two, one 42.5, three 43.4; M = 1024 18.8 with four).  Over 224 shapes (K = 1280 ... 12288, M = 256 ... 2048, ranks 16 ...
-        // 128, both precisions) 1.3 % off the fastest division measured, 2.5 % at most behind the rule before, which was 5.4 % off.  From 16 rows per compute unit on the
-        // forms below are faster (M = 4096: 11.5 us against 13.0).
-        if (p.M_pad <= 8 * ncu) {
+        // 128, both precisions) 1.3 % off the fastest division measured, 2.5 % at most behind the rule before, which was 5.4 % off.
+        // More rows than 8 per compute unit: two shares of the quantizing where that takes no more rounds of the workgroups that are resident
+        // at once than one (M = 3072, rank 64: 10.7 us, with one 11.0; M = 2304, rank 64 8.2 with one, two 9.3), one in INT4 at ranks above 64 (M = 2304, rank
+        // 128, K = 12288: 43.9, with two 52.0; NVFP4 51.0 and 47.1).
+        if (RT == 0 ? p.M_pad <= 8 * ncu : p.M_pad <= few_rows_most(RT, p.K, FP4) * ncu) {
             QuantParams q = p;
             const int row_blocks = p.M_pad / 16, most = (p.K / 128 + 7) / 8;
             const bool one = RT == 1 || row_blocks * (RT + 2) <= ncu;
@@ -546,11 +575,18 @@ int dispatch(const QuantParams &p, hipStream_t stream) {
             q.splits = ncu / row_blocks - projecting;
             if (q.splits < 2 && RT > 2) {
                 q.splits = 2 * ncu / row_blocks - projecting;
-                if (q.splits < 1) q.splits = 2;
+                if (q.splits < 1) q.splits = RT > 8 ? 3 : 2;
             }
             if (q.splits < 1) q.splits = 1;
+            if (RT == 1 && p.K > 9216 && q.splits < 2) q.splits = 2;
+            if (p.M_pad > 8 * ncu) {
+                auto rounds = [&](int splits) { return (row_blocks * (splits + projecting) + 2 * ncu - 1) / (2 * ncu); };
+                q.splits = (FP4 || projecting <= 2) && rounds(2) == rounds(1) ? 2 : 1;
+            }
             if (q.splits > most) q.splits = most;
-            return one ? launch_few_rows<1, FP4>(q, stream) : launch_few_rows<2, FP4>(q, stream);
+            if (!one) return launch_few_rows<2, FP4>(q, stream);
+            const bool deep = row_blocks * (q.splits + projecting) <= ncu && p.K <= 8192;
+            return deep ? launch_few_rows<1, FP4>(q, stream) : launch_few_rows<3, FP4>(q, stream);
         }
         // High ranks with many rows: the waves split the rows (eight waves, 128 rows per workgroup) and share each chunk
         // of proj_down through LDS.  Ranks 80 ... 128, K = 3072: M = 18432 52.4 us (four waves on 32 rows each: 61.8; the

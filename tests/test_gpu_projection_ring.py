@@ -24,3 +24,12 @@ def test_chunks_per_wave(dev, M, R, chunks):
     _, _, la = _run(dev, x, layer, fp4=False, smooth=True)
     want = olin.quantize_act_fuse_lora(x, layer.proj_down, layer.smooth)[2]
     assert (la - want).abs().max().item() <= 2e-5 * want.abs().max().item() + 1e-6  # (fp32 sums of K products in another order)
+
+
+@pytest.mark.parametrize("M,K,R,fp4", [(2304, 640, 16, True), (2100, 1152, 64, False), (3072, 3200, 48, False), (4600, 384, 32, True), (4600, 3072, 32, True), (4096, 1152, 128, False),
+                                       (6000, 640, 112, True), (1000, 9344, 16, False)])
+def test_quantizing_and_projecting_apart_beyond_8_rows_per_compute_unit(dev, M, K, R, fp4):
+    """One and two shares of the quantizing, one and two rank tiles per projecting workgroup, a rank tile left over, rows and chunks
+    that end early; long rows with fewer chunks on their way."""
+    announce(f"apart M={M} K={K} R={R} fp4={fp4}")
+    _check_row_sample(dev, M, K, R, fp4, True)
