@@ -608,14 +608,45 @@ int gemm_fp4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t st
 }
 
 // ---- few rows, either precision: small tiles, operands straight to registers (gemm_direct_kernel.h) ------
+// The tile of a few-rows launch with the plain epilogue, in blocks of 32 x 32.  What takes the time is the fetching of the operands: a
+// compute unit gets 120 GB/s in requests of 16 bytes a lane, 80 in those of 8, however few of them fetch and however many waves do (48
+// or 192 workgroups, 4 ... 16 waves each), and a tile of mt x nc blocks fetches mt + nc fragments per k-group.  Square tiles fetch least per
+// product, small ones bring more compute units to bear: the sums cost a tile nothing before the end.  A model of the time in us, linear in the
+// tiles of the busiest compute unit and in the k-groups, fitted to 844 shapes (M = 16 ... 1000, K = 1024 ... 13824, N = 1024 ... 21504)
+// times the six tiles: its choice is 0.1 % (INT4) and 0.05 % (NVFP4) off the fastest on average and 5.4 % at most; tiles of 128 columns only,
+// 18 and 21 %.  Measured, layer calls, 128 columns / the choice, us:
+//   INT4   M = 64, K = N = 3072  13.3 / 10.2 (32 x 32)    NVFP4  14.6 / 10.3
+//          M = 256               14.1 / 13.1 (64 x 64)           15.3 / 14.1
+//          M = 64, K = 12288     32.3 / 21.4 (32 x 32)           34.6 / 21.6
+//          M = 256, K = 12288    34.7 / 30.3 (64 x 64)           37.4 / 34.0
+struct FewRowsTile {
+    int mt, nc;  // blocks of 32 rows, of 32 columns
+    double launch, tile, kgroup;
+    double time;
+};
+FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu) {
+    constexpr FewRowsTile int4[] = {{1, 1, -0.18, 0.18, 0.0382, 0.0}, {1, 2, -0.46, 0.68, 0.0551, 0.0}, {2, 1, -0.46, 0.75, 0.0499, 0.0},
+                                    {2, 2, 0.18, 0.64, 0.0702, 0.0},  {1, 4, -0.13, 0.64, 0.0948, 0.0}, {2, 4, 1.04, 0.53, 0.1378, 0.0}};
+    constexpr FewRowsTile nvfp4[] = {{1, 1, -0.85, 0.16, 0.0323, 0.0}, {1, 2, -0.52, 0.14, 0.0515, 0.0}, {2, 1, -0.64, 0.24, 0.0498, 0.0},
+                                     {2, 2, -0.17, 0.46, 0.0719, 0.0}, {1, 4, 0.22, 0.47, 0.0876, 0.0},  {2, 4, 1.96, -0.07, 0.1112, 0.0}};
+    const long long row_blocks = (rows_needed(a) + 31) / 32, column_blocks = a->N / 32;
+    FewRowsTile best{};
+    for (const FewRowsTile &c : a->fp4 ? nvfp4 : int4) {
+        const long long tiles = (row_blocks + c.mt - 1) / c.mt * (column_blocks / c.nc);
+        const double t = c.launch + (double)((tiles + ncu - 1) / ncu) * (c.tile + c.kgroup * (double)(a->K / 64));
+        if (best.mt == 0 || t < best.time) {
+            best = c;
+            best.time = t;
+        }
+    }
+    return best;
+}
+
 // Which of the two shapes of the few-rows kernel (0: neither) a launch takes.  Shape 1: tiles of 32 rows, four waves split
 // K.  Shape 2: tiles of 64 rows, a quarter fewer operand bytes per product, from about 400 tiles of 32 rows on; INT4: two waves
 // split K and two the columns, NVFP4: four waves split K.  Models of the time in us fitted to launches at K = 1024 ... 12288
-// on 256 compute units, linear in the number of tiles that the busiest compute unit works through and in the k-groups; they meet
-// the measurements within about 10 %.  When they were fitted the choice took 0.6 % (NVFP4) and 0.3 % (INT4) longer than the fastest of the
-// three over 2200 random shapes, and was more than 3 % slower than the large tiles in 17, 14 of them short rows whose large tiles would be shared
-// (below); with the kernels as they are now it is 1.6 % (NVFP4, 316 shapes) and 0.8 % (INT4, 323).  A refit of the NVFP4 side gives 0.1 %, and
-// moves choices at 4608 rows.  Measured at K = 3072 at the time of the fit, large tiles (split along K where that pays) / shape 1 / shape 2:
+// on 256 compute units, linear in the number of tiles that the busiest compute unit works through and in the k-groups; they met
+// the measurements within about 10 % when they were fitted, over 2200 random shapes; what has changed since is in the factors below.  Measured at K = 3072 at the time of the fit, large tiles (split along K where that pays) / shape 1 / shape 2:
 //   INT4   M = 256, N = 3072   22.8 /  9.6 / 12.3     NVFP4  60.7 / 11.8 / 13.8
 //          M = 505, N = 9216   28.7 / 33.1 / 30.6            62.9 / 38.4 / 34.1
 //          M = 1157, N = 3072  29.7 / 27.6 / 21.8            62.1 / 31.7 / 25.7
@@ -659,11 +690,25 @@ int choose_direct(const svdq_gemm_args *a, int ncu) {
             t1 += 0.9 * c1;
             t2 += 1.0 * c2;
         }
+        // The models of this kernel predate its buffers: against whole large tiles it is up to 14 % faster than they say (3100 shapes, M = 300 ... 5200,
+        // layer calls: where they say 1.0 ... 1.05 of the large tiles' time it takes 0.90, from 1.2 on 1.04).  Choosing so takes 0.5 % longer than the
+        // fastest on average, 1 % without: M = 1057, K = 10240, N = 14208 296 -> 254 us, M = 1131, K = 2048, N = 10112 58 -> 52, with norm and rotation M = 1614, K = 3968,
+        // N = 11904 183 -> 155, MLP M = 2154, K = 1792 132 -> 121.  (Against shared ones the models stand at 4608 rows.)
+        if (kg > 12 && (tiles <= 1.0 || nwg > 0)) t_large *= 1.14;
     } else {
         svdq_gemm_plan tiles;
         t_large = choose_tiles_int4(a, ncu, &tiles);
         t1 = 3.5 + c1 * (1.1 + 0.106 * kg);
         t2 = 3.3 + c2 * (1.6 + 0.158 * kg);
+        if (a->qout) {
+            t_large *= 1.05;  // (1158 MLPs of 100 ... 2600 rows: 0.4 % off the fastest, 0.7 without; M = 1486, K = 1024 51.3 -> 45.8 us)
+        } else if (!needs_next_epilogue(a)) {
+            // (the plain epilogue's tiles are faster than these two, the model of their time has no offset: 2277 layers of 100 ... 2600 rows 0.3 % off the
+            // fastest, 0.6 without; M = 225, K = 4992, N = 10624 36.4 -> 30.5 us, M = 175, K = 9984, N = 14976 59 -> 51, M = 506, K = 9600, N = 6912 61 -> 59)
+            const double t_plain = 5.0 + 1.3 * plain_tile(a, ncu).time;
+            if (t_plain < t_large) return t1 < t2 ? 1 : 2;
+            t_large *= 0.95;
+        }
     }
     if (t1 < t2) return t1 < t_large ? 1 : 0;
     return t2 < t_large ? 2 : 0;
@@ -686,40 +731,6 @@ void make_plan(const svdq_gemm_args *a, int ncu, svdq_gemm_plan *plan) {
     if (shape) plan->row_blocks = (rows_needed(a) + 32 * shape - 1) / (32 * shape);  // (shape s: tiles of 32 s rows)
     else if (a->fp4) plan_fp4(a, ncu, plan);
     else plan_int4(a, ncu, plan);
-}
-
-// The tile of a few-rows launch with the plain epilogue, in blocks of 32 x 32.  What takes the time is the fetching of the operands: a
-// compute unit gets 120 GB/s in requests of 16 bytes a lane, 80 in those of 8, however few of them fetch and however many waves do (48
-// or 192 workgroups, 4 ... 16 waves each), and a tile of mt x nc blocks fetches mt + nc fragments per k-group.  Square tiles fetch least per
-// product, small ones bring more compute units to bear: the sums cost a tile nothing before the end.  A model of the time in us, linear in the
-// tiles of the busiest compute unit and in the k-groups, fitted to 844 shapes (M = 16 ... 1000, K = 1024 ... 13824, N = 1024 ... 21504)
-// times the six tiles: its choice is 0.1 % (INT4) and 0.05 % (NVFP4) off the fastest on average and 5.4 % at most; tiles of 128 columns only,
-// 18 and 21 %.  Measured, layer calls, 128 columns / the choice, us:
-//   INT4   M = 64, K = N = 3072  13.3 / 10.2 (32 x 32)    NVFP4  14.6 / 10.3
-//          M = 256               14.1 / 13.1 (64 x 64)           15.3 / 14.1
-//          M = 64, K = 12288     32.3 / 21.4 (32 x 32)           34.6 / 21.6
-//          M = 256, K = 12288    34.7 / 30.3 (64 x 64)           37.4 / 34.0
-struct FewRowsTile {
-    int mt, nc;  // blocks of 32 rows, of 32 columns
-    double launch, tile, kgroup;
-};
-FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu) {
-    constexpr FewRowsTile int4[] = {{1, 1, -0.18, 0.18, 0.0382}, {1, 2, -0.46, 0.68, 0.0551}, {2, 1, -0.46, 0.75, 0.0499},
-                                    {2, 2, 0.18, 0.64, 0.0702},  {1, 4, -0.13, 0.64, 0.0948}, {2, 4, 1.04, 0.53, 0.1378}};
-    constexpr FewRowsTile nvfp4[] = {{1, 1, -0.85, 0.16, 0.0323}, {1, 2, -0.52, 0.14, 0.0515}, {2, 1, -0.64, 0.24, 0.0498},
-                                     {2, 2, -0.17, 0.46, 0.0719}, {1, 4, 0.22, 0.47, 0.0876},  {2, 4, 1.96, -0.07, 0.1112}};
-    const long long row_blocks = (rows_needed(a) + 31) / 32, column_blocks = a->N / 32;
-    FewRowsTile best{};
-    double best_t = 0.0;
-    for (const FewRowsTile &c : a->fp4 ? nvfp4 : int4) {
-        const long long tiles = (row_blocks + c.mt - 1) / c.mt * (column_blocks / c.nc);
-        const double t = c.launch + (double)((tiles + ncu - 1) / ncu) * (c.tile + c.kgroup * (double)(a->K / 64));
-        if (best.mt == 0 || t < best_t) {
-            best = c;
-            best_t = t;
-        }
-    }
-    return best;
 }
 
 int gemm_direct(const svdq_gemm_args *a, const svdq_gemm_plan &plan, int ncu, hipStream_t st, int dev, bool noalloc) {

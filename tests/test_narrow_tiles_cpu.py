@@ -6,7 +6,7 @@ import ctypes
 import pytest
 
 from nunchaku_amd import _native as nv
-from plan_util import call
+from plan_util import call, plan_of
 from test_address_model import FRAG, buffer_read
 from test_build_guard import compiled  # noqa: F401  (the fixture)
 
@@ -79,3 +79,13 @@ def test_narrow_tiles_fit_their_registers(compiled, variant):  # noqa: F811
     assert len(kernels) == 4, list(usage)
     for name, u in kernels.items():
         assert u["VGPRs"] <= 256 and u["AGPRs"] == 0 and u["ScratchSize"] == 0 and u["Occupancy"] >= 2, (name, u)
+
+
+# On either side of the lines between the few-rows kernel and the large tiles that the factors in choose_direct draw.
+@pytest.mark.parametrize("kind,M,K,N,fp4,few", [
+    ("plain", 1131, 2048, 10112, True, 2), ("plain", 4608, 15360, 3072, True, 0), ("rope", 1614, 3968, 11904, True, 2), ("next", 2154, 1792, 7168, True, 2),
+    ("plain", 225, 4992, 10624, False, 2), ("plain", 175, 9984, 14976, False, 2), ("plain", 506, 9600, 6912, False, 0), ("next", 1486, 1024, 4096, False, 2),
+    ("next", 1486, 2048, 8192, False, 0),
+])
+def test_few_rows_or_large_tiles(kind, M, K, N, fp4, few):
+    assert plan_of(call(kind, M, K, N, 32, fp4)).few_rows == few
