@@ -57,14 +57,15 @@ __global__ void zero_f32_kernel(float *p, int64_t n) {
     else for (int64_t j = i; j < n; j++) p[j] = 0.f;
 }
 
-// The sum of float4 number `item` over n shares that lie `stride` float4 apart, worked out by the eight threads of a
-// workgroup that have the same threadIdx.x % 32: each adds an eighth of the shares in ascending order, eight requests in
-// flight, and the first of them adds the eighths in ascending order.  `item` of the threads without work is any valid one.
+// The sum of float4 number `item` over n shares that lie `stride` float4 apart, worked out by the PARTS threads of a
+// workgroup that have the same threadIdx.x % 32: each adds a PARTS-th of the shares in ascending order, eight requests in
+// flight, and the first of them adds the parts in ascending order.  `item` of the threads without work is any valid one.
 // Valid in the workgroup's first 32 threads.
+template <int PARTS>
 __device__ inline float4_t sum_of_shares(const float4_t *part, size_t item, size_t stride, int n) {
-    __shared__ float4_t eighth[8][32];
+    __shared__ float4_t parts[PARTS][32];
     const int e = threadIdx.x >> 5, lane = threadIdx.x & 31;
-    const int first = n * e / 8, last = n * (e + 1) / 8;
+    const int first = n * e / PARTS, last = n * (e + 1) / PARTS;
     float4_t sum = float4_t{0.f, 0.f, 0.f, 0.f};
     for (int b0 = first; b0 < last; b0 += 8) {
         float4_t v[8];
@@ -74,11 +75,11 @@ __device__ inline float4_t sum_of_shares(const float4_t *part, size_t item, size
         for (int u = 0; u < 8; u++)
             if (b0 + u < last) sum += v[u];
     }
-    eighth[e][lane] = sum;
+    parts[e][lane] = sum;
     __syncthreads();
     if (e == 0) {
 #pragma unroll
-        for (int u = 1; u < 8; u++) sum += eighth[u][lane];
+        for (int u = 1; u < PARTS; u++) sum += parts[u][lane];
     }
     return sum;
 }
@@ -89,10 +90,11 @@ __device__ inline float4_t sum_of_shares(const float4_t *part, size_t item, size
 // rank l % 16 of a 16 x 16 tile (the result registers of the matrix instruction).
 // Bound by latency at few rows, where one thread per sum had 6 to 12 rounds of requests to wait for: 96 shares of 1280 rows, rank
 // 32, 11.5 us before and 5.5 now; 48 shares of 4608 rows (28 MB) 6.2 and 6.2.
-__global__ void __launch_bounds__(256) reduce_shares_kernel(const float4_t *part, float *out, int nshares, int M_pad, int R) {
+template <int PARTS>
+__global__ void __launch_bounds__(32 * PARTS) reduce_shares_kernel(const float4_t *part, float *out, int nshares, int M_pad, int R) {
     const int RT = R / 16, quads = M_pad * R / 4;  // (M_pad is a multiple of 256 and R of 16: whole workgroups)
     const int item = blockIdx.x * 32 + (threadIdx.x & 31);
-    const float4_t sum = sum_of_shares(part, item, quads, nshares);
+    const float4_t sum = sum_of_shares<PARTS>(part, item, quads, nshares);
     if (threadIdx.x >= 32) return;
     const int ln = item & 63, m2 = (item >> 6) & 1, rest = item >> 7;  // rest = slab * RT + rank tile
     const int rt = rest % RT, slab32 = rest / RT;
@@ -107,14 +109,15 @@ __global__ void __launch_bounds__(256) reduce_shares_kernel(const float4_t *part
 // out_vk [batch][head][33][32].  A workgroup's 32 float4 are 4 rows i of all 32 columns j, or the 8 of the column sums.
 // The shares are those of row blocks of vk_block rows up to row `full_rows` and of 64 rows from there on; a batch entry is
 // vk_rows of them.
-__global__ void __launch_bounds__(256) reduce_vk_kernel(const float4_t *part, float *out, int vk_rows, int vk_block, int full_rows, int heads) {
+template <int PARTS>
+__global__ void __launch_bounds__(32 * PARTS) reduce_vk_kernel(const float4_t *part, float *out, int vk_rows, int vk_block, int full_rows, int heads) {
     constexpr int QUADS = VK_HEAD_FLOATS / 4, PIECES = (QUADS + 31) / 32;
     const int piece = blockIdx.x % PIECES, head = (blockIdx.x / PIECES) % heads, b = blockIdx.x / (PIECES * heads);
     const int lane = threadIdx.x & 31, quad = piece * 32 + lane;
     auto slots_before = [&](int row) { return row <= full_rows ? row / vk_block : full_rows / vk_block + (row - full_rows) / 64; };
     const int slot = slots_before(b * vk_rows);
     const size_t item = ((size_t)slot * heads + head) * QUADS + (quad < QUADS ? quad : QUADS - 1);
-    const float4_t sum = sum_of_shares(part, item, (size_t)heads * QUADS, slots_before((b + 1) * vk_rows) - slot);
+    const float4_t sum = sum_of_shares<PARTS>(part, item, (size_t)heads * QUADS, slots_before((b + 1) * vk_rows) - slot);
     if (threadIdx.x >= 32 || quad >= QUADS) return;
     float *o = out + ((size_t)b * heads + head) * VK_HEAD_FLOATS;
     if (piece == PIECES - 1) {
@@ -243,17 +246,29 @@ bool acquire_workspace(bool noalloc, int dev, hipStream_t st, size_t zero_bytes,
 // (one per column block) and the linear-attention sums (one per vk_block rows, from row `full_rows` on one per 64), each
 // added in ascending order.
 template <typename P>
-int add_shares(const P &p, int nshares, int vk_block, int full_rows, hipStream_t st) {
+int add_shares(const P &p, int rows, int nshares, int vk_block, int full_rows, hipStream_t st) {
     if (p.next_down) {
-        const int quads = p.M_pad * p.R_down / 4;
-        SVDQ_LAUNCH(reduce_shares_kernel, dim3((unsigned)(quads / 32)), dim3(256), 0, st, (const float4_t *)p.next_lora_part,
-                    p.next_lora_out, nshares, p.M_pad, p.R_down);
+        const int quads = (rows + 31) / 32 * 32 * p.R_down / 4;
+        auto launch = [&](auto PARTS) {
+            constexpr int parts = decltype(PARTS)::value;
+            SVDQ_LAUNCH(reduce_shares_kernel<parts>, dim3((unsigned)(quads / 32)), dim3(32 * parts), 0, st, (const float4_t *)p.next_lora_part, p.next_lora_out, nshares,
+                        p.M_pad, p.R_down);
+        };
+        if (nshares <= 32) launch(std::integral_constant<int, 4>{});
+        else if (nshares <= 64) launch(std::integral_constant<int, 8>{});
+        else launch(std::integral_constant<int, 16>{});
         const int rc = check_launch("gemm_w4a4 (low-rank shares)");
         if (rc != SVDQ_OK) return rc;
     }
     if (p.vk) {
         const int heads = p.N / 96, batch = p.M_pad / p.vk_rows;
-        SVDQ_LAUNCH(reduce_vk_kernel, dim3((unsigned)(batch * heads * 9)), dim3(256), 0, st, (const float4_t *)p.vk_part, p.vk, p.vk_rows, vk_block, full_rows, heads);
+        auto launch = [&](auto PARTS) {
+            constexpr int parts = decltype(PARTS)::value;
+            SVDQ_LAUNCH(reduce_vk_kernel<parts>, dim3((unsigned)(batch * heads * 9)), dim3(32 * parts), 0, st, (const float4_t *)p.vk_part, p.vk, p.vk_rows, vk_block, full_rows,
+                        heads);
+        };
+        if (p.vk_rows <= 1024) launch(std::integral_constant<int, 4>{});
+        else launch(std::integral_constant<int, 8>{});
         return check_launch("gemm_w4a4 (linear-attention sums)");
     }
     return SVDQ_OK;
@@ -510,7 +525,7 @@ int gemm_int4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t s
     p.next_lora_part = (float *)(w.scratch + part_bytes);
     p.vk_part = (float *)(w.scratch + part_bytes + share_bytes);
     int rc = launch(ntiles * kparts);
-    if (rc == SVDQ_OK) rc = add_shares(p, nblocks, g6::BM, p.full_blocks * g6::BM, st);
+    if (rc == SVDQ_OK) rc = add_shares(p, rows_needed(a), nblocks, g6::BM, p.full_blocks * g6::BM, st);
     if (rc != SVDQ_OK && w.owner) w.owner->dirty = true;
     return rc;
 }
@@ -602,7 +617,7 @@ int gemm_fp4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t st
     p.next_lora_part = (float *)(w.scratch + part_bytes);
     p.vk_part = (float *)(w.scratch + part_bytes + share_bytes);
     int rc = next ? launch_gemm_fp4_v5(p, nwg, st) : launch_gemm_fp4_v4(p, nwg, st);
-    if (rc == SVDQ_OK) rc = add_shares(p, p.N / 128, 32, p.M_pad, st);
+    if (rc == SVDQ_OK) rc = add_shares(p, rows_needed(a), p.N / 128, 32, p.M_pad, st);
     if (rc != SVDQ_OK && w.owner) w.owner->dirty = true;
     return rc;
 }
@@ -759,7 +774,7 @@ int gemm_direct(const svdq_gemm_args *a, const svdq_gemm_plan &plan, int ncu, hi
     p.next_lora_part = (float *)w.scratch;
     p.vk_part = (float *)(w.scratch + share_bytes);
     int rc = launch();
-    if (rc == SVDQ_OK) rc = add_shares(p, p.N / 128, 32, p.M_pad, st);
+    if (rc == SVDQ_OK) rc = add_shares(p, rows_needed(a), p.N / 128, 32, p.M_pad, st);
     return rc;
 }
 }  // namespace
