@@ -15,6 +15,8 @@ int launch_fp4_plain(const GemmParams &p, int shape, hipStream_t stream);
 int launch_fp4_next(const GemmParams &p, int shape, hipStream_t stream);
 int launch_square(const GemmParams &p, bool fp4, int mt, hipStream_t stream);
 int launch_oblong(const GemmParams &p, bool fp4, int mt, hipStream_t stream);
+int launch_staged_plain(const GemmParams &p, hipStream_t stream);
+int launch_staged_next(const GemmParams &p, hipStream_t stream);
 }  // namespace direct
 namespace g6 {
 int launch_plain(const Params &p, int nwg, hipStream_t stream);
@@ -657,6 +659,16 @@ FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu) {
     return best;
 }
 
+// INT4 launches whose tiles of 64 x 128 are between one and two per compute unit: the waves split the columns and share the rows' operands
+// through LDS (gemm_direct_kernel.h).  A tile alone on its compute unit is a chain of latencies, 0.22 us per k-group, two overlap; three
+// issue more instructions per product than the large tiles.  Layer calls, the best other form / this one, K = 3072: QKV M = 256, N = 9216 26.9 / 24.7
+// us, M = 505 (2.25 tiles) 32.4 / 33.7; plain M = 384, N = 9216 25.0 / 23.3, M = 256 22.3 / 23.0 (1.1 tiles, where narrow tiles are better).  On average over
+// 5000 layers: with the norm and rotation 6.5 % faster from 1 to 2 tiles, MLPs 4 %, plain 0 at 1.5, 4 to 9 % from 1.6 to 2; 1 to 4 % slower beyond.
+bool staged_rows(const svdq_gemm_args *a, int ncu) {
+    const long long tiles = (rows_needed(a) + 63) / 64 * (a->N / 128);
+    return !a->fp4 && a->K >= 256 && tiles <= 2 * ncu && (needs_next_epilogue(a) ? tiles > ncu : 5 * tiles > 8 * ncu);
+}
+
 // Which of the two shapes of the few-rows kernel (0: neither) a launch takes.  Shape 1: tiles of 32 rows, four waves split
 // K.  Shape 2: tiles of 64 rows, a quarter fewer operand bytes per product, from about 400 tiles of 32 rows on; INT4: two waves
 // split K and two the columns, NVFP4: four waves split K.  Models of the time in us fitted to launches at K = 1024 ... 12288
@@ -676,6 +688,7 @@ FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu) {
 int choose_direct(const svdq_gemm_args *a, int ncu) {
     if (a->k_split > 0) return 0;  // (the caller asks for the tiles that k_split is about)
     if (((uintptr_t)a->bias | (uintptr_t)a->wcscales | (uintptr_t)a->oscales) % 8 || (uintptr_t)a->colnorm % 16) return 0;  // (read four columns at a time)
+    if (staged_rows(a, ncu)) return 2;
     const int rows = rows_needed(a), kg = (int)(a->K / 64);
     const long long ncols = a->N / 128;
     const double c1 = (double)((((rows + 31) / 32) * ncols + ncu - 1) / ncu), c2 = (double)((((rows + 63) / 64) * ncols + ncu - 1) / ncu);
@@ -719,7 +732,7 @@ int choose_direct(const svdq_gemm_args *a, int ncu) {
             t_large *= 1.05;  // (1158 MLPs of 100 ... 2600 rows: 0.4 % off the fastest, 0.7 without; M = 1486, K = 1024 51.3 -> 45.8 us)
         } else if (!needs_next_epilogue(a)) {
             // (the plain epilogue's tiles are faster than these two, the model of their time has no offset: 2277 layers of 100 ... 2600 rows 0.3 % off the
-            // fastest, 0.6 without; M = 225, K = 4992, N = 10624 36.4 -> 30.5 us, M = 175, K = 9984, N = 14976 59 -> 51, M = 506, K = 9600, N = 6912 61 -> 59)
+            // fastest, 0.6 without; M = 225, K = 4992, N = 10624 36.4 -> 30.5 us, M = 175, K = 9984, N = 14976 59 -> 51, M = 261, K = 1152, N = 14208 18 -> 17)
             const double t_plain = 5.0 + 1.3 * plain_tile(a, ncu).time;
             if (t_plain < t_large) return t1 < t2 ? 1 : 2;
             t_large *= 0.95;
@@ -754,7 +767,9 @@ int gemm_direct(const svdq_gemm_args *a, const svdq_gemm_plan &plan, int ncu, hi
     const bool next = needs_next_epilogue(a);
     int shape = plan.few_rows;
     p.row_blocks = plan.row_blocks;
-    if (!next) {
+    if (shape == 2 && staged_rows(a, ncu)) {
+        if (!next) return direct::launch_staged_plain(p, st);
+    } else if (!next) {
         const FewRowsTile t = plain_tile(a, ncu);
         p.row_blocks = ((int)rows_needed(a) + 32 * t.mt - 1) / (32 * t.mt);
         if (t.nc < 4) return t.nc == t.mt ? direct::launch_square(p, a->fp4 != 0, t.mt, st) : direct::launch_oblong(p, a->fp4 != 0, t.mt, st);
@@ -762,6 +777,7 @@ int gemm_direct(const svdq_gemm_args *a, const svdq_gemm_plan &plan, int ncu, hi
     }
     auto launch = [&]() {
         if (a->fp4) return next ? direct::launch_fp4_next(p, shape, st) : direct::launch_fp4_plain(p, shape, st);
+        if (shape == 2 && staged_rows(a, ncu)) return direct::launch_staged_next(p, st);
         return next ? direct::launch_int4_next(p, shape, st) : direct::launch_int4_plain(p, shape, st);
     };
     // every 128-column chunk's share of the next layer's low-rank projection, every 32-row block's linear-attention sums

@@ -56,16 +56,26 @@ constexpr int SLAB_BYTES = 32 * OUT_LD * 2;
 // squares of the RMS norm, [MT][4][32] floats.  The bf16 slabs take the place of the sums.
 // Tiles narrower than 128 columns: the sums of all row blocks at once, and a slab of its own for every wave behind them.
 constexpr int NARROW_LD = 40, NARROW_SLAB_BYTES = 32 * NARROW_LD * 2;
-template <int MT, int NC, int KP>
+template <int MT, int KP>
+constexpr int ssq_offset() {
+    return KP * 16384 > MT * SLAB_BYTES ? KP * 16384 : MT * SLAB_BYTES;
+}
+// Waves that split the columns only (WN = 4, INT4, 64 rows): a stage of the rows' operands of one k-group in LDS, two fragments and the scales of
+// 64 rows, eight times over in a whole KB.
+constexpr int STAGE_BYTES = 2 * FRAG_BYTES + 1024;
+template <int MT, int NC, int KP, int DEPTH>
 constexpr int lds_bytes() {
-    return NC == 4 ? KP * 16384 + MT * 512 : KP * MT * NC * 4096 + MT * NC * NARROW_SLAB_BYTES;
+    constexpr int epilogue = NC == 4 ? ssq_offset<MT, KP>() + MT * 512 : KP * MT * NC * 4096 + MT * NC * NARROW_SLAB_BYTES;
+    return KP == 1 && (DEPTH + 1) * STAGE_BYTES > epilogue ? (DEPTH + 1) * STAGE_BYTES : epilogue;
 }
 
 template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT>
-__global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams p) {
+__global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_kernel(GemmParams p) {
     constexpr int NC = NT * WN;  // 32-column tiles of the workgroup; a wave has NT of them
     constexpr int WAVES = WN * KP;
     constexpr bool NARROW = NC < 4;
+    constexpr bool STAGED = WN == 4;
+    static_assert(!STAGED || (!FP4 && MT == 2 && NT == 1 && KP == 1 && (DEPTH + 1) * STAGE_BYTES <= lds_bytes<MT, NC, KP, DEPTH>()));
     static_assert(WAVES == 4 && MT * NC <= (NARROW ? 4 : 8), "the epilogue gives each wave one column tile, of one row block where the tile is narrow");
     static_assert(!NARROW || !NEXT, "the norm, the rotation and the next layer's operands need whole 128-column blocks");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -225,34 +235,124 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
         }
     };
 
-    each(std::make_integer_sequence<int, DEPTH>{}, [&](auto D) { load(D); });
-    if constexpr (FP4) {
-        auto &st = sets[0];
-        read_row_scales(st.as);
+    if constexpr (STAGED) {
+        // Every wave multiplies one column tile by both row blocks: the columns' operands come straight to registers, DEPTH k-groups ahead, the
+        // rows', which all four need, to LDS by asynchronous copies, a KB per wave and k-group, into DEPTH + 1 stages.  Six fragments per
+        // k-group and tile where waves that split K two ways fetch eight, no sums to exchange, 32 accumulators per lane.  One tile per compute unit
+        // takes 0.22 us per k-group with three on their way (0.33 with two: the latency of the requests), two or three share it better than
+        // that, until the vector instructions bound them (which launches, and what they gain: staged_rows in gemm.hip).
+        const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds + wave * 1024;
+        const bool rows = wave < 3;
+        const uint8_t *src = rows ? p.act + ((size_t)(f0 >> 2) * kgroups) * (4 * FRAG_BYTES) + (f0 & 3) * FRAG_BYTES + wave * 1024 : (const uint8_t *)(p.ascales + f0 * 32);
+        const uint32_t stride = rows ? 4 * FRAG_BYTES : (uint32_t)p.M_pad * 2, voff = rows ? lane * 16 : (lane & 7) * 16;
+        constexpr int RING = DEPTH + 1;
+        v6i_t w[RING];
+        uint32_t ws[RING];
+        auto request = [&](auto S) {
+            constexpr int st = decltype(S)::value;
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(base + st * STAGE_BYTES), "v"(voff), "s"(src) : "memory", "m0");
+            w[st] = codes6(*(const u32x4_t *)(wp + off16), *(const u32x2_t *)(wp + off8));
+            ws[st] = *(const uint32_t *)(sp + off_ws);
+            src += stride;
+            wp += 8 * FRAG_BYTES;
+            sp += 2048;
+        };
+        v6i_t X[MT];
+        uint32_t as[MT];
+        auto read_rows = [&](auto S) {
+            const uint8_t *stage = lds + decltype(S)::value * STAGE_BYTES;
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) xop[0][mt] = dequant_word_fp4(st.x[mt][0], row_scale(mt, false));
-        wop[0] = dequant_word_fp4(st.w[0][0], column_scale(st.ws[0], false));
-    }
-    int g = kpart;
-    auto step = [&](auto S) {
-        load(std::integral_constant<int, (decltype(S)::value + DEPTH) % (DEPTH + 1)>{});
-        __builtin_amdgcn_sched_barrier(0);
-        compute(S);
-        g += KP;
-    };
-    // (whole turns of the ring in the loop, what is left behind it: leaving the loop in the middle of a turn makes the
-    // compiler carry two copies of the accumulators)
-    while (g + DEPTH * KP < kgroups) each(std::make_integer_sequence<int, DEPTH + 1>{}, step);
-    if (g < kgroups) step(std::integral_constant<int, 0>{});
-    if constexpr (DEPTH > 1) {
-        if (g < kgroups) step(std::integral_constant<int, 1>{});
-    }
-    if constexpr (DEPTH > 2) {
-        if (g < kgroups) step(std::integral_constant<int, 2>{});
-    }
-    if constexpr (!FP4 && LAG) {
+            for (int mt = 0; mt < MT; mt++) {
+                X[mt] = codes6(*(const u32x4_t *)(stage + mt * FRAG_BYTES + off16), *(const u32x2_t *)(stage + mt * FRAG_BYTES + off8));
+                as[mt] = *(const uint16_t *)(stage + 2 * FRAG_BYTES + (mt * 32 + r32) * 2);
+            }
+        };
+        // A wave's copy of a k-group has landed once no more requests are left than were made after it: three for its columns, then a copy and three more
+        // for every k-group requested behind it (each of them is used, so that the compiler drops none; what it waits for its own loads with
+        // does not count the copies and is stricter).  All waves' copies have landed behind the barrier.
+        auto landed = [&](auto BEHIND) { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(3 + 4 * decltype(BEHIND)::value) : "memory"); };
+        // A k-group and the LEFT that follow it and are requested by its end (DEPTH: one more is requested here)
+        auto body = [&](auto S, auto LEFT) {
+            constexpr int st = decltype(S)::value, left = decltype(LEFT)::value;
+            // (the stage was that of the k-group before this one, read before the last barrier)
+            if constexpr (left == DEPTH) request(std::integral_constant<int, (st + DEPTH) % RING>{});
+            __builtin_amdgcn_sched_barrier(0);
+            // the first tile's instructions, and between them the additions of the second one of the k-group before
+            auto add = [&](int mt) {
 #pragma unroll
-        for (int e = 0; e < 16; e++) acc[NT * MT - 1][e] = __builtin_fmaf(P[1][e], F[1][e], acc[NT * MT - 1][e]);
+                for (int e = 0; e < 16; e++) acc[mt][e] = __builtin_fmaf(P[mt][e], F[mt][e], acc[mt][e]);
+            };
+            P[0] = mfma_codes6(w[st], X[0]);
+            F[0] = mfma_factor(u32x2_t{ws[st], 0u}, u32x2_t{h ? 0u : as[0], 0u});
+            add(1);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 9, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            P[1] = mfma_codes6(w[st], X[1]);
+            F[1] = mfma_factor(u32x2_t{ws[st], 0u}, u32x2_t{h ? 0u : as[1], 0u});
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (left > 0) {
+                landed(std::integral_constant<int, left - 1>{});
+                read_rows(std::integral_constant<int, (st + 1) % RING>{});
+            }
+            add(0);
+            if constexpr (left == 0) add(1);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // What whole turns of the ring leave over of the k-groups before the last DEPTH comes first: the register sets at the end are then the same
+        // ones whatever their number (an end for each carried the accumulators through scratch memory).
+        constexpr std::integral_constant<int, DEPTH> ALL;
+        auto start = [&](auto ODD) {
+            constexpr int odd = decltype(ODD)::value;
+            each(std::make_integer_sequence<int, DEPTH>{}, [&](auto I) { request(std::integral_constant<int, (decltype(I)::value + RING - odd) % RING>{}); });
+            landed(std::integral_constant<int, DEPTH - 1>{});
+            read_rows(std::integral_constant<int, (RING - odd) % RING>{});
+            each(std::make_integer_sequence<int, odd>{}, [&](auto I) { body(std::integral_constant<int, (decltype(I)::value + RING - odd) % RING>{}, ALL); });
+        };
+        const int odd = (kgroups - DEPTH) % RING;  // (kgroups >= DEPTH)
+        each(std::make_integer_sequence<int, RING>{}, [&](auto O) {
+            if (odd == decltype(O)::value) start(O);
+        });
+        for (int g = odd; g + DEPTH < kgroups; g += RING) each(std::make_integer_sequence<int, RING>{}, [&](auto I) { body(I, ALL); });
+        each(std::make_integer_sequence<int, DEPTH>{}, [&](auto I) { body(I, std::integral_constant<int, DEPTH - 1 - decltype(I)::value>{}); });
+        // (the sums are wanted here: the compiler would move the last additions behind the epilogue's requests, and their operands to scratch memory)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) asm volatile("" : "+v"(acc[mt][e]));
+        __syncthreads();  // everybody has read the last stage: the slabs take the stages' place
+    } else {
+        each(std::make_integer_sequence<int, DEPTH>{}, [&](auto D) { load(D); });
+        if constexpr (FP4) {
+            auto &st = sets[0];
+            read_row_scales(st.as);
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) xop[0][mt] = dequant_word_fp4(st.x[mt][0], row_scale(mt, false));
+            wop[0] = dequant_word_fp4(st.w[0][0], column_scale(st.ws[0], false));
+        }
+        int g = kpart;
+        auto step = [&](auto S) {
+            load(std::integral_constant<int, (decltype(S)::value + DEPTH) % (DEPTH + 1)>{});
+            __builtin_amdgcn_sched_barrier(0);
+            compute(S);
+            g += KP;
+        };
+        // (whole turns of the ring in the loop, what is left behind it: leaving the loop in the middle of a turn makes the
+        // compiler carry two copies of the accumulators)
+        while (g + DEPTH * KP < kgroups) each(std::make_integer_sequence<int, DEPTH + 1>{}, step);
+        if (g < kgroups) step(std::integral_constant<int, 0>{});
+        if constexpr (DEPTH > 1) {
+            if (g < kgroups) step(std::integral_constant<int, 1>{});
+        }
+        if constexpr (DEPTH > 2) {
+            if (g < kgroups) step(std::integral_constant<int, 2>{});
+        }
+        if constexpr (!FP4 && LAG) {
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[NT * MT - 1][e] = __builtin_fmaf(P[1][e], F[1][e], acc[NT * MT - 1][e]);
+        }
     }
 
     // ---- the epilogue's own operands, requested before the waves meet ------------------------------------
@@ -296,7 +396,10 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
     // ---- the waves' sums meet, 32 rows at a time, added in ascending order of the waves ---------------------
     float16_t val[OWN];
     float4_t *park = (float4_t *)lds;
-    if constexpr (NARROW) {
+    if constexpr (STAGED) {
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) val[mt] = acc[mt];
+    } else if constexpr (NARROW) {
 #pragma unroll
         for (int t = 0; t < NT * MT; t++) {
             const int tile = t % MT * NC + cw * NT + t / MT;
@@ -337,7 +440,7 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
         __syncthreads();  // the sums have been read: the slabs take their place
     }
 
-    float *ssq = (float *)(lds + KP * 16384);  // [MT][4 column tiles][32 rows]
+    float *ssq = (float *)(lds + ssq_offset<MT, KP>());  // [MT][4 column tiles][32 rows]
     const bool rope = NEXT && p.rotary && n0 < p.rope_cols;  // the tile is one head of q or k
 #pragma unroll
     for (int o = 0; o < OWN; o++)
@@ -539,7 +642,7 @@ __global__ void __launch_bounds__(64 * WN * KP, 2) gemm_direct_kernel(GemmParams
 template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT>
 int launch_direct(const GemmParams &p, hipStream_t stream) {
     auto kern = gemm_direct_kernel<FP4, MT, NT, WN, KP, DEPTH, NEXT>;
-    constexpr int smem = lds_bytes<MT, NT * WN, KP>();
+    constexpr int smem = lds_bytes<MT, NT * WN, KP, DEPTH>();
     static bool lds_reserved[64] = {false};  // set once per device (racing first calls both set it, which is harmless)
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(SVDQ_ELAUNCH, "gemm: cannot identify the current device");

@@ -21,6 +21,13 @@ int launch_narrow(const GemmParams &p, int mt, hipStream_t stream) {
 #endif
 }
 
+// INT4, tiles of 64 rows x 128 columns whose waves split the columns only: plain epilogue (0), the others (1)
+#if SVDQ_VARIANT == 0
+int launch_staged_plain(const GemmParams &p, hipStream_t stream) { return launch_direct<false, 2, 1, 4, 1, 3, false>(p, stream); }
+#else
+int launch_staged_next(const GemmParams &p, hipStream_t stream) { return launch_direct<false, 2, 1, 4, 1, 3, true>(p, stream); }
+#endif
+
 int SVDQ_NAME(const GemmParams &p, bool fp4, int mt, hipStream_t stream) { return fp4 ? launch_narrow<true>(p, mt, stream) : launch_narrow<false>(p, mt, stream); }
 
 }  // namespace direct

@@ -2,6 +2,7 @@
 a launch takes, that no operand is read outside its buffer, and that the kernels keep out of scratch memory."""
 
 import ctypes
+import re
 
 import pytest
 
@@ -76,7 +77,7 @@ def test_addresses_stay_inside_their_buffers(fp4):
 def test_narrow_tiles_fit_their_registers(compiled, variant):  # noqa: F811
     usage, _ = compiled[("gemm_narrow_variant.hip", variant)]
     kernels = {k: u for k, u in usage.items() if "gemm_direct_kernel" in k}
-    assert len(kernels) == 4, list(usage)
+    assert len(kernels) == 5, list(usage)  # two tiles of either precision, and one whose waves share the rows' operands
     for name, u in kernels.items():
         assert u["VGPRs"] <= 256 and u["AGPRs"] == 0 and u["ScratchSize"] == 0 and u["Occupancy"] >= 2, (name, u)
 
@@ -84,8 +85,52 @@ def test_narrow_tiles_fit_their_registers(compiled, variant):  # noqa: F811
 # On either side of the lines between the few-rows kernel and the large tiles that the factors in choose_direct draw.
 @pytest.mark.parametrize("kind,M,K,N,fp4,few", [
     ("plain", 1131, 2048, 10112, True, 2), ("plain", 4608, 15360, 3072, True, 0), ("rope", 1614, 3968, 11904, True, 2), ("next", 2154, 1792, 7168, True, 2),
-    ("plain", 225, 4992, 10624, False, 2), ("plain", 175, 9984, 14976, False, 2), ("plain", 506, 9600, 6912, False, 0), ("next", 1486, 1024, 4096, False, 2),
+    ("plain", 225, 4992, 10624, False, 2), ("plain", 175, 9984, 14976, False, 2), ("plain", 261, 1152, 14208, False, 0), ("next", 1486, 1024, 4096, False, 2),
     ("next", 1486, 2048, 8192, False, 0),
 ])
 def test_few_rows_or_large_tiles(kind, M, K, N, fp4, few):
     assert plan_of(call(kind, M, K, N, 32, fp4)).few_rows == few
+
+
+@pytest.mark.parametrize("variant", [0, 1])
+def test_waits_for_the_copies_of_shared_rows(compiled, variant):  # noqa: F811
+    """The kernels whose waves share the rows' operands wait for an asynchronous copy by the number of requests made after it: three for
+    the columns behind every copy, none dropped, none of another kind between them."""
+    _, lines = compiled[("gemm_narrow_variant.hip", variant)]
+    text = "\n".join(lines)
+    start = next(m.start() for m in re.finditer(r"^_ZN\S*gemm_direct_kernelILb0ELi2ELi1ELi4E\S*:", text, re.M))
+    body = text[start:text.index("s_endpgm", start)].split("\n")
+    ops = []
+    for line in body:
+        t = line.strip()
+        wait = re.match(r"s_waitcnt vmcnt\((\d+)\) lgkmcnt\(0\)$", t)
+        if t.startswith("global_load_lds"):
+            ops.append("C")
+        elif re.match(r"(global|buffer|flat|scratch)_(load|store|atomic)", t):
+            ops.append("w")
+        elif wait and int(wait[1]) % 4 == 3:
+            ops.append(str(int(wait[1]) // 4))
+        elif t.startswith("s_barrier"):
+            ops.append("B")
+    main = "".join(ops)
+    main = main[:main.index("0B") + 2]  # (the last wait leaves the last k-group's own requests)
+    assert re.fullmatch(r"((Cwww)+2B|1B|0B)+", main), main
+    assert set(re.findall(r"(?:Cwww)+", main)) <= {"Cwww", "Cwww" * 3}, main  # a k-group's, or the first three k-groups'
+    assert re.search(r"2B1B0B$", main), main
+
+
+def test_addresses_of_shared_rows():
+    """The asynchronous copies of a k-group's rows (three KB of two fragments, 128 bytes of scales) and the columns' operands."""
+    for M, K, N in ((1, 256, 128), (100, 640, 768), (505, 3072, 6144), (1153, 512, 3072)):
+        M_pad, kgroups, padded = (M + 255) // 256 * 256, K // 64, (N + 255) // 256 * 256
+        act_bytes, asc_bytes, wgt_bytes, wsc_bytes = M_pad * K * 3 // 4, kgroups * M_pad * 2, padded * K * 3 // 4, padded // 256 * kgroups * 2048
+        for f0 in range(0, (M + 63) // 64 * 2, 2):
+            for g in (0, kgroups - 1):
+                first = (f0 // 4 * kgroups + g) * 4 * FRAG + f0 % 4 * FRAG
+                assert first % 16 == 0 and first + 2 * 1024 + 63 * 16 + 16 == first + 2 * FRAG <= act_bytes
+                assert (g * M_pad + f0 * 32) * 2 % 16 == 0 and (g * M_pad + f0 * 32) * 2 + 7 * 16 + 16 <= asc_bytes
+        for nb in range(N // 128):
+            for wave in range(4):
+                tile = nb % 2 * 4 + wave
+                assert (nb // 2 * kgroups + kgroups - 1) * 8 * FRAG + tile * FRAG + 1024 + 63 * 8 + 8 <= wgt_bytes
+                assert (nb // 2 * kgroups + kgroups - 1) * 2048 + tile * 256 + 31 * 8 + 4 <= wsc_bytes
