@@ -659,14 +659,17 @@ FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu) {
     return best;
 }
 
-// INT4 launches whose tiles of 64 x 128 are between one and two per compute unit: the waves split the columns and share the rows' operands
-// through LDS (gemm_direct_kernel.h).  A tile alone on its compute unit is a chain of latencies, 0.22 us per k-group, two overlap; three
-// issue more instructions per product than the large tiles.  Layer calls, the best other form / this one, K = 3072: QKV M = 256, N = 9216 26.9 / 24.7
-// us, M = 505 (2.25 tiles) 32.4 / 33.7; plain M = 384, N = 9216 25.0 / 23.3, M = 256 22.3 / 23.0 (1.1 tiles, where narrow tiles are better).  On average over
-// 5000 layers: with the norm and rotation 6.5 % faster from 1 to 2 tiles, MLPs 4 %, plain 0 at 1.5, 4 to 9 % from 1.6 to 2; 1 to 4 % slower beyond.
+// INT4 launches whose tiles of 64 x 128 are between one and two per compute unit (three with the quantizing epilogue, one and a half and two with the
+// plain one): the waves split the columns and share the rows' operands through LDS (gemm_direct_kernel.h).  A tile alone on its
+// compute unit is a chain of latencies, 0.2 us per k-group, two overlap; more issue more instructions per product than the large tiles.  Layer calls,
+// the best other form / this one, us: QKV M = 256, K = 3072, N = 9216 27.2 / 23.5, M = 505, K = 2048 22.0 / 19.5, at 2.25 tiles M = 505, K = 3072 32.6 / 33.8, at 0.75
+// M = 256, K = 2048 15.7 / 17.4; MLP M = 256, K = 3072 52.4 / 48.8, M = 505 (three tiles) 78.6 / 75.1, M = 600 79.8 / 85.1; plain M = 384, K = 3072, N = 9216
+// 26.3 / 22.8, M = 320 (1.4 tiles, where narrow ones are better) 22.4 / 22.6, M = 505 30.4 / 32.1.
 bool staged_rows(const svdq_gemm_args *a, int ncu) {
+    if (a->fp4 || a->K < 256) return false;
     const long long tiles = (rows_needed(a) + 63) / 64 * (a->N / 128);
-    return !a->fp4 && a->K >= 256 && tiles <= 2 * ncu && (needs_next_epilogue(a) ? tiles > ncu : 5 * tiles > 8 * ncu);
+    if (!needs_next_epilogue(a)) return 2 * tiles >= 3 * ncu && tiles <= 2 * ncu;
+    return tiles > ncu && tiles <= (a->qout ? 3 : 2) * ncu;
 }
 
 // Which of the two shapes of the few-rows kernel (0: neither) a launch takes.  Shape 1: tiles of 32 rows, four waves split

@@ -61,8 +61,8 @@ constexpr int ssq_offset() {
     return KP * 16384 > MT * SLAB_BYTES ? KP * 16384 : MT * SLAB_BYTES;
 }
 // Waves that split the columns only (WN = 4, INT4, 64 rows): a stage of the rows' operands of one k-group in LDS, two fragments and the scales of
-// 64 rows, eight times over in a whole KB.
-constexpr int STAGE_BYTES = 2 * FRAG_BYTES + 1024;
+// 64 rows, eight times over in a whole KB; behind them zeros, what the upper half-wave reads as its scale.
+constexpr int STAGE_ZEROS = 2 * FRAG_BYTES + 1024, STAGE_BYTES = STAGE_ZEROS + 128;
 template <int MT, int NC, int KP, int DEPTH>
 constexpr int lds_bytes() {
     constexpr int epilogue = NC == 4 ? ssq_offset<MT, KP>() + MT * 512 : KP * MT * NC * 4096 + MT * NC * NARROW_SLAB_BYTES;
@@ -239,32 +239,46 @@ __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_ker
         // Every wave multiplies one column tile by both row blocks: the columns' operands come straight to registers, DEPTH k-groups ahead, the
         // rows', which all four need, to LDS by asynchronous copies, a KB per wave and k-group, into DEPTH + 1 stages.  Six fragments per
         // k-group and tile where waves that split K two ways fetch eight, no sums to exchange, 32 accumulators per lane.  One tile per compute unit
-        // takes 0.22 us per k-group with three on their way (0.33 with two: the latency of the requests), two or three share it better than
-        // that, until the vector instructions bound them (which launches, and what they gain: staged_rows in gemm.hip).
+        // takes 0.2 us per k-group with three on their way (0.33 with two: the latency of the requests), two share it better than that, until the
+        // vector instructions bound them: 50 per k-group, with the columns through buffers and the scales as lasting pairs (61 before: QKV M = 256, K =
+        // 3072, N = 9216 24.7 -> 23.5 us).  Which launches, and what they gain: staged_rows in gemm.hip.
         const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds + wave * 1024;
         const bool rows = wave < 3;
         const uint8_t *src = rows ? p.act + ((size_t)(f0 >> 2) * kgroups) * (4 * FRAG_BYTES) + (f0 & 3) * FRAG_BYTES + wave * 1024 : (const uint8_t *)(p.ascales + f0 * 32);
         const uint32_t stride = rows ? 4 * FRAG_BYTES : (uint32_t)p.M_pad * 2, voff = rows ? lane * 16 : (lane & 7) * 16;
         constexpr int RING = DEPTH + 1;
         v6i_t w[RING];
-        uint32_t ws[RING];
+        u32x2_t ws[RING], as[MT];  // (pairs whose second register stays zero: opaque, so that it is not made again with every scale)
+#pragma unroll
+        for (int i = 0; i < RING; i++) {
+            ws[i] = u32x2_t{0u, 0u};
+            asm volatile("" : "+v"(ws[i]));
+        }
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            as[i] = u32x2_t{0u, 0u};
+            asm volatile("" : "+v"(as[i]));
+        }
+        if (threadIdx.x < RING * 32) *(uint32_t *)(lds + (threadIdx.x >> 5) * STAGE_BYTES + STAGE_ZEROS + (threadIdx.x & 31) * 4) = 0u;
+        const uint32_t off_rows = h ? (uint32_t)STAGE_ZEROS : 2u * FRAG_BYTES + (uint32_t)r32 * 2u;
+        const __amdgpu_buffer_rsrc_t wbuf = buffer(wp, (uint32_t)(kgroups - 1) * (8 * FRAG_BYTES) + FRAG_BYTES), sbuf = buffer(sp, (uint32_t)(kgroups - 1) * 2048 + 256);
+        int g_req = 0;
         auto request = [&](auto S) {
             constexpr int st = decltype(S)::value;
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(base + st * STAGE_BYTES), "v"(voff), "s"(src) : "memory", "m0");
-            w[st] = codes6(*(const u32x4_t *)(wp + off16), *(const u32x2_t *)(wp + off8));
-            ws[st] = *(const uint32_t *)(sp + off_ws);
+            w[st] = codes6(__builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(wbuf, off16, g_req * (8 * FRAG_BYTES), 0)),
+                           __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(wbuf, off8, g_req * (8 * FRAG_BYTES), 0)));
+            ws[st][0] = __builtin_amdgcn_raw_buffer_load_b32(sbuf, off_ws, g_req * 2048, 0);
             src += stride;
-            wp += 8 * FRAG_BYTES;
-            sp += 2048;
+            g_req++;
         };
         v6i_t X[MT];
-        uint32_t as[MT];
         auto read_rows = [&](auto S) {
             const uint8_t *stage = lds + decltype(S)::value * STAGE_BYTES;
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) {
                 X[mt] = codes6(*(const u32x4_t *)(stage + mt * FRAG_BYTES + off16), *(const u32x2_t *)(stage + mt * FRAG_BYTES + off8));
-                as[mt] = *(const uint16_t *)(stage + 2 * FRAG_BYTES + (mt * 32 + r32) * 2);
+                as[mt][0] = *(const uint16_t *)(stage + mt * 64 + off_rows);
             }
         };
         // A wave's copy of a k-group has landed once no more requests are left than were made after it: three for its columns, then a copy and three more
@@ -283,7 +297,7 @@ __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_ker
                 for (int e = 0; e < 16; e++) acc[mt][e] = __builtin_fmaf(P[mt][e], F[mt][e], acc[mt][e]);
             };
             P[0] = mfma_codes6(w[st], X[0]);
-            F[0] = mfma_factor(u32x2_t{ws[st], 0u}, u32x2_t{h ? 0u : as[0], 0u});
+            F[0] = mfma_factor(ws[st], as[0]);
             add(1);
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
@@ -291,7 +305,7 @@ __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_ker
             __builtin_amdgcn_sched_group_barrier(0x002, 9, 0);
             __builtin_amdgcn_sched_barrier(0);
             P[1] = mfma_codes6(w[st], X[1]);
-            F[1] = mfma_factor(u32x2_t{ws[st], 0u}, u32x2_t{h ? 0u : as[1], 0u});
+            F[1] = mfma_factor(ws[st], as[1]);
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (left > 0) {
                 landed(std::integral_constant<int, left - 1>{});
