@@ -514,12 +514,12 @@ int project_further(const QuantParams &p0, hipStream_t stream) {
     return SVDQ_OK;
 }
 
-template <int FEW, bool FP4>
+template <int FEW, bool FP4, int NW = 8>
 int launch_few_rows(const QuantParams &p, hipStream_t stream) {
     constexpr int RTW = FEW == 2 ? 2 : 1;
     const dim3 grid(p.M_pad / 16, p.splits + (p.R / 16 + RTW - 1) / RTW);
-    if (p.smooth_rcp) SVDQ_LAUNCH((quantize_fuse_lora_kernel<8, 1, 1, 1, FP4, 2, false, false, true, FEW>), grid, dim3(512), 0, stream, p);
-    else SVDQ_LAUNCH((quantize_fuse_lora_kernel<8, 1, 1, 1, FP4, 0, false, false, true, FEW>), grid, dim3(512), 0, stream, p);
+    if (p.smooth_rcp) SVDQ_LAUNCH((quantize_fuse_lora_kernel<NW, 1, 1, 1, FP4, 2, false, false, true, FEW>), grid, dim3(64 * NW), 0, stream, p);
+    else SVDQ_LAUNCH((quantize_fuse_lora_kernel<NW, 1, 1, 1, FP4, 0, false, false, true, FEW>), grid, dim3(64 * NW), 0, stream, p);
     return check_launch("quantize_w4a4_act_fuse_lora (few rows)");
 }
 
@@ -530,14 +530,14 @@ int launch_few_rows(const QuantParams &p, hipStream_t stream) {
 //          rank 128  M = 2304 19.1 / 11.4, M = 3072 21.8 / 15.3, M = 4096 23.5 / 21.7, M = 4608 24.9 / 24.7; K = 12288: M = 3072 73.6 / 61.0, M = 4096 74.5 / 84.4
 //          rank 32   M = 2304 7.4 / 7.2, M = 3072 7.9 / 8.0
 //   NVFP4  rank 64   M = 2304 15.3 / 7.4, M = 4608 16.7 / 14.2, M = 6144 18.4 / 19.7; K = 12288: M = 3072 47.6 / 41.5, M = 4096 48.6 / 49.2
-//          rank 128  M = 4608 29.4 / 20.5, M = 6144 30.5 / 28.0, M = 7168 30.8 / 33.5; K = 12288: M = 4608 98.5 / 88.5, M = 6144 99.6 / 118
-//          rank 32   M = 2304 7.8 / 6.5, M = 4096 9.1 / 8.0, M = 4608 13.1 / 12.3 (the layer is no faster); K = 2304: M = 4608 10.7 / 9.8; K = 6144: M = 4096 17.1 / 16.0, M = 4608 24.2 / 25.9
+//          rank 128  M = 3072 22.8 / 12.8, M = 4608 29.4 / 22.1, M = 6144 30.4 / 27.3; K = 12288: M = 2304 93.5 / 41.4, M = 4608 99.0 / 98.0
+//          rank 32   M = 2304 7.8 / 6.5, M = 4096 9.1 / 8.0; K = 6144: M = 4096 17.1 / 16.0 (M = 4608 is another number of waves, see dispatch)
 //          rank 16   M = 2304 7.6 / 6.5, M = 4096 8.8 / 9.2
 int few_rows_most(int RT, int K, bool fp4) {
     if (RT > 8) return 8;
     if (!fp4) return RT <= 2 ? 8 : K <= 4096 ? 16 : 12;
     if (RT == 1) return K <= 6144 ? 9 : 8;
-    if (RT == 2) return K <= 2304 ? 18 : K <= 6144 ? 16 : 8;
+    if (RT == 2) return K <= 6144 ? 16 : 8;
     if (RT <= 4) return K <= 4096 ? 18 : K <= 6144 ? 16 : 12;
     return K <= 3072 ? 24 : 18;
 }
@@ -565,8 +565,8 @@ int dispatch(const QuantParams &p, hipStream_t stream) {
         // M = 2048 37.8 with two, one 42.5, three 43.4; M = 1024 18.8 with four).  Over 224 shapes (K = 1280 ... 12288, M = 256 ... 2048, ranks 16 ...
         // 128, both precisions) 1.3 % off the fastest division measured, 2.5 % at most behind the rule before, which was 5.4 % off.
         // More rows than 8 per compute unit: two shares of the quantizing where that takes no more rounds of the workgroups that are resident
-        // at once than one (M = 3072, rank 64: 10.7 us, with one 11.0; M = 2304, rank 64 8.2 with one, two 9.3), one in INT4 at ranks above 64 (M = 2304, rank
-        // 128, K = 12288: 43.9, with two 52.0; NVFP4 51.0 and 47.1).
+        // at once than one (M = 3072, rank 64: 10.7 us, with one 11.0; M = 2304, rank 64 8.2 with one, two 9.3), one at ranks above 64 (M = 2304, rank
+        // 128, K = 12288: 43.9, with two 52.0).
         if (RT == 0 ? p.M_pad <= 8 * ncu : p.M_pad <= few_rows_most(RT, p.K, FP4) * ncu) {
             QuantParams q = p;
             const int row_blocks = p.M_pad / 16, most = (p.K / 128 + 7) / 8;
@@ -581,7 +581,13 @@ int dispatch(const QuantParams &p, hipStream_t stream) {
             if (RT == 1 && p.K > 9216 && q.splits < 2) q.splits = 2;
             if (p.M_pad > 8 * ncu) {
                 auto rounds = [&](int splits) { return (row_blocks * (splits + projecting) + 2 * ncu - 1) / (2 * ncu); };
-                q.splits = (FP4 || projecting <= 2) && rounds(2) == rounds(1) ? 2 : 1;
+                q.splits = projecting <= 2 && rounds(2) == rounds(1) ? 2 : 1;
+                // (the waves' sums are those of the form that more rows take, bit for bit: in another order they move 4-bit codes of an MLP's second layer.
+                // NVFP4 at ranks above 64 therefore has four waves, which are faster too: M = 3072, rank 128 12.8 us, eight 13.4, M = 2304 10.1 and 10.7)
+                if constexpr (FP4) {
+                    q.splits = RT > 4 ? 1 : q.splits;
+                    if (RT > 4) return launch_few_rows<2, FP4, 4>(q, stream);
+                }
             }
             if (q.splits > most) q.splits = most;
             if (!one) return launch_few_rows<2, FP4>(q, stream);

@@ -33,3 +33,15 @@ def test_quantizing_and_projecting_apart_beyond_8_rows_per_compute_unit(dev, M, 
     that end early; long rows with fewer chunks on their way."""
     announce(f"apart M={M} K={K} R={R} fp4={fp4}")
     _check_row_sample(dev, M, K, R, fp4, True)
+
+
+@pytest.mark.parametrize("K,R,fp4,apart,together", [(1152, 64, False, 2304, 4608), (640, 112, True, 2304, 9216), (1152, 48, True, 3072, 9216), (640, 32, True, 4096, 2048)])
+def test_projections_keep_their_bits_from_form_to_form(dev, K, R, fp4, apart, together):
+    """A row's projection is the same whether quantizing and projecting are apart or not: the sums of the waves are added in one order."""
+    from gpu_util import make_module
+
+    announce(f"projection bits K={K} R={R} fp4={fp4}")
+    m = make_module(synth.make_layer(128, K, R, seed=R, fp4=fp4), dev)
+    x = synth.make_activations(max(apart, together), K, seed=K).to(dev)
+    n = min(apart, together)
+    assert m.quantize(x[:apart])[2][:n].equal(m.quantize(x[:together])[2][:n])
