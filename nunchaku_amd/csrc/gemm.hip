@@ -637,24 +637,25 @@ int gemm_fp4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t st
 //          M = 64, K = 12288     32.3 / 21.4 (32 x 32)           34.6 / 21.6
 //          M = 256, K = 12288    34.7 / 30.3 (64 x 64)           37.4 / 34.0
 struct FewRowsTile {
-    int mt, nc;  // blocks of 32 rows, of 32 columns
-    double launch, tile, kgroup;
+    int mt, nc;  // blocks of 32 rows, of 32 columns (none: large tiles)
+    bool shared_rows;
     double time;
 };
 FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu) {
-    constexpr FewRowsTile int4[] = {{1, 1, -0.18, 0.18, 0.0382, 0.0}, {1, 2, -0.46, 0.68, 0.0551, 0.0}, {2, 1, -0.46, 0.75, 0.0499, 0.0},
-                                    {2, 2, 0.18, 0.64, 0.0702, 0.0},  {1, 4, -0.13, 0.64, 0.0948, 0.0}, {2, 4, 1.04, 0.53, 0.1378, 0.0}};
-    constexpr FewRowsTile nvfp4[] = {{1, 1, -0.85, 0.16, 0.0323, 0.0}, {1, 2, -0.52, 0.14, 0.0515, 0.0}, {2, 1, -0.64, 0.24, 0.0498, 0.0},
-                                     {2, 2, -0.17, 0.46, 0.0719, 0.0}, {1, 4, 0.22, 0.47, 0.0876, 0.0},  {2, 4, 1.96, -0.07, 0.1112, 0.0}};
+    struct Model {
+        int mt, nc;
+        double launch, tile, kgroup;
+    };
+    constexpr Model int4[] = {{1, 1, -0.18, 0.18, 0.0382}, {1, 2, -0.46, 0.68, 0.0551}, {2, 1, -0.46, 0.75, 0.0499},
+                              {2, 2, 0.18, 0.64, 0.0702},  {1, 4, -0.13, 0.64, 0.0948}, {2, 4, 1.04, 0.53, 0.1378}};
+    constexpr Model nvfp4[] = {{1, 1, -0.85, 0.16, 0.0323}, {1, 2, -0.52, 0.14, 0.0515}, {2, 1, -0.64, 0.24, 0.0498},
+                               {2, 2, -0.17, 0.46, 0.0719}, {1, 4, 0.22, 0.47, 0.0876},  {2, 4, 1.96, -0.07, 0.1112}};
     const long long row_blocks = (rows_needed(a) + 31) / 32, column_blocks = a->N / 32;
     FewRowsTile best{};
-    for (const FewRowsTile &c : a->fp4 ? nvfp4 : int4) {
-        const long long tiles = (row_blocks + c.mt - 1) / c.mt * (column_blocks / c.nc);
-        const double t = c.launch + (double)((tiles + ncu - 1) / ncu) * (c.tile + c.kgroup * (double)(a->K / 64));
-        if (best.mt == 0 || t < best.time) {
-            best = c;
-            best.time = t;
-        }
+    for (const Model &m : a->fp4 ? nvfp4 : int4) {
+        const long long tiles = (row_blocks + m.mt - 1) / m.mt * (column_blocks / m.nc);
+        const double t = m.launch + (double)((tiles + ncu - 1) / ncu) * (m.tile + m.kgroup * (double)(a->K / 64));
+        if (best.mt == 0 || t < best.time) best = FewRowsTile{m.mt, m.nc, false, t};
     }
     return best;
 }
@@ -672,8 +673,8 @@ bool staged_rows(const svdq_gemm_args *a, int ncu) {
     return tiles > ncu && tiles <= (a->qout ? 3 : 2) * ncu;
 }
 
-// Which of the two shapes of the few-rows kernel (0: neither) a launch takes.  Shape 1: tiles of 32 rows, four waves split
-// K.  Shape 2: tiles of 64 rows, a quarter fewer operand bytes per product, from about 400 tiles of 32 rows on; INT4: two waves
+// Which tiles of the few-rows kernel a launch takes, if any.  Shape 1: tiles of 32 rows x 128 columns, four waves split
+// K.  Shape 2: tiles of 64 rows x 128 columns, a quarter fewer operand bytes per product, from about 400 tiles of 32 rows on; INT4: two waves
 // split K and two the columns, NVFP4: four waves split K.  Models of the time in us fitted to launches at K = 1024 ... 12288
 // on 256 compute units, linear in the number of tiles that the busiest compute unit works through and in the k-groups; they met
 // the measurements within about 10 % when they were fitted, over 2200 random shapes; what has changed since is in the factors below.  Measured at K = 3072 at the time of the fit, large tiles (split along K where that pays) / shape 1 / shape 2:
@@ -688,10 +689,12 @@ bool staged_rows(const svdq_gemm_args *a, int ncu) {
 //          M = 1157            66.6 / 86.6 / 65.6           127.5 / 99.5 / 81.2
 // (Since then: INT4 large tiles 3 to 10 % faster, M = 505, N = 9216 24.9, M = 1024, N = 9216 32.3; NVFP4 large tiles with the quantizing epilogue M = 1157,
 // N = 12288 100; NVFP4 in the few-rows kernel M = 1157, K = 12288 76.4.)
-int choose_direct(const svdq_gemm_args *a, int ncu) {
-    if (a->k_split > 0) return 0;  // (the caller asks for the tiles that k_split is about)
-    if (((uintptr_t)a->bias | (uintptr_t)a->wcscales | (uintptr_t)a->oscales) % 8 || (uintptr_t)a->colnorm % 16) return 0;  // (read four columns at a time)
-    if (staged_rows(a, ncu)) return 2;
+FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
+    constexpr FewRowsTile none{};
+    if (a->k_split > 0) return none;  // (the caller asks for the tiles that k_split is about)
+    if (((uintptr_t)a->bias | (uintptr_t)a->wcscales | (uintptr_t)a->oscales) % 8 || (uintptr_t)a->colnorm % 16) return none;  // (read four columns at a time)
+    if (staged_rows(a, ncu)) return FewRowsTile{2, 4, true};
+    const bool plain = !needs_next_epilogue(a);
     const int rows = rows_needed(a), kg = (int)(a->K / 64);
     const long long ncols = a->N / 128;
     const double c1 = (double)((((rows + 31) / 32) * ncols + ncu - 1) / ncu), c2 = (double)((((rows + 63) / 64) * ncols + ncu - 1) / ncu);
@@ -733,55 +736,54 @@ int choose_direct(const svdq_gemm_args *a, int ncu) {
         t2 = 3.3 + c2 * (1.6 + 0.158 * kg);
         if (a->qout) {
             t_large *= 1.05;  // (1158 MLPs of 100 ... 2600 rows: 0.4 % off the fastest, 0.7 without; M = 1486, K = 1024 51.3 -> 45.8 us)
-        } else if (!needs_next_epilogue(a)) {
+        } else if (plain) {
             // (the plain epilogue's tiles are faster than these two, the model of their time has no offset: 2277 layers of 100 ... 2600 rows 0.3 % off the
             // fastest, 0.6 without; M = 225, K = 4992, N = 10624 36.4 -> 30.5 us, M = 175, K = 9984, N = 14976 59 -> 51, M = 261, K = 1152, N = 14208 18 -> 17)
             const double t_plain = 5.0 + 1.3 * plain_tile(a, ncu).time;
-            if (t_plain < t_large) return t1 < t2 ? 1 : 2;
+            if (t_plain < t_large) return plain_tile(a, ncu);
             t_large *= 0.95;
         }
     }
-    if (t1 < t2) return t1 < t_large ? 1 : 0;
-    return t2 < t_large ? 2 : 0;
+    if ((t1 < t2 ? t1 : t2) >= t_large) return none;
+    return plain ? plain_tile(a, ncu) : FewRowsTile{t1 < t2 ? 1 : 2, 4};
 }
 
 // Which kernel a call takes and how it divides the work.  A function of the arguments and the number of compute units alone:
 // the entry points with and without an allocation give the same bits.
 void make_plan(const svdq_gemm_args *a, int ncu, svdq_gemm_plan *plan) {
     *plan = svdq_gemm_plan{};
-    int shape = choose_direct(a, ncu);
+    FewRowsTile t = choose_direct(a, ncu);
     // Its shares are those of 128 columns and 32 rows each.  Where only the shares of the INT4 kernel's larger tiles fit the fixed
     // scratch, that one is taken.  (NVFP4: the shares of both kernels are as many.)
-    if (shape && !a->fp4) {
+    if (t.mt && !a->fp4) {
         auto shares = [&](int64_t column_blocks, int64_t row_blocks) {
             return (a->next_lora_down ? lora_share_bytes(a, column_blocks) : 0) + (a->out_vk ? vk_share_bytes(a, row_blocks) : 0);
         };
-        if (shares(a->N / 128, a->M_pad / 32) > NOALLOC_SCRATCH_BYTES && shares((a->N + g6::BN - 1) / g6::BN, a->M_pad / g6::BM) <= NOALLOC_SCRATCH_BYTES) shape = 0;
+        if (shares(a->N / 128, a->M_pad / 32) > NOALLOC_SCRATCH_BYTES && shares((a->N + g6::BN - 1) / g6::BN, a->M_pad / g6::BM) <= NOALLOC_SCRATCH_BYTES) t = FewRowsTile{};
     }
-    plan->few_rows = shape;
-    if (shape) plan->row_blocks = (rows_needed(a) + 32 * shape - 1) / (32 * shape);  // (shape s: tiles of 32 s rows)
-    else if (a->fp4) plan_fp4(a, ncu, plan);
-    else plan_int4(a, ncu, plan);
+    if (t.mt) {
+        plan->few_rows = t.mt;
+        plan->columns = 32 * t.nc;
+        plan->shared_rows = t.shared_rows;
+        plan->row_blocks = (rows_needed(a) + 32 * t.mt - 1) / (32 * t.mt);
+    } else if (a->fp4) {
+        plan_fp4(a, ncu, plan);
+    } else {
+        plan_int4(a, ncu, plan);
+    }
 }
 
-int gemm_direct(const svdq_gemm_args *a, const svdq_gemm_plan &plan, int ncu, hipStream_t st, int dev, bool noalloc) {
+int gemm_direct(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t st, int dev, bool noalloc) {
     GemmParams p;
     fill_params(a, p);
-    const bool next = needs_next_epilogue(a);
-    int shape = plan.few_rows;
     p.row_blocks = plan.row_blocks;
-    if (shape == 2 && staged_rows(a, ncu)) {
-        if (!next) return direct::launch_staged_plain(p, st);
-    } else if (!next) {
-        const FewRowsTile t = plain_tile(a, ncu);
-        p.row_blocks = ((int)rows_needed(a) + 32 * t.mt - 1) / (32 * t.mt);
-        if (t.nc < 4) return t.nc == t.mt ? direct::launch_square(p, a->fp4 != 0, t.mt, st) : direct::launch_oblong(p, a->fp4 != 0, t.mt, st);
-        shape = t.mt;
-    }
+    const bool next = needs_next_epilogue(a), fp4 = a->fp4 != 0;
+    const int mt = plan.few_rows;
     auto launch = [&]() {
-        if (a->fp4) return next ? direct::launch_fp4_next(p, shape, st) : direct::launch_fp4_plain(p, shape, st);
-        if (shape == 2 && staged_rows(a, ncu)) return direct::launch_staged_next(p, st);
-        return next ? direct::launch_int4_next(p, shape, st) : direct::launch_int4_plain(p, shape, st);
+        if (plan.columns < 128) return plan.columns == 32 * mt ? direct::launch_square(p, fp4, mt, st) : direct::launch_oblong(p, fp4, mt, st);
+        if (plan.shared_rows) return next ? direct::launch_staged_next(p, st) : direct::launch_staged_plain(p, st);
+        if (fp4) return next ? direct::launch_fp4_next(p, mt, st) : direct::launch_fp4_plain(p, mt, st);
+        return next ? direct::launch_int4_next(p, mt, st) : direct::launch_int4_plain(p, mt, st);
     };
     // every 128-column chunk's share of the next layer's low-rank projection, every 32-row block's linear-attention sums
     const size_t share_bytes = p.next_down ? lora_share_bytes(a, a->N / 128) : 0;
@@ -887,7 +889,7 @@ int gemm_entry(const svdq_gemm_args *a, void *stream, bool noalloc) {
     if (ncu <= 0) return fail(SVDQ_ELAUNCH, "gemm: cannot query the number of compute units");
     svdq_gemm_plan plan;
     make_plan(a, ncu, &plan);
-    if (plan.few_rows) return gemm_direct(a, plan, ncu, (hipStream_t)stream, dev, noalloc);
+    if (plan.few_rows) return gemm_direct(a, plan, (hipStream_t)stream, dev, noalloc);
     return a->fp4 ? gemm_fp4(a, plan, (hipStream_t)stream, dev, noalloc) : gemm_int4(a, plan, (hipStream_t)stream, dev, noalloc);
 }
 }  // namespace
@@ -919,16 +921,6 @@ extern "C" int svdq_gemm_plan_of(const svdq_gemm_args *a, int64_t rows, int comp
     if (!a->out) some.M_out = rows;
     const int rc = check_arguments(&some);
     if (rc == SVDQ_OK) make_plan(&some, compute_units, plan);
-    return rc;
-}
-
-extern "C" int svdq_gemm_plain_tile_of(const svdq_gemm_args *a, int compute_units, int32_t *rows, int32_t *columns) {
-    SVDQ_REQUIRE(rows && columns && compute_units > 0, "gemm: where does the tile go");
-    const int rc = check_arguments(a);
-    if (rc != SVDQ_OK) return rc;
-    const FewRowsTile t = plain_tile(a, compute_units);
-    *rows = 32 * t.mt;
-    *columns = 32 * t.nc;
     return rc;
 }
 

@@ -14,22 +14,20 @@ int svdq_gemm_w4a4_rows(const svdq_gemm_args *args, int64_t rows, int noalloc, v
 
 // Which kernel a GEMM call takes and how it divides the work (zero where a field does not apply).
 typedef struct svdq_gemm_plan {
-    int32_t few_rows;      // 0: a kernel with large tiles; 1, 2: the few-rows kernel in tiles of 32, 64 rows x 128 columns (plain epilogue: see below)
-    int32_t row_blocks;    // few rows: tiles along M
+    int32_t few_rows;      // 0: a kernel with large tiles; 1, 2: the few-rows kernel in tiles of 32, 64 rows,
+    int32_t row_blocks;    // so many along M
     int32_t full_blocks;   // INT4, large tiles: row blocks of 128 rows,
     int32_t half_blocks;   // of 64 rows behind them,
     int32_t kparts;        // and parts along K of every tile
     int32_t workgroups;    // NVFP4, large tiles: persistent workgroups;
     int32_t shared_tiles;  // some tiles are shared by two or more of them
+    int32_t columns;       // few rows: columns of a tile (32, 64 or 128),
+    int32_t shared_rows;   // its waves split the columns and share the rows' operands through LDS
 } svdq_gemm_plan;
 
 // What svdq_gemm_w4a4 (`rows` > 0: svdq_gemm_w4a4_rows) would do with these arguments on a GPU of so many compute units.  Checks the
 // arguments as the call does, launches nothing and needs no GPU.
 int svdq_gemm_plan_of(const svdq_gemm_args *args, int64_t rows, int compute_units, svdq_gemm_plan *plan);
-
-// The tile of a few-rows launch that writes `out` alone, without norm, rotation, SiLU or linear-attention sums: such a launch chooses among
-// more tiles than the plan's two.
-int svdq_gemm_plain_tile_of(const svdq_gemm_args *args, int compute_units, int32_t *rows, int32_t *columns);
 
 // The work of workgroup `block` of an INT4 launch with large tiles.
 typedef struct svdq_gemm_tile {

@@ -2,13 +2,11 @@
 large tiles (``K_SPLIT = 1``): rows and columns that end inside a tile, fewer k-groups than waves and counts that the ring of requests
 does not divide, ranks 0 to 80, outputs narrower than the padded layer, and no byte written outside the output."""
 
-import ctypes
-
 import pytest
 import torch
 
 from conftest import announce
-from gpu_util import Guarded, bf16_ulp, make_module
+from gpu_util import Guarded, bf16_ulp, make_module, record_plans
 from oracle import synth
 
 pytestmark = pytest.mark.gpu
@@ -25,7 +23,6 @@ CASES = [
 @pytest.mark.parametrize("fp4", [False, True])
 @pytest.mark.parametrize("tile,M,K,N,R", CASES)
 def test_against_large_tiles(dev, tile, M, K, N, R, fp4, monkeypatch):
-    from nunchaku_amd import _native as nv
     from nunchaku_amd.ops import gemm as gemm_mod
 
     announce(f"narrow tiles {tile} M={M} K={K} N={N} R={R} fp4={fp4}")
@@ -38,16 +35,7 @@ def test_against_large_tiles(dev, tile, M, K, N, R, fp4, monkeypatch):
     kw = dict(act=act, wgt=t["qweight"], ascales=asc, wscales=t["wscales"], bias=t["bias"], fp4=fp4, alpha=m.alpha if fp4 else 1.5, wcscales=t["wcscales"])
     if R:
         kw.update(lora_act_in=la, lora_up=t["proj_up"], lora_scales=[0.5 + 0.25 * i for i in range((R + 15) // 16)])
-    tiles, real, ncu = [], nv.launch, torch.cuda.get_device_properties(dev).multi_processor_count
-
-    def launch(entry, args_ref, device):
-        rows, columns = ctypes.c_int32(), ctypes.c_int32()
-        nv.check(nv.lib().svdq_gemm_plain_tile_of(args_ref, ncu, ctypes.byref(rows), ctypes.byref(columns)))
-        tiles.append((rows.value, columns.value))
-        return real(entry, args_ref, device)
-
-    monkeypatch.setattr(nv, "launch", launch)
-    outs = []
+    plans, outs = record_plans(monkeypatch, dev), []
     for split in (1, None, None):
         monkeypatch.setattr(gemm_mod, "K_SPLIT", split)
         out = Guarded((M, N - 8), torch.bfloat16, dev)  # (the last column tile ends 8 columns early)
@@ -55,8 +43,9 @@ def test_against_large_tiles(dev, tile, M, K, N, R, fp4, monkeypatch):
         torch.cuda.synchronize()
         out.check("out")
         outs.append(out.t.cpu())
-    if ncu == 256:
-        assert tiles[1] == tiles[2] == (tile[fp4] if isinstance(tile[0], tuple) else tile), tiles
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+        want = tile[fp4] if isinstance(tile[0], tuple) else tile
+        assert plans[0].few_rows == 0 and all((32 * p.few_rows, p.columns) == want for p in plans[1:]), plans
     assert torch.equal(outs[1].view(torch.int16), outs[2].view(torch.int16)), "changed between two launches"
     a, b = outs[1].float(), outs[0].float()
     # sums of K products and R more in another order: 2^-24 (K + R) of the largest value at most; then one rounding that may go

@@ -1,23 +1,13 @@
 """The few-rows GEMM's tiles with the plain epilogue (csrc/gemm.hip, ``plain_tile``; csrc/gemm_narrow_variant.hip) on the CPU: which one
 a launch takes, that no operand is read outside its buffer, and that the kernels keep out of scratch memory."""
 
-import ctypes
 import re
 
 import pytest
 
-from nunchaku_amd import _native as nv
 from plan_util import call, plan_of
 from test_address_model import FRAG, buffer_read
 from test_build_guard import compiled  # noqa: F401  (the fixture)
-
-TILES = [(32, 32), (32, 64), (64, 32), (64, 64), (32, 128), (64, 128)]
-
-
-def plain_tile(M, K, N, fp4, compute_units=256):
-    rows, columns = ctypes.c_int32(), ctypes.c_int32()
-    nv.check(nv.lib().svdq_gemm_plain_tile_of(ctypes.byref(call("plain", M, K, N, 32, fp4)), compute_units, ctypes.byref(rows), ctypes.byref(columns)))
-    return rows.value, columns.value
 
 
 # (shape, the tile on 256 compute units; the same for both precisions)
@@ -27,7 +17,9 @@ def plain_tile(M, K, N, fp4, compute_units=256):
 ])
 @pytest.mark.parametrize("fp4", [False, True])
 def test_the_tile_of_a_launch(M, K, N, want, fp4):
-    assert plain_tile(M, K, N, fp4) == want
+    p = plan_of(call("plain", M, K, N, 32, fp4))
+    assert (32 * p.few_rows, p.columns) == want and p.shared_rows == ((M, fp4) == (1157, False)), p
+    assert p.row_blocks == (M + want[0] - 1) // want[0], p
 
 
 def check_addresses(M, K, N, fp4, MT, NC):
