@@ -625,7 +625,13 @@ int gemm_fp4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t st
 }
 
 // ---- few rows, either precision: small tiles, operands straight to registers (gemm_direct_kernel.h) ------
-// The tile of a few-rows launch with the plain epilogue, in blocks of 32 x 32.  What takes the time is the fetching of the operands: a
+struct FewRowsTile {
+    int mt, nc;  // blocks of 32 rows, of 32 columns (none: large tiles)
+    bool shared_rows;
+    double time;
+};
+// The tile of a few-rows launch with the plain epilogue, in blocks of 32 x 32: that of 128 columns which the launch would have otherwise
+// (32 rows: shape 1, 64: shape 2) or a narrower one.  What takes the time is the fetching of the operands: a
 // compute unit gets 120 GB/s in requests of 16 bytes a lane, 80 in those of 8, however few of them fetch and however many waves do (48
 // or 192 workgroups, 4 ... 16 waves each), and a tile of mt x nc blocks fetches mt + nc fragments per k-group.  Square tiles fetch least per
 // product, small ones bring more compute units to bear: the sums cost a tile nothing before the end.  A model of the time in us, linear in the
@@ -636,12 +642,11 @@ int gemm_fp4(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t st
 //          M = 256               14.1 / 13.1 (64 x 64)           15.3 / 14.1
 //          M = 64, K = 12288     32.3 / 21.4 (32 x 32)           34.6 / 21.6
 //          M = 256, K = 12288    34.7 / 30.3 (64 x 64)           37.4 / 34.0
-struct FewRowsTile {
-    int mt, nc;  // blocks of 32 rows, of 32 columns (none: large tiles)
-    bool shared_rows;
-    double time;
-};
-FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu) {
+// Where the launch would have 64-row tiles, compute units have several narrow ones, and the model, which knows neither the fixed part of a
+// tile nor its rank, favours them too much: they are taken if it says 15 % and a row is 512 long.  Over 2500 INT4 and 2000 NVFP4 shapes (M = 1 ... 36864, K =
+// 128 ... 15360, N = 128 ... 21504, ranks 0 ... 160) 13 and 12 then lose 3 % or more to the tiles of 128 columns, without this 75 and 30:
+// INT4 M = 9677, K = 640, N = 128 9.8 with 64 x 128, 32 x 32 13.3; M = 10384, K = 384, N = 256 9.2, 64 x 64 10.8; NVFP4 M = 1083, K = 384, N = 3584 7.9, 32 x 64 9.3.
+FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu, int shape) {
     struct Model {
         int mt, nc;
         double launch, tile, kgroup;
@@ -650,14 +655,21 @@ FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu) {
                               {2, 2, 0.18, 0.64, 0.0702},  {1, 4, -0.13, 0.64, 0.0948}, {2, 4, 1.04, 0.53, 0.1378}};
     constexpr Model nvfp4[] = {{1, 1, -0.85, 0.16, 0.0323}, {1, 2, -0.52, 0.14, 0.0515}, {2, 1, -0.64, 0.24, 0.0498},
                                {2, 2, -0.17, 0.46, 0.0719}, {1, 4, 0.22, 0.47, 0.0876},  {2, 4, 1.96, -0.07, 0.1112}};
+    const Model *models = a->fp4 ? nvfp4 : int4;
     const long long row_blocks = (rows_needed(a) + 31) / 32, column_blocks = a->N / 32;
-    FewRowsTile best{};
-    for (const Model &m : a->fp4 ? nvfp4 : int4) {
+    auto tile = [&](const Model &m) {
         const long long tiles = (row_blocks + m.mt - 1) / m.mt * (column_blocks / m.nc);
-        const double t = m.launch + (double)((tiles + ncu - 1) / ncu) * (m.tile + m.kgroup * (double)(a->K / 64));
-        if (best.mt == 0 || t < best.time) best = FewRowsTile{m.mt, m.nc, false, t};
+        return FewRowsTile{m.mt, m.nc, false, m.launch + (double)((tiles + ncu - 1) / ncu) * (m.tile + m.kgroup * (double)(a->K / 64))};
+    };
+    const FewRowsTile wide = tile(models[3 + shape]);
+    FewRowsTile best = wide;
+    if (shape == 2 && a->K < 512) return wide;
+    if (shape == 2) best.time *= 0.85;
+    for (int i = 0; i < 4; i++) {
+        const FewRowsTile t = tile(models[i]);
+        if (t.time < best.time) best = t;
     }
-    return best;
+    return best.nc == 4 ? wide : best;
 }
 
 // INT4 launches whose tiles of 64 x 128 are between one and two per compute unit (three with the quantizing epilogue, one and a half and two with the
@@ -739,13 +751,14 @@ FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
         } else if (plain) {
             // (the plain epilogue's tiles are faster than these two, the model of their time has no offset: 2277 layers of 100 ... 2600 rows 0.3 % off the
             // fastest, 0.6 without; M = 225, K = 4992, N = 10624 36.4 -> 30.5 us, M = 175, K = 9984, N = 14976 59 -> 51, M = 261, K = 1152, N = 14208 18 -> 17)
-            const double t_plain = 5.0 + 1.3 * plain_tile(a, ncu).time;
-            if (t_plain < t_large) return plain_tile(a, ncu);
+            const FewRowsTile t = plain_tile(a, ncu, t1 < t2 ? 1 : 2);
+            if (5.0 + 1.3 * t.time < t_large) return t;
             t_large *= 0.95;
         }
     }
     if ((t1 < t2 ? t1 : t2) >= t_large) return none;
-    return plain ? plain_tile(a, ncu) : FewRowsTile{t1 < t2 ? 1 : 2, 4};
+    const int shape = t1 < t2 ? 1 : 2;
+    return plain ? plain_tile(a, ncu, shape) : FewRowsTile{shape, 4};
 }
 
 // Which kernel a call takes and how it divides the work.  A function of the arguments and the number of compute units alone:
