@@ -672,17 +672,17 @@ FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu, int shape) {
     return best.nc == 4 ? wide : best;
 }
 
-// INT4 launches whose tiles of 64 x 128 are between one and two per compute unit (three with the quantizing epilogue, one and a half and two with the
-// plain one): the waves split the columns and share the rows' operands through LDS (gemm_direct_kernel.h).  A tile alone on its
-// compute unit is a chain of latencies, 0.2 us per k-group, two overlap; more issue more instructions per product than the large tiles.  Layer calls,
-// the best other form / this one, us: QKV M = 256, K = 3072, N = 9216 27.2 / 23.5, M = 505, K = 2048 22.0 / 19.5, at 2.25 tiles M = 505, K = 3072 32.6 / 33.8, at 0.75
-// M = 256, K = 2048 15.7 / 17.4; MLP M = 256, K = 3072 52.4 / 48.8, M = 505 (three tiles) 78.6 / 75.1, M = 600 79.8 / 85.1; plain M = 384, K = 3072, N = 9216
-// 26.3 / 22.8, M = 320 (1.4 tiles, where narrow ones are better) 22.4 / 22.6, M = 505 30.4 / 32.1.
+// INT4 launches with more than one tile of 64 x 128 per compute unit and up to two (plain epilogue: from one and a half on): such tiles, where they are
+// chosen (choose_direct), have waves that split the columns and share the rows' operands through LDS (gemm_direct_kernel.h).  A tile alone on its
+// compute unit is a chain of latencies, 0.2 us per k-group, two overlap; more issue more instructions per product than the large tiles.  The GEMM alone,
+// waves that split K / large tiles / this one, us, rank 32: norm and rotary M = 256, K = 3072, N = 9216 23.6 / 22.5 / 19.6, M = 505, K = 2048, N = 6144 18.0 / 17.1 / 15.7, at
+// 2.25 tiles M = 505, K = 3072, N = 9216 34.6 / 29.6 / 30.6; quantizing epilogue K = 3072, N = 12288 M = 256 29.8 / 29.2 / 26.7, M = 300 30.8 / 30.4 / 28.8, at three tiles M = 505
+// 43.6 / 39.4 / 39.3, rank 128 59.4 / 47.3 / 52.6; layer calls, plain M = 384, K = 3072, N = 9216 26.3 / 22.8 with this one, M = 320 (1.4 tiles, where narrow ones are better)
+// 22.4 / 22.6, M = 505 30.4 / 32.1.
 bool staged_rows(const svdq_gemm_args *a, int ncu) {
     if (a->fp4 || a->K < 256) return false;
     const long long tiles = (rows_needed(a) + 63) / 64 * (a->N / 128);
-    if (!needs_next_epilogue(a)) return 2 * tiles >= 3 * ncu && tiles <= 2 * ncu;
-    return tiles > ncu && tiles <= (a->qout ? 3 : 2) * ncu;
+    return 2 * tiles >= (needs_next_epilogue(a) ? 2 * ncu + 2 : 3 * ncu) && tiles <= 2 * ncu;
 }
 
 // Which tiles of the few-rows kernel a launch takes, if any.  Shape 1: tiles of 32 rows x 128 columns, four waves split
@@ -705,7 +705,6 @@ FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
     constexpr FewRowsTile none{};
     if (a->k_split > 0) return none;  // (the caller asks for the tiles that k_split is about)
     if (((uintptr_t)a->bias | (uintptr_t)a->wcscales | (uintptr_t)a->oscales) % 8 || (uintptr_t)a->colnorm % 16) return none;  // (read four columns at a time)
-    if (staged_rows(a, ncu)) return FewRowsTile{2, 4, true};
     const bool plain = !needs_next_epilogue(a);
     const int rows = rows_needed(a), kg = (int)(a->K / 64);
     const long long ncols = a->N / 128;
@@ -746,9 +745,16 @@ FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
         t_large = choose_tiles_int4(a, ncu, &tiles);
         t1 = 3.5 + c1 * (1.1 + 0.106 * kg);
         t2 = 3.3 + c2 * (1.6 + 0.158 * kg);
-        if (a->qout) {
-            t_large *= 1.05;  // (1158 MLPs of 100 ... 2600 rows: 0.4 % off the fastest, 0.7 without; M = 1486, K = 1024 51.3 -> 45.8 us)
-        } else if (plain) {
+        // Tiles whose waves share the rows' operands take shape 2's place where that is the fastest by the models, and with 0.9 of its time where the others say
+        // so; not against whole tiles in launches with the quantizing epilogue, whose low-rank term costs the large tiles less (rank 128, M = 1294,
+        // K = 1152, N = 4608 0.85 times as fast).  Over 2500 launches of 1 ... 36864 rows with all epilogues but the plain one, ranks 0 ... 160, 0.7 % off the fastest
+        // and none 3 % slower than without this form; taken wherever it can be, and with up to three tiles in MLPs, 1.0 % and 86, up to 1.4 times as slow
+        // (quantizing epilogue, M = 4357, K = 1024, N = 1152, rank 128; SiLU, M = 408, K = 512, N = 4864, rank 96 8.7 us in shape 1, 12.0 so).
+        if (staged_rows(a, ncu)) {
+            const double t = t2 * (!a->qout || tiles.kparts > 1 ? 0.9 : 1.0);
+            if (t <= t1 && t < t_large) return FewRowsTile{2, 4, true};
+        }
+        if (plain) {
             // (the plain epilogue's tiles are faster than these two, the model of their time has no offset: 2277 layers of 100 ... 2600 rows 0.3 % off the
             // fastest, 0.6 without; M = 225, K = 4992, N = 10624 36.4 -> 30.5 us, M = 175, K = 9984, N = 14976 59 -> 51, M = 261, K = 1152, N = 14208 18 -> 17)
             const FewRowsTile t = plain_tile(a, ncu, t1 < t2 ? 1 : 2);

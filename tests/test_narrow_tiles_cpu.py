@@ -89,11 +89,23 @@ def test_narrow_tiles_fit_their_registers(compiled, variant):  # noqa: F811
 # On either side of the lines between the few-rows kernel and the large tiles that the factors in choose_direct draw.
 @pytest.mark.parametrize("kind,M,K,N,fp4,few", [
     ("plain", 1131, 2048, 10112, True, 2), ("plain", 4608, 15360, 3072, True, 0), ("rope", 1614, 3968, 11904, True, 2), ("next", 2154, 1792, 7168, True, 2),
-    ("plain", 225, 4992, 10624, False, 2), ("plain", 175, 9984, 14976, False, 2), ("plain", 261, 1152, 14208, False, 0), ("next", 1486, 1024, 4096, False, 2),
+    ("plain", 225, 4992, 10624, False, 2), ("plain", 175, 9984, 14976, False, 2), ("plain", 261, 1152, 14208, False, 0), ("next", 1486, 1024, 4096, False, 0),
     ("next", 1486, 2048, 8192, False, 0),
 ])
 def test_few_rows_or_large_tiles(kind, M, K, N, fp4, few):
     assert plan_of(call(kind, M, K, N, 32, fp4)).few_rows == few
+
+
+# (few_rows, shared_rows) on either side of the lines of the shared-rows form: the tiles per compute unit, and the other forms where these are faster.
+@pytest.mark.parametrize("kind,M,K,N,R,want", [
+    ("rope", 256, 3072, 9216, 32, (2, 1)), ("rope", 505, 2048, 6144, 128, (2, 1)), ("rope", 505, 3072, 9216, 32, (0, 0)), ("plain", 384, 3072, 9216, 32, (2, 1)),
+    ("next", 256, 3072, 12288, 32, (2, 1)), ("next", 256, 3072, 12288, 128, (2, 1)), ("next", 505, 3072, 12288, 128, (0, 0)), ("next", 1280, 1152, 4608, 128, (0, 0)),
+    ("next", 4357, 1024, 1152, 128, (0, 0)), ("silu", 408, 512, 4864, 96, (1, 0)), ("silu", 607, 2176, 3328, 0, (1, 0)), ("rope", 347, 4992, 5760, 32, (1, 0)),
+    ("split", 196, 12416, 10752, 128, (0, 0)), ("next", 585, 11392, 4224, 64, (2, 1)), ("split", 1280, 128, 3072, 32, (2, 0)),
+])
+def test_where_waves_share_the_rows(kind, M, K, N, R, want):
+    p = plan_of(call(kind, M, K, N, R, False))
+    assert (p.few_rows, p.shared_rows) == want, p
 
 
 @pytest.mark.parametrize("variant", [0, 1])
