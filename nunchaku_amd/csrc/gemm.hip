@@ -735,11 +735,16 @@ FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
             t1 += 0.9 * c1;
             t2 += 1.0 * c2;
         }
-        // The models of this kernel predate its buffers: against whole large tiles it is up to 14 % faster than they say (3100 shapes, M = 300 ... 5200,
-        // layer calls: where they say 1.0 ... 1.05 of the large tiles' time it takes 0.90, from 1.2 on 1.04).  Choosing so takes 0.5 % longer than the
-        // fastest on average, 1 % without: M = 1057, K = 10240, N = 14208 296 -> 254 us, M = 1131, K = 2048, N = 10112 58 -> 52, with norm and rotation M = 1614, K = 3968,
-        // N = 11904 183 -> 155, MLP M = 2154, K = 1792 132 -> 121.  (Against shared ones the models stand at 4608 rows.)
-        if (kg > 12 && (tiles <= 1.0 || nwg > 0)) t_large *= 1.14;
+        // The models of this kernel predate its buffers: against whole large tiles it is up to 14 % faster than they say (the GEMM alone, us: M = 1836,
+        // K = 12032, N = 5888 256 -> 199, M = 2284, K = 2816, N = 4864 68 -> 54, norm, rotary and three outputs M = 711, K = 10624, N = 14976 228 -> 184, SiLU M = 1129,
+        // K = 4224, N = 9472, rank 64 103 -> 82, quantizing epilogue M = 5132, K = 5504, N = 2432 156 -> 131; rank 32 unless noted).  Its tiles each pay for
+        // their rank, and short rows gain nothing (M = 10224, K = 1152, N = 3072, rank 160 94 -> 143 us, M = 3771, K = 1152, N = 3072, rank 128 44 -> 51).  Over 1700 shapes between
+        // the two (M up to 36864, ranks 0 ... 160, all epilogues) 1.8 % faster than without the factor and five of them 3 to 5 % slower; with the factor
+        // for all rows longer than 768 and all ranks 1.0 % and 166, up to 1.6 times as slow.  (Against shared ones the models stand at 4608 rows.)
+        if (kg >= 24 && (tiles <= 1.0 || nwg > 0)) {
+            const double rank = a->R_up > 32 ? 0.4 * c2 * (double)(a->R_up / 16 - 2) : 0.0;
+            if (0.14 * t_large > rank) t_large = 1.14 * t_large - rank;
+        }
     } else {
         svdq_gemm_plan tiles;
         t_large = choose_tiles_int4(a, ncu, &tiles);

@@ -96,6 +96,16 @@ def test_few_rows_or_large_tiles(kind, M, K, N, fp4, few):
     assert plan_of(call(kind, M, K, N, 32, fp4)).few_rows == few
 
 
+# The lines that rank and the rows' length draw between the NVFP4 few-rows kernel and whole large tiles.
+@pytest.mark.parametrize("kind,M,K,N,R,few", [
+    ("plain", 10224, 1152, 3072, 160, 0), ("plain", 3771, 1152, 3072, 128, 0), ("plain", 1049, 1152, 13056, 160, 0), ("rope", 3662, 1024, 3456, 160, 0),
+    ("silu", 20295, 1280, 12416, 128, 0), ("split", 1857, 896, 6912, 128, 0), ("plain", 1836, 12032, 5888, 32, 2), ("plain", 1131, 2048, 10112, 32, 2),
+    ("split", 711, 10624, 14976, 32, 2), ("silu", 1129, 4224, 9472, 64, 2), ("next", 2154, 1792, 7168, 32, 2),
+])
+def test_nvfp4_few_rows_or_large_tiles_by_rank(kind, M, K, N, R, few):
+    assert plan_of(call(kind, M, K, N, R, True)).few_rows == few
+
+
 # (few_rows, shared_rows) on either side of the lines of the shared-rows form: the tiles per compute unit, and the other forms where these are faster.
 @pytest.mark.parametrize("kind,M,K,N,R,want", [
     ("rope", 256, 3072, 9216, 32, (2, 1)), ("rope", 505, 2048, 6144, 128, (2, 1)), ("rope", 505, 3072, 9216, 32, (0, 0)), ("plain", 384, 3072, 9216, 32, (2, 1)),
