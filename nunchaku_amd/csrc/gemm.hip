@@ -24,6 +24,7 @@ int launch_next(const Params &p, int nwg, hipStream_t stream);
 }  // namespace g6
 }  // namespace svdq
 
+#include <math.h>
 #include <mutex>
 #include <stdlib.h>
 #include <vector>
@@ -679,10 +680,11 @@ FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu, int shape) {
 // 2.25 tiles M = 505, K = 3072, N = 9216 34.6 / 29.6 / 30.6; quantizing epilogue K = 3072, N = 12288 M = 256 29.8 / 29.2 / 26.7, M = 300 30.8 / 30.4 / 28.8, at three tiles M = 505
 // 43.6 / 39.4 / 39.3, rank 128 59.4 / 47.3 / 52.6; layer calls, plain M = 384, K = 3072, N = 9216 26.3 / 22.8 with this one, M = 320 (1.4 tiles, where narrow ones are better)
 // 22.4 / 22.6, M = 505 30.4 / 32.1.
-bool staged_rows(const svdq_gemm_args *a, int ncu) {
+// (`split`: the large tiles would be split along K, see choose_direct)
+bool staged_rows(const svdq_gemm_args *a, int ncu, bool split) {
     if (a->fp4 || a->K < 256) return false;
     const long long tiles = (rows_needed(a) + 63) / 64 * (a->N / 128);
-    return 2 * tiles >= (needs_next_epilogue(a) ? 2 * ncu + 2 : 3 * ncu) && tiles <= 2 * ncu;
+    return 2 * tiles >= (needs_next_epilogue(a) ? 2 * ncu + 2 : 3 * ncu) && tiles <= (a->qout && split ? 3 : 2) * ncu;
 }
 
 // Which tiles of the few-rows kernel a launch takes, if any.  Shape 1: tiles of 32 rows x 128 columns, four waves split
@@ -752,11 +754,15 @@ FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
         t2 = 3.3 + c2 * (1.6 + 0.158 * kg);
         // Tiles whose waves share the rows' operands take shape 2's place where that is the fastest by the models, and with 0.9 of its time where the others say
         // so; not against whole tiles in launches with the quantizing epilogue, whose low-rank term costs the large tiles less (rank 128, M = 1294,
-        // K = 1152, N = 4608 0.85 times as fast).  Over 2500 launches of 1 ... 36864 rows with all epilogues but the plain one, ranks 0 ... 160, 0.7 % off the fastest
-        // and none 3 % slower than without this form; taken wherever it can be, and with up to three tiles in MLPs, 1.0 % and 86, up to 1.4 times as slow
+        // K = 1152, N = 4608 0.85 times as fast).  Beside tiles split along K they are always taken, though those are up to 1.14 times as fast at K of
+        // 8192 and more (1.06 times as slow on average): the sums need workspace, and a program may capture a call that does not without a call before.
+        // Over 2500 launches of 1 ... 36864 rows with all epilogues but the plain one, ranks 0 ... 160, 0.7 % off the fastest, and 17 of them, those beside split
+        // tiles, 3 % and more slower than without this form; taken wherever it can be, and with up to three tiles in MLPs, 1.0 % and 86, up to 1.4 times as slow
         // (quantizing epilogue, M = 4357, K = 1024, N = 1152, rank 128; SiLU, M = 408, K = 512, N = 4864, rank 96 8.7 us in shape 1, 12.0 so).
-        if (staged_rows(a, ncu)) {
-            const double t = t2 * (!a->qout || tiles.kparts > 1 ? 0.9 : 1.0);
+        const bool split = tiles.kparts > 1;
+        if (staged_rows(a, ncu, split)) {
+            if (split) t_large = HUGE_VAL;
+            const double t = a->qout ? t2 : 0.9 * t2;
             if (t <= t1 && t < t_large) return FewRowsTile{2, 4, true};
         }
         if (plain) {

@@ -111,7 +111,7 @@ def test_nvfp4_few_rows_or_large_tiles_by_rank(kind, M, K, N, R, few):
     ("rope", 256, 3072, 9216, 32, (2, 1)), ("rope", 505, 2048, 6144, 128, (2, 1)), ("rope", 505, 3072, 9216, 32, (0, 0)), ("plain", 384, 3072, 9216, 32, (2, 1)),
     ("next", 256, 3072, 12288, 32, (2, 1)), ("next", 256, 3072, 12288, 128, (2, 1)), ("next", 505, 3072, 12288, 128, (0, 0)), ("next", 1280, 1152, 4608, 128, (0, 0)),
     ("next", 4357, 1024, 1152, 128, (0, 0)), ("silu", 408, 512, 4864, 96, (1, 0)), ("silu", 607, 2176, 3328, 0, (1, 0)), ("rope", 347, 4992, 5760, 32, (1, 0)),
-    ("split", 196, 12416, 10752, 128, (0, 0)), ("next", 585, 11392, 4224, 64, (2, 1)), ("split", 1280, 128, 3072, 32, (2, 0)),
+    ("split", 196, 12416, 10752, 128, (2, 1)), ("next", 585, 11392, 4224, 64, (2, 1)), ("next", 1641, 8192, 2560, 32, (2, 1)), ("split", 1280, 128, 3072, 32, (2, 0)),
 ])
 def test_where_waves_share_the_rows(kind, M, K, N, R, want):
     p = plan_of(call(kind, M, K, N, R, False))
