@@ -631,8 +631,8 @@ struct FewRowsTile {
     bool shared_rows;
     double time;
 };
-// The tile of a few-rows launch with the plain epilogue, in blocks of 32 x 32: that of 128 columns which the launch would have otherwise
-// (32 rows: shape 1, 64: shape 2) or a narrower one.  What takes the time is the fetching of the operands: a
+// The tile of a few-rows launch with the plain epilogue, in blocks of 32 x 32 (`shape`: the better one of 128 columns by the models of
+// choose_direct, of 32 rows (1) or 64 (2)).  What takes the time is the fetching of the operands: a
 // compute unit gets 120 GB/s in requests of 16 bytes a lane, 80 in those of 8, however few of them fetch and however many waves do (48
 // or 192 workgroups, 4 ... 16 waves each), and a tile of mt x nc blocks fetches mt + nc fragments per k-group.  Square tiles fetch least per
 // product, small ones bring more compute units to bear: the sums cost a tile nothing before the end.  A model of the time in us, linear in the
@@ -643,10 +643,10 @@ struct FewRowsTile {
 //          M = 256               14.1 / 13.1 (64 x 64)           15.3 / 14.1
 //          M = 64, K = 12288     32.3 / 21.4 (32 x 32)           34.6 / 21.6
 //          M = 256, K = 12288    34.7 / 30.3 (64 x 64)           37.4 / 34.0
-// Where the launch would have 64-row tiles, compute units have several narrow ones, and the model, which knows neither the fixed part of a
-// tile nor its rank, favours them too much: they are taken if it says 15 % and a row is 512 long.  Over 2500 INT4 and 2000 NVFP4 shapes (M = 1 ... 36864, K =
-// 128 ... 15360, N = 128 ... 21504, ranks 0 ... 160) 13 and 12 then lose 3 % or more to the tiles of 128 columns, without this 75 and 30:
-// INT4 M = 9677, K = 640, N = 128 9.8 with 64 x 128, 32 x 32 13.3; M = 10384, K = 384, N = 256 9.2, 64 x 64 10.8; NVFP4 M = 1083, K = 384, N = 3584 7.9, 32 x 64 9.3.
+// INT4, rows or columns fewer than 1024, where 64-row tiles are the better ones of 128 columns: compute units have several tiles, and the model, which does
+// not know the fixed part of a tile well, favours narrow ones too much.  There they are taken if it says 8 %, and not with K = 128 (M = 125, N = 11392,
+// rank 16 5.1 us with 64 x 128, 32 x 32 6.3).  Over 325 INT4 shapes with few columns, short rows or more than 9216 rows 0.9 % off the fastest tile, without this
+// 1.1; the 1111 others 0.2 %, 1727 NVFP4 shapes 0.4 % (M = 1 ... 20000, K = 128 ... 16640, N = 128 ... 21504, ranks 0 ... 160).
 FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu, int shape) {
     struct Model {
         int mt, nc;
@@ -656,21 +656,17 @@ FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu, int shape) {
                               {2, 2, 0.18, 0.64, 0.0702},  {1, 4, -0.13, 0.64, 0.0948}, {2, 4, 1.04, 0.53, 0.1378}};
     constexpr Model nvfp4[] = {{1, 1, -0.85, 0.16, 0.0323}, {1, 2, -0.52, 0.14, 0.0515}, {2, 1, -0.64, 0.24, 0.0498},
                                {2, 2, -0.17, 0.46, 0.0719}, {1, 4, 0.22, 0.47, 0.0876},  {2, 4, 1.96, -0.07, 0.1112}};
-    const Model *models = a->fp4 ? nvfp4 : int4;
     const long long row_blocks = (rows_needed(a) + 31) / 32, column_blocks = a->N / 32;
-    auto tile = [&](const Model &m) {
+    const bool favour_wide = !a->fp4 && shape == 2 && (a->K < 1024 || a->N < 1024);
+    FewRowsTile best{};
+    for (const Model &m : a->fp4 ? nvfp4 : int4) {
+        const bool wide = m.mt == 2 && m.nc == 4;
+        if (favour_wide && a->K < 256 && !wide) continue;
         const long long tiles = (row_blocks + m.mt - 1) / m.mt * (column_blocks / m.nc);
-        return FewRowsTile{m.mt, m.nc, false, m.launch + (double)((tiles + ncu - 1) / ncu) * (m.tile + m.kgroup * (double)(a->K / 64))};
-    };
-    const FewRowsTile wide = tile(models[3 + shape]);
-    FewRowsTile best = wide;
-    if (shape == 2 && a->K < 512) return wide;
-    if (shape == 2) best.time *= 0.85;
-    for (int i = 0; i < 4; i++) {
-        const FewRowsTile t = tile(models[i]);
-        if (t.time < best.time) best = t;
+        const double t = (m.launch + (double)((tiles + ncu - 1) / ncu) * (m.tile + m.kgroup * (double)(a->K / 64))) * (favour_wide && wide ? 0.92 : 1.0);
+        if (best.mt == 0 || t < best.time) best = FewRowsTile{m.mt, m.nc, false, t};
     }
-    return best.nc == 4 ? wide : best;
+    return best;
 }
 
 // INT4 launches with more than one tile of 64 x 128 per compute unit and up to two (plain epilogue: from one and a half on): such tiles, where they are

@@ -12,7 +12,7 @@ from oracle import synth
 pytestmark = pytest.mark.gpu
 
 # (epilogue, M, K, N, R); the launcher takes 32-row tiles for the first two rows of this list, and 64-row tiles, on 256 compute
-# units, for the others
+# units, for the others (plain epilogue: the tile that its model says, see test_gpu_narrow_tiles.py)
 CASES = [
     ("plain", 1, 128, 128, 16), ("plain", 31, 128, 256, 0), ("plain", 33, 640, 384, 48), ("plain", 64, 1152, 128, 80), ("plain", 65, 256, 640, 32),
     ("silu", 96, 384, 256, 16), ("next", 33, 128, 128, 16), ("next", 97, 640, 384, 48), ("rope", 40, 384, 384, 32), ("split", 256, 256, 768, 16),
@@ -70,7 +70,7 @@ def test_against_large_tiles(dev, kind, M, K, N, R, fp4, monkeypatch):
     want, got, again = run(1), run(None), run(None)
     assert plans[0].few_rows == 0
     if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
-        assert plans[1].few_rows == plans[2].few_rows == (1 if M <= 256 else 2), plans
+        assert repr(plans[1]) == repr(plans[2]) and plans[1].few_rows in ((1, 2) if kind == "plain" else (1,) if M <= 256 else (2,)), plans
     for name in got:
         a, b = got[name].cpu(), want[name].cpu()
         assert torch.equal(a.view(torch.uint8), again[name].cpu().view(torch.uint8)), f"{name} changed between two launches"

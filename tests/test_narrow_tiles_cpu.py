@@ -22,12 +22,11 @@ def test_the_tile_of_a_launch(M, K, N, want, fp4):
     assert p.row_blocks == (M + want[0] - 1) // want[0], p
 
 
-# Launches whose narrow tiles the model takes for faster than the 64 x 128 ones, which they are not: short rows, several tiles per
-# compute unit; and ones where they are.  (The same sizes as in the comment at plain_tile, and others measured with them.)
+# Launches whose narrow tiles the INT4 model takes for faster than the 64 x 128 ones, which they are not: short rows and few columns, several tiles
+# per compute unit; and ones where a tile of another height than that of the better one of 128 columns is the fastest.
 @pytest.mark.parametrize("M,K,N,fp4,want", [
-    (9677, 640, 128, False, (64, 128)), (100, 128, 10496, False, (64, 128)), (10384, 384, 256, False, (64, 128)), (5494, 2560, 256, False, (64, 128)),
-    (285, 384, 8832, False, (64, 128)), (1083, 384, 3584, True, (64, 128)), (2721, 128, 1408, True, (64, 128)), (25047, 256, 128, True, (64, 128)),
-    (556, 2944, 4096, False, (64, 64)), (297, 1280, 3456, True, (32, 64)),
+    (125, 128, 11392, False, (64, 128)), (500, 128, 2176, False, (64, 128)), (5494, 2560, 256, False, (64, 128)), (556, 2944, 4096, False, (64, 64)),
+    (297, 1280, 3456, True, (32, 64)), (788, 4224, 7680, True, (64, 128)), (261, 1280, 21376, True, (64, 128)),
 ])
 def test_narrow_tiles_only_where_they_are_faster(M, K, N, fp4, want):
     p = plan_of(call("plain", M, K, N, 32, fp4))
