@@ -709,39 +709,55 @@ FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
     const double c1 = (double)((((rows + 31) / 32) * ncols + ncu - 1) / ncu), c2 = (double)((((rows + 63) / 64) * ncols + ncu - 1) / ncu);
     double t_large, t1, t2;
     if (a->fp4) {
-        // Large tiles: one per compute unit 62 us at K = 3072 with 48 tiles, 78 with 216; 32 at K = 1024.  Whole tiles of several
-        // rounds cost that many times as much, even shares of them 26 to 40 us for the sums that meet in the workspace.
         const long long ntiles = (a->M_pad / BM) * ((a->N + BN - 1) / BN);
-        const double tiles = (double)ntiles / ncu, one = (1.0 + 0.3 * (tiles < 1.0 ? tiles : 1.0)) * kg + 14.0;
+        const double tiles = (double)ntiles / ncu;
         const int nwg = whole_tiles_fp4(ntiles, ncu);
-        const double rounds = tiles <= 1.0 ? 1.0 : nwg ? (double)(ntiles / nwg) : tiles;
-        t_large = one * rounds + (tiles > 1.0 && !nwg ? 33.0 : 0.0);
         t1 = 4.3 + c1 * (1.1 + 0.127 * kg);
         t2 = 5.0 + c2 * (1.6 + 0.205 * kg) - (c2 < 3.0 ? 0.04 * kg : 0.0);
-        // Short rows and many rounds without the quantizing epilogue: the outputs set the pace, and whole large tiles write them faster (M =
-        // 4608, K = 384, N = 9088 69 us in shape 2 against 63; N = 19200 138 against 121; M = 4096, K = 384, N = 14592 with norm and rotary 117
-        // against 110; of 500 random shapes of 257 large tiles and more 14 take them by this term, 1.12 times as fast, none slower).  Not
-        // where the large tiles would be shared, up to 17 % faster still at such sizes (M = 6400, K = 640, N = 16384 210 against 181): those
-        // need 128 MB of workspace, more than the fixed scratch has, and a call gives the same bits with either.
-        if (nwg > 0 && kg <= 12 && c2 > 12.0 && !a->qout) t2 += 0.9 * (c2 - 12.0);
-        if (a->qout) {  // (the quantizing epilogue: M = 4608, K = 3072, N = 12288 298 -> 387 us in large tiles, 317 -> 358 in shape 2)
-            t_large += 20.0 * rounds;
+        if (a->qout) {
             t1 += 1.1 * c1;
             t2 += 1.4 * c2;
-        } else if (a->rotary_emb) {  // (M = 4608, K = 3072, N = 9216 223 -> 253 and 241 -> 261)
-            t_large += 10.0 * rounds;
+        } else if (a->rotary_emb) {
             t1 += 0.9 * c1;
             t2 += 1.0 * c2;
         }
-        // The models of this kernel predate its buffers: against whole large tiles it is up to 14 % faster than they say (the GEMM alone, us: M = 1836,
-        // K = 12032, N = 5888 256 -> 199, M = 2284, K = 2816, N = 4864 68 -> 54, norm, rotary and three outputs M = 711, K = 10624, N = 14976 228 -> 184, SiLU M = 1129,
-        // K = 4224, N = 9472, rank 64 103 -> 82, quantizing epilogue M = 5132, K = 5504, N = 2432 156 -> 131; rank 32 unless noted).  Its tiles each pay for
-        // their rank, and short rows gain nothing (M = 10224, K = 1152, N = 3072, rank 160 94 -> 143 us, M = 3771, K = 1152, N = 3072, rank 128 44 -> 51).  Over 1700 shapes between
-        // the two (M up to 36864, ranks 0 ... 160, all epilogues) 1.8 % faster than without the factor and five of them 3 to 5 % slower; with the factor
-        // for all rows longer than 768 and all ranks 1.0 % and 166, up to 1.6 times as slow.  (Against shared ones the models stand at 4608 rows.)
-        if (kg >= 24 && (tiles <= 1.0 || nwg > 0)) {
-            const double rank = a->R_up > 32 ? 0.4 * c2 * (double)(a->R_up / 16 - 2) : 0.0;
-            if (0.14 * t_large > rank) t_large = 1.14 * t_large - rank;
+        if (tiles > 1.0 && !nwg) {
+            // Large tiles shared by workgroups: 26 to 40 us for the sums that meet in the workspace.  (They need 128 MB of it, more than the fixed scratch
+            // has, and a call gives the same bits with either: they stay where these models put them, though up to 17 % faster beyond, M = 6400, K = 640,
+            // N = 16384 210 us against 181.)
+            t_large = (1.3 * kg + 14.0 + (a->qout ? 20.0 : a->rotary_emb ? 10.0 : 0.0)) * tiles + 33.0;
+        } else {
+            // Whole large tiles, in one round or several.  Their time and that of the few-rows kernel beside them, fitted to 555 and 400 launches in which the two are
+            // within 1.6 of each other (M up to 20000, K = 128 ... 16640, ranks 0 ... 160, all epilogues): a tile's rank and epilogue cost either kernel, small
+            // tiles more of it.  0.1 and 0.4 % off the faster one, 10 and 22 of them 3 % and more slower; with the models above and a factor between the kernels 1.3 and
+            // 4.1 %, 70 and 130.  The GEMM alone, large tiles / few rows, us: M = 1836, K = 12032, N = 5888 256 / 199, SiLU M = 1098, K = 1792, N = 12288,
+            // rank 48 63.7 / 52.2, M = 901, K = 4736, N = 11264, rank 128 115.5 / 100.5; M = 2972, K = 1792, N = 4864, rank 128 59.7 / 72.1, M = 8470, K = 1280,
+            // N = 3584, rank 128 92 / 131, M = 4608, K = 3072, N = 21504 497 / 536.  Long rows: no tiling gets past the power limit, where large tiles are as fast (M = 4608,
+            // K = 15360, N = 3072 322 / 325; 1.25 to 1.39 PFLOP/s in the fastest tenth of either).
+            struct Model {
+                double launch, tile, kgroup, rank, next, vk, rotary, silu;
+                double time(const svdq_gemm_args *a, double rounds) const {
+                    const double epilogue = a->qout ? next : a->out_vk ? vk : a->rotary_emb ? rotary : a->fuse_silu ? silu : 0.0;
+                    return launch + rounds * (tile + kgroup * (double)(a->K / 64) + rank * (double)(a->R_up / 16) + epilogue);
+                }
+            };
+            constexpr Model shape1{3.7, 1.06, 0.1132, 0.248, 1.37, 0.79, 0.49, 0.16};
+            double t_few;
+            if (tiles <= 1.0) {
+                constexpr Model shape2{4.43, 1.19, 0.165, 0.423, 2.48, 1.51, 0.92, 0.48};
+                const Model large{6.65, 6.65, 0.344 + 1.179 * tiles, 1.23, 27.7, 15.8, 8.0, 6.4};
+                t_large = large.time(a, 1.0);
+                t_few = t1 < t2 ? shape1.time(a, c1) : shape2.time(a, c2);
+            } else {
+                constexpr Model shape2{0.65, 1.394, 0.1719, 0.441, 2.21, 0.99, 0.99, 0.48};
+                constexpr Model large{8.14, 8.39, 1.398, 1.09, 20.0, 12.8, 8.4, 7.6};
+                t_large = large.time(a, (double)(ntiles / nwg));
+                t_few = t1 < t2 ? shape1.time(a, c1) : shape2.time(a, c2);
+            }
+            const double t_power = 2.0 * rows * (double)a->K * (double)a->N / 1.28e9;  // (us at 1.28 PFLOP/s)
+            if (t_few < t_power) t_few = t_power;
+            if (t_few >= t_large && 2 * ntiles > ncu) return none;  // (fewer would be split along K, and need workspace for their sums)
+            t_large = HUGE_VAL;
         }
     } else {
         svdq_gemm_plan tiles;

@@ -95,11 +95,14 @@ def test_few_rows_or_large_tiles(kind, M, K, N, fp4, few):
     assert plan_of(call(kind, M, K, N, 32, fp4)).few_rows == few
 
 
-# The lines that rank and the rows' length draw between the NVFP4 few-rows kernel and whole large tiles.
+# The lines that rank, epilogue and the rows' length draw between the NVFP4 few-rows kernel and whole large tiles, in one round and in several.
 @pytest.mark.parametrize("kind,M,K,N,R,few", [
     ("plain", 10224, 1152, 3072, 160, 0), ("plain", 3771, 1152, 3072, 128, 0), ("plain", 1049, 1152, 13056, 160, 0), ("rope", 3662, 1024, 3456, 160, 0),
     ("silu", 20295, 1280, 12416, 128, 0), ("split", 1857, 896, 6912, 128, 0), ("plain", 1836, 12032, 5888, 32, 2), ("plain", 1131, 2048, 10112, 32, 2),
-    ("split", 711, 10624, 14976, 32, 2), ("silu", 1129, 4224, 9472, 64, 2), ("next", 2154, 1792, 7168, 32, 2),
+    ("split", 711, 10624, 14976, 32, 2), ("silu", 1129, 4224, 9472, 64, 2), ("next", 2154, 1792, 7168, 32, 2), ("silu", 1098, 1792, 12288, 48, 2),
+    ("plain", 901, 4736, 11264, 128, 2), ("plain", 2972, 1792, 4864, 128, 0), ("plain", 8470, 1280, 3584, 128, 0), ("plain", 4608, 3072, 21504, 32, 0),
+    ("plain", 4608, 15360, 3072, 32, 0), ("plain", 2666, 1664, 15360, 48, 2), ("rope", 3877, 2304, 14208, 16, 2), ("next", 4178, 2432, 16512, 16, 2),
+    ("litela", 1280, 3072, 8448, 128, 2), ("split", 1280, 1152, 8448, 32, 2),
 ])
 def test_nvfp4_few_rows_or_large_tiles_by_rank(kind, M, K, N, R, few):
     assert plan_of(call(kind, M, K, N, R, True)).few_rows == few
@@ -159,3 +162,11 @@ def test_addresses_of_shared_rows():
                 tile = nb % 2 * 4 + wave
                 assert (nb // 2 * kgroups + kgroups - 1) * 8 * FRAG + tile * FRAG + 1024 + 63 * 8 + 8 <= wgt_bytes
                 assert (nb // 2 * kgroups + kgroups - 1) * 2048 + tile * 256 + 31 * 8 + 4 <= wsc_bytes
+
+
+def test_nvfp4_large_tiles_that_few_rows_calls_could_take_need_no_workspace():
+    """Where the models would have the large tiles, but so few of them that they are split along K, the few-rows kernel stays: a program may
+    capture its call without a call before."""
+    for kind, M, K, N in (("plain", 1214, 3456, 5760), ("plain", 1763, 5888, 3584), ("silu", 2263, 2816, 2944)):
+        p = plan_of(call(kind, M, K, N, 512, True))
+        assert p.few_rows == 2 and not p.shared_tiles, p
