@@ -6,7 +6,8 @@
 // a tile of 32 MT rows x 32 NT WN columns; its waves split the columns WN ways and take the k-groups g = part, part + KP, ...
 // of their part of K in turn, and the parts' sums meet in LDS at the end.  An operand fragment is contiguous in memory in
 // the lanes' order (svdq_common.h), so a wave fetches it with one or two wide loads, DEPTH of its k-groups ahead, and
-// neither LDS nor barriers appear in the main loop.
+// neither LDS nor barriers appear in the main loop (but for INT4 tiles whose waves split the columns only and share the rows'
+// operands through LDS: STAGED, below).
 // What bounds it where compute units have one tile or two: the vector memory path of a compute unit.  It hands out 120 GB/s to requests of
 // 16 bytes a lane and 80 to those of 8 (operands in the L2, 48 or 192 compute units at work, 4, 8 or 16 waves each: the same), so that a
 // k-group of an INT4 tile of 32 x 128 takes 90 ns, its five fragments 75 of them, and neither more waves nor more k-groups on their way change
@@ -325,10 +326,11 @@ __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_ker
             read_rows(std::integral_constant<int, (RING - odd) % RING>{});
             each(std::make_integer_sequence<int, odd>{}, [&](auto I) { body(std::integral_constant<int, (decltype(I)::value + RING - odd) % RING>{}, ALL); });
         };
-        const int odd = (kgroups - DEPTH) % RING;  // (kgroups >= DEPTH)
-        each(std::make_integer_sequence<int, RING>{}, [&](auto O) {
-            if (odd == decltype(O)::value) start(O);
-        });
+        // (kgroups > DEPTH, and even: K is a multiple of 128.  So one or three are left over.)
+        static_assert(RING == 4);
+        const int odd = (kgroups - DEPTH) % RING;
+        if (odd == 1) start(std::integral_constant<int, 1>{});
+        else start(std::integral_constant<int, 3>{});
         for (int g = odd; g + DEPTH < kgroups; g += RING) each(std::make_integer_sequence<int, RING>{}, [&](auto I) { body(I, ALL); });
         each(std::make_integer_sequence<int, DEPTH>{}, [&](auto I) { body(I, std::integral_constant<int, DEPTH - 1 - decltype(I)::value>{}); });
         // (the sums are wanted here: the compiler would move the last additions behind the epilogue's requests, and their operands to scratch memory)

@@ -1,5 +1,5 @@
 """The INT4 few-rows GEMM whose waves share the rows' operands through LDS (csrc/gemm_direct_kernel.h, ``staged_rows`` in csrc/gemm.hip):
-every remainder of the k-groups by its ring of four, the fewest it takes, rows that end inside a tile; the same bits as one wave
+both remainders that an even number of k-groups leaves by its ring of four (one and three, before the whole turns), the fewest it takes, rows that end inside a tile; the same bits as one wave
 per tile adds up (the large tiles: the same order of the k-groups) where the epilogue is plain."""
 
 import pytest
@@ -31,7 +31,7 @@ def test_against_large_tiles(dev, M, N, K, monkeypatch):
         out.check("out")
         outs.append(out.t.cpu())
     if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
-        assert plans[0].few_rows == 0 and plans[1].few_rows == 2
+        assert plans[0].few_rows == 0 and plans[1].few_rows == 2 and plans[1].shared_rows, plans
     assert torch.equal(outs[1].view(torch.int16), outs[2].view(torch.int16))
     # the main sums have the same bits; bias and low-rank term are added in one order too, the low-rank products 16 ranks at a time
     a, b = outs[1].float(), outs[0].float()
