@@ -144,7 +144,8 @@ def test_fp6_conversion_never_overwrites_its_own_inputs():
     assert not fp6_conversions_with_overlap(["\tv_cvt_scalef32_2xpk16_fp6_f32 v[34:39], v[2:17], v[18:33], s52"])[1]
     flags = [f for f in nv.HIPCC_FLAGS if f not in ("-shared", "-fPIC")]
     with tempfile.TemporaryDirectory(prefix="svdq_guard_") as tmp:
-        for src, extra in (("quantize.hip", []), ("gemm6_variant.hip", ["-DSVDQ_VARIANT=1"]), ("gemm_direct_variant.hip", ["-DSVDQ_VARIANT=1"])):
+        for src, extra in (("quantize.hip", []), ("gemm6_variant.hip", ["-DSVDQ_VARIANT=1"]), ("gemm_direct_variant.hip", ["-DSVDQ_VARIANT=1"]),
+                           ("gemm_narrow_variant.hip", ["-DSVDQ_VARIANT=1"])):
             out = Path(tmp) / (src + ".s")
             res = subprocess.run(["/opt/rocm/bin/hipcc", *flags, *extra, "-S", "--cuda-device-only", str(CSRC / src), "-o", str(out)],
                                  capture_output=True, text=True)
@@ -254,6 +255,6 @@ def test_gemm_requests_are_not_made_lane_by_lane(compiled, unit):
 @pytest.mark.parametrize("unit", nv.GEMM_VARIANT_UNITS)
 def test_no_condition_code_kept_across_inline_asm(compiled, unit):
     _, lines = compiled[unit]
-    # (of the few-rows kernels only the INT4 one with the quantizing epilogue has inline assembly, the fp6 conversion)
+    # (of the few-rows kernels with 32-row tiles or waves that split K only the INT4 one with the quantizing epilogue has inline assembly, the fp6 conversion)
     assert sum("#ASMSTART" in l for l in lines) > 0 or (unit[0] == "gemm_direct_variant.hip" and unit[1] != 1)
     assert scc_live_across_asm(lines) == []

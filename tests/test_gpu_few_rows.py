@@ -18,13 +18,40 @@ CASES = [
     ("silu", 96, 384, 256, 16), ("next", 33, 128, 128, 16), ("next", 97, 640, 384, 48), ("rope", 40, 384, 384, 32), ("split", 256, 256, 768, 16),
     ("litela", 256, 256, 384, 16),
     ("plain", 1200, 384, 3072, 32), ("next", 1185, 256, 3072, 32), ("rope", 1217, 256, 3072, 16), ("split", 1280, 128, 3072, 32), ("litela", 1024, 256, 3456, 32),
-    ("plain", 1217, 640, 3072, 32), ("next", 1200, 1152, 3072, 48), ("rope", 1153, 512, 3072, 0),  # (5 and 4, 3 and 2, 2 k-groups per wave)
+    ("plain", 1217, 640, 3072, 32), ("next", 1200, 1152, 3072, 48), ("rope", 1153, 512, 3072, 0),  # (NVFP4: 3 and 2, 5 and 4, 2 k-groups per wave)
+]
+
+# INT4, 64 x 128 tiles, on 256 compute units.  Two waves split K and two the columns: two to nine k-groups per wave, which its ring of two divides and does not.
+SPLIT_K_CASES = [
+    ("plain", 505, 384, 3072, 48), ("plain", 1000, 512, 1536, 16), ("plain", 1281, 640, 1152, 80), ("plain", 1500, 1152, 768, 32),
+    ("next", 320, 256, 2304, 48), ("next", 769, 384, 1152, 16), ("next", 320, 640, 2304, 32), ("next", 769, 1152, 1152, 80), ("silu", 193, 384, 5376, 32),
+    ("rope", 193, 640, 5376, 32), ("rope", 1000, 256, 1152, 0), ("split", 512, 384, 2304, 16), ("litela", 512, 512, 2304, 32), ("litela", 1024, 640, 1152, 32),
+]
+# The waves split the columns and share the rows: one and three k-groups before the whole turns of its ring, every epilogue but the plain one.
+SHARED_ROWS_CASES = [
+    ("next", 1185, 256, 3072, 32), ("next", 1200, 1152, 3072, 48), ("next", 1200, 384, 3072, 16), ("rope", 1217, 256, 3072, 16), ("rope", 1153, 640, 3072, 0),
+    ("split", 1280, 256, 3072, 32), ("split", 1280, 384, 3072, 16), ("silu", 1200, 384, 3072, 0), ("silu", 1153, 512, 3072, 32), ("litela", 1024, 256, 3456, 32),
+    ("litela", 1024, 384, 3456, 48),
 ]
 
 
 @pytest.mark.parametrize("fp4", [False, True])
 @pytest.mark.parametrize("kind,M,K,N,R", CASES)
 def test_against_large_tiles(dev, kind, M, K, N, R, fp4, monkeypatch):
+    plan = _compare(dev, kind, M, K, N, R, fp4, monkeypatch)
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+        assert plan.few_rows in ((1, 2) if kind == "plain" else (1,) if M <= 256 else (2,)), plan
+
+
+@pytest.mark.parametrize("shared,case", [(0, c) for c in SPLIT_K_CASES] + [(1, c) for c in SHARED_ROWS_CASES])
+def test_int4_64_x_128_tiles(dev, case, shared, monkeypatch):
+    plan = _compare(dev, *case, False, monkeypatch)
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+        assert (plan.few_rows, plan.columns, plan.shared_rows) == (2, 128, shared), plan
+
+
+def _compare(dev, kind, M, K, N, R, fp4, monkeypatch):
+    """Compares the launch that the library chooses with the large tiles' and returns its plan."""
     from nunchaku_amd import packing
     from nunchaku_amd.ops import gemm as gemm_mod
 
@@ -68,9 +95,7 @@ def test_against_large_tiles(dev, kind, M, K, N, R, fp4, monkeypatch):
         rot = packing.repack_rotemb(torch.stack((ang.sin(), ang.cos()), dim=-1).reshape(M_pad, 128).to(dev))
         nq = (1.0 + 0.2 * torch.randn(128, generator=g)).to(torch.bfloat16).to(dev)
     want, got, again = run(1), run(None), run(None)
-    assert plans[0].few_rows == 0
-    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
-        assert repr(plans[1]) == repr(plans[2]) and plans[1].few_rows in ((1, 2) if kind == "plain" else (1,) if M <= 256 else (2,)), plans
+    assert plans[0].few_rows == 0 and repr(plans[1]) == repr(plans[2])
     for name in got:
         a, b = got[name].cpu(), want[name].cpu()
         assert torch.equal(a.view(torch.uint8), again[name].cpu().view(torch.uint8)), f"{name} changed between two launches"
@@ -97,6 +122,7 @@ def test_against_large_tiles(dev, kind, M, K, N, R, fp4, monkeypatch):
         logical = packing.act_to_logical(got["qout"].cpu(), N, fp4=fp4, unsigned=not fp4)
         assert torch.equal(logical.to(codes.dtype), codes)
         assert torch.equal(packing.scales_to_logical(got["oscales"].cpu(), fp4).view(torch.uint8), scales.view(torch.uint8))
+    return plans[1]
 
 
 @pytest.mark.parametrize("fp4", [False, True])

@@ -16,8 +16,9 @@ CASES = [
     ((32, 32), 1, 128, 128, 16), ((32, 32), 31, 640, 384, 0), ((32, 32), 33, 384, 256, 48), ((32, 32), 64, 1664, 1152, 80),
     ((32, 64), 32, 1152, 12288, 32), (((32, 64), (32, 32)), 17, 128, 12416, 16), (((32, 64), (64, 32)), 97, 640, 4096, 48), ((64, 32), 128, 3072, 3072, 32),
     (((64, 64), (32, 32)), 256, 1152, 3072, 32), ((64, 64), 225, 2176, 3200, 0), ((64, 64), 300, 2304, 3072, 64),
-    ((32, 128), 89, 2432, 20480, 32), ((64, 128), 1157, 640, 3072, 48),
+    ((32, 128), 89, 2432, 20480, 32), ((64, 128), 1157, 640, 3072, 48), (((64, 128), (32, 64)), 505, 384, 3072, 48), (((64, 128), (32, 64)), 1000, 512, 1536, 0),
 ]
+SHARED_ROWS = [(1157, 640, 3072)]  # (M, K, N) of INT4 launches whose waves share the rows' operands; those of all others split K
 
 
 @pytest.mark.parametrize("fp4", [False, True])
@@ -46,6 +47,7 @@ def test_against_large_tiles(dev, tile, M, K, N, R, fp4, monkeypatch):
     if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
         want = tile[fp4] if isinstance(tile[0], tuple) else tile
         assert plans[0].few_rows == 0 and all((32 * p.few_rows, p.columns) == want for p in plans[1:]), plans
+        assert all(bool(p.shared_rows) == (not fp4 and (M, K, N) in SHARED_ROWS) for p in plans[1:]), plans
     assert torch.equal(outs[1].view(torch.int16), outs[2].view(torch.int16)), "changed between two launches"
     a, b = outs[1].float(), outs[0].float()
     # sums of K products and R more in another order: 2^-24 (K + R) of the largest value at most; then one rounding that may go

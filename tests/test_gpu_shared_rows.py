@@ -1,6 +1,7 @@
 """The INT4 few-rows GEMM whose waves share the rows' operands through LDS (csrc/gemm_direct_kernel.h, ``staged_rows`` in csrc/gemm.hip):
-both remainders that an even number of k-groups leaves by its ring of four (one and three, before the whole turns), the fewest it takes, rows that end inside a tile; the same bits as one wave
-per tile adds up (the large tiles: the same order of the k-groups) where the epilogue is plain."""
+both remainders that an even number of k-groups leaves by its ring of four (one and three, before the whole turns), the fewest it
+takes, rows that end inside a tile; the same bits as one wave per tile adds up (the large tiles: the same order of the k-groups) where the
+epilogue is plain.  (The other epilogues: test_gpu_few_rows.py.)"""
 
 import pytest
 import torch
