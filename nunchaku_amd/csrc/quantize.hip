@@ -583,7 +583,8 @@ int dispatch(const QuantParams &p, hipStream_t stream) {
                 auto rounds = [&](int splits) { return (row_blocks * (splits + projecting) + 2 * ncu - 1) / (2 * ncu); };
                 q.splits = projecting <= 2 && rounds(2) == rounds(1) ? 2 : 1;
                 // (the waves' sums are those of the form that more rows take, bit for bit: in another order they move 4-bit codes of an MLP's second layer.
-                // NVFP4 at ranks above 64 therefore has four waves, which are faster too: M = 3072, rank 128 12.8 us, eight 13.4, M = 2304 10.1 and 10.7)
+                // NVFP4 at ranks above 64 therefore has four waves from here on, eight up to 8 rows per compute unit.  K = 3072, rank 128, eight / four: M = 2304 10.7 / 10.1 us,
+                // M = 3072 13.4 / 12.8, but M = 4608 20.5 / 22.1, K = 12288 88.5 / 98.0.)
                 if constexpr (FP4) {
                     q.splits = RT > 4 ? 1 : q.splits;
                     if (RT > 4) return launch_few_rows<2, FP4, 4>(q, stream);

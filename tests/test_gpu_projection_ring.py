@@ -35,9 +35,12 @@ def test_quantizing_and_projecting_apart_beyond_8_rows_per_compute_unit(dev, M, 
     _check_row_sample(dev, M, K, R, fp4, True)
 
 
-@pytest.mark.parametrize("K,R,fp4,apart,together", [(1152, 64, False, 2304, 4608), (640, 112, True, 2304, 9216), (1152, 48, True, 3072, 9216), (640, 32, True, 4096, 2048)])
+@pytest.mark.parametrize("K,R,fp4,apart,together", [(1152, 64, False, 2304, 4608), (640, 112, True, 2304, 9216), (1152, 48, True, 3072, 9216),
+                                                     (1152, 32, False, 2048, 4096), (6272, 32, True, 2048, 4096)])
 def test_projections_keep_their_bits_from_form_to_form(dev, K, R, fp4, apart, together):
-    """A row's projection is the same whether quantizing and projecting are apart or not: the sums of the waves are added in one order."""
+    """On either side of the most rows for which quantizing and projecting go apart a row's projection is the same: the sums of the waves are added in one
+    order.  (It does change, on 256 compute units, for NVFP4 at ranks 80 ... 128 from 2048 rows to more and at rank 32, K <= 6144, from 4096 to more, where
+    eight waves become four, and beyond 8192 rows for INT4 at ranks 80 ... 128, where the rows are split.)"""
     from gpu_util import make_module
 
     announce(f"projection bits K={K} R={R} fp4={fp4}")

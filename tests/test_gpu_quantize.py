@@ -218,22 +218,27 @@ def test_high_rank_many_rows(dev, M, K, R, fp4, smooth):
 
 @pytest.mark.parametrize("M,K,R,fp4", [(2300, 384, 32, False), (4000, 128, 16, True), (4608, 256, 32, False), (9000, 384, 32, False), (4500, 6272, 16, False),
                                        (2300, 256, 128, False), (2300, 384, 64, False), (9000, 256, 128, False), (2300, 256, 256, False), (1000, 256, 144, False),
-                                       (4608, 256, 32, True), (2300, 256, 128, True), (2300, 384, 64, True), (9000, 256, 32, True)])
+                                       (4608, 256, 32, True), (2300, 256, 128, True), (2300, 384, 64, True), (9000, 256, 32, True),
+                                       (4900, 384, 64, False), (4900, 256, 48, False), (4900, 384, 64, True), (4900, 256, 128, False), (8100, 384, 80, False),
+                                       (6400, 256, 128, True), (6400, 384, 80, True), (4700, 3200, 128, True)])
 def test_workgroup_shapes_by_rows_and_rank(dev, M, K, R, fp4):
     """The launcher picks the workgroup's shape (waves, rows, requests ahead, rows or chunks split among the waves) by
     precision, rank, row count and row length; one case per branch of that choice beyond those the other tests take:
     16 rows on eight waves with two chunks ahead (from 8 to 16 rows per compute unit at ranks up to 32), 32 rows on eight
-    waves (M = 4608; long rows; ranks 64 and 128 from 8 rows per compute unit on; the windows of rank 256), 16 rows on four
-    waves with two chunks ahead (many short rows; NVFP4 at 4608 rows and at rank 128), the rows-split form from 32 rows
-    per compute unit on at rank 128; 1000 rows of rank 144 in quantizing and projecting workgroups."""
+    waves (M = 4608; long rows; ranks 48 ... 64 from 4097 rows on, NVFP4 from 4609, INT4 ranks 80 ... 128 from 4097 to 8192; the windows of rank
+    256), 16 rows on four waves with two chunks ahead (many short rows; NVFP4 at 4608 rows, and at ranks 80 ... 128 from 6145 on, with K > 3072
+    from 4609), the rows-split form from 32 rows per compute unit on at rank 128; 2300 rows of ranks 64 and 128 and 1000 of rank 144 in
+    quantizing and projecting workgroups.  (All on 256 compute units.)"""
     announce(f"quantize workgroup shapes M={M} K={K} R={R} fp4={fp4}")
     _check_row_sample(dev, M, K, R, fp4, True)
 
 
-@pytest.mark.parametrize("M,K,R,fp4", [(2049, 16512, 16, False), (2100, 16512, 64, True), (2304, 16512, 128, False), (8300, 16512, 80, False)])
+@pytest.mark.parametrize("M,K,R,fp4", [(2049, 16512, 16, False), (2100, 16512, 64, True), (2304, 16512, 128, False), (8300, 16512, 80, False),
+                                       (3100, 16512, 64, True), (3100, 16512, 64, False), (3100, 16512, 128, False), (4700, 16512, 128, True)])
 def test_long_k_beyond_the_few_rows(dev, M, K, R, fp4):
-    """The forms that read the smoothing factors from global memory for more rows than the few-rows form takes: 16 rows on eight
-    waves, 32 rows on eight waves at ranks 64 and 128, the rows-split form."""
+    """The forms that read the smoothing factors from global memory for more rows than the few-rows form takes (12 per compute unit at ranks
+    above 32, NVFP4 at ranks above 64 18): 16 rows on eight waves, 32 rows on eight waves at ranks 64 and 128, the rows-split form, 16 rows on four
+    waves (NVFP4, rank 128); and at 2100 and 2304 rows that form, which reads them so at any K."""
     announce(f"quantize long K M={M} K={K} R={R} fp4={fp4}")
     _check_row_sample(dev, M, K, R, fp4, True)
 
