@@ -643,10 +643,11 @@ struct FewRowsTile {
 //          M = 256               14.1 / 13.1 (64 x 64)           15.3 / 14.1
 //          M = 64, K = 12288     32.3 / 21.4 (32 x 32)           34.6 / 21.6
 //          M = 256, K = 12288    34.7 / 30.3 (64 x 64)           37.4 / 34.0
-// INT4, rows or columns fewer than 1024, where 64-row tiles are the better ones of 128 columns: compute units have several tiles, and the model, which does
-// not know the fixed part of a tile well, favours narrow ones too much.  There they are taken if it says 8 %, and not with K = 128 (M = 125, N = 11392,
-// rank 16 5.1 us with 64 x 128, 32 x 32 6.3).  Over 325 INT4 shapes with few columns, short rows or more than 9216 rows 0.9 % off the fastest tile, without this
-// 1.1; the 1111 others 0.2 %, 1727 NVFP4 shapes 0.4 % (M = 1 ... 20000, K = 128 ... 16640, N = 128 ... 21504, ranks 0 ... 160).
+// Few columns, and INT4 with short rows (fewer than 1024), where 64-row tiles are the better ones of 128 columns: compute units have several tiles, and the
+// model, which does not know the fixed part of a tile well, favours narrow ones too much.  There they are taken if it says 8 %, and in INT4 not
+// with K = 128: M = 125, K = 128, N = 11392, rank 16 5.1 us with 64 x 128, 32 x 32 6.3; NVFP4 M = 5041, K = 8448, N = 512 48.2, 64 x 64 55.8.  Over 325 INT4 and 357 NVFP4
+// shapes with few columns, short rows or more than 9216 rows 0.9 and 0.6 % off the fastest tile, without this 1.1 and 0.6; 1111 and 1370 others 0.2 and 0.3 % (M = 1 ...
+// 20000, K = 128 ... 16640, N = 128 ... 21504, ranks 0 ... 160).
 FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu, int shape) {
     struct Model {
         int mt, nc;
@@ -657,11 +658,11 @@ FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu, int shape) {
     constexpr Model nvfp4[] = {{1, 1, -0.85, 0.16, 0.0323}, {1, 2, -0.52, 0.14, 0.0515}, {2, 1, -0.64, 0.24, 0.0498},
                                {2, 2, -0.17, 0.46, 0.0719}, {1, 4, 0.22, 0.47, 0.0876},  {2, 4, 1.96, -0.07, 0.1112}};
     const long long row_blocks = (rows_needed(a) + 31) / 32, column_blocks = a->N / 32;
-    const bool favour_wide = !a->fp4 && shape == 2 && (a->K < 1024 || a->N < 1024);
+    const bool favour_wide = shape == 2 && (a->N < 1024 || (!a->fp4 && a->K < 1024));
     FewRowsTile best{};
     for (const Model &m : a->fp4 ? nvfp4 : int4) {
         const bool wide = m.mt == 2 && m.nc == 4;
-        if (favour_wide && a->K < 256 && !wide) continue;
+        if (favour_wide && !a->fp4 && a->K < 256 && !wide) continue;
         const long long tiles = (row_blocks + m.mt - 1) / m.mt * (column_blocks / m.nc);
         const double t = (m.launch + (double)((tiles + ncu - 1) / ncu) * (m.tile + m.kgroup * (double)(a->K / 64))) * (favour_wide && wide ? 0.92 : 1.0);
         if (best.mt == 0 || t < best.time) best = FewRowsTile{m.mt, m.nc, false, t};
@@ -687,7 +688,7 @@ bool staged_rows(const svdq_gemm_args *a, int ncu, bool split) {
 // K.  Shape 2: tiles of 64 rows x 128 columns, a quarter fewer operand bytes per product, from about 400 tiles of 32 rows on; INT4: two waves
 // split K and two the columns, NVFP4: four waves split K.  Models of the time in us fitted to launches at K = 1024 ... 12288
 // on 256 compute units, linear in the number of tiles that the busiest compute unit works through and in the k-groups; they met
-// the measurements within about 10 % when they were fitted, over 2200 random shapes; what has changed since is in the factors below.  Measured at K = 3072 at the time of the fit, large tiles (split along K where that pays) / shape 1 / shape 2:
+// the measurements within about 10 % when they were fitted, over 2200 random shapes; what has changed since is in the terms below (NVFP4 beside whole large tiles: other models).  Measured at K = 3072 at the time of the fit, large tiles (split along K where that pays) / shape 1 / shape 2:
 //   INT4   M = 256, N = 3072   22.8 /  9.6 / 12.3     NVFP4  60.7 / 11.8 / 13.8
 //          M = 505, N = 9216   28.7 / 33.1 / 30.6            62.9 / 38.4 / 34.1
 //          M = 1157, N = 3072  29.7 / 27.6 / 21.8            62.1 / 31.7 / 25.7

@@ -26,7 +26,7 @@ def test_the_tile_of_a_launch(M, K, N, want, fp4):
 # per compute unit; and ones where a tile of another height than that of the better one of 128 columns is the fastest.
 @pytest.mark.parametrize("M,K,N,fp4,want", [
     (125, 128, 11392, False, (64, 128)), (500, 128, 2176, False, (64, 128)), (5494, 2560, 256, False, (64, 128)), (556, 2944, 4096, False, (64, 64)),
-    (297, 1280, 3456, True, (32, 64)), (788, 4224, 7680, True, (64, 128)), (261, 1280, 21376, True, (64, 128)),
+    (297, 1280, 3456, True, (32, 64)), (788, 4224, 7680, True, (64, 128)), (261, 1280, 21376, True, (64, 128)), (5041, 8448, 512, True, (64, 128)),
 ])
 def test_narrow_tiles_only_where_they_are_faster(M, K, N, fp4, want):
     p = plan_of(call("plain", M, K, N, 32, fp4))
