@@ -442,6 +442,7 @@ void fill_params(const svdq_gemm_args *a, GemmParams &p) {
     p.counters = nullptr;
     p.whole_band = 0;
     p.row_blocks = 0;
+    p.lr_steps = 0;
 }
 
 // ---- INT4: fp6 matrix instruction on the bare codes (gemm6_kernel.h) --------------------------------

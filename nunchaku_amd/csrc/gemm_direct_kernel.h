@@ -15,7 +15,7 @@
 // plain_tile in gemm.hip: square ones fetch least per product, small ones use more compute units.  The others have 128 columns, which a
 // head of the norm and a chunk of the next layer's projection have.  With several tiles per compute
 // unit the matrix core and the conversions bound it (M = 1157, K = 12288, NVFP4: 10 % waits for operands, 49 and 34 % the others).
-// M = 256, K = N = 3072: 22.8 -> 8.8 -> 7.9 us (INT4; 4 us of it do not depend on K), 59.9 -> 10.6 -> 9.4 us (NVFP4); M = 64: 8.6 -> 5.6 and 9.7 -> 5.5.
+// M = 256, K = N = 3072: 22.8 -> 8.8 -> 7.6 us (INT4; 4 us of it do not depend on K), 59.9 -> 10.6 -> 9.2 us (NVFP4); M = 64: 8.6 -> 5.1 and 9.7 -> 5.4.
 //
 // INT4: one fp6 matrix instruction on the codes, one factor instruction and 16 multiply-adds per 32 x 32 tile and
 // k-group (gemm6_kernel.h).  NVFP4: both operands are dequantized to fp16 in registers by the wave that uses them
@@ -53,22 +53,32 @@ struct Stage<true, MT, NT> {
 };
 
 constexpr int SLAB_BYTES = 32 * OUT_LD * 2;
-// LDS: the waves' sums of 32 rows x 128 columns, [KP][4 column tiles][4 quads][64 lanes] x float4; behind them the sums of
-// squares of the RMS norm, [MT][4][32] floats.  The bf16 slabs take the place of the sums.
-// Tiles narrower than 128 columns: the sums of all row blocks at once, and a slab of its own for every wave behind them.
-constexpr int NARROW_LD = 40, NARROW_SLAB_BYTES = 32 * NARROW_LD * 2;
-template <int MT, int KP>
-constexpr int ssq_offset() {
-    return KP * 16384 > MT * SLAB_BYTES ? KP * 16384 : MT * SLAB_BYTES;
-}
 // Waves that split the columns only (WN = 4, INT4, 64 rows): a stage of the rows' operands of one k-group in LDS, two fragments and the scales of
 // 64 rows, eight times over in a whole KB; behind them zeros, what the upper half-wave reads as its scale.
 constexpr int STAGE_ZEROS = 2 * FRAG_BYTES + 1024, STAGE_BYTES = STAGE_ZEROS + 128;
-template <int MT, int NC, int KP, int DEPTH>
-constexpr int lds_bytes() {
-    constexpr int epilogue = NC == 4 ? ssq_offset<MT, KP>() + MT * 512 : KP * MT * NC * 4096 + MT * NC * NARROW_SLAB_BYTES;
-    return KP == 1 && (DEPTH + 1) * STAGE_BYTES > epilogue ? (DEPTH + 1) * STAGE_BYTES : epilogue;
-}
+// LDS.  First the waves' sums, [KP][column tiles (tiles narrower than 128 columns: and row blocks)][4 quads][64 lanes] x float4, 32 rows at a time in tiles of 128 columns,
+// or the stages of waves that share the rows' operands; the bf16 slabs take their place, narrow tiles have a slab of its own for every wave behind the sums.  Then the sums of
+// squares of the RMS norm, [MT][4][32] floats, and for every wave the factors and biases of its 32 columns.  Beside the stages stand what is copied there while the main loop runs:
+// bias and wcscales of the tile's columns, and the low-rank operands of up to LR_AHEAD 16-rank steps, per 32 ranks [columns][4 pieces of 16 bytes of lora_up], then [rows][8 pieces
+// of lora_act], piece q of a row at place q ^ swizzle(row) (gemm_params.h).
+constexpr int NARROW_LD = 40, NARROW_SLAB_BYTES = 32 * NARROW_LD * 2;
+template <int MT, int NT, int WN, int KP, int DEPTH>
+struct Lds {
+    static constexpr int NC = NT * WN;
+    static constexpr bool NARROW = NC < 4, STAGED = KP == 1;
+    static constexpr int SUMS = STAGED ? (DEPTH + 1) * STAGE_BYTES : KP * (NARROW ? MT * NC : 4) * 4096;
+    static constexpr int SLABS = NARROW ? SUMS : 0, SLABS_END = SLABS + (NARROW ? MT * NC * NARROW_SLAB_BYTES : MT * SLAB_BYTES);
+    static constexpr int SSQ = SUMS > SLABS_END ? SUMS : SLABS_END, TAB = SSQ + (NARROW ? 0 : MT * 512), LR = TAB + 4 * 256;  // (beside the stages: bias at TAB, wcscales behind it)
+    static constexpr int LR_ACT = NC * 32 * 64, LR_CHUNK = LR_ACT + MT * 32 * 128, LR_AHEAD = STAGED ? 6 : 0;
+    // (a compute unit has LDS for two workgroups with six steps ahead or for three with four: M = 256, K = 8064, N = 19840, rank 96, quantizing, 2.4 tiles per compute unit, 80 us
+    // with four steps, 87 with six; M = 256, K = 3072, N = 9216, rank 128 22.5 and 20.9)
+    static constexpr int lr_steps(int R, bool three) {
+        const int most = three && LR_AHEAD > 4 ? 4 : LR_AHEAD;
+        return R / 16 < most ? R / 16 : most;
+    }
+    static constexpr int bytes(int steps) { return LR + (steps + 1) / 2 * LR_CHUNK; }
+    static_assert(bytes(LR_AHEAD) <= 80 * 1024 && (!STAGED || 3 * bytes(4) <= 160 * 1024));
+};
 
 template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT>
 __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_kernel(GemmParams p) {
@@ -76,7 +86,8 @@ __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_ker
     constexpr int WAVES = WN * KP;
     constexpr bool NARROW = NC < 4;
     constexpr bool STAGED = WN == 4;
-    static_assert(!STAGED || (!FP4 && MT == 2 && NT == 1 && KP == 1 && (DEPTH + 1) * STAGE_BYTES <= lds_bytes<MT, NC, KP, DEPTH>()));
+    using L = Lds<MT, NT, WN, KP, DEPTH>;
+    static_assert(!STAGED || (!FP4 && MT == 2 && NT == 1 && KP == 1));
     static_assert(WAVES == 4 && MT * NC <= (NARROW ? 4 : 8), "the epilogue gives each wave one column tile, of one row block where the tile is narrow");
     static_assert(!NARROW || !NEXT, "the norm, the rotation and the next layer's operands need whole 128-column blocks");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -161,6 +172,68 @@ __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_ker
         g_load += more ? KP : 0;
     };
 
+    // ---- the epilogue's own operands -------------------------------------------------------------------
+    // Wave w gets the 32 columns 32 w ... of all MT row blocks; of a narrow tile one of the MT NC blocks of 32 x 32, where there is one.  What it needs for them is requested ahead
+    // of the main loop as far as there is room for it: factors and biases; in narrow INT4 tiles the low-rank operands of EARLY 16-rank steps, in registers; beside the stages all of it,
+    // in LDS and in whole pieces of rows (a lane that fetches 16 bytes of each of 32 rows for itself costs the vector memory path four times as much).  Requested behind the main loop /
+    // as it is, us: INT4 M = 256, K = N = 3072, rank 32 7.84 / 7.55, rank 64 8.8 / 7.9, rank 128 10.0 / 9.3, M = 64 5.24 / 5.01; NVFP4 M = 300 9.3 / 8.9; tiles of 128 columns M = 100,
+    // K = 2048, N = 8192, quantizing 15.95 / 15.2, NVFP4 M = 300, K = 3072, N = 9216 with norm and rotary 33.5 / 32.1; shared rows M = 256, K = 3072, N = 9216 with norm and rotary
+    // 18.8 / 17.5, rank 128 25.1 / 20.8, quantizing, N = 12288 25.3 / 23.5, M = 200, K = 1024, N = 15360, rank 128 16.2 / 11.6.  Same bits.  Slower: low-rank operands ahead in
+    // narrow NVFP4 tiles (several of them share a compute unit: M = 916, K = 1920, N = 1152 10.4 us, 10.7 with), more than two steps in registers, all of them through the place of the
+    // sums, which takes two barriers more, the rotary table and the smoothing factors ahead too.  (With three INT4 tiles of 64 x 64 per compute unit it costs 1 %: M = 1979, K = 4096,
+    // N = 1152 22.0 / 22.3.)
+    constexpr int OWN = NARROW ? 1 : MT, LR_AHEAD = L::LR_AHEAD, EARLY = NARROW && !FP4 ? 2 : 0;
+    constexpr bool TABLE = !STAGED && (!NARROW || FP4 || MT * NC < 4);  // factors and biases through a table of the wave's
+    const bool owner = !NARROW || wave < MT * NC;
+    const int nt = NARROW ? wave % NC : wave, c0 = n0 + nt * 32, row0 = f0 * 32 + (NARROW ? wave / NC * 32 : 0);
+    const int nsteps = p.R_up / 16, lr_steps = p.lr_steps;
+    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
+    struct LowRank {
+        float4_t la[OWN][2];
+        u32x4_t up;
+    };
+    auto load_low_rank = [&](LowRank &l, int step) {
+#pragma unroll
+        for (int o = 0; o < OWN; o++) {
+            const float4_t *ap = (const float4_t *)(p.lora_act + (size_t)(row0 + o * 32 + r32) * p.R_up + 16 * step + 8 * h);
+            l.la[o][0] = ap[0];
+            l.la[o][1] = ap[1];
+        }
+        l.up = *(const u32x4_t *)(p.lora_up + (size_t)(c0 + r32) * p.R_up + 16 * step + 8 * h);
+    };
+    LowRank early[EARLY > 0 ? EARLY : 1];
+    if (owner) {
+#pragma unroll
+        for (int s = 0; s < EARLY; s++)
+            if (nsteps > 0) load_low_rank(early[s], s < nsteps ? s : nsteps - 1);
+    }
+    // INT4 tiles of 64 x 64 have room for the scales and biases of the lane's columns c0 + 8 q + 4 h + i, the others for those of column c0 + r32.
+    constexpr bool RAW = !TABLE && !STAGED;
+    u32x2_t wcscales4[RAW ? 4 : 1], bias4[RAW ? 4 : 1];
+    float colnorm1 = 1.f;
+    uint16_t wcscale1 = 0x3F80, bias1 = 0;
+    if constexpr (RAW) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            wcscales4[q] = u32x2_t{0x3F803F80u, 0x3F803F80u};
+            bias4[q] = u32x2_t{0u, 0u};
+        }
+        if (p.wcscales) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) wcscales4[q] = *(const u32x2_t *)(p.wcscales + c0 + 8 * q + 4 * h);
+        }
+        if (p.bias) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) bias4[q] = *(const u32x2_t *)(p.bias + c0 + 8 * q + 4 * h);
+        }
+    } else if constexpr (TABLE) {
+        if (owner) {
+            if (FP4) colnorm1 = p.colnorm[c0 + r32];
+            if (p.wcscales) wcscale1 = p.wcscales[c0 + r32];
+            if (p.bias) bias1 = p.bias[c0 + r32];
+        }
+    }
+
     // ---- main loop -----------------------------------------------------------------------------------
     float16_t acc[NT * MT];  // tile t = nt MT + mt
 #pragma unroll
@@ -243,7 +316,7 @@ __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_ker
         // takes 0.2 us per k-group with three on their way (0.33 with two: the latency of the requests), two share it better than that, until the
         // vector instructions bound them: 50 per k-group, with the columns through buffers and the scales as lasting pairs (61 before: QKV M = 256, K =
         // 3072, N = 9216 24.7 -> 23.5 us).  Which launches, and what they gain: staged_rows in gemm.hip.
-        const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds + wave * 1024;
+        const uint32_t base = lds_base + wave * 1024;
         const bool rows = wave < 3;
         const uint8_t *src = rows ? p.act + ((size_t)(f0 >> 2) * kgroups) * (4 * FRAG_BYTES) + (f0 & 3) * FRAG_BYTES + wave * 1024 : (const uint8_t *)(p.ascales + f0 * 32);
         const uint32_t stride = rows ? 4 * FRAG_BYTES : (uint32_t)p.M_pad * 2, voff = rows ? lane * 16 : (lane & 7) * 16;
@@ -264,6 +337,27 @@ __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_ker
         const uint32_t off_rows = h ? (uint32_t)STAGE_ZEROS : 2u * FRAG_BYTES + (uint32_t)r32 * 2u;
         const __amdgpu_buffer_rsrc_t wbuf = buffer(wp, (uint32_t)(kgroups - 1) * (8 * FRAG_BYTES) + FRAG_BYTES), sbuf = buffer(sp, (uint32_t)(kgroups - 1) * 2048 + 256);
         int g_req = 0;
+        // The epilogue's operands: the oldest requests, landed when the first k-group has, with all others' behind the same barrier.  (Code of its own behind the kernel's.)
+        if (__builtin_expect(lr_steps > 0 || p.bias || p.wcscales, 0)) {
+            const uint8_t *columns = (const uint8_t *)(wave == 0 ? p.bias : wave == 1 ? p.wcscales : nullptr);  // 128 bf16: a word a lane
+            if (columns)
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" :: "s"(lds_base + L::TAB + wave * 256), "v"(lane * 4), "s"(columns + n0 * 2) : "memory", "m0");
+            // (32 ranks at a time; which 16 bytes of its row a lane fetches is permuted as in gemm6_kernel.h)
+            for (int c = 0; 2 * c < lr_steps; c++) {
+                const bool half = nsteps - 2 * c < 2;  // 16 ranks only: the other half of the places is filled with anything
+                const uint32_t place = lds_base + L::LR + c * L::LR_CHUNK;
+                const uint8_t *up = (const uint8_t *)p.lora_up + (size_t)n0 * p.R_up * 2 + c * 64, *la = (const uint8_t *)p.lora_act + (size_t)row0 * p.R_up * 4 + c * 128;
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const int col = (wave * 2 + i) * 16 + (lane >> 2), row = (wave * 2 + i) * 8 + (lane >> 3);
+                    const int up_piece = (lane & 3) ^ g6::lr_up_swizzle(col), act_piece = (lane & 7) ^ g6::lr_act_swizzle(row);
+                    const uint32_t up_off = (uint32_t)col * (uint32_t)(p.R_up * 2) + (half ? up_piece & 1 : up_piece) * 16;
+                    const uint32_t act_off = (uint32_t)row * (uint32_t)(p.R_up * 4) + (half ? act_piece & 3 : act_piece) * 16;
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(place + (wave * 2 + i) * 1024), "v"(up_off), "s"(up) : "memory", "m0");
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(place + L::LR_ACT + (wave * 2 + i) * 1024), "v"(act_off), "s"(la) : "memory", "m0");
+                }
+            }
+        }
         auto request = [&](auto S) {
             constexpr int st = decltype(S)::value;
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(base + st * STAGE_BYTES), "v"(voff), "s"(src) : "memory", "m0");
@@ -371,43 +465,42 @@ __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_ker
         }
     }
 
-    // ---- the epilogue's own operands, requested before the waves meet ------------------------------------
-    // Wave w gets the 32 columns 32 w ... of all MT row blocks; of a narrow tile one of the MT NC blocks of 32 x 32, where there is one.
-    constexpr int OWN = NARROW ? 1 : MT;
-    const bool owner = !NARROW || wave < MT * NC;
-    const int nt = NARROW ? wave % NC : wave, c0 = n0 + nt * 32, row0 = f0 * 32 + (NARROW ? wave / NC * 32 : 0);
-    const int nsteps = p.R_up / 16;
-    constexpr int LSTEPS = 2;  // 16-rank steps of the low-rank up projection requested at once
-    float4_t la_raw[OWN][LSTEPS][2];
-    u32x4_t up_raw[LSTEPS];
-    auto load_lora = [&](int s0) {
+    // The low-rank operands that have not been requested yet, two steps at a time (four, three of two row blocks or six in narrow tiles: slower).
+    constexpr int LSTEPS = 2;
+    const int LFIRST = STAGED ? lr_steps : EARLY;
+    LowRank more[LSTEPS];
+    auto load_more = [&](int s0) {
 #pragma unroll
-        for (int s = 0; s < LSTEPS; s++) {
-            const int step = s0 + s < nsteps ? s0 + s : nsteps - 1;
-#pragma unroll
-            for (int o = 0; o < OWN; o++) {
-                const float4_t *ap = (const float4_t *)(p.lora_act + (size_t)(row0 + o * 32 + r32) * p.R_up + 16 * step + 8 * h);
-                la_raw[o][s][0] = ap[0];
-                la_raw[o][s][1] = ap[1];
-            }
-            up_raw[s] = *(const u32x4_t *)(p.lora_up + (size_t)(c0 + r32) * p.R_up + 16 * step + 8 * h);
-        }
+        for (int s = 0; s < LSTEPS; s++)
+            if (s0 + s < nsteps) load_low_rank(more[s], s0 + s);
     };
-    float cf[4][4], bs[4][4];  // factor and bias of the lane's columns c0 + 8 q + 4 h + i
-    if (owner && nsteps > 0) load_lora(0);
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        if (!owner) break;
-        const int c = c0 + 8 * q + 4 * h;
-        const float4_t cn = FP4 ? *(const float4_t *)(p.colnorm + c) : float4_t{1.f, 1.f, 1.f, 1.f};
-        const u32x2_t wc = p.wcscales ? *(const u32x2_t *)(p.wcscales + c) : u32x2_t{0x3F803F80u, 0x3F803F80u};
-        const u32x2_t bi = p.bias ? *(const u32x2_t *)(p.bias + c) : u32x2_t{0u, 0u};
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            cf[q][i] = cn[i] * p.alpha * bits_f32(i & 1 ? wc[i >> 1] & 0xFFFF0000u : wc[i >> 1] << 16);
-            bs[q][i] = bits_f32(i & 1 ? bi[i >> 1] & 0xFFFF0000u : bi[i >> 1] << 16);
-        }
+    if (owner) load_more(LFIRST);
+    // Factor and bias of the lane's columns c0 + 8 q + 4 h + i.
+    float *tab = (float *)(lds + L::TAB + wave * 256);
+    if (TABLE && h == 0) {
+        tab[r32] = colnorm1 * p.alpha * bf16_bits_to_f32(wcscale1);
+        tab[32 + r32] = bf16_bits_to_f32(bias1);
     }
+    auto four = [](u32x2_t w) {
+        return float4_t{bits_f32(w[0] << 16), bits_f32(w[0] & 0xFFFF0000u), bits_f32(w[1] << 16), bits_f32(w[1] & 0xFFFF0000u)};
+    };
+    auto factors = [&](int q) {
+        if constexpr (TABLE) return *(const float4_t *)(tab + 8 * q + 4 * h);
+        float4_t f = {1.f, 1.f, 1.f, 1.f}, w;
+        if constexpr (STAGED) {
+            w = p.wcscales ? four(*(const u32x2_t *)(lds + L::TAB + 256 + (nt * 32 + 8 * q + 4 * h) * 2)) : f;
+        } else {
+            w = four(wcscales4[q]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) f[i] = f[i] * p.alpha * w[i];
+        return f;
+    };
+    auto biases = [&](int q) {
+        if constexpr (TABLE) return *(const float4_t *)(tab + 32 + 8 * q + 4 * h);
+        else if constexpr (STAGED) return p.bias ? four(*(const u32x2_t *)(lds + L::TAB + (nt * 32 + 8 * q + 4 * h) * 2)) : float4_t{0.f, 0.f, 0.f, 0.f};
+        else return four(bias4[q]);
+    };
 
     // ---- the waves' sums meet, 32 rows at a time, added in ascending order of the waves ---------------------
     float16_t val[OWN];
@@ -456,38 +549,65 @@ __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_ker
         __syncthreads();  // the sums have been read: the slabs take their place
     }
 
-    float *ssq = (float *)(lds + ssq_offset<MT, KP>());  // [MT][4 column tiles][32 rows]
+    float *ssq = (float *)(lds + L::SSQ);  // [MT][4 column tiles][32 rows]
     const bool rope = NEXT && p.rotary && n0 < p.rope_cols;  // the tile is one head of q or k
+    if (FP4 || p.wcscales || p.alpha != 1.f) {
 #pragma unroll
-    for (int o = 0; o < OWN; o++)
+        for (int q = 0; q < 4; q++) {
+            const float4_t cf = factors(q);
 #pragma unroll
-        for (int e = 0; e < 16; e++) val[o][e] *= cf[e >> 2][e & 3];
-    // Low-rank up projection (lora.cuh:110-241): out += bf16(lora_act * scale) @ up^T
-    for (int s0 = 0; s0 < nsteps; s0 += LSTEPS) {
-        if (s0 > 0) load_lora(s0);
+            for (int o = 0; o < OWN; o++)
 #pragma unroll
-        for (int s = 0; s < LSTEPS; s++) {
-            if (s0 + s >= nsteps) break;
-            const float ls = p.lora_scales[s0 + s];
-#pragma unroll
-            for (int o = 0; o < OWN; o++) {
-                const float4_t v0 = la_raw[o][s][0], v1 = la_raw[o][s][1];
-                u32x4_t w;
-                w[0] = pack_bf16x2(v0[0] * ls, v0[1] * ls);
-                w[1] = pack_bf16x2(v0[2] * ls, v0[3] * ls);
-                w[2] = pack_bf16x2(v1[0] * ls, v1[1] * ls);
-                w[3] = pack_bf16x2(v1[2] * ls, v1[3] * ls);
-                val[o] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, up_raw[s]), __builtin_bit_cast(bf16x8_t, w), val[o], 0, 0, 0);
-            }
+                for (int i = 0; i < 4; i++) val[o][4 * q + i] *= cf[i];
         }
     }
+    // Low-rank up projection (lora.cuh:110-241): out += bf16(lora_act * scale) @ up^T
+    auto add_low_rank = [&](int o, int step, float4_t v0, float4_t v1, u32x4_t up) {
+        const float ls = p.lora_scales[step];
+        u32x4_t w;
+        w[0] = pack_bf16x2(v0[0] * ls, v0[1] * ls);
+        w[1] = pack_bf16x2(v0[2] * ls, v0[3] * ls);
+        w[2] = pack_bf16x2(v1[0] * ls, v1[1] * ls);
+        w[3] = pack_bf16x2(v1[2] * ls, v1[3] * ls);
+        val[o] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, up), __builtin_bit_cast(bf16x8_t, w), val[o], 0, 0, 0);
+    };
+    auto add_step = [&](const LowRank &l, int step) {
 #pragma unroll
-    for (int o = 0; o < OWN; o++)
+        for (int o = 0; o < OWN; o++) add_low_rank(o, step, l.la[o][0], l.la[o][1], l.up);
+    };
 #pragma unroll
-        for (int e = 0; e < 16; e++) val[o][e] += bs[e >> 2][e & 3];
+    for (int s = 0; s < EARLY; s++)
+        if (s < nsteps) add_step(early[s], s);
+#pragma unroll
+    for (int s = 0; s < LR_AHEAD; s++) {
+        if (s >= lr_steps) break;
+        const uint8_t *buf = lds + L::LR + (s / 2) * L::LR_CHUNK;
+        const int col = wave * 32 + r32, k = s % 2;
+        const u32x4_t up = *(const u32x4_t *)(buf + col * 64 + (((2 * k + h) ^ g6::lr_up_swizzle(col)) << 4));
+#pragma unroll
+        for (int o = 0; o < OWN; o++) {
+            const int row = o * 32 + r32;
+            const uint8_t *ap = buf + L::LR_ACT + row * 128;
+            add_low_rank(o, s, *(const float4_t *)(ap + (((4 * k + 2 * h) ^ g6::lr_act_swizzle(row)) << 4)), *(const float4_t *)(ap + (((4 * k + 2 * h + 1) ^ g6::lr_act_swizzle(row)) << 4)), up);
+        }
+    }
+    for (int s0 = LFIRST; s0 < nsteps; s0 += LSTEPS) {
+        if (s0 > LFIRST) load_more(s0);
+#pragma unroll
+        for (int s = 0; s < LSTEPS; s++)
+            if (s0 + s < nsteps) add_step(more[s], s0 + s);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const float4_t bs = biases(q);
+#pragma unroll
+        for (int o = 0; o < OWN; o++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) val[o][4 * q + i] += bs[i];
+    }
     if constexpr (NARROW) {
         // the wave's 32 x 32 block through its own slab, in rows of 64 contiguous bytes
-        uint16_t *slab = (uint16_t *)(lds + KP * MT * NC * 4096 + wave * NARROW_SLAB_BYTES);
+        uint16_t *slab = (uint16_t *)(lds + L::SLABS + wave * NARROW_SLAB_BYTES);
 #pragma unroll
         for (int q = 0; q < 4; q++) {
             u32x2_t w;
@@ -656,18 +776,21 @@ __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_ker
 }
 
 template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT>
-int launch_direct(const GemmParams &p, hipStream_t stream) {
+int launch_direct(const GemmParams &params, hipStream_t stream) {
     auto kern = gemm_direct_kernel<FP4, MT, NT, WN, KP, DEPTH, NEXT>;
-    constexpr int smem = lds_bytes<MT, NT * WN, KP, DEPTH>();
+    using L = Lds<MT, NT, WN, KP, DEPTH>;
     static bool lds_reserved[64] = {false};  // set once per device (racing first calls both set it, which is harmless)
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(SVDQ_ELAUNCH, "gemm: cannot identify the current device");
     if (!lds_reserved[dev]) {
-        hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-        if (e != hipSuccess) return fail(SVDQ_ELAUNCH, "gemm: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
+        hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, L::bytes(L::LR_AHEAD));
+        if (e != hipSuccess) return fail(SVDQ_ELAUNCH, "gemm: cannot reserve %d bytes of LDS: %s", L::bytes(L::LR_AHEAD), hipGetErrorString(e));
         lds_reserved[dev] = true;
     }
-    SVDQ_LAUNCH(kern, dim3((unsigned)(p.row_blocks * (p.N / (32 * NT * WN)))), dim3(64 * WN * KP), smem, stream, p);
+    GemmParams p = params;
+    const int tiles = p.row_blocks * (p.N / (32 * NT * WN));
+    p.lr_steps = L::lr_steps(p.R_up, tiles > 2 * compute_units(dev));
+    SVDQ_LAUNCH(kern, dim3((unsigned)tiles), dim3(64 * WN * KP), L::bytes(p.lr_steps), stream, p);
     return check_launch("gemm_w4a4 (few rows)");
 }
 
