@@ -68,6 +68,12 @@ class GemmArgs(ctypes.Structure):
     ]
 
 
+class GemmCall(GemmArgs):
+    """A GEMM's argument block and the low-rank factors it points to (``host().gemm_call`` fills both in)."""
+
+    _fields_ = [("scales", ctypes.c_float * 64)]
+
+
 class AwqGemvArgs(ctypes.Structure):
     """Mirror of ``svdq_awq_gemv_args``."""
 

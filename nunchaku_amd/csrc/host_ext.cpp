@@ -3,7 +3,11 @@
 // A forward pass of one quantized layer is two kernel launches of a few microseconds each.  Checking the arguments, looking
 // at the parameters' version counters, allocating four tensors and filling two argument blocks took 19.6 us in Python (31.2
 // for the fused MLP, 29.4 for the QKV projection, 11.4 for the AWQ layer), more than the GPU needs for a few hundred tokens;
-// here it takes 8.8 (14.1, 8.4 and 5.1), most of it the launches themselves.
+// here it takes 8.8 (14.1, 8.4 and 5.1), most of it the launches themselves.  The operators called one by one keep their one
+// way to the library (_native.launch); what is here is their checks, allocations and argument blocks.  They took 12.7 us
+// (quantize), 13.9 (GEMM; 17.8 with linear attention, which clears out_vk in a launch of its own) and 8.5
+// (linearattn_vk_mul_q) of the caller's time, and take 8.8, 5.4 (8.3) and 3.5: linear attention over 256 tokens at K = 1024,
+// four launches of which the GPU runs 18 us, went from 46.5 us to 25.9.
 //
 // Every function returns None when anything about the call is not the plain case it handles (another dtype, a parameter
 // that has been replaced since the layer was converted, a tensor that is not contiguous, ...): the Python code behind it
@@ -46,6 +50,7 @@ struct Layer {
 const char *LAYER = "nunchaku_amd._host.Layer";
 
 PyObject *s_parameters, *s_lora_scales, *s_qweight, *s_wscales, *s_wzeros, *s_bias, *s_in_features, *s_out_features, *s_group_size;
+PyObject *s_native, *s_logical_shape, *s_colnorm, *s_nonzero, *s_lora_up, *s_lora_down, *s_vector, *s_smooth_rcp;
 
 void free_layer(PyObject *capsule) {
     Layer *l = (Layer *)PyCapsule_GetPointer(capsule, LAYER);
@@ -452,8 +457,192 @@ PyObject *awq_linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
+// ---- the operators: checks, allocations and argument blocks --------------------------------------------------------------
+// an attribute of a tensor (new reference) or null without an exception
+PyObject *attribute(PyObject *o, PyObject *name) {
+    PyObject *a = PyObject_GetAttr(o, name);
+    if (!a) PyErr_Clear();
+    return a;
+}
+// `o` is a tensor in the layout `kind` of the kernels, contiguous, on x's device
+bool native_tensor(PyObject *o, PyObject *kind, const at::Tensor &x, const at::Tensor **t) {
+    if (!as_tensor(o, t) || (*t)->device() != x.device() || !(*t)->is_contiguous()) return false;
+    PyObject *a = attribute(o, s_native);
+    const bool ok = a && (a == kind || (PyUnicode_Check(a) && PyUnicode_Compare(a, kind) == 0));
+    Py_XDECREF(a);
+    return ok;
+}
+bool shape_is(const at::Tensor &t, at::IntArrayRef sizes) { return t.sizes() == sizes; }
+bool checked(PyObject *o, const at::Tensor &x, at::ScalarType dt, at::IntArrayRef sizes, const at::Tensor **t) {
+    return as_tensor(o, t) && (*t)->device() == x.device() && (*t)->scalar_type() == dt && (*t)->is_contiguous() && shape_is(**t, sizes);
+}
+at::Tensor new_tensor(at::IntArrayRef sizes, at::ScalarType dt, const at::Tensor &x) {
+    return at::empty(sizes, at::TensorOptions().dtype(dt).device(x.device()));
+}
+
+// quantize_call(block address, input, lora_down, smooth or None, fp4, pad_size) -> (output, oscales, lora_act_out) with the block filled in, or None
+PyObject *quantize_call(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    SVDQ_NARGS(6)
+    svdq_quantize_args *q = (svdq_quantize_args *)PyLong_AsVoidPtr(args[0]);
+    if (!q) return PyErr_Occurred() ? nullptr : (PyErr_SetString(PyExc_ValueError, "quantize_call: null argument block"), nullptr);
+    const at::Tensor *x, *down, *smooth = nullptr;
+    bool fp4;
+    int64_t pad;
+    if (!as_tensor(args[1], &x) || !x->is_cuda() || x->dim() != 2 || x->scalar_type() != at::kBFloat16 || !x->is_contiguous() || x->size(0) <= 0 ||
+        !as_bool(args[4], &fp4) || !as_int(args[5], &pad) || pad <= 0 || pad % 256) Py_RETURN_NONE;
+    const int64_t M = x->size(0), K = x->size(1), M_pad = (M + pad - 1) / pad * pad, G = fp4 ? 16 : 64;
+    if (K % 128 || !native_tensor(args[2], s_lora_down, *x, &down) || down->dim() != 2 || down->size(0) != K || down->scalar_type() != at::kBFloat16) Py_RETURN_NONE;
+    if (args[3] != Py_None && (!native_tensor(args[3], s_smooth_rcp, *x, &smooth) || smooth->numel() != K || smooth->scalar_type() != at::kFloat)) Py_RETURN_NONE;
+    const int64_t R = down->size(1);
+    at::Tensor out = new_tensor({M_pad, fp4 ? K / 2 : K * 3 / 4}, at::kByte, *x), scales = new_tensor({K / G, M_pad}, fp4 ? at::kFloat8_e4m3fn : at::kBFloat16, *x),
+               lora = new_tensor({M_pad, R}, at::kFloat, *x);
+    *q = svdq_quantize_args{};
+    q->input = x->data_ptr();
+    q->output = out.data_ptr();
+    q->oscales = scales.data_ptr();
+    q->lora_down = R ? down->data_ptr() : nullptr;
+    q->lora_act_out = R ? (float *)lora.data_ptr() : nullptr;
+    q->smooth_rcp = smooth ? (const float *)smooth->data_ptr() : nullptr;
+    q->M = M;
+    q->M_pad = M_pad;
+    q->K = K;
+    q->R = R;
+    q->fp4 = fp4;
+    PyObject *r = PyTuple_New(3);
+    if (!r) return nullptr;
+    PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(out));
+    PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(scales));
+    PyTuple_SET_ITEM(r, 2, THPVariable_Wrap(lora));
+    return r;
+    END_HANDLE_TH_ERRORS
+}
+
+// gemm_call(block address, address of MAX_GROUPS floats, act, wgt, ascales, wscales, out or None, out_vk or None, out_linearattn or None, lora_act_in or None, lora_up or
+// None, bias or None, wcscales or None, lora_scales or None, alpha, act_unsigned, fuse_silu, fp4, k_split) -> True with the block filled in, or None
+PyObject *gemm_call(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    SVDQ_NARGS(19)
+    svdq_gemm_args *g = (svdq_gemm_args *)PyLong_AsVoidPtr(args[0]);
+    float *sc = (float *)PyLong_AsVoidPtr(args[1]);
+    if (!g || !sc) return PyErr_Occurred() ? nullptr : (PyErr_SetString(PyExc_ValueError, "gemm_call: null argument block"), nullptr);
+    const at::Tensor *act, *wgt, *asc, *wsc, *out = nullptr, *vk = nullptr, *la = nullptr, *up = nullptr, *bias = nullptr, *wcs = nullptr, *colnorm = nullptr;
+    bool unsigned_codes, silu, fp4;
+    int64_t k_split, N, K;
+    if (!as_bool(args[15], &unsigned_codes) || !as_bool(args[16], &silu) || !as_bool(args[17], &fp4) || !as_int(args[18], &k_split)) Py_RETURN_NONE;
+    if (!as_tensor(args[2], &act) || !act->is_cuda() || act->dim() != 2 || act->scalar_type() != at::kByte || !act->is_contiguous() || !native_tensor(args[3], s_qweight, *act, &wgt) ||
+        !native_tensor(args[5], s_wscales, *act, &wsc)) Py_RETURN_NONE;
+    {
+        PyObject *shape = attribute(args[3], s_logical_shape);
+        const bool ok = shape && PyTuple_Check(shape) && PyTuple_GET_SIZE(shape) == 2 && as_int(PyTuple_GET_ITEM(shape, 0), &N) && as_int(PyTuple_GET_ITEM(shape, 1), &K);
+        Py_XDECREF(shape);
+        if (!ok) Py_RETURN_NONE;
+    }
+    const int64_t M_pad = act->size(0), G = fp4 ? 16 : 64;
+    // (the native scales of the two precisions differ in type: those of the other one are not the plain case)
+    if (M_pad <= 0 || M_pad % 256 || K <= 0 || K % 128 || N <= 0 || N % 128 || act->size(1) != (fp4 ? K / 2 : K * 3 / 4) ||
+        !checked(args[4], *act, fp4 ? at::kFloat8_e4m3fn : at::kBFloat16, {K / G, M_pad}, &asc) || wsc->scalar_type() != (fp4 ? at::kHalf : at::kLong) ||
+        wsc->numel() != (fp4 ? K / 16 * N : (N + 255) / 256 * (K / 64) * 256) || wgt->numel() != (fp4 ? N * (K / 2) : (N + 255) / 256 * 256 * (K * 3 / 4))) Py_RETURN_NONE;
+    if (fp4) {
+        // (the tensor is an attribute of the scales, which the caller holds)
+        PyObject *c = attribute(args[5], s_colnorm);
+        const bool ok = c && as_tensor(c, &colnorm) && colnorm->device() == act->device() && colnorm->numel() == N && colnorm->scalar_type() == at::kFloat;
+        Py_XDECREF(c);
+        if (!ok) Py_RETURN_NONE;
+    }
+    if (args[11] != Py_None && (!native_tensor(args[11], s_vector, *act, &bias) || bias->scalar_type() != at::kBFloat16 || !shape_is(*bias, {N}))) Py_RETURN_NONE;
+    if (args[12] != Py_None && (!native_tensor(args[12], s_vector, *act, &wcs) || wcs->scalar_type() != at::kBFloat16 || !shape_is(*wcs, {N}))) Py_RETURN_NONE;
+    int64_t R = 0;
+    if ((args[9] == Py_None) != (args[10] == Py_None)) Py_RETURN_NONE;
+    if (args[10] != Py_None) {
+        if (!native_tensor(args[10], s_lora_up, *act, &up) || up->dim() != 2 || up->scalar_type() != at::kBFloat16 || up->size(0) != N || up->size(1) <= 0 ||
+            up->size(1) > 16 * MAX_GROUPS) Py_RETURN_NONE;
+        R = up->size(1);
+        if (!checked(args[9], *act, at::kFloat, {M_pad, R}, &la)) Py_RETURN_NONE;
+        if (fp4 && wcs) {  // (the wrapper's check for zeros, once per tensor, has been made)
+            PyObject *z = attribute(args[12], s_nonzero);
+            const bool ok = z == Py_True;
+            Py_XDECREF(z);
+            if (!ok) Py_RETURN_NONE;
+        }
+    }
+    const int groups = (int)((R + 15) / 16);
+    for (int i = 0; i < groups; i++) sc[i] = args[13] == Py_None ? 1.f : 0.f;
+    if (args[13] != Py_None) {
+        if (!PyList_Check(args[13])) Py_RETURN_NONE;
+        for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[13]) && i < groups; i++) {
+            PyObject *v = PyList_GET_ITEM(args[13], i);
+            if (!PyFloat_CheckExact(v)) Py_RETURN_NONE;
+            sc[i] = (float)PyFloat_AS_DOUBLE(v);
+        }
+    }
+    if (!PyFloat_CheckExact(args[14])) Py_RETURN_NONE;
+    int64_t vk_rows = 0;
+    if (args[7] != Py_None) {
+        if (args[6] != Py_None || silu || N % 384 || !as_tensor(args[8], &out) || out->dim() != 3) Py_RETURN_NONE;
+        const int64_t B = out->size(0);
+        vk_rows = out->size(1);
+        if (!checked(args[8], *act, at::kBFloat16, {B, vk_rows, N / 3}, &out) || !checked(args[7], *act, at::kFloat, {B, N / 96, 33, 32}, &vk) || vk_rows <= 0 || vk_rows % 256 ||
+            B * vk_rows != M_pad) Py_RETURN_NONE;
+    } else if (args[8] != Py_None || !as_tensor(args[6], &out) || out->device() != act->device() || out->scalar_type() != at::kBFloat16 || !out->is_contiguous() || out->dim() < 1 ||
+               out->numel() == 0) {
+        Py_RETURN_NONE;
+    }
+    *g = svdq_gemm_args{};
+    g->act = act->data_ptr();
+    g->ascales = asc->data_ptr();
+    g->wgt = wgt->data_ptr();
+    g->wscales = wsc->data_ptr();
+    g->colnorm = colnorm ? (const float *)colnorm->data_ptr() : nullptr;
+    g->bias = bias ? bias->data_ptr() : nullptr;
+    g->wcscales = wcs ? wcs->data_ptr() : nullptr;
+    g->lora_act_in = la ? (const float *)la->data_ptr() : nullptr;
+    g->lora_up = up ? up->data_ptr() : nullptr;
+    g->lora_scales = sc;
+    g->out = out->data_ptr();
+    g->M_pad = M_pad;
+    g->N = N;
+    g->K = K;
+    g->N_out = out->size(-1);
+    g->M_out = out->numel() / g->N_out;
+    g->R_up = R;
+    g->alpha = (float)PyFloat_AS_DOUBLE(args[14]);
+    g->act_unsigned = unsigned_codes;
+    g->fuse_silu = silu;
+    g->fp4 = fp4;
+    g->k_split = (int)k_split;
+    g->out_vk = vk ? (float *)vk->data_ptr() : nullptr;
+    g->vk_rows = vk_rows;
+    Py_RETURN_TRUE;
+    END_HANDLE_TH_ERRORS
+}
+
+// vk_mul_q(q, vk, num_tokens, eps): linearattn_vk_mul_q on the current stream -> True, or None
+PyObject *vk_mul_q(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    SVDQ_NARGS(4)
+    const at::Tensor *q, *vk;
+    int64_t tokens;
+    if (!as_tensor(args[0], &q) || !q->is_cuda() || q->dim() != 3 || q->scalar_type() != at::kBFloat16 || !q->is_contiguous() || q->device().index() != c10::hip::current_device() ||
+        !as_tensor(args[1], &vk) || vk->dim() != 4 || !PyFloat_CheckExact(args[3])) Py_RETURN_NONE;
+    const int64_t B = q->size(0), tokens_pad = q->size(1), heads = vk->size(1);
+    if (!checked(args[1], *q, at::kFloat, {B, heads, 33, 32}, &vk) || q->size(2) != heads * 32) Py_RETURN_NONE;
+    if (args[2] == Py_None) tokens = tokens_pad;
+    else if (!PyLong_CheckExact(args[2]) || !as_int(args[2], &tokens)) Py_RETURN_NONE;
+    hipStream_t st = c10::hip::getCurrentHIPStream(q->device().index()).stream();
+    int rc;
+    const float eps = (float)PyFloat_AS_DOUBLE(args[3]);
+    Py_BEGIN_ALLOW_THREADS
+    rc = svdq_linearattn_vk_mul_q(q->data_ptr(), (const float *)vk->data_ptr(), B, tokens, tokens_pad, heads, eps, st);
+    Py_END_ALLOW_THREADS
+    if (rc != SVDQ_OK) return raise(rc);
+    Py_RETURN_TRUE;
+    END_HANDLE_TH_ERRORS
+}
+
 #define SVDQ_METHOD(f) {#f, (PyCFunction)(void (*)(void))f, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {SVDQ_METHOD(make_layer), SVDQ_METHOD(linear), SVDQ_METHOD(gelu_mlp), SVDQ_METHOD(qkv_norm_rope), SVDQ_METHOD(awq_gemv), SVDQ_METHOD(awq_linear),
+                         SVDQ_METHOD(quantize_call), SVDQ_METHOD(gemm_call), SVDQ_METHOD(vk_mul_q),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_host", "Per-call host code of the quantized layers.", -1, methods, nullptr, nullptr, nullptr, nullptr};
 
@@ -469,5 +658,13 @@ PyMODINIT_FUNC PyInit__host(void) {
     s_in_features = PyUnicode_InternFromString("in_features");
     s_out_features = PyUnicode_InternFromString("out_features");
     s_group_size = PyUnicode_InternFromString("group_size");
+    s_native = PyUnicode_InternFromString("_svdq_native");
+    s_logical_shape = PyUnicode_InternFromString("logical_shape");
+    s_colnorm = PyUnicode_InternFromString("colnorm");
+    s_nonzero = PyUnicode_InternFromString("_svdq_nonzero");
+    s_lora_up = PyUnicode_InternFromString("lora_up");
+    s_lora_down = PyUnicode_InternFromString("lora_down");
+    s_vector = PyUnicode_InternFromString("vector");
+    s_smooth_rcp = PyUnicode_InternFromString("smooth_rcp");
     return PyModule_Create(&module_def);
 }

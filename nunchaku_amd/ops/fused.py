@@ -99,6 +99,8 @@ def linearattn_vk_mul_q(q: torch.Tensor, vk: torch.Tensor, num_tokens: int | Non
     in place (kernels::linearattn_vk_mul_q, gemm_w4a4_launch_impl.cuh:427-448).  q bf16 [B, tokens_pad, heads * 32]
     (``out_linearattn`` of ``svdq_gemm_w4a4``), vk fp32 [B, heads, 33, 32] (its ``out_vk``); only the first
     ``num_tokens`` rows of every batch entry are touched (all by default, as in the reference)."""
+    if getattr(q, "is_cuda", False) and nv.host().vk_mul_q(q, vk, num_tokens, eps):  # (the plain case, with the same checks)
+        return q
     nv.require_gpu(q, "q")
     nv.require_gpu(vk, "vk")
     if q.dim() != 3 or vk.dim() != 4 or q.dtype != torch.bfloat16 or vk.dtype != torch.float32:

@@ -87,6 +87,16 @@ def svdq_gemm_w4a4(
     out_vk[b, h, i, j] = sum over tokens of v[i] * relu(k[j]) (i < 32) and of relu(k[j]) (i = 32), where the
     columns after q hold, per head, 32 of k then 32 of v.  out_vk is cleared first.
     """
+    if (getattr(act, "is_cuda", False) and qout is None and rotary_emb is None and out_q is None and out_k is None and out_v is None and norm_q is None
+            and norm_k is None and lora_down is None and lora_act_out is None and poolout is None):
+        # the plain and the linear-attention form with converted tensors: checked and filled in by the host extension
+        call = nv.GemmCall()
+        at = ctypes.addressof(call)
+        if nv.host().gemm_call(at, at + nv.GemmCall.scales.offset, act, wgt, ascales, wscales, out, out_vk, out_linearattn, lora_act_in, lora_up, bias, wcscales,
+                               lora_scales, alpha, act_unsigned, fuse_silu, fp4, K_SPLIT or 0):
+            nv.launch(nv.lib().svdq_gemm_w4a4_noalloc if NO_ALLOC else nv.lib().svdq_gemm_w4a4, ctypes.byref(call), act.device)
+            return
+    # (any other call: converted and checked here)
     local = locals()
     for name in _NOT_BUILT:
         if local[name] is not None:

@@ -35,6 +35,13 @@ def svdq_quantize_w4a4_act_fuse_lora(
     [M_pad, K/2], also in a private order); NVFP4 keeps [M_pad, K/2].  ``packing.act_to_logical`` gives
     one code per element.
     """
+    if getattr(input, "is_cuda", False) and output is None and oscales is None and lora_act_out is None and not fuse_glu:
+        # the plain form with converted tensors: checked, allocated and filled in by the host extension
+        call = nv.QuantizeArgs()
+        made = nv.host().quantize_call(ctypes.addressof(call), input, lora_down, smooth, fp4, pad_size)
+        if made is not None:
+            nv.launch(nv.lib().svdq_quantize_w4a4_act_fuse_lora, ctypes.byref(call), input.device)
+            return made
     if input.dim() != 2:
         raise ValueError("input must be [M, K]")
     nv.require_gpu(input, "input")

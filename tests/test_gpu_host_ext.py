@@ -127,3 +127,106 @@ def test_a_true_NO_ALLOC_of_any_type(dev, monkeypatch):
             fused_gelu_mlp(x, m1, m2)
         with pytest.raises(NotImplementedError, match="fixed scratch"):
             fused_qkv_norm_rottary(x, m3, norm, norm, rot)
+
+
+@pytest.mark.parametrize("R,fp4", [(0, False), (48, False), (48, True)])
+def test_operators_fast_and_checked_path(dev, R, fp4, monkeypatch):
+    """Each operator hands the library the same argument block, and refuses the same calls with the same words, whether the
+    extension fills the block in or the Python code does."""
+    from nunchaku_amd import _native as nv
+    from nunchaku_amd import packing
+    from nunchaku_amd.ops import gemm as gemm_mod
+    from nunchaku_amd.ops import linearattn_vk_mul_q, svdq_gemm_w4a4, svdq_quantize_w4a4_act_fuse_lora
+
+    announce(f"host extension: operators R={R} fp4={fp4}")
+    M, K, N = 300, 256, 384
+    t = make_module(synth.make_layer(N, K, R, seed=M, fp4=fp4), dev).native_tensors()
+    x = synth.make_activations(M, K, seed=M).to(dev)
+    act, asc, la = svdq_quantize_w4a4_act_fuse_lora(x, lora_down=t["proj_down"], smooth=t["smooth_factor"], fp4=fp4)
+    host, real_launch = nv.host(), nv.launch
+    taken, blocks = [], []
+
+    class Host:
+        def __init__(self, declines):
+            self.declines = declines
+
+        def __getattr__(self, name):
+            def call(*args):
+                r = None if self.declines else getattr(host, name)(*args)
+                taken.append(r is not None)
+                return r
+
+            return call
+
+    def launch(entry, ref, device):  # (no kernel: what it would be given.  Where a result lies that the call itself allocates is the allocator's choice)
+        a = ref._obj
+        own = ("output", "oscales", "lora_act_out") if isinstance(a, nv.QuantizeArgs) else ("lora_scales", "qkv_head_stride", "norm_eps")  # (read with a rotary table only)
+        fields = (nv.QuantizeArgs if isinstance(a, nv.QuantizeArgs) else nv.GemmArgs)._fields_
+        block = {n: getattr(a, n) for n, _ in fields if n not in own}
+        if isinstance(a, nv.GemmArgs):
+            block["lora_scales"] = [a.lora_scales[i] for i in range((a.R_up + 15) // 16)]
+        blocks.append((entry is nv.lib().svdq_gemm_w4a4_noalloc, block))
+
+    monkeypatch.setattr(nv, "launch", launch)
+
+    def run(declines, f, kw):
+        monkeypatch.setattr(nv, "_host_module", Host(declines))
+        blocks.clear(), taken.clear()
+        try:
+            r = f(**kw)
+            shapes = [(tuple(o.shape), o.dtype, o.is_contiguous()) for o in r] if isinstance(r, tuple) else None
+            return shapes, list(blocks), list(taken)
+        except Exception as e:
+            return (type(e), str(e)), None, list(taken)
+
+    def same(f, plain, **kw):
+        fast, checked = run(False, f, kw), run(True, f, kw)
+        assert fast[:2] == checked[:2] and fast[2] == [plain], (f.__name__, {k: v for k, v in kw.items() if not isinstance(v, torch.Tensor)}, fast, checked)
+
+    quant = lambda plain, **kw: same(svdq_quantize_w4a4_act_fuse_lora, plain, **{**dict(input=x, lora_down=t["proj_down"], smooth=t["smooth_factor"], fp4=fp4), **kw})
+    quant(True)
+    quant(True, smooth=None, pad_size=512, input=x[:1])
+    for kw in (dict(pad_size=128), dict(input=x.half()), dict(input=x[0]), dict(input=x[:, :128]), dict(input=x.T.contiguous().T), dict(smooth=t["smooth_factor"][:128]), dict(lora_down=None), dict(input=x[:0]), dict(input=x.cpu())):
+        fast, checked = (run(d, svdq_quantize_w4a4_act_fuse_lora, {**dict(input=x, lora_down=t["proj_down"], smooth=t["smooth_factor"], fp4=fp4), **kw}) for d in (False, True))
+        assert fast[:2] == checked[:2] and not any(fast[2]), (kw.keys(), fast, checked)
+
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+    q, vk = torch.empty(2, 256, N // 3, dtype=torch.bfloat16, device=dev), torch.empty(2, N // 96, 33, 32, device=dev)
+    base = dict(act=act, wgt=t["qweight"], out=out, ascales=asc, wscales=t["wscales"], lora_act_in=la, lora_up=t["proj_up"], bias=t["bias"], wcscales=t["wcscales"], fp4=fp4)
+    lowrank = R > 0  # (an empty low-rank branch is not the plain case)
+    gemm = lambda plain, **kw: same(svdq_gemm_w4a4, plain, **{**base, **kw})
+    gemm(lowrank)
+    gemm(True, lora_act_in=None, lora_up=None, bias=None, alpha=0.25)
+    gemm(lowrank, act_unsigned=True, fuse_silu=True, out=out[:, :100].contiguous())
+    gemm(lowrank, lora_scales=[0.5, 2.0], out=out.view(1, M, N))
+    gemm(lowrank, lora_scales=[0.5] * 9)
+    gemm(False, lora_scales=(0.5, 1, 2))
+    gemm(False, alpha=torch.tensor(0.5))
+    gemm(lowrank, out=None, out_vk=vk, out_linearattn=q)
+    for split, no_alloc in ((3, False), (None, 1)):
+        monkeypatch.setattr(gemm_mod, "K_SPLIT", split), monkeypatch.setattr(gemm_mod, "NO_ALLOC", no_alloc)
+        gemm(lowrank)
+    for kw in (dict(act=None), dict(wgt=None), dict(act=act[:, :-16].contiguous()), dict(act=act[:128]), dict(ascales=asc[:-1]), dict(ascales=asc.view(torch.uint8)), dict(out=None),
+               dict(lora_up=None), dict(lora_act_in=la[:256]), dict(bias=t["bias"][:-1]), dict(out=out.half()), dict(out=out.T), dict(out=out.cpu()), dict(act=act.cpu()),
+               dict(out_vk=vk), dict(out=None, out_vk=vk, out_linearattn=q, fuse_silu=True), dict(out=None, out_vk=vk[:1], out_linearattn=q), dict(out=None, out_vk=vk.half(), out_linearattn=q),
+               dict(out=None, out_vk=vk, out_linearattn=q[:1]), dict(poolout=out), dict(norm_q=t["bias"]), dict(lora_down=t["proj_down"])):
+        fast, checked = run(False, svdq_gemm_w4a4, {**base, **kw}), run(True, svdq_gemm_w4a4, {**base, **kw})
+        assert fast[:2] == checked[:2] and (isinstance(fast[0], tuple) or not lowrank) and not any(fast[2]), (kw.keys(), fast, checked)
+
+    monkeypatch.setattr(nv, "launch", real_launch)
+    vk.uniform_(0.5, 1.0)
+    x3 = torch.rand(2, 256, N // 3, device=dev).bfloat16()
+    for tokens in (None, 77):
+        got = []
+        for declines in (False, True):
+            monkeypatch.setattr(nv, "_host_module", Host(declines))
+            got.append(linearattn_vk_mul_q(x3.clone(), vk, tokens))
+        assert torch.equal(*got)
+    for args in ((x3, vk, 257), (x3, vk, 0), (x3[:1], vk), (x3.half(), vk), (x3, vk.cpu()), (x3.transpose(0, 1), vk), (x3.cpu(), vk)):
+        seen = []
+        for declines in (False, True):
+            monkeypatch.setattr(nv, "_host_module", Host(declines))
+            with pytest.raises((ValueError, RuntimeError)) as e:
+                linearattn_vk_mul_q(*args)
+            seen.append((type(e.value), str(e.value)))
+        assert seen[0] == seen[1], seen
