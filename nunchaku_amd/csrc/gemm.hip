@@ -441,7 +441,7 @@ void fill_params(const svdq_gemm_args *a, GemmParams &p) {
     p.partials = nullptr;
     p.counters = nullptr;
     p.whole_band = 0;
-    p.row_blocks = 0;
+    p.row_blocks = p.full_blocks = 0;
     p.lr_steps = 0;
 }
 
@@ -685,6 +685,43 @@ bool staged_rows(const svdq_gemm_args *a, int ncu, bool split) {
     return 2 * tiles >= (needs_next_epilogue(a) ? 2 * ncu + 2 : 3 * ncu) && tiles <= (a->qout && split ? 3 : 2) * ncu;
 }
 
+// NVFP4 launches of 64 x 128 tiles: how many blocks of 64 rows, what they leave of the rows in blocks of 32 behind them (nothing, where the last block is
+// partly padding), and the time of the busiest compute unit in tiles of 64 rows.  With tiles of one height the last ones keep a few compute units busy for
+// the time of a whole tile, also where most of its rows are padding; the hardware hands tiles to the emptiest compute unit, and two of them on one share
+// its matrix core, so that its time is the sum of theirs.  A tile of 32 rows takes 0.68 of one of 64 (0.66 at long rows, 0.7 at K = 1024: the columns'
+// operands are converted for half as many products).  Considered are whole blocks only, the last 32 rows by themselves, and 64-row tiles up to the last and
+// the last but one multiple of the compute units; 1.5 % have to be gained, equal ones go to the fewest 64-row tiles.  The GEMM alone, one height / two, us, rank 32, K = 3072: norm and
+// rotary, N = 9216, M = 300 21.0 / 19.2, M = 505 33.1 / 29.9, M = 700 43.5 / 40.1, M = 1200 66.3 / 63.8; quantizing, N = 12288, M = 400 40.2 / 37.0, M = 1157 97.2 / 91.9; plain, N = 3072,
+// M = 2300 41.0 / 39.4.  4.5 % faster over 4600 launches of 16 ... 9216 rows (with the epilogue's requests ahead of the main loop, which came before), 6 of them slower by more than 3 %.  (Slower:
+// 32-row tiles where the model sees no gain, up to 9 % where all rows are in them; INT4, whose launches of several tiles per compute unit share the rows or are large tiles.)
+struct Heights {
+    int full;
+    double time;
+};
+Heights few_rows_heights(int rows, int column_blocks, int ncu) {
+    constexpr double HALF = 0.68;
+    const int units = (rows + 31) / 32, all = (units + 1) / 2;
+    auto time = [&](int full) {
+        const long long whole = (long long)full * column_blocks, half = (long long)(units - 2 * full) * column_blocks;
+        const long long q = whole / ncu, more = whole % ncu, fewer = ncu - more;  // compute units with q + 1 whole tiles, with q
+        for (int h0 = 0, h1 = 0;;) {  // half tiles on each unit of either kind
+            const double t0 = (double)q + HALF * h0, t1 = (double)(q + 1) + HALF * h1, t = more && t1 > t0 ? t1 : t0;
+            if (h0 * fewer + h1 * more >= half) return t;
+            if (!more || t0 + HALF <= t1 + HALF) h0++;
+            else h1++;
+        }
+    };
+    Heights best{all, (double)(((long long)all * column_blocks + ncu - 1) / ncu)};
+    const double limit = 0.985 * best.time;
+    const int q = (int)((long long)(units / 2) * column_blocks / ncu);
+    for (int full : {units / 2, (int)((long long)q * ncu / column_blocks), (int)((long long)(q - 1) * ncu / column_blocks)}) {
+        if (full < 0 || full > units / 2 || 2 * full == units) continue;
+        const double t = time(full);
+        if (t <= limit && t <= best.time) best = Heights{full, t};
+    }
+    return best;
+}
+
 // Which tiles of the few-rows kernel a launch takes, if any.  Shape 1: tiles of 32 rows x 128 columns, four waves split
 // K.  Shape 2: tiles of 64 rows x 128 columns, a quarter fewer operand bytes per product, from about 400 tiles of 32 rows on; INT4: two waves
 // split K and two the columns, NVFP4: four waves split K.  Models of the time in us fitted to launches at K = 1024 ... 12288
@@ -810,6 +847,7 @@ void make_plan(const svdq_gemm_args *a, int ncu, svdq_gemm_plan *plan) {
         plan->columns = 32 * t.nc;
         plan->shared_rows = t.shared_rows;
         plan->row_blocks = (rows_needed(a) + 32 * t.mt - 1) / (32 * t.mt);
+        if (a->fp4 && t.mt == 2 && t.nc == 4) plan->full_blocks = few_rows_heights(rows_needed(a), (int)(a->N / 128), ncu).full;
     } else if (a->fp4) {
         plan_fp4(a, ncu, plan);
     } else {
@@ -820,9 +858,14 @@ void make_plan(const svdq_gemm_args *a, int ncu, svdq_gemm_plan *plan) {
 int gemm_direct(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t st, int dev, bool noalloc) {
     GemmParams p;
     fill_params(a, p);
-    p.row_blocks = plan.row_blocks;
     const bool next = needs_next_epilogue(a), fp4 = a->fp4 != 0;
     const int mt = plan.few_rows;
+    p.row_blocks = plan.row_blocks;
+    if (fp4 && mt == 2 && plan.columns == 128) {
+        p.full_blocks = plan.full_blocks;
+        const int units = (rows_needed(a) + 31) / 32;
+        p.row_blocks = 2 * plan.full_blocks > units ? plan.full_blocks : units - plan.full_blocks;
+    }
     auto launch = [&]() {
         if (plan.columns < 128) return plan.columns == 32 * mt ? direct::launch_square(p, fp4, mt, st) : direct::launch_oblong(p, fp4, mt, st);
         if (plan.shared_rows) return next ? direct::launch_staged_next(p, st) : direct::launch_staged_plain(p, st);

@@ -80,8 +80,12 @@ struct Lds {
     static_assert(bytes(LR_AHEAD) <= 80 * 1024 && (!STAGED || 3 * bytes(4) <= 160 * 1024));
 };
 
+// NVFP4 launches of 64 x 128 tiles have tiles of half the height behind them (few_rows_heights in gemm.hip).
+constexpr bool two_heights(bool fp4, int MT, int NC) { return fp4 && MT == 2 && NC == 4; }
+
+// One tile: MT blocks of 32 rows from block f0 on, column block nb.
 template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT>
-__global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_kernel(GemmParams p) {
+__device__ __forceinline__ void output_tile(const GemmParams &p, const int nb, const int f0) {
     constexpr int NC = NT * WN;  // 32-column tiles of the workgroup; a wave has NT of them
     constexpr int WAVES = WN * KP;
     constexpr bool NARROW = NC < 4;
@@ -96,13 +100,7 @@ __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_ker
     const int r32 = lane & 31, h = lane >> 5;
     const int kgroups = p.K / 64;
     const int kpart = wave / WN, cw = wave % WN;
-
-    // Workgroups go to the XCDs round robin (blockIdx % 8): each XCD gets one contiguous run of numbers, down the rows
-    // first, so that the row blocks of a weight column meet in one L2 and every XCD streams its own share of the weights.
-    const int total = (int)gridDim.x, xcd = (int)blockIdx.x % 8, extra = total % 8;
-    const int v = xcd * (total / 8) + (xcd < extra ? xcd : extra) + (int)blockIdx.x / 8;
-    const int nb = v / p.row_blocks, mb = v - nb * p.row_blocks;
-    const int n0 = nb * (32 * NC), f0 = mb * MT;  // first column; first 32-row block
+    const int n0 = nb * (32 * NC);  // first column
 
     // ---- operands ----------------------------------------------------------------------------------
     // (DEPTH + 1 register sets, indexed by compile-time constants.  The lambdas below reach them through their captures: taken
@@ -772,6 +770,31 @@ __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_ker
             *(u32x4_t *)(p.qout + ((size_t)(m / 32) * ngroups_out + gidx) * TILE_BYTES + (m % 32) * 32 + 16 * (qc & 1)) = words;
         }
     }
+    }
+}
+
+// Tile number `block` of `total`: workgroups go to the XCDs round robin (number % 8), and each XCD gets one contiguous run of tiles, down the rows
+// first, so that the row blocks of a weight column meet in one L2 and every XCD streams its own share of the weights.
+__device__ inline int tile_of(int block, int total) {
+    const int xcd = block % 8, extra = total % 8;
+    return xcd * (total / 8) + (xcd < extra ? xcd : extra) + block / 8;
+}
+
+template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT>
+__global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_kernel(GemmParams p) {
+    if constexpr (two_heights(FP4, MT, NT * WN)) {
+        const int full = p.full_blocks * (p.N / (32 * NT * WN)), block = (int)blockIdx.x;
+        if (block < full) {
+            const int v = tile_of(block, full), nb = v / p.full_blocks;
+            output_tile<FP4, 2, NT, WN, KP, DEPTH, NEXT>(p, nb, (v - nb * p.full_blocks) * 2);
+        } else {
+            // (as deep a ring as the launches of 32-row tiles alone have)
+            const int half_blocks = p.row_blocks - p.full_blocks, v = tile_of(block - full, (int)gridDim.x - full), nb = v / half_blocks;
+            output_tile<FP4, 1, NT, WN, KP, 2, NEXT>(p, nb, p.full_blocks * 2 + v - nb * half_blocks);
+        }
+    } else {
+        const int v = tile_of((int)blockIdx.x, (int)gridDim.x), nb = v / p.row_blocks;
+        output_tile<FP4, MT, NT, WN, KP, DEPTH, NEXT>(p, nb, (v - nb * p.row_blocks) * MT);
     }
 }
 

@@ -197,7 +197,7 @@ struct GemmParams {
     float *vk, *vk_part;
     int vk_rows;
     int whole_band;              // 0, or (whole tiles only) the band height of the tile numbering in row blocks
-    int row_blocks;              // few-rows kernels: tiles along M,
+    int row_blocks, full_blocks; // few-rows kernels: tiles along M; NVFP4, 64 x 128 tiles: the first so many of 64 rows, the rest of 32
     int lr_steps;                // 16-rank steps of the low-rank operands that are copied to LDS ahead of the main loop
     float *next_lora_part;  // [N/128 column chunks][M_pad/32 slabs][R_down/16][2][64 lanes] x float4
 };

@@ -16,7 +16,7 @@ int svdq_gemm_w4a4_rows(const svdq_gemm_args *args, int64_t rows, int noalloc, v
 typedef struct svdq_gemm_plan {
     int32_t few_rows;      // 0: a kernel with large tiles; 1, 2: the few-rows kernel in tiles of 32, 64 rows,
     int32_t row_blocks;    // so many along M
-    int32_t full_blocks;   // INT4, large tiles: row blocks of 128 rows,
+    int32_t full_blocks;   // INT4, large tiles: row blocks of 128 rows (NVFP4, few rows, 64 x 128: of 64 rows, in blocks of 32 what they leave),
     int32_t half_blocks;   // of 64 rows behind them,
     int32_t kparts;        // and parts along K of every tile
     int32_t workgroups;    // NVFP4, large tiles: persistent workgroups;

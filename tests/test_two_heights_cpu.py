@@ -1,0 +1,69 @@
+"""How NVFP4 few-rows launches of 64 x 128 tiles divide their rows into blocks of 64 and 32 rows (csrc/gemm.hip, ``few_rows_heights``) and number the tiles
+(csrc/gemm_direct_kernel.h, ``gemm_direct_kernel``)."""
+
+import random
+
+import pytest
+
+from plan_util import call, plan_of
+
+
+def tile_of(block: int, total: int) -> int:  # (as in the kernel)
+    xcd, extra = block % 8, total % 8
+    return xcd * (total // 8) + min(xcd, extra) + block // 8
+
+
+def tiles(full: int, half: int, columns: int):
+    """(first row, rows, column block) of every workgroup, as the kernel works them out."""
+    whole, total = full * columns, (full + half) * columns
+    for block in range(total):
+        if block < whole:
+            nb, mb = divmod(tile_of(block, whole), full)
+            yield mb * 64, 64, nb
+        else:
+            nb, mb = divmod(tile_of(block - whole, total - whole), half)
+            yield full * 64 + mb * 32, 32, nb
+
+
+@pytest.mark.parametrize("full,half,columns", [(1, 1, 1), (3, 4, 72), (16, 5, 96), (5, 1, 7), (2, 0, 9)])
+def test_every_tile_once(full, half, columns):
+    got = sorted(tiles(full, half, columns))
+    want = [(64 * i, 64, n) for i in range(full) for n in range(columns)] + [(64 * full + 32 * i, 32, n) for i in range(half) for n in range(columns)]
+    assert got == want
+
+
+def test_rows_are_covered_inside_the_padded_tensor():
+    """Against the busiest compute unit's tiles, counted one by one: never more than with 64-row tiles alone."""
+    rng, mixed = random.Random(1), 0
+    for _ in range(4000):
+        kind, M, K, N = rng.choice(["plain", "silu", "rope", "litela"]), rng.randint(1, 3000), 128 * rng.randint(1, 30), 384 * rng.randint(1, 40)
+        if kind == "litela":
+            M = (M + 255) // 256 * 256
+        ncu = rng.choice([256, 256, 304, 64])
+        p = plan_of(call(kind, M, K, N, 32, True), compute_units=ncu)
+        if (p.few_rows, p.columns) != (2, 128):
+            assert p.full_blocks == 0
+            continue
+        units, nb = (M + 31) // 32, N // 128
+        half = max(units - 2 * p.full_blocks, 0)
+        assert p.row_blocks == (M + 63) // 64 and 0 <= p.full_blocks <= p.row_blocks and M <= 64 * p.full_blocks + 32 * half <= (M + 255) // 256 * 256
+        load = [0.0] * ncu
+        for cost, n in ((1.0, p.full_blocks * nb), (0.68, half * nb)):
+            for _ in range(n):  # the emptiest one takes the next tile
+                i = min(range(ncu), key=load.__getitem__) if half else 0
+                load[i] += cost if half else 0.0
+        if half:
+            mixed += 1
+            assert max(load) <= 0.985 * -(-p.row_blocks * nb // ncu) + 1e-9
+    assert mixed > 100
+
+
+@pytest.mark.parametrize("kind,M,K,N,want", [
+    ("rope", 505, 3072, 9216, 7), ("rope", 300, 3072, 9216, 3), ("silu", 201, 2688, 15744, 4), ("plain", 2300, 3072, 3072, 32), ("rope", 1200, 3072, 9216, 17),
+    ("split", 17, 3968, 11904, 4),
+])
+def test_blocks_of_64_rows(kind, M, K, N, want):
+    p = plan_of(call(kind, M, K, N, 32, True))
+    assert (p.few_rows, p.columns, p.full_blocks) == (2, 128, want), p
+    assert plan_of(call(kind, M, K, N, 32, False)).few_rows * plan_of(call(kind, M, K, N, 32, False)).full_blocks == 0
+    assert plan_of(call("next", 1157, 3072, 12288, 32, True, with_out=False), rows=1157).full_blocks == 16
