@@ -632,59 +632,6 @@ struct FewRowsTile {
     bool shared_rows;
     double time;
 };
-// The tile of a few-rows launch with the plain epilogue, in blocks of 32 x 32 (`shape`: the better one of 128 columns by the models of
-// choose_direct, of 32 rows (1) or 64 (2)).  What takes the time is the fetching of the operands: a
-// compute unit gets 120 GB/s in requests of 16 bytes a lane, 80 in those of 8, however few of them fetch and however many waves do (48
-// or 192 workgroups, 4 ... 16 waves each), and a tile of mt x nc blocks fetches mt + nc fragments per k-group.  Square tiles fetch least per
-// product, small ones bring more compute units to bear: the sums cost a tile nothing before the end.  A model of the time in us, linear in the
-// tiles of the busiest compute unit and in the k-groups, fitted to 844 shapes (M = 16 ... 1000, K = 1024 ... 13824, N = 1024 ... 21504)
-// times the six tiles: its choice is 0.1 % (INT4) and 0.05 % (NVFP4) off the fastest on average and 5.4 % at most; tiles of 128 columns only,
-// 18 and 21 %.  Measured, layer calls, 128 columns / the choice, us:
-//   INT4   M = 64, K = N = 3072  13.3 / 10.2 (32 x 32)    NVFP4  14.6 / 10.3
-//          M = 256               14.1 / 13.1 (64 x 64)           15.3 / 14.1
-//          M = 64, K = 12288     32.3 / 21.4 (32 x 32)           34.6 / 21.6
-//          M = 256, K = 12288    34.7 / 30.3 (64 x 64)           37.4 / 34.0
-// Few columns, and INT4 with short rows (fewer than 1024), where 64-row tiles are the better ones of 128 columns: compute units have several tiles, and the
-// model, which does not know the fixed part of a tile well, favours narrow ones too much.  There they are taken if it says 8 %, and in INT4 not
-// with K = 128: M = 125, K = 128, N = 11392, rank 16 5.1 us with 64 x 128, 32 x 32 6.3; NVFP4 M = 5041, K = 8448, N = 512 48.2, 64 x 64 55.8.  Over 325 INT4 and 357 NVFP4
-// shapes with few columns, short rows or more than 9216 rows 0.9 and 0.6 % off the fastest tile, without this 1.1 and 0.6; 1111 and 1370 others 0.2 and 0.3 % (M = 1 ...
-// 20000, K = 128 ... 16640, N = 128 ... 21504, ranks 0 ... 160).
-FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu, int shape) {
-    struct Model {
-        int mt, nc;
-        double launch, tile, kgroup;
-    };
-    constexpr Model int4[] = {{1, 1, -0.18, 0.18, 0.0382}, {1, 2, -0.46, 0.68, 0.0551}, {2, 1, -0.46, 0.75, 0.0499},
-                              {2, 2, 0.18, 0.64, 0.0702},  {1, 4, -0.13, 0.64, 0.0948}, {2, 4, 1.04, 0.53, 0.1378}};
-    constexpr Model nvfp4[] = {{1, 1, -0.85, 0.16, 0.0323}, {1, 2, -0.52, 0.14, 0.0515}, {2, 1, -0.64, 0.24, 0.0498},
-                               {2, 2, -0.17, 0.46, 0.0719}, {1, 4, 0.22, 0.47, 0.0876},  {2, 4, 1.96, -0.07, 0.1112}};
-    const long long row_blocks = (rows_needed(a) + 31) / 32, column_blocks = a->N / 32;
-    const bool favour_wide = shape == 2 && (a->N < 1024 || (!a->fp4 && a->K < 1024));
-    FewRowsTile best{};
-    for (const Model &m : a->fp4 ? nvfp4 : int4) {
-        const bool wide = m.mt == 2 && m.nc == 4;
-        if (favour_wide && !a->fp4 && a->K < 256 && !wide) continue;
-        const long long tiles = (row_blocks + m.mt - 1) / m.mt * (column_blocks / m.nc);
-        const double t = (m.launch + (double)((tiles + ncu - 1) / ncu) * (m.tile + m.kgroup * (double)(a->K / 64))) * (favour_wide && wide ? 0.92 : 1.0);
-        if (best.mt == 0 || t < best.time) best = FewRowsTile{m.mt, m.nc, false, t};
-    }
-    return best;
-}
-
-// INT4 launches with more than one tile of 64 x 128 per compute unit and up to two (plain epilogue: from one and a half on): such tiles, where they are
-// chosen (choose_direct), have waves that split the columns and share the rows' operands through LDS (gemm_direct_kernel.h).  A tile alone on its
-// compute unit is a chain of latencies, 0.2 us per k-group, two overlap; more issue more instructions per product than the large tiles.  The GEMM alone,
-// waves that split K / large tiles / this one, us, rank 32: norm and rotary M = 256, K = 3072, N = 9216 23.6 / 22.5 / 19.6, M = 505, K = 2048, N = 6144 18.0 / 17.1 / 15.7, at
-// 2.25 tiles M = 505, K = 3072, N = 9216 34.6 / 29.6 / 30.6; quantizing epilogue K = 3072, N = 12288 M = 256 29.8 / 29.2 / 26.7, M = 300 30.8 / 30.4 / 28.8, at three tiles M = 505
-// 43.6 / 39.4 / 39.3, rank 128 59.4 / 47.3 / 52.6; layer calls, plain M = 384, K = 3072, N = 9216 26.3 / 22.8 with this one, M = 320 (1.4 tiles, where narrow ones are better)
-// 22.4 / 22.6, M = 505 30.4 / 32.1.
-// (`split`: the large tiles would be split along K, see choose_direct)
-bool staged_rows(const svdq_gemm_args *a, int ncu, bool split) {
-    if (a->fp4 || a->K < 256) return false;
-    const long long tiles = (rows_needed(a) + 63) / 64 * (a->N / 128);
-    return 2 * tiles >= (needs_next_epilogue(a) ? 2 * ncu + 2 : 3 * ncu) && tiles <= (a->qout && split ? 3 : 2) * ncu;
-}
-
 // NVFP4 launches of 64 x 128 tiles: how many blocks of 64 rows, what they leave of the rows in blocks of 32 behind them (nothing, where the last block is
 // partly padding), and the time of the busiest compute unit in tiles of 64 rows.  With tiles of one height the last ones keep a few compute units busy for
 // the time of a whole tile, also where most of its rows are padding; the hardware hands tiles to the emptiest compute unit, and two of them on one share
@@ -715,11 +662,71 @@ Heights few_rows_heights(int rows, int column_blocks, int ncu) {
     const double limit = 0.985 * best.time;
     const int q = (int)((long long)(units / 2) * column_blocks / ncu);
     for (int full : {units / 2, (int)((long long)q * ncu / column_blocks), (int)((long long)(q - 1) * ncu / column_blocks)}) {
-        if (full < 0 || full > units / 2 || 2 * full == units) continue;
+        if (full <= 0 || full > units / 2 || 2 * full == units) continue;  // (32-row tiles alone are shape 1)
         const double t = time(full);
         if (t <= limit && t <= best.time) best = Heights{full, t};
     }
     return best;
+}
+
+// The tile of a few-rows launch with the plain epilogue, in blocks of 32 x 32 (`shape`: the better one of 128 columns by the models of
+// choose_direct, of 32 rows (1) or 64 (2)).  What takes the time is the fetching of the operands: a
+// compute unit gets 120 GB/s in requests of 16 bytes a lane, 80 in those of 8, however few of them fetch and however many waves do (48
+// or 192 workgroups, 4 ... 16 waves each), and a tile of mt x nc blocks fetches mt + nc fragments per k-group.  Square tiles fetch least per
+// product, small ones bring more compute units to bear: the sums cost a tile nothing before the end.  A model of the time in us, linear in the
+// tiles of the busiest compute unit and in the k-groups, fitted to 844 shapes (M = 16 ... 1000, K = 1024 ... 13824, N = 1024 ... 21504)
+// times the six tiles: its choice is 0.1 % (INT4) and 0.05 % (NVFP4) off the fastest on average and 5.4 % at most; tiles of 128 columns only,
+// 18 and 21 %.  Measured, layer calls, 128 columns / the choice, us:
+//   INT4   M = 64, K = N = 3072  13.3 / 10.2 (32 x 32)    NVFP4  14.6 / 10.3
+//          M = 256               14.1 / 13.1 (64 x 64)           15.3 / 14.1
+//          M = 64, K = 12288     32.3 / 21.4 (32 x 32)           34.6 / 21.6
+//          M = 256, K = 12288    34.7 / 30.3 (64 x 64)           37.4 / 34.0
+// Few columns, and INT4 with short rows (fewer than 1024), where 64-row tiles are the better ones of 128 columns: compute units have several tiles, and the
+// model, which does not know the fixed part of a tile well, favours narrow ones too much.  There they are taken if it says 8 %, and in INT4 not
+// with K = 128: M = 125, K = 128, N = 11392, rank 16 5.1 us with 64 x 128, 32 x 32 6.3; NVFP4 M = 5041, K = 8448, N = 512 48.2, 64 x 64 55.8.  Over 325 INT4 and 357 NVFP4
+// shapes with few columns, short rows or more than 9216 rows 0.9 and 0.6 % off the fastest tile, without this 1.1 and 0.6; 1111 and 1370 others 0.2 and 0.3 % (M = 1 ...
+// 20000, K = 128 ... 16640, N = 128 ... 21504, ranks 0 ... 160).  NVFP4, 64 x 128 tiles with 32-row ones behind them at their time: 0.3 % off over 1100 shapes, 0.7 at
+// that of 64-row ones alone (M = 800, K = N = 3072 17.9 us in 64 x 64, 16.7 so).
+FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu, int shape) {
+    struct Model {
+        int mt, nc;
+        double launch, tile, kgroup;
+    };
+    constexpr Model int4[] = {{1, 1, -0.18, 0.18, 0.0382}, {1, 2, -0.46, 0.68, 0.0551}, {2, 1, -0.46, 0.75, 0.0499},
+                              {2, 2, 0.18, 0.64, 0.0702},  {1, 4, -0.13, 0.64, 0.0948}, {2, 4, 1.04, 0.53, 0.1378}};
+    constexpr Model nvfp4[] = {{1, 1, -0.85, 0.16, 0.0323}, {1, 2, -0.52, 0.14, 0.0515}, {2, 1, -0.64, 0.24, 0.0498},
+                               {2, 2, -0.17, 0.46, 0.0719}, {1, 4, 0.22, 0.47, 0.0876},  {2, 4, 1.96, -0.07, 0.1112}};
+    const long long row_blocks = (rows_needed(a) + 31) / 32, column_blocks = a->N / 32;
+    const bool favour_wide = shape == 2 && (a->N < 1024 || (!a->fp4 && a->K < 1024));
+    FewRowsTile best{};
+    for (const Model &m : a->fp4 ? nvfp4 : int4) {
+        const bool wide = m.mt == 2 && m.nc == 4;
+        if (favour_wide && !a->fp4 && a->K < 256 && !wide) continue;
+        const long long tiles = (row_blocks + m.mt - 1) / m.mt * (column_blocks / m.nc);
+        double rounds = (double)((tiles + ncu - 1) / ncu), launch = m.launch;
+        if (a->fp4 && wide) {
+            const double time = few_rows_heights(rows_needed(a), (int)(a->N / 128), ncu).time;
+            if (time < rounds) launch += 0.25;  // (two heights)
+            rounds = time;
+        }
+        const double t = (launch + rounds * (m.tile + m.kgroup * (double)(a->K / 64))) * (favour_wide && wide ? 0.92 : 1.0);
+        if (best.mt == 0 || t < best.time) best = FewRowsTile{m.mt, m.nc, false, t};
+    }
+    return best;
+}
+
+// INT4 launches with more than one tile of 64 x 128 per compute unit and up to two (plain epilogue: from one and a half on): such tiles, where they are
+// chosen (choose_direct), have waves that split the columns and share the rows' operands through LDS (gemm_direct_kernel.h).  A tile alone on its
+// compute unit is a chain of latencies, 0.2 us per k-group, two overlap; more issue more instructions per product than the large tiles.  The GEMM alone,
+// waves that split K / large tiles / this one, us, rank 32: norm and rotary M = 256, K = 3072, N = 9216 23.6 / 22.5 / 19.6, M = 505, K = 2048, N = 6144 18.0 / 17.1 / 15.7, at
+// 2.25 tiles M = 505, K = 3072, N = 9216 34.6 / 29.6 / 30.6; quantizing epilogue K = 3072, N = 12288 M = 256 29.8 / 29.2 / 26.7, M = 300 30.8 / 30.4 / 28.8, at three tiles M = 505
+// 43.6 / 39.4 / 39.3, rank 128 59.4 / 47.3 / 52.6; layer calls, plain M = 384, K = 3072, N = 9216 26.3 / 22.8 with this one, M = 320 (1.4 tiles, where narrow ones are better)
+// 22.4 / 22.6, M = 505 30.4 / 32.1.
+// (`split`: the large tiles would be split along K, see choose_direct)
+bool staged_rows(const svdq_gemm_args *a, int ncu, bool split) {
+    if (a->fp4 || a->K < 256) return false;
+    const long long tiles = (rows_needed(a) + 63) / 64 * (a->N / 128);
+    return 2 * tiles >= (needs_next_epilogue(a) ? 2 * ncu + 2 : 3 * ncu) && tiles <= (a->qout && split ? 3 : 2) * ncu;
 }
 
 // Which tiles of the few-rows kernel a launch takes, if any.  Shape 1: tiles of 32 rows x 128 columns, four waves split
@@ -751,20 +758,20 @@ FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
         const long long ntiles = (a->M_pad / BM) * ((a->N + BN - 1) / BN);
         const double tiles = (double)ntiles / ncu;
         const int nwg = whole_tiles_fp4(ntiles, ncu);
-        t1 = 4.3 + c1 * (1.1 + 0.127 * kg);
-        t2 = 5.0 + c2 * (1.6 + 0.205 * kg) - (c2 < 3.0 ? 0.04 * kg : 0.0);
-        if (a->qout) {
-            t1 += 1.1 * c1;
-            t2 += 1.4 * c2;
-        } else if (a->rotary_emb) {
-            t1 += 0.9 * c1;
-            t2 += 1.0 * c2;
-        }
+        const double own1 = a->qout ? 1.1 : a->rotary_emb ? 0.9 : 0.0, own2 = a->qout ? 1.4 : a->rotary_emb ? 1.0 : 0.0;  // of the epilogue
+        auto shape2_time = [&](double tiles) { return 5.0 + tiles * (1.6 + 0.205 * kg + own2) - (tiles < 3.0 ? 0.04 * kg : 0.0); };
+        // (32-row tiles behind the 64-row ones at their time: 0.2 % off the better shape over 3500 launches, 2 of them more than 10 %; at that of 64-row ones alone
+        // 0.35 %, 58)
+        const double tall = few_rows_heights(rows, (int)ncols, ncu).time;
+        t1 = 4.3 + c1 * (1.1 + 0.127 * kg + own1);
+        t2 = shape2_time(tall);
         if (tiles > 1.0 && !nwg) {
             // Large tiles shared by workgroups: 26 to 40 us for the sums that meet in the workspace.  (They need 128 MB of it, more than the fixed scratch
             // has, and a call gives the same bits with either: they stay where these models put them, though up to 17 % faster beyond, M = 6400, K = 640,
-            // N = 16384 210 us against 181.)
+            // N = 16384 210 us against 181; with 64-row tiles alone beside them, as when the models were fitted.)
             t_large = (1.3 * kg + 14.0 + (a->qout ? 20.0 : a->rotary_emb ? 10.0 : 0.0)) * tiles + 33.0;
+            if (t1 >= t_large && shape2_time(c2) >= t_large) return none;
+            t_large = HUGE_VAL;
         } else {
             // Whole large tiles, in one round or several.  Their time and that of the few-rows kernel beside them, fitted to 555 and 400 launches in which the two are
             // within 1.6 of each other (M up to 20000, K = 128 ... 16640, ranks 0 ... 160, all epilogues): a tile's rank and epilogue cost either kernel, small
@@ -786,12 +793,12 @@ FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
                 constexpr Model shape2{4.43, 1.19, 0.165, 0.423, 2.48, 1.51, 0.92, 0.48};
                 const Model large{6.65, 6.65, 0.344 + 1.179 * tiles, 1.23, 27.7, 15.8, 8.0, 6.4};
                 t_large = large.time(a, 1.0);
-                t_few = t1 < t2 ? shape1.time(a, c1) : shape2.time(a, c2);
+                t_few = t1 < t2 ? shape1.time(a, c1) : shape2.time(a, tall);
             } else {
                 constexpr Model shape2{0.65, 1.394, 0.1719, 0.441, 2.21, 0.99, 0.99, 0.48};
                 constexpr Model large{8.14, 8.39, 1.398, 1.09, 20.0, 12.8, 8.4, 7.6};
                 t_large = large.time(a, (double)(ntiles / nwg));
-                t_few = t1 < t2 ? shape1.time(a, c1) : shape2.time(a, c2);
+                t_few = t1 < t2 ? shape1.time(a, c1) : shape2.time(a, tall);
             }
             const double t_power = 2.0 * rows * (double)a->K * (double)a->N / 1.28e9;  // (us at 1.28 PFLOP/s)
             if (t_few < t_power) t_few = t_power;

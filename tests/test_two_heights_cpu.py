@@ -46,7 +46,7 @@ def test_rows_are_covered_inside_the_padded_tensor():
             continue
         units, nb = (M + 31) // 32, N // 128
         half = max(units - 2 * p.full_blocks, 0)
-        assert p.row_blocks == (M + 63) // 64 and 0 <= p.full_blocks <= p.row_blocks and M <= 64 * p.full_blocks + 32 * half <= (M + 255) // 256 * 256
+        assert p.row_blocks == (M + 63) // 64 and 0 < p.full_blocks <= p.row_blocks and M <= 64 * p.full_blocks + 32 * half <= (M + 255) // 256 * 256
         load = [0.0] * ncu
         for cost, n in ((1.0, p.full_blocks * nb), (0.68, half * nb)):
             for _ in range(n):  # the emptiest one takes the next tile
@@ -60,7 +60,7 @@ def test_rows_are_covered_inside_the_padded_tensor():
 
 @pytest.mark.parametrize("kind,M,K,N,want", [
     ("rope", 505, 3072, 9216, 7), ("rope", 300, 3072, 9216, 3), ("silu", 201, 2688, 15744, 4), ("plain", 2300, 3072, 3072, 32), ("rope", 1200, 3072, 9216, 17),
-    ("split", 17, 3968, 11904, 4),
+    ("split", 17, 3968, 11904, 4), ("plain", 800, 3072, 3072, 10), ("plain", 405, 2944, 5120, 6), ("split", 2422, 1920, 5760, 39),  # (the last three in other tiles but for those of 32 rows)
 ])
 def test_blocks_of_64_rows(kind, M, K, N, want):
     p = plan_of(call(kind, M, K, N, 32, True))
