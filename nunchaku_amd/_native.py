@@ -85,11 +85,11 @@ class AwqGemvArgs(ctypes.Structure):
 
 
 # kernel variants, one translation unit each (-DSVDQ_VARIANT=n): the INT4 GEMM (gemm6_variant.hip: plain, next-layer epilogue), the NVFP4
-# GEMM (gemm_variant.hip: the same two), the few-rows GEMM (gemm_direct_variant.hip: the same two of INT4, then of NVFP4) and its narrow
+# GEMM (gemm_variant.hip: the same two), the few-rows GEMM (gemm_direct_variant.hip: the same two of INT4, then of NVFP4; gemm_direct_ranks_variant.hip: NVFP4 at ranks above 32) and its narrow
 # tiles (gemm_narrow_variant.hip: both precisions in each)
 GEMM_VARIANT_UNITS = [("gemm6_variant.hip", 0), ("gemm6_variant.hip", 1), ("gemm_variant.hip", 4), ("gemm_variant.hip", 5),
                       ("gemm_direct_variant.hip", 0), ("gemm_direct_variant.hip", 1), ("gemm_direct_variant.hip", 2), ("gemm_direct_variant.hip", 3),
-                      ("gemm_narrow_variant.hip", 0), ("gemm_narrow_variant.hip", 1)]
+                      ("gemm_direct_ranks_variant.hip", 0), ("gemm_direct_ranks_variant.hip", 1), ("gemm_narrow_variant.hip", 0), ("gemm_narrow_variant.hip", 1)]
 
 
 HOST_PATH = _PKG_DIR / "_host.so"

@@ -13,6 +13,8 @@ int launch_int4_plain(const GemmParams &p, int shape, hipStream_t stream);
 int launch_int4_next(const GemmParams &p, int shape, hipStream_t stream);
 int launch_fp4_plain(const GemmParams &p, int shape, hipStream_t stream);
 int launch_fp4_next(const GemmParams &p, int shape, hipStream_t stream);
+int launch_fp4_ranks_plain(const GemmParams &p, int shape, hipStream_t stream);
+int launch_fp4_ranks_next(const GemmParams &p, int shape, hipStream_t stream);
 int launch_square(const GemmParams &p, bool fp4, int mt, hipStream_t stream);
 int launch_oblong(const GemmParams &p, bool fp4, int mt, hipStream_t stream);
 int launch_staged_plain(const GemmParams &p, hipStream_t stream);
@@ -885,6 +887,7 @@ int gemm_direct(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t
     auto launch = [&]() {
         if (plan.columns < 128) return plan.columns == 32 * mt ? direct::launch_square(p, fp4, mt, st) : direct::launch_oblong(p, fp4, mt, st);
         if (plan.shared_rows) return next ? direct::launch_staged_next(p, st) : direct::launch_staged_plain(p, st);
+        if (fp4 && p.R_up > 32) return next ? direct::launch_fp4_ranks_next(p, mt, st) : direct::launch_fp4_ranks_plain(p, mt, st);  // (see output_tile)
         if (fp4) return next ? direct::launch_fp4_next(p, mt, st) : direct::launch_fp4_plain(p, mt, st);
         return next ? direct::launch_int4_next(p, mt, st) : direct::launch_int4_plain(p, mt, st);
     };

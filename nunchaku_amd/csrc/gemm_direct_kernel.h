@@ -84,7 +84,12 @@ struct Lds {
 constexpr bool two_heights(bool fp4, int MT, int NC) { return fp4 && MT == 2 && NC == 4; }
 
 // One tile: MT blocks of 32 rows from block f0 on, column block nb.
-template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT>
+// RANKS (NVFP4, tiles of 128 columns, ranks above 32): all four waves need the low-rank operands of the same rows, and a lane that fetches 16 bytes of a row for itself costs
+// the vector memory path four times as much as whole pieces of rows do.  The operands go to the place of the sums by asynchronous copies, once these have been
+// read, up to rank 128 all at once; two steps requested ahead of the sums and the others behind them, a memory latency each / so, us, the GEMM alone: K = 1408, N = 15872, M = 213, rank 64
+// 15.1 / 13.7, rank 128 18.2 / 15.0; norm and rotary, M = 505, K = 3072, N = 9216, rank 64 32.9 / 31.8, rank 128 38.1 / 33.8, rank 160 43.0 / 36.8; quantizing, M = 1157, N = 12288, rank 64 102.7 / 100.6,
+// rank 128 122.5 / 115.6; rank 48 equal to 3 %.  Same bits.  (A kernel of its own: beside the other way in one, ranks up to 32 lost up to 2 %.  INT4: no gain.)
+template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT, bool RANKS>
 __device__ __forceinline__ void output_tile(const GemmParams &p, const int nb, const int f0) {
     constexpr int NC = NT * WN;  // 32-column tiles of the workgroup; a wave has NT of them
     constexpr int WAVES = WN * KP;
@@ -469,10 +474,12 @@ __device__ __forceinline__ void output_tile(const GemmParams &p, const int nb, c
     LowRank more[LSTEPS];
     auto load_more = [&](int s0) {
 #pragma unroll
-        for (int s = 0; s < LSTEPS; s++)
-            if (s0 + s < nsteps) load_low_rank(more[s], s0 + s);
+        for (int s = 0; s < LSTEPS; s++) load_low_rank(more[s], s0 + s < nsteps ? s0 + s : nsteps - 1);  // (a request behind a branch makes the compiler wait for those before it)
     };
-    if (owner) load_more(LFIRST);
+    static_assert(!RANKS || (!NARROW && !STAGED && KP == 4));
+    constexpr int COPIED = RANKS ? 2 * (L::SUMS / L::LR_CHUNK) : 0;  // steps that the place of the sums holds
+    const int copied = nsteps < COPIED ? nsteps : COPIED;
+    if (!RANKS && owner && LFIRST < nsteps) load_more(LFIRST);
     // Factor and bias of the lane's columns c0 + 8 q + 4 h + i.
     float *tab = (float *)(lds + L::TAB + wave * 256);
     if (TABLE && h == 0) {
@@ -544,7 +551,25 @@ __device__ __forceinline__ void output_tile(const GemmParams &p, const int nb, c
                 for (int i = 0; i < 4; i++) val[mt][4 * q + i] = s[i];
             }
         }
-        __syncthreads();  // the sums have been read: the slabs take their place
+        __syncthreads();  // the sums have been read: the low-rank operands (RANKS) and then the slabs take their place
+        // (32 ranks at a time; which 16 bytes of its row a lane fetches is permuted as in gemm6_kernel.h)
+        for (int c = 0; 2 * c < copied; c++) {
+            const bool half = nsteps - 2 * c < 2;  // 16 ranks only: the other half of the places is filled with anything
+            const uint32_t place = lds_base + c * L::LR_CHUNK;
+            const uint8_t *up = (const uint8_t *)p.lora_up + (size_t)n0 * p.R_up * 2 + c * 64, *la = (const uint8_t *)p.lora_act + (size_t)row0 * p.R_up * 4 + c * 128;
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const int col = (wave * 2 + i) * 16 + (lane >> 2), up_piece = (lane & 3) ^ g6::lr_up_swizzle(col);
+                const uint32_t up_off = (uint32_t)col * (uint32_t)(p.R_up * 2) + (half ? up_piece & 1 : up_piece) * 16;
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(place + (wave * 2 + i) * 1024), "v"(up_off), "s"(up) : "memory", "m0");
+            }
+#pragma unroll
+            for (int i = 0; i < MT; i++) {
+                const int row = (wave * MT + i) * 8 + (lane >> 3), act_piece = (lane & 7) ^ g6::lr_act_swizzle(row);
+                const uint32_t act_off = (uint32_t)row * (uint32_t)(p.R_up * 4) + (half ? act_piece & 3 : act_piece) * 16;
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(place + L::LR_ACT + (wave * MT + i) * 1024), "v"(act_off), "s"(la) : "memory", "m0");
+            }
+        }
     }
 
     float *ssq = (float *)(lds + L::SSQ);  // [MT][4 column tiles][32 rows]
@@ -576,10 +601,8 @@ __device__ __forceinline__ void output_tile(const GemmParams &p, const int nb, c
 #pragma unroll
     for (int s = 0; s < EARLY; s++)
         if (s < nsteps) add_step(early[s], s);
-#pragma unroll
-    for (int s = 0; s < LR_AHEAD; s++) {
-        if (s >= lr_steps) break;
-        const uint8_t *buf = lds + L::LR + (s / 2) * L::LR_CHUNK;
+    auto add_copied = [&](const uint8_t *chunk, int s) {
+        const uint8_t *buf = chunk + (s / 2) * L::LR_CHUNK;
         const int col = wave * 32 + r32, k = s % 2;
         const u32x4_t up = *(const u32x4_t *)(buf + col * 64 + (((2 * k + h) ^ g6::lr_up_swizzle(col)) << 4));
 #pragma unroll
@@ -588,9 +611,26 @@ __device__ __forceinline__ void output_tile(const GemmParams &p, const int nb, c
             const uint8_t *ap = buf + L::LR_ACT + row * 128;
             add_low_rank(o, s, *(const float4_t *)(ap + (((4 * k + 2 * h) ^ g6::lr_act_swizzle(row)) << 4)), *(const float4_t *)(ap + (((4 * k + 2 * h + 1) ^ g6::lr_act_swizzle(row)) << 4)), up);
         }
+    };
+#pragma unroll
+    for (int s = 0; s < LR_AHEAD; s++) {
+        if (s >= lr_steps) break;
+        add_copied(lds + L::LR, s);
     }
-    for (int s0 = LFIRST; s0 < nsteps; s0 += LSTEPS) {
-        if (s0 > LFIRST) load_more(s0);
+    if constexpr (RANKS) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        for (int c = 0; 2 * c < copied; c++) {
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                if (2 * c + k >= copied) break;
+                add_copied(lds, 2 * c + k);
+            }
+        }
+        __syncthreads();  // (read: the slabs take their place)
+    }
+    for (int s0 = RANKS ? copied : LFIRST; s0 < nsteps; s0 += LSTEPS) {
+        if (RANKS || s0 > LFIRST) load_more(s0);
 #pragma unroll
         for (int s = 0; s < LSTEPS; s++)
             if (s0 + s < nsteps) add_step(more[s], s0 + s);
@@ -780,27 +820,27 @@ __device__ inline int tile_of(int block, int total) {
     return xcd * (total / 8) + (xcd < extra ? xcd : extra) + block / 8;
 }
 
-template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT>
+template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT, bool RANKS>
 __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_kernel(GemmParams p) {
     if constexpr (two_heights(FP4, MT, NT * WN)) {
         const int full = p.full_blocks * (p.N / (32 * NT * WN)), block = (int)blockIdx.x;
         if (block < full) {
             const int v = tile_of(block, full), nb = v / p.full_blocks;
-            output_tile<FP4, 2, NT, WN, KP, DEPTH, NEXT>(p, nb, (v - nb * p.full_blocks) * 2);
+            output_tile<FP4, 2, NT, WN, KP, DEPTH, NEXT, RANKS>(p, nb, (v - nb * p.full_blocks) * 2);
         } else {
             // (as deep a ring as the launches of 32-row tiles alone have)
             const int half_blocks = p.row_blocks - p.full_blocks, v = tile_of(block - full, (int)gridDim.x - full), nb = v / half_blocks;
-            output_tile<FP4, 1, NT, WN, KP, 2, NEXT>(p, nb, p.full_blocks * 2 + v - nb * half_blocks);
+            output_tile<FP4, 1, NT, WN, KP, 2, NEXT, RANKS>(p, nb, p.full_blocks * 2 + v - nb * half_blocks);
         }
     } else {
         const int v = tile_of((int)blockIdx.x, (int)gridDim.x), nb = v / p.row_blocks;
-        output_tile<FP4, MT, NT, WN, KP, DEPTH, NEXT>(p, nb, (v - nb * p.row_blocks) * MT);
+        output_tile<FP4, MT, NT, WN, KP, DEPTH, NEXT, RANKS>(p, nb, (v - nb * p.row_blocks) * MT);
     }
 }
 
-template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT>
+template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT, bool RANKS = false>
 int launch_direct(const GemmParams &params, hipStream_t stream) {
-    auto kern = gemm_direct_kernel<FP4, MT, NT, WN, KP, DEPTH, NEXT>;
+    auto kern = gemm_direct_kernel<FP4, MT, NT, WN, KP, DEPTH, NEXT, RANKS>;
     using L = Lds<MT, NT, WN, KP, DEPTH>;
     static bool lds_reserved[64] = {false};  // set once per device (racing first calls both set it, which is harmless)
     int dev = 0;
