@@ -797,14 +797,18 @@ FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
                 }
             };
             constexpr Model shape1{3.7, 1.06, 0.1132, 0.248, 1.37, 0.79, 0.49, 0.16};
+            // Ranks above 32, whose operands come through LDS in the few-rows kernel, cost it 0.17 us per 16 ranks and tile of 64 rows: over 1014 launches of ranks 48 ... 96 0.2 % off the
+            // faster kernel, 25 of them 3 % and more; with the cost of ranks up to 32 2.7 %, 323.  (From rank 128 on it stands at 0.33, with which the short rows near the
+            // line keep the kernel they had: 541 launches 1.7 % off, 4.5 before.)
+            auto shape2_rank = [&](double up_to_32) { return a->R_up <= 32 ? up_to_32 : a->R_up < 128 ? 0.17 : 0.33; };
             double t_few;
             if (tiles <= 1.0) {
-                constexpr Model shape2{4.43, 1.19, 0.165, 0.423, 2.48, 1.51, 0.92, 0.48};
+                const Model shape2{4.43, 1.19, 0.165, shape2_rank(0.423), 2.48, 1.51, 0.92, 0.48};
                 const Model large{6.65, 6.65, 0.344 + 1.179 * tiles, 1.23, 27.7, 15.8, 8.0, 6.4};
                 t_large = large.time(a, 1.0);
                 t_few = t1 < t2 ? shape1.time(a, c1) : shape2.time(a, tall);
             } else {
-                constexpr Model shape2{0.65, 1.394, 0.1719, 0.441, 2.21, 0.99, 0.99, 0.48};
+                const Model shape2{0.65, 1.394, 0.1719, shape2_rank(0.441), 2.21, 0.99, 0.99, 0.48};
                 constexpr Model large{8.14, 8.39, 1.398, 1.09, 20.0, 12.8, 8.4, 7.6};
                 t_large = large.time(a, (double)(ntiles / nwg));
                 t_few = t1 < t2 ? shape1.time(a, c1) : shape2.time(a, tall);

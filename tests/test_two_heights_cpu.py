@@ -67,3 +67,11 @@ def test_blocks_of_64_rows(kind, M, K, N, want):
     assert (p.few_rows, p.columns, p.full_blocks) == (2, 128, want), p
     assert plan_of(call(kind, M, K, N, 32, False)).few_rows * plan_of(call(kind, M, K, N, 32, False)).full_blocks == 0
     assert plan_of(call("next", 1157, 3072, 12288, 32, True, with_out=False), rows=1157).full_blocks == 16
+
+
+# Ranks above 32 cost the few-rows kernel less (their operands come through LDS): on either side of the line to whole large tiles.
+@pytest.mark.parametrize("kind,M,K,N,R,few", [
+    ("split", 3235, 1408, 4224, 80, 2), ("rope", 6509, 1536, 4608, 64, 2), ("silu", 2881, 1408, 18304, 128, 2), ("plain", 4709, 1408, 3328, 128, 0), ("plain", 4608, 3072, 21504, 32, 0),
+])
+def test_few_rows_or_large_tiles_at_higher_ranks(kind, M, K, N, R, few):
+    assert plan_of(call(kind, M, K, N, R, True)).few_rows == few
