@@ -643,6 +643,9 @@ struct FewRowsTile {
 // rotary, N = 9216, M = 300 21.0 / 19.2, M = 505 33.1 / 29.9, M = 700 43.5 / 40.1, M = 1200 66.3 / 63.8; quantizing, N = 12288, M = 400 40.2 / 37.0, M = 1157 97.2 / 91.9; plain, N = 3072,
 // M = 2300 41.0 / 39.4.  4.5 % faster over 4600 launches of 16 ... 9216 rows (with the epilogue's requests ahead of the main loop, which came before), 6 of them slower by more than 3 %.  (Slower:
 // 32-row tiles where the model sees no gain, up to 9 % where all rows are in them; INT4, whose launches of several tiles per compute unit share the rows or are large tiles.)
+// Not where tiles of 32 rows alone would be two per compute unit at most: so few are not handed to the emptiest one, and what bounds them is the requests, not the matrix core
+// that the model is about.  1508 such launches are 14 % faster in 32-row tiles than in two heights, none of them slower by 4 %: SiLU, M = 67, K = 2944, N = 19840 15.7 / 18.6 us,
+// quantizing, M = 65, K = 6272, N = 18176, rank 64 34.9 / 40.9.  (At three 185 launches 34 % faster.)
 struct Heights {
     int full;
     double time;
@@ -661,6 +664,7 @@ Heights few_rows_heights(int rows, int column_blocks, int ncu) {
         }
     };
     Heights best{all, (double)(((long long)all * column_blocks + ncu - 1) / ncu)};
+    if ((long long)units * column_blocks <= 2ll * ncu) return best;
     const double limit = 0.985 * best.time;
     const int q = (int)((long long)(units / 2) * column_blocks / ncu);
     for (int full : {units / 2, (int)((long long)q * ncu / column_blocks), (int)((long long)(q - 1) * ncu / column_blocks)}) {

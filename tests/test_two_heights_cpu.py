@@ -69,6 +69,16 @@ def test_blocks_of_64_rows(kind, M, K, N, want):
     assert plan_of(call("next", 1157, 3072, 12288, 32, True, with_out=False), rows=1157).full_blocks == 16
 
 
+# No two heights where 32-row tiles alone are two per compute unit at most (465 to 507 of them in the first seven, 513 and 520 in the others), whichever model chooses the tile.
+@pytest.mark.parametrize("kind,M,K,N,R,mt", [
+    ("silu", 67, 2944, 19840, 16, 1), ("silu", 66, 7424, 19072, 32, 1), ("next", 65, 6272, 18176, 64, 1), ("plain", 68, 12928, 19584, 64, 1), ("silu", 587, 13568, 3328, 32, 1),
+    ("next", 1227, 3584, 1664, 32, 1), ("plain", 513, 11904, 3712, 0, 1), ("silu", 587, 13568, 3456, 32, 2), ("next", 1250, 3584, 1664, 32, 2),
+])
+def test_two_heights_from_three_32_row_tiles_on(kind, M, K, N, R, mt):
+    p = plan_of(call(kind, M, K, N, R, True, with_out=kind != "next", R_down=R), rows=M if kind == "next" else 0)
+    assert (p.few_rows, p.columns) == (mt, 128), p
+
+
 # Ranks above 32 cost the few-rows kernel less (their operands come through LDS): on either side of the line to whole large tiles.
 @pytest.mark.parametrize("kind,M,K,N,R,few", [
     ("split", 3235, 1408, 4224, 80, 2), ("rope", 6509, 1536, 4608, 64, 2), ("silu", 2881, 1408, 18304, 128, 2), ("plain", 4709, 1408, 3328, 128, 0), ("plain", 4608, 3072, 21504, 32, 0),
