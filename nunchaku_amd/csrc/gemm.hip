@@ -742,6 +742,15 @@ SharedRows staged_rows(const svdq_gemm_args *a, int ncu, bool split) {
     return may ? SharedRows::IF_FASTEST : SharedRows::NO;
 }
 
+// NVFP4 launches of tiles of 128 columns whose low-rank operands come through LDS (gemm_direct_kernel.h, RANKS).  They are copied 32 ranks at a time, and 16 that are left over take
+// as long as 32, so an odd number of them pays only where the copies of one tile pass beside another one: wave by wave / through LDS over 15000 launches, tiles of 32 rows 0.97 at ranks 48,
+// 80, 112 and 144 (silu, M = 66, K = 640, N = 2688, rank 48 6.3 / 6.7 us), 0.96 at 176 to 240, at 64 1.00, at 96 1.01, at 128 to 512 1.03 to 1.05; of 64 rows, one per compute unit 0.98 at
+// 48, 0.99 at 80 and 112, 0.96 at 144 and more, several 1.00 at 48, 1.02 at 80, 1.04 at 112, 1.01 to 1.02 at 144 and more, at 64 1.02 and 1.06, at 96 1.06 and 1.12, at 128 1.09 and 1.2.
+bool copies_ranks(const svdq_gemm_args *a, int ncu, int mt) {
+    if (a->R_up <= 32) return false;
+    return a->R_up % 32 == 0 || (a->R_up > 48 && mt == 2 && (rows_needed(a) + 63) / 64 * (a->N / 128) > ncu);
+}
+
 // Which tiles of the few-rows kernel a launch takes, if any.  Shape 1: tiles of 32 rows x 128 columns, four waves split
 // K.  Shape 2: tiles of 64 rows x 128 columns, a quarter fewer operand bytes per product, from about 400 tiles of 32 rows on; INT4: two waves
 // split K and two the columns, NVFP4: four waves split K.  Models of the time in us fitted to launches at K = 1024 ... 12288
@@ -873,6 +882,7 @@ void make_plan(const svdq_gemm_args *a, int ncu, svdq_gemm_plan *plan) {
         plan->columns = 32 * t.nc;
         plan->shared_rows = t.shared_rows;
         plan->row_blocks = (rows_needed(a) + 32 * t.mt - 1) / (32 * t.mt);
+        plan->copied_ranks = a->fp4 && t.nc == 4 && copies_ranks(a, ncu, t.mt);
         if (a->fp4 && t.mt == 2 && t.nc == 4) plan->full_blocks = few_rows_heights(rows_needed(a), (int)(a->N / 128), ncu).full;
     } else if (a->fp4) {
         plan_fp4(a, ncu, plan);
@@ -895,7 +905,7 @@ int gemm_direct(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t
     auto launch = [&]() {
         if (plan.columns < 128) return plan.columns == 32 * mt ? direct::launch_square(p, fp4, mt, st) : direct::launch_oblong(p, fp4, mt, st);
         if (plan.shared_rows) return next ? direct::launch_staged_next(p, st) : direct::launch_staged_plain(p, st);
-        if (fp4 && p.R_up > 32) return next ? direct::launch_fp4_ranks_next(p, mt, st) : direct::launch_fp4_ranks_plain(p, mt, st);  // (see output_tile)
+        if (plan.copied_ranks) return next ? direct::launch_fp4_ranks_next(p, mt, st) : direct::launch_fp4_ranks_plain(p, mt, st);
         if (fp4) return next ? direct::launch_fp4_next(p, mt, st) : direct::launch_fp4_plain(p, mt, st);
         return next ? direct::launch_int4_next(p, mt, st) : direct::launch_int4_plain(p, mt, st);
     };

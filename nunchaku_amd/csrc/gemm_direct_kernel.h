@@ -84,11 +84,11 @@ struct Lds {
 constexpr bool two_heights(bool fp4, int MT, int NC) { return fp4 && MT == 2 && NC == 4; }
 
 // One tile: MT blocks of 32 rows from block f0 on, column block nb.
-// RANKS (NVFP4, tiles of 128 columns, ranks above 32): all four waves need the low-rank operands of the same rows, and a lane that fetches 16 bytes of a row for itself costs
+// RANKS (NVFP4, tiles of 128 columns, ranks above 32; which launches: copies_ranks in gemm.hip): all four waves need the low-rank operands of the same rows, and a lane that fetches 16 bytes of a row for itself costs
 // the vector memory path four times as much as whole pieces of rows do.  The operands go to the place of the sums by asynchronous copies, once these have been
 // read, up to rank 128 all at once; two steps requested ahead of the sums and the others behind them, a memory latency each / so, us, the GEMM alone: K = 1408, N = 15872, M = 213, rank 64
 // 15.1 / 13.7, rank 128 18.2 / 15.0; norm and rotary, M = 505, K = 3072, N = 9216, rank 64 32.9 / 31.8, rank 128 38.1 / 33.8, rank 160 43.0 / 36.8; quantizing, M = 1157, N = 12288, rank 64 102.7 / 100.6,
-// rank 128 122.5 / 115.6; rank 48 equal to 3 %.  Same bits.  (A kernel of its own: beside the other way in one, ranks up to 32 lost up to 2 %.  INT4: no gain.)
+// rank 128 122.5 / 115.6.  Same bits.  (A kernel of its own: beside the other way in one, ranks up to 32 lost up to 2 %.  INT4: no gain.)
 template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT, bool RANKS>
 __device__ __forceinline__ void output_tile(const GemmParams &p, const int nb, const int f0) {
     constexpr int NC = NT * WN;  // 32-column tiles of the workgroup; a wave has NT of them

@@ -22,7 +22,8 @@ typedef struct svdq_gemm_plan {
     int32_t workgroups;    // NVFP4, large tiles: persistent workgroups;
     int32_t shared_tiles;  // some tiles are shared by two or more of them
     int32_t columns;       // few rows: columns of a tile (32, 64 or 128),
-    int32_t shared_rows;   // its waves split the columns and share the rows' operands through LDS
+    int32_t shared_rows;   // its waves split the columns and share the rows' operands through LDS;
+    int32_t copied_ranks;  // the low-rank operands come through LDS (NVFP4, tiles of 128 columns)
 } svdq_gemm_plan;
 
 // What svdq_gemm_w4a4 (`rows` > 0: svdq_gemm_w4a4_rows) would do with these arguments on a GPU of so many compute units.  Checks the
