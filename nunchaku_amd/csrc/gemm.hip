@@ -813,21 +813,25 @@ FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
                 }
             };
             constexpr Model shape1{3.7, 1.06, 0.1132, 0.248, 1.37, 0.79, 0.49, 0.16};
-            // Ranks above 32, whose operands come through LDS in the few-rows kernel, cost it 0.17 us per 16 ranks and tile of 64 rows: over 1014 launches of ranks 48 ... 96 0.2 % off the
-            // faster kernel, 25 of them 3 % and more; with the cost of ranks up to 32 2.7 %, 323.  (From rank 128 on it stands at 0.33, with which the short rows near the
-            // line keep the kernel they had: 541 launches 1.7 % off, 4.5 before.)
-            auto shape2_rank = [&](double up_to_32) { return a->R_up <= 32 ? up_to_32 : a->R_up < 128 ? 0.17 : 0.33; };
+            // Ranks above 32, whose operands come through LDS in the few-rows kernel, cost it 0.17 us per 16 ranks and tile of 64 rows, and more at K below 1536, where the copies of a tile
+            // have fewer products of another to pass beside: 0.31 (large tiles in several rounds: 0.41) at K = 0.  Of 1062 launches that this brings here 30 are slower than in large tiles by 3 %
+            // and more, 12 % at most; with 0.17 at any K 267 of 1500, up to 28 % (large tiles / few rows, us: plain, M = 15370, K = 128, N = 1920, rank 80 37.7 / 48.3, norm and rotary, M = 10352, K = 384, N = 3072,
+            // rank 64 58.0 / 67.7).  (From rank 128 on it stands at 0.33, with which the short rows near the line keep the kernel they had.)  Ranks up to 32 at K = 128: by the 64-row tiles alone,
+            // 32-row ones behind them gain nothing there (plain, M = 11853, K = 128, N = 1280, rank 0 14.8 / 17.4).
+            const double shorter = a->K < 1536 ? 1.0 - (double)a->K / 1536 : 0.0;
+            auto shape2_rank = [&](double up_to_32, double short_rows) { return a->R_up <= 32 ? up_to_32 : a->R_up < 128 ? 0.17 + short_rows * shorter : 0.33; };
+            const double rounds2 = a->R_up <= 32 && a->K < 256 ? c2 : tall;
             double t_few;
             if (tiles <= 1.0) {
-                const Model shape2{4.43, 1.19, 0.165, shape2_rank(0.423), 2.48, 1.51, 0.92, 0.48};
+                const Model shape2{4.43, 1.19, 0.165, shape2_rank(0.423, 0.14), 2.48, 1.51, 0.92, 0.48};
                 const Model large{6.65, 6.65, 0.344 + 1.179 * tiles, 1.23, 27.7, 15.8, 8.0, 6.4};
                 t_large = large.time(a, 1.0);
-                t_few = t1 < t2 ? shape1.time(a, c1) : shape2.time(a, tall);
+                t_few = t1 < t2 ? shape1.time(a, c1) : shape2.time(a, rounds2);
             } else {
-                const Model shape2{0.65, 1.394, 0.1719, shape2_rank(0.441), 2.21, 0.99, 0.99, 0.48};
+                const Model shape2{0.65, 1.394, 0.1719, shape2_rank(0.441, 0.24), 2.21, 0.99, 0.99, 0.48};
                 constexpr Model large{8.14, 8.39, 1.398, 1.09, 20.0, 12.8, 8.4, 7.6};
                 t_large = large.time(a, (double)(ntiles / nwg));
-                t_few = t1 < t2 ? shape1.time(a, c1) : shape2.time(a, tall);
+                t_few = t1 < t2 ? shape1.time(a, c1) : shape2.time(a, rounds2);
             }
             const double t_power = 2.0 * rows * (double)a->K * (double)a->N / 1.28e9;  // (us at 1.28 PFLOP/s)
             if (t_few < t_power) t_few = t_power;
