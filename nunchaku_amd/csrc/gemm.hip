@@ -633,6 +633,7 @@ struct FewRowsTile {
     int mt, nc;  // blocks of 32 rows, of 32 columns (none: large tiles)
     bool shared_rows;
     double time;
+    int full_blocks;  // NVFP4, 64 x 128: blocks of 64 rows (few_rows_heights)
 };
 // NVFP4 launches of 64 x 128 tiles: how many blocks of 64 rows, what they leave of the rows in blocks of 32 behind them (nothing, where the last block is
 // partly padding), and the time of the busiest compute unit in tiles of 64 rows.  With tiles of one height the last ones keep a few compute units busy for
@@ -669,6 +670,8 @@ Heights few_rows_heights(int rows, int column_blocks, int ncu) {
     const int q = (int)((long long)(units / 2) * column_blocks / ncu);
     for (int full : {units / 2, (int)((long long)q * ncu / column_blocks), (int)((long long)(q - 1) * ncu / column_blocks)}) {
         if (full <= 0 || full > units / 2 || 2 * full == units) continue;  // (32-row tiles alone are shape 1)
+        // (the busiest compute unit has no less than all have on average)
+        if (((double)full + HALF * (units - 2 * full)) * column_blocks > limit * ncu * (1.0 + 1e-9)) continue;
         const double t = time(full);
         if (t <= limit && t <= best.time) best = Heights{full, t};
     }
@@ -693,7 +696,7 @@ Heights few_rows_heights(int rows, int column_blocks, int ncu) {
 // shapes with few columns, short rows or more than 9216 rows 0.9 and 0.6 % off the fastest tile, without this 1.1 and 0.6; 1111 and 1370 others 0.2 and 0.3 % (M = 1 ...
 // 20000, K = 128 ... 16640, N = 128 ... 21504, ranks 0 ... 160).  NVFP4, 64 x 128 tiles with 32-row ones behind them at their time: 0.3 % off over 1100 shapes, 0.7 at
 // that of 64-row ones alone (M = 800, K = N = 3072 17.9 us in 64 x 64, 16.7 so).
-FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu, int shape) {
+FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu, int shape, const Heights &tall) {
     struct Model {
         int mt, nc;
         double launch, tile, kgroup;
@@ -711,12 +714,11 @@ FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu, int shape) {
         const long long tiles = (row_blocks + m.mt - 1) / m.mt * (column_blocks / m.nc);
         double rounds = (double)((tiles + ncu - 1) / ncu), launch = m.launch;
         if (a->fp4 && wide) {
-            const double time = few_rows_heights(rows_needed(a), (int)(a->N / 128), ncu).time;
-            if (time < rounds) launch += 0.25;  // (two heights)
-            rounds = time;
+            if (tall.time < rounds) launch += 0.25;  // (two heights)
+            rounds = tall.time;
         }
         const double t = (launch + rounds * (m.tile + m.kgroup * (double)(a->K / 64))) * (favour_wide && wide ? 0.92 : 1.0);
-        if (best.mt == 0 || t < best.time) best = FewRowsTile{m.mt, m.nc, false, t};
+        if (best.mt == 0 || t < best.time) best = FewRowsTile{m.mt, m.nc, false, t, a->fp4 && wide ? tall.full : 0};
     }
     return best;
 }
@@ -779,6 +781,7 @@ FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
     const long long ncols = a->N / 128;
     const double c1 = (double)((((rows + 31) / 32) * ncols + ncu - 1) / ncu), c2 = (double)((((rows + 63) / 64) * ncols + ncu - 1) / ncu);
     double t_large, t1, t2;
+    Heights tall{};  // (worked out once a call: 20 to 70 ns of it)
     if (a->fp4) {
         const long long ntiles = (a->M_pad / BM) * ((a->N + BN - 1) / BN);
         const double tiles = (double)ntiles / ncu;
@@ -787,9 +790,9 @@ FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
         auto shape2_time = [&](double tiles) { return 5.0 + tiles * (1.6 + 0.205 * kg + own2) - (tiles < 3.0 ? 0.04 * kg : 0.0); };
         // (32-row tiles behind the 64-row ones at their time: 0.2 % off the better shape over 3500 launches, 2 of them more than 10 %; at that of 64-row ones alone
         // 0.35 %, 58)
-        const double tall = few_rows_heights(rows, (int)ncols, ncu).time;
+        tall = few_rows_heights(rows, (int)ncols, ncu);
         t1 = 4.3 + c1 * (1.1 + 0.127 * kg + own1);
-        t2 = shape2_time(tall);
+        t2 = shape2_time(tall.time);
         if (tiles > 1.0 && !nwg) {
             // Large tiles shared by workgroups: 26 to 40 us for the sums that meet in the workspace.  (They need 128 MB of it, more than the fixed scratch
             // has, and a call gives the same bits with either: they stay where these models put them, though up to 17 % faster beyond, M = 6400, K = 640,
@@ -820,7 +823,7 @@ FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
             // 32-row ones behind them gain nothing there (plain, M = 11853, K = 128, N = 1280, rank 0 14.8 / 17.4).
             const double shorter = a->K < 1536 ? 1.0 - (double)a->K / 1536 : 0.0;
             auto shape2_rank = [&](double up_to_32, double short_rows) { return a->R_up <= 32 ? up_to_32 : a->R_up < 128 ? 0.17 + short_rows * shorter : 0.33; };
-            const double rounds2 = a->R_up <= 32 && a->K < 256 ? c2 : tall;
+            const double rounds2 = a->R_up <= 32 && a->K < 256 ? c2 : tall.time;
             double t_few;
             if (tiles <= 1.0) {
                 const Model shape2{4.43, 1.19, 0.165, shape2_rank(0.423, 0.14), 2.48, 1.51, 0.92, 0.48};
@@ -861,14 +864,14 @@ FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
         if (plain) {
             // (the plain epilogue's tiles are faster than these two, the model of their time has no offset: 2277 layers of 100 ... 2600 rows 0.3 % off the
             // fastest, 0.6 without; M = 225, K = 4992, N = 10624 36.4 -> 30.5 us, M = 175, K = 9984, N = 14976 59 -> 51, M = 261, K = 1152, N = 14208 18 -> 17)
-            const FewRowsTile t = plain_tile(a, ncu, t1 < t2 ? 1 : 2);
+            const FewRowsTile t = plain_tile(a, ncu, t1 < t2 ? 1 : 2, tall);
             if (5.0 + 1.3 * t.time < t_large) return t;
             t_large *= 0.95;
         }
     }
     if ((t1 < t2 ? t1 : t2) >= t_large) return none;
     const int shape = t1 < t2 ? 1 : 2;
-    return plain ? plain_tile(a, ncu, shape) : FewRowsTile{shape, 4};
+    return plain ? plain_tile(a, ncu, shape, tall) : FewRowsTile{shape, 4, false, 0.0, shape == 2 ? tall.full : 0};
 }
 
 // Which kernel a call takes and how it divides the work.  A function of the arguments and the number of compute units alone:
@@ -890,7 +893,7 @@ void make_plan(const svdq_gemm_args *a, int ncu, svdq_gemm_plan *plan) {
         plan->shared_rows = t.shared_rows;
         plan->row_blocks = (rows_needed(a) + 32 * t.mt - 1) / (32 * t.mt);
         plan->copied_ranks = a->fp4 && t.nc == 4 && copies_ranks(a, ncu, t.mt);
-        if (a->fp4 && t.mt == 2 && t.nc == 4) plan->full_blocks = few_rows_heights(rows_needed(a), (int)(a->N / 128), ncu).full;
+        plan->full_blocks = t.full_blocks;
     } else if (a->fp4) {
         plan_fp4(a, ncu, plan);
     } else {
