@@ -894,6 +894,8 @@ void make_plan(const svdq_gemm_args *a, int ncu, svdq_gemm_plan *plan) {
         plan->row_blocks = (rows_needed(a) + 32 * t.mt - 1) / (32 * t.mt);
         plan->copied_ranks = a->fp4 && t.nc == 4 && copies_ranks(a, ncu, t.mt);
         plan->full_blocks = t.full_blocks;
+        const int low = (rows_needed(a) + 31) / 32 - 2 * t.full_blocks;
+        plan->low_blocks = t.full_blocks && low > 0 ? low : 0;
     } else if (a->fp4) {
         plan_fp4(a, ncu, plan);
     } else {
@@ -906,12 +908,8 @@ int gemm_direct(const svdq_gemm_args *a, const svdq_gemm_plan &plan, hipStream_t
     fill_params(a, p);
     const bool next = needs_next_epilogue(a), fp4 = a->fp4 != 0;
     const int mt = plan.few_rows;
-    p.row_blocks = plan.row_blocks;
-    if (fp4 && mt == 2 && plan.columns == 128) {
-        p.full_blocks = plan.full_blocks;
-        const int units = (rows_needed(a) + 31) / 32;
-        p.row_blocks = 2 * plan.full_blocks > units ? plan.full_blocks : units - plan.full_blocks;
-    }
+    p.full_blocks = plan.full_blocks;
+    p.row_blocks = plan.full_blocks ? plan.full_blocks + plan.low_blocks : plan.row_blocks;
     auto launch = [&]() {
         if (plan.columns < 128) return plan.columns == 32 * mt ? direct::launch_square(p, fp4, mt, st) : direct::launch_oblong(p, fp4, mt, st);
         if (plan.shared_rows) return next ? direct::launch_staged_next(p, st) : direct::launch_staged_plain(p, st);
@@ -1065,6 +1063,17 @@ extern "C" void svdq_gemm_int4_tile(const svdq_gemm_plan *plan, int64_t N, int b
     const g6::TileOf t = g6::tile_of(p, block, (p.full_blocks * p.kparts + p.half_blocks) * nblocks, nblocks);
     const int rows = t.whole ? g6::BM : g6::BM / 2, before = t.whole ? 0 : plan->full_blocks;
     *tile = svdq_gemm_tile{before * g6::BM + t.row_block * rows, rows, t.column_block, t.part, before + t.row_block, t.tile};
+}
+
+// (as gemm_direct_kernel takes them)
+extern "C" int svdq_gemm_few_rows_tile(const svdq_gemm_plan *plan, int64_t N, int block, svdq_gemm_tile *tile) {
+    const int column_blocks = (int)(N / plan->columns), full = plan->full_blocks * column_blocks;
+    const int total = (plan->full_blocks ? plan->full_blocks + plan->low_blocks : plan->row_blocks) * column_blocks;
+    const bool low = plan->full_blocks && block >= full;
+    const int blocks = low ? plan->low_blocks : plan->full_blocks ? plan->full_blocks : plan->row_blocks, mt = low ? 1 : plan->few_rows;
+    const int v = low ? direct::tile_of(block - full, total - full) : direct::tile_of(block, plan->full_blocks ? full : total), nb = v / blocks, mb = v - nb * blocks;
+    *tile = svdq_gemm_tile{(low ? plan->full_blocks * 64 : 0) + mb * mt * 32, mt * 32, nb, 0, (low ? plan->full_blocks : 0) + mb, (low ? full : 0) + v};
+    return total;
 }
 
 extern "C" int svdq_release_workspaces(void) {

@@ -813,13 +813,6 @@ __device__ __forceinline__ void output_tile(const GemmParams &p, const int nb, c
     }
 }
 
-// Tile number `block` of `total`: workgroups go to the XCDs round robin (number % 8), and each XCD gets one contiguous run of tiles, down the rows
-// first, so that the row blocks of a weight column meet in one L2 and every XCD streams its own share of the weights.
-__device__ inline int tile_of(int block, int total) {
-    const int xcd = block % 8, extra = total % 8;
-    return xcd * (total / 8) + (xcd < extra ? xcd : extra) + block / 8;
-}
-
 template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT, bool RANKS>
 __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_kernel(GemmParams p) {
     if constexpr (two_heights(FP4, MT, NT * WN)) {

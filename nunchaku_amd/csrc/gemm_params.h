@@ -197,7 +197,7 @@ struct GemmParams {
     float *vk, *vk_part;
     int vk_rows;
     int whole_band;              // 0, or (whole tiles only) the band height of the tile numbering in row blocks
-    int row_blocks, full_blocks; // few-rows kernels: tiles along M; NVFP4, 64 x 128 tiles: the first so many of 64 rows, the rest of 32
+    int row_blocks, full_blocks; // few-rows kernels: tiles along M; NVFP4, 64 x 128 tiles: the first so many of 64 rows, the rest of 32 (0: any other launch)
     int lr_steps;                // 16-rank steps of the low-rank operands that are copied to LDS ahead of the main loop
     float *next_lora_part;  // [N/128 column chunks][M_pad/32 slabs][R_down/16][2][64 lanes] x float4
 };
@@ -315,5 +315,15 @@ struct Params {
     int vk_rows;         // rows per batch entry, a multiple of 256
 };
 }  // namespace g6
+
+namespace direct {
+// The number of the tile that a workgroup of a few-rows launch takes, of `total`.  Workgroups go to the XCDs round robin (number % 8), and each XCD gets one contiguous run of tiles, down the rows
+// first, so that the row blocks of a weight column meet in one L2 and every XCD streams its own share of the weights; the 32-row tiles behind 64-row ones likewise.  (A
+// function that returns column block and rows too makes the compiler load the kernel's arguments behind the division: 0.2 us a launch.)
+__host__ __device__ inline int tile_of(int block, int total) {
+    const int xcd = block % 8, extra = total % 8;
+    return xcd * (total / 8) + (xcd < extra ? xcd : extra) + block / 8;
+}
+}  // namespace direct
 
 }  // namespace svdq

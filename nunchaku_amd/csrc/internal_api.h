@@ -15,15 +15,16 @@ int svdq_gemm_w4a4_rows(const svdq_gemm_args *args, int64_t rows, int noalloc, v
 // Which kernel a GEMM call takes and how it divides the work (zero where a field does not apply).
 typedef struct svdq_gemm_plan {
     int32_t few_rows;      // 0: a kernel with large tiles; 1, 2: the few-rows kernel in tiles of 32, 64 rows,
-    int32_t row_blocks;    // so many along M
-    int32_t full_blocks;   // INT4, large tiles: row blocks of 128 rows (NVFP4, few rows, 64 x 128: of 64 rows, in blocks of 32 what they leave),
+    int32_t row_blocks;    // so many along M (64-row blocks of the rows, where 32-row ones take the place of some: full_blocks, low_blocks)
+    int32_t full_blocks;   // INT4, large tiles: row blocks of 128 rows (NVFP4, few rows, 64 x 128: of 64 rows),
     int32_t half_blocks;   // of 64 rows behind them,
     int32_t kparts;        // and parts along K of every tile
     int32_t workgroups;    // NVFP4, large tiles: persistent workgroups;
     int32_t shared_tiles;  // some tiles are shared by two or more of them
     int32_t columns;       // few rows: columns of a tile (32, 64 or 128),
     int32_t shared_rows;   // its waves split the columns and share the rows' operands through LDS;
-    int32_t copied_ranks;  // the low-rank operands come through LDS (NVFP4, tiles of 128 columns)
+    int32_t copied_ranks;  // the low-rank operands come through LDS (NVFP4, tiles of 128 columns);
+    int32_t low_blocks;    // NVFP4, 64 x 128: row blocks of 32 rows behind the full ones
 } svdq_gemm_plan;
 
 // What svdq_gemm_w4a4 (`rows` > 0: svdq_gemm_w4a4_rows) would do with these arguments on a GPU of so many compute units.  Checks the
@@ -39,6 +40,8 @@ typedef struct svdq_gemm_tile {
     int32_t tile;          // the number that the parts of a tile meet under
 } svdq_gemm_tile;
 void svdq_gemm_int4_tile(const svdq_gemm_plan *plan, int64_t N, int block, svdq_gemm_tile *tile);
+// The same of a few-rows launch (column_block: of plan->columns; part 0, tile its number down the rows first); returns the number of workgroups.
+int svdq_gemm_few_rows_tile(const svdq_gemm_plan *plan, int64_t N, int block, svdq_gemm_tile *tile);
 
 #ifdef __cplusplus
 }

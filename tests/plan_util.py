@@ -9,7 +9,7 @@ from nunchaku_amd import _native as nv
 class Plan(ctypes.Structure):
     """Mirror of ``svdq_gemm_plan``."""
 
-    _fields_ = [(n, ctypes.c_int32) for n in ("few_rows", "row_blocks", "full_blocks", "half_blocks", "kparts", "workgroups", "shared_tiles", "columns", "shared_rows", "copied_ranks")]
+    _fields_ = [(n, ctypes.c_int32) for n in ("few_rows", "row_blocks", "full_blocks", "half_blocks", "kparts", "workgroups", "shared_tiles", "columns", "shared_rows", "copied_ranks", "low_blocks")]
 
     def __repr__(self):
         return "Plan(" + ", ".join(f"{n}={getattr(self, n)}" for n, _ in self._fields_ if getattr(self, n)) + ")"
