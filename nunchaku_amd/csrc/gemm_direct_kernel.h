@@ -80,6 +80,22 @@ struct Lds {
     static_assert(bytes(LR_AHEAD) <= 80 * 1024 && (!STAGED || 3 * bytes(4) <= 160 * 1024));
 };
 
+// The asynchronous copies of the low-rank operands.  A wave's request fetches 16 bytes a lane and fills a KB of LDS in the lanes' order: 16 columns of lora_up, 8 rows of lora_act, of
+// 32 ranks (`half`: of the last 16; the other half of the places is then filled with anything).  Where the request's lane reads, from the tile's first column or row and the chunk's first
+// rank on (up_base, act_base), and where the multiplying lanes find piece q of a row, counted from the chunk's first column or row.  Used by the host's model of the addresses too.
+__host__ __device__ __forceinline__ uint32_t up_copied(int request, int lane, int R, bool half) {
+    const int col = request * 16 + (lane >> 2), piece = (lane & 3) ^ g6::lr_up_swizzle(col);
+    return (uint32_t)col * (uint32_t)(R * 2) + (half ? piece & 1 : piece) * 16;
+}
+__host__ __device__ __forceinline__ uint32_t act_copied(int request, int lane, int R, bool half) {
+    const int row = request * 8 + (lane >> 3), piece = (lane & 7) ^ g6::lr_act_swizzle(row);
+    return (uint32_t)row * (uint32_t)(R * 4) + (half ? piece & 3 : piece) * 16;
+}
+__host__ __device__ __forceinline__ size_t up_base(int n0, int R, int chunk) { return (size_t)n0 * R * 2 + chunk * 64; }
+__host__ __device__ __forceinline__ size_t act_base(int row0, int R, int chunk) { return (size_t)row0 * R * 4 + chunk * 128; }
+__host__ __device__ __forceinline__ int up_place(int col, int piece) { return col * 64 + ((piece ^ g6::lr_up_swizzle(col)) << 4); }
+__host__ __device__ __forceinline__ int act_place(int row, int piece) { return row * 128 + ((piece ^ g6::lr_act_swizzle(row)) << 4); }
+
 // NVFP4 launches of 64 x 128 tiles have tiles of half the height behind them (few_rows_heights in gemm.hip).
 constexpr bool two_heights(bool fp4, int MT, int NC) { return fp4 && MT == 2 && NC == 4; }
 
@@ -347,15 +363,12 @@ __device__ __forceinline__ void output_tile(const GemmParams &p, const int nb, c
                 asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" :: "s"(lds_base + L::TAB + wave * 256), "v"(lane * 4), "s"(columns + n0 * 2) : "memory", "m0");
             // (32 ranks at a time; which 16 bytes of its row a lane fetches is permuted as in gemm6_kernel.h)
             for (int c = 0; 2 * c < lr_steps; c++) {
-                const bool half = nsteps - 2 * c < 2;  // 16 ranks only: the other half of the places is filled with anything
+                const bool half = nsteps - 2 * c < 2;
                 const uint32_t place = lds_base + L::LR + c * L::LR_CHUNK;
-                const uint8_t *up = (const uint8_t *)p.lora_up + (size_t)n0 * p.R_up * 2 + c * 64, *la = (const uint8_t *)p.lora_act + (size_t)row0 * p.R_up * 4 + c * 128;
+                const uint8_t *up = (const uint8_t *)p.lora_up + up_base(n0, p.R_up, c), *la = (const uint8_t *)p.lora_act + act_base(row0, p.R_up, c);
 #pragma unroll
                 for (int i = 0; i < 2; i++) {
-                    const int col = (wave * 2 + i) * 16 + (lane >> 2), row = (wave * 2 + i) * 8 + (lane >> 3);
-                    const int up_piece = (lane & 3) ^ g6::lr_up_swizzle(col), act_piece = (lane & 7) ^ g6::lr_act_swizzle(row);
-                    const uint32_t up_off = (uint32_t)col * (uint32_t)(p.R_up * 2) + (half ? up_piece & 1 : up_piece) * 16;
-                    const uint32_t act_off = (uint32_t)row * (uint32_t)(p.R_up * 4) + (half ? act_piece & 3 : act_piece) * 16;
+                    const uint32_t up_off = up_copied(wave * 2 + i, lane, p.R_up, half), act_off = act_copied(wave * 2 + i, lane, p.R_up, half);
                     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(place + (wave * 2 + i) * 1024), "v"(up_off), "s"(up) : "memory", "m0");
                     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(place + L::LR_ACT + (wave * 2 + i) * 1024), "v"(act_off), "s"(la) : "memory", "m0");
                 }
@@ -554,19 +567,17 @@ __device__ __forceinline__ void output_tile(const GemmParams &p, const int nb, c
         __syncthreads();  // the sums have been read: the low-rank operands (RANKS) and then the slabs take their place
         // (32 ranks at a time; which 16 bytes of its row a lane fetches is permuted as in gemm6_kernel.h)
         for (int c = 0; 2 * c < copied; c++) {
-            const bool half = nsteps - 2 * c < 2;  // 16 ranks only: the other half of the places is filled with anything
+            const bool half = nsteps - 2 * c < 2;
             const uint32_t place = lds_base + c * L::LR_CHUNK;
-            const uint8_t *up = (const uint8_t *)p.lora_up + (size_t)n0 * p.R_up * 2 + c * 64, *la = (const uint8_t *)p.lora_act + (size_t)row0 * p.R_up * 4 + c * 128;
+            const uint8_t *up = (const uint8_t *)p.lora_up + up_base(n0, p.R_up, c), *la = (const uint8_t *)p.lora_act + act_base(row0, p.R_up, c);
 #pragma unroll
             for (int i = 0; i < 2; i++) {
-                const int col = (wave * 2 + i) * 16 + (lane >> 2), up_piece = (lane & 3) ^ g6::lr_up_swizzle(col);
-                const uint32_t up_off = (uint32_t)col * (uint32_t)(p.R_up * 2) + (half ? up_piece & 1 : up_piece) * 16;
+                const uint32_t up_off = up_copied(wave * 2 + i, lane, p.R_up, half);
                 asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(place + (wave * 2 + i) * 1024), "v"(up_off), "s"(up) : "memory", "m0");
             }
 #pragma unroll
             for (int i = 0; i < MT; i++) {
-                const int row = (wave * MT + i) * 8 + (lane >> 3), act_piece = (lane & 7) ^ g6::lr_act_swizzle(row);
-                const uint32_t act_off = (uint32_t)row * (uint32_t)(p.R_up * 4) + (half ? act_piece & 3 : act_piece) * 16;
+                const uint32_t act_off = act_copied(wave * MT + i, lane, p.R_up, half);
                 asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(place + L::LR_ACT + (wave * MT + i) * 1024), "v"(act_off), "s"(la) : "memory", "m0");
             }
         }
@@ -604,12 +615,12 @@ __device__ __forceinline__ void output_tile(const GemmParams &p, const int nb, c
     auto add_copied = [&](const uint8_t *chunk, int s) {
         const uint8_t *buf = chunk + (s / 2) * L::LR_CHUNK;
         const int col = wave * 32 + r32, k = s % 2;
-        const u32x4_t up = *(const u32x4_t *)(buf + col * 64 + (((2 * k + h) ^ g6::lr_up_swizzle(col)) << 4));
+        const u32x4_t up = *(const u32x4_t *)(buf + up_place(col, 2 * k + h));
 #pragma unroll
         for (int o = 0; o < OWN; o++) {
             const int row = o * 32 + r32;
-            const uint8_t *ap = buf + L::LR_ACT + row * 128;
-            add_low_rank(o, s, *(const float4_t *)(ap + (((4 * k + 2 * h) ^ g6::lr_act_swizzle(row)) << 4)), *(const float4_t *)(ap + (((4 * k + 2 * h + 1) ^ g6::lr_act_swizzle(row)) << 4)), up);
+            const uint8_t *ap = buf + L::LR_ACT;
+            add_low_rank(o, s, *(const float4_t *)(ap + act_place(row, 4 * k + 2 * h)), *(const float4_t *)(ap + act_place(row, 4 * k + 2 * h + 1)), up);
         }
     };
 #pragma unroll

@@ -1,6 +1,7 @@
 // The few-rows GEMM with tiles narrower than 128 columns (plain epilogue, either precision): -DSVDQ_VARIANT=0 tiles as wide as high,
 // 1 the others; two translation units that build in parallel.
 #include "gemm_direct_kernel.h"
+#include "internal_api.h"
 
 namespace svdq {
 namespace direct {
@@ -32,3 +33,29 @@ int SVDQ_NAME(const GemmParams &p, bool fp4, int mt, hipStream_t stream) { retur
 
 }  // namespace direct
 }  // namespace svdq
+
+#if SVDQ_VARIANT == 0
+// The host's model of the low-rank operands' copies asks the kernel's own functions and layouts.
+using Shared = svdq::direct::Lds<2, 1, 4, 1, 3>;
+extern "C" void svdq_gemm_low_rank_of(int form, int rank, int three, svdq_gemm_low_rank *copies) {
+    using namespace svdq::direct;
+    if (form == 0) {
+        const int steps = Shared::lr_steps(rank, three != 0);
+        *copies = svdq_gemm_low_rank{Shared::LR, Shared::bytes(steps), steps, Shared::LR_CHUNK, Shared::LR_ACT, 8, 8};
+        return;
+    }
+    auto ranks = [&](auto layout, int mt) {
+        using L = decltype(layout);
+        const int most = 2 * (L::SUMS / L::LR_CHUNK), steps = rank / 16 < most ? rank / 16 : most;
+        *copies = svdq_gemm_low_rank{0, L::SUMS, steps, L::LR_CHUNK, L::LR_ACT, 8, 4 * mt};
+    };
+    if (form == 1) ranks(Lds<1, 4, 1, 4, 2>{}, 1);
+    else ranks(Lds<2, 4, 1, 4, 1>{}, 2);
+}
+extern "C" int64_t svdq_gemm_low_rank_copied(int act, int first, int rank, int chunk, int request, int lane) {
+    using namespace svdq::direct;
+    const bool half = rank / 16 - 2 * chunk < 2;
+    return act ? (int64_t)act_base(first, rank, chunk) + act_copied(request, lane, rank, half) : (int64_t)up_base(first, rank, chunk) + up_copied(request, lane, rank, half);
+}
+extern "C" int svdq_gemm_low_rank_place(int act, int index, int piece) { return act ? svdq::direct::act_place(index, piece) : svdq::direct::up_place(index, piece); }
+#endif

@@ -43,6 +43,19 @@ void svdq_gemm_int4_tile(const svdq_gemm_plan *plan, int64_t N, int block, svdq_
 // The same of a few-rows launch (column_block: of plan->columns; part 0, tile its number down the rows first); returns the number of workgroups.
 int svdq_gemm_few_rows_tile(const svdq_gemm_plan *plan, int64_t N, int block, svdq_gemm_tile *tile);
 
+// The asynchronous copies of the low-rank operands in tiles of 64 x 128 whose waves share the rows (`form` 0) and in tiles of 32 (1) and 64 rows (2) of copied_ranks.
+typedef struct svdq_gemm_low_rank {
+    int32_t first, end;       // LDS that may hold them, in bytes: what the launch has (form 0, three workgroups per compute unit or two), the place of the sums
+    int32_t steps;            // 16-rank steps that come this way
+    int32_t chunk, act;       // bytes of 32 ranks; where in them lora_act's stand
+    int32_t up_requests, act_requests;  // a KB each, 64 lanes of 16 bytes, of 32 ranks
+} svdq_gemm_low_rank;
+void svdq_gemm_low_rank_of(int form, int rank, int three, svdq_gemm_low_rank *copies);
+// Byte offsets of what lane `lane` of request `request` of chunk `chunk` reads, from the operand's first column (`act`: row) of the tile, which is `first`, on
+int64_t svdq_gemm_low_rank_copied(int act, int first, int rank, int chunk, int request, int lane);
+// and of 16-byte piece `piece` of a column's (row's) 32 ranks in LDS, from the chunk's lora_up (lora_act) on.
+int svdq_gemm_low_rank_place(int act, int index, int piece);
+
 #ifdef __cplusplus
 }
 #endif
