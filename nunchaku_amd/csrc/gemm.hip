@@ -643,7 +643,7 @@ struct FewRowsTile {
 // the last but one multiple of the compute units; 1.5 % have to be gained, equal ones go to the fewest 64-row tiles.  The GEMM alone, one height / two, us, rank 32, K = 3072: norm and
 // rotary, N = 9216, M = 300 21.0 / 19.2, M = 505 33.1 / 29.9, M = 700 43.5 / 40.1, M = 1200 66.3 / 63.8; quantizing, N = 12288, M = 400 40.2 / 37.0, M = 1157 97.2 / 91.9; plain, N = 3072,
 // M = 2300 41.0 / 39.4.  4.5 % faster over 4600 launches of 16 ... 9216 rows (with the epilogue's requests ahead of the main loop, which came before), 6 of them slower by more than 3 %.  (Slower:
-// 32-row tiles where the model sees no gain, up to 9 % where all rows are in them; INT4, whose launches of several tiles per compute unit share the rows or are large tiles.)
+// 32-row tiles where the model sees no gain, up to 9 % where all rows are in them.  Not built for INT4, whose launches of several tiles per compute unit share the rows or are large tiles.)
 // Not where tiles of 32 rows alone would be two per compute unit at most: so few are not handed to the emptiest one, and what bounds them is the requests, not the matrix core
 // that the model is about.  1508 such launches are 14 % faster in 32-row tiles than in two heights, none of them slower by 4 %: SiLU, M = 67, K = 2944, N = 19840 15.7 / 18.6 us,
 // quantizing, M = 65, K = 6272, N = 18176, rank 64 34.9 / 40.9.  (At three 185 launches 34 % faster.)
@@ -735,7 +735,8 @@ FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu, int shape, const Height
 // rotary, M = 640, K = 3072, N = 9216 27.7 / 26.4 us), 19 of them 3 to 10 % slower (about 5000 or 6000 columns, 323 ... 360 large tiles).  Not with few columns: 377 launches of less than 1536 at K = 1536
 // and more, and of less than 3072 at K = 4096 and more, neither faster nor slower on average, 33 of them 3 to 8 % slower (plain, M = 4184, K = 5376, N = 1280 42.0 / 45.3); less than 1024 up to 14 % slower
 // (linear attention, M = 15360, K = 256, N = 384 16.0 / 18.6); rank 128, whose operands do not all fit beside the stages of three
-// workgroups, 8.8 % slower, above three tiles 12 to 25 % slower.  (Between two and two and a half, where it is 4 %, and at three calls keep the kernel they had.)
+// workgroups, 8.8 % slower, above three tiles 12 to 25 % slower.  (Between two and two and a half large tiles are kept though 4 % slower: a gain that has not been
+// taken yet.)
 enum class SharedRows { NO, IF_FASTEST, YES };
 // (`split`: the large tiles would be split along K, see choose_direct)
 SharedRows staged_rows(const svdq_gemm_args *a, int ncu, bool split) {
@@ -819,7 +820,7 @@ FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
             // Ranks above 32, whose operands come through LDS in the few-rows kernel, cost it 0.17 us per 16 ranks and tile of 64 rows, and more at K below 1536, where the copies of a tile
             // have fewer products of another to pass beside: 0.31 (large tiles in several rounds: 0.41) at K = 0.  Of 1062 launches that this brings here 30 are slower than in large tiles by 3 %
             // and more, 12 % at most; with 0.17 at any K 267 of 1500, up to 28 % (large tiles / few rows, us: plain, M = 15370, K = 128, N = 1920, rank 80 37.7 / 48.3, norm and rotary, M = 10352, K = 384, N = 3072,
-            // rank 64 58.0 / 67.7).  (From rank 128 on it stands at 0.33, with which the short rows near the line keep the kernel they had.)  Ranks up to 32 at K = 128: by the 64-row tiles alone,
+            // rank 64 58.0 / 67.7).  (From rank 128 on it stands at 0.33, not fitted again.)  Ranks up to 32 at K = 128: by the 64-row tiles alone,
             // 32-row ones behind them gain nothing there (plain, M = 11853, K = 128, N = 1280, rank 0 14.8 / 17.4).
             const double shorter = a->K < 1536 ? 1.0 - (double)a->K / 1536 : 0.0;
             auto shape2_rank = [&](double up_to_32, double short_rows) { return a->R_up <= 32 ? up_to_32 : a->R_up < 128 ? 0.17 + short_rows * shorter : 0.33; };

@@ -102,9 +102,9 @@ constexpr bool two_heights(bool fp4, int MT, int NC) { return fp4 && MT == 2 && 
 // One tile: MT blocks of 32 rows from block f0 on, column block nb.
 // RANKS (NVFP4, tiles of 128 columns, ranks above 32; which launches: copies_ranks in gemm.hip): all four waves need the low-rank operands of the same rows, and a lane that fetches 16 bytes of a row for itself costs
 // the vector memory path four times as much as whole pieces of rows do.  The operands go to the place of the sums by asynchronous copies, once these have been
-// read, up to rank 128 all at once; two steps requested ahead of the sums and the others behind them, a memory latency each / so, us, the GEMM alone: K = 1408, N = 15872, M = 213, rank 64
-// 15.1 / 13.7, rank 128 18.2 / 15.0; norm and rotary, M = 505, K = 3072, N = 9216, rank 64 32.9 / 31.8, rank 128 38.1 / 33.8, rank 160 43.0 / 36.8; quantizing, M = 1157, N = 12288, rank 64 102.7 / 100.6,
-// rank 128 122.5 / 115.6.  Same bits.  (A kernel of its own: beside the other way in one, ranks up to 32 lost up to 2 %.  INT4: no gain.)
+// read, up to rank 128 all at once; two steps requested ahead of the sums and the others behind them, a memory latency each / so, us, the GEMM alone: SiLU, K = 1408, N = 15872, M = 213, rank 64
+// 17.4 / 16.3, rank 128 20.4 / 17.5; norm and rotary, M = 505, K = 3072, N = 9216, rank 64 33.9 / 32.3, rank 128 38.9 / 34.1, rank 160 43.0 / 36.1; quantizing, M = 1157, N = 12288, rank 64 100.9 / 98.3,
+// rank 128 123.4 / 114.2.  Same bits.  (A kernel of its own: beside the other way in one, ranks up to 32 lost up to 2 %.  INT4: no gain.)
 template <bool FP4, int MT, int NT, int WN, int KP, int DEPTH, bool NEXT, bool RANKS>
 __device__ __forceinline__ void output_tile(const GemmParams &p, const int nb, const int f0) {
     constexpr int NC = NT * WN;  // 32-column tiles of the workgroup; a wave has NT of them
@@ -199,8 +199,10 @@ __device__ __forceinline__ void output_tile(const GemmParams &p, const int nb, c
     // K = 2048, N = 8192, quantizing 15.95 / 15.2, NVFP4 M = 300, K = 3072, N = 9216 with norm and rotary 33.5 / 32.1; shared rows M = 256, K = 3072, N = 9216 with norm and rotary
     // 18.8 / 17.5, rank 128 25.1 / 20.8, quantizing, N = 12288 25.3 / 23.5, M = 200, K = 1024, N = 15360, rank 128 16.2 / 11.6.  Same bits.  Slower: low-rank operands ahead in
     // narrow NVFP4 tiles (several of them share a compute unit: M = 916, K = 1920, N = 1152 10.4 us, 10.7 with), more than two steps in registers, all of them through the place of the
-    // sums, which takes two barriers more, the rotary table and the smoothing factors ahead too.  (With three INT4 tiles of 64 x 64 per compute unit it costs 1 %: M = 1979, K = 4096,
-    // N = 1152 22.0 / 22.3.)
+    // sums, which takes two barriers more, the rotary table and the smoothing factors ahead too.  It costs 3 to 4 %
+    // where INT4 tiles of 64 x 64 are one to two per compute unit at ranks of 80 and more (M = 600, K = 2048, N = 3200, rank 144 11.5 / 12.0; all such tiles 6 % faster), and 0.1 to 0.2 of 4 us at ranks 16 and 32 with K up
+    // to 512 in INT4 tiles of 32 x 64, and of 32 x 32 where there are more than two (all of 32 x 32 6 % faster, of 32 x 64 2).  There too it stays: low-rank operands requested behind the loop's first
+    // ones take 4 % of what 32 x 32 tiles gain and 3 % of 32 x 64 ones at rank 0, a branch on K costs 1 to 7 %, and other tiles are no faster.
     constexpr int OWN = NARROW ? 1 : MT, LR_AHEAD = L::LR_AHEAD, EARLY = NARROW && !FP4 ? 2 : 0;
     constexpr bool TABLE = !STAGED && (!NARROW || FP4 || MT * NC < 4);  // factors and biases through a table of the wave's
     const bool owner = !NARROW || wave < MT * NC;

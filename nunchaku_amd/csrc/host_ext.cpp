@@ -4,10 +4,10 @@
 // at the parameters' version counters, allocating four tensors and filling two argument blocks took 19.6 us in Python (31.2
 // for the fused MLP, 29.4 for the QKV projection, 11.4 for the AWQ layer), more than the GPU needs for a few hundred tokens;
 // here it takes 8.8 (14.1, 8.4 and 5.1), most of it the launches themselves.  The operators called one by one keep their one
-// way to the library (_native.launch); what is here is their checks, allocations and argument blocks.  They took 12.7 us
-// (quantize), 13.9 (GEMM; 17.8 with linear attention, which clears out_vk in a launch of its own) and 8.5
-// (linearattn_vk_mul_q) of the caller's time, and take 8.8, 5.4 (8.3) and 3.5: linear attention over 256 tokens at K = 1024,
-// four launches of which the GPU runs 18 us, went from 46.5 us to 25.9.
+// way to the library (_native.launch); what is here is their checks, allocations and argument blocks.  They took 11.4 us
+// (quantize), 14.8 (GEMM; 18.8 with linear attention, which adds up the shares of out_vk in a launch of its own) and 8.8
+// (linearattn_vk_mul_q) of the caller's time, and take 7.3, 5.6 (8.4) and 3.5: linear attention over 256 tokens at K = 1024,
+// four launches, went from 40.2 us to 19.4.
 //
 // Every function returns None when anything about the call is not the plain case it handles (another dtype, a parameter
 // that has been replaced since the layer was converted, a tensor that is not contiguous, ...): the Python code behind it

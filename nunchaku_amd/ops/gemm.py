@@ -85,7 +85,7 @@ def svdq_gemm_w4a4(
     out_linearattn bf16 [B, tokens_pad, N/3] with out_vk fp32 [B, heads, 33, 32] (N = 3 * heads * 32, tokens_pad a
     multiple of 256): linear attention (launch_impl.cuh:311-345): relu(q) goes to out_linearattn;
     out_vk[b, h, i, j] = sum over tokens of v[i] * relu(k[j]) (i < 32) and of relu(k[j]) (i = 32), where the
-    columns after q hold, per head, 32 of k then 32 of v.  out_vk is cleared first.
+    columns after q hold, per head, 32 of k then 32 of v.  What out_vk held before does not matter.
     """
     if (getattr(act, "is_cuda", False) and qout is None and rotary_emb is None and out_q is None and out_k is None and out_v is None and norm_q is None
             and norm_k is None and lora_down is None and lora_act_out is None and poolout is None):
