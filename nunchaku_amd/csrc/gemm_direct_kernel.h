@@ -98,6 +98,10 @@ __host__ __device__ __forceinline__ int act_place(int row, int piece) { return r
 
 // NVFP4 launches of 64 x 128 tiles have tiles of half the height behind them (few_rows_heights in gemm.hip).
 constexpr bool two_heights(bool fp4, int MT, int NC) { return fp4 && MT == 2 && NC == 4; }
+// Of NVFP4 tiles of 128 columns the ring of k-groups on their way is as deep as the registers of two waves per SIMD allow (64 rows: a second k-group would fit, and costs 3 % where compute
+// units have several tiles).
+template <int MT>
+constexpr int FP4_RING = MT == 1 ? 2 : 1;
 
 // One tile: MT blocks of 32 rows from block f0 on, column block nb.
 // RANKS (NVFP4, tiles of 128 columns, ranks above 32; which launches: copies_ranks in gemm.hip): all four waves need the low-rank operands of the same rows, and a lane that fetches 16 bytes of a row for itself costs
@@ -836,7 +840,7 @@ __global__ void __launch_bounds__(64 * WN * KP, WN == 4 ? 3 : 2) gemm_direct_ker
         } else {
             // (as deep a ring as the launches of 32-row tiles alone have)
             const int half_blocks = p.row_blocks - p.full_blocks, v = tile_of(block - full, (int)gridDim.x - full), nb = v / half_blocks;
-            output_tile<FP4, 1, NT, WN, KP, 2, NEXT, RANKS>(p, nb, p.full_blocks * 2 + v - nb * half_blocks);
+            output_tile<FP4, 1, NT, WN, KP, FP4_RING<1>, NEXT, RANKS>(p, nb, p.full_blocks * 2 + v - nb * half_blocks);
         }
     } else {
         const int v = tile_of((int)blockIdx.x, (int)gridDim.x), nb = v / p.row_blocks;
@@ -861,6 +865,13 @@ int launch_direct(const GemmParams &params, hipStream_t stream) {
     p.lr_steps = L::lr_steps(p.R_up, tiles > 2 * compute_units(dev));
     SVDQ_LAUNCH(kern, dim3((unsigned)tiles), dim3(64 * WN * KP), L::bytes(p.lr_steps), stream, p);
     return check_launch("gemm_w4a4 (few rows)");
+}
+
+// NVFP4, tiles of 32 (shape 1) or 64 rows x 128 columns
+template <bool NEXT, bool RANKS>
+int launch_fp4(const GemmParams &p, int shape, hipStream_t stream) {
+    if (shape == 1) return launch_direct<true, 1, 4, 1, 4, FP4_RING<1>, NEXT, RANKS>(p, stream);
+    return launch_direct<true, 2, 4, 1, 4, FP4_RING<2>, NEXT, RANKS>(p, stream);
 }
 
 }  // namespace direct

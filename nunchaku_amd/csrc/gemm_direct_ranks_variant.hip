@@ -1,5 +1,5 @@
 // The NVFP4 few-rows GEMM of ranks above 32 in tiles of 128 columns (compiled with -DSVDQ_VARIANT=0: plain epilogue, 1: the others): two translation
-// units that build in parallel.  Tiles and rings are those of gemm_direct_variant.hip.
+// units that build in parallel.
 #include "gemm_direct_kernel.h"
 
 namespace svdq {
@@ -10,9 +10,7 @@ int launch_fp4_ranks_plain(const GemmParams &p, int shape, hipStream_t stream) {
 #else
 int launch_fp4_ranks_next(const GemmParams &p, int shape, hipStream_t stream) {
 #endif
-    constexpr bool NEXT = SVDQ_VARIANT;
-    if (shape == 1) return launch_direct<true, 1, 4, 1, 4, 2, NEXT, true>(p, stream);
-    return launch_direct<true, 2, 4, 1, 4, 1, NEXT, true>(p, stream);
+    return launch_fp4<SVDQ_VARIANT != 0, true>(p, shape, stream);
 }
 
 }  // namespace direct

@@ -16,11 +16,14 @@ namespace direct {
 #endif
 
 int SVDQ_NAME(const GemmParams &p, int shape, hipStream_t stream) {
-    constexpr bool FP4 = SVDQ_VARIANT >= 2, NEXT = SVDQ_VARIANT & 1;
-    // (the ring of k-groups on their way as deep as the registers of two waves per SIMD allow; NVFP4, 64 rows: a second k-group would
-    // fit, and costs 3 % where compute units have several tiles)
-    if (shape == 1) return launch_direct<FP4, 1, 4, 1, 4, FP4 ? 2 : 1, NEXT>(p, stream);
-    return launch_direct<FP4, 2, FP4 ? 4 : 2, FP4 ? 1 : 2, FP4 ? 4 : 2, 1, NEXT>(p, stream);
+    constexpr bool NEXT = SVDQ_VARIANT & 1;
+#if SVDQ_VARIANT >= 2
+    return launch_fp4<NEXT, false>(p, shape, stream);
+#else
+    // (the ring of k-groups on their way as deep as the registers of two waves per SIMD allow)
+    if (shape == 1) return launch_direct<false, 1, 4, 1, 4, 1, NEXT>(p, stream);
+    return launch_direct<false, 2, 2, 2, 2, 1, NEXT>(p, stream);
+#endif
 }
 
 }  // namespace direct

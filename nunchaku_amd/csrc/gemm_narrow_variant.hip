@@ -49,8 +49,8 @@ extern "C" void svdq_gemm_low_rank_of(int form, int rank, int three, svdq_gemm_l
         const int most = 2 * (L::SUMS / L::LR_CHUNK), steps = rank / 16 < most ? rank / 16 : most;
         *copies = svdq_gemm_low_rank{0, L::SUMS, steps, L::LR_CHUNK, L::LR_ACT, 8, 4 * mt};
     };
-    if (form == 1) ranks(Lds<1, 4, 1, 4, 2>{}, 1);
-    else ranks(Lds<2, 4, 1, 4, 1>{}, 2);
+    if (form == 1) ranks(Lds<1, 4, 1, 4, FP4_RING<1>>{}, 1);
+    else ranks(Lds<2, 4, 1, 4, FP4_RING<2>>{}, 2);
 }
 extern "C" int64_t svdq_gemm_low_rank_copied(int act, int first, int rank, int chunk, int request, int lane) {
     using namespace svdq::direct;
