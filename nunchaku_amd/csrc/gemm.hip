@@ -730,10 +730,10 @@ FewRowsTile plain_tile(const svdq_gemm_args *a, int ncu, int shape, const Height
 // 2.25 tiles M = 505, K = 3072, N = 9216 34.6 / 29.6 / 30.6; quantizing epilogue K = 3072, N = 12288 M = 256 29.8 / 29.2 / 26.7, M = 300 30.8 / 30.4 / 28.8, at three tiles M = 505
 // 43.6 / 39.4 / 39.3, rank 128 59.4 / 47.3 / 52.6; layer calls, plain M = 384, K = 3072, N = 9216 26.3 / 22.8 with this one, M = 320 (1.4 tiles, where narrow ones are better)
 // 22.4 / 22.6, M = 505 30.4 / 32.1.
-// Also with two and a half to (less than) three tiles per compute unit and ranks up to 64: whole large tiles are then one and a half per compute unit at best, where the
-// second one doubles the time of the first.  1123 launches (K = 256 ... 16640, all epilogues) 6 % faster than large tiles, 12 % with K below 1024, 5 with N = 6144 and more at K = 8192 ... 16640 (norm and
-// rotary, M = 640, K = 3072, N = 9216 27.7 / 26.4 us), 19 of them 3 to 10 % slower (about 5000 or 6000 columns, 323 ... 360 large tiles).  Not with few columns: 377 launches of less than 1536 at K = 1536
-// and more, and of less than 3072 at K = 4096 and more, neither faster nor slower on average, 33 of them 3 to 8 % slower (plain, M = 4184, K = 5376, N = 1280 42.0 / 45.3); less than 1024 up to 14 % slower
+// Also with two and a half to (less than) three tiles per compute unit, ranks up to 64 and 1024 columns: whole large tiles are then one and a half per compute unit at best, where the
+// second one doubles the time of the first.  2075 launches (K = 256 ... 16640, all epilogues) 5 % faster than large tiles, 12 % with K below 1024, 5 with N = 6144 and more at K = 8192 ... 16640 (norm and
+// rotary, M = 640, K = 3072, N = 9216 27.7 / 26.4 us), 33 of them 3 to 10 % slower (half of them of 4500 to 6200 columns, 323 ... 360 large tiles).  Not with less than 2048 columns that large tiles have whole blocks of
+// 256 of, and K = 1536 or more: 1.3 % slower over 197 launches, 25 of them 3 to 8 % (plain, M = 4184, K = 5376, N = 1280 42.0 / 45.3; where half of the last block is none, as at N = 1152 and 1408, 1 % faster).  Less than 1024 columns up to 14 % slower
 // (linear attention, M = 15360, K = 256, N = 384 16.0 / 18.6); rank 128, whose operands do not all fit beside the stages of three
 // workgroups, 8.8 % slower, above three tiles 12 to 25 % slower.  (Between two and two and a half large tiles are kept though 4 % slower: a gain that has not been
 // taken yet.)
@@ -742,8 +742,8 @@ enum class SharedRows { NO, IF_FASTEST, YES };
 SharedRows staged_rows(const svdq_gemm_args *a, int ncu, bool split) {
     if (a->fp4 || a->K < 256) return SharedRows::NO;
     const long long tiles = (rows_needed(a) + 63) / 64 * (a->N / 128);
-    const int64_t columns = a->K < 1536 ? 1024 : a->K < 4096 ? 1536 : 3072;
-    if (!split && a->R_up <= 64 && a->N >= columns && 2 * tiles >= 5 * ncu && tiles < 3 * ncu) return SharedRows::YES;
+    const bool whole_blocks = a->N % 256 == 0 && a->N < 2048 && a->K >= 1536;
+    if (!split && a->R_up <= 64 && a->N >= 1024 && !whole_blocks && 2 * tiles >= 5 * ncu && tiles < 3 * ncu) return SharedRows::YES;
     const bool may = 2 * tiles >= (needs_next_epilogue(a) ? 2 * ncu + 2 : 3 * ncu) && tiles <= (a->qout && split ? 3 : 2) * ncu;
     return may ? SharedRows::IF_FASTEST : SharedRows::NO;
 }

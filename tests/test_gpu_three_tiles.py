@@ -31,10 +31,10 @@ def test_which_launches(kind, M, K, N, R, shared):
     assert p.shared_rows == shared, p
 
 
-# Few columns go with short rows only: 1024 up to K = 1408, 1536 up to 3968, 3072 at any K.
+# Less than 2048 columns that are whole blocks of 256: up to K = 1408.
 @pytest.mark.parametrize("kind,M,K,N,R,shared", [
-    ("plain", 5300, 1408, 1152, 32, 1), ("plain", 5300, 1536, 1152, 32, 0), ("plain", 4184, 5376, 1280, 16, 0), ("rope", 3700, 3968, 1536, 32, 1), ("rope", 3700, 4096, 1536, 32, 0),
-    ("silu", 1860, 4096, 2944, 64, 0), ("silu", 1860, 4096, 3072, 64, 1), ("rope", 640, 15360, 9216, 32, 1), ("next", 1700, 15360, 3072, 16, 1),
+    ("plain", 4184, 1408, 1280, 32, 1), ("plain", 4184, 1536, 1280, 32, 0), ("plain", 4184, 5376, 1280, 16, 0), ("silu", 5451, 5504, 1024, 32, 0), ("rope", 3700, 2304, 1536, 32, 0),
+    ("plain", 4864, 5376, 1152, 32, 1), ("plain", 3000, 1536, 1920, 32, 1), ("plain", 2700, 5376, 2048, 32, 1), ("rope", 640, 15360, 9216, 32, 1), ("next", 1700, 15360, 3072, 16, 1),
 ])
 def test_which_columns(kind, M, K, N, R, shared):
     p = plan_of(call(kind, M, K, N, R, False))
