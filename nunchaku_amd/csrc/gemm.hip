@@ -818,13 +818,13 @@ FewRowsTile choose_direct(const svdq_gemm_args *a, int ncu) {
             };
             constexpr Model shape1{3.7, 1.06, 0.1132, 0.248, 1.37, 0.79, 0.49, 0.16};
             // Ranks above 32, whose operands come through LDS in the few-rows kernel, cost it 0.17 us per 16 ranks and tile of 64 rows, and more at K below 1536, where the copies of a tile
-            // have fewer products of another to pass beside: 0.31 (large tiles in several rounds: 0.41) at K = 0.  Of 1062 launches that this brings here 30 are slower than in large tiles by 3 %
+            // have fewer products of another to pass beside: 0.31 (large tiles in several rounds: 0.41) at K = 0.  Of 1071 launches that this brings here 31 are slower than in large tiles by 3 %
             // and more, 12 % at most; with 0.17 at any K 267 of 1500, up to 28 % (large tiles / few rows, us: plain, M = 15370, K = 128, N = 1920, rank 80 37.7 / 48.3, norm and rotary, M = 10352, K = 384, N = 3072,
-            // rank 64 58.0 / 67.7).  (From rank 128 on it stands at 0.33, not fitted again.)  Ranks up to 32 at K = 128: by the 64-row tiles alone,
-            // 32-row ones behind them gain nothing there (plain, M = 11853, K = 128, N = 1280, rank 0 14.8 / 17.4).
+            // rank 64 58.0 / 67.7).  (From rank 128 on it stands at 0.33, not fitted again.)  Ranks 0 and 16 at K = 128: by the 64-row tiles alone,
+            // 32-row ones behind them gain nothing there (plain, M = 11853, K = 128, N = 1280, rank 0 14.8 / 17.4; rank 32, where large tiles take longer, N = 896, M = 12799 17.4 / 15.0).
             const double shorter = a->K < 1536 ? 1.0 - (double)a->K / 1536 : 0.0;
             auto shape2_rank = [&](double up_to_32, double short_rows) { return a->R_up <= 32 ? up_to_32 : a->R_up < 128 ? 0.17 + short_rows * shorter : 0.33; };
-            const double rounds2 = a->R_up <= 32 && a->K < 256 ? c2 : tall.time;
+            const double rounds2 = a->R_up < 32 && a->K < 256 ? c2 : tall.time;
             double t_few;
             if (tiles <= 1.0) {
                 const Model shape2{4.43, 1.19, 0.165, shape2_rank(0.423, 0.14), 2.48, 1.51, 0.92, 0.48};
